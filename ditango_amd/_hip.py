@@ -40,6 +40,9 @@ _SIGNATURES = {
                                              c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_vp]),
     "dt_attn_chunk_f32_fwd": (ctypes.c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_i32, c_i32, c_i32, c_i32, c_i32,
                                              c_i64, c_i64, c_i64, c_i64, c_i64, c_i64, c_f32, c_vp]),
+    "dt_attn_jobs_f32_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
+                                            c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), _P(c_i64), _P(c_i64),
+                                            c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_f32, c_vp]),
     "dt_attn_jobs_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                         c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                         c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_f32, c_vp]),
@@ -158,6 +161,7 @@ def _check_qkv(q: torch.Tensor, name: str = "q", dtype: Optional[torch.dtype] = 
 
 
 def _attn_flags(q: torch.Tensor, q_prescaled: bool) -> int:
+    _require(q.dtype in HALF_DTYPES, f"the MFMA kernels take bf16 or fp16 tensors (got {q.dtype})")
     _require(not (q_prescaled and q.dtype == torch.float16), "a prescaled q is a bf16 mode")
     return (DT_ATTN_Q_PRESCALED if q_prescaled else 0) | (DT_ATTN_FP16 if q.dtype == torch.float16 else 0)
 
@@ -210,21 +214,50 @@ def attn_chunk_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_sc
 
 def attn_chunk_f32_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softmax_scale: float = 0.0):
     """(out fp32 [B,Sq,H,D], lse fp32 [B,H,Sq]) of fp32 q against one fp32 KV chunk, computed in fp32."""
+    return attn_jobs_f32_fwd(q, [k], [v], [[0]], softmax_scale)[0]
+
+
+def attn_jobs_f32_fwd(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor],
+                      jobs: Sequence[Sequence[int]], softmax_scale: float = 0.0) -> List[Tuple[torch.Tensor, torch.Tensor]]:
+    """One launch: the fp32 states (out [B,Sq,H,D], lse [B,H,Sq]) of fp32 q against the concatenations of the fp32
+    chunks ``jobs[j]``.  Each chunk may have strides of its own.  More jobs or chunks than one launch addresses run in
+    several."""
     lib = load_library()
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        _require(t.is_cuda and t.dtype == torch.float32 and t.dim() == 4 and t.stride(-1) == 1,
-                 f"{name} must be fp32 [B,S,H,D] on the GPU with contiguous D")
     B, Sq, H, D = q.shape
-    Sk = k.shape[1]
-    _require(k.shape == v.shape and k.shape[0] == B and k.shape[2] == H and k.shape[3] == D, "k/v shape mismatch")
-    _require(k.stride() == v.stride(), "k and v must share strides")
-    out = torch.empty((B, Sq, H, D), dtype=torch.float32, device=q.device)
-    lse = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)
-    rc = lib.dt_attn_chunk_f32_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
-                                   B, Sq, Sk, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                   k.stride(0), k.stride(1), k.stride(2), float(softmax_scale), _stream())
-    _check(rc, "dt_attn_chunk_f32_fwd")
-    return out, lse
+    _check_qkv(q, "q", torch.float32)
+    for i, (k, v) in enumerate(zip(k_chunks, v_chunks)):
+        _check_qkv(k, f"k[{i}]", torch.float32)
+        _check_qkv(v, f"v[{i}]", torch.float32)
+        _require(k.shape == v.shape and k.shape[0] == B and k.shape[2] == H and k.shape[3] == D, "k/v shape mismatch")
+        _require(k.stride() == v.stride(), "k and v must share strides")
+    states = [(torch.empty((B, Sq, H, D), dtype=torch.float32, device=q.device),
+               torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)) for _ in jobs]
+    start = 0
+    while start < len(jobs):
+        ids: List[int] = []          # chunks of this launch, in order of first use
+        begin, flat, end = [0], [], start
+        while end < len(jobs) and end - start < DT_MAX_JOBS and len(flat) + len(jobs[end]) <= DT_MAX_JOB_ENTRIES:
+            more = ids + [c for c in dict.fromkeys(jobs[end]) if c not in ids]
+            if len(more) > DT_MAX_CHUNKS:
+                break
+            ids = more
+            flat += [ids.index(c) for c in jobs[end]]
+            begin.append(len(flat))
+            end += 1
+        _require(end > start, f"job {start} references more chunks than one launch addresses: split it and merge the parts")
+        n, m = end - start, max(1, len(ids))
+        ks, vs = [k_chunks[c] for c in ids], [v_chunks[c] for c in ids]
+        rc = lib.dt_attn_jobs_f32_fwd(
+            q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2), len(ids),
+            (c_vp * m)(*[k.data_ptr() for k in ks]), (c_vp * m)(*[v.data_ptr() for v in vs]),
+            (c_i32 * m)(*[k.shape[1] for k in ks]), (c_i64 * m)(*[k.stride(0) for k in ks]),
+            (c_i64 * m)(*[k.stride(1) for k in ks]), (c_i64 * m)(*[k.stride(2) for k in ks]),
+            n, (c_i32 * (n + 1))(*begin), (c_i32 * max(1, len(flat)))(*flat),
+            (c_vp * n)(*[s[0].data_ptr() for s in states[start:end]]), (c_vp * n)(*[s[1].data_ptr() for s in states[start:end]]),
+            float(softmax_scale), _stream())
+        _check(rc, "dt_attn_jobs_f32_fwd")
+        start = end
+    return states
 
 
 _workspaces: "dict" = {}   # (device type, index, stream handle) -> tensor, in order of last use

@@ -200,8 +200,8 @@ class proAttention:
         self.q_prescaled = False
         # What happens to fp32 inputs (flash_attn_func takes none; the reference's CPU-runnable configuration is
         # stated in fp32): "round" = rounded to bf16 at the kernel boundary, the bf16 MFMA kernels run;
-        # "exact" = every fresh state is computed in fp32 from the fp32 tensors (dt_attn_chunk_f32_fwd, a
-        # plain vector-ALU kernel for small problems) and only cached states are rounded to bf16.
+        # "exact" = every fresh state is computed in fp32 from the fp32 tensors (dt_attn_jobs_f32_fwd, fp32
+        # matrix instructions) and only cached states are rounded to bf16.
         self.fp32_inputs = "round"
         self._exact_f32 = False
         # while a variable-length call runs: (cu_seqlens_q, chunk -> cu_seqlens_kv) as host lists, or a
@@ -307,25 +307,34 @@ class proAttention:
         v_c = v_c if v_c.dim() == 4 else v_c.view(B, v_c.shape[0] // B, v_c.shape[1], v_c.shape[2])
         return k_c, v_c
 
-    def _job_state_f32(self, query, chunks, key, value):
-        """The fp32 state of ``query`` against the concatenation of ``chunks``, computed in fp32."""
+    def _job_states_f32(self, query, jobs, key, value):
+        """The fp32 states of ``query`` against the concatenations of the chunks ``jobs[j]``, computed in fp32."""
         if self._segments is not None:
             raise NotImplementedError("fp32_inputs = 'exact' does not cover variable-length calls")
         B = query.shape[0]
-        states = [_hip.attn_chunk_f32_fwd(query, *self._chunk_f32(c, key, value, B)) for c in chunks]
-        if len(states) == 1:
-            return states[0]
-        return _hip.merge_states([s[0] for s in states], [s[1] for s in states], dst_dtype=torch.float32)
+        needed = sorted({c for job in jobs for c in job})
+        kv = [self._chunk_f32(c, key, value, B) for c in needed]
+        index = {c: i for i, c in enumerate(needed)}
+        # (a block of more chunks than one launch addresses is computed in pieces)
+        pieces = [[job[i:i + self._MAX_JOB_CHUNKS] for i in range(0, len(job), self._MAX_JOB_CHUNKS)] for job in jobs]
+        states = iter(_hip.attn_jobs_f32_fwd(query, [k for k, _ in kv], [v for _, v in kv],
+                                             [[index[c] for c in piece] for job in pieces for piece in job]))
+        result = []
+        for job in pieces:
+            parts = [next(states) for _ in job]
+            if len(parts) > 1:
+                parts = [_hip.merge_states([p[0] for p in parts], [p[1] for p in parts], dst_dtype=torch.float32)]
+            result.append(parts[0])
+        return result
 
     def _execute(self, plan: CallPlan, query, key, value, merge_outs, merge_lses, segments=None) -> torch.Tensor:
         B, Sq, H, D = query.shape
         N, r = self.isp_size, self.local_chunk_id
         dev = query.device
         if self._exact_f32:
-            seen = {}
+            distinct = list(dict.fromkeys(job.chunks for job in plan.jobs))
+            seen = dict(zip(distinct, self._job_states_f32(query, distinct, key, value)))
             for job in plan.jobs:
-                if job.chunks not in seen:
-                    seen[job.chunks] = self._job_state_f32(query, job.chunks, key, value)
                 o, l = seen[job.chunks]
                 if job.store_slot is not None:
                     self.cache.store_block(job.store_slot, o, l)      # rounded to bf16 on its way into the cache
@@ -504,8 +513,8 @@ class proAttention:
                 raise RuntimeError(f"T{t}L{l}: mask asks to reuse chunk {c} but no state was ever stored for it")
             outs.append(cache.arena_out[c])
             lses.append(cache.arena_lse[c])
-        for c in compute:
-            o, s = self._job_state_f32(query, (c,), key if c == diag else None, value if c == diag else None)
+        states = self._job_states_f32(query, [(c,) for c in compute], key if diag == self.local_chunk_id else None, value)
+        for c, (o, s) in zip(compute, states):
             if c != diag and have_arena:
                 _hip.cache_store(o, s, cache.arena_out[c], cache.arena_lse[c])
                 cache.arena_valid[c] = True

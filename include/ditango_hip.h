@@ -90,20 +90,33 @@ int dt_attn_chunk_f16_fwd(const void* q, const void* k, const void* v, void* out
                           float softmax_scale, void* stream);
 
 /*
- * The same call site (core/attention.py:185-191) for fp32 tensors, computed in fp32 throughout (vector
- * ALU, expf / logf): the attention of the fp32 numbers themselves, not of their bf16 roundings.
+ * The same call site (core/attention.py:185-191) for fp32 tensors, computed in fp32 throughout (fp32 matrix
+ * instructions, fp32 exponentials): the attention of the fp32 numbers themselves, not of their bf16 roundings.
  * flash_attn_func takes no fp32; the
  * reference runs its CPU-runnable configuration (fp32, B=1, H=4, d=64, 512 queries x 4 chunks of
  * 512 keys) on its torch math path, and this entry point is that path's counterpart here.  q / k / v
  * fp32 with element strides and a contiguous last dimension; out fp32 [B,Sq,H,D] contiguous, lse
- * fp32 [B,H,Sq].  Sk = 0 yields out = 0, lse = -inf.  Not tuned (about 1 TFLOP/s): model-sized
- * bf16 work belongs on dt_attn_chunk_fwd.
+ * fp32 [B,H,Sq].  Sk = 0 yields out = 0, lse = -inf.
  */
 int dt_attn_chunk_f32_fwd(const float* q, const float* k, const float* v, float* out, float* lse,
                           int32_t B, int32_t Sq, int32_t Sk, int32_t H, int32_t D,
                           int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
                           int64_t kv_stride_b, int64_t kv_stride_s, int64_t kv_stride_h,
                           float softmax_scale, void* stream);
+
+/*
+ * Several fp32 states in one launch (core/attention.py:185-196): job j attends q to the concatenation of the
+ * chunks job_chunks[job_begin[j] .. job_begin[j+1]) and writes (out_ptrs[j], lse_ptrs[j]), fp32 throughout as
+ * above.  At most DT_MAX_CHUNKS chunks, DT_MAX_JOBS jobs and DT_MAX_JOB_ENTRIES chunk references; the tables
+ * are HOST arrays, with strides of their own for every chunk.
+ */
+int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
+                         int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                         int32_t n_chunks, const float* const* k_ptrs, const float* const* v_ptrs,
+                         const int32_t* kv_lens, const int64_t* kv_stride_b, const int64_t* kv_stride_s,
+                         const int64_t* kv_stride_h, int32_t n_jobs, const int32_t* job_begin,
+                         const int32_t* job_chunks, float* const* out_ptrs, float* const* lse_ptrs,
+                         float softmax_scale, void* stream);
 
 /*
  * Several attention states in one launch.  Job j attends q to the

@@ -95,6 +95,31 @@ def test_fp32_chunk_attention_matches_fp64_closed_form(hip, B, Sq, Sk, H, D):
         assert torch.equal(out2, out) and torch.equal(lse2, lse)
 
 
+@pytest.mark.parametrize("B,Sq,H,D,lens,jobs", [
+    (1, 97, 2, 64, [33, 1, 0, 128], [[0, 1], [2], [3, 2, 0], [1]]),   # tiles that end inside a chunk, an empty chunk, one key
+    (1, 32, 1, 128, [31, 32, 65], [[0, 1, 2], [2]]),
+    (2, 1024, 48, 64, [70], [[0]]),                                   # the form without a key split: 3072 query tiles
+    (1, 1025, 48, 128, [40, 33], [[0, 1], [1]]),
+])
+def test_fp32_jobs_match_fp64_closed_form(hip, B, Sq, H, D, lens, jobs):
+    """Several fp32 states of one launch, chunks with strides of their own (every second one a slice of a fused
+    projection).  Bound as above: 1e-5, fp32 rounding of sums over at most 256 keys."""
+    g = torch.Generator().manual_seed(Sq + D)
+    q = torch.randn(B, Sq, H, D, generator=g)
+    kv = [torch.randn(B, n, 2, H, D, generator=g) for n in lens]
+    dev = [t.cuda() if i % 2 else t.transpose(1, 2).contiguous().cuda().transpose(1, 2) for i, t in enumerate(kv)]
+    got = hip.attn_jobs_f32_fwd(q.cuda(), [t[:, :, 0] for t in dev], [t[:, :, 1] for t in dev], jobs)
+    torch.cuda.synchronize()
+    for job, (out, lse) in zip(jobs, got):
+        k, v = (torch.cat([kv[c][:, :, i] for c in job], 1) for i in (0, 1))
+        if k.shape[1] == 0:
+            assert (out == 0).all() and torch.isneginf(lse).all()
+            continue
+        ref_out, ref_lse = om.chunk_attention(q, k, v, compute_dtype=torch.float64)
+        assert (out.double().cpu() - ref_out).abs().max().item() <= 1e-5, job
+        assert (lse.double().cpu() - ref_lse).abs().max().item() <= 1e-5, job
+
+
 def test_chunk_attention_strided_inputs(hip):
     """q/k/v as slices of a fused [B,S,3,H,D] projection (non-contiguous token stride)."""
     B, S, H, D = 1, 300, 2, 128
