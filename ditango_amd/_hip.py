@@ -80,6 +80,14 @@ _SIGNATURES = {
                                                 c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                                 c_vp, c_vp, c_i32, c_vp, c_i64, c_vp, c_i64, c_i32, c_vp, c_vp,
                                                 c_i32, c_vp, _P(c_vp), c_i32, c_f32, c_i32, c_vp]),
+    "dt_attn_varlen_jobs_ws_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
+                                               c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
+                                               c_i32, _P(c_i32), _P(c_i32), _P(c_i32), c_i32, c_vp, _P(c_vp), c_i32,
+                                               _P(c_vp), _P(c_vp), c_f32, c_i32, c_vp, c_i64, c_vp]),
+    "dt_attn_sched_varlen_ws_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
+                                                c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
+                                                c_vp, c_vp, c_i32, c_vp, c_i64, c_vp, c_i64, c_i32, c_vp, c_vp,
+                                                c_i32, c_vp, _P(c_vp), c_i32, c_f32, c_i32, c_vp, c_i64, c_vp]),
     "dt_zero_rows_from": (ctypes.c_int, [c_vp, c_i64, c_i64, c_vp, c_vp]),
     "dt_merge_states": (ctypes.c_int, [c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i32), c_vp, c_i32, c_vp, c_i32,
                                        c_i32, c_i32, c_i32, c_i32, c_vp]),
@@ -270,12 +278,14 @@ def attn_workspace(device) -> torch.Tensor:
     different streams never share one.  At most ``MAX_WORKSPACES`` streams keep theirs: the least recently used
     entry is dropped (its memory goes back to the allocator in stream order, so launches still in flight on that
     stream are safe).  The first call on a stream allocates: make it before capturing that stream in a graph --
-    a workspace first created under capture would live in the graph's private pool -- or use the allocation-free
+    one created under capture lives in the graph's private pool and serves that launch only -- or use the allocation-free
     entry point (``attn_jobs_fwd(..., no_alloc=True)``)."""
     dev = torch.device(device)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (dev.type, index, torch.cuda.current_stream(index).cuda_stream)
     ws = _workspaces.pop(key, None)
+    if ws is None and torch.cuda.is_current_stream_capturing():
+        return torch.empty(int(load_library().dt_attn_workspace_bytes()), dtype=torch.uint8, device=dev)   # the graph's, not kept
     if ws is None:
         while len(_workspaces) >= MAX_WORKSPACES:
             _workspaces.pop(next(iter(_workspaces)))
@@ -287,6 +297,11 @@ def attn_workspace(device) -> torch.Tensor:
 def release_workspaces() -> None:
     """Drop every attention workspace (they are re-created on demand)."""
     _workspaces.clear()
+
+
+def _workspace_args(workspace: Optional[torch.Tensor]):
+    """The (pointer, bytes) pair of an optional workspace."""
+    return (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
 
 
 class ChunkTable:
@@ -469,12 +484,12 @@ def attn_jobs_fwd(q: torch.Tensor, table: ChunkTable, jobs: Sequence[Sequence[in
         if dev_segments is not None:
             seg_ids = (c_i32 * n)(*[int(job_segments[start + jj]) for jj in range(n)])
             cu_kv = dev_segments.kv_pointers(range(table.n) if local is None else ids)
-            rc = lib.dt_attn_varlen_jobs_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                             t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
-                                             n, begin, chunks, seg_ids, dev_segments.n_seg, dev_segments.cu_q.data_ptr(),
-                                             cu_kv, int(dev_segments.max_seqlen_q), out_ptrs, lse_ptrs,
-                                             float(softmax_scale), flags, _stream())
-            _check(rc, "dt_attn_varlen_jobs_fwd")
+            rc = lib.dt_attn_varlen_jobs_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
+                                                t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
+                                                n, begin, chunks, seg_ids, dev_segments.n_seg, dev_segments.cu_q.data_ptr(),
+                                                cu_kv, int(dev_segments.max_seqlen_q), out_ptrs, lse_ptrs,
+                                                float(softmax_scale), flags, *_workspace_args(workspace), _stream())
+            _check(rc, "dt_attn_varlen_jobs_ws_fwd")
         elif no_alloc:
             rc = lib.dt_attn_seg_jobs_noalloc_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
                                                   t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
@@ -485,10 +500,7 @@ def attn_jobs_fwd(q: torch.Tensor, table: ChunkTable, jobs: Sequence[Sequence[in
             rc = lib.dt_attn_seg_jobs_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
                                              t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
                                              n, begin, chunks, a_kvb, a_kvl, a_qb, a_ql, out_ptrs, lse_ptrs,
-                                             float(softmax_scale), flags,
-                                             workspace.data_ptr() if workspace is not None else None,
-                                             workspace.numel() * workspace.element_size() if workspace is not None else 0,
-                                             _stream())
+                                             float(softmax_scale), flags, *_workspace_args(workspace), _stream())
             _check(rc, "dt_attn_seg_jobs_ws_fwd")
         start = end
 
@@ -525,16 +537,16 @@ def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Te
         # segment boundaries in device memory: every scheduled chunk runs once per segment, the host reads nothing
         _require(seg_q is None and seg_kv is None, "device segment boundaries replace the host ranges")
         _require(len(dev_segments.cu_kv) == table.n, "one cu_seqlens_kv per chunk of the table")
-        rc = lib.dt_attn_sched_varlen_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                          table.n, table.k_ptrs, table.v_ptrs, table.lens, table.sb, table.ss, table.sh,
-                                          dev_compute_ids.data_ptr(), dev_count.data_ptr(), int(max_jobs),
-                                          slot_out.data_ptr(), slot_out.stride(0), slot_lse.data_ptr(), slot_lse.stride(0),
-                                          int(diag), diag_out.data_ptr() if diag_out is not None else None,
-                                          diag_lse.data_ptr() if diag_lse is not None else None,
-                                          dev_segments.n_seg, dev_segments.cu_q.data_ptr(),
-                                          dev_segments.kv_pointers(range(table.n)), dev_segments.max_seqlen_q,
-                                          float(softmax_scale), flags, _stream())
-        _check(rc, "dt_attn_sched_varlen_fwd")
+        rc = lib.dt_attn_sched_varlen_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
+                                             table.n, table.k_ptrs, table.v_ptrs, table.lens, table.sb, table.ss, table.sh,
+                                             dev_compute_ids.data_ptr(), dev_count.data_ptr(), int(max_jobs),
+                                             slot_out.data_ptr(), slot_out.stride(0), slot_lse.data_ptr(), slot_lse.stride(0),
+                                             int(diag), diag_out.data_ptr() if diag_out is not None else None,
+                                             diag_lse.data_ptr() if diag_lse is not None else None,
+                                             dev_segments.n_seg, dev_segments.cu_q.data_ptr(),
+                                             dev_segments.kv_pointers(range(table.n)), dev_segments.max_seqlen_q,
+                                             float(softmax_scale), flags, *_workspace_args(workspace), _stream())
+        _check(rc, "dt_attn_sched_varlen_ws_fwd")
         return
     n_seg, a_qb, a_ql, a_kb, a_kl = 0, None, None, None, None
     if seg_q is not None:
@@ -554,8 +566,7 @@ def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Te
                                    int(diag), diag_out.data_ptr() if diag_out is not None else None,
                                    diag_lse.data_ptr() if diag_lse is not None else None,
                                    n_seg, a_qb, a_ql, a_kb, a_kl, float(softmax_scale), flags,
-                                   workspace.data_ptr() if workspace is not None else None,
-                                   workspace.numel() * workspace.element_size() if workspace is not None else 0, _stream())
+                                   *_workspace_args(workspace), _stream())
     _check(rc, "dt_attn_sched_seg_ws_fwd")
 
 

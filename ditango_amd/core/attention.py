@@ -402,7 +402,8 @@ class proAttention:
             table = _hip.ChunkTable(ks, vs)
             if dev_seg is not None:
                 _hip.attn_jobs_fwd(query, table, job_lists, [d[0] for d in dests], [d[1] for d in dests],
-                                   q_prescaled=self.q_prescaled, dev_segments=dev_seg.over(needed), job_segments=job_segs)
+                                   workspace=_hip.attn_workspace(dev), q_prescaled=self.q_prescaled,
+                                   dev_segments=dev_seg.over(needed), job_segments=job_segs)
             else:
                 _hip.attn_jobs_fwd(query, table, job_lists, [d[0] for d in dests], [d[1] for d in dests],
                                    q_ranges=q_ranges, kv_ranges=kv_ranges, workspace=_hip.attn_workspace(dev),
@@ -547,8 +548,8 @@ class proAttention:
                     d_out.append(o)
                     d_lse.append(l_)
                     job_segs.append(i)
-            _hip.attn_jobs_fwd(query, _hip.ChunkTable(ks, vs), jobs, d_out, d_lse, q_prescaled=self.q_prescaled,
-                               dev_segments=src.over(range(len(ks))), job_segments=job_segs)
+            _hip.attn_jobs_fwd(query, _hip.ChunkTable(ks, vs), jobs, d_out, d_lse, workspace=_hip.attn_workspace(dev),
+                               q_prescaled=self.q_prescaled, dev_segments=src.over(range(len(ks))), job_segments=job_segs)
             out, lse = _hip.merge_states(outs, lses, dst_dtype=self.out_dtype, dst_lse_bsh=True)
             self.last_lse = lse
             return out

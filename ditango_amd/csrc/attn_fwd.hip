@@ -47,6 +47,7 @@
 //     through a contiguous range of heads: the workgroups that share an XCD's
 //     L2 stream the same K/V.
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <type_traits>
 
@@ -57,6 +58,7 @@ namespace dt {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // The 16-bit element type of q, K, V, P and the output states: bfloat16, or IEEE half (kHalf).  Loads, LDS
@@ -276,6 +278,76 @@ __device__ __forceinline__ void load_next_block_to_lds(u32x4 rsrc, uint32_t lane
                : "memory");
 }
 
+// Segment boundaries are read through the constant address space, i.e. with scalar loads: the lists were
+// written before the launch and the address is uniform.  (As a vector load the compiler follows it with
+// vmcnt(0), which inside the loop would also wait for every tile load in flight.)
+typedef const int32_t __attribute__((address_space(4))) ConstI32;
+__device__ __forceinline__ int boundary(const int32_t* list, int i) { return ((ConstI32*)list)[i]; }
+
+// What launch job `job` is: its chunk references, its query rows, its destination.
+struct JobView {
+  int seg_begin, seg_end, single;   // chunk references [seg_begin, seg_end), or the one chunk `single` >= 0
+  int q_begin, q_end;
+  int vseg;                         // segment of a packed variable-length batch (device-listed jobs only)
+  int dseg;                         // segment whose boundaries are read from device memory (a.cu_q != nullptr)
+  uint16_t* out;
+  float* lse;
+};
+template <typename Args>
+__device__ __forceinline__ bool view_job(Args& a, int job, JobView& v) {
+  v.single = -1;
+  v.q_begin = 0;
+  v.q_end = a.Sq;
+  v.vseg = -1;
+  v.dseg = -1;
+  if (a.dev_ids != nullptr) {
+    int slot = job;
+    if (a.n_seg > 0) {
+      const int r = job / a.n_slots;
+      slot = job - r * a.n_slots;
+      v.vseg = a.n_seg - 1 - r;
+    }
+    if (slot >= *a.dev_count) return false;
+    v.single = __builtin_amdgcn_readfirstlane(a.dev_ids[slot]);  // uniform by construction; tell the compiler
+    if (v.single < 0 || v.single >= a.n_chunks) return false;  // never index the tables with a bad id
+    v.seg_begin = 0;
+    v.seg_end = 1;
+    if (v.single == a.diag) {
+      v.out = a.diag_out;
+      v.lse = a.diag_lse;
+    } else {
+      v.out = a.slot_out + (int64_t)v.single * a.slot_out_stride;
+      v.lse = a.slot_lse + (int64_t)v.single * a.slot_lse_stride;
+    }
+    if (v.vseg >= 0) {
+      if (a.cu_q != nullptr) {
+        v.dseg = v.vseg;
+      } else {
+        v.q_begin = a.seg_q_begin[v.vseg];
+        v.q_end = v.q_begin + a.seg_q_len[v.vseg];
+      }
+    }
+  } else {
+    v.seg_begin = a.job_begin[job];
+    v.seg_end = a.job_begin[job + 1];
+    v.out = a.job_out[job];
+    v.lse = a.job_lse[job];
+    if (a.cu_q != nullptr) {
+      v.dseg = a.job_q_begin[job];
+    } else {
+      v.q_begin = a.job_q_begin[job];
+      v.q_end = v.q_begin + a.job_q_len[job];
+    }
+  }
+  if (v.dseg >= 0) {
+    // boundaries from device memory: nothing on the host has looked at them, so they are clamped
+    // to the rows that exist (a malformed list then yields wrong rows, never a stray access)
+    v.q_begin = min(max(boundary(a.cu_q, v.dseg), 0), a.Sq);
+    v.q_end = min(max(boundary(a.cu_q, v.dseg + 1), v.q_begin), a.Sq);
+  }
+  return true;
+}
+
 // Wavefronts per SIMD the register budget is set for.  D = 128: two (one workgroup per CU: its LDS
 // tiles fill the CU).  D = 64: four, i.e. TWO workgroups per CU (64 KB of LDS and at most 128
 // registers each): the second workgroup's wavefronts issue into the barrier waits, the start-up and
@@ -304,18 +376,19 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   int job = blockIdx.y;
   const int xcd = blockIdx.x & (kXcds - 1);
   int idx = blockIdx.x >> 3;
-  int part = 0;          // which of the part_ways key-tile ranges of a tail item
-  bool is_part = false;  // this workgroup computes one part of a tail item
-  if (job >= a.n_jobs) {
-    // planes behind the jobs hold the parts of the tail items, in dispatch order
-    const int pi = (job - a.n_jobs) * (int)(gridDim.x >> 3) + idx;
+  int part = 0, unit = 0;  // which of the part_ways key-tile ranges of which split item (counted per XCD)
+  bool is_part = false;    // this workgroup computes one part of a split item
+  if (job >= a.job_planes) {
+    // planes behind the jobs hold the parts of the split items, in dispatch order
+    const int pi = (job - a.job_planes) * (int)(gridDim.x >> 3) + idx;
     if (pi >= a.tail_items * a.part_ways) return;
-    job = a.tail_job;
-    const int u = pi / a.part_ways;
-    part = pi - u * a.part_ways;
-    idx = a.tail_idx0 + u;
+    unit = pi / a.part_ways;
+    part = pi - unit * a.part_ways;
+    const int flat = a.tail_start + unit;
+    job = flat / a.per_xcd;
+    idx = flat - job * a.per_xcd;
     is_part = true;
-  } else if (job == a.tail_job && idx >= a.tail_idx0) {
+  } else if ((int64_t)job * a.per_xcd + idx >= a.tail_start) {
     return;  // runs as parts
   }
   const int item = xcd * a.per_xcd + idx;
@@ -325,61 +398,10 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   const int b = bh / a.H;
   const int h = bh - b * a.H;
 
-  int seg_begin, seg_end, single = -1;
-  int q_begin = 0, q_end = a.Sq;   // query rows of this job
-  uint16_t* out_ptr;
-  float* lse_ptr;
-  int vseg = -1;  // segment of a packed variable-length batch (device-listed jobs only)
-  int dseg = -1;  // segment whose boundaries are read from device memory (a.cu_q != nullptr)
-  if (a.dev_ids != nullptr) {
-    int slot = job;
-    if (a.n_seg > 0) {
-      slot = job / a.n_seg;
-      vseg = job - slot * a.n_seg;
-    }
-    if (slot >= *a.dev_count) return;
-    single = __builtin_amdgcn_readfirstlane(a.dev_ids[slot]);  // uniform by construction; tell the compiler
-    if (single < 0 || single >= a.n_chunks) return;  // never index the tables with a bad id
-    seg_begin = 0;
-    seg_end = 1;
-    if (single == a.diag) {
-      out_ptr = a.diag_out;
-      lse_ptr = a.diag_lse;
-    } else {
-      out_ptr = a.slot_out + (int64_t)single * a.slot_out_stride;
-      lse_ptr = a.slot_lse + (int64_t)single * a.slot_lse_stride;
-    }
-    if (vseg >= 0) {
-      if (a.cu_q != nullptr) {
-        dseg = vseg;
-      } else {
-        q_begin = a.seg_q_begin[vseg];
-        q_end = q_begin + a.seg_q_len[vseg];
-      }
-    }
-  } else {
-    seg_begin = a.job_begin[job];
-    seg_end = a.job_begin[job + 1];
-    out_ptr = a.job_out[job];
-    lse_ptr = a.job_lse[job];
-    if (a.cu_q != nullptr) {
-      dseg = a.job_q_begin[job];
-    } else {
-      q_begin = a.job_q_begin[job];
-      q_end = q_begin + a.job_q_len[job];
-    }
-  }
-  // Segment boundaries are read through the constant address space, i.e. with scalar loads: the lists were
-  // written before the launch and the address is uniform.  (As a vector load the compiler follows it with
-  // vmcnt(0), which inside the loop would also wait for every tile load in flight.)
-  typedef const int32_t __attribute__((address_space(4))) ConstI32;
-  auto boundary = [](const int32_t* list, int i) __attribute__((always_inline)) -> int { return ((ConstI32*)list)[i]; };
-  if (dseg >= 0) {
-    // boundaries from device memory: nothing on the host has looked at them, so they are clamped
-    // to the rows that exist (a malformed list then yields wrong rows, never a stray access)
-    q_begin = min(max(boundary(a.cu_q, dseg), 0), a.Sq);
-    q_end = min(max(boundary(a.cu_q, dseg + 1), q_begin), a.Sq);
-  }
+  JobView view;
+  if (!view_job(a, job, view)) return;
+  const int seg_begin = view.seg_begin, seg_end = view.seg_end, single = view.single;
+  const int q_begin = view.q_begin, q_end = view.q_end, vseg = view.vseg, dseg = view.dseg;
   if (qt * kBQ >= q_end - q_begin) return;  // the grid is sized for the longest job / segment
   auto chunk_of = [&](int seg) __attribute__((always_inline)) -> int { return single >= 0 ? single : a.job_chunks[seg]; };
   // keys [begin, begin + len) of chunk reference `seg`
@@ -889,13 +911,23 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   const float lse = l_tot > 0.f ? (m_ref * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : -INFINITY;
   const int qrow = q0 + col;
-  // tail launch: the partial state goes to this workgroup's workspace slot, [256 queries][D] + [256]
-  const int64_t ws_slot = (((int64_t)(idx - a.tail_idx0) * kXcds + xcd) * a.part_ways + part);
   if (is_part) {
-    if (hh == 0) a.ws_lse[ws_slot * kBQ + wave * 32 + col] = lse;
-  } else if (hh == 0 && qrow < q_end) {
-    lse_ptr[((int64_t)b * a.H + h) * a.Sq + qrow] = lse;
+    // A part's state goes to the workspace as it lies in the registers, in fp32: whole kilobytes per store, no rounding.
+    const int64_t slot = ((int64_t)unit * kXcds + xcd) * a.part_ways + part;
+    if (hh == 0) a.ws_lse[slot * kBQ + wave * 32 + col] = lse;
+    float* dst = a.ws_out + (slot * kWaves + wave) * (32 * D) + lane * 4;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 val;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) val[e] = o_acc[db][4 * g + e] * inv;
+        *reinterpret_cast<f32x4*>(dst + (4 * db + g) * 256) = val;
+      }
+    return;
   }
+  if (hh == 0 && qrow < q_end) view.lse[((int64_t)b * a.H + h) * a.Sq + qrow] = lse;
 
   // O^T (registers, [d][query]) -> LDS [query][d] in the element type -> coalesced 16-byte stores.
   phase_barrier();  // every wavefront is done with the tile buffers
@@ -926,87 +958,110 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     const int row = p * kRowsPerPass + rr;
     const int qg = q0 + row;
     const u32x4 val = *reinterpret_cast<const u32x4*>(ol + row * T::kPitchO + cc * 16);
-    if (is_part) {
-      uint16_t* dst = a.ws_out + (ws_slot * kBQ + wave * 32 + row) * D + cc * 8;
-      *reinterpret_cast<u32x4*>(dst) = val;
-    } else if (qg < q_end) {
-      uint16_t* dst = out_ptr + (((int64_t)b * a.Sq + qg) * a.H + h) * D + cc * 8;
+    if (qg < q_end) {
+      uint16_t* dst = view.out + (((int64_t)b * a.Sq + qg) * a.H + h) * D + cc * 8;
       __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
     }
   }
 }
 
-// Folds the part_ways partial states of every tail item into the item's rows of its destination.
-// One workgroup per item and slice of 256 / (D/8) rows; a group of D/8 lanes owns a row.
+// Folds the part_ways partial states of every split item into the item's rows of its destination.  A workgroup takes 64
+// columns of the 32 query rows of one wavefront of the item's workgroup: its four wavefronts share the 4-element groups
+// of a row, lane L of a group holds query L % 32 as in the attention kernel, and the rows go through the LDS so that
+// the stores are 128 contiguous bytes.  Latency-bound (a few hundred KB per CU): many small workgroups with the loads of
+// four parts in flight.
+constexpr int kFoldThreads = 256;
 template <int D, bool kHalf>
-__global__ __launch_bounds__(256) void attn_tail_fold_kernel(const AttnArgs a) {
-  using E = Elem<kHalf>;
-  constexpr int kSlices = kBQ / (256 / (D / 8));
-  const int slot_id = blockIdx.x / kSlices;
-  const int slice = blockIdx.x - slot_id * kSlices;
-  const int xcd = slot_id & (kXcds - 1);
-  const int u = slot_id >> 3;
-  const int idx = a.tail_idx0 + u;
-  const int item = xcd * a.per_xcd + idx;
-  if (idx >= a.per_xcd || item >= a.total) return;
+__global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const AttnArgs args_by_value) {
+  typedef const AttnArgs __attribute__((address_space(4))) KernArgs;
+  KernArgs& a = *(KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  (void)args_by_value;
+  typedef typename Elem<kHalf>::x2 ex2;
+  typedef typename Elem<kHalf>::x4 ex4;
+  constexpr int kHalves = D / 64;
+  constexpr int kMine = 8 / (kFoldThreads / 64);       // 4-element groups of a lane
+  constexpr int kPitch = 64 * 2 + 16;
+  constexpr int kInFlight = 4;
+  __shared__ __attribute__((aligned(16))) uint8_t rows[32 * kPitch];
+  const int xcd = blockIdx.x & (kXcds - 1);   // the XCD the parts ran on: what is left of them in its L2 is read from there
+  const int half = (blockIdx.x >> 3) % kHalves;
+  const int rest = (blockIdx.x >> 3) / kHalves;
+  const int slice = rest & (kWaves - 1);
+  const int unit = rest >> 3;
+  const int flat = a.tail_start + unit;
+  const int job = flat / a.per_xcd;
+  const int item = xcd * a.per_xcd + flat - job * a.per_xcd;
+  if (item >= a.total) return;
   const int bh = item / a.nqt;
   const int qt = item - bh * a.nqt;
   const int b = bh / a.H;
   const int h = bh - b * a.H;
-  const int job = a.tail_job;
-  uint16_t* out_ptr;
-  float* lse_ptr;
-  if (a.dev_ids != nullptr) {
-    if (job >= *a.dev_count) return;
-    const int single = a.dev_ids[job];
-    if (single < 0 || single >= a.n_chunks) return;
-    out_ptr = single == a.diag ? a.diag_out : a.slot_out + (int64_t)single * a.slot_out_stride;
-    lse_ptr = single == a.diag ? a.diag_lse : a.slot_lse + (int64_t)single * a.slot_lse_stride;
-  } else {
-    out_ptr = a.job_out[job];
-    lse_ptr = a.job_lse[job];
-  }
-  constexpr int kLanes = D / 8;
-  constexpr int kRows = 256 / kLanes;
-  const int rr = threadIdx.x / kLanes;
-  const int cc = threadIdx.x % kLanes;
-  const int64_t slot0 = ((int64_t)u * kXcds + xcd) * a.part_ways;
-  {
-    const int row = slice * kRows + rr;
-    const int qg = qt * kBQ + row;
-    if (qg >= a.Sq) return;
-    float m = -INFINITY;
-    for (int p = 0; p < a.part_ways; ++p) m = fmaxf(m, a.ws_lse[(slot0 + p) * kBQ + row]);
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float den = 0.f;
-    if (m > -INFINITY) {
-      for (int p = 0; p < a.part_ways; ++p) {
-        const float w = __expf(a.ws_lse[(slot0 + p) * kBQ + row] - m);
-        const u32x4 v = *reinterpret_cast<const u32x4*>(a.ws_out + ((slot0 + p) * kBQ + row) * D + cc * 8);
-        const uint32_t e[4] = {v.x, v.y, v.z, v.w};
-        den += w;
+  JobView view;
+  if (!view_job(a, job, view)) return;
+  const int q0 = view.q_begin + qt * kBQ + slice * 32;
+  if (q0 >= view.q_end) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 31, hh = lane >> 5;
+  const int ways = a.part_ways;
+  const int64_t slot0 = ((int64_t)unit * kXcds + xcd) * ways;
+  const float* lses = a.ws_lse + slot0 * kBQ + slice * 32 + col;
+  const float* parts = a.ws_out + (slot0 * kWaves + slice) * (32 * D) + (8 * half + wave * kMine) * 256 + lane * 4;
+  float m = -INFINITY, den = 0.f;
+  f32x4 acc[kMine];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const f32x2 x = E::widen(e[k]);
-          acc[2 * k] = __builtin_fmaf(w, x.x, acc[2 * k]);
-          acc[2 * k + 1] = __builtin_fmaf(w, x.y, acc[2 * k + 1]);
-        }
-      }
-    }
-    const float inv = den > 0.f ? 1.f / den : 0.f;
-    u32x4 o;
-    uint32_t pk[4];
+  for (int g = 0; g < kMine; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < ways; p0 += kInFlight) {
+    float l[kInFlight];
+    f32x4 x[kInFlight][kMine];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      f32x2 f;
-      f.x = acc[2 * k] * inv;
-      f.y = acc[2 * k + 1] * inv;
-      pk[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, typename E::x2));
+    for (int i = 0; i < kInFlight; ++i) {
+      const int p = min(p0 + i, ways - 1);
+      l[i] = lses[p * kBQ];
+#pragma unroll
+      for (int g = 0; g < kMine; ++g) x[i][g] = *reinterpret_cast<const f32x4*>(parts + (int64_t)p * (kBQ * D) + g * 256);
     }
-    o.x = pk[0]; o.y = pk[1]; o.z = pk[2]; o.w = pk[3];
-    *reinterpret_cast<u32x4*>(out_ptr + (((int64_t)b * a.Sq + qg) * a.H + h) * D + cc * 8) = o;
-    if (cc == 0) lse_ptr[((int64_t)b * a.H + h) * a.Sq + qg] = den > 0.f ? m + __logf(den) : -INFINITY;
+    float m_new = m;
+#pragma unroll
+    for (int i = 0; i < kInFlight; ++i) {
+      if (p0 + i >= ways) l[i] = -INFINITY;
+      m_new = fmaxf(m_new, l[i]);
+    }
+    const float alpha = m > -INFINITY ? __expf(m - m_new) : 0.f;
+    m = m_new;
+    den *= alpha;
+#pragma unroll
+    for (int g = 0; g < kMine; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[g][e] *= alpha;
+#pragma unroll
+    for (int i = 0; i < kInFlight; ++i) {
+      const float w = l[i] > -INFINITY ? __expf(l[i] - m) : 0.f;
+      den += w;
+#pragma unroll
+      for (int g = 0; g < kMine; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[g][e] = __builtin_fmaf(w, x[i][g][e], acc[g][e]);
+    }
   }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+#pragma unroll
+  for (int g = 0; g < kMine; ++g) {
+    f32x2 lo, hi;
+    lo.x = acc[g][0] * inv; lo.y = acc[g][1] * inv;
+    hi.x = acc[g][2] * inv; hi.y = acc[g][3] * inv;
+    const ex2 l2 = __builtin_convertvector(lo, ex2);
+    const ex2 h2 = __builtin_convertvector(hi, ex2);
+    ex4 pk;
+    pk.x = l2.x; pk.y = l2.y; pk.z = h2.x; pk.w = h2.y;
+    *reinterpret_cast<ex4*>(rows + col * kPitch + (8 * (wave * kMine + g) + 4 * hh) * 2) = pk;
+  }
+  if (half == 0 && wave == 0 && hh == 0 && q0 + col < view.q_end)
+    view.lse[((int64_t)b * a.H + h) * a.Sq + q0 + col] = den > 0.f ? m + __logf(den) : -INFINITY;
+  __syncthreads();
+  const int row = threadIdx.x >> 3, cc = threadIdx.x & 7;
+  if (q0 + row < view.q_end)
+    __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(rows + row * kPitch + cc * 16),
+                                reinterpret_cast<u32x4*>(view.out + (((int64_t)b * a.Sq + q0 + row) * a.H + h) * D + 64 * half + cc * 8));
 }
 
 static_assert(Tile<128>::kLdsBytes == kAttnLdsBytes128 && Tile<64>::kLdsBytes == kAttnLdsBytes64,
@@ -1088,8 +1143,121 @@ int static_tail_scratch(void** ptr, int64_t* bytes) {
   return DT_OK;
 }
 
-int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, void* workspace,
-                int64_t workspace_bytes, bool balance) {
+// What the planner knows about a launch job: key tiles of one of its work items, query rows.
+struct JobSize {
+  int32_t tiles, rows;
+};
+
+// Puts host-listed jobs in the order that leaves the fewest idle CUs at the end: jobs with few query rows first (they
+// are gone in no time), then by falling length, so that the last work items to start are the shortest.
+static void order_jobs(AttnArgs& a, int n_jobs, JobSize* size) {
+  int order[DT_MAX_JOBS];
+  for (int j = 0; j < n_jobs; ++j) order[j] = j;
+  auto before = [&](int x, int y) {
+    return size[x].rows != size[y].rows ? size[x].rows < size[y].rows : size[x].tiles > size[y].tiles;
+  };
+  bool sorted = true;
+  for (int j = 1; j < n_jobs; ++j) sorted = sorted && !before(j, j - 1);
+  if (sorted) return;
+  std::stable_sort(order, order + n_jobs, before);
+  const AttnArgs o = a;
+  JobSize was[DT_MAX_JOBS];
+  std::copy(size, size + n_jobs, was);
+  int e = 0;
+  for (int j = 0; j < n_jobs; ++j) {
+    const int from = order[j];
+    size[j] = was[from];
+    a.job_out[j] = o.job_out[from];
+    a.job_lse[j] = o.job_lse[from];
+    a.job_q_begin[j] = o.job_q_begin[from];
+    a.job_q_len[j] = o.job_q_len[from];
+    a.job_begin[j] = e;
+    for (int x = o.job_begin[from]; x < o.job_begin[from + 1]; ++x, ++e) {
+      a.job_chunks[e] = o.job_chunks[x];
+      a.entry_kv_begin[e] = o.entry_kv_begin[x];
+      a.entry_kv_len[e] = o.entry_kv_len[x];
+    }
+  }
+  a.job_begin[n_jobs] = e;
+}
+
+// Sizes of the launch's jobs.  Device-listed jobs count as the longest chunk.  Where the boundaries are in device memory
+// a job counts with its whole chunks, and the query rows are taken to belong to the first segment (max_seqlen_q of them;
+// the model passes the valid tokens and, behind them, one padding segment).
+static void job_sizes(const AttnArgs& a, int n_jobs, JobSize* size) {
+  auto tiles_of = [](int keys) { return (keys + kBK - 1) / kBK; };
+  const int rows_first = std::min(a.nqt * kBQ, a.Sq), rows_other = std::max(0, std::min(rows_first, a.Sq - rows_first));
+  int longest = 0;
+  for (int c = 0; c < a.n_chunks; ++c) longest = std::max(longest, tiles_of(a.kv_len[c]));
+  for (int j = 0; j < n_jobs; ++j) {
+    const bool listed = a.dev_ids == nullptr;
+    int seg = listed ? a.job_q_begin[j] : a.n_seg > 0 ? a.n_seg - 1 - j / a.n_slots : -1;
+    size[j].tiles = 0;
+    if (!listed) size[j].tiles = longest;
+    else
+      for (int e = a.job_begin[j]; e < a.job_begin[j + 1]; ++e)
+        size[j].tiles += tiles_of(a.cu_q ? a.kv_len[a.job_chunks[e]] : a.entry_kv_len[e]);
+    if (a.cu_q) size[j].rows = seg == 0 ? rows_first : rows_other;
+    else if (listed) size[j].rows = a.job_q_len[j];
+    else size[j].rows = seg >= 0 ? a.seg_q_len[seg] : a.Sq;
+  }
+}
+
+// Which work items at the end of the launch run as how many parts each (tail_start, tail_items, part_ways).
+//
+// Time is counted in key tiles, on one XCD (workgroups go to the XCDs in turn, so each works through its own share of
+// every job).  Jobs come by falling length: the short ones behind fill the gaps that the long ones leave, so the
+// launch ends as if it consisted of items of the last job's length T only, in ceil(units / cus) rounds of them.  The
+// items of the last, partly filled round are cut into w parts each, which are handed to CUs as they come free: they take
+// ceil(rem * w / cus) rounds of (T / w + overhead) instead of one of T, plus the fold kernel.  A launch of less than one
+// round is split as a whole.
+// Measured on the HunyuanVideo, Step-Video and CogVideoX shares: a part costs about 6 tiles on top of its own (start-up,
+// epilogue, partial state) when all parts run at once and about 10 when they take several rounds, so many small parts
+// only pay in the first case; the fold kernel and the parts' stores cost about 4 (D = 128: 6, twice the bytes).
+// Launches of less than a round that used to run unsplit (us, before -> now): 1 head x 8000 queries x 8000 keys, D = 128
+// 140 -> 49; 3 heads x 2048 x 4096 77 -> 36; 10 heads x 1154 queries, two states over 1 and 2 chunks of 1154 keys 53 -> 45;
+// 4 heads x 5777 queries x 4 chunks of 5777 keys (368 work items, 23 per head) 270 -> 250.
+static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus, int64_t slots_cap) {
+  constexpr double kPartOverheadOneRound = 6.0, kPartOverheadRounds = 10.0;
+  const double fold_overhead = D == 128 ? 6.0 : 4.0;
+  const int last = size[n_jobs - 1].tiles, last_rows = size[n_jobs - 1].rows;
+  if (last < 1 || (int64_t)n_jobs * a.per_xcd >= INT32_MAX) return;
+  double units = 0;
+  int same = 0, longest = 0;   // jobs at the end that are like the last one
+  for (int j = 0; j < n_jobs; ++j) {
+    const double r = (double)size[j].tiles / last;
+    const int items = a.B * a.H * ((size[j].rows + kBQ - 1) / kBQ);
+    units += (double)((items + kXcds - 1) / kXcds) * (r < 0.75 ? r : std::floor(r + 0.5));
+    same = size[j].rows == last_rows && r > 0.9 && r < 1.1 ? same + 1 : 0;
+    longest = std::max(longest, size[j].tiles);
+  }
+  int rem, T;
+  if (n_jobs * a.per_xcd <= cus) {   // less than one round
+    rem = n_jobs * a.per_xcd;
+    T = longest;
+  } else {
+    // (with boundaries that only the device knows the last round may be full for all the host can tell)
+    rem = a.cu_q ? 0 : (int)std::ceil(units - 1e-9) % cus;
+    T = last;
+    if (rem > same * a.per_xcd) return;
+  }
+  if (rem <= 0 || T < 16) return;
+  double best = 0.1 * T;   // least gain worth the extra kernel
+  for (int w = 2; w <= 16; ++w) {
+    if ((int64_t)rem * kXcds * w > slots_cap || T / w < 6) break;
+    const int rounds = (rem * w + cus - 1) / cus;
+    const double part = (double)T / w, overhead = rounds == 1 ? kPartOverheadOneRound : kPartOverheadRounds;
+    const double gain = T - rounds * (part + overhead) - fold_overhead;
+    if (gain > best) {
+      best = gain;
+      a.tail_items = rem;
+      a.part_ways = w;
+    }
+  }
+  if (a.tail_items > 0) a.tail_start = n_jobs * a.per_xcd - a.tail_items;
+}
+
+int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
   if (n_jobs <= 0 || a_in.total <= 0) return DT_OK;
   if (D != 128 && D != 64) {
     set_error("head dim %d not built (64 and 128 are)", D);
@@ -1100,71 +1268,45 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
     return DT_ERR_UNSUPPORTED;
   }
   AttnArgs a = a_in;
-  a.n_jobs = n_jobs;
-  a.tail_job = -1;
-  a.tail_idx0 = 0;
+  a.job_planes = n_jobs;
+  a.tail_start = INT32_MAX;
   a.tail_items = 0;
   a.part_ways = 0;
-  const int slots_per_job = a.per_xcd * kXcds;
-  // ---- tail balancing: is the last round of workgroups worth splitting? -------------------
-  // Time is counted in key tiles.  Unsplit, the launch takes ceil(n / cus) rounds of one item
-  // (n_tiles tiles each).  With the last `rem` items cut into w parts, the parts are handed to
-  // CUs as they come free (same launch, no barrier in between), so the tail takes
-  // ceil(rem * w / cus) rounds of (n_tiles / w + kPartOverhead) tiles plus the fold kernel.
-  int tail = 0, ways = 0;
-  const int cus = balance && workspace ? cu_count() : 0;
-  const int64_t slot_bytes = (int64_t)kBQ * D * 2 + (int64_t)kBQ * 4;
-  if (cus >= 64 && cus % kXcds == 0 && a.total == slots_per_job) {
-    int n_tiles = 0;  // key tiles of one item of the last job (device-listed jobs: of the longest chunk)
-    if (a.dev_ids != nullptr) {
-      for (int c = 0; c < a.n_chunks; ++c) n_tiles = std::max(n_tiles, (a.kv_len[c] + kBK - 1) / kBK);
-    } else {
-      for (int e = a.job_begin[n_jobs - 1]; e < a.job_begin[n_jobs]; ++e) n_tiles += (a.entry_kv_len[e] + kBK - 1) / kBK;
-    }
-    // Measured on the HunyuanVideo, Step-Video and CogVideoX shares: a part costs about 6 tiles on
-    // top of its own (start-up, epilogue, partial state) when all parts run at once and about 10
-    // when they take several rounds, so many small parts only pay in the first case.
-    constexpr double kPartOverheadOneRound = 6.0, kPartOverheadRounds = 10.0;
-    constexpr double kFoldOverhead = 4.0;  // the fold kernel's launch
-    const int64_t n = (int64_t)n_jobs * slots_per_job;
-    const int rem = (int)(n % cus);
-    const int64_t cap = std::min<int64_t>(workspace_bytes / slot_bytes, kMaxTailSlots);
-    if (rem > 0 && rem <= slots_per_job && rem < n && n_tiles >= 16) {
-      double best = 0.1 * n_tiles;  // least gain worth the extra kernel
-      for (int w = 2; w <= 16; ++w) {
-        if ((int64_t)rem * w > cap || n_tiles / w < 6) break;
-        const int rounds = (int)(((int64_t)rem * w + cus - 1) / cus);
-        const double split = rounds * ((double)n_tiles / w + (rounds == 1 ? kPartOverheadOneRound : kPartOverheadRounds)) + kFoldOverhead;
-        if (n_tiles - split > best) {
-          best = n_tiles - split;
-          tail = rem;
-          ways = w;
-        }
-      }
-    }
+  constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
+  const int64_t slot_bytes = (int64_t)kBQ * D * 4 + (int64_t)kBQ * 4;
+  if (n_jobs <= kMaxLaunchJobs) {
+    JobSize size[kMaxLaunchJobs];
+    job_sizes(a, n_jobs, size);
+    if (a.dev_ids == nullptr) order_jobs(a, n_jobs, size);
+    const int cus = workspace ? cu_count() : 0;
+    if (cus >= 64 && cus % kXcds == 0)
+      plan_tail(a, D, n_jobs, size, cus / kXcds, std::min(workspace_bytes, kWorkspaceBytes) / slot_bytes);
   }
-  if (tail == 0) return launch_dim(a, D, dim3((unsigned)slots_per_job, (unsigned)n_jobs, 1), stream);
-  // (the planner only considers splits of at most `cap` slots, so this cannot fire; it guards later edits to it)
-  if ((int64_t)tail * ways * slot_bytes > workspace_bytes) {
-    set_error("internal: tail split of %d items x %d parts needs %lld bytes of scratch, %lld are there", tail, ways,
-              (long long)((int64_t)tail * ways * slot_bytes), (long long)workspace_bytes);
+  const unsigned planes_x = (unsigned)a.per_xcd * kXcds;
+  if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);
+  const int64_t slots = (int64_t)a.tail_items * kXcds * a.part_ways;
+  // (the planner only considers splits that fit, so this cannot fire; it guards later edits to it)
+  if (slots * slot_bytes > workspace_bytes) {
+    set_error("internal: tail split of %lld parts needs %lld bytes of scratch, %lld are there", (long long)slots,
+              (long long)(slots * slot_bytes), (long long)workspace_bytes);
     return DT_ERR_INVALID;
   }
-  a.tail_job = n_jobs - 1;
-  a.tail_idx0 = a.per_xcd - tail / kXcds;
-  a.tail_items = tail / kXcds;
-  a.part_ways = ways;
-  a.ws_out = static_cast<uint16_t*>(workspace);
-  a.ws_lse = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + (int64_t)tail * ways * kBQ * D * 2);
-  // parts per XCD lane of the grid: tail / 8 items x ways parts, spread over extra planes of per_xcd entries
-  const int part_planes = (a.tail_items * ways + a.per_xcd - 1) / a.per_xcd;
-  if (int rc = launch_dim(a, D, dim3((unsigned)slots_per_job, (unsigned)(n_jobs + part_planes), 1), stream)) return rc;
+  a.ws_out = static_cast<float*>(workspace);
+  a.ws_lse = a.ws_out + slots * kBQ * D;
+  if (a.tail_start <= 0) {   // every item is split: no job planes
+    a.tail_start = 0;
+    a.job_planes = 0;
+  }
+  // parts per XCD, spread over planes of per_xcd entries
+  const int part_planes = (a.tail_items * a.part_ways + a.per_xcd - 1) / a.per_xcd;
+  if (int rc = launch_dim(a, D, dim3(planes_x, (unsigned)(a.job_planes + part_planes), 1), stream)) return rc;
+  const dim3 fold_grid((unsigned)a.tail_items * kXcds * kWaves * (D / 64)), fold_block(kFoldThreads);
   if (D == 128) {
-    if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<128, true>), dim3((unsigned)tail * 16), dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((attn_tail_fold_kernel<128, false>), dim3((unsigned)tail * 16), dim3(256), 0, stream, a);
+    if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<128, true>), fold_grid, fold_block, 0, stream, a);
+    else hipLaunchKernelGGL((attn_tail_fold_kernel<128, false>), fold_grid, fold_block, 0, stream, a);
   } else {
-    if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<64, true>), dim3((unsigned)tail * 8), dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((attn_tail_fold_kernel<64, false>), dim3((unsigned)tail * 8), dim3(256), 0, stream, a);
+    if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<64, true>), fold_grid, fold_block, 0, stream, a);
+    else hipLaunchKernelGGL((attn_tail_fold_kernel<64, false>), fold_grid, fold_block, 0, stream, a);
   }
   return hip_fail(hipGetLastError(), "attn tail fold launch");
 }

@@ -98,7 +98,7 @@ static int fill_common(AttnArgs& a, const void* q, int32_t B, int32_t Sq, int32_
   return DT_OK;
 }
 
-extern "C" int64_t dt_attn_workspace_bytes(void) { return kMaxTailSlots * (256 * 128 * 2 + 256 * 4); }
+extern "C" int64_t dt_attn_workspace_bytes(void) { return kWorkspaceBytes; }
 
 static int check_workspace(const void* workspace, int64_t workspace_bytes) {
   if (workspace && (!aligned16(workspace) || workspace_bytes < 0)) {
@@ -194,8 +194,7 @@ extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int
   a.nqt = (longest + 255) / 256;
   a.total = B * H * a.nqt;
   a.per_xcd = (a.total + 7) / 8;
-  // the tail of the launch is only split when every job covers all query rows
-  return launch_attn(a, D, n_jobs, (hipStream_t)stream, workspace, workspace_bytes, job_q_begin == nullptr);
+  return launch_attn(a, D, n_jobs, (hipStream_t)stream, workspace, workspace_bytes);
 }
 
 // Device-resident segment boundaries: shared checks of the two varlen entry points.
@@ -230,14 +229,16 @@ static int fill_device_segments(AttnArgs& a, int32_t n_chunks, const int32_t* kv
   return DT_OK;
 }
 
-extern "C" int dt_attn_varlen_jobs_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+extern "C" int dt_attn_varlen_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
                                        int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
                                        const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
                                        int64_t kv_ss, int64_t kv_sh, int32_t n_jobs, const int32_t* job_begin,
                                        const int32_t* job_chunks, const int32_t* job_segment, int32_t n_seg,
                                        const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv,
                                        int32_t max_seqlen_q, void* const* out_ptrs, float* const* lse_ptrs,
-                                       float softmax_scale, int32_t flags, void* stream) {
+                                       float softmax_scale, int32_t flags, void* workspace, int64_t workspace_bytes,
+                                       void* stream) {
+  if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
   AttnArgs a{};
   if (int rc = fill_common(a, q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh,
                            softmax_scale))
@@ -282,7 +283,20 @@ extern "C" int dt_attn_varlen_jobs_fwd(const void* q, int32_t B, int32_t Sq, int
     }
     a.job_chunks[e] = c;
   }
-  return launch_attn(a, D, n_jobs, (hipStream_t)stream, nullptr, 0, false);
+  return launch_attn(a, D, n_jobs, (hipStream_t)stream, workspace, workspace_bytes);
+}
+
+extern "C" int dt_attn_varlen_jobs_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+                                       int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
+                                       const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
+                                       int64_t kv_ss, int64_t kv_sh, int32_t n_jobs, const int32_t* job_begin,
+                                       const int32_t* job_chunks, const int32_t* job_segment, int32_t n_seg,
+                                       const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv,
+                                       int32_t max_seqlen_q, void* const* out_ptrs, float* const* lse_ptrs,
+                                       float softmax_scale, int32_t flags, void* stream) {
+  return dt_attn_varlen_jobs_ws_fwd(q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh,
+                                    n_jobs, job_begin, job_chunks, job_segment, n_seg, cu_seqlens_q, cu_seqlens_kv,
+                                    max_seqlen_q, out_ptrs, lse_ptrs, softmax_scale, flags, nullptr, 0, stream);
 }
 
 // The same launch for callers that cannot allocate: the tail is split inside the library's own
@@ -457,16 +471,17 @@ extern "C" int dt_attn_sched_seg_ws_fwd(const void* q, int32_t B, int32_t Sq, in
         a.entry_kv_len[e] = kl;
       }
     a.n_seg = n_seg;
+    a.n_slots = max_jobs;
     // size the grid for the longest segment; shorter ones leave their surplus workgroups at once
     a.nqt = (longest + 255) / 256;
     a.total = B * H * a.nqt;
     a.per_xcd = (a.total + 7) / 8;
     jobs = max_jobs * n_seg;
   }
-  return launch_attn(a, D, jobs, (hipStream_t)stream, workspace, workspace_bytes, n_seg == 0);
+  return launch_attn(a, D, jobs, (hipStream_t)stream, workspace, workspace_bytes);
 }
 
-extern "C" int dt_attn_sched_varlen_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+extern "C" int dt_attn_sched_varlen_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
                                         int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
                                         const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
                                         int64_t kv_ss, int64_t kv_sh, const int32_t* dev_compute_ids,
@@ -474,7 +489,9 @@ extern "C" int dt_attn_sched_varlen_fwd(const void* q, int32_t B, int32_t Sq, in
                                         int64_t slot_out_stride, float* slot_lse, int64_t slot_lse_stride,
                                         int32_t diag, void* diag_out, float* diag_lse, int32_t n_seg,
                                         const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv,
-                                        int32_t max_seqlen_q, float softmax_scale, int32_t flags, void* stream) {
+                                        int32_t max_seqlen_q, float softmax_scale, int32_t flags, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+  if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
   AttnArgs a{};
   if (int rc = fill_common(a, q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh,
                            softmax_scale))
@@ -491,7 +508,23 @@ extern "C" int dt_attn_sched_varlen_fwd(const void* q, int32_t B, int32_t Sq, in
   if (int rc = fill_device_segments(a, n_chunks, kv_lens, n_seg, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q, B, Sq, H))
     return rc;
   a.n_seg = n_seg;
-  return launch_attn(a, D, max_jobs * n_seg, (hipStream_t)stream, nullptr, 0, false);
+  a.n_slots = max_jobs;
+  return launch_attn(a, D, max_jobs * n_seg, (hipStream_t)stream, workspace, workspace_bytes);
+}
+
+extern "C" int dt_attn_sched_varlen_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+                                        int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
+                                        const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
+                                        int64_t kv_ss, int64_t kv_sh, const int32_t* dev_compute_ids,
+                                        const int32_t* dev_count, int32_t max_jobs, void* slot_out,
+                                        int64_t slot_out_stride, float* slot_lse, int64_t slot_lse_stride,
+                                        int32_t diag, void* diag_out, float* diag_lse, int32_t n_seg,
+                                        const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv,
+                                        int32_t max_seqlen_q, float softmax_scale, int32_t flags, void* stream) {
+  return dt_attn_sched_varlen_ws_fwd(q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh,
+                                     dev_compute_ids, dev_count, max_jobs, slot_out, slot_out_stride, slot_lse,
+                                     slot_lse_stride, diag, diag_out, diag_lse, n_seg, cu_seqlens_q, cu_seqlens_kv,
+                                     max_seqlen_q, softmax_scale, flags, nullptr, 0, stream);
 }
 
 extern "C" int dt_attn_sched_seg_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,

@@ -63,19 +63,18 @@ struct AttnArgs {
   // segment in job_q_begin[job]; a device-listed job is segment job % n_seg as above.
   const int32_t* cu_q;
   const int32_t* cu_kv[DT_MAX_CHUNKS];
-  // Tail balancing (workspace launches only).  The workgroups of a launch are equal pieces of
-  // work, so its last round usually fills only part of the chip.  The main launch then leaves
-  // the work items with index >= tail_idx0 of job tail_job alone (tail_job < 0: nothing is left);
-  // extra grid planes behind the jobs run each of them as part_ways workgroups over disjoint
-  // ranges of key tiles that write partial states into the workspace (same launch, so a part
-  // starts as soon as a CU is free), and a small second kernel folds the parts into the
-  // destination.
-  int32_t n_jobs;      // grid planes (blockIdx.y) that are jobs; planes behind them hold tail parts
-  int32_t tail_job;
-  int32_t tail_idx0;
-  int32_t tail_items;  // tail items per XCD lane of the grid (= tail workgroup slots / 8)
+  // device-listed jobs come segment-major, the first segment last: launch job j is slot j % n_slots of the schedule
+  int32_t n_slots;
+  // Tail balancing (workspace launches only).  The work items of a launch, in dispatch order: those of an XCD are
+  // numbered flat = job * per_xcd + idx (idx: position in the XCD's share of the job).  Items with flat < tail_start run
+  // as one workgroup each; the tail_items behind them run as part_ways workgroups over disjoint ranges of key
+  // tiles, in grid planes of their own behind the job planes (same launch, so a part starts as soon as a CU is
+  // free).  The parts write fp32 partial states into the workspace and a small second kernel folds them into the destination.
+  int32_t job_planes;  // grid planes (blockIdx.y) that are jobs (0: every item is split); planes behind them hold parts
+  int32_t tail_start;  // INT32_MAX: nothing is split
+  int32_t tail_items;  // per XCD
   int32_t part_ways;
-  uint16_t* ws_out;   // [slot][256 queries][D]
+  float* ws_out;    // [slot][8 wavefronts][D / 8 groups of 4 elements][64 lanes][4], the accumulators as they lie in registers
   float* ws_lse;    // [slot][256]
 };
 
@@ -84,19 +83,19 @@ struct AttnArgs {
 constexpr int kAttnLdsBytes128 = 131072;
 constexpr int kAttnLdsBytes64 = 65536;
 
-// Workspace bytes the tail balancing can use at most (what dt_attn_workspace_bytes reports).
-constexpr int64_t kMaxTailSlots = 1536;
+// Workspace bytes the tail balancing can use at most (what dt_attn_workspace_bytes reports): 775 partial states of
+// 256 queries at D = 128, 1536 at D = 64.
+constexpr int64_t kWorkspaceBytes = 1536ll * (256 * 128 * 2 + 256 * 4);
 
-// The allocation-free entry point splits tails inside a device array of this many partial-state
-// slots (sized for D = 128: 256 queries x 128 bf16 + 256 lse values each).
-constexpr int64_t kStaticTailSlots = DT_NOALLOC_TAIL_SLOTS;
-constexpr int64_t kStaticTailBytes = kStaticTailSlots * (256 * 128 * 2 + 256 * 4);
+// The allocation-free entry point splits tails inside a device array of this many bytes (258 partial states at
+// D = 128, 512 at D = 64).
+constexpr int64_t kStaticTailBytes = (int64_t)DT_NOALLOC_TAIL_SLOTS * (256 * 128 * 2 + 256 * 4);
 // Device address and size of that array on the current device (looked up once per device).
 int static_tail_scratch(void** ptr, int64_t* bytes);
 
 static_assert(sizeof(AttnArgs) <= 4096, "the kernel arguments travel in the 4 KB kernarg segment");
 
 int launch_attn(const AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace = nullptr,
-                int64_t workspace_bytes = 0, bool balance = false);
+                int64_t workspace_bytes = 0);
 
 }  // namespace dt

@@ -222,7 +222,7 @@ int dt_attn_sched_seg_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32
  * dt_attn_varlen_jobs_fwd: job j is segment job_segment[j] (HOST array) of the state (out_ptrs[j],
  * lse_ptrs[j]) over its chunk list; the segments of one state are separate jobs with one destination.
  * dt_attn_sched_varlen_fwd: every scheduled chunk runs once per segment, as in dt_attn_sched_seg_fwd.
- * No tail balancing (the jobs cover row sub-ranges), hence no workspace.
+ * The _ws forms take a workspace for tail balancing as dt_attn_seg_jobs_ws_fwd does.
  */
 int dt_attn_varlen_jobs_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
                             int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
@@ -234,6 +234,17 @@ int dt_attn_varlen_jobs_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int
                             const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv, int32_t max_seqlen_q,
                             void* const* out_ptrs, float* const* lse_ptrs,
                             float softmax_scale, int32_t flags, void* stream);
+int dt_attn_varlen_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
+                            int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                            int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,
+                            const int32_t* kv_lens, const int64_t* kv_stride_b,
+                            int64_t kv_stride_s, int64_t kv_stride_h,
+                            int32_t n_jobs, const int32_t* job_begin, const int32_t* job_chunks,
+                            const int32_t* job_segment, int32_t n_seg,
+                            const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv, int32_t max_seqlen_q,
+                            void* const* out_ptrs, float* const* lse_ptrs,
+                            float softmax_scale, int32_t flags, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 int dt_attn_sched_varlen_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
                              int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
                              int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,
@@ -244,6 +255,17 @@ int dt_attn_sched_varlen_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, in
                              int32_t diag, void* diag_out, float* diag_lse,
                              int32_t n_seg, const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv,
                              int32_t max_seqlen_q, float softmax_scale, int32_t flags, void* stream);
+int dt_attn_sched_varlen_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
+                             int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                             int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,
+                             const int32_t* kv_lens, const int64_t* kv_stride_b,
+                             int64_t kv_stride_s, int64_t kv_stride_h,
+                             const int32_t* dev_compute_ids, const int32_t* dev_count, int32_t max_jobs,
+                             void* slot_out, int64_t slot_out_stride, float* slot_lse, int64_t slot_lse_stride,
+                             int32_t diag, void* diag_out, float* diag_lse,
+                             int32_t n_seg, const int32_t* cu_seqlens_q, const int32_t* const* cu_seqlens_kv,
+                             int32_t max_seqlen_q, float softmax_scale, int32_t flags, void* workspace,
+                             int64_t workspace_bytes, void* stream);
 
 /*
  * Zeroes the rows [*first_row, n_rows) of a dense [n_rows, row_bytes] tensor, first_row read from
@@ -258,10 +280,9 @@ int dt_zero_rows_from(void* dst, int64_t n_rows, int64_t row_bytes, const int32_
  * dt_attn_seg_jobs_fwd and dt_attn_sched_seg_fwd with a workspace (device memory, 16-byte aligned, at most
  * dt_attn_workspace_bytes() are used; NULL or too small: plain launch).  All workgroups of an
  * attention launch are equal pieces of work, so its last round usually fills only part of the
- * chip; with a workspace the work items of that round are each cut into several ranges of key
- * tiles that run side by side and write partial states into the workspace, and a small kernel
- * folds them into the destination -- 2 to 8 % off a launch.  Used only when every job covers all
- * query rows.  Calls that share a workspace must not overlap (same stream, or disjoint
+ * chip; with a workspace the work items of that round (all of them, in a launch of less than one
+ * round) are each cut into several ranges of key tiles that run side by side and write fp32 partial
+ * states into the workspace, and a small kernel folds them into the destination.  Calls that share a workspace must not overlap (same stream, or disjoint
  * workspaces).  No counterpart in the reference.
  *
  * flags: DT_ATTN_Q_PRESCALED says that the caller has folded softmax_scale * log2(e) into q before
@@ -269,7 +290,7 @@ int dt_zero_rows_from(void* dst, int64_t n_rows, int64_t row_bytes, const int32_
  * q k^T are then exponents of 2 as they stand, softmax_scale is ignored, and the softmax needs a
  * quarter fewer vector instructions (4 % faster at D = 128, 10 % at D = 64).  out and lse are those
  * of softmax(q k^T * ln 2).  The reference has no such mode (flash_attn_func scales inside).
- * DT_ATTN_FP16 says that q, k, v, the output states (and the partial states in the workspace) are IEEE
+ * DT_ATTN_FP16 says that q, k, v and the output states are IEEE
  * half instead of bfloat16, as in dt_attn_chunk_f16_fwd; it does not combine with DT_ATTN_Q_PRESCALED
  * (DT_ERR_UNSUPPORTED).
  */
@@ -304,7 +325,7 @@ int dt_attn_sched_seg_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, in
  * dt_attn_seg_jobs_ws_fwd for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc): no workspace argument, the tail of the
  * launch is split inside a device array that is part of the library (DT_NOALLOC_TAIL_SLOTS partial
- * states of 256 queries x 128 bf16 + 256 lse values = 34 078 720 bytes, held by every GPU the
+ * states of 256 queries x 64 fp32 + 256 lse values = 34 078 720 bytes, half as many at D = 128; held by every GPU the
  * library runs on until the process ends).  No counterpart in the reference.  Arguments, limits,
  * errors and results are those of dt_attn_seg_jobs_ws_fwd called with a workspace of exactly that
  * size: the split is planned to fit the array (a tail that would need more parts gets fewer), so the

@@ -204,6 +204,69 @@ def test_tail_balancing_matches_plain_launch_and_oracle(hip, D, H, nq, lens, job
         _check(bo[j][:, rows.cuda()], bl[j][:, :, rows.cuda()], ref_out, ref_lse, f"balanced job {j}")
 
 
+@pytest.mark.parametrize("D,H,Sq,lens,jobs,dtype", [
+    (128, 3, 700, [2100, 40], [[0]], torch.bfloat16),                  # 9 items: the whole launch is split, per_xcd = 2
+    (64, 1, 300, [2305], [[0]], torch.float16),                        # 2 items on 2 of 8 XCDs, one key in the last tile
+    (128, 5, 513, [1030, 1500, 64], [[2], [0, 1, 2]], torch.bfloat16), # jobs of 1 and 41 tiles: reordered, the short one's parts mostly empty
+    (64, 7, 1030, [2100, 2090], [[0], [1]], torch.bfloat16),           # 35 items a job: not a multiple of 8
+    (128, 37, 1900, [3000, 3000], [[0, 1], [1]], torch.bfloat16),      # 2 x 296 items, the shorter job's tail of a launch of several rounds
+])
+def test_split_launches_match_plain_launch_and_oracle(hip, D, H, Sq, lens, jobs, dtype):
+    """Launches of less than one round are split as a whole, jobs run longest first: every row of every state
+    against the launch without a workspace.  P is rounded relative to another running maximum in a part, so a row differs
+    by up to one rounding of P (2^-8 in bf16, weights summing to 1) and one of the output: 2^-7 of the largest value."""
+    g = torch.Generator().manual_seed(D + Sq)
+    q = torch.randn(1, Sq, H, D, generator=g).to(dtype)
+    ks = [torch.randn(1, n, H, D, generator=g).to(dtype) for n in lens]
+    vs = [torch.randn(1, n, H, D, generator=g).to(dtype) for n in lens]
+    table = hip.ChunkTable([k.cuda() for k in ks], [v.cuda() for v in vs])
+    res = []
+    for ws in (None, hip.attn_workspace("cuda")):
+        outs = [torch.full((1, Sq, H, D), float("nan"), dtype=dtype, device="cuda") for _ in jobs]
+        lses = [torch.full((1, H, Sq), float("nan"), device="cuda") for _ in jobs]
+        hip.attn_jobs_fwd(q.cuda(), table, jobs, outs, lses, workspace=ws)
+        torch.cuda.synchronize()
+        res.append((outs, lses))
+    assert any(not torch.equal(a, b) for a, b in zip(res[0][0], res[1][0])), "the launch was expected to be split"
+    rows = torch.cat([torch.arange(0, 40), torch.arange(Sq - 40, Sq)])
+    for j, chunks in enumerate(jobs):
+        po, bo, bl = res[0][0][j].float(), res[1][0][j].float(), res[1][1][j]
+        assert torch.isfinite(bo).all()
+        assert (po - bo).abs().max() <= 2.0 ** -7 * po.abs().max()
+        assert (res[0][1][j] - bl).abs().max() <= 1e-5
+        ref_out, ref_lse = om.full_attention(q[:, rows].float(), [ks[c].float() for c in chunks], [vs[c].float() for c in chunks])
+        _check(bo[:, rows.cuda()], bl[:, :, rows.cuda()], ref_out, ref_lse, f"split job {j}")
+
+
+@pytest.mark.parametrize("sched", [False, True])
+def test_split_varlen_launches_match_plain_launch(hip, sched):
+    """Device-resident boundaries with a workspace: the parts read them as the whole items do.  Bound as above."""
+    H, D, Sq, Sk = 2, 128, 700, 1500
+    g = torch.Generator(device="cuda").manual_seed(4)
+    q = torch.randn(1, Sq, H, D, generator=g, device="cuda").bfloat16()
+    ks, vs = ([torch.randn(1, Sk, H, D, generator=g, device="cuda").bfloat16() for _ in range(2)] for _ in range(2))
+    table = hip.ChunkTable(ks, vs)
+    cu_q, cu_kv = (torch.tensor(x, dtype=torch.int32, device="cuda") for x in ([0, 611, 690], [0, 1401, 1490]))
+    seg = hip.DeviceSegments(cu_q, [cu_kv, cu_kv], Sq)
+    res = []
+    for ws in (None, hip.attn_workspace("cuda")):
+        outs = torch.zeros(2, 1, Sq, H, D, dtype=torch.bfloat16, device="cuda")
+        lses = torch.zeros(2, 1, H, Sq, device="cuda")
+        if sched:
+            ids = torch.tensor([1, 0], dtype=torch.int32, device="cuda")
+            cnt = torch.tensor([2], dtype=torch.int32, device="cuda")
+            hip.attn_sched_fwd(q, table, ids, cnt, 2, outs, lses, -1, None, None, workspace=ws, dev_segments=seg)
+        else:
+            hip.attn_jobs_fwd(q, table, [[0], [0], [1], [1]], [outs[0], outs[0], outs[1], outs[1]],
+                              [lses[0], lses[0], lses[1], lses[1]], workspace=ws, dev_segments=seg, job_segments=[0, 1, 0, 1])
+        torch.cuda.synchronize()
+        res.append((outs.float(), lses))
+    assert not torch.equal(res[0][0], res[1][0]), "the launch was expected to be split"
+    assert (res[0][0] - res[1][0]).abs().max() <= 2.0 ** -7 * res[0][0].abs().max()
+    assert (res[0][1] - res[1][1]).abs().max() <= 1e-5
+    assert (res[1][0][:, :, 690:] == 0).all()            # rows behind the last boundary are nobody's
+
+
 def test_tail_balancing_in_the_device_scheduled_launch(hip):
     B, H, D, C = 1, 8, 128, 3
     Sq = 256 * 36
