@@ -137,8 +137,12 @@ def _check(rc: int, what: str) -> None:
         raise DitangoHipError(f"{what} failed with code {rc}: {msg}")
 
 
+_raw_stream = torch._C._cuda_getCurrentRawStream   # device index -> handle of its current stream, without building a Stream
+_current_device = torch._C._cuda_getDevice
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def _dtype_code(t: torch.Tensor) -> int:
@@ -280,9 +284,9 @@ def attn_workspace(device) -> torch.Tensor:
     stream are safe).  The first call on a stream allocates: make it before capturing that stream in a graph --
     one created under capture lives in the graph's private pool and serves that launch only -- or use the allocation-free
     entry point (``attn_jobs_fwd(..., no_alloc=True)``)."""
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
-    key = (dev.type, index, torch.cuda.current_stream(index).cuda_stream)
+    key = (dev.type, index, _raw_stream(index))
     ws = _workspaces.pop(key, None)
     if ws is None and torch.cuda.is_current_stream_capturing():
         return torch.empty(int(load_library().dt_attn_workspace_bytes()), dtype=torch.uint8, device=dev)   # the graph's, not kept
