@@ -1,12 +1,14 @@
-"""ctypes binding of ``libditango_hip.so`` (the C ABI declared in ``include/ditango_hip.h``).
+"""Binding of ``libditango_hip.so`` (the C ABI declared in ``include/ditango_hip.h``).
 
-There is no fallback: if the library has not been built, or an entry point
-returns an error code, the call raises.  PyTorch only supplies device memory
-(``tensor.data_ptr()``) and the stream (``torch.cuda.current_stream()``).
+The launches of a layer call go through ``_ditango_host`` (``csrc/host_binding.cpp``), an extension module that checks
+the tensors and fills the C ABI's argument tables; what runs once per generation goes through ctypes.  There is
+no fallback: if a library has not been built, or an entry point returns an error code, the call raises.  PyTorch
+only supplies device memory (``tensor.data_ptr()``) and the current stream.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 from pathlib import Path
 from typing import List, Optional, Sequence, Tuple
@@ -14,6 +16,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libditango_hip.so"
+HOST_PATH = LIB_PATH.parent / "_ditango_host.so"
 
 DT_BF16, DT_FP32, DT_FP16 = 0, 1, 2
 DT_LSE_BHS, DT_LSE_BSH = 0, 1
@@ -131,6 +134,23 @@ def load_library(path: Optional[os.PathLike] = None) -> ctypes.CDLL:
     return lib
 
 
+_host_module = None
+
+
+def _host():
+    """The extension module (loaded once; raises if it is absent)."""
+    global _host_module
+    if _host_module is None:
+        if not HOST_PATH.exists():
+            raise DitangoHipError(f"{HOST_PATH} is missing: build it with `python -m ditango_amd.build`")
+        spec = importlib.util.spec_from_file_location("_ditango_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        module.set_error_class(DitangoHipError)
+        _host_module = module
+    return _host_module
+
+
 def _check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load_library().dt_last_error().decode("utf-8", "replace")
@@ -182,20 +202,7 @@ def lse_layout_of(lse: torch.Tensor, B: int, S: int, H: int) -> int:
     """Classify an lse tensor as [B,H,S] or [B,S,H(,1)] storage; it must be dense in that order.  Where the
     shape alone cannot tell (S == H), a 4-D tensor is read as the running layout [B,S,H,1] of utils.py:49 and a
     3-D tensor as flash-attn's [B,H,S]."""
-    four_d = lse.dim() == 4 and lse.shape[-1] == 1
-    if four_d:
-        lse = lse.squeeze(-1)
-    _require(lse.dim() == 3 and lse.dtype == torch.float32, "lse must be fp32 with 3 (or 4, last=1) dims")
-    named = [((B, S, H), DT_LSE_BSH, DT_LSE_BHS), ((B, H, S), DT_LSE_BHS, DT_LSE_BSH)]
-    if not four_d:
-        named.reverse()
-    for shape, as_is, transposed in named:
-        if tuple(lse.shape) == shape:
-            if lse.is_contiguous():
-                return as_is
-            if lse.transpose(1, 2).is_contiguous():
-                return transposed
-    raise DitangoHipError(f"lse of shape {tuple(lse.shape)} / strides {lse.stride()} is not a dense [B,H,S] or [B,S,H]")
+    return _host().lse_layout(lse, B, S, H)
 
 
 # ---------------------------------------------------------------------------------------------
@@ -303,73 +310,27 @@ def release_workspaces() -> None:
     _workspaces.clear()
 
 
-def _workspace_args(workspace: Optional[torch.Tensor]):
-    """The (pointer, bytes) pair of an optional workspace."""
-    return (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
-
-
 class ChunkTable:
     """Host-side table of the KV chunks one layer call can touch (pointers, lengths, strides).  A table
     may hold more chunks than one launch can address (``DT_MAX_CHUNKS``); the job launches then pass the
-    sub-table of the chunks their jobs reference."""
+    sub-table of the chunks their jobs reference.  ``batch``: 3-D chunks are packed ``[batch * S, H, D]``;
+    ``convert`` is called on chunks that are neither bf16 nor fp16."""
 
-    def __init__(self, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor]):
-        n = len(k_chunks)
-        _require(n > 0 and n == len(v_chunks), "need at least one KV chunk and as many V as K chunks")
-        self.n = n
-        self.keep = (list(k_chunks), list(v_chunks))  # keep the tensors alive while pointers are in use
-        self._k: List[int] = []
-        self._v: List[int] = []
-        self._len: List[int] = []
-        self._sb: List[int] = []
-        ss = sh = None
-        self.dtype = k_chunks[0].dtype
-        for i, (k, v) in enumerate(zip(k_chunks, v_chunks)):
-            _check_qkv(k, f"k[{i}]", self.dtype); _check_qkv(v, f"v[{i}]", self.dtype)
-            _require(k.shape == v.shape and k.stride() == v.stride(), f"k[{i}] / v[{i}] mismatch")
-            if k.shape[1] > 0:
-                if ss is None:
-                    ss, sh = k.stride(1), k.stride(2)
-                    self.B, self.H, self.D = k.shape[0], k.shape[2], k.shape[3]
-                _require((k.stride(1), k.stride(2)) == (ss, sh), "all chunks must share token/head strides")
-                _require((k.shape[0], k.shape[2], k.shape[3]) == (self.B, self.H, self.D), "chunk B/H/D mismatch")
-            self._k.append(k.data_ptr())
-            self._v.append(v.data_ptr())
-            self._len.append(k.shape[1])
-            self._sb.append(k.stride(0))
-        _require(ss is not None, "all KV chunks are empty")
-        self.ss, self.sh = ss, sh
-        self._whole = self.arrays(range(n)) if n <= DT_MAX_CHUNKS else None
+    def __init__(self, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor], batch: int = 0, convert=None):
+        self.native = _host().ChunkTable(list(k_chunks), list(v_chunks), batch, convert)
 
-    def arrays(self, ids: Sequence[int]):
-        """ctypes arrays (k_ptrs, v_ptrs, lens, batch strides) of the chunks ``ids``, in that order."""
-        ids = list(ids)
-        m = len(ids)
-        _require(0 < m <= DT_MAX_CHUNKS, f"one launch addresses 1..{DT_MAX_CHUNKS} KV chunks, not {m}")
-        return ((c_vp * m)(*[self._k[i] for i in ids]), (c_vp * m)(*[self._v[i] for i in ids]),
-                (c_i32 * m)(*[self._len[i] for i in ids]), (c_i64 * m)(*[self._sb[i] for i in ids]))
+        t = self.native
+        self.n, self.B, self.H, self.D, self.ss, self.sh = t.n, t.B, t.H, t.D, t.ss, t.sh
 
     def whole(self):
-        """The arrays of all chunks (tables that fit one launch)."""
-        _require(self._whole is not None, f"the table holds {self.n} chunks, one launch addresses {DT_MAX_CHUNKS}")
-        return self._whole
+        """ctypes arrays (k_ptrs, v_ptrs, lens, batch strides) of the whole table, for callers of the C ABI."""
+        _require(self.n <= DT_MAX_CHUNKS, f"the table holds {self.n} chunks, one launch addresses {DT_MAX_CHUNKS}")
+        return tuple((ct * self.n)(*xs) for ct, xs in zip((c_vp, c_vp, c_i32, c_i64), self.native.arrays))
 
-    # the whole-table arrays under their old names
-    @property
-    def k_ptrs(self):
-        return self.whole()[0]
-
-    @property
-    def v_ptrs(self):
-        return self.whole()[1]
-
-    @property
-    def lens(self):
-        return self.whole()[2]
-
-    @property
-    def sb(self):
-        return self.whole()[3]
+    k_ptrs = property(lambda self: self.whole()[0])
+    v_ptrs = property(lambda self: self.whole()[1])
+    lens = property(lambda self: self.whole()[2])
+    sb = property(lambda self: self.whole()[3])
 
 
 class DeviceSegments:
@@ -379,20 +340,11 @@ class DeviceSegments:
     host-side upper bound of a segment's length that sizes the grid.  Nothing here reads device memory."""
 
     def __init__(self, cu_q: torch.Tensor, cu_kv: Sequence[Optional[torch.Tensor]], max_seqlen_q: int):
-        for name, t in [("cu_seqlens_q", cu_q)] + [(f"cu_seqlens_kv[{i}]", t) for i, t in enumerate(cu_kv) if t is not None]:
-            _require(torch.is_tensor(t) and t.is_cuda and t.dtype == torch.int32 and t.dim() == 1 and t.is_contiguous(),
-                     f"{name} must be a contiguous int32 vector on the GPU")
-            _require(t.numel() == cu_q.numel(), f"{name} must have as many entries as cu_seqlens_q")
-        _require(cu_q.numel() >= 2, "cu_seqlens_q needs at least two entries")
-        _require(int(max_seqlen_q) > 0, "max_seqlen_q must be positive")
         self.cu_q = cu_q
         self.cu_kv = list(cu_kv)
-        self.n_seg = cu_q.numel() - 1
         self.max_seqlen_q = int(max_seqlen_q)
-
-    def kv_pointers(self, ids: Sequence[int]):
-        ids = list(ids)
-        return (c_vp * len(ids))(*[self.cu_kv[i].data_ptr() if self.cu_kv[i] is not None else None for i in ids])
+        self.native = _host().Segments(cu_q, self.cu_kv, self.max_seqlen_q)
+        self.n_seg = self.native.n_seg
 
     def window(self, w0: int, w1: int) -> "DeviceSegments":
         return DeviceSegments(self.cu_q, self.cu_kv[w0:w1], self.max_seqlen_q)
@@ -420,93 +372,9 @@ def attn_jobs_fwd(q: torch.Tensor, table: ChunkTable, jobs: Sequence[Sequence[in
     ``dev_segments`` with ``job_segments``: the segment boundaries stay in device memory
     (``dt_attn_varlen_jobs_fwd``); job j is segment ``job_segments[j]`` of its state and the host reads none
     of the boundaries."""
-    lib = load_library()
-    _check_qkv(q, "q", table.dtype)
-    flags = _attn_flags(q, q_prescaled)
-    B, Sq, H, D = q.shape
-    _require((B, H, D) == (table.B, table.H, table.D), "q and KV chunks disagree on B/H/D")
-    _require(not (no_alloc and workspace is not None), "no_alloc launches take no workspace")
-    nj = len(jobs)
-    if dev_segments is not None:
-        _require(q_ranges is None and kv_ranges is None and not no_alloc, "device segment boundaries replace the host ranges")
-        _require(job_segments is not None and len(job_segments) == nj, "one segment index per job")
-        _require(len(dev_segments.cu_kv) == table.n, "one cu_seqlens_kv per chunk of the table")
-    _require(nj == len(outs) == len(lses), "one destination per job")
-    _require(q_ranges is None or len(q_ranges) == nj, "one query range per job")
-    _require(kv_ranges is None or len(kv_ranges) == nj, "one list of key ranges per job")
-    for j in range(nj):
-        o, l = outs[j], lses[j]
-        _require(o.dtype == q.dtype and o.is_contiguous() and tuple(o.shape) == (B, Sq, H, D), f"outs[{j}] must be contiguous [B,Sq,H,D] in q's dtype")
-        _require(l.dtype == torch.float32 and l.is_contiguous() and tuple(l.shape) == (B, H, Sq), f"lses[{j}] must be contiguous fp32 [B,H,Sq]")
-        _require(len(jobs[j]) <= DT_MAX_JOB_ENTRIES, f"job {j} references more than {DT_MAX_JOB_ENTRIES} chunks")
-    # split into launches that fit the per-launch limits (jobs, chunk references, distinct chunks)
-    start = 0
-    while start < nj:
-        end, entries = start, 0
-        used = set()
-        while end < nj and end - start < DT_MAX_JOBS and entries + len(jobs[end]) <= DT_MAX_JOB_ENTRIES:
-            more = used | {int(c) for c in jobs[end]}
-            if table.n > DT_MAX_CHUNKS and len(more) > DT_MAX_CHUNKS:
-                break
-            used = more
-            entries += len(jobs[end])
-            end += 1
-        _require(end > start, f"job {start} references more than {DT_MAX_CHUNKS} distinct chunks: split it and merge the parts")
-        n = end - start
-        if table.n <= DT_MAX_CHUNKS:
-            t_k, t_v, t_len, t_sb = table.whole()
-            t_n = table.n
-            local = None
-        else:
-            ids = sorted(used) or [0]
-            t_k, t_v, t_len, t_sb = table.arrays(ids)
-            t_n = len(ids)
-            local = {c: i for i, c in enumerate(ids)}
-        begin = (c_i32 * (n + 1))()
-        flat: List[int] = []
-        kvb: List[int] = []
-        kvl: List[int] = []
-        for jj in range(n):
-            j = start + jj
-            begin[jj] = len(flat)
-            for i, c in enumerate(jobs[j]):
-                c = int(c)
-                _require(0 <= c < table.n, f"job {j} references chunk {c} outside the table of {table.n}")
-                flat.append(c if local is None else local[c])
-                if kv_ranges is not None:
-                    kvb.append(int(kv_ranges[j][i][0]))
-                    kvl.append(int(kv_ranges[j][i][1]))
-        begin[n] = len(flat)
-        m = max(1, len(flat))
-        chunks = (c_i32 * m)(*flat)
-        a_kvb = (c_i32 * m)(*kvb) if kv_ranges is not None else None
-        a_kvl = (c_i32 * m)(*kvl) if kv_ranges is not None else None
-        a_qb = (c_i32 * n)(*[int(q_ranges[start + jj][0]) for jj in range(n)]) if q_ranges is not None else None
-        a_ql = (c_i32 * n)(*[int(q_ranges[start + jj][1]) for jj in range(n)]) if q_ranges is not None else None
-        out_ptrs = (c_vp * n)(*[outs[start + jj].data_ptr() for jj in range(n)])
-        lse_ptrs = (c_vp * n)(*[lses[start + jj].data_ptr() for jj in range(n)])
-        if dev_segments is not None:
-            seg_ids = (c_i32 * n)(*[int(job_segments[start + jj]) for jj in range(n)])
-            cu_kv = dev_segments.kv_pointers(range(table.n) if local is None else ids)
-            rc = lib.dt_attn_varlen_jobs_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                                t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
-                                                n, begin, chunks, seg_ids, dev_segments.n_seg, dev_segments.cu_q.data_ptr(),
-                                                cu_kv, int(dev_segments.max_seqlen_q), out_ptrs, lse_ptrs,
-                                                float(softmax_scale), flags, *_workspace_args(workspace), _stream())
-            _check(rc, "dt_attn_varlen_jobs_ws_fwd")
-        elif no_alloc:
-            rc = lib.dt_attn_seg_jobs_noalloc_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                                  t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
-                                                  n, begin, chunks, a_kvb, a_kvl, a_qb, a_ql, out_ptrs,
-                                                  lse_ptrs, float(softmax_scale), flags, _stream())
-            _check(rc, "dt_attn_seg_jobs_noalloc_fwd")
-        else:
-            rc = lib.dt_attn_seg_jobs_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                             t_n, t_k, t_v, t_len, t_sb, table.ss, table.sh,
-                                             n, begin, chunks, a_kvb, a_kvl, a_qb, a_ql, out_ptrs, lse_ptrs,
-                                             float(softmax_scale), flags, *_workspace_args(workspace), _stream())
-            _check(rc, "dt_attn_seg_jobs_ws_fwd")
-        start = end
+    _host().attn_jobs(q, table.native, jobs, outs, lses, softmax_scale, q_ranges, kv_ranges, workspace,
+                      _attn_flags(q, q_prescaled), no_alloc, None if dev_segments is None else dev_segments.native,
+                      job_segments, _stream())
 
 
 def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor,
@@ -515,87 +383,21 @@ def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Te
                    softmax_scale: float = 0.0, seg_q: Optional[Sequence[Tuple[int, int]]] = None,
                    seg_kv: Optional[Sequence[Sequence[Tuple[int, int]]]] = None,
                    workspace: Optional[torch.Tensor] = None, q_prescaled: bool = False,
-                   dev_segments: Optional[DeviceSegments] = None) -> None:
-    """Device-scheduled launch: chunk ids come from ``dev_compute_ids[:dev_count]`` in device memory and
+                   dev_segments: Optional[DeviceSegments] = None, row: int = 0) -> None:
+    """Device-scheduled launch: chunk ids come from ``dev_compute_ids[:dev_count]`` in device memory (of a whole
+    schedule, ``[..., C]`` and ``[..., 2]``: from its row ``row``) and
     each state lands in its slot of the arena (``slot_out [C,B,Sq,H,D]`` in q's dtype, ``slot_lse [C,B,H,Sq]`` fp32).
 
     On a packed variable-length batch, ``seg_q[s] = (begin, length)`` are the query rows of segment s and
     ``seg_kv[c][s] = (begin, length)`` its keys inside chunk c; every scheduled chunk then runs once per segment."""
-    lib = load_library()
-    _check_qkv(q, "q", table.dtype)
-    flags = _attn_flags(q, q_prescaled)
-    B, Sq, H, D = q.shape
-    _require((B, H, D) == (table.B, table.H, table.D), "q and KV chunks disagree on B/H/D")
-    _require(dev_compute_ids.dtype == torch.int32 and dev_count.dtype == torch.int32 and dev_compute_ids.is_cuda and dev_count.is_cuda,
-             "schedule tensors must be int32 on the GPU")
-    _require(dev_compute_ids.is_contiguous() and dev_compute_ids.numel() >= max_jobs, "compute id list shorter than max_jobs")
-    _require(slot_out.dtype == q.dtype and slot_out.is_contiguous() and tuple(slot_out.shape[1:]) == (B, Sq, H, D)
-             and slot_out.shape[0] >= table.n, "slot_out must be contiguous [C,B,Sq,H,D] in q's dtype")
-    _require(slot_lse.dtype == torch.float32 and slot_lse.is_contiguous() and tuple(slot_lse.shape[1:]) == (B, H, Sq)
-             and slot_lse.shape[0] >= table.n, "slot_lse must be contiguous fp32 [C,B,H,Sq]")
-    if 0 <= diag < table.n:
-        _require(diag_out is not None and diag_lse is not None, "a diag chunk needs (diag_out, diag_lse)")
-        _require(diag_out.dtype == q.dtype and diag_out.is_contiguous() and tuple(diag_out.shape) == (B, Sq, H, D), "diag_out must be contiguous [B,Sq,H,D] in q's dtype")
-        _require(diag_lse.dtype == torch.float32 and diag_lse.is_contiguous() and tuple(diag_lse.shape) == (B, H, Sq), "diag_lse must be contiguous fp32 [B,H,Sq]")
-    if dev_segments is not None:
-        # segment boundaries in device memory: every scheduled chunk runs once per segment, the host reads nothing
-        _require(seg_q is None and seg_kv is None, "device segment boundaries replace the host ranges")
-        _require(len(dev_segments.cu_kv) == table.n, "one cu_seqlens_kv per chunk of the table")
-        rc = lib.dt_attn_sched_varlen_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                             table.n, table.k_ptrs, table.v_ptrs, table.lens, table.sb, table.ss, table.sh,
-                                             dev_compute_ids.data_ptr(), dev_count.data_ptr(), int(max_jobs),
-                                             slot_out.data_ptr(), slot_out.stride(0), slot_lse.data_ptr(), slot_lse.stride(0),
-                                             int(diag), diag_out.data_ptr() if diag_out is not None else None,
-                                             diag_lse.data_ptr() if diag_lse is not None else None,
-                                             dev_segments.n_seg, dev_segments.cu_q.data_ptr(),
-                                             dev_segments.kv_pointers(range(table.n)), dev_segments.max_seqlen_q,
-                                             float(softmax_scale), flags, *_workspace_args(workspace), _stream())
-        _check(rc, "dt_attn_sched_varlen_ws_fwd")
-        return
-    n_seg, a_qb, a_ql, a_kb, a_kl = 0, None, None, None, None
-    if seg_q is not None:
-        n_seg = len(seg_q)
-        _require(seg_kv is not None and len(seg_kv) == table.n and all(len(r) == n_seg for r in seg_kv),
-                 "seg_kv needs one (begin, length) per chunk and segment")
-        _require(0 < n_seg <= DT_MAX_SEGMENTS and n_seg * table.n <= DT_MAX_JOB_ENTRIES,
-                 f"need 1..{DT_MAX_SEGMENTS} segments and at most {DT_MAX_JOB_ENTRIES} (chunk, segment) pairs")
-        a_qb = (c_i32 * n_seg)(*[int(b) for b, _ in seg_q])
-        a_ql = (c_i32 * n_seg)(*[int(n) for _, n in seg_q])
-        a_kb = (c_i32 * (n_seg * table.n))(*[int(b) for row in seg_kv for b, _ in row])
-        a_kl = (c_i32 * (n_seg * table.n))(*[int(n) for row in seg_kv for _, n in row])
-    rc = lib.dt_attn_sched_seg_ws_fwd(q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2),
-                                   table.n, table.k_ptrs, table.v_ptrs, table.lens, table.sb, table.ss, table.sh,
-                                   dev_compute_ids.data_ptr(), dev_count.data_ptr(), int(max_jobs),
-                                   slot_out.data_ptr(), slot_out.stride(0), slot_lse.data_ptr(), slot_lse.stride(0),
-                                   int(diag), diag_out.data_ptr() if diag_out is not None else None,
-                                   diag_lse.data_ptr() if diag_lse is not None else None,
-                                   n_seg, a_qb, a_ql, a_kb, a_kl, float(softmax_scale), flags,
-                                   *_workspace_args(workspace), _stream())
-    _check(rc, "dt_attn_sched_seg_ws_fwd")
+    _host().attn_sched(q, table.native, dev_compute_ids, dev_count, row, max_jobs, slot_out, slot_lse, diag, diag_out, diag_lse,
+                       softmax_scale, seg_q, seg_kv, workspace, _attn_flags(q, q_prescaled),
+                       None if dev_segments is None else dev_segments.native, _stream())
 
 
 # ---------------------------------------------------------------------------------------------
 # K2: merge, K3: cache store/load
 # ---------------------------------------------------------------------------------------------
-
-def _merge_once(outs, lses, dst_out, dst_lse, B, Sq, H, D) -> None:
-    lib = load_library()
-    n = len(outs)
-    out_ptrs = (c_vp * n)()
-    lse_ptrs = (c_vp * n)()
-    dts = (c_i32 * n)()
-    lays = (c_i32 * n)()
-    for i, (o, l) in enumerate(zip(outs, lses)):
-        _require(o.is_cuda and o.is_contiguous() and tuple(o.shape) == (B, Sq, H, D), f"outs[{i}] must be contiguous [B,Sq,H,D] on the GPU")
-        out_ptrs[i] = o.data_ptr()
-        lse_ptrs[i] = l.data_ptr()
-        dts[i] = _dtype_code(o)
-        lays[i] = lse_layout_of(l, B, Sq, H)
-    dlay = lse_layout_of(dst_lse, B, Sq, H)
-    rc = lib.dt_merge_states(n, out_ptrs, lse_ptrs, dts, lays, dst_out.data_ptr(), _dtype_code(dst_out),
-                             dst_lse.data_ptr(), dlay, B, Sq, H, D, _stream())
-    _check(rc, "dt_merge_states")
-
 
 def merge_states(outs: Sequence[torch.Tensor], lses: Sequence[torch.Tensor],
                  dst_out: Optional[torch.Tensor] = None, dst_lse: Optional[torch.Tensor] = None,
@@ -604,77 +406,28 @@ def merge_states(outs: Sequence[torch.Tensor], lses: Sequence[torch.Tensor],
     [B,H,Sq] or [B,Sq,H(,1)] storage.  Returns (dst_out, dst_lse).  Up to ``DT_MAX_MERGE`` states are one
     pass over HBM; more are folded in rounds through a running fp32 state that is updated in place (the
     merge is associative; the running state is never rounded below fp32)."""
-    n = len(outs)
-    _require(n > 0 and n == len(lses), "need at least one state and one lse per state")
-    B, Sq, H, D = outs[0].shape
-    dev = outs[0].device
-    if dst_out is None:
-        dst_out = torch.empty((B, Sq, H, D), dtype=dst_dtype, device=dev)
-    if dst_lse is None:
-        dst_lse = torch.empty((B, Sq, H, 1) if dst_lse_bsh else (B, H, Sq), dtype=torch.float32, device=dev)
-    _require(dst_out.is_contiguous() and tuple(dst_out.shape) == (B, Sq, H, D), "dst_out must be contiguous [B,Sq,H,D]")
-    outs, lses = list(outs), list(lses)
-    if n > DT_MAX_MERGE:
-        run_out = torch.empty((B, Sq, H, D), dtype=torch.float32, device=dev)
-        run_lse = torch.empty((B, H, Sq), dtype=torch.float32, device=dev)
-        _merge_once(outs[:DT_MAX_MERGE], lses[:DT_MAX_MERGE], run_out, run_lse, B, Sq, H, D)
-        i = DT_MAX_MERGE
-        while n - i > DT_MAX_MERGE - 1:
-            _merge_once([run_out] + outs[i:i + DT_MAX_MERGE - 1], [run_lse] + lses[i:i + DT_MAX_MERGE - 1],
-                        run_out, run_lse, B, Sq, H, D)
-            i += DT_MAX_MERGE - 1
-        outs, lses = [run_out] + outs[i:], [run_lse] + lses[i:]
-    _merge_once(outs, lses, dst_out, dst_lse, B, Sq, H, D)
-    return dst_out, dst_lse
+    return _host().merge(outs, lses, dst_out, dst_lse, dst_dtype, dst_lse_bsh, _stream())
+
+
+def merge_arena(arena_out: torch.Tensor, arena_lse: torch.Tensor, diag: int, diag_out: torch.Tensor, diag_lse: torch.Tensor,
+                dst_dtype: torch.dtype = torch.float32):
+    """Merge of every slot of an arena ``[C,B,Sq,H,D]`` / ``[C,B,H,Sq]``, slot ``diag`` replaced by
+    (diag_out, diag_lse).  Returns (out ``[B,Sq,H,D]``, lse ``[B,Sq,H,1]``)."""
+    return _host().merge_arena(arena_out, arena_lse, diag, diag_out, diag_lse, dst_dtype, _stream())
 
 
 def cache_store(src_out: torch.Tensor, src_lse: torch.Tensor, slot_out: torch.Tensor, slot_lse: torch.Tensor) -> None:
-    lib = load_library()
-    B, Sq, H, D = src_out.shape
-    _require(src_out.is_cuda and src_out.is_contiguous(), "src_out must be contiguous on the GPU")
-    _require(slot_out.dtype in HALF_DTYPES and slot_out.is_contiguous() and tuple(slot_out.shape) == (B, Sq, H, D), "slot_out must be contiguous bf16 or fp16 [B,Sq,H,D]")
-    _require(slot_lse.dtype == torch.float32 and slot_lse.is_contiguous() and tuple(slot_lse.shape) == (B, H, Sq), "slot_lse must be contiguous fp32 [B,H,Sq]")
-    if slot_out.dtype == torch.bfloat16:
-        rc = lib.dt_cache_store(src_out.data_ptr(), _dtype_code(src_out), src_lse.data_ptr(), lse_layout_of(src_lse, B, Sq, H),
-                                slot_out.data_ptr(), slot_lse.data_ptr(), B, Sq, H, D, _stream())
-    else:   # fp16 slots of a model that runs in fp16
-        rc = lib.dt_state_copy(src_out.data_ptr(), _dtype_code(src_out), src_lse.data_ptr(), lse_layout_of(src_lse, B, Sq, H),
-                               slot_out.data_ptr(), DT_FP16, slot_lse.data_ptr(), DT_LSE_BHS, B, Sq, H, D, _stream())
-    _check(rc, "dt_cache_store")
+    _host().cache_store(src_out, src_lse, slot_out, slot_lse, _stream())
 
 
 def cache_load(slot_out: torch.Tensor, slot_lse: torch.Tensor, dst_dtype: torch.dtype = torch.float32,
                dst_lse_bsh: bool = False, dst_out: Optional[torch.Tensor] = None, dst_lse: Optional[torch.Tensor] = None):
-    lib = load_library()
-    B, Sq, H, D = slot_out.shape
-    _require(slot_out.dtype in HALF_DTYPES and slot_out.is_contiguous(), "slot_out must be contiguous bf16 or fp16")
-    _require(slot_lse.dtype == torch.float32 and slot_lse.is_contiguous() and tuple(slot_lse.shape) == (B, H, Sq), "slot_lse must be contiguous fp32 [B,H,Sq]")
-    if dst_out is None:
-        dst_out = torch.empty((B, Sq, H, D), dtype=dst_dtype, device=slot_out.device)
-    if dst_lse is None:
-        dst_lse = torch.empty((B, Sq, H, 1) if dst_lse_bsh else (B, H, Sq), dtype=torch.float32, device=slot_out.device)
-    _require(dst_out.is_contiguous() and tuple(dst_out.shape) == (B, Sq, H, D), "dst_out must be contiguous [B,Sq,H,D]")
-    dst_lse_bsh = lse_layout_of(dst_lse, B, Sq, H) == DT_LSE_BSH
-    if slot_out.dtype == torch.bfloat16:
-        rc = lib.dt_cache_load(slot_out.data_ptr(), slot_lse.data_ptr(), dst_out.data_ptr(), _dtype_code(dst_out),
-                               dst_lse.data_ptr(), DT_LSE_BSH if dst_lse_bsh else DT_LSE_BHS, B, Sq, H, D, _stream())
-    else:
-        rc = lib.dt_state_copy(slot_out.data_ptr(), DT_FP16, slot_lse.data_ptr(), DT_LSE_BHS, dst_out.data_ptr(),
-                               _dtype_code(dst_out), dst_lse.data_ptr(), DT_LSE_BSH if dst_lse_bsh else DT_LSE_BHS,
-                               B, Sq, H, D, _stream())
-    _check(rc, "dt_cache_load")
-    return dst_out, dst_lse
+    return _host().cache_load(slot_out, slot_lse, dst_dtype, dst_lse_bsh, dst_out, dst_lse, _stream())
 
 
 def zero_rows_from(t: torch.Tensor, first_row: torch.Tensor) -> None:
     """Zero the rows ``[first_row[0], n)`` of ``t`` (contiguous, rows along dim 0), the index read on the device."""
-    lib = load_library()
-    _require(t.is_cuda and t.is_contiguous() and t.dim() >= 1, "t must be a contiguous device tensor")
-    _require(first_row.is_cuda and first_row.dtype == torch.int32 and first_row.numel() >= 1, "first_row must be int32 on the GPU")
-    n = t.shape[0]
-    row_bytes = (t.numel() // max(n, 1)) * t.element_size()
-    rc = lib.dt_zero_rows_from(t.data_ptr(), n, row_bytes, first_row.data_ptr(), _stream())
-    _check(rc, "dt_zero_rows_from")
+    _host().zero_rows_from(t, first_row, _stream())
 
 
 # ---------------------------------------------------------------------------------------------

@@ -2,7 +2,8 @@
 
 ``python -m ditango_amd.build`` compiles every translation unit under
 ``ditango_amd/csrc`` and links ``ditango_amd/lib/libditango_hip.so`` (the drop-in
-library) and ``ditango_amd/lib/libditango_probes.so`` (the benchmark's measurement
+library), ``ditango_amd/lib/_ditango_host.so`` (the Python extension module of ``csrc/host_binding.cpp``, host code
+only) and ``ditango_amd/lib/libditango_probes.so`` (the benchmark's measurement
 aids, a library of its own that only ``bench.py`` loads).  hipcc
 cross-compiles for gfx950 without a GPU.  Packed-FP32 instruction selection is
 switched off for all device code (``-target-feature -packed-fp32-ops``).
@@ -14,6 +15,7 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -22,6 +24,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB_DIR = PKG / "lib"
 LIB_PATH = LIB_DIR / "libditango_hip.so"
+HOST_PATH = LIB_DIR / "_ditango_host.so"             # Python extension: the host side of the launches (csrc/host_binding.cpp)
 PROBES_PATH = LIB_DIR / "libditango_probes.so"
 DEMO_PATH = LIB_DIR / "dt_capi_demo"
 RESOURCES_PATH = LIB_DIR / "kernel_resources.json"   # per-kernel registers / scratch / occupancy of the last build
@@ -75,8 +78,21 @@ def build_lib(verbose: bool = False, extra_flags=()) -> Path:
         resources[src] = parse_resource_remarks(_run(cmd).stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=6) as ex:
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    host_obj = LIB_DIR / "host_binding.o"
+    host_compile = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-DTORCH_EXTENSION_NAME=_ditango_host",
+                    f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{ROOT / 'include'}",
+                    f"-I{sysconfig.get_paths()['include']}", *(f"-I{d}" for d in include_paths()),
+                    "-c", str(CSRC / "host_binding.cpp"), "-o", str(host_obj)]
+    host_link = [host_compile[0], "-shared", str(host_obj), *(f"-L{d}" for d in library_paths()), "-ltorch", "-ltorch_cpu",
+                 "-lc10", "-ltorch_python", f"-L{LIB_DIR}", "-lditango_hip", "-Wl,-rpath,$ORIGIN", "-o", str(HOST_PATH)]
+    if verbose:
+        print(" ".join(host_compile), flush=True)
+    with ThreadPoolExecutor(max_workers=7) as ex:
+        host = ex.submit(_run, host_compile)
         all_objs = list(ex.map(compile_one, SOURCES + PROBE_SOURCES))
+        host.result()
     objs, probe_objs = all_objs[:len(SOURCES)], all_objs[len(SOURCES):]
     # a version script keeps everything but the C entry points out of the dynamic symbol table
     for out, members, exports in ((LIB_PATH, objs, "exports_hip.map"), (PROBES_PATH, probe_objs, "exports_probes.map")):
@@ -85,6 +101,9 @@ def build_lib(verbose: bool = False, extra_flags=()) -> Path:
         if verbose:
             print(" ".join(cmd), flush=True)
         _run(cmd)
+    if verbose:
+        print(" ".join(host_link), flush=True)
+    _run(host_link)
     RESOURCES_PATH.write_text(json.dumps(resources, indent=1, sort_keys=True) + "\n")
     # a host program that uses nothing but the C header and the HIP runtime (tests/test_capi_demo_gpu.py runs it)
     cmd = [HIPCC, "-O2", "-std=c++17", "-Wno-unused-result", f"-I{ROOT / 'include'}", str(CSRC / "capi_demo.cpp"),

@@ -28,6 +28,7 @@ contiguous per-layer arena.
 from __future__ import annotations
 
 from dataclasses import dataclass, field
+from functools import lru_cache
 from typing import List, Optional, Tuple
 
 import torch
@@ -43,7 +44,7 @@ from .redundancy_map import get_redundancy_map
 logger = init_logger(__name__)
 
 
-@dataclass
+@dataclass(frozen=True)
 class Job:
     chunks: Tuple[int, ...]   # KV chunk ids attended to as one concatenated sequence
     kind: str                 # 'local' (computed while the first fetch is in flight), 'own', 'fresh'
@@ -146,6 +147,19 @@ def plan_call(N: int, r: int, curr: int, nxt: int, targets: List[int], use_ditan
     return plan, targets
 
 
+@lru_cache(maxsize=256)
+def _planned(N: int, r: int, curr: int, nxt: int, targets: Tuple[int, ...], use_ditango: bool, small_ring_stride: int):
+    return plan_call(N, r, curr, nxt, list(targets), use_ditango, small_ring_stride)
+
+
+def _plan_of_call(N: int, r: int, curr: int, nxt: int, targets: List[int], use_ditango: bool, small_ring_stride: int):
+    """``plan_call`` looked up: a schedule visits few distinct integer states, the same ones in every layer."""
+    p, new_targets = _planned(N, r, curr, nxt, tuple(targets), use_ditango, small_ring_stride)
+    plan = CallPlan(0, 0, p.rank, p.curr_stride, p.next_stride, list(p.reuse_probed), [], list(p.computed), list(p.jobs),
+                    list(p.stores), list(p.flushes), p.target_after)
+    return plan, list(new_targets)
+
+
 _warned_cast = set()
 
 
@@ -240,7 +254,7 @@ class proAttention:
         if self._ring_targets[r] != self.target_chunk_id:  # the pointer was set from outside: same offset everywhere
             shift = (self.target_chunk_id - self._ring_targets[r]) % N
             self._ring_targets = [(tg + shift) % N for tg in self._ring_targets]
-        plan, new_targets = plan_call(N, r, curr, nxt, self._ring_targets, self.use_ditango, self.small_ring_stride)
+        plan, new_targets = _plan_of_call(N, r, curr, nxt, self._ring_targets, self.use_ditango, self.small_ring_stride)
         new_target = new_targets[r]
         plan.timestep, plan.layer_id = timestep, self.layer_id
 
@@ -351,8 +365,8 @@ class proAttention:
         for c in needed:
             index[c] = len(ks)
             k_c, v_c = (key, value) if c == r else self.group.kv_chunk(c)
-            ks.append(_as4d(k_c, B))
-            vs.append(_as4d(v_c, B))
+            ks.append(k_c)
+            vs.append(v_c)
         # one launch for all distinct states; a chunk computed twice by the reference
         # (local + own) is computed once and merged twice
         job_lists, dests, seen = [], [], {}
@@ -399,7 +413,7 @@ class proAttention:
             seen[job.chunks] = (o, l)
             states.append((o, l))
         if job_lists:
-            table = _hip.ChunkTable(ks, vs)
+            table = _hip.ChunkTable(ks, vs, B, _kernel_input)
             if dev_seg is not None:
                 _hip.attn_jobs_fwd(query, table, job_lists, [d[0] for d in dests], [d[1] for d in dests],
                                    workspace=_hip.attn_workspace(dev), q_prescaled=self.q_prescaled,
@@ -424,43 +438,42 @@ class proAttention:
     def _attn_masked(self, query, key, value) -> torch.Tensor:
         rm = get_redundancy_map()
         t, l = get_timestep(), self.layer_id
-        C = rm.chunk_mask.shape[2]
         diag = rm.mask_diag
         B, Sq, H, D = query.shape
         cache = self.cache
-        row = rm.chunk_mask[t, l]
-        ks, vs = [], []
-        for c in range(C):
-            use_local = (c == self.local_chunk_id and c == diag and key is not None)
-            k_c, v_c = (key, value) if use_local else self.group.kv_chunk(c)
-            ks.append(_as4d(k_c, B))
-            vs.append(_as4d(v_c, B))
+        row = rm.mask_rows[t][l]
+        C = len(row)
+        local = self.local_chunk_id if (self.local_chunk_id == diag and key is not None) else -1
+        kv = [(key, value) if c == local else self.group.kv_chunk(c) for c in range(C)]
+        ks, vs = [k for k, _ in kv], [v for _, v in kv]
         if not cache.ensure_arena(C, B, Sq, H, D, query.device, query.dtype):
-            out = self._attn_uncached(query, ks, vs)
+            out = self._attn_uncached(query, [_as4d(k, B) for k in ks], [_as4d(v, B) for v in vs])
             rm.record_out_redundancy(timestep=t, layer_id=l, curr_out=out)
             return out
+        valid = cache.arena_valid
         for c in range(C):
-            if c != diag and row[c] != 0 and not cache.arena_valid[c]:
+            if row[c] != 0 and c != diag and not valid[c]:
                 raise RuntimeError(f"T{t}L{l}: mask asks to reuse chunk {c} but no state was ever stored for it")
         seg_q = seg_kv = dev_seg = None
-        if isinstance(self._segments, _DeviceSegmentSource):
-            dev_seg = self._segments.over(range(C))
-        elif self._segments is not None:
-            # packed variable-length batch: every scheduled chunk runs once per segment
-            cu_q, cu_kv_of = self._segments
-            seg_q = [(cu_q[i], cu_q[i + 1] - cu_q[i]) for i in range(len(cu_q) - 1)]
-            seg_kv = [[(cu_kv_of(c)[i], cu_kv_of(c)[i + 1] - cu_kv_of(c)[i]) for i in range(len(cu_q) - 1)]
-                      for c in range(C)]
+        if self._segments is not None:
+            if isinstance(self._segments, _DeviceSegmentSource):
+                dev_seg = self._segments.over(range(C))
+            else:
+                # packed variable-length batch: every scheduled chunk runs once per segment
+                cu_q, cu_kv_of = self._segments
+                seg_q = [(cu_q[i], cu_q[i + 1] - cu_q[i]) for i in range(len(cu_q) - 1)]
+                seg_kv = [[(cu_kv_of(c)[i], cu_kv_of(c)[i + 1] - cu_kv_of(c)[i]) for i in range(len(cu_q) - 1)]
+                          for c in range(C)]
         ws = _hip.attn_workspace(query.device)
         if not rm.sched_windows:
-            n_comp = int(rm.sched_counts_host[t, l, 0])
-            _hip.attn_sched_fwd(query, _hip.ChunkTable(ks, vs), rm.sched_compute_ids[t, l], rm.sched_counts[t, l, 0:1],
-                                n_comp, cache.arena_out, cache.arena_lse, diag, cache.diag_out, cache.diag_lse,
-                                seg_q=seg_q, seg_kv=seg_kv, workspace=ws, q_prescaled=self.q_prescaled,
-                                dev_segments=dev_seg)
+            _hip.attn_sched_fwd(query, _hip.ChunkTable(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
+                                rm.compute_counts[t][l], cache.arena_out, cache.arena_lse, diag, cache.diag_out,
+                                cache.diag_lse, seg_q=seg_q, seg_kv=seg_kv, workspace=ws, q_prescaled=self.q_prescaled,
+                                dev_segments=dev_seg, row=t * rm.num_layers + l)
         else:
             # more chunks than one launch addresses: one launch per window of chunk ids (ordered on the
             # stream, so they can share the workspace)
+            ks, vs = [_as4d(k, B) for k in ks], [_as4d(v, B) for v in vs]
             for w0, w1, d_w, comp_w, cnt_w, cnt_host_w in rm.sched_windows:
                 n_comp = int(cnt_host_w[t, l, 0])
                 if n_comp == 0:
@@ -481,17 +494,10 @@ class proAttention:
                                     cache.diag_lse, seg_q=seg_q, seg_kv=None if seg_kv is None else seg_kv[w0:w1],
                                     workspace=ws, q_prescaled=self.q_prescaled,
                                     dev_segments=None if dev_seg is None else dev_seg.window(w0, w1))
-        outs, lses = [], []
         for c in range(C):
-            if c == diag:
-                outs.append(cache.diag_out)
-                lses.append(cache.diag_lse)
-            else:
-                if row[c] == 0:
-                    cache.arena_valid[c] = True
-                outs.append(cache.arena_out[c])
-                lses.append(cache.arena_lse[c])
-        out, lse = _hip.merge_states(outs, lses, dst_dtype=self.out_dtype, dst_lse_bsh=True)
+            if row[c] == 0 and c != diag:
+                valid[c] = True
+        out, lse = _hip.merge_arena(cache.arena_out, cache.arena_lse, diag, cache.diag_out, cache.diag_lse, self.out_dtype)
         self.last_lse = lse
         rm.record_out_redundancy(timestep=t, layer_id=l, curr_out=out)
         return out
@@ -620,6 +626,11 @@ class proAttention:
         return out.view(total_q, H, D)
 
 
+def _int32(t: torch.Tensor) -> torch.Tensor:
+    """``t`` itself for the contiguous int32 vectors the callers pass."""
+    return t if t.dtype is torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
+
+
 class _DeviceSegmentSource:
     """The segment boundaries of one variable-length call while they stay in device memory: hands the
     launches a ``_hip.DeviceSegments`` over the chunks they address."""
@@ -628,8 +639,8 @@ class _DeviceSegmentSource:
         if not (torch.is_tensor(local_cu_kv) and local_cu_kv.is_cuda):
             raise TypeError("cu_seqlens_q is on the GPU, so cu_seqlens_kv must be as well")
         self.attn = attn
-        self.cu_q = cu_q.to(torch.int32).contiguous()            # (no-ops for the int32 vectors the callers pass)
-        self.local = local_cu_kv.to(torch.int32).contiguous()
+        self.cu_q = _int32(cu_q)
+        self.local = _int32(local_cu_kv)
         self.max_seqlen_q = int(max_seqlen_q) if max_seqlen_q else int(total_q)
         self.n_seg = self.cu_q.numel() - 1
 
@@ -639,7 +650,7 @@ class _DeviceSegmentSource:
         cu = self.attn.group.kv_cu_seqlens(c)
         if not torch.is_tensor(cu):                              # a host list beside device boundaries: one small upload
             cu = torch.tensor(list(cu), dtype=torch.int32, device=self.cu_q.device)
-        return cu.to(torch.int32).contiguous()
+        return _int32(cu)
 
     def over(self, chunk_ids) -> "_hip.DeviceSegments":
         """Boundaries of the chunks ``chunk_ids`` in that order (the local chunk's are the call's ``cu_seqlens_kv``)."""

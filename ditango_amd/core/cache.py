@@ -26,6 +26,12 @@ from ..utils import get_timestep
 logger = init_logger(__name__)
 
 
+def _allocated_mb() -> float:
+    """``torch.cuda.memory_allocated()`` in MB; that function flattens and sorts every statistic first, 80 us a call."""
+    stats = torch.cuda.memory_stats_as_nested_dict()
+    return stats["allocated_bytes"]["all"]["current"] / (1024 * 1024) if stats else 0.0
+
+
 class proCache:
     def __init__(self, isp_size: int, layer_id: int):
         self.isp_size = isp_size
@@ -38,7 +44,7 @@ class proCache:
         self.block_size_mb: Optional[float] = None
         self._memory_constraint: Optional[float] = None
         # injectable probes (MB): current allocation and the budget (0.72 of device memory, cache.py:22)
-        self.memory_probe: Callable[[], float] = lambda: torch.cuda.memory_allocated() / (1024 * 1024)
+        self.memory_probe: Callable[[], float] = _allocated_mb
         # mask-mode arena
         self.arena_out: Optional[torch.Tensor] = None
         self.arena_lse: Optional[torch.Tensor] = None

@@ -54,6 +54,8 @@ class RedundancyMap:
         self.sched_reuse_ids: Optional[torch.Tensor] = None
         self.sched_counts: Optional[torch.Tensor] = None  # int32 [T,L,2] device
         self.sched_counts_host: Optional[np.ndarray] = None
+        self.mask_rows: list = []       # chunk_mask and the number of chunks to compute as nested lists: [t][l] is what a call reads
+        self.compute_counts: list = []
         self.sched_windows: list = []  # (first chunk, end, diag in window, compute ids, counts, counts on host)
 
     # ---- divider map / strides ---------------------------------------------------------------
@@ -276,6 +278,8 @@ class RedundancyMap:
         comp, reu, cnt = _hip.build_schedule_table(dmask, self.mask_diag)
         self.sched_compute_ids, self.sched_reuse_ids, self.sched_counts = comp, reu, cnt
         self.sched_counts_host = cnt.cpu().numpy()  # one read-back at install time, none per call
+        self.mask_rows = m.tolist()
+        self.compute_counts = self.sched_counts_host[:, :, 0].tolist()
         # One attention launch addresses at most DT_MAX_CHUNKS chunks: more chunks run as one launch per
         # window of chunk ids, each with its own compute list (ids relative to the window's first chunk).
         self.sched_windows = []

@@ -1,0 +1,529 @@
+// Host side of the launches: a Python extension module that checks tensors, allocates results and fills the argument
+// tables of the C ABI (include/ditango_hip.h), which it calls.  A layer call of a small problem lasts about as long on
+// the GPU as the checks of its two dozen tensors in Python did: with 4 KV chunks of 512 keys 59 us a call through
+// ctypes, of which 20 are kernels.
+//
+// Nothing here reads device memory, synchronises or keeps state between calls.  Errors are raised as the exception class
+// that ditango_amd._hip hands over (DitangoHipError).
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <cstdarg>
+#include <cstdio>
+#include <optional>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "ditango_hip.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+py::handle g_error;   // the exception class (kept alive by the module that set it)
+
+[[noreturn]] void fail(const std::string& msg) {
+  PyErr_SetString(g_error ? g_error.ptr() : PyExc_RuntimeError, msg.c_str());
+  throw py::error_already_set();
+}
+template <typename... Parts>
+std::string text(const Parts&... parts) {
+  std::string s;
+  (s.append(parts), ...);
+  return s;
+}
+// name[i], spelled only when a check fails
+struct Name {
+  const char* base;
+  int64_t i = -1;
+  std::string str() const { return i < 0 ? std::string(base) : text(base, "[", std::to_string(i), "]"); }
+};
+#define REQUIRE(cond, ...)              \
+  do {                                  \
+    if (!(cond)) [[unlikely]]           \
+      fail(text(__VA_ARGS__));          \
+  } while (0)
+
+void check(int rc, const char* what) {
+  if (rc != 0) fail(text(what, " failed with code ", std::to_string(rc), ": ", dt_last_error()));
+}
+
+bool is_half(const Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
+
+int dtype_code(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kBFloat16: return DT_BF16;
+    case at::kFloat: return DT_FP32;
+    case at::kHalf: return DT_FP16;
+    default: fail("unsupported state dtype (bf16, fp16 or fp32)");
+  }
+}
+
+bool shape_is(const Tensor& t, std::initializer_list<int64_t> want) { return t.sizes() == at::IntArrayRef(want); }
+
+struct Dims {
+  int64_t B, S, H, D;
+};
+
+Dims check_bshd(const Tensor& t, const Name& name) {
+  REQUIRE(t.is_cuda(), name.str(), " must live on the GPU");
+  REQUIRE(is_half(t), name.str(), " must be bf16 or fp16");
+  REQUIRE(t.dim() == 4 && t.stride(3) == 1, name.str(), " must be [B,S,H,D] with contiguous D");
+  return {t.size(0), t.size(1), t.size(2), t.size(3)};
+}
+
+// DT_LSE_BHS or DT_LSE_BSH of a dense lse tensor of (B, S, H) rows.  Where the shape alone cannot tell (S == H), a 4-D
+// tensor is read as the running layout [B,S,H,1] (utils.py:49) and a 3-D one as flash-attn's [B,H,S].
+int lse_layout(const Tensor& lse, int64_t B, int64_t S, int64_t H) {
+  const auto sizes = lse.sizes();
+  const auto strides = lse.strides();
+  const bool four = lse.dim() == 4 && sizes[3] == 1;
+  REQUIRE((lse.dim() == 3 || four) && lse.scalar_type() == at::kFloat, "lse must be fp32 with 3 (or 4, last=1) dims");
+  // dense in the order (d0, d1, d2) of its first three dimensions (strides of dimensions of size 1 do not matter)
+  auto dense = [&](int a, int b, int c) {
+    return (sizes[c] == 1 || strides[c] == 1) && (sizes[b] == 1 || strides[b] == sizes[c]) &&
+           (sizes[a] == 1 || strides[a] == sizes[b] * sizes[c]);
+  };
+  const bool empty = lse.numel() == 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    const bool bsh = four == (pass == 0);
+    if (!(sizes[0] == B && sizes[1] == (bsh ? S : H) && sizes[2] == (bsh ? H : S))) continue;
+    if (empty || dense(0, 1, 2)) return bsh ? DT_LSE_BSH : DT_LSE_BHS;
+    if (dense(0, 2, 1)) return bsh ? DT_LSE_BHS : DT_LSE_BSH;
+  }
+  fail("lse is not a dense [B,H,S] or [B,S,H] of the state's rows");
+}
+
+void* ptr(const Tensor& t) { return t.data_ptr(); }
+void* ptr(const std::optional<Tensor>& t) { return t ? t->data_ptr() : nullptr; }
+void* stream_of(uint64_t s) { return reinterpret_cast<void*>(s); }
+
+void check_state(const Tensor& o, const Tensor& l, const Dims& d, at::ScalarType dtype, const Name& on, const Name& ln) {
+  REQUIRE(o.scalar_type() == dtype && o.is_contiguous() && shape_is(o, {d.B, d.S, d.H, d.D}), on.str(),
+          " must be contiguous [B,Sq,H,D] in q's dtype");
+  REQUIRE(l.scalar_type() == at::kFloat && l.is_contiguous() && shape_is(l, {d.B, d.H, d.S}), ln.str(),
+          " must be contiguous fp32 [B,H,Sq]");
+}
+
+// ---- KV chunks ---------------------------------------------------------------------------------------------
+
+// The KV chunks one layer call can touch: pointers, lengths, strides.
+struct ChunkTable {
+  std::vector<Tensor> keep;   // alive while the pointers are in use
+  std::vector<const void*> k, v;
+  std::vector<int32_t> len;
+  std::vector<int64_t> sb;
+  int64_t n = 0, B = 0, H = 0, D = 0, ss = 0, sh = 0;
+  at::ScalarType dtype = at::kBFloat16;
+
+  // batch > 0: 3-D chunks are packed [batch * S, H, D] (the variable-length entry's layout); `convert` is called on
+  // chunks that are neither bf16 nor fp16
+  ChunkTable(const std::vector<Tensor>& ks, const std::vector<Tensor>& vs, int64_t batch, const py::object& convert) {
+    n = (int64_t)ks.size();
+    REQUIRE(n > 0 && ks.size() == vs.size(), "need at least one KV chunk and as many V as K chunks");
+    keep.reserve(2 * n);
+    k.reserve(n); v.reserve(n); len.reserve(n); sb.reserve(n);
+    bool any = false;
+    for (int64_t i = 0; i < n; ++i) {
+      Tensor kt = ks[i], vt = vs[i];
+      if (!convert.is_none()) {
+        if (!is_half(kt)) kt = py::cast<Tensor>(convert(kt));
+        if (!is_half(vt)) vt = py::cast<Tensor>(convert(vt));
+      }
+      if (batch > 0 && kt.dim() == 3) kt = kt.view({batch, kt.size(0) / batch, kt.size(1), kt.size(2)});
+      if (batch > 0 && vt.dim() == 3) vt = vt.view({batch, vt.size(0) / batch, vt.size(1), vt.size(2)});
+      if (i == 0) dtype = kt.scalar_type();
+      const Dims d = check_bshd(kt, {"k", i});
+      check_bshd(vt, {"v", i});
+      REQUIRE(kt.scalar_type() == dtype && vt.scalar_type() == dtype, Name{"k", i}.str(),
+              " / v must have one dtype with the other attention inputs");
+      REQUIRE(kt.sizes() == vt.sizes() && kt.strides() == vt.strides(), Name{"k", i}.str(), " / v mismatch");
+      if (d.S > 0) {
+        if (!any) {
+          ss = kt.stride(1); sh = kt.stride(2);
+          B = d.B; H = d.H; D = d.D;
+          any = true;
+        }
+        REQUIRE(kt.stride(1) == ss && kt.stride(2) == sh, "all chunks must share token/head strides");
+        REQUIRE(d.B == B && d.H == H && d.D == D, "chunk B/H/D mismatch");
+      }
+      k.push_back(kt.data_ptr());
+      v.push_back(vt.data_ptr());
+      len.push_back((int32_t)d.S);
+      sb.push_back(kt.stride(0));
+      keep.push_back(std::move(kt));
+      keep.push_back(std::move(vt));
+    }
+    REQUIRE(any, "all KV chunks are empty");
+  }
+};
+
+Dims check_query(const Tensor& q, const ChunkTable& t) {
+  const Dims d = check_bshd(q, {"q"});
+  REQUIRE(q.scalar_type() == t.dtype, "q must have the dtype of the KV chunks");
+  REQUIRE(d.B == t.B && d.H == t.H && d.D == t.D, "q and KV chunks disagree on B/H/D");
+  return d;
+}
+
+// Segment boundaries in device memory (see ditango_amd._hip.DeviceSegments).
+struct Segments {
+  Tensor cu_q;
+  std::vector<std::optional<Tensor>> cu_kv;
+  int64_t max_q = 0;
+  int32_t n_seg() const { return (int32_t)cu_q.numel() - 1; }
+};
+void check_boundaries(const Tensor& t, const Name& name) {
+  REQUIRE(t.is_cuda() && t.scalar_type() == at::kInt && t.dim() == 1 && t.is_contiguous(), name.str(),
+          " must be a contiguous int32 vector on the GPU");
+}
+Segments make_segments(const Tensor& cu_q, std::vector<std::optional<Tensor>> cu_kv, int64_t max_q) {
+  check_boundaries(cu_q, {"cu_seqlens_q"});
+  for (size_t i = 0; i < cu_kv.size(); ++i)
+    if (cu_kv[i]) {
+      check_boundaries(*cu_kv[i], {"cu_seqlens_kv", (int64_t)i});
+      REQUIRE(cu_kv[i]->numel() == cu_q.numel(), Name{"cu_seqlens_kv", (int64_t)i}.str(),
+              " must have as many entries as cu_seqlens_q");
+    }
+  REQUIRE(cu_q.numel() >= 2, "cu_seqlens_q needs at least two entries");
+  REQUIRE(max_q > 0, "max_seqlen_q must be positive");
+  return {cu_q, std::move(cu_kv), max_q};
+}
+
+typedef std::pair<int32_t, int32_t> Range;   // (begin, length)
+
+int64_t bytes_of(const std::optional<Tensor>& t) { return t ? (int64_t)t->nbytes() : 0; }
+
+// One launch or, where the jobs exceed the limits of one, several (ditango_amd._hip.attn_jobs_fwd).
+void attn_jobs(const Tensor& q, const ChunkTable& table, const std::vector<std::vector<int32_t>>& jobs,
+               const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, double scale,
+               const std::optional<std::vector<Range>>& q_ranges,
+               const std::optional<std::vector<std::vector<Range>>>& kv_ranges, const std::optional<Tensor>& workspace,
+               int32_t flags, bool no_alloc, const Segments* seg, const std::optional<std::vector<int32_t>>& job_segments,
+               uint64_t stream) {
+  const Dims d = check_query(q, table);
+  const size_t nj = jobs.size();
+  REQUIRE(!(no_alloc && workspace), "no_alloc launches take no workspace");
+  if (seg) {
+    REQUIRE(!q_ranges && !kv_ranges && !no_alloc, "device segment boundaries replace the host ranges");
+    REQUIRE(job_segments && job_segments->size() == nj, "one segment index per job");
+    REQUIRE((int64_t)seg->cu_kv.size() == table.n, "one cu_seqlens_kv per chunk of the table");
+  }
+  REQUIRE(nj == outs.size() && nj == lses.size(), "one destination per job");
+  REQUIRE(!q_ranges || q_ranges->size() == nj, "one query range per job");
+  REQUIRE(!kv_ranges || kv_ranges->size() == nj, "one list of key ranges per job");
+  for (size_t j = 0; j < nj; ++j) {
+    check_state(outs[j], lses[j], d, q.scalar_type(), {"outs", (int64_t)j}, {"lses", (int64_t)j});
+    REQUIRE(jobs[j].size() <= DT_MAX_JOB_ENTRIES, "a job references more than ", std::to_string(DT_MAX_JOB_ENTRIES), " chunks");
+    REQUIRE(!kv_ranges || (*kv_ranges)[j].size() >= jobs[j].size(), "one key range per chunk reference");
+    for (int32_t c : jobs[j])
+      REQUIRE(c >= 0 && c < table.n, "job ", std::to_string(j), " references chunk ", std::to_string(c), " outside the table of ",
+              std::to_string(table.n));
+  }
+  const bool whole = table.n <= DT_MAX_CHUNKS;   // every chunk is in the launch's table under its own number
+  std::vector<int32_t> local(whole ? 0 : table.n);
+  size_t start = 0;
+  while (start < nj) {
+    // the jobs of this launch: within the limits on jobs, chunk references and (a larger table) distinct chunks
+    size_t end = start, entries = 0;
+    std::vector<int32_t> ids;
+    if (!whole) std::fill(local.begin(), local.end(), -1);
+    while (end < nj && end - start < DT_MAX_JOBS && entries + jobs[end].size() <= DT_MAX_JOB_ENTRIES) {
+      if (!whole) {
+        const size_t before = ids.size();
+        for (int32_t c : jobs[end])
+          if (local[c] < 0) {
+            local[c] = (int32_t)ids.size();
+            ids.push_back(c);
+          }
+        if (ids.size() > DT_MAX_CHUNKS) {
+          for (size_t i = before; i < ids.size(); ++i) local[ids[i]] = -1;
+          ids.resize(before);
+          break;
+        }
+      }
+      entries += jobs[end].size();
+      ++end;
+    }
+    REQUIRE(end > start, "job ", std::to_string(start), " references more than ", std::to_string(DT_MAX_CHUNKS),
+            " distinct chunks: split it and merge the parts");
+    if (!whole && ids.empty()) ids.push_back(0);
+    const void *kp[DT_MAX_CHUNKS], *vp[DT_MAX_CHUNKS];
+    int32_t lens[DT_MAX_CHUNKS];
+    int64_t sbs[DT_MAX_CHUNKS];
+    const int32_t* cu_kv[DT_MAX_CHUNKS];
+    const int32_t nc = whole ? (int32_t)table.n : (int32_t)ids.size();
+    for (int32_t i = 0; i < nc; ++i) {
+      const int32_t c = whole ? i : ids[i];
+      kp[i] = table.k[c]; vp[i] = table.v[c];
+      lens[i] = table.len[c]; sbs[i] = table.sb[c];
+      if (seg) cu_kv[i] = static_cast<const int32_t*>(ptr(seg->cu_kv[c]));
+    }
+    int32_t begin[DT_MAX_JOBS + 1], chunks[DT_MAX_JOB_ENTRIES], kb[DT_MAX_JOB_ENTRIES], kl[DT_MAX_JOB_ENTRIES];
+    int32_t qb[DT_MAX_JOBS], ql[DT_MAX_JOBS], segs[DT_MAX_JOBS];
+    void* op[DT_MAX_JOBS];
+    float* lp[DT_MAX_JOBS];
+    const int32_t n = (int32_t)(end - start);
+    int32_t e = 0;
+    for (int32_t jj = 0; jj < n; ++jj) {
+      const size_t j = start + jj;
+      begin[jj] = e;
+      for (size_t i = 0; i < jobs[j].size(); ++i, ++e) {
+        chunks[e] = whole ? jobs[j][i] : local[jobs[j][i]];
+        if (kv_ranges) { kb[e] = (*kv_ranges)[j][i].first; kl[e] = (*kv_ranges)[j][i].second; }
+      }
+      if (q_ranges) { qb[jj] = (*q_ranges)[j].first; ql[jj] = (*q_ranges)[j].second; }
+      if (seg) segs[jj] = (*job_segments)[j];
+      op[jj] = outs[j].data_ptr();
+      lp[jj] = static_cast<float*>(lses[j].data_ptr());
+    }
+    begin[n] = e;
+    const auto sq = q.strides();
+    if (seg)
+      check(dt_attn_varlen_jobs_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
+                                       begin, chunks, segs, seg->n_seg(), static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv,
+                                       (int32_t)seg->max_q, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace),
+                                       stream_of(stream)),
+            "dt_attn_varlen_jobs_ws_fwd");
+    else if (no_alloc)
+      check(dt_attn_seg_jobs_noalloc_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
+                                         begin, chunks, kv_ranges ? kb : nullptr, kv_ranges ? kl : nullptr,
+                                         q_ranges ? qb : nullptr, q_ranges ? ql : nullptr, op, lp, (float)scale, flags,
+                                         stream_of(stream)),
+            "dt_attn_seg_jobs_noalloc_fwd");
+    else
+      check(dt_attn_seg_jobs_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
+                                    begin, chunks, kv_ranges ? kb : nullptr, kv_ranges ? kl : nullptr, q_ranges ? qb : nullptr,
+                                    q_ranges ? ql : nullptr, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace),
+                                    stream_of(stream)),
+            "dt_attn_seg_jobs_ws_fwd");
+    start = end;
+  }
+}
+
+// Device-scheduled launch over a table that fits one launch (ditango_amd._hip.attn_sched_fwd).  The schedule is row `row`
+// of ids [rows, C] and counts [rows, 2] (or the tensors themselves, row 0).
+void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, const Tensor& count, int64_t row, int32_t max_jobs,
+                const Tensor& slot_out, const Tensor& slot_lse, int32_t diag, const std::optional<Tensor>& diag_out,
+                const std::optional<Tensor>& diag_lse, double scale, const std::optional<std::vector<Range>>& seg_q,
+                const std::optional<std::vector<std::vector<Range>>>& seg_kv, const std::optional<Tensor>& workspace,
+                int32_t flags, const Segments* seg, uint64_t stream) {
+  const Dims d = check_query(q, table);
+  REQUIRE(table.n <= DT_MAX_CHUNKS, "the table holds ", std::to_string(table.n), " chunks, one launch addresses ",
+          std::to_string(DT_MAX_CHUNKS));
+  REQUIRE(ids.scalar_type() == at::kInt && count.scalar_type() == at::kInt && ids.is_cuda() && count.is_cuda(),
+          "schedule tensors must be int32 on the GPU");
+  const int64_t per_row = ids.dim() > 1 ? ids.size(-1) : ids.numel(), per_count = count.dim() > 1 ? count.size(-1) : count.numel();
+  REQUIRE(ids.is_contiguous() && count.is_contiguous() && per_row >= max_jobs && per_count >= 1 && row >= 0 &&
+              (row + 1) * per_row <= ids.numel() && (row + 1) * per_count <= count.numel(),
+          "compute id list shorter than max_jobs");
+  REQUIRE(slot_out.scalar_type() == q.scalar_type() && slot_out.is_contiguous() && slot_out.dim() == 5 &&
+              slot_out.sizes().slice(1) == at::IntArrayRef({d.B, d.S, d.H, d.D}) && slot_out.size(0) >= table.n,
+          "slot_out must be contiguous [C,B,Sq,H,D] in q's dtype");
+  REQUIRE(slot_lse.scalar_type() == at::kFloat && slot_lse.is_contiguous() && slot_lse.dim() == 4 &&
+              slot_lse.sizes().slice(1) == at::IntArrayRef({d.B, d.H, d.S}) && slot_lse.size(0) >= table.n,
+          "slot_lse must be contiguous fp32 [C,B,H,Sq]");
+  if (diag >= 0 && diag < table.n) {
+    REQUIRE(diag_out && diag_lse, "a diag chunk needs (diag_out, diag_lse)");
+    check_state(*diag_out, *diag_lse, d, q.scalar_type(), {"diag_out"}, {"diag_lse"});
+  }
+  const auto sq = q.strides();
+  const int32_t* dev_ids = static_cast<const int32_t*>(ptr(ids)) + row * per_row;
+  const int32_t* dev_count = static_cast<const int32_t*>(ptr(count)) + row * per_count;
+  float* sl = static_cast<float*>(ptr(slot_lse));
+  float* dl = static_cast<float*>(ptr(diag_lse));
+  if (seg) {
+    REQUIRE(!seg_q && !seg_kv, "device segment boundaries replace the host ranges");
+    REQUIRE((int64_t)seg->cu_kv.size() == table.n, "one cu_seqlens_kv per chunk of the table");
+    const int32_t* cu_kv[DT_MAX_CHUNKS];
+    for (int64_t c = 0; c < table.n; ++c) cu_kv[c] = static_cast<const int32_t*>(ptr(seg->cu_kv[c]));
+    check(dt_attn_sched_varlen_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(), table.v.data(),
+                                      table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs,
+                                      ptr(slot_out), slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl,
+                                      seg->n_seg(), static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv, (int32_t)seg->max_q,
+                                      (float)scale, flags, ptr(workspace), bytes_of(workspace), stream_of(stream)),
+          "dt_attn_sched_varlen_ws_fwd");
+    return;
+  }
+  int32_t n_seg = 0, qb[DT_MAX_SEGMENTS], ql[DT_MAX_SEGMENTS], kb[DT_MAX_JOB_ENTRIES], kl[DT_MAX_JOB_ENTRIES];
+  if (seg_q) {
+    n_seg = (int32_t)seg_q->size();
+    REQUIRE(seg_kv && (int64_t)seg_kv->size() == table.n, "seg_kv needs one (begin, length) per chunk and segment");
+    REQUIRE(n_seg > 0 && n_seg <= DT_MAX_SEGMENTS && n_seg * table.n <= DT_MAX_JOB_ENTRIES, "need 1..",
+            std::to_string(DT_MAX_SEGMENTS), " segments and at most ", std::to_string(DT_MAX_JOB_ENTRIES), " (chunk, segment) pairs");
+    for (int32_t s = 0; s < n_seg; ++s) { qb[s] = (*seg_q)[s].first; ql[s] = (*seg_q)[s].second; }
+    int32_t e = 0;
+    for (const auto& r : *seg_kv) {
+      REQUIRE((int32_t)r.size() == n_seg, "seg_kv needs one (begin, length) per chunk and segment");
+      for (const Range& x : r) { kb[e] = x.first; kl[e++] = x.second; }
+    }
+  }
+  check(dt_attn_sched_seg_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(), table.v.data(),
+                                 table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs, ptr(slot_out),
+                                 slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl, n_seg, n_seg ? qb : nullptr,
+                                 n_seg ? ql : nullptr, n_seg ? kb : nullptr, n_seg ? kl : nullptr, (float)scale, flags,
+                                 ptr(workspace), bytes_of(workspace), stream_of(stream)),
+        "dt_attn_sched_seg_ws_fwd");
+}
+
+// ---- states ------------------------------------------------------------------------------------------------
+
+struct StateList {   // the states of one merge launch
+  int32_t n = 0;
+  const void* out[DT_MAX_MERGE];
+  const float* lse[DT_MAX_MERGE];
+  int32_t dtype[DT_MAX_MERGE], layout[DT_MAX_MERGE];
+  void add(const void* o, const void* l, int32_t dt, int32_t lay) {
+    out[n] = o;
+    lse[n] = static_cast<const float*>(l);
+    dtype[n] = dt;
+    layout[n++] = lay;
+  }
+  void launch(const Tensor& dst_out, const Tensor& dst_lse, const Dims& d, uint64_t stream) const {
+    check(dt_merge_states(n, out, lse, dtype, layout, ptr(dst_out), dtype_code(dst_out), static_cast<float*>(ptr(dst_lse)),
+                          lse_layout(dst_lse, d.B, d.S, d.H), d.B, d.S, d.H, d.D, stream_of(stream)),
+          "dt_merge_states");
+  }
+};
+
+Tensor new_out(const Dims& d, at::ScalarType dtype, const Tensor& like) {
+  return at::empty({d.B, d.S, d.H, d.D}, like.options().dtype(dtype));
+}
+Tensor new_lse(const Dims& d, bool bsh, const Tensor& like) {
+  const auto opt = like.options().dtype(at::kFloat);
+  return bsh ? at::empty({d.B, d.S, d.H, 1}, opt) : at::empty({d.B, d.H, d.S}, opt);
+}
+
+// N-way merge; more states than one launch folds run in rounds through a running fp32 state (ditango_amd._hip.merge_states).
+std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, std::optional<Tensor> dst_out,
+                                std::optional<Tensor> dst_lse, at::ScalarType dst_dtype, bool dst_bsh, uint64_t stream) {
+  const size_t n = outs.size();
+  REQUIRE(n > 0 && n == lses.size(), "need at least one state and one lse per state");
+  REQUIRE(outs[0].dim() == 4, "outs[0] must be contiguous [B,Sq,H,D] on the GPU");
+  const Dims d{outs[0].size(0), outs[0].size(1), outs[0].size(2), outs[0].size(3)};
+  if (!dst_out) dst_out = new_out(d, dst_dtype, outs[0]);
+  if (!dst_lse) dst_lse = new_lse(d, dst_bsh, outs[0]);
+  REQUIRE(dst_out->is_contiguous() && shape_is(*dst_out, {d.B, d.S, d.H, d.D}), "dst_out must be contiguous [B,Sq,H,D]");
+  StateList s;
+  Tensor run_out, run_lse;
+  for (size_t i = 0; i < n; ++i) {
+    const Tensor &o = outs[i], &l = lses[i];
+    REQUIRE(o.is_cuda() && o.is_contiguous() && shape_is(o, {d.B, d.S, d.H, d.D}), Name{"outs", (int64_t)i}.str(),
+            " must be contiguous [B,Sq,H,D] on the GPU");
+    if (s.n == DT_MAX_MERGE) {
+      if (!run_out.defined()) {
+        run_out = new_out(d, at::kFloat, outs[0]);
+        run_lse = new_lse(d, false, outs[0]);
+      }
+      s.launch(run_out, run_lse, d, stream);
+      s.n = 0;
+      s.add(ptr(run_out), ptr(run_lse), DT_FP32, DT_LSE_BHS);
+    }
+    s.add(ptr(o), ptr(l), dtype_code(o), lse_layout(l, d.B, d.S, d.H));
+  }
+  s.launch(*dst_out, *dst_lse, d, stream);
+  return {*dst_out, *dst_lse};
+}
+
+// Merge of every slot of an arena ([C,B,Sq,H,D] / [C,B,H,Sq]), slot `diag` replaced by (diag_out, diag_lse).
+std::pair<Tensor, Tensor> merge_arena(const Tensor& arena_out, const Tensor& arena_lse, int64_t diag, const Tensor& diag_out,
+                                      const Tensor& diag_lse, at::ScalarType dst_dtype, uint64_t stream) {
+  REQUIRE(arena_out.dim() == 5 && arena_out.is_cuda() && arena_out.is_contiguous(), "the arena must be contiguous [C,B,Sq,H,D]");
+  const int64_t C = arena_out.size(0);
+  const Dims d{arena_out.size(1), arena_out.size(2), arena_out.size(3), arena_out.size(4)};
+  REQUIRE(arena_lse.scalar_type() == at::kFloat && arena_lse.is_contiguous() && shape_is(arena_lse, {C, d.B, d.H, d.S}),
+          "the arena's lse must be contiguous fp32 [C,B,H,Sq]");
+  if (diag >= 0 && diag < C) check_state(diag_out, diag_lse, d, arena_out.scalar_type(), {"diag_out"}, {"diag_lse"});
+  const Tensor dst_out = new_out(d, dst_dtype, arena_out), dst_lse = new_lse(d, true, arena_out);
+  const int32_t dt = dtype_code(arena_out);
+  const int64_t out_bytes = arena_out.stride(0) * arena_out.element_size(), lse_bytes = arena_lse.stride(0) * 4;
+  StateList s;
+  Tensor run_out, run_lse;
+  for (int64_t c = 0; c < C; ++c) {
+    if (s.n == DT_MAX_MERGE) {
+      if (!run_out.defined()) {
+        run_out = new_out(d, at::kFloat, arena_out);
+        run_lse = new_lse(d, false, arena_out);
+      }
+      s.launch(run_out, run_lse, d, stream);
+      s.n = 0;
+      s.add(ptr(run_out), ptr(run_lse), DT_FP32, DT_LSE_BHS);
+    }
+    if (c == diag) s.add(ptr(diag_out), ptr(diag_lse), dt, DT_LSE_BHS);
+    else s.add(static_cast<const char*>(ptr(arena_out)) + c * out_bytes, static_cast<const char*>(ptr(arena_lse)) + c * lse_bytes, dt, DT_LSE_BHS);
+  }
+  s.launch(dst_out, dst_lse, d, stream);
+  return {dst_out, dst_lse};
+}
+
+// One pass from (src_out, src_lse) into (dst_out, dst_lse), any dtypes and lse layouts.
+void copy_state(const Tensor& src_out, const Tensor& src_lse, const Tensor& dst_out, const Tensor& dst_lse, uint64_t stream) {
+  REQUIRE(src_out.dim() == 4 && src_out.is_cuda() && src_out.is_contiguous(), "the source must be contiguous [B,Sq,H,D] on the GPU");
+  const Dims d{src_out.size(0), src_out.size(1), src_out.size(2), src_out.size(3)};
+  REQUIRE(dst_out.is_cuda() && dst_out.is_contiguous() && shape_is(dst_out, {d.B, d.S, d.H, d.D}),
+          "the destination must be contiguous [B,Sq,H,D] on the GPU");
+  check(dt_state_copy(ptr(src_out), dtype_code(src_out), static_cast<const float*>(ptr(src_lse)), lse_layout(src_lse, d.B, d.S, d.H),
+                      ptr(dst_out), dtype_code(dst_out), static_cast<float*>(ptr(dst_lse)), lse_layout(dst_lse, d.B, d.S, d.H),
+                      d.B, d.S, d.H, d.D, stream_of(stream)),
+        "dt_state_copy");
+}
+void cache_store(const Tensor& src_out, const Tensor& src_lse, const Tensor& slot_out, const Tensor& slot_lse, uint64_t stream) {
+  REQUIRE(is_half(slot_out), "slot_out must be contiguous bf16 or fp16 [B,Sq,H,D]");
+  REQUIRE(slot_lse.is_contiguous() && src_out.dim() == 4 && shape_is(slot_lse, {src_out.size(0), src_out.size(2), src_out.size(1)}),
+          "slot_lse must be contiguous fp32 [B,H,Sq]");
+  copy_state(src_out, src_lse, slot_out, slot_lse, stream);
+}
+std::pair<Tensor, Tensor> cache_load(const Tensor& slot_out, const Tensor& slot_lse, at::ScalarType dst_dtype, bool dst_bsh,
+                                     std::optional<Tensor> dst_out, std::optional<Tensor> dst_lse, uint64_t stream) {
+  REQUIRE(is_half(slot_out) && slot_out.dim() == 4, "slot_out must be contiguous bf16 or fp16");
+  const Dims d{slot_out.size(0), slot_out.size(1), slot_out.size(2), slot_out.size(3)};
+  REQUIRE(slot_lse.is_contiguous() && shape_is(slot_lse, {d.B, d.H, d.S}), "slot_lse must be contiguous fp32 [B,H,Sq]");
+  if (!dst_out) dst_out = new_out(d, dst_dtype, slot_out);
+  if (!dst_lse) dst_lse = new_lse(d, dst_bsh, slot_out);
+  copy_state(slot_out, slot_lse, *dst_out, *dst_lse, stream);
+  return {*dst_out, *dst_lse};
+}
+
+void zero_rows_from(const Tensor& t, const Tensor& first_row, uint64_t stream) {
+  REQUIRE(t.is_cuda() && t.is_contiguous() && t.dim() >= 1, "t must be a contiguous device tensor");
+  REQUIRE(first_row.is_cuda() && first_row.scalar_type() == at::kInt && first_row.numel() >= 1, "first_row must be int32 on the GPU");
+  const int64_t n = t.size(0);
+  check(dt_zero_rows_from(ptr(t), n, t.numel() / (n > 0 ? n : 1) * t.element_size(), static_cast<const int32_t*>(ptr(first_row)),
+                          stream_of(stream)),
+        "dt_zero_rows_from");
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_ditango_host, m) {
+  m.def("set_error_class", [](py::object cls) { g_error = cls.release(); });
+  m.def("lse_layout", &lse_layout);
+  py::class_<ChunkTable>(m, "ChunkTable")
+      .def(py::init<const std::vector<Tensor>&, const std::vector<Tensor>&, int64_t, const py::object&>())
+      .def_readonly("n", &ChunkTable::n)
+      .def_readonly("B", &ChunkTable::B)
+      .def_readonly("H", &ChunkTable::H)
+      .def_readonly("D", &ChunkTable::D)
+      .def_readonly("ss", &ChunkTable::ss)
+      .def_readonly("sh", &ChunkTable::sh)
+      .def_property_readonly("arrays", [](const ChunkTable& t) {
+        std::vector<uint64_t> k, v;
+        for (int64_t i = 0; i < t.n; ++i) {
+          k.push_back(reinterpret_cast<uint64_t>(t.k[i]));
+          v.push_back(reinterpret_cast<uint64_t>(t.v[i]));
+        }
+        return py::make_tuple(k, v, t.len, t.sb);
+      });
+  py::class_<Segments>(m, "Segments").def(py::init(&make_segments)).def_property_readonly("n_seg", &Segments::n_seg);
+  m.def("attn_jobs", &attn_jobs);
+  m.def("attn_sched", &attn_sched);
+  m.def("merge", &merge);
+  m.def("merge_arena", &merge_arena);
+  m.def("cache_store", &cache_store);
+  m.def("cache_load", &cache_load);
+  m.def("zero_rows_from", &zero_rows_from);
+}
