@@ -241,42 +241,7 @@ def attn_jobs_f32_fwd(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunk
     """One launch: the fp32 states (out [B,Sq,H,D], lse [B,H,Sq]) of fp32 q against the concatenations of the fp32
     chunks ``jobs[j]``.  Each chunk may have strides of its own.  More jobs or chunks than one launch addresses run in
     several."""
-    lib = load_library()
-    B, Sq, H, D = q.shape
-    _check_qkv(q, "q", torch.float32)
-    for i, (k, v) in enumerate(zip(k_chunks, v_chunks)):
-        _check_qkv(k, f"k[{i}]", torch.float32)
-        _check_qkv(v, f"v[{i}]", torch.float32)
-        _require(k.shape == v.shape and k.shape[0] == B and k.shape[2] == H and k.shape[3] == D, "k/v shape mismatch")
-        _require(k.stride() == v.stride(), "k and v must share strides")
-    states = [(torch.empty((B, Sq, H, D), dtype=torch.float32, device=q.device),
-               torch.empty((B, H, Sq), dtype=torch.float32, device=q.device)) for _ in jobs]
-    start = 0
-    while start < len(jobs):
-        ids: List[int] = []          # chunks of this launch, in order of first use
-        begin, flat, end = [0], [], start
-        while end < len(jobs) and end - start < DT_MAX_JOBS and len(flat) + len(jobs[end]) <= DT_MAX_JOB_ENTRIES:
-            more = ids + [c for c in dict.fromkeys(jobs[end]) if c not in ids]
-            if len(more) > DT_MAX_CHUNKS:
-                break
-            ids = more
-            flat += [ids.index(c) for c in jobs[end]]
-            begin.append(len(flat))
-            end += 1
-        _require(end > start, f"job {start} references more chunks than one launch addresses: split it and merge the parts")
-        n, m = end - start, max(1, len(ids))
-        ks, vs = [k_chunks[c] for c in ids], [v_chunks[c] for c in ids]
-        rc = lib.dt_attn_jobs_f32_fwd(
-            q.data_ptr(), B, Sq, H, D, q.stride(0), q.stride(1), q.stride(2), len(ids),
-            (c_vp * m)(*[k.data_ptr() for k in ks]), (c_vp * m)(*[v.data_ptr() for v in vs]),
-            (c_i32 * m)(*[k.shape[1] for k in ks]), (c_i64 * m)(*[k.stride(0) for k in ks]),
-            (c_i64 * m)(*[k.stride(1) for k in ks]), (c_i64 * m)(*[k.stride(2) for k in ks]),
-            n, (c_i32 * (n + 1))(*begin), (c_i32 * max(1, len(flat)))(*flat),
-            (c_vp * n)(*[s[0].data_ptr() for s in states[start:end]]), (c_vp * n)(*[s[1].data_ptr() for s in states[start:end]]),
-            float(softmax_scale), _stream())
-        _check(rc, "dt_attn_jobs_f32_fwd")
-        start = end
-    return states
+    return _host().attn_states_f32(q, k_chunks, v_chunks, jobs, softmax_scale, _stream())
 
 
 _workspaces: "dict" = {}   # (device type, index, stream handle) -> tensor, in order of last use
@@ -375,6 +340,19 @@ def attn_jobs_fwd(q: torch.Tensor, table: ChunkTable, jobs: Sequence[Sequence[in
     _host().attn_jobs(q, table.native, jobs, outs, lses, softmax_scale, q_ranges, kv_ranges, workspace,
                       _attn_flags(q, q_prescaled), no_alloc, None if dev_segments is None else dev_segments.native,
                       job_segments, _stream())
+
+
+def attn_states(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor],
+                jobs: Sequence[Sequence[int]], max_chunks: int, workspace: Optional[torch.Tensor] = None,
+                q_prescaled: bool = False, cu_q: Optional[Sequence[int]] = None,
+                cu_kv: Optional[Sequence[Sequence[int]]] = None, dev_segments: Optional[DeviceSegments] = None,
+                convert=None) -> List[Tuple[torch.Tensor, torch.Tensor]]:
+    """The fresh states (out [B,Sq,H,D] in q's dtype, lse [B,H,Sq]) of q against the concatenations of the chunks
+    ``jobs[j]``, computed in one launch where its limits allow.  A job of more than ``max_chunks`` chunks is computed in
+    pieces.  A packed variable-length batch brings its boundaries as host lists (``cu_q``, ``cu_kv[chunk]``) or as
+    ``dev_segments``; rows outside every segment are left as they are.  ``convert`` as in ``ChunkTable``."""
+    return _host().attn_states(q, k_chunks, v_chunks, jobs, max_chunks, cu_q, cu_kv, workspace, _attn_flags(q, q_prescaled),
+                               None if dev_segments is None else dev_segments.native, convert, _stream())
 
 
 def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor,

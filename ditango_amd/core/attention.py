@@ -68,6 +68,9 @@ class CallPlan:
     target_after: int = 0
     nblk_after: int = 0
     occupancy_after: List[bool] = field(default_factory=list)
+    # what the launch takes: the chunks the jobs reference, the distinct jobs as positions in that list, and which of
+    # them each job of `jobs` is
+    launch: Optional[Tuple[list, list, list]] = field(default=None, repr=False, compare=False)
 
 
 def plan_call(N: int, r: int, curr: int, nxt: int, targets: List[int], use_ditango: bool = True,
@@ -149,15 +152,31 @@ def plan_call(N: int, r: int, curr: int, nxt: int, targets: List[int], use_ditan
 
 @lru_cache(maxsize=256)
 def _planned(N: int, r: int, curr: int, nxt: int, targets: Tuple[int, ...], use_ditango: bool, small_ring_stride: int):
-    return plan_call(N, r, curr, nxt, list(targets), use_ditango, small_ring_stride)
+    plan, new_targets = plan_call(N, r, curr, nxt, list(targets), use_ditango, small_ring_stride)
+    plan.launch = _launch_of(plan.jobs)
+    return plan, new_targets
 
 
 def _plan_of_call(N: int, r: int, curr: int, nxt: int, targets: List[int], use_ditango: bool, small_ring_stride: int):
     """``plan_call`` looked up: a schedule visits few distinct integer states, the same ones in every layer."""
     p, new_targets = _planned(N, r, curr, nxt, tuple(targets), use_ditango, small_ring_stride)
     plan = CallPlan(0, 0, p.rank, p.curr_stride, p.next_stride, list(p.reuse_probed), [], list(p.computed), list(p.jobs),
-                    list(p.stores), list(p.flushes), p.target_after)
+                    list(p.stores), list(p.flushes), p.target_after, launch=p.launch)
     return plan, list(new_targets)
+
+
+def _launch_of(jobs: List[Job]) -> Tuple[list, list, list]:
+    """See ``CallPlan.launch``.  A chunk computed twice by the reference (local + own) is computed once and merged twice; a
+    state that enters the cache is nobody else's."""
+    needed = sorted({c for job in jobs for c in job.chunks})
+    index = {c: i for i, c in enumerate(needed)}
+    lists, which, seen = [], [], {}
+    for job in jobs:
+        if job.store_slot is not None or job.chunks not in seen:
+            seen[job.chunks] = len(lists)
+            lists.append([index[c] for c in job.chunks])
+        which.append(seen[job.chunks])
+    return needed, lists, which
 
 
 _warned_cast = set()
@@ -342,9 +361,7 @@ class proAttention:
         return result
 
     def _execute(self, plan: CallPlan, query, key, value, merge_outs, merge_lses, segments=None) -> torch.Tensor:
-        B, Sq, H, D = query.shape
-        N, r = self.isp_size, self.local_chunk_id
-        dev = query.device
+        r = self.local_chunk_id
         if self._exact_f32:
             distinct = list(dict.fromkeys(job.chunks for job in plan.jobs))
             seen = dict(zip(distinct, self._job_states_f32(query, distinct, key, value)))
@@ -357,75 +374,23 @@ class proAttention:
             out, lse = _hip.merge_states(merge_outs, merge_lses, dst_dtype=self.out_dtype, dst_lse_bsh=True)
             self.last_lse = lse
             return out
-        # chunk table: the local chunk is (key, value); the others come from the ring stand-in
-        needed = sorted({c for job in plan.jobs for c in job.chunks})
-        ks: List[torch.Tensor] = []
-        vs: List[torch.Tensor] = []
-        index = {}
-        for c in needed:
-            index[c] = len(ks)
-            k_c, v_c = (key, value) if c == r else self.group.kv_chunk(c)
-            ks.append(k_c)
-            vs.append(v_c)
-        # one launch for all distinct states; a chunk computed twice by the reference
-        # (local + own) is computed once and merged twice
-        job_lists, dests, seen = [], [], {}
-        pieced = []  # states computed in pieces: [(o, l) of the first piece = destination, the others...]
-        dev_seg = segments if isinstance(segments, _DeviceSegmentSource) else None
-        q_ranges, kv_ranges = ([], []) if segments is not None and dev_seg is None else (None, None)
-        job_segs = [] if dev_seg is not None else None
-        states = []
-        for job in plan.jobs:
-            if job.chunks in seen and job.store_slot is None:
-                states.append(seen[job.chunks])
-                continue
-            o = torch.empty((B, Sq, H, D), dtype=query.dtype, device=dev)
-            l = torch.empty((B, H, Sq), dtype=torch.float32, device=dev)
-            if len(set(job.chunks)) > self._MAX_JOB_CHUNKS:
-                # a block of more chunks than one launch addresses (rings of 128 positions and more): its
-                # state is computed in pieces that are folded into (o, l) behind the attention launch
-                pieces = [job.chunks[i:i + self._MAX_JOB_CHUNKS] for i in range(0, len(job.chunks), self._MAX_JOB_CHUNKS)]
-                piece_states = [(o, l)] + [(torch.empty_like(o), torch.empty_like(l)) for _ in pieces[1:]]
-                pieced.append(piece_states)
-            else:
-                pieces, piece_states = [job.chunks], [(o, l)]
-            if segments is None:
-                for piece, st in zip(pieces, piece_states):
-                    job_lists.append([index[c] for c in piece])
-                    dests.append(st)
-            elif len(pieces) > 1:
+        # the local chunk is (key, value); the others come from the ring stand-in
+        needed, jobs, which = plan.launch
+        kv = [(key, value) if c == r else self.group.kv_chunk(c) for c in needed]
+        cu_q = cu_kv = dev_seg = None
+        if segments is not None:
+            if any(len(job) > self._MAX_JOB_CHUNKS for job in jobs):
                 raise NotImplementedError("variable-length calls with blocks of more than "
                                           f"{self._MAX_JOB_CHUNKS} chunks are not supported")
-            elif dev_seg is not None:
-                # one kernel job per segment; the kernel reads the segment's rows and keys from device memory
-                for i in range(dev_seg.n_seg):
-                    job_lists.append([index[c] for c in job.chunks])
-                    dests.append((o, l))
-                    job_segs.append(i)
+            if isinstance(segments, _DeviceSegmentSource):
+                dev_seg = segments.over(needed)
             else:
-                # one kernel job per segment: its query rows against its key rows of every chunk
                 cu_q, cu_kv_of = segments
-                for i in range(len(cu_q) - 1):
-                    job_lists.append([index[c] for c in job.chunks])
-                    dests.append((o, l))
-                    q_ranges.append((cu_q[i], cu_q[i + 1] - cu_q[i]))
-                    kv_ranges.append([(cu_kv_of(c)[i], cu_kv_of(c)[i + 1] - cu_kv_of(c)[i]) for c in job.chunks])
-            seen[job.chunks] = (o, l)
-            states.append((o, l))
-        if job_lists:
-            table = _hip.ChunkTable(ks, vs, B, _kernel_input)
-            if dev_seg is not None:
-                _hip.attn_jobs_fwd(query, table, job_lists, [d[0] for d in dests], [d[1] for d in dests],
-                                   workspace=_hip.attn_workspace(dev), q_prescaled=self.q_prescaled,
-                                   dev_segments=dev_seg.over(needed), job_segments=job_segs)
-            else:
-                _hip.attn_jobs_fwd(query, table, job_lists, [d[0] for d in dests], [d[1] for d in dests],
-                                   q_ranges=q_ranges, kv_ranges=kv_ranges, workspace=_hip.attn_workspace(dev),
-                                   q_prescaled=self.q_prescaled)
-        for piece_states in pieced:
-            _hip.merge_states([s[0] for s in piece_states], [s[1] for s in piece_states],
-                              dst_out=piece_states[0][0], dst_lse=piece_states[0][1])
-        for job, (o, l) in zip(plan.jobs, states):
+                cu_kv = [cu_kv_of(c) for c in needed]
+        states = _hip.attn_states(query, [k for k, _ in kv], [v for _, v in kv], jobs, self._MAX_JOB_CHUNKS,
+                                  _hip.attn_workspace(query.device), self.q_prescaled, cu_q, cu_kv, dev_seg, _kernel_input)
+        for job, i in zip(plan.jobs, which):
+            o, l = states[i]
             if job.store_slot is not None:
                 self.cache.store_block(job.store_slot, o, l)  # :207-211
             merge_outs.append(o)

@@ -11,8 +11,7 @@
 #include <ATen/ops/empty.h>
 #include <torch/csrc/utils/pybind.h>
 
-#include <cstdarg>
-#include <cstdio>
+#include <algorithm>
 #include <optional>
 #include <string>
 #include <utility>
@@ -305,6 +304,135 @@ void attn_jobs(const Tensor& q, const ChunkTable& table, const std::vector<std::
   }
 }
 
+Tensor new_out(const Dims& d, at::ScalarType dtype, const Tensor& like) {
+  return at::empty({d.B, d.S, d.H, d.D}, like.options().dtype(dtype));
+}
+Tensor new_lse(const Dims& d, bool bsh, const Tensor& like) {
+  const auto opt = like.options().dtype(at::kFloat);
+  return bsh ? at::empty({d.B, d.S, d.H, 1}, opt) : at::empty({d.B, d.H, d.S}, opt);
+}
+typedef std::vector<std::pair<Tensor, Tensor>> States;
+
+std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, std::optional<Tensor> dst_out,
+                                std::optional<Tensor> dst_lse, at::ScalarType dst_dtype, bool dst_bsh, uint64_t stream);
+
+// The fresh states (out in q's dtype, lse [B,H,Sq]) of q against the concatenations of the chunks jobs[j]
+// (ditango_amd._hip.attn_states): one launch, unless the jobs exceed its limits; a job of more than max_chunks chunks is
+// computed in pieces that are folded into its state.
+States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs,
+                   const std::vector<std::vector<int32_t>>& jobs, int64_t max_chunks, const std::optional<std::vector<int32_t>>& cu_q,
+                   const std::optional<std::vector<std::vector<int32_t>>>& cu_kv, const std::optional<Tensor>& workspace,
+                   int32_t flags, const Segments* seg, const py::object& convert, uint64_t stream) {
+  REQUIRE(q.dim() == 4, "q must be [B,S,H,D] with contiguous D");
+  const Dims d{q.size(0), q.size(1), q.size(2), q.size(3)};
+  const ChunkTable table(ks, vs, d.B, convert);
+  States states, pieces;
+  std::vector<std::vector<int32_t>> lists;
+  std::vector<Tensor> outs, lses;
+  std::vector<int32_t> segs;
+  std::vector<Range> q_ranges;
+  std::vector<std::vector<Range>> kv_ranges;
+  std::vector<std::pair<size_t, size_t>> folds;   // (first piece, number of pieces) of the states computed in pieces
+  const size_t n_seg = seg ? seg->n_seg() : cu_q ? cu_q->size() - 1 : 1;
+  REQUIRE(!cu_q || (cu_kv && cu_kv->size() == ks.size()), "one cu_seqlens_kv per chunk");
+  for (const auto& job : jobs) {
+    states.emplace_back(new_out(d, q.scalar_type(), q), new_lse(d, false, q));
+    const size_t first = pieces.size();
+    for (size_t at = 0; at == 0 || at < job.size(); at += max_chunks) {
+      pieces.push_back(at == 0 ? states.back() : std::make_pair(new_out(d, q.scalar_type(), q), new_lse(d, false, q)));
+      const std::vector<int32_t> piece(job.begin() + at, job.begin() + std::min(job.size(), at + (size_t)max_chunks));
+      for (size_t s = 0; s < n_seg; ++s) {   // a segment of a packed batch is a job of its own on the state's rows
+        lists.push_back(piece);
+        outs.push_back(pieces.back().first);
+        lses.push_back(pieces.back().second);
+        if (seg) segs.push_back((int32_t)s);
+        if (cu_q) {
+          q_ranges.emplace_back((*cu_q)[s], (*cu_q)[s + 1] - (*cu_q)[s]);
+          auto& r = kv_ranges.emplace_back();
+          for (int32_t c : piece) {
+            REQUIRE((*cu_kv)[c].size() == cu_q->size(), "cu_seqlens_kv must have as many entries as cu_seqlens_q");
+            r.emplace_back((*cu_kv)[c][s], (*cu_kv)[c][s + 1] - (*cu_kv)[c][s]);
+          }
+        }
+      }
+    }
+    if (pieces.size() - first > 1) folds.emplace_back(first, pieces.size() - first);
+  }
+  if (lists.empty()) return states;
+  attn_jobs(q, table, lists, outs, lses, 0.0, cu_q ? std::optional(std::move(q_ranges)) : std::nullopt,
+            cu_q ? std::optional(std::move(kv_ranges)) : std::nullopt, workspace, flags, false, seg,
+            seg ? std::optional(std::move(segs)) : std::nullopt, stream);
+  for (const auto& [first, n] : folds) {
+    std::vector<Tensor> o, l;
+    for (size_t i = 0; i < n; ++i) {
+      o.push_back(pieces[first + i].first);
+      l.push_back(pieces[first + i].second);
+    }
+    merge(o, l, o[0], l[0], q.scalar_type(), false, stream);
+  }
+  return states;
+}
+
+// The fp32 states of fp32 q against the concatenations of the fp32 chunks jobs[j] (ditango_amd._hip.attn_jobs_f32_fwd); every
+// chunk may have strides of its own.
+States attn_states_f32(const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs,
+                       const std::vector<std::vector<int32_t>>& jobs, double scale, uint64_t stream) {
+  auto check_f32 = [](const Tensor& t, const Name& name) {
+    REQUIRE(t.is_cuda() && t.scalar_type() == at::kFloat && t.dim() == 4 && t.stride(3) == 1, name.str(),
+            " must be fp32 [B,S,H,D] on the GPU with contiguous D");
+  };
+  check_f32(q, {"q"});
+  const Dims d{q.size(0), q.size(1), q.size(2), q.size(3)};
+  REQUIRE(ks.size() == vs.size(), "need as many V as K chunks");
+  for (size_t i = 0; i < ks.size(); ++i) {
+    check_f32(ks[i], {"k", (int64_t)i});
+    check_f32(vs[i], {"v", (int64_t)i});
+    REQUIRE(ks[i].sizes() == vs[i].sizes() && ks[i].size(0) == d.B && ks[i].size(2) == d.H && ks[i].size(3) == d.D, "k/v shape mismatch");
+    REQUIRE(ks[i].strides() == vs[i].strides(), "k and v must share strides");
+  }
+  States states;
+  for (size_t j = 0; j < jobs.size(); ++j) {
+    states.emplace_back(new_out(d, at::kFloat, q), new_lse(d, false, q));
+    for (int32_t c : jobs[j]) REQUIRE(c >= 0 && (size_t)c < ks.size(), "job ", std::to_string(j), " references a chunk outside the table");
+  }
+  for (size_t start = 0; start < jobs.size();) {
+    std::vector<int32_t> local(ks.size(), -1);
+    const float *kp[DT_MAX_CHUNKS], *vp[DT_MAX_CHUNKS];
+    int32_t lens[DT_MAX_CHUNKS], begin[DT_MAX_JOBS + 1], chunks[DT_MAX_JOB_ENTRIES];
+    int64_t sb[DT_MAX_CHUNKS], ss[DT_MAX_CHUNKS], sh[DT_MAX_CHUNKS];
+    float *op[DT_MAX_JOBS], *lp[DT_MAX_JOBS];
+    int32_t nc = 0, e = 0, n = 0;
+    begin[0] = 0;
+    for (; start + n < jobs.size() && n < DT_MAX_JOBS; ++n) {
+      const auto& job = jobs[start + n];
+      int32_t fresh = 0;
+      for (size_t i = 0; i < job.size(); ++i)
+        if (local[job[i]] < 0 && std::find(job.begin(), job.begin() + i, job[i]) == job.begin() + i) ++fresh;
+      if (nc + fresh > DT_MAX_CHUNKS || e + job.size() > DT_MAX_JOB_ENTRIES) break;
+      for (int32_t c : job) {
+        if (local[c] < 0) {
+          local[c] = nc;
+          kp[nc] = static_cast<const float*>(ptr(ks[c]));
+          vp[nc] = static_cast<const float*>(ptr(vs[c]));
+          lens[nc] = (int32_t)ks[c].size(1);
+          sb[nc] = ks[c].stride(0); ss[nc] = ks[c].stride(1); sh[nc] = ks[c].stride(2);
+          ++nc;
+        }
+        chunks[e++] = local[c];
+      }
+      begin[n + 1] = e;
+      op[n] = static_cast<float*>(ptr(states[start + n].first));
+      lp[n] = static_cast<float*>(ptr(states[start + n].second));
+    }
+    REQUIRE(n > 0, "job ", std::to_string(start), " references more chunks than one launch addresses: split it and merge the parts");
+    check(dt_attn_jobs_f32_fwd(static_cast<const float*>(ptr(q)), d.B, d.S, d.H, d.D, q.stride(0), q.stride(1), q.stride(2), nc, kp, vp,
+                               lens, sb, ss, sh, n, begin, chunks, op, lp, (float)scale, stream_of(stream)),
+          "dt_attn_jobs_f32_fwd");
+    start += n;
+  }
+  return states;
+}
+
 // Device-scheduled launch over a table that fits one launch (ditango_amd._hip.attn_sched_fwd).  The schedule is row `row`
 // of ids [rows, C] and counts [rows, 2] (or the tensors themselves, row 0).
 void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, const Tensor& count, int64_t row, int32_t max_jobs,
@@ -389,14 +517,6 @@ struct StateList {   // the states of one merge launch
           "dt_merge_states");
   }
 };
-
-Tensor new_out(const Dims& d, at::ScalarType dtype, const Tensor& like) {
-  return at::empty({d.B, d.S, d.H, d.D}, like.options().dtype(dtype));
-}
-Tensor new_lse(const Dims& d, bool bsh, const Tensor& like) {
-  const auto opt = like.options().dtype(at::kFloat);
-  return bsh ? at::empty({d.B, d.S, d.H, 1}, opt) : at::empty({d.B, d.H, d.S}, opt);
-}
 
 // N-way merge; more states than one launch folds run in rounds through a running fp32 state (ditango_amd._hip.merge_states).
 std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, std::optional<Tensor> dst_out,
@@ -520,6 +640,8 @@ PYBIND11_MODULE(_ditango_host, m) {
       });
   py::class_<Segments>(m, "Segments").def(py::init(&make_segments)).def_property_readonly("n_seg", &Segments::n_seg);
   m.def("attn_jobs", &attn_jobs);
+  m.def("attn_states", &attn_states);
+  m.def("attn_states_f32", &attn_states_f32);
   m.def("attn_sched", &attn_sched);
   m.def("merge", &merge);
   m.def("merge_arena", &merge_arena);
