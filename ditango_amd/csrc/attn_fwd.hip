@@ -48,6 +48,7 @@
 //     L2 stream the same K/V.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <mutex>
 #include <type_traits>
 
@@ -328,15 +329,15 @@ __device__ __forceinline__ bool view_job(Args& a, int job, JobView& v) {
       }
     }
   } else {
-    v.seg_begin = a.job_begin[job];
-    v.seg_end = a.job_begin[job + 1];
-    v.out = a.job_out[job];
-    v.lse = a.job_lse[job];
+    v.seg_begin = a.job[job].begin;
+    v.seg_end = a.job[job].end;
+    v.out = a.job[job].out;
+    v.lse = a.job[job].lse;
     if (a.cu_q != nullptr) {
-      v.dseg = a.job_q_begin[job];
+      v.dseg = a.job[job].q_begin;
     } else {
-      v.q_begin = a.job_q_begin[job];
-      v.q_end = v.q_begin + a.job_q_len[job];
+      v.q_begin = a.job[job].q_begin;
+      v.q_end = v.q_begin + a.job[job].q_len;
     }
   }
   if (v.dseg >= 0) {
@@ -353,6 +354,27 @@ __device__ __forceinline__ bool view_job(Args& a, int job, JobView& v) {
 // registers each): the second workgroup's wavefronts issue into the barrier waits, the start-up and
 // the epilogue of the first, which at 35 key tiles per work item are a tenth of its time (+10 %).
 constexpr int kWavesPerSimdD64 = 4;
+// Brings the cache lines of the arguments that a workgroup is about to read into the scalar cache, all at once: the
+// header, the first jobs, chunks and chunk references.  Read one after the other as the control flow gets to them, each
+// line is a cache miss of 0.5 us of its own when a launch starts (stamps of a launch of 4 heads x 512 queries: 2.9 us
+// for the argument reads in front of the first tile load, 1.4 with them prefetched; the launch against one key tile 9.5 -> 7.9 us at
+// D = 64, 10.3 -> 9.4 at D = 128, together with the wait for Q behind the first tile loads).  The loads and their wait are one asm statement, so no register is pending behind it.
+constexpr int kArgLine = 64;
+__device__ __forceinline__ void prefetch_args(uint64_t args) {
+  uint32_t t0, t1, t2, t3, t4, t5, t6, t7, t8, t9, t10, t11, t12, t13;
+  constexpr int kJob = (int)offsetof(AttnArgs, job), kChunk = (int)offsetof(AttnArgs, chunk), kEntry = (int)offsetof(AttnArgs, entry);
+  asm volatile(
+      "s_load_dword %0, %14, 0x0\n\ts_load_dword %1, %14, 0x40\n\ts_load_dword %2, %14, 0x80\n\ts_load_dword %3, %14, 0xc0\n\t"
+      "s_load_dword %4, %14, %15\n\ts_load_dword %5, %14, %16\n\ts_load_dword %6, %14, %17\n\ts_load_dword %7, %14, %18\n\t"
+      "s_load_dword %8, %14, %19\n\ts_load_dword %9, %14, %20\n\ts_load_dword %10, %14, %21\n\ts_load_dword %11, %14, %22\n\t"
+      "s_load_dword %12, %14, %23\n\ts_load_dword %13, %14, %24\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8), "=&s"(t9), "=&s"(t10),
+        "=&s"(t11), "=&s"(t12), "=&s"(t13)
+      : "s"(args), "i"(kJob), "i"(kJob + kArgLine), "i"(kJob + 2 * kArgLine), "i"(kJob + 3 * kArgLine), "i"(kChunk),
+        "i"(kChunk + kArgLine), "i"(kChunk + 2 * kArgLine), "i"(kChunk + 3 * kArgLine), "i"(kEntry), "i"(kEntry + kArgLine)
+      : "memory");
+}
+
 template <int D, bool kPre, bool kHalf>
 __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn_fwd_kernel(const AttnArgs args_by_value) {
   using T = Tile<D>;
@@ -368,8 +390,16 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   // never needed; with the tables indexed at run time from several branches it sometimes cannot, and every lane
   // then copies the whole struct into scratch memory before it starts (seven times the run time of a short launch).
   typedef const AttnArgs __attribute__((address_space(4))) KernArgs;
-  KernArgs& a = *(KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   (void)args_by_value;
+  prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+  // A reference of its own for every place that reads arguments, unrelated to the others as far as the compiler can see:
+  // it otherwise reads whole lines at the top and holds what later places need in 120 spilled scalar registers.
+  auto args = []() __attribute__((always_inline)) -> KernArgs& {
+    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(KernArgs*)p;
+  };
+  KernArgs& a = args();
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   // ---- which (job, batch, head, query tile) ------------------------------------------
@@ -403,25 +433,27 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   const int seg_begin = view.seg_begin, seg_end = view.seg_end, single = view.single;
   const int q_begin = view.q_begin, q_end = view.q_end, vseg = view.vseg, dseg = view.dseg;
   if (qt * kBQ >= q_end - q_begin) return;  // the grid is sized for the longest job / segment
-  auto chunk_of = [&](int seg) __attribute__((always_inline)) -> int { return single >= 0 ? single : a.job_chunks[seg]; };
+  auto chunk_of = [&](int seg) __attribute__((always_inline)) -> int { return single >= 0 ? single : args().entry[seg].chunk; };
   // keys [begin, begin + len) of chunk reference `seg`
   auto kv_begin_of = [&](int seg) __attribute__((always_inline)) -> int {
+    KernArgs& a = args();
     if (dseg >= 0) {
       const int cid = chunk_of(seg);
-      return min(max(boundary(a.cu_kv[cid], dseg), 0), a.kv_len[cid]);
+      return min(max(boundary(a.cu_kv[cid], dseg), 0), a.chunk[cid].len);
     }
-    if (single < 0) return a.entry_kv_begin[seg];
-    return vseg >= 0 ? a.entry_kv_begin[single * a.n_seg + vseg] : 0;
+    if (single < 0) return a.entry[seg].kv_begin;
+    return vseg >= 0 ? a.entry[single * a.n_seg + vseg].kv_begin : 0;
   };
   auto kv_len_of = [&](int seg) __attribute__((always_inline)) -> int {
+    KernArgs& a = args();
     if (dseg >= 0) {
       const int cid = chunk_of(seg);
-      const int lo = min(max(boundary(a.cu_kv[cid], dseg), 0), a.kv_len[cid]);
-      const int hi = min(max(boundary(a.cu_kv[cid], dseg + 1), lo), a.kv_len[cid]);
+      const int lo = min(max(boundary(a.cu_kv[cid], dseg), 0), a.chunk[cid].len);
+      const int hi = min(max(boundary(a.cu_kv[cid], dseg + 1), lo), a.chunk[cid].len);
       return hi - lo;
     }
-    if (single < 0) return a.entry_kv_len[seg];
-    return vseg >= 0 ? a.entry_kv_len[single * a.n_seg + vseg] : a.kv_len[single];
+    if (single < 0) return a.entry[seg].kv_len;
+    return vseg >= 0 ? a.entry[single * a.n_seg + vseg].kv_len : a.chunk[single].len;
   };
 
   const int tid = threadIdx.x;
@@ -441,13 +473,6 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) qf[s] = *reinterpret_cast<const ex8*>(qp + 16 * s);
   }
-  // Route the fragments through an empty asm: they are then defined by it, not by loads.  The
-  // compiler otherwise keeps "Q may still be in flight" alive round the loop and waits for ALL
-  // outstanding vector-memory loads (including the K/V prefetch just issued) before the first
-  // MFMA that reads Q in every iteration.
-#pragma unroll
-  for (int s = 0; s < D / 16; ++s) asm volatile("" : "+v"(qf[s]));
-
   // ---- tile bookkeeping -----------------------------------------------------------------
   int n_tiles = 0;
   for (int s = seg_begin; s < seg_end; ++s) n_tiles += (kv_len_of(s) + kBK - 1) / kBK;
@@ -470,12 +495,13 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     k_off = 0u;
     if (ld_seg < seg_end) {
       const int cid = chunk_of(ld_seg);
+      KernArgs& a = args();
       const int64_t head_off =
-          (int64_t)b * a.kv_sb[cid] + (int64_t)h * a.kv_sh + (int64_t)kv_begin_of(ld_seg) * a.kv_ss;
+          (int64_t)b * a.chunk[cid].sb + (int64_t)h * a.kv_sh + (int64_t)kv_begin_of(ld_seg) * a.kv_ss;
       ld_left = kv_len_of(ld_seg);
       const uint32_t valid = (uint32_t)(ld_left - 1) * row_bytes + (uint32_t)(D * 2);
-      rk = make_rsrc(a.k[cid] + head_off, valid);
-      rv = make_rsrc(a.v[cid] + head_off, valid);
+      rk = make_rsrc(a.chunk[cid].k + head_off, valid);
+      rv = make_rsrc(a.chunk[cid].v + head_off, valid);
     } else {
       // past the last chunk: an empty descriptor, loads store zeros without touching memory
       rk = make_rsrc(nullptr, 0u);
@@ -739,6 +765,12 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
 #pragma unroll
     for (int y = DT_SCHED_PROLOGUE_CALLS_LEADING; y < DT_SCHED_PROLOGUE_CALLS_TRAILING; ++y) load_tile(y);
   }
+  // Route the fragments through an empty asm: they are then defined by it, not by loads.  The
+  // compiler otherwise keeps "Q may still be in flight" alive round the loop and waits for ALL
+  // outstanding vector-memory loads (including the K/V prefetch just issued) before the first
+  // MFMA that reads Q in every iteration.  (Here, behind the first tile loads: Q and the tiles arrive together.)
+#pragma unroll
+  for (int s = 0; s < D / 16; ++s) asm volatile("" : "+v"(qf[s]));
   // in flight behind this wait: K of tile 1 and the calls after it (kLoads + 2 kLoads (1 + g) loads)
   if (group == 0) wait_tile_loads<DT_SCHED_PROLOGUE_INFLIGHT_LEADING * T::kLoads>();
   else wait_tile_loads<DT_SCHED_PROLOGUE_INFLIGHT_TRAILING * T::kLoads>();
@@ -911,11 +943,12 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   const float lse = l_tot > 0.f ? (m_ref * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : -INFINITY;
   const int qrow = q0 + col;
+  KernArgs& e = args();
   if (is_part) {
     // A part's state goes to the workspace as it lies in the registers, in fp32: whole kilobytes per store, no rounding.
-    const int64_t slot = ((int64_t)unit * kXcds + xcd) * a.part_ways + part;
-    if (hh == 0) a.ws_lse[slot * kBQ + wave * 32 + col] = lse;
-    float* dst = a.ws_out + (slot * kWaves + wave) * (32 * D) + lane * 4;
+    const int64_t slot = ((int64_t)unit * kXcds + xcd) * e.part_ways + part;
+    if (hh == 0) e.ws_lse[slot * kBQ + wave * 32 + col] = lse;
+    float* dst = e.ws_out + (slot * kWaves + wave) * (32 * D) + lane * 4;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -927,7 +960,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
       }
     return;
   }
-  if (hh == 0 && qrow < q_end) view.lse[((int64_t)b * a.H + h) * a.Sq + qrow] = lse;
+  if (hh == 0 && qrow < q_end) view.lse[((int64_t)b * e.H + h) * e.Sq + qrow] = lse;
 
   // O^T (registers, [d][query]) -> LDS [query][d] in the element type -> coalesced 16-byte stores.
   phase_barrier();  // every wavefront is done with the tile buffers
@@ -959,7 +992,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     const int qg = q0 + row;
     const u32x4 val = *reinterpret_cast<const u32x4*>(ol + row * T::kPitchO + cc * 16);
     if (qg < q_end) {
-      uint16_t* dst = view.out + (((int64_t)b * a.Sq + qg) * a.H + h) * D + cc * 8;
+      uint16_t* dst = view.out + (((int64_t)b * e.Sq + qg) * e.H + h) * D + cc * 8;
       __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
     }
   }
@@ -976,6 +1009,7 @@ __global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const Attn
   typedef const AttnArgs __attribute__((address_space(4))) KernArgs;
   KernArgs& a = *(KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   (void)args_by_value;
+  prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
   typedef typename Elem<kHalf>::x2 ex2;
   typedef typename Elem<kHalf>::x4 ex4;
   constexpr int kHalves = D / 64;
@@ -1167,18 +1201,11 @@ static void order_jobs(AttnArgs& a, int n_jobs, JobSize* size) {
   for (int j = 0; j < n_jobs; ++j) {
     const int from = order[j];
     size[j] = was[from];
-    a.job_out[j] = o.job_out[from];
-    a.job_lse[j] = o.job_lse[from];
-    a.job_q_begin[j] = o.job_q_begin[from];
-    a.job_q_len[j] = o.job_q_len[from];
-    a.job_begin[j] = e;
-    for (int x = o.job_begin[from]; x < o.job_begin[from + 1]; ++x, ++e) {
-      a.job_chunks[e] = o.job_chunks[x];
-      a.entry_kv_begin[e] = o.entry_kv_begin[x];
-      a.entry_kv_len[e] = o.entry_kv_len[x];
-    }
+    a.job[j] = o.job[from];
+    a.job[j].begin = e;
+    for (int x = o.job[from].begin; x < o.job[from].end; ++x, ++e) a.entry[e] = o.entry[x];
+    a.job[j].end = e;
   }
-  a.job_begin[n_jobs] = e;
 }
 
 // Sizes of the launch's jobs.  Device-listed jobs count as the longest chunk.  Where the boundaries are in device memory
@@ -1188,17 +1215,17 @@ static void job_sizes(const AttnArgs& a, int n_jobs, JobSize* size) {
   auto tiles_of = [](int keys) { return (keys + kBK - 1) / kBK; };
   const int rows_first = std::min(a.nqt * kBQ, a.Sq), rows_other = std::max(0, std::min(rows_first, a.Sq - rows_first));
   int longest = 0;
-  for (int c = 0; c < a.n_chunks; ++c) longest = std::max(longest, tiles_of(a.kv_len[c]));
+  for (int c = 0; c < a.n_chunks; ++c) longest = std::max(longest, tiles_of(a.chunk[c].len));
   for (int j = 0; j < n_jobs; ++j) {
     const bool listed = a.dev_ids == nullptr;
-    int seg = listed ? a.job_q_begin[j] : a.n_seg > 0 ? a.n_seg - 1 - j / a.n_slots : -1;
+    int seg = listed ? a.job[j].q_begin : a.n_seg > 0 ? a.n_seg - 1 - j / a.n_slots : -1;
     size[j].tiles = 0;
     if (!listed) size[j].tiles = longest;
     else
-      for (int e = a.job_begin[j]; e < a.job_begin[j + 1]; ++e)
-        size[j].tiles += tiles_of(a.cu_q ? a.kv_len[a.job_chunks[e]] : a.entry_kv_len[e]);
+      for (int e = a.job[j].begin; e < a.job[j].end; ++e)
+        size[j].tiles += tiles_of(a.cu_q ? a.chunk[a.entry[e].chunk].len : a.entry[e].kv_len);
     if (a.cu_q) size[j].rows = seg == 0 ? rows_first : rows_other;
-    else if (listed) size[j].rows = a.job_q_len[j];
+    else if (listed) size[j].rows = a.job[j].q_len;
     else size[j].rows = seg >= 0 ? a.seg_q_len[seg] : a.Sq;
   }
 }

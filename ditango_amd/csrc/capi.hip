@@ -87,10 +87,10 @@ static int fill_common(AttnArgs& a, const void* q, int32_t B, int32_t Sq, int32_
       set_error("chunk %d: one (batch, head) plane spans 2 GiB or more; split the chunk", i);
       return DT_ERR_INVALID;
     }
-    a.k[i] = static_cast<const uint16_t*>(k_ptrs[i]);
-    a.v[i] = static_cast<const uint16_t*>(v_ptrs[i]);
-    a.kv_len[i] = kv_lens[i];
-    a.kv_sb[i] = kv_sb[i];
+    a.chunk[i].k = static_cast<const uint16_t*>(k_ptrs[i]);
+    a.chunk[i].v = static_cast<const uint16_t*>(v_ptrs[i]);
+    a.chunk[i].len = kv_lens[i];
+    a.chunk[i].sb = kv_sb[i];
   }
   a.n_chunks = n_chunks;
   a.kv_ss = kv_ss;
@@ -160,20 +160,20 @@ extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int
       set_error("job %d: null or misaligned destination", j);
       return DT_ERR_INVALID;
     }
-    a.job_out[j] = static_cast<uint16_t*>(out_ptrs[j]);
-    a.job_lse[j] = lse_ptrs[j];
-    a.job_begin[j] = job_begin[j];
+    a.job[j].out = static_cast<uint16_t*>(out_ptrs[j]);
+    a.job[j].lse = lse_ptrs[j];
+    a.job[j].begin = job_begin[j];
+    a.job[j].end = job_begin[j + 1];
     const int32_t qb = job_q_begin ? job_q_begin[j] : 0;
     const int32_t ql = job_q_len ? job_q_len[j] : Sq;
     if (qb < 0 || ql < 0 || (int64_t)qb + ql > Sq) {
       set_error("job %d: query rows [%d, %d) outside [0, %d)", j, qb, qb + ql, Sq);
       return DT_ERR_INVALID;
     }
-    a.job_q_begin[j] = qb;
-    a.job_q_len[j] = ql;
+    a.job[j].q_begin = qb;
+    a.job[j].q_len = ql;
     longest = ql > longest ? ql : longest;
   }
-  a.job_begin[n_jobs] = job_begin[n_jobs];
   for (int e = 0; e < job_begin[n_jobs]; ++e) {
     const int32_t c = job_chunks[e];
     if (c < 0 || c >= n_chunks) {
@@ -186,9 +186,9 @@ extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int
       set_error("chunk reference %d: keys [%d, %d) outside chunk %d of length %d", e, kb, kb + kl, c, kv_lens[c]);
       return DT_ERR_INVALID;
     }
-    a.job_chunks[e] = c;
-    a.entry_kv_begin[e] = kb;
-    a.entry_kv_len[e] = kl;
+    a.entry[e].chunk = c;
+    a.entry[e].kv_begin = kb;
+    a.entry[e].kv_len = kl;
   }
   // size the grid for the longest job; shorter jobs leave their surplus workgroups at once
   a.nqt = (longest + 255) / 256;
@@ -268,20 +268,20 @@ extern "C" int dt_attn_varlen_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, 
       set_error("job %d: segment %d outside 0..%d", j, job_segment[j], n_seg - 1);
       return DT_ERR_INVALID;
     }
-    a.job_out[j] = static_cast<uint16_t*>(out_ptrs[j]);
-    a.job_lse[j] = lse_ptrs[j];
-    a.job_begin[j] = job_begin[j];
-    a.job_q_begin[j] = job_segment[j];   // with device boundaries this field names the segment
-    a.job_q_len[j] = 0;
+    a.job[j].out = static_cast<uint16_t*>(out_ptrs[j]);
+    a.job[j].lse = lse_ptrs[j];
+    a.job[j].begin = job_begin[j];
+    a.job[j].end = job_begin[j + 1];
+    a.job[j].q_begin = job_segment[j];   // with device boundaries this field names the segment
+    a.job[j].q_len = 0;
   }
-  a.job_begin[n_jobs] = job_begin[n_jobs];
   for (int e = 0; e < job_begin[n_jobs]; ++e) {
     const int32_t c = job_chunks[e];
     if (c < 0 || c >= n_chunks) {
       set_error("job chunk reference %d is outside the chunk table", c);
       return DT_ERR_INVALID;
     }
-    a.job_chunks[e] = c;
+    a.entry[e].chunk = c;
   }
   return launch_attn(a, D, n_jobs, (hipStream_t)stream, workspace, workspace_bytes);
 }
@@ -467,8 +467,8 @@ extern "C" int dt_attn_sched_seg_ws_fwd(const void* q, int32_t B, int32_t Sq, in
           set_error("segment %d: keys [%d, %d) outside chunk %d of length %d", s, kb, kb + kl, c, kv_lens[c]);
           return DT_ERR_INVALID;
         }
-        a.entry_kv_begin[e] = kb;
-        a.entry_kv_len[e] = kl;
+        a.entry[e].kv_begin = kb;
+        a.entry[e].kv_len = kl;
       }
     a.n_seg = n_seg;
     a.n_slots = max_jobs;

@@ -9,62 +9,40 @@ namespace dt {
 void set_error(const char* fmt, ...);
 int hip_fail(hipError_t e, const char* what);
 
+// One KV chunk, one reference of a job to a chunk, one job of an attention launch: a record each, so that a workgroup finds
+// what it needs in one or two cache lines.
+struct AttnChunk {
+  const uint16_t* k;
+  const uint16_t* v;
+  int64_t sb;       // batch stride, elements
+  int32_t len;      // keys
+  int32_t unused;
+};
+struct AttnEntry {
+  int32_t chunk;
+  int32_t kv_begin, kv_len;   // keys [kv_begin, kv_begin + kv_len) of the chunk
+};
+struct AttnJob {
+  uint16_t* out;
+  float* lse;
+  int32_t begin, end;         // chunk references
+  // query rows [q_begin, q_begin + q_len): a segment of a packed variable-length batch is a job on sub-ranges (with
+  // boundaries in device memory q_begin names the segment)
+  int32_t q_begin, q_len;
+};
+
 // Kernel arguments of the chunk-attention kernel.  Passed by value, so the
 // chunk and job tables travel in the kernarg segment: no device-side table,
-// no host-to-device copy per call.
+// no host-to-device copy per call.  q, K, V and the output states are 16-bit elements: bfloat16, or IEEE half when
+// elem_f16 is set.
 struct AttnArgs {
-  // q, K, V and the output states are 16-bit elements: bfloat16, or IEEE half when elem_f16 is set
+  // ---- what every workgroup reads: the first three cache lines
   const uint16_t* q;
   int64_t q_sb, q_ss, q_sh;
-  int32_t B, H, Sq;
+  int32_t H, Sq;
   int32_t nqt;        // query tiles per (batch, head)
   int32_t total;      // B*H*nqt work items per job
   int32_t per_xcd;    // work items handed to each of the 8 XCDs
-  float scale_log2;   // softmax scale * log2(e)
-  int32_t q_prescaled;  // the caller folded scale_log2 into q: scores are already in log2 units
-  int32_t elem_f16;     // the 16-bit tensors are IEEE half instead of bfloat16
-  // chunk table
-  int32_t n_chunks;
-  const uint16_t* k[DT_MAX_CHUNKS];
-  const uint16_t* v[DT_MAX_CHUNKS];
-  int64_t kv_sb[DT_MAX_CHUNKS];
-  int32_t kv_len[DT_MAX_CHUNKS];
-  int64_t kv_ss, kv_sh;
-  // host-listed jobs
-  uint16_t* job_out[DT_MAX_JOBS];
-  float* job_lse[DT_MAX_JOBS];
-  int32_t job_begin[DT_MAX_JOBS + 1];
-  int32_t job_chunks[DT_MAX_JOB_ENTRIES];
-  // query rows [job_q_begin, job_q_begin + job_q_len) of each job; keys [kv_begin, kv_begin + kv_len)
-  // of each chunk reference (a segment of a packed variable-length batch is a job on sub-ranges)
-  int32_t job_q_begin[DT_MAX_JOBS];
-  int32_t job_q_len[DT_MAX_JOBS];
-  int32_t entry_kv_begin[DT_MAX_JOB_ENTRIES];
-  int32_t entry_kv_len[DT_MAX_JOB_ENTRIES];
-  // device-listed jobs (dev_ids != nullptr): job j computes chunk dev_ids[j] if j < *dev_count
-  const int32_t* dev_ids;
-  const int32_t* dev_count;
-  uint16_t* slot_out;
-  float* slot_lse;
-  int64_t slot_out_stride, slot_lse_stride;
-  int32_t diag;
-  uint16_t* diag_out;
-  float* diag_lse;
-  // device-listed jobs on a packed variable-length batch (n_seg > 0): launch job j is segment
-  // j % n_seg of the chunk listed at j / n_seg; the keys of segment s inside chunk c are
-  // entry_kv_begin/len[c * n_seg + s]
-  int32_t n_seg;
-  int32_t seg_q_begin[DT_MAX_SEGMENTS];
-  int32_t seg_q_len[DT_MAX_SEGMENTS];
-  // Segment boundaries that live in DEVICE memory (cu_q != nullptr), the calling convention of
-  // flash_attn_varlen_func: cu_q[s], cu_q[s + 1] bound the query rows of segment s and cu_kv[c][s],
-  // cu_kv[c][s + 1] its keys inside chunk c (every chunk brings its own boundaries).  The host never
-  // reads them; the kernel clamps them to the tensors' extents.  A host-listed job then names its
-  // segment in job_q_begin[job]; a device-listed job is segment job % n_seg as above.
-  const int32_t* cu_q;
-  const int32_t* cu_kv[DT_MAX_CHUNKS];
-  // device-listed jobs come segment-major, the first segment last: launch job j is slot j % n_slots of the schedule
-  int32_t n_slots;
   // Tail balancing (workspace launches only).  The work items of a launch, in dispatch order: those of an XCD are
   // numbered flat = job * per_xcd + idx (idx: position in the XCD's share of the job).  Items with flat < tail_start run
   // as one workgroup each; the tail_items behind them run as part_ways workgroups over disjoint ranges of key
@@ -74,8 +52,41 @@ struct AttnArgs {
   int32_t tail_start;  // INT32_MAX: nothing is split
   int32_t tail_items;  // per XCD
   int32_t part_ways;
+  int32_t n_chunks;
+  int32_t n_seg;
+  float scale_log2;    // softmax scale * log2(e)
+  int64_t kv_ss, kv_sh;
+  // Device-listed jobs (dev_ids != nullptr): job j computes chunk dev_ids[j] if j < *dev_count.  On a packed
+  // variable-length batch (n_seg > 0) they come segment-major, the first segment last: launch job j is slot
+  // j % n_slots of the schedule, and the keys of segment s inside chunk c are those of entry[c * n_seg + s].
+  const int32_t* dev_ids;
+  const int32_t* dev_count;
+  // Segment boundaries that live in DEVICE memory (cu_q != nullptr), the calling convention of
+  // flash_attn_varlen_func: cu_q[s], cu_q[s + 1] bound the query rows of segment s and cu_kv[c][s],
+  // cu_kv[c][s + 1] its keys inside chunk c (every chunk brings its own boundaries).  The host never
+  // reads them; the kernel clamps them to the tensors' extents.
+  const int32_t* cu_q;
+  int32_t n_slots;
+  int32_t diag;
+  uint16_t* slot_out;
+  float* slot_lse;
+  int64_t slot_out_stride, slot_lse_stride;
+  uint16_t* diag_out;
+  float* diag_lse;
   float* ws_out;    // [slot][8 wavefronts][D / 8 groups of 4 elements][64 lanes][4], the accumulators as they lie in registers
   float* ws_lse;    // [slot][256]
+  // ---- the host's own
+  int32_t B;
+  int32_t q_prescaled;  // the caller folded scale_log2 into q: scores are already in log2 units
+  int32_t elem_f16;     // the 16-bit tensors are IEEE half instead of bfloat16
+  int32_t unused;
+  // ---- tables
+  AttnJob job[DT_MAX_JOBS];
+  AttnChunk chunk[DT_MAX_CHUNKS];
+  AttnEntry entry[DT_MAX_JOB_ENTRIES];
+  int32_t seg_q_begin[DT_MAX_SEGMENTS];
+  int32_t seg_q_len[DT_MAX_SEGMENTS];
+  const int32_t* cu_kv[DT_MAX_CHUNKS];
 };
 
 // Dynamic LDS of one attention workgroup by head dimension (four 64-key buffers per operand).  The
