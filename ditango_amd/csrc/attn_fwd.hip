@@ -213,12 +213,13 @@ struct Tile {
   static constexpr int kBlocks = kBytesK / 1024;      // direct-load instructions per tile and operand
   static constexpr int kLoads = kBlocks / kWaves;     // ... per wavefront (2 or 1)
   static constexpr int kRowsPerBlock = 1024 / kRowBytes;
-  static constexpr int kPitchO = D * 2 + 16;          // epilogue row pitch
   static constexpr int kLdsTiles = kNumBuf * (kBytesK + kBytesV);
-  static constexpr int kLdsEpilogue = kWaves * 32 * kPitchO;
-  static constexpr int kLdsBytes = kLdsTiles > kLdsEpilogue ? kLdsTiles : kLdsEpilogue;
+  static constexpr int kStageBytes = 32 * D;          // epilogue: 32 rows x half the columns of a wavefront's output
+  static constexpr int kLdsBytes = kLdsTiles + kWaves * kStageBytes;   // all of a CU's 160 KB: one workgroup at 128, two at 64
   static_assert(D == 128 || D == 64, "swizzles are written for these two head dimensions");
   __device__ static constexpr int swz_k(int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); }
+  // staging rows are written 8 bytes per lane, 32 rows side by side: 16 of them in distinct banks
+  __device__ static constexpr int swz_o(int row) { return D == 128 ? ((row >> 1) & 7) : ((row >> 2) & 3); }
   __device__ static constexpr int swz_v(int row) { return D == 128 ? (row & 3) : ((row >> 1) & 1); }
 };
 
@@ -433,27 +434,33 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   const int seg_begin = view.seg_begin, seg_end = view.seg_end, single = view.single;
   const int q_begin = view.q_begin, q_end = view.q_end, vseg = view.vseg, dseg = view.dseg;
   if (qt * kBQ >= q_end - q_begin) return;  // the grid is sized for the longest job / segment
-  auto chunk_of = [&](int seg) __attribute__((always_inline)) -> int { return single >= 0 ? single : args().entry[seg].chunk; };
-  // keys [begin, begin + len) of chunk reference `seg`
-  auto kv_begin_of = [&](int seg) __attribute__((always_inline)) -> int {
-    KernArgs& a = args();
-    if (dseg >= 0) {
-      const int cid = chunk_of(seg);
-      return min(max(boundary(a.cu_kv[cid], dseg), 0), a.chunk[cid].len);
-    }
-    if (single < 0) return a.entry[seg].kv_begin;
-    return vseg >= 0 ? a.entry[single * a.n_seg + vseg].kv_begin : 0;
+  // chunk reference `seg`: keys [begin, begin + len) of chunk cid
+  struct Ref {
+    int cid, begin, len;
   };
-  auto kv_len_of = [&](int seg) __attribute__((always_inline)) -> int {
+  auto ref_at = [&](int seg) __attribute__((always_inline)) -> Ref {
     KernArgs& a = args();
-    if (dseg >= 0) {
-      const int cid = chunk_of(seg);
-      const int lo = min(max(boundary(a.cu_kv[cid], dseg), 0), a.chunk[cid].len);
-      const int hi = min(max(boundary(a.cu_kv[cid], dseg + 1), lo), a.chunk[cid].len);
-      return hi - lo;
+    Ref r;
+    if (single < 0) {
+      r.cid = a.entry[seg].chunk;
+      r.begin = a.entry[seg].kv_begin;
+      r.len = a.entry[seg].kv_len;
+    } else {
+      r.cid = single;
+      r.begin = 0;
+      if (vseg >= 0) {
+        r.begin = a.entry[single * a.n_seg + vseg].kv_begin;
+        r.len = a.entry[single * a.n_seg + vseg].kv_len;
+      } else {
+        r.len = a.chunk[single].len;
+      }
     }
-    if (single < 0) return a.entry[seg].kv_len;
-    return vseg >= 0 ? a.entry[single * a.n_seg + vseg].kv_len : a.chunk[single].len;
+    if (dseg >= 0) {
+      const int keys = a.chunk[r.cid].len;
+      r.begin = min(max(boundary(a.cu_kv[r.cid], dseg), 0), keys);
+      r.len = min(max(boundary(a.cu_kv[r.cid], dseg + 1), r.begin), keys) - r.begin;
+    }
+    return r;
   };
 
   const int tid = threadIdx.x;
@@ -474,46 +481,57 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     for (int s = 0; s < D / 16; ++s) qf[s] = *reinterpret_cast<const ex8*>(qp + 16 * s);
   }
   // ---- tile bookkeeping -----------------------------------------------------------------
-  int n_tiles = 0;
-  for (int s = seg_begin; s < seg_end; ++s) n_tiles += (kv_len_of(s) + kBK - 1) / kBK;
-
   // Two cursors walk the job's chunks tile by tile, all in scalar registers: the load cursor
   // (ahead of the compute cursor: base pointers of the tile and keys left in its chunk) and
   // the compute cursor (keys left in the chunk of the tile whose scores are being computed).
-  int ld_seg = seg_begin - 1, ld_left = 0;
-  int cp_seg = seg_begin - 1, cp_left = 0;
   // The load cursor addresses a tile as (buffer descriptor of its chunk, byte offset of its first key from the
   // chunk's first key).  The descriptors (base of the chunk's keys for this batch and head, number of valid
   // bytes) only change with the chunk; per tile the cursor moves one scalar offset.  A chunk's (batch, head)
   // plane is below 2 GiB (checked on the host), so offsets fit 32 bits with room for the lane's part.
   const uint32_t row_bytes = (uint32_t)a.kv_ss * 2u;
   const uint32_t tile_bytes = (uint32_t)kBK * row_bytes;
-  u32x4 rk = make_rsrc(nullptr, 0u), rv = rk;   // K and V of the chunk under the load cursor
+  u32x4 rk, rv;   // K and V of the chunk under the load cursor
   uint32_t k_off = 0u;
-  auto ld_next_chunk = [&]() __attribute__((always_inline)) {
-    do { ++ld_seg; } while (ld_seg < seg_end && kv_len_of(ld_seg) == 0);
+  int ld_seg = seg_begin, ld_left = 0;
+  int cp_seg = seg_begin, cp_left = 0;
+  auto ld_open = [&](const Ref& r) __attribute__((always_inline)) {
     k_off = 0u;
-    if (ld_seg < seg_end) {
-      const int cid = chunk_of(ld_seg);
+    ld_left = r.len;
+    if (r.len > 0) {
       KernArgs& a = args();
-      const int64_t head_off =
-          (int64_t)b * a.chunk[cid].sb + (int64_t)h * a.kv_sh + (int64_t)kv_begin_of(ld_seg) * a.kv_ss;
-      ld_left = kv_len_of(ld_seg);
-      const uint32_t valid = (uint32_t)(ld_left - 1) * row_bytes + (uint32_t)(D * 2);
-      rk = make_rsrc(a.chunk[cid].k + head_off, valid);
-      rv = make_rsrc(a.chunk[cid].v + head_off, valid);
+      const int64_t head_off = (int64_t)b * a.chunk[r.cid].sb + (int64_t)h * a.kv_sh + (int64_t)r.begin * a.kv_ss;
+      const uint32_t valid = (uint32_t)(r.len - 1) * row_bytes + (uint32_t)(D * 2);
+      rk = make_rsrc(a.chunk[r.cid].k + head_off, valid);
+      rv = make_rsrc(a.chunk[r.cid].v + head_off, valid);
     } else {
       // past the last chunk: an empty descriptor, loads store zeros without touching memory
       rk = make_rsrc(nullptr, 0u);
       rv = rk;
     }
   };
-  auto cp_next_chunk = [&]() __attribute__((always_inline)) {
-    do { ++cp_seg; } while (cp_seg < seg_end && kv_len_of(cp_seg) == 0);
-    if (cp_seg < seg_end) cp_left = kv_len_of(cp_seg);
+  auto ld_next_chunk = [&]() __attribute__((always_inline)) {
+    Ref r;
+    r.len = 0;
+    while (r.len == 0 && ++ld_seg < seg_end) r = ref_at(ld_seg);
+    ld_open(r);
   };
-  ld_next_chunk();
-  cp_next_chunk();
+  auto cp_next_chunk = [&]() __attribute__((always_inline)) {
+    cp_left = 0;
+    while (cp_left == 0 && ++cp_seg < seg_end) cp_left = ref_at(cp_seg).len;
+  };
+  // the first reference opens both cursors (most jobs have no other)
+  Ref first;
+  first.len = 0;
+  if (seg_begin < seg_end) first = ref_at(seg_begin);
+  int n_tiles = (first.len + kBK - 1) / kBK;
+  for (int s = seg_begin + 1; s < seg_end; ++s) n_tiles += (ref_at(s).len + kBK - 1) / kBK;
+  if (__builtin_expect(first.len > 0, 1)) {
+    ld_open(first);
+    cp_left = first.len;
+  } else {
+    ld_next_chunk();
+    cp_next_chunk();
+  }
   if (is_part) {
     // this workgroup covers key tiles [t0, t1) of the item: walk both cursors to t0
     const int t0 = (int)((int64_t)n_tiles * part / a.part_ways);
@@ -793,7 +811,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   phase_barrier_after_matrix(s_acc, o_acc);
 
   // one iteration = vector phase of tile t, then matrix phase (P V of tile t, scores of t+1)
-  auto iteration = [&](int t, auto u_tag) __attribute__((always_inline)) {
+  auto iteration = [&](int t, auto u_tag) __attribute__((always_inline)) -> bool {
     constexpr int kU = decltype(u_tag)::value;  // t & 3
     // ======== vector phase: tile loads for later, online softmax of tile t ========
     // The vector phase runs at raised wave priority: where the two wavefronts of a SIMD compete for
@@ -919,24 +937,20 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     cp_valid = t + 1 < n_tiles ? cp_left : 0;
     cp_left -= kBK;
     if (cp_left <= 0) cp_next_chunk();
+    if (__builtin_expect(t + 1 >= n_tiles, 0)) return false;
     phase_barrier_after_matrix(s_acc, o_acc);
+    return true;
   };
   // Iterations come in fours (one per LDS buffer, so that buffer offsets are immediates); the last
   // round stops after the last tile.
-  for (int t = 0; t < n_tiles; t += 4) {
-    iteration(t, U0{});
-    if (t + 1 >= n_tiles) break;
-    iteration(t + 1, U1{});
-    if (t + 2 >= n_tiles) break;
-    iteration(t + 2, U2{});
-    if (t + 3 >= n_tiles) break;
-    iteration(t + 3, U3{});
-  }
-  // tile loads issued for tiles past the end are still on their way (they store zeros): let them
-  // land before the epilogue reuses the tile buffers
+  for (int t = 0; t < n_tiles; t += 4)
+    if (!iteration(t, U0{}) || !iteration(t + 1, U1{}) || !iteration(t + 2, U2{}) || !iteration(t + 3, U3{})) break;
+  // The trailing group waits for the end of the leading group's last matrix phase; its own is the last thing that
+  // happens to the tile buffers, nobody waits for it.  (Without a tile the trailing group is one barrier ahead.)
+  if (group == 0) phase_barrier_after_matrix(s_acc, o_acc);
+  // tile loads issued for tiles past the end are still on their way (they store zeros): let them land before the
+  // workgroup ends and its LDS becomes another's
   wait_tile_loads<0>();
-  // the leading group waits out the phase it is ahead
-  if (group == 0) phase_barrier();
 
   // ---- epilogue -------------------------------------------------------------------------
   const float l_tot = l_run + __shfl_xor(l_run, 32);
@@ -962,38 +976,40 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   }
   if (hh == 0 && qrow < q_end) view.lse[((int64_t)b * e.H + h) * e.Sq + qrow] = lse;
 
-  // O^T (registers, [d][query]) -> LDS [query][d] in the element type -> coalesced 16-byte stores.
-  phase_barrier();  // every wavefront is done with the tile buffers
-  uint8_t* ol = lds + wave * (32 * T::kPitchO);
+  // O^T (registers, [d][query]) -> LDS [query][d] in the element type -> coalesced 16-byte stores, half of the columns at
+  // a time through this wavefront's own staging rows.  No barrier: the staging rows are nobody else's and no part of the
+  // tile buffers, so the leading group writes its output while the trailing group is still in its last matrix phase.
+  uint8_t* stage = lds + T::kLdsTiles + wave * T::kStageBytes;
+  constexpr int kHalfChunks = D / 16;                 // 16-byte chunks in half a row
+  constexpr int kRowsPerPass = 64 / kHalfChunks;
+  const int rr = lane / kHalfChunks, cc = lane % kHalfChunks;
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db)
+  for (int half = 0; half < 2; ++half) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f32x2 lo, hi;
-      lo.x = o_acc[db][4 * g + 0] * inv;
-      lo.y = o_acc[db][4 * g + 1] * inv;
-      hi.x = o_acc[db][4 * g + 2] * inv;
-      hi.y = o_acc[db][4 * g + 3] * inv;
-      const ex2 l2 = __builtin_convertvector(lo, ex2);
-      const ex2 h2 = __builtin_convertvector(hi, ex2);
-      ex4 pk;
-      pk.x = l2.x; pk.y = l2.y; pk.z = h2.x; pk.w = h2.y;
-      const int d = 32 * db + 8 * g + 4 * hh;
-      *reinterpret_cast<ex4*>(ol + col * T::kPitchO + d * 2) = pk;
-    }
-  phase_barrier();
-  constexpr int kLanesPerRow = D / 8;
-  constexpr int kRowsPerPass = 64 / kLanesPerRow;
-  const int rr = lane / kLanesPerRow;
-  const int cc = lane % kLanesPerRow;
+    for (int i = 0; i < D / 64; ++i)
 #pragma unroll
-  for (int p = 0; p < 32 / kRowsPerPass; ++p) {
-    const int row = p * kRowsPerPass + rr;
-    const int qg = q0 + row;
-    const u32x4 val = *reinterpret_cast<const u32x4*>(ol + row * T::kPitchO + cc * 16);
-    if (qg < q_end) {
-      uint16_t* dst = view.out + (((int64_t)b * e.Sq + qg) * e.H + h) * D + cc * 8;
-      __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& o = o_acc[half * (D / 64) + i];
+        f32x2 lo, hi;
+        lo.x = o[4 * g + 0] * inv;
+        lo.y = o[4 * g + 1] * inv;
+        hi.x = o[4 * g + 2] * inv;
+        hi.y = o[4 * g + 3] * inv;
+        const ex2 l2 = __builtin_convertvector(lo, ex2);
+        const ex2 h2 = __builtin_convertvector(hi, ex2);
+        ex4 pk;
+        pk.x = l2.x; pk.y = l2.y; pk.z = h2.x; pk.w = h2.y;
+        *reinterpret_cast<ex4*>(stage + col * D + (((4 * i + g) ^ T::swz_o(col)) << 4) + 8 * hh) = pk;
+      }
+#pragma unroll
+    for (int p = 0; p < 32 / kRowsPerPass; ++p) {
+      const int row = p * kRowsPerPass + rr;
+      const int qg = q0 + row;
+      const u32x4 val = *reinterpret_cast<const u32x4*>(stage + row * D + ((cc ^ T::swz_o(row)) << 4));
+      if (qg < q_end) {
+        uint16_t* dst = view.out + (((int64_t)b * e.Sq + qg) * e.H + h) * D + half * (D / 2) + cc * 8;
+        __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
+      }
     }
   }
 }

@@ -89,10 +89,11 @@ struct AttnArgs {
   const int32_t* cu_kv[DT_MAX_CHUNKS];
 };
 
-// Dynamic LDS of one attention workgroup by head dimension (four 64-key buffers per operand).  The
+// Dynamic LDS of one attention workgroup by head dimension (four 64-key buffers per operand and the epilogue's
+// staging rows).  The
 // occupancy of a CU follows from it: one workgroup at 128, two at 64.
-constexpr int kAttnLdsBytes128 = 131072;
-constexpr int kAttnLdsBytes64 = 65536;
+constexpr int kAttnLdsBytes128 = 163840;
+constexpr int kAttnLdsBytes64 = 81920;
 
 // Workspace bytes the tail balancing can use at most (what dt_attn_workspace_bytes reports): 775 partial states of
 // 256 queries at D = 128, 1536 at D = 64.
