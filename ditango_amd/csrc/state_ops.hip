@@ -33,6 +33,7 @@ struct MergeArgs {
   float* dst_lse;
   int32_t dst_dtype;    // DT_BF16 / DT_FP32 / DT_FP16
   int32_t dst_bsh;
+  int32_t keep;         // the destination is stored without the non-temporal hint (see launch_merge)
 };
 
 // The two 16-bit elements of a word, widened (f16: IEEE half, else bfloat16), and back (round to nearest even).
@@ -419,8 +420,13 @@ __global__ __launch_bounds__(kThreads) void merge_states_kernel(const MergeArgs 
         v0[i] = __float_as_uint(o[i]);
         v1[i] = __float_as_uint(o[4 + i]);
       }
-      if (live_lo) __builtin_nontemporal_store(v0, reinterpret_cast<u32x4*>(q));
-      if (live_hi) __builtin_nontemporal_store(v1, reinterpret_cast<u32x4*>(q + 64));
+      if (a.keep) {   // uniform
+        if (live_lo) *reinterpret_cast<u32x4*>(q) = v0;
+        if (live_hi) *reinterpret_cast<u32x4*>(q + 64) = v1;
+      } else {
+        if (live_lo) __builtin_nontemporal_store(v0, reinterpret_cast<u32x4*>(q));
+        if (live_hi) __builtin_nontemporal_store(v1, reinterpret_cast<u32x4*>(q + 64));
+      }
     } else {
       uint16_t* q = reinterpret_cast<uint16_t*>(a.dst_out) + u[p].elem + 4 * cc;
       const bool f16 = a.dst_dtype == DT_FP16;
@@ -782,7 +788,21 @@ static void launch_merge_d(const MergeArgs& a, bool tiled, int passes, unsigned 
   }
 }
 
-int launch_merge(const MergeArgs& a, int D, hipStream_t stream) {
+// Largest fp32 destination that is left in the 256 MB of memory-side cache: a running state (one block opens it, every
+// further one is merged into it) is read again by the next update, so its stores carry no non-temporal hint.  Its reads
+// keep the hint, the version that was read is dead.  Three updates of a bf16 block, plain against non-temporal stores (us):
+// state of 170 MB 197 -> 186, 184 MB 212 -> 203, 246 MB 278 -> 263; 367 MB, which no longer fits, 404 -> 418.  A merge of
+// more states is a layer's result, whose stores would only push out what it still has to read (8 states of 91 MB into
+// 184 MB: 204 -> 224), so those keep the hint at any size.
+constexpr int64_t kKeepBytes = 256 << 20;
+static bool keeps_destination(const MergeArgs& a, int D) {
+  const bool running = a.n == 1 || (a.n == 2 && a.fp32_mask != 0);
+  return running && a.dst_dtype == DT_FP32 && (int64_t)a.B * a.Sq * a.H * D * 4 <= kKeepBytes;
+}
+
+int launch_merge(const MergeArgs& a_in, int D, hipStream_t stream) {
+  MergeArgs a = a_in;
+  a.keep = keeps_destination(a, D);
   if (D != 128 && D != 64) {
     set_error("head dim %d not built (64 and 128 are)", D);
     return DT_ERR_UNSUPPORTED;

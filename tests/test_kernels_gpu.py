@@ -529,3 +529,20 @@ def test_rel_l1_sums_at_the_hunyuan_shape(hip):
     got = (d / cnt) / (sb / cnt + 1e-8)                 # mean|new - ori| / (mean|ori| + 1e-8), new = b, ori = a
     want = om.rel_l1(b.cpu(), a.cpu())
     assert abs(got - want) <= 1e-5 * want
+
+
+@pytest.mark.parametrize("rows", [1, 65536, 65537])
+def test_running_state_on_both_sides_of_the_kept_size(hip, rows):
+    """fp32 destinations of one state and of an update, up to 256 MiB (65536 rows of 8 heads of 128) and beyond."""
+    from ditango_amd.utils import update_out_and_lse
+    g = torch.Generator(device="cuda:0").manual_seed(rows)
+    blocks = [(torch.randn(1, rows, 8, 128, generator=g, device="cuda:0").bfloat16(), torch.randn(1, 8, rows, generator=g, device="cuda:0"))
+              for _ in range(2)]
+    out, lse = update_out_and_lse(None, None, *blocks[0])
+    assert torch.equal(out, blocks[0][0].float())
+    torch.testing.assert_close(lse[..., 0], blocks[0][1].transpose(1, 2), rtol=0, atol=1e-6)   # one exp / log pair of fp32
+    out, lse = update_out_and_lse(out, lse, *blocks[1])
+    w = torch.sigmoid(blocks[1][1] - blocks[0][1]).transpose(1, 2).unsqueeze(-1)
+    ref = blocks[0][0].float() * (1 - w) + blocks[1][0].float() * w
+    torch.testing.assert_close(out, ref, rtol=2e-6, atol=4e-6)   # the weights carry a few ulp, the terms are below 6
+    torch.testing.assert_close(lse[..., 0], torch.logaddexp(blocks[0][1], blocks[1][1]).transpose(1, 2), rtol=0, atol=2e-6)
