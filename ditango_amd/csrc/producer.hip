@@ -20,7 +20,11 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;
-constexpr int kHeads = 8;  // heads of one token handled by a lane group with one set of table loads
+// Heads of one token handled by a lane group with one set of table loads.  Four instead of eight: the rows in flight take
+// half the registers, and a launch of the usual size ends in more, smaller workgroups (with eight, 14882 tokens x 24 heads
+// are 2.2 rounds of the chip).  HBM-bound; us per launch with 8 / 4 / 2 heads: 14882 x 24 heads of 128 41.7 / 39.5 / 41.3,
+// 12444 x 48 of 64 35.8 / 31.8 / 32.3, 9000 x 20 of 128 26.9 / 23.6 / 22.5, 119056 x 24 of 128 (6.0 TB/s) 262 / 260 / 278.
+constexpr int kHeads = 4;
 
 struct PrepArgs {
   const uint16_t* x;   // bfloat16, or IEEE half (DT_IO_FP16)
