@@ -22,7 +22,7 @@ DT_BF16, DT_FP32, DT_FP16 = 0, 1, 2
 DT_LSE_BHS, DT_LSE_BSH = 0, 1
 DT_NORM_NONE, DT_NORM_RMS, DT_NORM_LAYER = 0, 1, 2
 DT_ROPE_NONE, DT_ROPE_INTERLEAVED, DT_ROPE_HALVES = 0, 1, 2
-DT_ROUND_NORM_BF16, DT_ROUND_ROPE_BF16, DT_IO_FP16 = 1, 2, 4
+DT_ROUND_NORM_BF16, DT_ROUND_ROPE_BF16, DT_IO_FP16, DT_WEIGHTS_16 = 1, 2, 4, 8
 DT_ATTN_Q_PRESCALED, DT_ATTN_FP16 = 1, 2
 DT_MAX_CHUNKS = 40
 DT_MAX_JOBS = 40
@@ -457,7 +457,8 @@ def qk_norm_rope(x: torch.Tensor, *, norm: int = DT_NORM_NONE, weight: Optional[
     """x bf16 or fp16 ``[B,S,H,D]`` (any strides with a contiguous last dimension) -> ``[B,S,H,D]`` contiguous in
     the same dtype, normalised over D and rotated on token rows ``[rope_begin, rope_end)``.  cos/sin are fp32
     ``[rope_end-rope_begin, D]`` or ``[B, rope_end-rope_begin, D]``.  ``out_scale`` multiplies the result
-    before its rounding to the output dtype; the ``DT_ROUND_*`` bits round to x's dtype."""
+    before its rounding to the output dtype; the ``DT_ROUND_*`` bits round to x's dtype.  weight / bias are fp32, or
+    with ``DT_WEIGHTS_16`` in ``rounding`` of x's dtype."""
     lib = load_library()
     _require(x.is_cuda and x.dtype in HALF_DTYPES and x.dim() == 4 and x.stride(3) == 1, "x must be bf16 or fp16 [B,S,H,D] on the GPU")
     B, S, H, D = x.shape
@@ -466,9 +467,10 @@ def qk_norm_rope(x: torch.Tensor, *, norm: int = DT_NORM_NONE, weight: Optional[
     _require(out.is_cuda and out.dtype == x.dtype and out.is_contiguous() and tuple(out.shape) == (B, S, H, D),
              "out must be a contiguous [B,S,H,D] in x's dtype")
     rounding = int(rounding) | (DT_IO_FP16 if x.dtype == torch.float16 else 0)
+    w_dtype = x.dtype if rounding & DT_WEIGHTS_16 else torch.float32
     for name, t in (("weight", weight), ("bias", bias)):
-        _require(t is None or (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.numel() == D),
-                 f"{name} must be fp32 [D] on the GPU")
+        _require(t is None or (t.is_cuda and t.dtype == w_dtype and t.is_contiguous() and t.numel() == D),
+                 f"{name} must be {'of the dtype of x' if rounding & DT_WEIGHTS_16 else 'fp32'}, [D] on the GPU")
     if rope_end is None:
         rope_end = S
     tab_sb = 0

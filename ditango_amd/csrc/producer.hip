@@ -32,8 +32,9 @@ struct PrepArgs {
   int64_t xs_b, xs_s, xs_h;
   int32_t B, S, H;
   int32_t norm, rope, rounding;
-  const float* w;
-  const float* bias;
+  const void* w;       // fp32, or x's type (w16)
+  const void* bias;
+  int32_t w16;
   float eps;
   float out_scale;  // multiplies the result before its rounding to the output type
   const float* cos;
@@ -73,6 +74,19 @@ __device__ __forceinline__ void unpack8(const u32x4 r, float (&v)[8]) {
       v[2 * i] = __builtin_bit_cast(float, u[i] << 16);
       v[2 * i + 1] = __builtin_bit_cast(float, u[i] & 0xffff0000u);
     }
+  }
+}
+
+// 8 consecutive norm weights, fp32 or in x's type (their widening is exact)
+template <bool kHalf>
+__device__ __forceinline__ void load_weights8(const void* base, bool w16, int d0, float (&v)[8]) {
+  if (w16) {   // uniform
+    unpack8<kHalf>(*reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(base) + d0), v);
+  } else {
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + d0);
+    const f32x4 hi = *reinterpret_cast<const f32x4*>(static_cast<const float*>(base) + d0 + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { v[i] = lo[i]; v[4 + i] = hi[i]; }
   }
 }
 
@@ -127,18 +141,8 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(const PrepArgs a
     w[i] = 1.0f;
     bias[i] = 0.0f;
   }
-  if (a.norm != DT_NORM_NONE && a.w) {
-    const f32x4 w0 = *reinterpret_cast<const f32x4*>(a.w + d0);
-    const f32x4 w1 = *reinterpret_cast<const f32x4*>(a.w + d0 + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { w[i] = w0[i]; w[4 + i] = w1[i]; }
-  }
-  if (a.norm == DT_NORM_LAYER && a.bias) {
-    const f32x4 b0 = *reinterpret_cast<const f32x4*>(a.bias + d0);
-    const f32x4 b1 = *reinterpret_cast<const f32x4*>(a.bias + d0 + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { bias[i] = b0[i]; bias[4 + i] = b1[i]; }
-  }
+  if (a.norm != DT_NORM_NONE && a.w) load_weights8<kHalf>(a.w, a.w16 != 0, d0, w);
+  if (a.norm == DT_NORM_LAYER && a.bias) load_weights8<kHalf>(a.bias, a.w16 != 0, d0, bias);
 
   // rotate-half partner of this lane inside its section
   int partner = 0;
@@ -238,8 +242,8 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 using namespace dt;
 
 extern "C" int dt_qk_norm_rope(const void* x, int64_t x_stride_b, int64_t x_stride_s, int64_t x_stride_h, void* y,
-                               int32_t B, int32_t S, int32_t H, int32_t D, int32_t norm, const float* weight,
-                               const float* bias, float eps, int32_t rope, const float* cos, const float* sin,
+                               int32_t B, int32_t S, int32_t H, int32_t D, int32_t norm, const void* weight,
+                               const void* bias, float eps, int32_t rope, const float* cos, const float* sin,
                                int64_t table_stride_b, int32_t rope_begin, int32_t rope_end,
                                const int32_t* sections, int32_t n_sections, int32_t rounding, float out_scale,
                                void* stream) {
@@ -256,7 +260,7 @@ extern "C" int dt_qk_norm_rope(const void* x, int64_t x_stride_b, int64_t x_stri
     return DT_ERR_INVALID;
   }
   if (norm < DT_NORM_NONE || norm > DT_NORM_LAYER || rope < DT_ROPE_NONE || rope > DT_ROPE_HALVES ||
-      (rounding & ~(DT_ROUND_NORM_BF16 | DT_ROUND_ROPE_BF16 | DT_IO_FP16))) {
+      (rounding & ~(DT_ROUND_NORM_BF16 | DT_ROUND_ROPE_BF16 | DT_IO_FP16 | DT_WEIGHTS_16))) {
     set_error("bad norm / rope / rounding code (%d, %d, %d)", norm, rope, rounding);
     return DT_ERR_INVALID;
   }
@@ -276,6 +280,7 @@ extern "C" int dt_qk_norm_rope(const void* x, int64_t x_stride_b, int64_t x_stri
   a.norm = norm; a.rope = rope; a.rounding = rounding & (DT_ROUND_NORM_BF16 | DT_ROUND_ROPE_BF16);
   const bool half = (rounding & DT_IO_FP16) != 0;
   a.w = weight; a.bias = bias; a.eps = eps;
+  a.w16 = (rounding & DT_WEIGHTS_16) != 0;
   a.out_scale = out_scale;
   a.sec_end[0] = a.sec_end[1] = a.sec_end[2] = D;
   if (rope != DT_ROPE_NONE) {

@@ -33,6 +33,13 @@ def _f32(t: Optional[torch.Tensor], device) -> Optional[torch.Tensor]:
     return t.detach().to(device=device, dtype=torch.float32).contiguous()
 
 
+def _read_in_place(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor]) -> bool:
+    """Norm parameters in x's own 16-bit type, as a model's modules hold them, are widened by the kernel as it reads them
+    (two conversion launches a call less); any other dtype, place or alignment goes through an fp32 copy."""
+    return all(t is None or (t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0)
+               for t in (weight, bias)) and x.dtype in _hip.HALF_DTYPES
+
+
 def prepare_qk(x: torch.Tensor, *, norm: Optional[str] = None, weight: Optional[torch.Tensor] = None,
                bias: Optional[torch.Tensor] = None, eps: float = 1e-6, rope: Optional[str] = None,
                freqs_cis: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, rope_begin: int = 0,
@@ -63,7 +70,12 @@ def prepare_qk(x: torch.Tensor, *, norm: Optional[str] = None, weight: Optional[
             raise ValueError("rope needs freqs_cis = (cos, sin)")
         cos, sin = _f32(freqs_cis[0], x.device), _f32(freqs_cis[1], x.device)
     rounding = (_hip.DT_ROUND_NORM_BF16 if match_eager_rounding else 0) | (_hip.DT_ROUND_ROPE_BF16 if bf16_rope_math else 0)
-    return _hip.qk_norm_rope(x, norm=_NORMS[norm], weight=_f32(weight, x.device), bias=_f32(bias, x.device), eps=eps,
+    if (weight is not None or bias is not None) and _read_in_place(x, weight, bias):
+        rounding |= _hip.DT_WEIGHTS_16
+        weight, bias = (t.detach() if t is not None else None for t in (weight, bias))
+    else:
+        weight, bias = _f32(weight, x.device), _f32(bias, x.device)
+    return _hip.qk_norm_rope(x, norm=_NORMS[norm], weight=weight, bias=bias, eps=eps,
                              rope=_ROPES[rope], cos=cos, sin=sin, rope_begin=rope_begin, rope_end=rope_end,
                              sections=sections, rounding=rounding, out=out,
                              out_scale=1.0 if fold_softmax_scale is None else folded_scale(x.shape[-1], fold_softmax_scale))

@@ -52,6 +52,7 @@ extern "C" {
 #define DT_ROUND_NORM_BF16 1 /* round to bf16 where the callers' bf16 norm modules do */
 #define DT_ROUND_ROPE_BF16 2 /* RoPE products and their sum each rounded to bf16 */
 #define DT_IO_FP16 4         /* x and y are fp16; the two bits above then round to fp16 */
+#define DT_WEIGHTS_16 8      /* weight and bias hold elements of x's type instead of fp32 */
 
 #define DT_MAX_CHUNKS 40       /* KV chunks one launch can address */
 #define DT_MAX_JOBS 40         /* attention states one launch can produce */
@@ -429,7 +430,7 @@ int dt_rel_l1_sums(const float* a, const float* b, int64_t n, double* sums, void
  * dimension, so q, k or v can be read in place out of a fused QKV projection; with
  * norm = rope = 0 the call is the strided-to-contiguous copy of v.  y may alias x when x is
  * already contiguous [B,S,H,D].
- * weight / bias: fp32 [D] or NULL (1 / 0).  cos / sin: fp32 [rope_end - rope_begin, D], row
+ * weight / bias: fp32 [D] (with DT_WEIGHTS_16 in `rounding`: x's type), 16-byte aligned, or NULL (1 / 0).  cos / sin: fp32 [rope_end - rope_begin, D], row
  * s - rope_begin belongs to token s; batch b reads its tables at + b * table_stride_b
  * elements (0 = shared).  out[d] = x[d] * cos[d] + rot(x)[d] * sin[d] with
  *   DT_ROPE_INTERLEAVED: rot(x)[2i] = -x[2i+1], rot(x)[2i+1] = x[2i];
@@ -444,7 +445,7 @@ int dt_rel_l1_sums(const float* a, const float* b, int64_t n, double* sums, void
  */
 int dt_qk_norm_rope(const void* x, int64_t x_stride_b, int64_t x_stride_s, int64_t x_stride_h, void* y,
                     int32_t B, int32_t S, int32_t H, int32_t D,
-                    int32_t norm, const float* weight, const float* bias, float eps,
+                    int32_t norm, const void* weight, const void* bias, float eps,
                     int32_t rope, const float* cos, const float* sin, int64_t table_stride_b,
                     int32_t rope_begin, int32_t rope_end, const int32_t* sections, int32_t n_sections,
                     int32_t rounding, float out_scale, void* stream);

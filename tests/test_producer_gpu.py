@@ -217,3 +217,25 @@ def test_full_kv_sequence_of_the_hunyuan_shape(hip):
         o = P.qk_norm_rope(xs[:, lo:hi], P.NORM_RMS, w, None, 1e-6, P.ROPE_INTERLEAVED if rot else P.ROPE_NONE,
                            cos[r] if rot else None, sin[r] if rot else None, 0, hi - lo, (), 0)
         _close(y[:, r.to(DEV)], o)
+
+
+@pytest.mark.parametrize("D,H", [(64, 3), (128, 6)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("norm", ["rms", "layer_norm"])
+def test_norm_parameters_in_the_dtype_of_x_are_read_in_place(hip, D, H, dtype, norm):
+    """Widening is exact, so the result is that of fp32 copies bit for bit; a misaligned or mixed pair still works."""
+    from ditango_amd.producer import _read_in_place, prepare_qk
+    g = torch.Generator().manual_seed(D)
+    x = torch.randn(2, 9, H, D, generator=g).to(dtype).to(DEV)
+    w = (torch.rand(D, generator=g) + 0.5).to(dtype).to(DEV)
+    b = torch.randn(D, generator=g).to(dtype).to(DEV) if norm == "layer_norm" else None
+    kw = dict(norm=norm, eps=1e-6, match_eager_rounding=True)
+    want = prepare_qk(x, weight=w.float(), bias=None if b is None else b.float(), **kw)
+    assert _read_in_place(x, w, b) and not _read_in_place(x, w.float(), b)
+    assert torch.equal(prepare_qk(x, weight=w, bias=b, **kw), want)
+    shifted = torch.empty(D + 1, dtype=dtype, device=DEV)[1:].copy_(w)
+    assert not _read_in_place(x, shifted, b)
+    assert torch.equal(prepare_qk(x, weight=shifted, bias=b, **kw), want)
+    assert torch.equal(prepare_qk(x, weight=w.float(), bias=b, **kw), want)
+    with pytest.raises(hip.DitangoHipError):
+        hip.qk_norm_rope(x, norm=P.NORM_RMS, weight=w)   # without the flag the binding takes fp32 only
