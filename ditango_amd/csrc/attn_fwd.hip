@@ -141,17 +141,20 @@ __device__ __forceinline__ void wait_tile_loads() {
 // produces S^T and updates O^T).
 // After a vector phase the wavefront also waits for the direct-to-LDS tile loads it issued earlier,
 // all but the kInFlight newest: behind the barrier they are visible to every wavefront.
-template <int kInFlight, typename V>
-__device__ __forceinline__ void phase_barrier_after_vector(V (&p)[2][2]) {
+template <int kInFlight, typename V, int NK>
+__device__ __forceinline__ void phase_barrier_after_vector(V (&p)[NK][2]) {
   __builtin_amdgcn_sched_barrier(0);
 #define DT_VECTOR_BARRIER(N)                                                      \
-  asm volatile("s_waitcnt vmcnt(" #N ") lgkmcnt(0)\n\ts_barrier"                   \
-               : "+v"(p[0][0]), "+v"(p[0][1]), "+v"(p[1][0]), "+v"(p[1][1])       \
-               :                                                                  \
-               : "memory")
-  if constexpr (kInFlight == 6) DT_VECTOR_BARRIER(6);
-  else if constexpr (kInFlight == 3) DT_VECTOR_BARRIER(3);
-  else if constexpr (kInFlight == 2) DT_VECTOR_BARRIER(2);
+  if constexpr (NK == 2)                                                          \
+    asm volatile("s_waitcnt vmcnt(" #N ") lgkmcnt(0)\n\ts_barrier"                 \
+                 : "+v"(p[0][0]), "+v"(p[0][1]), "+v"(p[1][0]), "+v"(p[1][1])     \
+                 :                                                                \
+                 : "memory");                                                     \
+  else                                                                            \
+    asm volatile("s_waitcnt vmcnt(" #N ") lgkmcnt(0)\n\ts_barrier" : "+v"(p[0][0]), "+v"(p[0][1]) : : "memory")
+  if constexpr (kInFlight == 6) { DT_VECTOR_BARRIER(6); }
+  else if constexpr (kInFlight == 3) { DT_VECTOR_BARRIER(3); }
+  else if constexpr (kInFlight == 2) { DT_VECTOR_BARRIER(2); }
   else {
     static_assert(kInFlight == 1, "loads in flight across the barrier: 1, 2, 3 or 6");
     DT_VECTOR_BARRIER(1);
@@ -159,20 +162,14 @@ __device__ __forceinline__ void phase_barrier_after_vector(V (&p)[2][2]) {
 #undef DT_VECTOR_BARRIER
   __builtin_amdgcn_sched_barrier(0);
 }
-template <typename V, int NO>
-__device__ __forceinline__ void phase_barrier_after_matrix(V (&sa)[2], V (&oa)[NO]) {
+template <typename V, int NK, int NO>
+__device__ __forceinline__ void phase_barrier_after_matrix(V (&sa)[NK], V (&oa)[NO]) {
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (NO == 4) {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier"
-                 : "+v"(sa[0]), "+v"(sa[1]), "+v"(oa[0]), "+v"(oa[1]), "+v"(oa[2]), "+v"(oa[3])
-                 :
-                 : "memory");
-  } else {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier"
-                 : "+v"(sa[0]), "+v"(sa[1]), "+v"(oa[0]), "+v"(oa[1])
-                 :
-                 : "memory");
-  }
+  // (two statements: the operands are tied to the first, the barrier follows it)
+  if constexpr (NK == 2) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sa[0]), "+v"(sa[1]) : : "memory");
+  else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sa[0]) : : "memory");
+  if constexpr (NO == 4) asm volatile("s_barrier" : "+v"(oa[0]), "+v"(oa[1]), "+v"(oa[2]), "+v"(oa[3]) : : "memory");
+  else asm volatile("s_barrier" : "+v"(oa[0]), "+v"(oa[1]) : : "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
 
@@ -350,6 +347,47 @@ __device__ __forceinline__ bool view_job(Args& a, int job, JobView& v) {
   return true;
 }
 
+// The arguments where they arrive (see attn_fwd_kernel), as a reference that the compiler cannot relate to another.
+typedef const AttnArgs __attribute__((address_space(4))) KernArgs;
+__device__ __forceinline__ KernArgs& kernel_args() {
+  uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(KernArgs*)p;
+}
+
+// Chunk reference `seg` of a job: keys [begin, begin + len) of chunk cid.
+struct KeyRef {
+  int cid, begin, len;
+};
+__device__ __forceinline__ KeyRef key_ref(const JobView& v, int seg) {
+  KernArgs& a = kernel_args();
+  KeyRef r;
+  if (v.single < 0) {
+    r.cid = a.entry[seg].chunk;
+    r.begin = a.entry[seg].kv_begin;
+    r.len = a.entry[seg].kv_len;
+  } else {
+    r.cid = v.single;
+    r.begin = 0;
+    if (v.vseg >= 0) {
+      r.begin = a.entry[v.single * a.n_seg + v.vseg].kv_begin;
+      r.len = a.entry[v.single * a.n_seg + v.vseg].kv_len;
+    } else {
+      r.len = a.chunk[v.single].len;
+    }
+  }
+  if (v.dseg >= 0) {
+    const int keys = a.chunk[r.cid].len;
+    r.begin = min(max(boundary(a.cu_kv[r.cid], v.dseg), 0), keys);
+    r.len = min(max(boundary(a.cu_kv[r.cid], v.dseg + 1), r.begin), keys) - r.begin;
+  }
+  return r;
+}
+
+// Work items of fewer key tiles than this are never cut along the keys or the rows: there is next to nothing to gain (an
+// item costs about four tiles on top of its own), and a segment of a few padding tokens keeps the sums of one pass.
+constexpr int kMinSplitTiles = 8;
+
 // Wavefronts per SIMD the register budget is set for.  D = 128: two (one workgroup per CU: its LDS
 // tiles fill the CU).  D = 64: four, i.e. TWO workgroups per CU (64 KB of LDS and at most 128
 // registers each): the second workgroup's wavefronts issue into the barrier waits, the start-up and
@@ -376,100 +414,38 @@ __device__ __forceinline__ void prefetch_args(uint64_t args) {
       : "memory");
 }
 
-template <int D, bool kPre, bool kHalf>
-__global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn_fwd_kernel(const AttnArgs args_by_value) {
+// The work of one workgroup: query rows from row0 on of one job, batch and head.
+//
+// kSplitKeys: no more than half of the 256 rows exist, or another workgroup has the other half.  Wavefronts w and w + 4 --
+// one of either group -- then share 32 queries: the leading group's takes the first 32 keys of every tile, the trailing
+// group's the others, and the two states meet in fp32 through the LDS at the end.  Loads, buffers, barriers and waits are
+// those of the other form, a wavefront's phases have half the MFMAs and half the softmax.  A tile then takes 0.60 of the
+// time of a full one (one round of items of 32 key tiles: D = 128 79 -> 49 us, D = 64 87 -> 52), not half: the load
+// instructions and barriers stay.  That much is saved on the last query tile of a head where up to 128 of its rows exist
+// (24 heads x 1400 queries x 4 chunks, D = 128: 121 -> 118 us), and by cutting the items of the last round in two (plan_tail).
+template <int D, bool kPre, bool kHalf, bool kSplitKeys>
+__device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int row0, bool is_part, int part, int unit, int xcd) {
   using T = Tile<D>;
   using E = Elem<kHalf>;
-  typedef typename E::t elem_t;
   typedef typename E::x8 ex8;
   typedef typename E::x4 ex4;
   typedef typename E::x2 ex2;
-  static_assert(!(kPre && kHalf), "the prescaled softmax keeps probabilities up to 2^40: bf16 only");
-  // The arguments are read where they arrive: in the kernarg segment (constant address space, scalar loads),
-  // through its base pointer -- AttnArgs is the kernel's only parameter, so it sits at offset 0.  Going through the
-  // by-value parameter instead leaves it to the optimiser to prove that its private copy of the 3.6 KB struct is
-  // never needed; with the tables indexed at run time from several branches it sometimes cannot, and every lane
-  // then copies the whole struct into scratch memory before it starts (seven times the run time of a short launch).
-  typedef const AttnArgs __attribute__((address_space(4))) KernArgs;
-  (void)args_by_value;
-  prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+  constexpr int kKeyBlocks = kSplitKeys ? 1 : 2;   // 32-key blocks of a tile that a wavefront works on
   // A reference of its own for every place that reads arguments, unrelated to the others as far as the compiler can see:
   // it otherwise reads whole lines at the top and holds what later places need in 120 spilled scalar registers.
-  auto args = []() __attribute__((always_inline)) -> KernArgs& {
-    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return *(KernArgs*)p;
-  };
+  auto args = []() __attribute__((always_inline)) -> KernArgs& { return kernel_args(); };
   KernArgs& a = args();
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-
-  // ---- which (job, batch, head, query tile) ------------------------------------------
-  int job = blockIdx.y;
-  const int xcd = blockIdx.x & (kXcds - 1);
-  int idx = blockIdx.x >> 3;
-  int part = 0, unit = 0;  // which of the part_ways key-tile ranges of which split item (counted per XCD)
-  bool is_part = false;    // this workgroup computes one part of a split item
-  if (job >= a.job_planes) {
-    // planes behind the jobs hold the parts of the split items, in dispatch order
-    const int pi = (job - a.job_planes) * (int)(gridDim.x >> 3) + idx;
-    if (pi >= a.tail_items * a.part_ways) return;
-    unit = pi / a.part_ways;
-    part = pi - unit * a.part_ways;
-    const int flat = a.tail_start + unit;
-    job = flat / a.per_xcd;
-    idx = flat - job * a.per_xcd;
-    is_part = true;
-  } else if ((int64_t)job * a.per_xcd + idx >= a.tail_start) {
-    return;  // runs as parts
-  }
-  const int item = xcd * a.per_xcd + idx;
-  if (idx >= a.per_xcd || item >= a.total) return;
-  const int bh = item / a.nqt;
-  const int qt = item - bh * a.nqt;
-  const int b = bh / a.H;
-  const int h = bh - b * a.H;
-
-  JobView view;
-  if (!view_job(a, job, view)) return;
-  const int seg_begin = view.seg_begin, seg_end = view.seg_end, single = view.single;
-  const int q_begin = view.q_begin, q_end = view.q_end, vseg = view.vseg, dseg = view.dseg;
-  if (qt * kBQ >= q_end - q_begin) return;  // the grid is sized for the longest job / segment
-  // chunk reference `seg`: keys [begin, begin + len) of chunk cid
-  struct Ref {
-    int cid, begin, len;
-  };
-  auto ref_at = [&](int seg) __attribute__((always_inline)) -> Ref {
-    KernArgs& a = args();
-    Ref r;
-    if (single < 0) {
-      r.cid = a.entry[seg].chunk;
-      r.begin = a.entry[seg].kv_begin;
-      r.len = a.entry[seg].kv_len;
-    } else {
-      r.cid = single;
-      r.begin = 0;
-      if (vseg >= 0) {
-        r.begin = a.entry[single * a.n_seg + vseg].kv_begin;
-        r.len = a.entry[single * a.n_seg + vseg].kv_len;
-      } else {
-        r.len = a.chunk[single].len;
-      }
-    }
-    if (dseg >= 0) {
-      const int keys = a.chunk[r.cid].len;
-      r.begin = min(max(boundary(a.cu_kv[r.cid], dseg), 0), keys);
-      r.len = min(max(boundary(a.cu_kv[r.cid], dseg + 1), r.begin), keys) - r.begin;
-    }
-    return r;
-  };
-
+  const int seg_begin = view.seg_begin, seg_end = view.seg_end;
+  const int q_begin = view.q_begin, q_end = view.q_end;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps group/buffer arithmetic scalar
   const int group = wave >> 2;  // 0: leads, 1: runs one phase behind
   const int col = lane & 31;    // query column (B operand) / operand row (A operand)
   const int hh = lane >> 5;     // which half of the contraction dimension this lane feeds
-  const int q0 = q_begin + qt * kBQ + wave * 32;
+  const int q0 = q_begin + row0 + (kSplitKeys ? wave & 3 : wave) * 32;
+  const int key0 = kSplitKeys ? 32 * group : 0;  // first key of a tile that this wavefront works on
 
   // ---- Q fragments: B operand of S^T = K Q^T, kept in registers ----------------------
   ex8 qf[D / 16];
@@ -494,7 +470,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   uint32_t k_off = 0u;
   int ld_seg = seg_begin, ld_left = 0;
   int cp_seg = seg_begin, cp_left = 0;
-  auto ld_open = [&](const Ref& r) __attribute__((always_inline)) {
+  auto ld_open = [&](const KeyRef& r) __attribute__((always_inline)) {
     k_off = 0u;
     ld_left = r.len;
     if (r.len > 0) {
@@ -510,21 +486,21 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     }
   };
   auto ld_next_chunk = [&]() __attribute__((always_inline)) {
-    Ref r;
+    KeyRef r;
     r.len = 0;
-    while (r.len == 0 && ++ld_seg < seg_end) r = ref_at(ld_seg);
+    while (r.len == 0 && ++ld_seg < seg_end) r = key_ref(view, ld_seg);
     ld_open(r);
   };
   auto cp_next_chunk = [&]() __attribute__((always_inline)) {
     cp_left = 0;
-    while (cp_left == 0 && ++cp_seg < seg_end) cp_left = ref_at(cp_seg).len;
+    while (cp_left == 0 && ++cp_seg < seg_end) cp_left = key_ref(view, cp_seg).len;
   };
   // the first reference opens both cursors (most jobs have no other)
-  Ref first;
+  KeyRef first;
   first.len = 0;
-  if (seg_begin < seg_end) first = ref_at(seg_begin);
+  if (seg_begin < seg_end) first = key_ref(view, seg_begin);
   int n_tiles = (first.len + kBK - 1) / kBK;
-  for (int s = seg_begin + 1; s < seg_end; ++s) n_tiles += (ref_at(s).len + kBK - 1) / kBK;
+  for (int s = seg_begin + 1; s < seg_end; ++s) n_tiles += (key_ref(view, s).len + kBK - 1) / kBK;
   if (__builtin_expect(first.len > 0, 1)) {
     ld_open(first);
     cp_left = first.len;
@@ -534,8 +510,9 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   }
   if (is_part) {
     // this workgroup covers key tiles [t0, t1) of the item: walk both cursors to t0
-    const int t0 = (int)((int64_t)n_tiles * part / a.part_ways);
-    const int t1 = (int)((int64_t)n_tiles * (part + 1) / a.part_ways);
+    const int ways = n_tiles < kMinSplitTiles ? 1 : a.part_ways;   // (then part 0 covers all, the others nothing)
+    const int t0 = min((int)((int64_t)n_tiles * part / ways), n_tiles);
+    const int t1 = min((int)((int64_t)n_tiles * (part + 1) / ways), n_tiles);
     int skip = t0;
     while (skip > 0 && ld_seg < seg_end) {
       const int in_chunk = (ld_left + kBK - 1) / kBK;
@@ -638,7 +615,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   // operand read addresses of this lane within a K / V buffer (the lane's part of the swizzle)
   uint32_t kld[D / 16];  // K fragment of k-step s: row key_of_row(col) (+32 for the second half tile)
   {
-    const int krow = key_of_row(col);
+    const int krow = key0 + key_of_row(col);
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) kld[s] = krow * T::kRowBytes + 16 * ((2 * s + hh) ^ T::swz_k(krow));
   }
@@ -646,20 +623,20 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   // d columns 16*(block parity) + 4m .. +3 of the fragment's 32-column segment
   uint32_t vld[T::kSegs];
   {
-    const int vrow = 8 * hh + ((lane & 15) >> 2);
+    const int vrow = key0 + 8 * hh + ((lane & 15) >> 2);
 #pragma unroll
     for (int g = 0; g < T::kSegs; ++g)
       vld[g] = T::kOffV + vrow * T::kRowBytes + 64 * (g ^ T::swz_v(vrow)) + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
   }
 
-  f32x16 s_acc[2];       // S^T of the tile whose softmax comes next
-  ex8 p_frag[2][2];      // P^T of the tile whose P V product comes next
+  f32x16 s_acc[kKeyBlocks];    // S^T of the tile whose softmax comes next
+  ex8 p_frag[kKeyBlocks][2];   // P^T of the tile whose P V product comes next
   int cp_valid = 0;      // keys that exist in the tile held in s_acc
 
   // S^T = K Q^T for tile 0 only (first matrix phase)
   auto qk_only = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < kKeyBlocks; ++kb) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) s_acc[kb][r] = 0.f;
 #pragma unroll
@@ -675,8 +652,8 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   // single wavefront of this SIMD that is in its matrix phase never waits for LDS latency.
   // (After the last tile the second half recomputes scores on a stale K buffer; they are unused.)
   // U = tile & 3 picks the buffers at compile time: all operand reads use immediate offsets.
-  constexpr int kPV = D / 32 * 4;       // fragments of the P V product
-  constexpr int kQK = 2 * (D / 16);     // fragments of the score product
+  constexpr int kPV = D / 32 * 2 * kKeyBlocks;   // fragments of the P V product
+  constexpr int kQK = kKeyBlocks * (D / 16);     // fragments of the score product
   constexpr int kFrags = kPV + kQK;
   constexpr int kRing = kRingDepth;
   // Where a wavefront issues its tile loads: at the start of its vector phase, or behind the
@@ -715,7 +692,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     auto frag = [&](int i) -> ex8 {
       if (i < kPV) return v_frag(kU, i);
       const int j = i - kPV;
-      const int kb = j & 1, sidx = j >> 1;
+      const int kb = j % kKeyBlocks, sidx = j / kKeyBlocks;
       return *reinterpret_cast<const ex8*>(lds + kld[sidx] + kUK * T::kBytesK + kb * 32 * T::kRowBytes);
     };
 #pragma unroll
@@ -727,7 +704,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
         o_acc[db] = E::mfma(cur, p_frag[kb][half], o_acc[db]);
       } else {
         const int j = i - kPV;
-        const int kb = j & 1, sidx = j >> 1;
+        const int kb = j % kKeyBlocks, sidx = j / kKeyBlocks;
         if (sidx == 0) {
           f32x16 zero;
 #pragma unroll
@@ -828,9 +805,9 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
       // the empty asm has side effects as far as the compiler knows, which keeps this a real
       // branch: otherwise the selects below are hoisted out and run for every tile
       asm volatile("" ::: "memory");
-      const int lim = cp_valid;
+      const int lim = cp_valid - key0;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < kKeyBlocks; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = 32 * kb + 16 * (r >> 3) + 8 * hh + (r & 7);
@@ -854,7 +831,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
       rs0 = INFINITY;
     } else
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < kKeyBlocks; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         f32x2 p;
@@ -880,8 +857,10 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
       float mx = s_acc[0][0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s_acc[0][r]);
+      if constexpr (kKeyBlocks == 2) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s_acc[1][r]);
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s_acc[1][r]);
+      }
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       float m_new, alpha;
       if constexpr (kPre) {
@@ -910,7 +889,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
       rs0 = 0.f;
       rs1 = 0.f;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < kKeyBlocks; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
           f32x2 p;
@@ -951,6 +930,44 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   // tile loads issued for tiles past the end are still on their way (they store zeros): let them land before the
   // workgroup ends and its LDS becomes another's
   wait_tile_loads<0>();
+
+  if constexpr (kSplitKeys) {
+    // The trailing group's accumulators, as they lie in the registers, through the tile buffers (everybody is past its
+    // last read of them and its last load behind the first barrier); reference and sum through its staging rows.
+    phase_barrier();
+    const int pair = wave & 3;
+    uint8_t* slot = lds + pair * (32 * D * 4) + lane * 16;
+    float* ml = reinterpret_cast<float*>(lds + T::kLdsTiles + (pair + 4) * T::kStageBytes) + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f32x4 x;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = o_acc[i][4 * g + e];
+          *reinterpret_cast<f32x4*>(slot + (4 * i + g) * 1024) = x;
+        }
+      ml[0] = m_ref;
+      ml[64] = l_run;
+    }
+    phase_barrier();
+    if (group == 1) return;
+    const float m_other = ml[0], m_new = fmaxf(m_ref, m_other);
+    // (neither half has seen a key: both sums are 0 and stay so)
+    const float mine = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m_ref - m_new) * c) : 0.f;
+    const float theirs = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m_other - m_new) * c) : 0.f;
+    l_run = l_run * mine + ml[64] * theirs;
+    m_ref = m_new;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(slot + (4 * i + g) * 1024);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o_acc[i][4 * g + e] = o_acc[i][4 * g + e] * mine + x[e] * theirs;
+      }
+  }
 
   // ---- epilogue -------------------------------------------------------------------------
   const float l_tot = l_run + __shfl_xor(l_run, 32);
@@ -1012,6 +1029,67 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
       }
     }
   }
+}
+
+template <int D, bool kPre, bool kHalf>
+__global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn_fwd_kernel(const AttnArgs args_by_value) {
+  static_assert(!(kPre && kHalf), "the prescaled softmax keeps probabilities up to 2^40: bf16 only");
+  // The arguments are read where they arrive: in the kernarg segment (constant address space, scalar loads),
+  // through its base pointer -- AttnArgs is the kernel's only parameter, so it sits at offset 0.  Going through the
+  // by-value parameter instead leaves it to the optimiser to prove that its private copy of the 3.6 KB struct is
+  // never needed; with the tables indexed at run time from several branches it sometimes cannot, and every lane
+  // then copies the whole struct into scratch memory before it starts (seven times the run time of a short launch).
+  (void)args_by_value;
+  prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+  KernArgs& a = kernel_args();
+
+  // ---- which (job, batch, head, query tile) ------------------------------------------
+  int job = blockIdx.y;
+  const int xcd = blockIdx.x & (kXcds - 1);
+  int idx = blockIdx.x >> 3;
+  int part = 0, unit = 0;  // which of the part_ways key-tile ranges of which split item (counted per XCD)
+  bool is_part = false;    // this workgroup computes one part of a split item
+  int row0 = 0;            // first query row of the tile that this workgroup computes
+  bool half_rows = false;  // ... and no more than half of the tile's rows
+  if (job >= a.job_planes) {
+    // planes behind the jobs hold the parts of the split items, in dispatch order
+    const int pi = (job - a.job_planes) * (int)(gridDim.x >> 3) + idx;
+    if (pi >= a.tail_items * a.part_ways) return;
+    unit = pi / a.part_ways;
+    part = pi - unit * a.part_ways;
+    const int flat = a.tail_start + unit;
+    job = flat / a.per_xcd;
+    idx = flat - job * a.per_xcd;
+    if (a.row_split) {
+      row0 = part * (kBQ / 2);
+      half_rows = true;
+    } else {
+      is_part = true;
+    }
+  } else if ((int64_t)job * a.per_xcd + idx >= a.tail_start) {
+    return;  // runs as parts
+  }
+  const int item = xcd * a.per_xcd + idx;
+  if (idx >= a.per_xcd || item >= a.total) return;
+  const int bh = item / a.nqt;
+  const int qt = item - bh * a.nqt;
+  const int b = bh / a.H;
+  const int h = bh - b * a.H;
+
+  JobView view;
+  if (!view_job(a, job, view)) return;
+  row0 += qt * kBQ;
+  const int rows = view.q_end - view.q_begin - row0;
+  if (rows <= 0) return;  // the grid is sized for the longest job / segment
+  bool split_keys = false;
+  if (!kPre && !is_part && (half_rows || rows <= kBQ / 2)) {
+    int n_tiles = 0;
+    for (int s = view.seg_begin; s < view.seg_end; ++s) n_tiles += (key_ref(view, s).len + kBK - 1) / kBK;
+    split_keys = n_tiles >= kMinSplitTiles;
+    if (!split_keys && half_rows && part > 0) return;   // part 0 does the whole tile
+  }
+  if (split_keys) attn_item<D, kPre, kHalf, !kPre>(view, b, h, row0, false, 0, 0, 0);
+  else attn_item<D, kPre, kHalf, false>(view, b, h, row0, is_part, part, unit, xcd);
 }
 
 // Folds the part_ways partial states of every split item into the item's rows of its destination.  A workgroup takes 64
@@ -1246,7 +1324,7 @@ static void job_sizes(const AttnArgs& a, int n_jobs, JobSize* size) {
   }
 }
 
-// Which work items at the end of the launch run as how many parts each (tail_start, tail_items, part_ways).
+// Which work items at the end of the launch run as how many parts each (tail_start, tail_items, part_ways, row_split).
 //
 // Time is counted in key tiles, on one XCD (workgroups go to the XCDs in turn, so each works through its own share of
 // every job).  Jobs come by falling length: the short ones behind fill the gaps that the long ones leave, so the
@@ -1257,11 +1335,18 @@ static void job_sizes(const AttnArgs& a, int n_jobs, JobSize* size) {
 // Measured on the HunyuanVideo, Step-Video and CogVideoX shares: a part costs about 6 tiles on top of its own (start-up,
 // epilogue, partial state) when all parts run at once and about 10 when they take several rounds, so many small parts
 // only pay in the first case; the fold kernel and the parts' stores cost about 4 (D = 128: 6, twice the bytes).
+// The other way to end a launch early: the items of the last round as two workgroups of half the query rows each, 0.6 of
+// an item's time (see attn_item) with no partial states and no fold kernel, where they fit the round side by side.  It
+// wins over the cut along the keys while items are short (about 70 key tiles at half a round) and needs no 16 tiles: us
+// per layer call, cut along the keys or not at all -> along the rows: 24 heads x 1000 queries x 4 chunks, D = 64 44.0 ->
+// 39.3; 30 heads x 1100 x 2, D = 128 73.2 -> 65.2, D = 64 44.4 -> 40.4; 10 heads x 1100 x 2, D = 64 30.2 -> 23.5; two samples of
+// 24 heads x 1861 x 3, D = 128 297 -> 287.  The planner counts short last query tiles as whole ones: counting them as 0.6
+// moved the cut of the last round by half an item and lost 1 ... 6 % (24 heads x 3700 x 4, D = 128 583 against 607).
 // Launches of less than a round that used to run unsplit (us, before -> now): 1 head x 8000 queries x 8000 keys, D = 128
 // 140 -> 49; 3 heads x 2048 x 4096 77 -> 36; 10 heads x 1154 queries, two states over 1 and 2 chunks of 1154 keys 53 -> 45;
 // 4 heads x 5777 queries x 4 chunks of 5777 keys (368 work items, 23 per head) 270 -> 250.
 static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus, int64_t slots_cap) {
-  constexpr double kPartOverheadOneRound = 6.0, kPartOverheadRounds = 10.0;
+  constexpr double kPartOverheadOneRound = 6.0, kPartOverheadRounds = 10.0, kHalfItem = 0.6;
   const double fold_overhead = D == 128 ? 6.0 : 4.0;
   const int last = size[n_jobs - 1].tiles, last_rows = size[n_jobs - 1].rows;
   if (last < 1 || (int64_t)n_jobs * a.per_xcd >= INT32_MAX) return;
@@ -1284,9 +1369,9 @@ static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int c
     T = last;
     if (rem > same * a.per_xcd) return;
   }
-  if (rem <= 0 || T < 16) return;
+  if (rem <= 0) return;
   double best = 0.1 * T;   // least gain worth the extra kernel
-  for (int w = 2; w <= 16; ++w) {
+  for (int w = 2; T >= 16 && w <= 16; ++w) {
     if ((int64_t)rem * kXcds * w > slots_cap || T / w < 6) break;
     const int rounds = (rem * w + cus - 1) / cus;
     const double part = (double)T / w, overhead = rounds == 1 ? kPartOverheadOneRound : kPartOverheadRounds;
@@ -1296,6 +1381,12 @@ static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int c
       a.tail_items = rem;
       a.part_ways = w;
     }
+  }
+  const double gain_rows = (1.0 - kHalfItem) * T - 2.0;
+  if (!a.q_prescaled && 2 * rem <= cus && last_rows > kBQ / 2 && T >= kMinSplitTiles && gain_rows > (a.tail_items > 0 ? best : 0.0)) {
+    a.tail_items = rem;
+    a.part_ways = 2;
+    a.row_split = 1;
   }
   if (a.tail_items > 0) a.tail_start = n_jobs * a.per_xcd - a.tail_items;
 }
@@ -1315,6 +1406,7 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   a.tail_start = INT32_MAX;
   a.tail_items = 0;
   a.part_ways = 0;
+  a.row_split = 0;
   constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
   const int64_t slot_bytes = (int64_t)kBQ * D * 4 + (int64_t)kBQ * 4;
   if (n_jobs <= kMaxLaunchJobs) {
@@ -1329,13 +1421,15 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);
   const int64_t slots = (int64_t)a.tail_items * kXcds * a.part_ways;
   // (the planner only considers splits that fit, so this cannot fire; it guards later edits to it)
-  if (slots * slot_bytes > workspace_bytes) {
+  if (!a.row_split && slots * slot_bytes > workspace_bytes) {
     set_error("internal: tail split of %lld parts needs %lld bytes of scratch, %lld are there", (long long)slots,
               (long long)(slots * slot_bytes), (long long)workspace_bytes);
     return DT_ERR_INVALID;
   }
-  a.ws_out = static_cast<float*>(workspace);
-  a.ws_lse = a.ws_out + slots * kBQ * D;
+  if (!a.row_split) {
+    a.ws_out = static_cast<float*>(workspace);
+    a.ws_lse = a.ws_out + slots * kBQ * D;
+  }
   if (a.tail_start <= 0) {   // every item is split: no job planes
     a.tail_start = 0;
     a.job_planes = 0;
@@ -1343,6 +1437,7 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   // parts per XCD, spread over planes of per_xcd entries
   const int part_planes = (a.tail_items * a.part_ways + a.per_xcd - 1) / a.per_xcd;
   if (int rc = launch_dim(a, D, dim3(planes_x, (unsigned)(a.job_planes + part_planes), 1), stream)) return rc;
+  if (a.row_split) return DT_OK;
   const dim3 fold_grid((unsigned)a.tail_items * kXcds * kWaves * (D / 64)), fold_block(kFoldThreads);
   if (D == 128) {
     if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<128, true>), fold_grid, fold_block, 0, stream, a);

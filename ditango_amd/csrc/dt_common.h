@@ -16,7 +16,7 @@ struct AttnChunk {
   const uint16_t* v;
   int64_t sb;       // batch stride, elements
   int32_t len;      // keys
-  int32_t unused;
+  int32_t row_split;    // the tail items are cut in two along the query rows instead of along the keys (no partial states)
 };
 struct AttnEntry {
   int32_t chunk;
@@ -48,6 +48,7 @@ struct AttnArgs {
   // as one workgroup each; the tail_items behind them run as part_ways workgroups over disjoint ranges of key
   // tiles, in grid planes of their own behind the job planes (same launch, so a part starts as soon as a CU is
   // free).  The parts write fp32 partial states into the workspace and a small second kernel folds them into the destination.
+  // With row_split the two parts of an item are its two halves of the query rows instead: no partial states, no fold.
   int32_t job_planes;  // grid planes (blockIdx.y) that are jobs (0: every item is split); planes behind them hold parts
   int32_t tail_start;  // INT32_MAX: nothing is split
   int32_t tail_items;  // per XCD
@@ -79,7 +80,7 @@ struct AttnArgs {
   int32_t B;
   int32_t q_prescaled;  // the caller folded scale_log2 into q: scores are already in log2 units
   int32_t elem_f16;     // the 16-bit tensors are IEEE half instead of bfloat16
-  int32_t unused;
+  int32_t row_split;    // the tail items are cut in two along the query rows instead of along the keys (no partial states)
   // ---- tables
   AttnJob job[DT_MAX_JOBS];
   AttnChunk chunk[DT_MAX_CHUNKS];

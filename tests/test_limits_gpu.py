@@ -238,6 +238,73 @@ def test_split_launches_match_plain_launch_and_oracle(hip, D, H, Sq, lens, jobs,
         _check(bo[:, rows.cuda()], bl[:, :, rows.cuda()], ref_out, ref_lse, f"split job {j}")
 
 
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (128, torch.float16), (64, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("lens", [[97], [449], [479], [480], [481], [512, 65], [200, 0, 320, 97], [0, 460]])
+def test_query_tiles_of_half_the_rows_match_whole_tiles_and_oracle(hip, D, dtype, lens):
+    """Query tiles of up to 128 rows share their keys (from 8 tiles of them on) between the two wavefront groups: every row against the same rows as
+    part of a tile of 256 and against the oracle, inputs read in place out of fused projections.  The reference maximum
+    differs between the two forms, so P does by its rounding: 2^-7 of the largest value as above."""
+    H, B = 3, 2
+    g = torch.Generator().manual_seed(D + sum(lens))
+    qkv = torch.randn(B, 256, 3, H, D, generator=g).to(dtype)
+    q = qkv[:, :, 0]
+    kvs = [torch.randn(B, n, 2, H, D, generator=g).to(dtype) for n in lens]
+    dev = [x.cuda() for x in kvs]
+    table = hip.ChunkTable([x[:, :, 0] for x in dev], [x[:, :, 1] for x in dev])
+    jobs = [list(range(len(lens))), [0]]
+
+    def states(rows):
+        outs = [torch.full((B, rows, H, D), float("nan"), dtype=dtype, device="cuda") for _ in jobs]
+        lses = [torch.full((B, H, rows), float("nan"), device="cuda") for _ in jobs]
+        hip.attn_jobs_fwd(qkv.cuda()[:, :rows, 0], table, jobs, outs, lses)
+        torch.cuda.synchronize()
+        return outs, lses
+
+    whole_o, whole_l = states(256)
+    for rows in (1, 31, 33, 128):
+        outs, lses = states(rows)
+        for j, chunks in enumerate(jobs):
+            o, w = outs[j].float(), whole_o[j][:, :rows].float()
+            wl = whole_l[j][:, :, :rows]
+            if sum(lens[c] for c in chunks) == 0:
+                assert (o == 0).all() and (lses[j] == float("-inf")).all()
+                continue
+            assert (o - w).abs().max() <= 2.0 ** -7 * w.abs().max()
+            assert (lses[j] - wl).abs().max() <= 1e-5
+            live = [c for c in chunks if lens[c]]
+            ref_out, ref_lse = om.full_attention(q[:, :rows].float(), [kvs[c][:, :, 0].float() for c in live], [kvs[c][:, :, 1].float() for c in live])
+            _check(o, lses[j], ref_out, ref_lse, f"{rows} rows, job {j}")
+
+
+@pytest.mark.parametrize("D,H,Sq,lens,dtype", [
+    (128, 2, 129, [450], torch.bfloat16), (128, 9, 256, [500, 97], torch.float16), (128, 3, 257, [450, 450], torch.bfloat16),
+    (64, 2, 129, [450], torch.float16), (64, 9, 256, [500, 97], torch.bfloat16), (64, 17, 511, [600], torch.bfloat16),
+    (128, 40, 900, [450, 450], torch.bfloat16),   # 160 items a job: 8 of the 40 per XCD run in the second round, in halves
+])
+def test_tail_items_cut_along_the_rows_match_plain_launch_and_oracle(hip, D, H, Sq, lens, dtype):
+    """The workspace launch of few key tiles runs its last items as two workgroups of 128 rows.  Bounds as above."""
+    g = torch.Generator().manual_seed(D + Sq + H)
+    q = torch.randn(1, Sq, H, D, generator=g).to(dtype)
+    ks, vs = ([torch.randn(1, n, H, D, generator=g).to(dtype) for n in lens] for _ in range(2))
+    table = hip.ChunkTable([k.cuda() for k in ks], [v.cuda() for v in vs])
+    jobs = [[c] for c in range(len(lens))]
+    res = []
+    for ws in (None, hip.attn_workspace("cuda")):
+        outs = [torch.full((1, Sq, H, D), float("nan"), dtype=dtype, device="cuda") for _ in jobs]
+        lses = [torch.full((1, H, Sq), float("nan"), device="cuda") for _ in jobs]
+        hip.attn_jobs_fwd(q.cuda(), table, jobs, outs, lses, workspace=ws)
+        torch.cuda.synchronize()
+        res.append((outs, lses))
+    assert any(not torch.equal(a, b) for a, b in zip(res[0][0], res[1][0])), "the launch was expected to be split"
+    for j, chunks in enumerate(jobs):
+        po, bo = res[0][0][j].float(), res[1][0][j].float()
+        assert torch.isfinite(bo).all()
+        assert (po - bo).abs().max() <= 2.0 ** -7 * po.abs().max()
+        assert (res[0][1][j] - res[1][1][j]).abs().max() <= 1e-5
+        ref_out, ref_lse = om.full_attention(q.float(), [ks[c].float() for c in chunks], [vs[c].float() for c in chunks])
+        _check(bo, res[1][1][j], ref_out, ref_lse, f"job {j}")
+
+
 @pytest.mark.parametrize("sched", [False, True])
 def test_split_varlen_launches_match_plain_launch(hip, sched):
     """Device-resident boundaries with a workspace: the parts read them as the whole items do.  Bound as above."""
