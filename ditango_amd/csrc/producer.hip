@@ -25,6 +25,8 @@ constexpr int kThreads = 256;
 // are 2.2 rounds of the chip).  HBM-bound; us per launch with 8 / 4 / 2 heads: 14882 x 24 heads of 128 41.7 / 39.5 / 41.3,
 // 12444 x 48 of 64 35.8 / 31.8 / 32.3, 9000 x 20 of 128 26.9 / 23.6 / 22.5, 119056 x 24 of 128 (6.0 TB/s) 262 / 260 / 278.
 constexpr int kHeads = 4;
+// 80 registers; 7 or 8 wavefronts would spill 24 or more of them.
+constexpr int kWavesPerSimd = 6;
 
 struct PrepArgs {
   const uint16_t* x;   // bfloat16, or IEEE half (DT_IO_FP16)
@@ -90,17 +92,49 @@ __device__ __forceinline__ void load_weights8(const void* base, bool w16, int d0
   }
 }
 
+// DPP: lane i of every row of 16 reads another lane of that row inside the vector instruction itself, where __shfl is an LDS
+// access.  Only whole groups of 8 or 16 neighbouring lanes leave the kernel early, so the lanes read are active.
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e;                 // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int kDppHalfMirror = 0x141, kDppMirror = 0x140;       // i -> 7 - i within 8 lanes, i -> 15 - i within 16
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), kCtrl, 0xf, 0xf, true));
+}
+
+// Sum over the lane group, the same in all of its lanes: neighbours, pairs, quads (all lanes of a quad agree by then, so the
+// mirrored lane is as good as lane ^ 4) and halves, the order and the bits of a butterfly with __shfl_xor.
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int m = 1; m < G; m <<= 1) v += __shfl_xor(v, m);
+  static_assert(G == 8 || G == 16, "a lane group is 8 or 16 lanes");
+  v += dpp<kDppXor1>(v);
+  v += dpp<kDppXor2>(v);
+  v += dpp<kDppHalfMirror>(v);
+  if constexpr (G == 16) v += dpp<kDppMirror>(v);
   return v;
+}
+
+// 1 / sqrt(ss / D + eps) of four rows.  The square root and the division are some 25 instructions at full precision, and all
+// lanes of a group would do the same ones: lane i of a quad takes row i and the quad exchanges the results.
+// With the LDS butterfly and a root per row the kernel took as long for its arithmetic as for its bytes; us per launch before, with
+// the sums by DPP, and with the shared roots too: 14882 tokens x 24 heads of 128 35.2 / 34.5 / 34.1, 119056 x 24 256 / 245 / 240
+// (6.6 TB/s), 9000 x 20 20.3 / 19.6 / 19.3, 12444 x 48 of 64 with LayerNorm 30.0 / 28.9 / 28.7; 14882 x 24 without a norm 32.8.
+// (The sums come as values: from an array the compiler makes the choice one of addresses and the array a piece of LDS, which
+// costs every launch 8 us.)
+template <int D>
+__device__ __forceinline__ void inverse_rms4(float s0, float s1, float s2, float s3, float eps, float (&rs)[4]) {
+  const int i = threadIdx.x & 3;
+  const float lo = i & 1 ? s1 : s0, hi = i & 1 ? s3 : s2;
+  const float mine = 1.0f / sqrtf((i & 2 ? hi : lo) * (1.0f / D) + eps);
+  rs[0] = dpp<0x00>(mine);   // quad_perm [0,0,0,0] ... [3,3,3,3]
+  rs[1] = dpp<0x55>(mine);
+  rs[2] = dpp<0xaa>(mine);
+  rs[3] = dpp<0xff>(mine);
 }
 
 // One lane group of D/8 lanes handles up to kHeads heads of one token; a lane owns the
 // 8 consecutive elements [8c, 8c+8) of each of those rows.
 template <int D, bool kHalf>
-__global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(const PrepArgs a) {
+__global__ __launch_bounds__(kThreads, kWavesPerSimd) void qk_norm_rope_kernel(const PrepArgs a) {
   constexpr int G = D / 8;
   const int c = threadIdx.x % G;
   const int hgroups = (a.H + kHeads - 1) / kHeads;
@@ -119,7 +153,7 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(const PrepArgs a
   u32x4 raw[kHeads];
 #pragma unroll
   for (int r = 0; r < kHeads; ++r)
-    if (r < nh) raw[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xp + (int64_t)r * a.xs_h));
+    raw[r] = r < nh ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xp + (int64_t)r * a.xs_h)) : u32x4{0, 0, 0, 0};
 
   const bool do_rope = a.rope != DT_ROPE_NONE && s >= a.rope_begin && s < a.rope_end;
   float cs[8], sn[8];
@@ -159,6 +193,33 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(const PrepArgs a
   const bool round_norm = (a.rounding & DT_ROUND_NORM_BF16) != 0;
   const bool round_rope = (a.rounding & DT_ROUND_ROPE_BF16) != 0;
 
+  // the statistics of all rows first: four independent chains
+  static_assert(kHeads == 4, "inverse_rms4 takes four rows");
+  float mean[kHeads] = {}, rs[kHeads] = {}, ss[kHeads];
+  if (a.norm != DT_NORM_NONE) {   // uniform
+#pragma unroll
+    for (int r = 0; r < kHeads; ++r) {
+      float v[8];
+      unpack8<kHalf>(raw[r], v);
+      if (a.norm == DT_NORM_LAYER) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum += v[i];
+        mean[r] = group_sum<G>(sum) * (1.0f / D);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] -= mean[r];
+      }
+      float t = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t += v[i] * v[i];
+      ss[r] = group_sum<G>(t);
+    }
+    inverse_rms4<D>(ss[0], ss[1], ss[2], ss[3], a.eps, rs);
+    // the rows stay packed in between: 16 registers instead of 32
+#pragma unroll
+    for (int r = 0; r < kHeads; ++r) asm volatile("" : "+v"(raw[r]));
+  }
+
   uint16_t* yp = a.y + (((int64_t)b * a.S + s) * a.H + h0) * D + d0;
 #pragma unroll
   for (int r = 0; r < kHeads; ++r) {
@@ -166,35 +227,18 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(const PrepArgs a
     float v[8];
     unpack8<kHalf>(raw[r], v);
     if (a.norm == DT_NORM_RMS) {
-      float ss = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
-      ss = group_sum<G>(ss);
-      const float rs = 1.0f / sqrtf(ss * (1.0f / D) + a.eps);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        float t = v[i] * rs;
+        float t = v[i] * rs[r];
         if (round_norm) t = round16<kHalf>(t);
         t *= w[i];
         if (round_norm) t = round16<kHalf>(t);
         v[i] = t;
       }
     } else if (a.norm == DT_NORM_LAYER) {
-      float sum = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) sum += v[i];
-      const float mean = group_sum<G>(sum) * (1.0f / D);
-      float ss = 0.0f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        v[i] -= mean;
-        ss += v[i] * v[i];
-      }
-      ss = group_sum<G>(ss);
-      const float rs = 1.0f / sqrtf(ss * (1.0f / D) + a.eps);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float t = v[i] * rs * w[i] + bias[i];
+        float t = (v[i] - mean[r]) * rs[r] * w[i] + bias[i];
         if (round_norm) t = round16<kHalf>(t);
         v[i] = t;
       }

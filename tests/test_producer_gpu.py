@@ -239,3 +239,22 @@ def test_norm_parameters_in_the_dtype_of_x_are_read_in_place(hip, D, H, dtype, n
     assert torch.equal(prepare_qk(x, weight=w.float(), bias=b, **kw), want)
     with pytest.raises(hip.DitangoHipError):
         hip.qk_norm_rope(x, norm=P.NORM_RMS, weight=w)   # without the flag the binding takes fp32 only
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H", [2, 3, 6, 7])
+@pytest.mark.parametrize("norm", [P.NORM_RMS, P.NORM_LAYER])
+def test_a_row_does_not_depend_on_the_heads_beside_it(hip, D, H, norm):
+    """The statistics of four heads are computed together: every head equals the same head alone bit for bit, next to rows of
+    other magnitudes, of zeros and with an infinity."""
+    g = torch.Generator().manual_seed(D + H)
+    x = torch.randn(2, 11, H, D, generator=g) * torch.logspace(-3, 3, H)[None, None, :, None]
+    x[0, 3, H // 2] = 0.0
+    x[1, 5, 0, 7] = float("inf")
+    x = x.bfloat16().to(DEV)
+    y = _run(hip, x, norm=norm, eps=1e-6)
+    for h in range(H):
+        alone = _run(hip, x[:, :, h:h + 1], norm=norm, eps=1e-6)
+        assert torch.equal(y[:, :, h:h + 1].isnan(), alone.isnan())
+        assert torch.equal(y[:, :, h:h + 1].nan_to_num(), alone.nan_to_num()), h
+    assert y[1, 5, 1:].isfinite().all() and not y[1, 5, 0].isfinite().all()
