@@ -369,7 +369,8 @@ __device__ __forceinline__ KeyRef key_ref(const JobView& v, int seg) {
   } else {
     r.cid = v.single;
     r.begin = 0;
-    if (v.vseg >= 0) {
+    // (with boundaries in device memory the table holds no ranges, and (chunk, segment) pairs are not bounded by its size)
+    if (v.vseg >= 0 && v.dseg < 0) {
       r.begin = a.entry[v.single * a.n_seg + v.vseg].kv_begin;
       r.len = a.entry[v.single * a.n_seg + v.vseg].kv_len;
     } else {

@@ -99,6 +99,37 @@ def test_segment_jobs_with_device_boundaries_equal_host_boundaries(hip, D, cu_q,
     assert torch.equal(torch.isfinite(got), finite) and (got[finite] - ref_lse[finite]).abs().max() <= LSE_TOL
 
 
+@pytest.mark.parametrize("D,C,n_seg", [(64, 2, 33), (128, 8, 13), (128, 40, 3), (64, 3, 300)])
+def test_scheduled_chunks_with_more_segments_than_the_tables_hold_equal_listed_jobs(hip, D, C, n_seg):
+    """Every scheduled chunk runs once per segment with the boundaries in device memory; (chunk, segment) pairs are only
+    limited by the launch's planes, not by the 64 chunk references a launch lists.  Each state against the same segments as
+    listed jobs, bit for bit."""
+    H, rows, keys = 1, 2 * n_seg + 5, 3 * n_seg + 4
+    g = torch.Generator(device="cuda").manual_seed(C * n_seg)
+    q = torch.randn(1, rows, H, D, generator=g, device="cuda").bfloat16()
+    ks, vs = ([torch.randn(1, keys, H, D, generator=g, device="cuda").bfloat16() for _ in range(C)] for _ in range(2))
+    table = hip.ChunkTable(ks, vs)
+    cut = lambda n, extra: torch.cat([torch.zeros(1, dtype=torch.int64), torch.arange(1, n_seg + 1) * n + extra]).to(torch.int32).cuda()
+    cu_q, cu_kv = cut(2, 3), [cut(3, c % 4) for c in range(C)]
+    seg = hip.DeviceSegments(cu_q, cu_kv, rows)
+    scheduled = list(range(C - 1, -1, -2))
+    ids = torch.tensor(scheduled, dtype=torch.int32, device="cuda")
+    cnt = torch.tensor([len(scheduled)], dtype=torch.int32, device="cuda")
+    got_o = torch.zeros(C, 1, rows, H, D, dtype=torch.bfloat16, device="cuda")
+    got_l = torch.zeros(C, 1, H, rows, device="cuda")
+    hip.attn_sched_fwd(q, table, ids, cnt, len(scheduled), got_o, got_l, -1, None, None, dev_segments=seg)
+    ref_o, ref_l = torch.zeros_like(got_o), torch.zeros_like(got_l)
+    jobs = [(c, s) for c in scheduled for s in range(n_seg)]
+    hip.attn_jobs_fwd(q, table, [[c] for c, _ in jobs], [ref_o[c] for c, _ in jobs], [ref_l[c] for c, _ in jobs],
+                      dev_segments=seg, job_segments=[s for _, s in jobs])
+    torch.cuda.synchronize()
+    assert got_o[scheduled[0]].any() and torch.equal(got_o, ref_o) and torch.equal(got_l, ref_l)
+    c = scheduled[-1]
+    o, l = om.varlen_chunk_attention(q[0].cpu(), ks[c][0].cpu(), vs[c][0].cpu(), cu_q.tolist(), cu_kv[c].tolist())
+    assert (got_o[c, 0].float().cpu() - o).abs().max() <= OUT_TOL
+    assert (got_l[c, 0].cpu() - l)[:, :cu_q[-1]].abs().max() <= LSE_TOL
+
+
 def test_device_boundaries_are_clamped_and_checked(hip):
     """Nothing on the host reads device-resident boundaries, so the kernel clamps them to the rows and keys that
     exist: a list that overshoots both ends yields the full-range result, never a stray access.  What the host can
