@@ -146,7 +146,8 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
 #pragma unroll
     for (int j = 0; j < kKL; ++j) kf[j] = *reinterpret_cast<const f32x4*>(p + 8 * j);
   };
-  // keys 8 (r / 4) + 4 hh + r % 4 of the tile (past the end: the last key, whose probability is then 0)
+  // keys 8 (r / 4) + 4 hh + r % 4 of the tile; past the end zeros, not some key: their probability is 0, and 0 times an
+  // infinity would be NaN
   auto load_v = [&]() __attribute__((always_inline)) {
     if (k0 + kTile <= len) {
       const float* p = vb + (int64_t)k0 * ss;
@@ -156,8 +157,11 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
         vf[r] = *reinterpret_cast<const vvec*>(p + (int64_t)(8 * (r >> 2) + (r & 3)) * ss + lane_off);
     } else {
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        vf[r] = *reinterpret_cast<const vvec*>(vb + (int64_t)min(k0 + 8 * (r >> 2) + 4 * hh + (r & 3), len - 1) * ss + kNB * col);
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+        vf[r] = *reinterpret_cast<const vvec*>(vb + (int64_t)min(key, len - 1) * ss + kNB * col);
+        if (key >= len) vf[r] = 0.f;
+      }
     }
   };
 

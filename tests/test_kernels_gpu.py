@@ -120,6 +120,30 @@ def test_fp32_jobs_match_fp64_closed_form(hip, B, Sq, H, D, lens, jobs):
         assert (lse.double().cpu() - ref_lse).abs().max().item() <= 1e-5, job
 
 
+@pytest.mark.parametrize("B,Sq,H,D,lens,job", [
+    (1, 64, 2, 64, [33], [0]),            # the key behind the last whole tile
+    (1, 40, 1, 128, [63, 5], [0, 1]),     # both chunks end inside a tile
+    (2, 1024, 48, 64, [70], [0]),         # the form without a key split
+    (1, 1025, 48, 128, [40, 97], [1, 0]),
+])
+def test_fp32_infinite_values_stay_what_the_formula_gives(hip, B, Sq, H, D, lens, job):
+    """V holds +inf / -inf in one element of the last key of every chunk: every probability is positive, so that column of the
+    output is that infinity and every other one the same as with a finite value there."""
+    g = torch.Generator().manual_seed(Sq + D)
+    q = torch.randn(B, Sq, H, D, generator=g)
+    ks, vs = ([torch.randn(B, n, H, D, generator=g) for n in lens] for _ in range(2))
+    dq, dk, dv = q.cuda(), [k.cuda() for k in ks], [v.cuda() for v in vs]
+    [(want, want_lse)] = hip.attn_jobs_f32_fwd(dq, dk, dv, [job])
+    for i, v in enumerate(dv):
+        v[:, -1, :, 3 + i] = float("inf") if i == 0 else float("-inf")
+    [(out, lse)] = hip.attn_jobs_f32_fwd(dq, dk, dv, [job])
+    want = want.clone()
+    for i in range(len(dv)):
+        want[..., 3 + i] = float("inf") if i == 0 else float("-inf")
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+
+
 def test_chunk_attention_strided_inputs(hip):
     """q/k/v as slices of a fused [B,S,3,H,D] projection (non-contiguous token stride)."""
     B, S, H, D = 1, 300, 2, 128
