@@ -200,7 +200,8 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     if (__any(mx > m)) {
       const float m_new = fmaxf(m, mx);
-      const float alpha = __builtin_amdgcn_exp2f((m - m_new) * c);   // exp2(-inf) = 0 on the first tile
+      // exp2(-inf) = 0 on the first tile; a row that has met nothing but scores of -inf has nothing to rescale
+      const float alpha = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m - m_new) * c) : 1.f;
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < kNB; ++i)
@@ -208,10 +209,12 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
         for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
       m = m_new;
     }
-    // the difference first, then the scale: the exponent is exact to its own rounding however large the scores are
+    // the difference first, then the scale: the exponent is exact to its own rounding however large the scores are (and
+    // exp2(-inf - 0) = 0 for a row of which all scores so far are -inf)
+    const float ref = m > -INFINITY ? m : 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f((s[r] - m) * c);
+      s[r] = __builtin_amdgcn_exp2f((s[r] - ref) * c);
       l += s[r];
     }
 #pragma unroll

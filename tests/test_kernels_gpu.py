@@ -144,6 +144,35 @@ def test_fp32_infinite_values_stay_what_the_formula_gives(hip, B, Sq, H, D, lens
     assert torch.equal(out, want) and torch.equal(lse, want_lse)
 
 
+@pytest.mark.parametrize("B,Sq,H,D,lens,job,dead", [
+    (1, 40, 2, 64, [64], [0], [(0, 0, 32)]),                  # the first tile of one wavefront's keys, the second is another's
+    (1, 33, 1, 128, [300, 70], [0, 1], [(0, 0, 40), (0, 128, 160), (1, 32, 70)]),
+    (2, 1024, 48, 64, [64], [0], [(0, 0, 32)]),               # the form without a key split
+    (2, 1024, 48, 64, [64], [0], [(0, 0, 64)]),               # no key at all is left
+])
+def test_fp32_scores_of_minus_infinity_weigh_nothing(hip, B, Sq, H, D, lens, job, dead):
+    """Whole key tiles whose scores are -inf (their K overflows against a positive q) leave the softmax over the other keys,
+    to the 1e-5 of fp32 sums; rows without any other key get the empty state."""
+    g = torch.Generator().manual_seed(Sq + D)
+    q = torch.randn(B, Sq, H, D, generator=g)
+    q[..., 0] = q[..., 0].abs() + 2.0
+    ks, vs = ([torch.randn(B, n, H, D, generator=g) for n in lens] for _ in range(2))
+    keep = [torch.ones(n, dtype=torch.bool) for n in lens]
+    for c, a, b in dead:
+        ks[c][:, a:b] = 0.0
+        ks[c][:, a:b, :, 0] = float("-inf")
+        keep[c][a:b] = False
+    [(out, lse)] = hip.attn_jobs_f32_fwd(q.cuda(), [k.cuda() for k in ks], [v.cuda() for v in vs], [job])
+    if not any(k.any() for k in keep):
+        assert (out == 0).all() and torch.isneginf(lse).all()
+        return
+    k, v = (torch.cat([t[c][:, keep[c]] for c in job], 1) for t in (ks, vs))
+    rows = torch.arange(0, Sq, max(1, Sq // 64))
+    ref_out, ref_lse = om.chunk_attention(q[:, rows], k, v, compute_dtype=torch.float64)
+    assert (out[:, rows.cuda()].double().cpu() - ref_out).abs().max().item() <= 1e-5
+    assert (lse[:, :, rows.cuda()].double().cpu() - ref_lse).abs().max().item() <= 1e-5
+
+
 def test_chunk_attention_strided_inputs(hip):
     """q/k/v as slices of a fused [B,S,3,H,D] projection (non-contiguous token stride)."""
     B, S, H, D = 1, 300, 2, 128
