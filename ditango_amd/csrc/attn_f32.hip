@@ -151,7 +151,7 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   auto load_v = [&]() __attribute__((always_inline)) {
     if (k0 + kTile <= len) {
       const float* p = vb + (int64_t)k0 * ss;
-      const uint32_t lane_off = (uint32_t)(4 * hh) * (uint32_t)ss + (uint32_t)(kNB * col);
+      const int64_t lane_off = 4 * hh * ss + kNB * col;   // (a token stride may be any number of elements)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         vf[r] = *reinterpret_cast<const vvec*>(p + (int64_t)(8 * (r >> 2) + (r & 3)) * ss + lane_off);

@@ -173,6 +173,29 @@ def test_fp32_scores_of_minus_infinity_weigh_nothing(hip, B, Sq, H, D, lens, job
     assert (lse[:, :, rows.cuda()].double().cpu() - ref_lse).abs().max().item() <= 1e-5
 
 
+def test_fp32_token_strides_beyond_32_bits(hip):
+    """Keys 2^30 elements apart (4 GiB), in tiles that end inside the chunk and in whole ones: the same states as from a
+    dense copy."""
+    Sk, D, stride = 33, 64, 2 ** 30
+    need = (Sk - 1) * stride + 2 * D
+    if torch.cuda.mem_get_info()[0] < 4 * need + (32 << 30):
+        pytest.skip("needs 160 GiB of device memory")
+    g = torch.Generator().manual_seed(30)
+    q = torch.randn(1, 40, 1, D, generator=g).cuda()
+    kv = torch.randn(2, 1, Sk, 1, D, generator=g).cuda()
+    far = torch.empty(need, device="cuda")
+    try:
+        k, v = (far.as_strided((1, Sk, 1, D), (Sk * stride, stride, D, 1), i * D) for i in (0, 1))
+        k.copy_(kv[0])
+        v.copy_(kv[1])
+        [(out, lse)] = hip.attn_jobs_f32_fwd(q, [k], [v], [[0]])
+        [(want, want_lse)] = hip.attn_jobs_f32_fwd(q, [kv[0]], [kv[1]], [[0]])
+        assert torch.equal(out, want) and torch.equal(lse, want_lse)
+    finally:
+        del far, k, v
+        torch.cuda.empty_cache()
+
+
 def test_chunk_attention_strided_inputs(hip):
     """q/k/v as slices of a fused [B,S,3,H,D] projection (non-contiguous token stride)."""
     B, S, H, D = 1, 300, 2, 128
