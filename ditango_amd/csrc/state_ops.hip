@@ -789,12 +789,15 @@ static void launch_merge_d(const MergeArgs& a, bool tiled, int passes, unsigned 
 }
 
 // Largest fp32 destination that is left in the 256 MB of memory-side cache: a running state (one block opens it, every
-// further one is merged into it) is read again by the next update, so its stores carry no non-temporal hint.  Its reads
-// keep the hint, the version that was read is dead.  Three updates of a bf16 block, plain against non-temporal stores (us):
-// state of 170 MB 197 -> 186, 184 MB 212 -> 203, 246 MB 278 -> 263; 367 MB, which no longer fits, 404 -> 418.  A merge of
-// more states is a layer's result, whose stores would only push out what it still has to read (8 states of 91 MB into
-// 184 MB: 204 -> 224), so those keep the hint at any size.
-constexpr int64_t kKeepBytes = 256 << 20;
+// further one is merged into it) is read again by the next update of a ring loop, so its stores carry no non-temporal hint.
+// Its reads keep the hint, the version that was read is dead.  Between two updates the loop launches the attention of a
+// chunk, whose q, K, V and result are twice the state's bytes, so a state of more than some 60 MB is gone by then and stores
+// without the hint only cost.  Ring loop of 8 chunks, each an attention launch and an update, with the hint -> without (us;
+// in brackets an update behind an attention launch): state of 20 MB 438 -> 434 (14.9 -> 14.0), 27 MB 602 -> 594 (19.6 ->
+// 17.6), 41 MB 1411 -> 1399 (25.7 -> 24.0), 50 MB 1861 -> 1846 (32.6 -> 31.5), 61 MB 2355 -> 2359, 74 MB 3682 -> 3689, 168 MB
+// 8652 -> 8690 (78.4 -> 79.5).  A state that is not read again soon pays 5 to 10 % (27 MB 16.2 -> 16.1 us, 55 MB 28.2 -> 30.0,
+// 183 MB 82.1 -> 87.6).  Merges of more states, a layer's result, keep the hint at any size.
+constexpr int64_t kKeepBytes = 48 << 20;
 static bool keeps_destination(const MergeArgs& a, int D) {
   const bool running = a.n == 1 || (a.n == 2 && a.fp32_mask != 0);
   return running && a.dst_dtype == DT_FP32 && (int64_t)a.B * a.Sq * a.H * D * 4 <= kKeepBytes;
