@@ -48,8 +48,22 @@ struct Name {
       fail(text(__VA_ARGS__));          \
   } while (0)
 
-void check(int rc, const char* what) {
+// A call of the C ABI, without the interpreter lock: a launch that waits for room in the GPU's queue must not stop the other
+// Python threads.  (The arguments are evaluated, and checked, before it is given up.)
+template <typename... P, typename... A>
+void call(const char* what, int (*fn)(P...), A... args) {
+  int rc;
+  {
+    py::gil_scoped_release unlocked;
+    rc = fn(args...);
+  }
   if (rc != 0) fail(text(what, " failed with code ", std::to_string(rc), ": ", dt_last_error()));
+}
+#define CALL(fn, ...) call(#fn, fn, __VA_ARGS__)
+// Uninitialised memory; without the lock as well, the allocator may wait for the device.
+Tensor empty(at::IntArrayRef sizes, at::TensorOptions options) {
+  py::gil_scoped_release unlocked;
+  return at::empty(sizes, options);
 }
 
 bool is_half(const Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
@@ -283,33 +297,27 @@ void attn_jobs(const Tensor& q, const ChunkTable& table, const std::vector<std::
     begin[n] = e;
     const auto sq = q.strides();
     if (seg)
-      check(dt_attn_varlen_jobs_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
-                                       begin, chunks, segs, seg->n_seg(), static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv,
-                                       (int32_t)seg->max_q, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace),
-                                       stream_of(stream)),
-            "dt_attn_varlen_jobs_ws_fwd");
+      CALL(dt_attn_varlen_jobs_ws_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss,
+           table.sh, n, begin, chunks, segs, seg->n_seg(), static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv,
+           (int32_t)seg->max_q, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace), stream_of(stream));
     else if (no_alloc)
-      check(dt_attn_seg_jobs_noalloc_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
-                                         begin, chunks, kv_ranges ? kb : nullptr, kv_ranges ? kl : nullptr,
-                                         q_ranges ? qb : nullptr, q_ranges ? ql : nullptr, op, lp, (float)scale, flags,
-                                         stream_of(stream)),
-            "dt_attn_seg_jobs_noalloc_fwd");
+      CALL(dt_attn_seg_jobs_noalloc_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss,
+           table.sh, n, begin, chunks, kv_ranges ? kb : nullptr, kv_ranges ? kl : nullptr, q_ranges ? qb : nullptr,
+           q_ranges ? ql : nullptr, op, lp, (float)scale, flags, stream_of(stream));
     else
-      check(dt_attn_seg_jobs_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
-                                    begin, chunks, kv_ranges ? kb : nullptr, kv_ranges ? kl : nullptr, q_ranges ? qb : nullptr,
-                                    q_ranges ? ql : nullptr, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace),
-                                    stream_of(stream)),
-            "dt_attn_seg_jobs_ws_fwd");
+      CALL(dt_attn_seg_jobs_ws_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss,
+           table.sh, n, begin, chunks, kv_ranges ? kb : nullptr, kv_ranges ? kl : nullptr, q_ranges ? qb : nullptr,
+           q_ranges ? ql : nullptr, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace), stream_of(stream));
     start = end;
   }
 }
 
 Tensor new_out(const Dims& d, at::ScalarType dtype, const Tensor& like) {
-  return at::empty({d.B, d.S, d.H, d.D}, like.options().dtype(dtype));
+  return empty({d.B, d.S, d.H, d.D}, like.options().dtype(dtype));
 }
 Tensor new_lse(const Dims& d, bool bsh, const Tensor& like) {
   const auto opt = like.options().dtype(at::kFloat);
-  return bsh ? at::empty({d.B, d.S, d.H, 1}, opt) : at::empty({d.B, d.H, d.S}, opt);
+  return bsh ? empty({d.B, d.S, d.H, 1}, opt) : empty({d.B, d.H, d.S}, opt);
 }
 typedef std::vector<std::pair<Tensor, Tensor>> States;
 
@@ -425,9 +433,8 @@ States attn_states_f32(const Tensor& q, const std::vector<Tensor>& ks, const std
       lp[n] = static_cast<float*>(ptr(states[start + n].second));
     }
     REQUIRE(n > 0, "job ", std::to_string(start), " references more chunks than one launch addresses: split it and merge the parts");
-    check(dt_attn_jobs_f32_fwd(static_cast<const float*>(ptr(q)), d.B, d.S, d.H, d.D, q.stride(0), q.stride(1), q.stride(2), nc, kp, vp,
-                               lens, sb, ss, sh, n, begin, chunks, op, lp, (float)scale, stream_of(stream)),
-          "dt_attn_jobs_f32_fwd");
+    CALL(dt_attn_jobs_f32_fwd, static_cast<const float*>(ptr(q)), d.B, d.S, d.H, d.D, q.stride(0), q.stride(1), q.stride(2),
+         nc, kp, vp, lens, sb, ss, sh, n, begin, chunks, op, lp, (float)scale, stream_of(stream));
     start += n;
   }
   return states;
@@ -469,12 +476,11 @@ void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, con
     REQUIRE((int64_t)seg->cu_kv.size() == table.n, "one cu_seqlens_kv per chunk of the table");
     const int32_t* cu_kv[DT_MAX_CHUNKS];
     for (int64_t c = 0; c < table.n; ++c) cu_kv[c] = static_cast<const int32_t*>(ptr(seg->cu_kv[c]));
-    check(dt_attn_sched_varlen_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(), table.v.data(),
-                                      table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs,
-                                      ptr(slot_out), slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl,
-                                      seg->n_seg(), static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv, (int32_t)seg->max_q,
-                                      (float)scale, flags, ptr(workspace), bytes_of(workspace), stream_of(stream)),
-          "dt_attn_sched_varlen_ws_fwd");
+    CALL(dt_attn_sched_varlen_ws_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(),
+         table.v.data(), table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs, ptr(slot_out),
+         slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl, seg->n_seg(),
+         static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv, (int32_t)seg->max_q, (float)scale, flags, ptr(workspace),
+         bytes_of(workspace), stream_of(stream));
     return;
   }
   int32_t n_seg = 0, qb[DT_MAX_SEGMENTS], ql[DT_MAX_SEGMENTS], kb[DT_MAX_JOB_ENTRIES], kl[DT_MAX_JOB_ENTRIES];
@@ -490,12 +496,11 @@ void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, con
       for (const Range& x : r) { kb[e] = x.first; kl[e++] = x.second; }
     }
   }
-  check(dt_attn_sched_seg_ws_fwd(ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(), table.v.data(),
-                                 table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs, ptr(slot_out),
-                                 slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl, n_seg, n_seg ? qb : nullptr,
-                                 n_seg ? ql : nullptr, n_seg ? kb : nullptr, n_seg ? kl : nullptr, (float)scale, flags,
-                                 ptr(workspace), bytes_of(workspace), stream_of(stream)),
-        "dt_attn_sched_seg_ws_fwd");
+  CALL(dt_attn_sched_seg_ws_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(),
+       table.v.data(), table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs, ptr(slot_out),
+       slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl, n_seg, n_seg ? qb : nullptr, n_seg ? ql : nullptr,
+       n_seg ? kb : nullptr, n_seg ? kl : nullptr, (float)scale, flags, ptr(workspace), bytes_of(workspace),
+       stream_of(stream));
 }
 
 // ---- states ------------------------------------------------------------------------------------------------
@@ -512,9 +517,8 @@ struct StateList {   // the states of one merge launch
     layout[n++] = lay;
   }
   void launch(const Tensor& dst_out, const Tensor& dst_lse, const Dims& d, uint64_t stream) const {
-    check(dt_merge_states(n, out, lse, dtype, layout, ptr(dst_out), dtype_code(dst_out), static_cast<float*>(ptr(dst_lse)),
-                          lse_layout(dst_lse, d.B, d.S, d.H), d.B, d.S, d.H, d.D, stream_of(stream)),
-          "dt_merge_states");
+    CALL(dt_merge_states, n, out, lse, dtype, layout, ptr(dst_out), dtype_code(dst_out), static_cast<float*>(ptr(dst_lse)),
+         lse_layout(dst_lse, d.B, d.S, d.H), d.B, d.S, d.H, d.D, stream_of(stream));
   }
 };
 
@@ -586,10 +590,9 @@ void copy_state(const Tensor& src_out, const Tensor& src_lse, const Tensor& dst_
   const Dims d{src_out.size(0), src_out.size(1), src_out.size(2), src_out.size(3)};
   REQUIRE(dst_out.is_cuda() && dst_out.is_contiguous() && shape_is(dst_out, {d.B, d.S, d.H, d.D}),
           "the destination must be contiguous [B,Sq,H,D] on the GPU");
-  check(dt_state_copy(ptr(src_out), dtype_code(src_out), static_cast<const float*>(ptr(src_lse)), lse_layout(src_lse, d.B, d.S, d.H),
-                      ptr(dst_out), dtype_code(dst_out), static_cast<float*>(ptr(dst_lse)), lse_layout(dst_lse, d.B, d.S, d.H),
-                      d.B, d.S, d.H, d.D, stream_of(stream)),
-        "dt_state_copy");
+  CALL(dt_state_copy, ptr(src_out), dtype_code(src_out), static_cast<const float*>(ptr(src_lse)),
+       lse_layout(src_lse, d.B, d.S, d.H), ptr(dst_out), dtype_code(dst_out), static_cast<float*>(ptr(dst_lse)),
+       lse_layout(dst_lse, d.B, d.S, d.H), d.B, d.S, d.H, d.D, stream_of(stream));
 }
 void cache_store(const Tensor& src_out, const Tensor& src_lse, const Tensor& slot_out, const Tensor& slot_lse, uint64_t stream) {
   REQUIRE(is_half(slot_out), "slot_out must be contiguous bf16 or fp16 [B,Sq,H,D]");
@@ -612,9 +615,8 @@ void zero_rows_from(const Tensor& t, const Tensor& first_row, uint64_t stream) {
   REQUIRE(t.is_cuda() && t.is_contiguous() && t.dim() >= 1, "t must be a contiguous device tensor");
   REQUIRE(first_row.is_cuda() && first_row.scalar_type() == at::kInt && first_row.numel() >= 1, "first_row must be int32 on the GPU");
   const int64_t n = t.size(0);
-  check(dt_zero_rows_from(ptr(t), n, t.numel() / (n > 0 ? n : 1) * t.element_size(), static_cast<const int32_t*>(ptr(first_row)),
-                          stream_of(stream)),
-        "dt_zero_rows_from");
+  CALL(dt_zero_rows_from, ptr(t), n, t.numel() / (n > 0 ? n : 1) * t.element_size(),
+       static_cast<const int32_t*>(ptr(first_row)), stream_of(stream));
 }
 
 }  // namespace

@@ -1,0 +1,70 @@
+"""The extension module between Python and the C ABI (ditango_amd/csrc/host_binding.cpp)."""
+import os
+import re
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+_CALLS = """
+    import importlib.util, sys, threading, time
+    import torch
+    spec = importlib.util.spec_from_file_location("_ditango_host", sys.argv[1])
+    host = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(host)
+    q = torch.zeros(1, 8, 2, 64, dtype=torch.bfloat16, device="cuda")
+    o, l = torch.zeros_like(q), torch.zeros(1, 2, 8, device="cuda")
+    table = host.ChunkTable([q], [q], 0, None)
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    seg = host.Segments(i32(0, 8), [i32(0, 8)], 8)
+    jobs = lambda **kw: host.attn_jobs(q, table, [[0]], [o], [l], 0.0, None, None, None, 0, kw.get("no_alloc", False),
+                                       kw.get("seg"), [0] if "seg" in kw else None, 0)
+    sched = lambda s: host.attn_sched(q, table, i32(0), i32(1), 0, 1, o[None], l[None], -1, None, None, 0.0, None, None, None, 0, s, 0)
+    calls = {
+        "jobs": jobs, "noalloc": lambda: jobs(no_alloc=True), "varlen": lambda: jobs(seg=seg),
+        "states": lambda: host.attn_states(q, [q], [q], [[0]], 32, None, None, None, 0, None, None, 0),
+        "f32": lambda: host.attn_states_f32(q.float(), [q.float()], [q.float()], [[0]], 0.0, 0),
+        "sched": lambda: sched(None), "sched varlen": lambda: sched(seg),
+        "merge": lambda: host.merge([o], [l], None, None, torch.float32, True, 0),
+        "arena": lambda: host.merge_arena(o[None], l[None], -1, o, l, torch.float32, 0),
+        "store": lambda: host.cache_store(o.float(), l, o, l, 0),
+        "load": lambda: host.cache_load(o, l, torch.float32, True, None, None, 0),
+        "zero": lambda: host.zero_rows_from(o, i32(0), 0),
+    }
+    torch.cuda.synchronize()
+    ticks = 0
+    def tick():
+        global ticks
+        while True:
+            ticks += 1
+            time.sleep(0.002)
+    threading.Thread(target=tick, daemon=True).start()
+    for name, call in calls.items():
+        before = ticks
+        call()
+        print(name, ticks - before, flush=True)
+    torch.cuda.synchronize()
+"""
+
+
+def test_other_python_threads_run_while_a_launch_waits(tmp_path):
+    """The module next to a library of the same entry points that do nothing but wait 200 ms: a second thread that wakes up every
+    2 ms gets on in the meantime, so no call holds the interpreter lock (50 of the 100 wake-ups leave room for a slow
+    machine; with the lock held there is one at most)."""
+    shutil.copy(os.path.join(ROOT, "ditango_amd", "lib", "_ditango_host.so"), tmp_path)
+    names = set(re.findall(r"^int (dt_\w+)\(", open(os.path.join(ROOT, "include", "ditango_hip.h")).read(), re.M))
+    (tmp_path / "stub.cpp").write_text(
+        "#include <unistd.h>\nextern \"C\" {\nconst char* dt_last_error(void) { return \"\"; }\n"
+        + "".join(f"int {n}(...) {{ usleep(200000); return 0; }}\n" for n in sorted(names)) + "}\n")
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", str(tmp_path / "libditango_hip.so"), str(tmp_path / "stub.cpp")], check=True)
+    (tmp_path / "calls.py").write_text(textwrap.dedent(_CALLS))
+    run = subprocess.run([sys.executable, "-u", str(tmp_path / "calls.py"), str(tmp_path / "_ditango_host.so")],
+                         capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stderr[-2000:]
+    counts = dict(line.rsplit(" ", 1) for line in run.stdout.splitlines())
+    assert len(counts) == 12 and all(int(n) >= 50 for n in counts.values()), counts
