@@ -341,9 +341,13 @@ States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::ve
   std::vector<Range> q_ranges;
   std::vector<std::vector<Range>> kv_ranges;
   std::vector<std::pair<size_t, size_t>> folds;   // (first piece, number of pieces) of the states computed in pieces
-  const size_t n_seg = seg ? seg->n_seg() : cu_q ? cu_q->size() - 1 : 1;
+  REQUIRE(max_chunks > 0, "a piece of a job needs at least one chunk");
+  REQUIRE(!cu_q || !cu_q->empty(), "cu_seqlens_q needs at least one entry");
   REQUIRE(!cu_q || (cu_kv && cu_kv->size() == ks.size()), "one cu_seqlens_kv per chunk");
+  const size_t n_seg = seg ? seg->n_seg() : cu_q ? cu_q->size() - 1 : 1;
   for (const auto& job : jobs) {
+    for (int32_t c : job)
+      REQUIRE(c >= 0 && c < table.n, "a job references chunk ", std::to_string(c), " outside the table of ", std::to_string(table.n));
     states.emplace_back(new_out(d, q.scalar_type(), q), new_lse(d, false, q));
     const size_t first = pieces.size();
     for (size_t at = 0; at == 0 || at < job.size(); at += max_chunks) {

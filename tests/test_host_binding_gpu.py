@@ -7,6 +7,7 @@ import sys
 import textwrap
 
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -68,3 +69,20 @@ def test_other_python_threads_run_while_a_launch_waits(tmp_path):
     assert run.returncode == 0, run.stderr[-2000:]
     counts = dict(line.rsplit(" ", 1) for line in run.stdout.splitlines())
     assert len(counts) == 12 and all(int(n) >= 50 for n in counts.values()), counts
+
+
+@pytest.mark.parametrize("jobs,max_chunks,cu_q,cu_kv,says", [
+    ([[0, 2]], 32, [0, 8], [[0, 8], [0, 8]], "outside the table of 2"),
+    ([[-1]], 32, [0, 8], [[0, 8], [0, 8]], "outside the table of 2"),
+    ([[5]], 32, None, None, "outside the table of 2"),
+    ([[0, 1]], 0, None, None, "at least one chunk"),
+    ([[0, 1]], -1, None, None, "at least one chunk"),
+    ([[0]], 32, [], [[], []], "at least one entry"),
+    ([[0]], 32, [0, 8], [[0, 8]], "one cu_seqlens_kv per chunk"),
+    ([[0]], 32, [0, 8], [[0, 4, 8], [0, 8]], "as many entries"),
+])
+def test_states_of_malformed_jobs_are_refused(hip, jobs, max_chunks, cu_q, cu_kv, says):
+    """Everything is checked before it is used as an index or a step: an error, not a stray read or a loop without an end."""
+    q = torch.zeros(1, 8, 2, 64, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(hip.DitangoHipError, match=says):
+        hip.attn_states(q, [q, q], [q, q], jobs, max_chunks, None, False, cu_q, cu_kv)
