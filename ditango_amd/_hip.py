@@ -29,7 +29,7 @@ DT_MAX_JOBS = 40
 DT_MAX_JOB_ENTRIES = 64
 DT_MAX_MERGE = 64
 DT_MAX_SEGMENTS = 8
-DT_NOALLOC_TAIL_SLOTS = 512
+DT_NOALLOC_TAIL_SLOTS = 1024
 
 c_i32, c_i64, c_f32, c_vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
 _P = ctypes.POINTER

@@ -1409,7 +1409,7 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   a.part_ways = 0;
   a.row_split = 0;
   constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
-  const int64_t slot_bytes = (int64_t)kBQ * D * 4 + (int64_t)kBQ * 4;
+  const int64_t slot_bytes = partial_state_bytes(D);
   if (n_jobs <= kMaxLaunchJobs) {
     JobSize size[kMaxLaunchJobs];
     job_sizes(a, n_jobs, size);

@@ -96,13 +96,18 @@ struct AttnArgs {
 constexpr int kAttnLdsBytes128 = 163840;
 constexpr int kAttnLdsBytes64 = 81920;
 
-// Workspace bytes the tail balancing can use at most (what dt_attn_workspace_bytes reports): 775 partial states of
-// 256 queries at D = 128, 1536 at D = 64.
-constexpr int64_t kWorkspaceBytes = 1536ll * (256 * 128 * 2 + 256 * 4);
+// Bytes of one partial state of a split item: 256 queries in fp32 and their lse.
+constexpr int64_t partial_state_bytes(int D) { return 256ll * D * 4 + 256 * 4; }
 
-// The allocation-free entry point splits tails inside a device array of this many bytes (258 partial states at
-// D = 128, 512 at D = 64).
-constexpr int64_t kStaticTailBytes = (int64_t)DT_NOALLOC_TAIL_SLOTS * (256 * 128 * 2 + 256 * 4);
+// Workspace bytes the tail balancing can use at most (what dt_attn_workspace_bytes reports).
+constexpr int64_t kWorkspaceBytes = 1536 * partial_state_bytes(64);
+static_assert(kWorkspaceBytes / partial_state_bytes(64) == 1536 && kWorkspaceBytes / partial_state_bytes(128) == 773);
+
+// The allocation-free entry point splits tails inside a device array of this many bytes.  At D = 128 a tail of 17 ... 31 items
+// per XCD takes two or three parts an item, up to 500 in all: with half the array it runs unsplit (24 heads x 14882 x one
+// chunk, D = 128 2156 -> 2145 us; D = 64, 1008 parts, 1271 -> 1253).
+constexpr int64_t kStaticTailBytes = DT_NOALLOC_TAIL_SLOTS * partial_state_bytes(64);
+static_assert(kStaticTailBytes / partial_state_bytes(64) == 1024 && kStaticTailBytes / partial_state_bytes(128) == 515);
 // Device address and size of that array on the current device (looked up once per device).
 int static_tail_scratch(void** ptr, int64_t* bytes);
 

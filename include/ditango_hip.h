@@ -326,7 +326,7 @@ int dt_attn_sched_seg_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, in
  * dt_attn_seg_jobs_ws_fwd for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc): no workspace argument, the tail of the
  * launch is split inside a device array that is part of the library (DT_NOALLOC_TAIL_SLOTS partial
- * states of 256 queries x 64 fp32 + 256 lse values = 34 078 720 bytes, half as many at D = 128; held by every GPU the
+ * states of 256 queries x 64 fp32 + 256 lse values = 68 157 440 bytes, half as many at D = 128; held by every GPU the
  * library runs on until the process ends).  No counterpart in the reference.  Arguments, limits,
  * errors and results are those of dt_attn_seg_jobs_ws_fwd called with a workspace of exactly that
  * size: the split is planned to fit the array (a tail that would need more parts gets fewer), so the
@@ -339,7 +339,7 @@ int dt_attn_sched_seg_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, in
  * on one GPU (different streams or threads) race on it; order them on one stream.  Nothing in the
  * array has to start at zero (every partial state that is read was written by the same call).
  */
-#define DT_NOALLOC_TAIL_SLOTS 512
+#define DT_NOALLOC_TAIL_SLOTS 1024
 int dt_attn_seg_jobs_noalloc_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
                                  int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
                                  int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,

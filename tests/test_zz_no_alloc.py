@@ -48,3 +48,20 @@ def test_noalloc_entry_matches_workspace_entry_twice(hip):
             assert (got_l[j] - plain_l[j]).abs().max().item() <= 1e-4
         # the split really ran: the tail rows went through bf16 partial states, which shows in the last bits
         assert any(not torch.equal(got_o[j], plain_o[j]) for j in range(len(jobs))), f"case {i}: tail was not split"
+
+
+def test_noalloc_scratch_holds_a_tail_of_two_rounds(hip):
+    """26 x 16 work items on 256 CUs leave 20 per XCD, whose three parts each take 480 partial states of 132 096 bytes: the launch
+    is split as with a workspace, out and lse bit for bit, and differs from the unsplit one by the rounding of P (2^-7 of
+    the largest value)."""
+    q, ks, vs = _inputs(1, 26, 128, 4096, [8192], seed=104)
+    table = hip.ChunkTable(ks, vs)
+    res = []
+    for how in ({}, dict(workspace=hip.attn_workspace("cuda")), dict(no_alloc=True)):
+        o, l = _states(1, 1, 4096, 26, 128)
+        hip.attn_jobs_fwd(q, table, [[0]], o, l, **how)
+        torch.cuda.synchronize()
+        res.append((o[0], l[0]))
+    (plain, _), (ws, ws_l), (got, got_l) = res
+    assert torch.equal(got, ws) and torch.equal(got_l, ws_l) and not torch.equal(got, plain)
+    assert (got.float() - plain.float()).abs().max() <= 2.0 ** -7 * plain.float().abs().max()
