@@ -253,15 +253,16 @@ def attn_workspace(device) -> torch.Tensor:
     bytes).  Launches that share a workspace must be ordered on one stream; keyed by the stream, launches made on
     different streams never share one.  At most ``MAX_WORKSPACES`` streams keep theirs: the least recently used
     entry is dropped (its memory goes back to the allocator in stream order, so launches still in flight on that
-    stream are safe).  The first call on a stream allocates: make it before capturing that stream in a graph --
-    one created under capture lives in the graph's private pool and serves that launch only -- or use the allocation-free
-    entry point (``attn_jobs_fwd(..., no_alloc=True)``)."""
+    stream are safe).  A stream that is being captured in a graph uses none of them: a replay would write into a workspace that
+    eager launches of that stream may be using at the same time, or that has been dropped since.  Launches under capture get
+    memory of the graph's own pool, which the launches behind them reuse; the allocation-free entry point
+    (``attn_jobs_fwd(..., no_alloc=True)``) needs none."""
     dev = device if isinstance(device, torch.device) else torch.device(device)
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(int(load_library().dt_attn_workspace_bytes()), dtype=torch.uint8, device=dev)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (dev.type, index, _raw_stream(index))
     ws = _workspaces.pop(key, None)
-    if ws is None and torch.cuda.is_current_stream_capturing():
-        return torch.empty(int(load_library().dt_attn_workspace_bytes()), dtype=torch.uint8, device=dev)   # the graph's, not kept
     if ws is None:
         while len(_workspaces) >= MAX_WORKSPACES:
             _workspaces.pop(next(iter(_workspaces)))

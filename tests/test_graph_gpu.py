@@ -151,3 +151,37 @@ def test_noalloc_attention_replays_in_a_graph(hip):
     call(plain)
     torch.cuda.synchronize()
     assert any(not torch.equal(a, b) for a, b in zip(graphed["o"], plain["o"])), "the tail was expected to be split"
+
+
+def test_graph_does_not_hold_the_workspace_of_its_stream(hip):
+    """A launch of less than a round, split inside a workspace, captured on a stream that has one from eager launches.  That
+    workspace is dropped and its memory handed to somebody else: every replay leaves it alone and gives the eager result."""
+    H, D, Sq, Sk = 3, 128, 700, 2100
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v = (torch.randn(1, n, H, D, generator=g, device="cuda").bfloat16() for n in (Sq, Sk, Sk))
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+
+    def call():
+        return hip.attn_states(q, [k], [v], [[0]], 32, hip.attn_workspace("cuda"))[0]
+
+    with torch.cuda.stream(stream):
+        size = hip.attn_workspace("cuda").numel()
+        want = [t.clone() for t in call()]
+        plain = hip.attn_states(q, [k], [v], [[0]], 32)[0]
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out, lse = call()
+        hip.release_workspaces()
+        other = torch.full((size,), 0x5a, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    assert not torch.equal(want[0], plain[0]), "the launch was expected to be split"
+    for step in range(4):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[0]) and torch.equal(lse, want[1]), f"replay {step}"
+        damaged = int((other != 0x5a).sum())
+        assert damaged == 0, f"replay {step}"
