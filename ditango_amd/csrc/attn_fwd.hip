@@ -1152,7 +1152,17 @@ __global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const Attn
     float m_new = m;
 #pragma unroll
     for (int i = 0; i < kInFlight; ++i) {
-      if (p0 + i >= ways) l[i] = -INFINITY;
+      // Behind the last part the loads repeat it, and nothing of that may be left: 0 times an infinity would be NaN.  (Masked,
+      // not assigned in a branch: the compiler would move the loads into it, and they would no longer be in flight together.)
+      const bool there = p0 + i < ways;
+      const uint32_t mask = there ? 0xffffffffu : 0u;
+      if (!there) l[i] = -INFINITY;
+#pragma unroll
+      for (int g = 0; g < kMine; ++g) {
+        u32x4 bits = __builtin_bit_cast(u32x4, x[i][g]);
+        bits &= mask;
+        x[i][g] = __builtin_bit_cast(f32x4, bits);
+      }
       m_new = fmaxf(m_new, l[i]);
     }
     const float alpha = m > -INFINITY ? __expf(m - m_new) : 0.f;

@@ -238,6 +238,34 @@ def test_split_launches_match_plain_launch_and_oracle(hip, D, H, Sq, lens, jobs,
         _check(bo[:, rows.cuda()], bl[:, :, rows.cuda()], ref_out, ref_lse, f"split job {j}")
 
 
+def _split_and_plain(hip, q, k, v):
+    res = []
+    for ws in (None, hip.attn_workspace("cuda")):
+        o, l = torch.full_like(q, 7.0), torch.full((q.shape[0], q.shape[2], q.shape[1]), 7.0, device="cuda")
+        hip.attn_jobs_fwd(q, hip.ChunkTable([k], [v]), [[0]], [o], [l], workspace=ws)
+        torch.cuda.synchronize()
+        res.append((o, l))
+    assert not torch.equal(res[0][0], res[1][0]), "the launch was expected to be split"
+    return res
+
+
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("keys", [1600, 1900, 2100, 2600, 3100])       # 4 ... 8 parts an item: whole batches of four and remainders
+def test_infinite_values_survive_the_fold_of_split_items(hip, D, dtype, keys):
+    """V holds infinities in a few columns of the first, a middle and the last key: those columns are that infinity in every row,
+    as in the unsplit launch, and every other one is as without them."""
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    q, k, v = (torch.randn(1, n, 3, D, generator=g, device="cuda").to(dtype) for n in (700, keys, keys))
+    (_, _), (want, want_l) = _split_and_plain(hip, q, k, v)
+    want = want.clone()
+    for key, col, x in ((0, 3, float("inf")), (keys // 2, 17, float("-inf")), (keys - 1, 40, float("inf"))):
+        v[:, key, :, col] = x
+        want[..., col] = x
+    (plain, _), (out, lse) = _split_and_plain(hip, q, k, v)
+    assert torch.equal(plain.isinf(), out.isinf())
+    assert torch.equal(out, want) and torch.equal(lse, want_l)
+
+
 @pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (128, torch.float16), (64, torch.bfloat16), (64, torch.float16)])
 @pytest.mark.parametrize("lens", [[97], [449], [479], [480], [481], [512, 65], [200, 0, 320, 97], [0, 460]])
 def test_query_tiles_of_half_the_rows_match_whole_tiles_and_oracle(hip, D, dtype, lens):
