@@ -979,7 +979,8 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   if (is_part) {
     // A part's state goes to the workspace as it lies in the registers, in fp32: whole kilobytes per store, no rounding.
     const int64_t slot = ((int64_t)unit * kXcds + xcd) * e.part_ways + part;
-    if (hh == 0) e.ws_lse[slot * kBQ + wave * 32 + col] = lse;
+    // (a NaN among the scores leaves no sum: the fold has to see that, an lse of -inf would be an empty part)
+    if (hh == 0) e.ws_lse[slot * kBQ + wave * 32 + col] = l_tot == l_tot ? lse : l_tot;
     float* dst = e.ws_out + (slot * kWaves + wave) * (32 * D) + lane * 4;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
@@ -1174,7 +1175,7 @@ __global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const Attn
       for (int e = 0; e < 4; ++e) acc[g][e] *= alpha;
 #pragma unroll
     for (int i = 0; i < kInFlight; ++i) {
-      const float w = l[i] > -INFINITY ? __expf(l[i] - m) : 0.f;
+      const float w = l[i] == -INFINITY ? 0.f : __expf(l[i] - m);   // (NaN stays NaN, and with it the row's sum)
       den += w;
 #pragma unroll
       for (int g = 0; g < kMine; ++g)

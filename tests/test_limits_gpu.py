@@ -266,6 +266,27 @@ def test_infinite_values_survive_the_fold_of_split_items(hip, D, dtype, keys):
     assert torch.equal(out, want) and torch.equal(lse, want_l)
 
 
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (64, torch.float16)])
+@pytest.mark.parametrize("keys", [1600, 2100])
+def test_nan_scores_in_split_items_give_what_the_unsplit_launch_gives(hip, D, dtype, keys):
+    """A NaN in one query and, in the second head, in one key: out and lse of the rows concerned as in the unsplit launch (NaN, and
+    no sum: -inf).  A row beside it in a wavefront takes another reference maximum, so P differs by its rounding: every
+    other row is within 2^-7 of the largest value, as above."""
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    q, k, v = (torch.randn(1, n, 3, D, generator=g, device="cuda").to(dtype) for n in (700, keys, keys))
+    (_, _), (want, want_l) = _split_and_plain(hip, q, k, v)
+    q[0, 300, 0, 5] = float("nan")
+    k[0, keys - 40, 1, 7] = float("nan")
+    (plain, plain_l), (out, lse) = _split_and_plain(hip, q, k, v)
+    bad = torch.zeros(700, 3, dtype=torch.bool, device="cuda")
+    bad[300, 0] = True
+    bad[:, 1] = True
+    for o, l in ((plain, plain_l), (out, lse)):
+        assert o[0][bad].isnan().all() and torch.isneginf(l[0].T[bad]).all()
+    assert (out[0][~bad].float() - want[0][~bad].float()).abs().max() <= 2.0 ** -7 * want.float().abs().max()
+    assert (lse[0].T[~bad] - want_l[0].T[~bad]).abs().max() <= 1e-5
+
+
 @pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (128, torch.float16), (64, torch.bfloat16), (64, torch.float16)])
 @pytest.mark.parametrize("lens", [[97], [449], [479], [480], [481], [512, 65], [200, 0, 320, 97], [0, 460]])
 def test_query_tiles_of_half_the_rows_match_whole_tiles_and_oracle(hip, D, dtype, lens):
