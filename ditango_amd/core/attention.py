@@ -434,7 +434,7 @@ class proAttention:
             _hip.attn_sched_fwd(query, _hip.ChunkTable(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
                                 rm.compute_counts[t][l], cache.arena_out, cache.arena_lse, diag, cache.diag_out,
                                 cache.diag_lse, seg_q=seg_q, seg_kv=seg_kv, workspace=ws, q_prescaled=self.q_prescaled,
-                                dev_segments=dev_seg, row=t * rm.num_layers + l)
+                                dev_segments=dev_seg, row=(t % rm.num_timesteps) * rm.num_layers + l % rm.num_layers)
         else:
             # more chunks than one launch addresses: one launch per window of chunk ids (ordered on the
             # stream, so they can share the workspace)

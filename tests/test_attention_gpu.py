@@ -309,6 +309,34 @@ def test_zero_padded_shards_of_an_uneven_sequence(env, N, rank, S_total, D):
     assert (out.cpu()[:, -1] - mean_v).abs().max() <= OUT_TOL
 
 
+@pytest.mark.parametrize("T,layer,step,same_as", [(3, 0, -1, (0, 2)), (3, 1, -2, (1, 1)), (3, -1, 1, (1, 1)), (4, -2, -1, (0, 3))])
+def test_mask_mode_steps_and_layers_count_from_the_end(env, T, layer, step, same_as):
+    """A step or layer number below zero means the mask's row counted from the end, for the host's lists and for the row of the
+    device schedule alike: the same chunks are recomputed and the same result comes out, bit for bit."""
+    from ditango_amd import utils
+    from ditango_amd.core import parallel_state
+    from ditango_amd.core.attention import proAttention
+    rm = env(4, 0, T, 2)
+    mask = np.zeros((T, 2, 4), dtype=np.uint8)
+    for t in range(1, T):
+        for l in range(2):
+            mask[t, l, 1 + (t + l) % 3] = 1
+    rm.set_chunk_mask(mask, diag=0)
+    q, ks, vs = _inputs(1, 200, [90] * 4, 2, 64, seed=3)
+    q = q.bfloat16().cuda()
+    outs = []
+    for l, t in ((same_as[0], same_as[1]), (layer, step)):
+        g = torch.Generator().manual_seed(5)
+        attn = proAttention(l, parallel_state.get_usp_group())
+        for now in (0, t):                       # other K and V at the second step: the reused chunk shows in the result
+            k, v = ([x.bfloat16().cuda() + 0.5 * torch.randn(x.shape, generator=g).bfloat16().cuda() for x in xs] for xs in (ks, vs))
+            parallel_state.get_usp_group().set_kv_chunks(k, v)
+            utils.update_timestep(now)
+            out = attn.attn(q, k[0], v[0])
+        outs.append((out, attn.last_lse))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
 def test_mask_mode_cold_reuse_is_an_error(env):
     from ditango_amd.core.attention import proAttention
     from ditango_amd.core.parallel_state import get_usp_group
