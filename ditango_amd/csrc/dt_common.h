@@ -16,7 +16,6 @@ struct AttnChunk {
   const uint16_t* v;
   int64_t sb;       // batch stride, elements
   int32_t len;      // keys
-  int32_t row_split;    // the tail items are cut in two along the query rows instead of along the keys (no partial states)
 };
 struct AttnEntry {
   int32_t chunk;
@@ -36,7 +35,7 @@ struct AttnJob {
 // no host-to-device copy per call.  q, K, V and the output states are 16-bit elements: bfloat16, or IEEE half when
 // elem_f16 is set.
 struct AttnArgs {
-  // ---- what every workgroup reads: the first three cache lines
+  // ---- what the workgroups read: three cache lines and the head of the fourth
   const uint16_t* q;
   int64_t q_sb, q_ss, q_sh;
   int32_t H, Sq;
@@ -76,11 +75,11 @@ struct AttnArgs {
   float* diag_lse;
   float* ws_out;    // [slot][8 wavefronts][D / 8 groups of 4 elements][64 lanes][4], the accumulators as they lie in registers
   float* ws_lse;    // [slot][256]
+  int32_t row_split;    // the tail items are cut in two along the query rows instead of along the keys (no partial states)
   // ---- the host's own
   int32_t B;
   int32_t q_prescaled;  // the caller folded scale_log2 into q: scores are already in log2 units
   int32_t elem_f16;     // the 16-bit tensors are IEEE half instead of bfloat16
-  int32_t row_split;    // the tail items are cut in two along the query rows instead of along the keys (no partial states)
   // ---- tables
   AttnJob job[DT_MAX_JOBS];
   AttnChunk chunk[DT_MAX_CHUNKS];
