@@ -12,12 +12,17 @@ kernel itself is compiled from (ditango_amd/csrc/attn_schedule.h), and asserts
        group, a wait that covers that group's share of the loads of tile X;
   (ii) every load into a buffer is issued after a barrier that comes after the last read of the buffer's
        previous tile by any group, and after the same wavefront's earlier load into that buffer has landed;
-  (iii) both groups pass the same number of barriers, and the epilogue (which reuses the tile buffers) starts
-       behind a barrier behind every group's wait for all of its loads.
+  (iii) both groups pass the same number of barriers, every wavefront has waited for all of its loads when it ends, and
+        where the tile buffers are used once more -- the form in which the two groups share the keys of their queries hands
+        one group's accumulators to the other through them -- that starts behind a barrier behind everybody's last read and
+        everybody's wait for all loads, and is read behind a barrier behind the writes.  The plain form ends without a
+        barrier: its output goes through rows of its own beside the buffers.
 
 The order of the operations mirrors the kernel's control flow (prologue, the loop's vector and matrix phases,
-epilogue); the COUNTS come from the table.  The model must reject the schedule without the trailing group's
-explicit wait for K of tile 1 (the race that a 48-chunk parity case once showed) and accept the current one.
+the end of either form, which a test compares with the source); the COUNTS come from the table.  In the form that shares
+keys a group reads half of every tile; the model lets it read all of it, which is stricter.  The model must reject the
+schedule without the trailing group's explicit wait for K of tile 1 (the race that a 48-chunk parity case once showed),
+every form of the end with a barrier or the wait left out, and accept the current one.
 """
 import os
 import re
@@ -55,10 +60,16 @@ class Schedule:
         self.vector_inflight = table[f"VECTOR_BARRIER_INFLIGHT_{s}"]
 
 
-def wave_program(s: Schedule, group: int, n_tiles: int):
+# What a wavefront does behind the loop, in program order: (operation, group it is limited to or None).  "hand over" writes
+# the tile buffers, "take" reads what was written there.
+END_PLAIN = [("barrier", 0), ("wait", None)]
+END_SHARED_KEYS = END_PLAIN + [("barrier", None), ("hand over", 1), ("barrier", None), ("take", 0)]
+
+
+def wave_program(s: Schedule, group: int, n_tiles: int, end=END_PLAIN):
     """The operations one wavefront of ``group`` issues for a work item of ``n_tiles`` tiles, in program order:
     ("load", operand, tile, buffer) | ("wait", shares that may stay in flight) | ("barrier",) |
-    ("read", operand, buffer, tile the reader expects) | ("epilogue",)."""
+    ("read", operand, buffer, tile the reader expects) | ("hand over",) | ("take",)."""
     ops = []
 
     def load_tile(y):
@@ -90,24 +101,22 @@ def wave_program(s: Schedule, group: int, n_tiles: int):
         ops.append(("read", "K", (u + 1) % s.num_buf, t + 1))   # scores of tile t + 1
         if s.load_after_matrix:
             load_tile(t + s.call_ahead + group)
-        ops.append(("barrier",))
-    # ---- epilogue: reuses the tile buffers
-    ops.append(("wait", 0))
-    if group == 0:
-        ops.append(("barrier",))                      # the leading group waits out the phase it is ahead
-    ops.append(("barrier",))
-    ops.append(("epilogue",))
+        if t + 1 < n_tiles:
+            ops.append(("barrier",))                  # (the loop ends in front of the last one)
+    for op, only in end:
+        if only is None or only == group:
+            ops.append(("wait", 0) if op == "wait" else (op,))
     return ops
 
 
-def replay(s: Schedule, n_tiles: int):
+def replay(s: Schedule, n_tiles: int, end=END_PLAIN):
     """Replays both groups.  Returns (violations, per-group facts).  An interval is the stretch between two
     barriers: operations of different groups in the same interval are concurrent."""
     facts = []
     for group in (0, 1):
-        ops = wave_program(s, group, n_tiles)
+        ops = wave_program(s, group, n_tiles, end)
         interval, issued = 0, []        # issued: [operand, tile, buffer, issue interval, landed-by interval or None]
-        loads, reads, waw, epilogue_at, all_landed_at = [], [], [], None, None
+        loads, reads, waw, at_end = [], [], [], {}
         for op in ops:
             if op[0] == "barrier":
                 interval += 1
@@ -124,15 +133,12 @@ def replay(s: Schedule, n_tiles: int):
                 for rec in issued[:max(0, len(issued) - op[1])]:
                     if rec[4] is None:
                         rec[4] = interval + 1
-                if op[1] == 0:
-                    all_landed_at = interval + 1
             elif op[0] == "read":
                 reads.append((op[1], op[2], op[3], interval))
-            elif op[0] == "epilogue":
-                epilogue_at = interval
+            else:
+                at_end[op[0]] = interval
         loads = [tuple(r) for r in issued]
-        facts.append(dict(barriers=interval, loads=loads, reads=reads, waw=waw, epilogue_at=epilogue_at,
-                          all_landed_at=all_landed_at))
+        facts.append(dict(barriers=interval, loads=loads, reads=reads, waw=waw, at_end=at_end))
     bad = []
     if facts[0]["barriers"] != facts[1]["barriers"]:
         bad.append(("barrier count differs", facts[0]["barriers"], facts[1]["barriers"]))
@@ -159,28 +165,48 @@ def replay(s: Schedule, n_tiles: int):
                     if r_operand == operand and r_buf == buf and r_tile < tile and r_tile < n_tiles and r_at >= at:
                         bad.append((f"group {g} loads {operand} of tile {tile} into buffer {buf} in interval {at} while group {g2} "
                                     f"still reads tile {r_tile} there in interval {r_at}",))
-        # (iii) the epilogue overwrites every buffer
-        for g2, f2 in enumerate(facts):
-            if f2["all_landed_at"] is None or f2["all_landed_at"] > f["epilogue_at"]:
-                bad.append((f"group {g}'s epilogue starts in interval {f['epilogue_at']}, group {g2}'s loads have all landed from",
-                            f2["all_landed_at"]))
-            for _, _, r_tile, r_at in f2["reads"]:
-                if r_at >= f["epilogue_at"]:
-                    bad.append((f"group {g}'s epilogue overlaps a tile read of group {g2} in interval {r_at}",))
+        # (iii) nothing is in flight when a wavefront ends; the buffers are free when they are used once more
+        for operand, tile, _, _, landed in f["loads"]:
+            if landed is None:
+                bad.append((f"group {g} ends with a load of {operand} of tile {tile} in flight",))
+        written = f["at_end"].get("hand over")
+        if written is not None:
+            for g2, f2 in enumerate(facts):
+                for operand, tile, _, _, landed in f2["loads"]:
+                    if landed is None or landed > written:
+                        bad.append((f"group {g} writes the buffers in interval {written}, group {g2}'s {operand} of tile {tile} has landed from",
+                                    landed))
+                for _, _, r_tile, r_at in f2["reads"]:
+                    if r_at >= written:
+                        bad.append((f"group {g} writes the buffers in interval {written}, group {g2} reads tile {r_tile} in interval {r_at}",))
+                taken = f2["at_end"].get("take")
+                if taken is not None and taken <= written:
+                    bad.append((f"group {g2} takes in interval {taken} what group {g} writes in interval {written}",))
     return bad, facts
 
 
 TILE_COUNTS = list(range(0, 13)) + [35, 59, 233]      # short items (parts of split items are 6 tiles and up), the real shapes
 
 
+@pytest.mark.parametrize("end", [END_PLAIN, END_SHARED_KEYS], ids=["plain", "shared keys"])
 @pytest.mark.parametrize("D", [128, 64])
-def test_current_schedule_is_race_free(D):
+def test_current_schedule_is_race_free(D, end):
     s = Schedule(read_table(), D)
     for n in TILE_COUNTS:
-        bad, facts = replay(s, n)
+        bad, facts = replay(s, n, end)
         assert not bad, (D, n, bad[:3])
         # every tile that is read was loaded by both groups, K three and V two tiles ahead of its first use
         assert all(len(f["loads"]) == 2 * (s.prologue_calls[g] + n) for g, f in enumerate(facts))
+
+
+@pytest.mark.parametrize("D", [128, 64])
+def test_an_end_without_a_barrier_or_the_wait_is_rejected(D):
+    s = Schedule(read_table(), D)
+    for end in (END_PLAIN, END_SHARED_KEYS):
+        for i, (op, _) in enumerate(end):
+            if op in ("barrier", "wait"):
+                short = end[:i] + end[i + 1:]
+                assert all(replay(s, n, short)[0] for n in (1, 2, 7, 35)), (D, short)
 
 
 @pytest.mark.parametrize("D", [128, 64])
@@ -208,6 +234,20 @@ def test_weaker_or_mistimed_waits_are_rejected(D):
         table[key] += delta
         s = Schedule(table, D)
         assert any(replay(s, n)[0] for n in range(1, 13)), (D, key)
+
+
+def test_the_kernel_ends_as_the_model_does():
+    """Barriers, waits and early returns behind the loop, in the order of the source: those of the model's two forms, the second
+    behind ``if constexpr (kSplitKeys)``, and none in the epilogue, which touches no byte of the tile buffers."""
+    code = re.sub(r"//[^\n]*", "", open(KERNEL).read())
+    item = code[code.index("for (int t = 0; t < n_tiles; t += 4)"):code.index("__global__", code.index("void attn_item("))]
+    steps = re.findall(r"if \(group == ([01])\) phase_barrier|(phase_barrier|wait_tile_loads<0>)|(if constexpr \(kSplitKeys\))"
+                       r"|if \(group == ([01])\) (return)|if \(group == ([01])\) (\{)", item)
+    found = [" ".join(x for x in step if x) for step in steps]
+    assert found == ["0", "wait_tile_loads<0>", "if constexpr (kSplitKeys)", "phase_barrier", "1 {", "phase_barrier", "1 return"], found
+    epilogue = item[item.index("if (group == 1) return"):]
+    epilogue = epilogue[epilogue.index("const float l_tot"):]
+    assert re.findall(r"\blds\b[^;]*", epilogue) == ["lds + T::kLdsTiles + wave * T::kStageBytes"]
 
 
 def test_kernel_takes_every_count_from_the_table():
