@@ -1403,6 +1403,15 @@ static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int c
   if (a.tail_items > 0) a.tail_start = n_jobs * a.per_xcd - a.tail_items;
 }
 
+// Held while a split launch and its fold kernel go into the queue: two threads may launch on one stream, with the workspace
+// that belongs to it, and nothing of the other's may come between the parts and their fold.  (One of a few locks, chosen by the
+// workspace: a thread that waits for room in its stream's queue holds up few others.)
+static std::mutex& workspace_lock(const void* workspace) {
+  constexpr int kBits = 6;
+  static std::mutex locks[1 << kBits];
+  return locks[(reinterpret_cast<uintptr_t>(workspace) >> 4) * 0x9e3779b97f4a7c15ull >> (64 - kBits)];
+}
+
 int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
   if (n_jobs <= 0 || a_in.total <= 0) return DT_OK;
   if (D != 128 && D != 64) {
@@ -1448,8 +1457,10 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   }
   // parts per XCD, spread over planes of per_xcd entries
   const int part_planes = (a.tail_items * a.part_ways + a.per_xcd - 1) / a.per_xcd;
-  if (int rc = launch_dim(a, D, dim3(planes_x, (unsigned)(a.job_planes + part_planes), 1), stream)) return rc;
-  if (a.row_split) return DT_OK;
+  const dim3 grid(planes_x, (unsigned)(a.job_planes + part_planes), 1);
+  if (a.row_split) return launch_dim(a, D, grid, stream);
+  std::lock_guard<std::mutex> pair(workspace_lock(workspace));
+  if (int rc = launch_dim(a, D, grid, stream)) return rc;
   const dim3 fold_grid((unsigned)a.tail_items * kXcds * kWaves * (D / 64)), fold_block(kFoldThreads);
   if (D == 128) {
     if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<128, true>), fold_grid, fold_block, 0, stream, a);

@@ -283,8 +283,9 @@ int dt_zero_rows_from(void* dst, int64_t n_rows, int64_t row_bytes, const int32_
  * attention launch are equal pieces of work, so its last round usually fills only part of the
  * chip; with a workspace the work items of that round (all of them, in a launch of less than one
  * round) are each cut into several ranges of key tiles that run side by side and write fp32 partial
- * states into the workspace, and a small kernel folds them into the destination.  Calls that share a workspace must not overlap (same stream, or disjoint
- * workspaces).  No counterpart in the reference.
+ * states into the workspace, and a small kernel folds them into the destination.  Launches that share a
+ * workspace must not overlap on the GPU: one stream, or disjoint workspaces.  (Several threads may launch
+ * on that stream: a call puts its two kernels into the queue together.)  No counterpart in the reference.
  *
  * flags: DT_ATTN_Q_PRESCALED says that the caller has folded softmax_scale * log2(e) into q before
  * rounding it to bf16 (in the QK-norm weight, or through dt_qk_norm_rope's out_scale): the scores

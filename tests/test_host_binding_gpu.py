@@ -5,6 +5,7 @@ import shutil
 import subprocess
 import sys
 import textwrap
+import threading
 
 import pytest
 import torch
@@ -86,3 +87,37 @@ def test_states_of_malformed_jobs_are_refused(hip, jobs, max_chunks, cu_q, cu_kv
     q = torch.zeros(1, 8, 2, 64, dtype=torch.bfloat16, device="cuda")
     with pytest.raises(hip.DitangoHipError, match=says):
         hip.attn_states(q, [q, q], [q, q], jobs, max_chunks, None, False, cu_q, cu_kv)
+
+
+def test_threads_that_launch_on_one_stream_share_its_workspace(hip):
+    """Launches that are split, from two threads on one stream and so with one workspace: what one thread launches may not come
+    between the partial states of the other and their fold.  Bit for bit what one thread alone gets."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda", dtype=torch.bfloat16)
+    sizes = [(700, 2100, 3, 64), (900, 2600, 2, 64)]   # of less than a round: every item in several parts
+    inputs = [[rnd(1, sq, h, d), rnd(1, sk, h, d), rnd(1, sk, h, d)] for sq, sk, h, d in sizes]
+    run = lambda q, k, v: hip.attn_states(q, [k], [v], [[0]], 32, hip.attn_workspace("cuda"))[0]
+    want = [run(*i) for i in inputs]
+    plain = [hip.attn_states(q, [k], [v], [[0]], 32, None)[0] for q, k, v in inputs]
+    assert all(not torch.equal(w[0], p[0]) for w, p in zip(want, plain))   # they are split
+    torch.cuda.synchronize()
+    got, errors = [[], []], []
+    start = threading.Barrier(2)
+
+    def work(i):
+        try:
+            start.wait()
+            for _ in range(150):
+                got[i].append(run(*inputs[i]))
+        except Exception as e:   # noqa: BLE001 (reported by the assertion below)
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for i in range(2):
+        assert len(got[i]) == 150
+        assert all(torch.equal(o, want[i][0]) and torch.equal(l, want[i][1]) for o, l in got[i])
