@@ -80,13 +80,22 @@ def test_other_python_threads_run_while_a_launch_waits(tmp_path):
     ([[0, 1]], -1, None, None, "at least one chunk"),
     ([[0]], 32, [], [[], []], "at least one entry"),
     ([[0]], 32, [0, 8], [[0, 8]], "one cu_seqlens_kv per chunk"),
-    ([[0]], 32, [0, 8], [[0, 4, 8], [0, 8]], "as many entries"),
+    ([[0]], 32, [0, 4, 8], [[0, 8], [0, 4, 8]], "as many entries"),
 ])
 def test_states_of_malformed_jobs_are_refused(hip, jobs, max_chunks, cu_q, cu_kv, says):
     """Everything is checked before it is used as an index or a step: an error, not a stray read or a loop without an end."""
     q = torch.zeros(1, 8, 2, 64, dtype=torch.bfloat16, device="cuda")
     with pytest.raises(hip.DitangoHipError, match=says):
         hip.attn_states(q, [q, q], [q, q], jobs, max_chunks, None, False, cu_q, cu_kv)
+
+
+def test_boundaries_of_a_chunk_behind_the_last_query_segment_are_not_read(hip):
+    """A chunk's host boundaries may go on behind the segments of the queries, in the state's launch as under a reuse mask."""
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v = (torch.randn(1, n, 2, 64, generator=gen, device="cuda", dtype=torch.bfloat16) for n in (70, 90, 90))
+    state = lambda cu_kv: hip.attn_states(q, [k], [v], [[0]], 32, None, False, [0, 30, 70], [cu_kv])[0]
+    for got, want in zip(state([0, 40, 80, 90]), state([0, 40, 80])):
+        assert torch.equal(got, want)
 
 
 def test_threads_that_launch_on_one_stream_share_its_workspace(hip):
