@@ -33,7 +33,6 @@ struct MergeArgs {
   float* dst_lse;
   int32_t dst_dtype;    // DT_BF16 / DT_FP32 / DT_FP16
   int32_t dst_bsh;
-  int32_t keep;         // the destination is stored without the non-temporal hint (see launch_merge)
 };
 
 // The two 16-bit elements of a word, widened (f16: IEEE half, else bfloat16), and back (round to nearest even).
@@ -420,13 +419,8 @@ __global__ __launch_bounds__(kThreads) void merge_states_kernel(const MergeArgs 
         v0[i] = __float_as_uint(o[i]);
         v1[i] = __float_as_uint(o[4 + i]);
       }
-      if (a.keep) {   // uniform
-        if (live_lo) *reinterpret_cast<u32x4*>(q) = v0;
-        if (live_hi) *reinterpret_cast<u32x4*>(q + 64) = v1;
-      } else {
-        if (live_lo) __builtin_nontemporal_store(v0, reinterpret_cast<u32x4*>(q));
-        if (live_hi) __builtin_nontemporal_store(v1, reinterpret_cast<u32x4*>(q + 64));
-      }
+      if (live_lo) __builtin_nontemporal_store(v0, reinterpret_cast<u32x4*>(q));
+      if (live_hi) __builtin_nontemporal_store(v1, reinterpret_cast<u32x4*>(q + 64));
     } else {
       uint16_t* q = reinterpret_cast<uint16_t*>(a.dst_out) + u[p].elem + 4 * cc;
       const bool f16 = a.dst_dtype == DT_FP16;
@@ -788,24 +782,7 @@ static void launch_merge_d(const MergeArgs& a, bool tiled, int passes, unsigned 
   }
 }
 
-// Largest fp32 destination that is left in the 256 MB of memory-side cache: a running state (one block opens it, every
-// further one is merged into it) is read again by the next update of a ring loop, so its stores carry no non-temporal hint.
-// Its reads keep the hint, the version that was read is dead.  Between two updates the loop launches the attention of a
-// chunk, whose q, K, V and result are twice the state's bytes, so a state of more than some 60 MB is gone by then and stores
-// without the hint only cost.  Ring loop of 8 chunks, each an attention launch and an update, with the hint -> without (us;
-// in brackets an update behind an attention launch): state of 20 MB 438 -> 434 (14.9 -> 14.0), 27 MB 602 -> 594 (19.6 ->
-// 17.6), 41 MB 1411 -> 1399 (25.7 -> 24.0), 50 MB 1861 -> 1846 (32.6 -> 31.5), 61 MB 2355 -> 2359, 74 MB 3682 -> 3689, 168 MB
-// 8652 -> 8690 (78.4 -> 79.5).  A state that is not read again soon pays 5 to 10 % (27 MB 16.2 -> 16.1 us, 55 MB 28.2 -> 30.0,
-// 183 MB 82.1 -> 87.6).  Merges of more states, a layer's result, keep the hint at any size.
-constexpr int64_t kKeepBytes = 48 << 20;
-static bool keeps_destination(const MergeArgs& a, int D) {
-  const bool running = a.n == 1 || (a.n == 2 && a.fp32_mask != 0);
-  return running && a.dst_dtype == DT_FP32 && (int64_t)a.B * a.Sq * a.H * D * 4 <= kKeepBytes;
-}
-
-int launch_merge(const MergeArgs& a_in, int D, hipStream_t stream) {
-  MergeArgs a = a_in;
-  a.keep = keeps_destination(a, D);
+int launch_merge(const MergeArgs& a, int D, hipStream_t stream) {
   if (D != 128 && D != 64) {
     set_error("head dim %d not built (64 and 128 are)", D);
     return DT_ERR_UNSUPPORTED;

@@ -608,8 +608,8 @@ def test_rel_l1_sums_at_the_hunyuan_shape(hip):
 
 
 @pytest.mark.parametrize("rows", [1, 12288, 12289, 65536, 65537])
-def test_running_state_on_both_sides_of_the_kept_size(hip, rows):
-    """fp32 destinations of one state and of an update, up to 48 MiB (12288 rows of 8 heads of 128) and beyond."""
+def test_running_state_from_one_row_to_256_mib(hip, rows):
+    """fp32 destinations of one state and of an update, from one row to 256 MiB (65536 rows of 8 heads of 128) and a row more."""
     from ditango_amd.utils import update_out_and_lse
     g = torch.Generator(device="cuda:0").manual_seed(rows)
     blocks = [(torch.randn(1, rows, 8, 128, generator=g, device="cuda:0").bfloat16(), torch.randn(1, 8, rows, generator=g, device="cuda:0"))
