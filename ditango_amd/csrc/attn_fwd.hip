@@ -1288,25 +1288,24 @@ struct JobSize {
   int32_t tiles, rows;
 };
 
-// Puts host-listed jobs in the order that leaves the fewest idle CUs at the end: jobs with few query rows first (they
-// are gone in no time), then by falling length, so that the last work items to start are the shortest.
-static void order_jobs(AttnArgs& a, int n_jobs, JobSize* size) {
-  int order[DT_MAX_JOBS];
+// The order of host-listed jobs by falling length, those with few query rows first (they are gone in no time).  False where
+// the jobs already come like that.
+static bool longest_first(const JobSize* size, int n_jobs, int* order) {
   for (int j = 0; j < n_jobs; ++j) order[j] = j;
   auto before = [&](int x, int y) {
     return size[x].rows != size[y].rows ? size[x].rows < size[y].rows : size[x].tiles > size[y].tiles;
   };
   bool sorted = true;
   for (int j = 1; j < n_jobs; ++j) sorted = sorted && !before(j, j - 1);
-  if (sorted) return;
-  std::stable_sort(order, order + n_jobs, before);
+  if (!sorted) std::stable_sort(order, order + n_jobs, before);
+  return !sorted;
+}
+
+static void reorder_jobs(AttnArgs& a, int n_jobs, const int* order) {
   const AttnArgs o = a;
-  JobSize was[DT_MAX_JOBS];
-  std::copy(size, size + n_jobs, was);
   int e = 0;
   for (int j = 0; j < n_jobs; ++j) {
     const int from = order[j];
-    size[j] = was[from];
     a.job[j] = o.job[from];
     a.job[j].begin = e;
     for (int x = o.job[from].begin; x < o.job[from].end; ++x, ++e) a.entry[e] = o.entry[x];
@@ -1336,11 +1335,16 @@ static void job_sizes(const AttnArgs& a, int n_jobs, JobSize* size) {
   }
 }
 
-// Which work items at the end of the launch run as how many parts each (tail_start, tail_items, part_ways, row_split).
-//
+// Which work items at the end of the launch run as how many parts each.
+struct TailPlan {
+  int32_t items = 0, ways = 0;   // per XCD; parts of an item
+  bool rows = false;             // the parts are halves of the rows
+};
+
 // Time is counted in key tiles, on one XCD (workgroups go to the XCDs in turn, so each works through its own share of
-// every job).  Jobs come by falling length: the short ones behind fill the gaps that the long ones leave, so the
-// launch ends as if it consisted of items of the last job's length T only, in ceil(units / cus) rounds of them.  The
+// every job).  Jobs by falling length: the short ones behind fill the gaps that the long ones leave, so the
+// launch ends as if it consisted of items of the last job's length T only, in ceil(units / cus) rounds of them.  Or
+// (`by_count`) the items are counted as they are, whatever their lengths: launch_time says which of the two is right.  The
 // items of the last, partly filled round are cut into w parts each, which are handed to CUs as they come free: they take
 // ceil(rem * w / cus) rounds of (T / w + overhead) instead of one of T, plus the fold kernel.  A launch of less than one
 // round is split as a whole.
@@ -1357,11 +1361,12 @@ static void job_sizes(const AttnArgs& a, int n_jobs, JobSize* size) {
 // Launches of less than a round that used to run unsplit (us, before -> now): 1 head x 8000 queries x 8000 keys, D = 128
 // 140 -> 49; 3 heads x 2048 x 4096 77 -> 36; 10 heads x 1154 queries, two states over 1 and 2 chunks of 1154 keys 53 -> 45;
 // 4 heads x 5777 queries x 4 chunks of 5777 keys (368 work items, 23 per head) 270 -> 250.
-static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus, int64_t slots_cap) {
+static TailPlan plan_tail(const AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus, int64_t slots_cap, bool by_count) {
+  TailPlan plan;
   constexpr double kPartOverheadOneRound = 6.0, kPartOverheadRounds = 10.0, kHalfItem = 0.6;
   const double fold_overhead = D == 128 ? 6.0 : 4.0;
   const int last = size[n_jobs - 1].tiles, last_rows = size[n_jobs - 1].rows;
-  if (last < 1 || (int64_t)n_jobs * a.per_xcd >= INT32_MAX) return;
+  if (last < 1 || (int64_t)n_jobs * a.per_xcd >= INT32_MAX) return plan;
   double units = 0;
   int same = 0, longest = 0;   // jobs at the end that are like the last one
   for (int j = 0; j < n_jobs; ++j) {
@@ -1377,11 +1382,11 @@ static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int c
     T = longest;
   } else {
     // (with boundaries that only the device knows the last round may be full for all the host can tell)
-    rem = a.cu_q ? 0 : (int)std::ceil(units - 1e-9) % cus;
+    rem = a.cu_q ? 0 : by_count ? n_jobs * a.per_xcd % cus : (int)std::ceil(units - 1e-9) % cus;
     T = last;
-    if (rem > same * a.per_xcd) return;
+    if (rem > (by_count ? 1 : same) * a.per_xcd) return plan;
   }
-  if (rem <= 0) return;
+  if (rem <= 0) return plan;
   double best = 0.1 * T;   // least gain worth the extra kernel
   for (int w = 2; T >= 16 && w <= 16; ++w) {
     if ((int64_t)rem * kXcds * w > slots_cap || T / w < 6) break;
@@ -1390,17 +1395,93 @@ static void plan_tail(AttnArgs& a, int D, int n_jobs, const JobSize* size, int c
     const double gain = T - rounds * (part + overhead) - fold_overhead;
     if (gain > best) {
       best = gain;
-      a.tail_items = rem;
-      a.part_ways = w;
+      plan.items = rem;
+      plan.ways = w;
     }
   }
   const double gain_rows = (1.0 - kHalfItem) * T - 2.0;
-  if (!a.q_prescaled && 2 * rem <= cus && last_rows > kBQ / 2 && T >= kMinSplitTiles && gain_rows > (a.tail_items > 0 ? best : 0.0)) {
-    a.tail_items = rem;
-    a.part_ways = 2;
-    a.row_split = 1;
+  if (!a.q_prescaled && 2 * rem <= cus && last_rows > kBQ / 2 && T >= kMinSplitTiles && gain_rows > (plan.items > 0 ? best : 0.0)) {
+    plan.items = rem;
+    plan.ways = 2;
+    plan.rows = true;
   }
-  if (a.tail_items > 0) a.tail_start = n_jobs * a.per_xcd - a.tail_items;
+  return plan;
+}
+
+// What a launch with jobs of unequal length takes, in key tiles.  An XCD hands its workgroups to its four shader engines in
+// turn, whether an engine has a CU free or not, so each engine works through every fourth workgroup on eight CUs: 42 items
+// of 210 and 105 tiles in this order, which would fill 32 CUs evenly, leave one engine with a third item for a CU.
+// (Differences between two orders and splits of a launch correlate with the measured ones at 0.87 in this model, at 0.63
+// in one that gives every item to the CU that is free first; 55 launches at D = 128.)  The clock rises where CUs are idle,
+// so that about 0.6 of a difference in the end times is seen: the rest of the price is the work done.
+static double launch_time(const AttnArgs& a, int n_jobs, const JobSize* size, int cus, const TailPlan& plan) {
+  constexpr int kEngines = 4, kMaxCus = 16;
+  constexpr double kItem = 4.0, kPart = 10.0, kHalfItem = 0.6, kFold = 6.0, kEndShare = 0.6;
+  const int per_engine = std::min(kMaxCus, cus / kEngines);
+  double busy[kEngines][kMaxCus] = {}, work = 0, end = 0;
+  int wg = 0;
+  auto run = [&](double tiles) {
+    double* cu = std::min_element(busy[wg % kEngines], busy[wg % kEngines] + per_engine);
+    *cu += tiles;
+    work += tiles;
+    end = std::max(end, *cu);
+    ++wg;
+  };
+  const int n = n_jobs * a.per_xcd, whole = n - plan.items;
+  auto exists = [&](int flat) { return flat % a.per_xcd % a.nqt * kBQ < size[flat / a.per_xcd].rows; };
+  for (int flat = 0; flat < n; ++flat) {
+    if (flat < whole && exists(flat)) run(size[flat / a.per_xcd].tiles + kItem);
+    else ++wg;
+  }
+  for (int flat = whole; flat < n; ++flat) {
+    const double tiles = size[flat / a.per_xcd].tiles;
+    for (int p = 0; p < plan.ways; ++p) {
+      if (exists(flat)) run(plan.rows ? kHalfItem * tiles + kItem : tiles / plan.ways + kPart);
+      else ++wg;
+    }
+  }
+  const double fold = plan.items > 0 && !plan.rows ? kFold : 0.0;
+  return kEndShare * (end + fold) + (1.0 - kEndShare) * work / (kEngines * per_engine);
+}
+
+// Order of the jobs and split of the last round (slots_cap < 0: no split).  Jobs of one length: there is one order, and the
+// items are counted.  Of several, in a launch of more than one round: the order of the caller with the remainder by count, or
+// the longest first with the remainder in units of the last job or by count, whatever takes least by launch_time.  Of two that
+// take the same, D = 128 keeps the caller's order (the shorter job in front, whose long items then run alone at a higher clock:
+// 24 heads x 3721 queries, 1 + 2 chunks 468 -> 463 us), D = 64 the longest first (30 heads x 2001 103 -> 99).
+// Over 318 launches of 4 ... 48 heads x 1200 ... 14 882 queries, 2 or 3 jobs of 1 ... 7 chunks: 2.3 % less time on average than
+// always the longest first in units (40 heads x 1596, D = 64, 1 + 7 chunks 309 -> 238 us; 48 x 6851, D = 128, 1 + 2 2896 -> 2826;
+// most lost 3.6 %, 24 x 3641, D = 128, 1 + 2 413 -> 426) and 3.0 % less than always the caller's order by count (D = 128: never
+// more; D = 64: up to 12 % more in launches of two or three rounds, where the two workgroups of a CU share it, which is not
+// modelled: 12 heads x 6902, 1 + 3 593 -> 656).
+static TailPlan plan_launch(AttnArgs& a, int D, int n_jobs, JobSize* size, int cus, int64_t slots_cap) {
+  constexpr int kMaxItems = 2048;   // of an XCD, 64 rounds: the end of a longer launch is nothing, and pricing it takes time
+  int order[DT_MAX_JOBS * DT_MAX_SEGMENTS];
+  JobSize sorted[DT_MAX_JOBS * DT_MAX_SEGMENTS];
+  const bool changes = a.dev_ids == nullptr && longest_first(size, n_jobs, order);
+  for (int j = 0; j < n_jobs; ++j) sorted[j] = size[changes ? order[j] : j];
+  const bool split = slots_cap >= 0;
+  bool uneven = false;
+  for (int j = 1; j < n_jobs; ++j) uneven = uneven || size[j].tiles != size[0].tiles;
+  TailPlan best = split ? plan_tail(a, D, n_jobs, sorted, cus, slots_cap, false) : TailPlan();
+  const int64_t items = (int64_t)n_jobs * a.per_xcd;
+  bool given = false;
+  if (a.dev_ids == nullptr && uneven && cus > 0 && items > cus && items <= kMaxItems) {
+    double least = launch_time(a, n_jobs, sorted, cus, best);
+    auto consider = [&](const JobSize* s, bool as_given) {
+      const TailPlan plan = split ? plan_tail(a, D, n_jobs, s, cus, slots_cap, true) : TailPlan();
+      const double time = launch_time(a, n_jobs, s, cus, plan);
+      if (as_given && D == 128 ? time < 1.001 * least : time < least) {
+        least = time;
+        best = plan;
+        given = as_given;
+      }
+    };
+    if (split) consider(sorted, false);
+    if (changes) consider(size, true);
+  }
+  if (changes && !given) reorder_jobs(a, n_jobs, order);
+  return best;
 }
 
 // Held while a split launch and its fold kernel go into the queue: two threads may launch on one stream, with the workspace
@@ -1433,10 +1514,14 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   if (n_jobs <= kMaxLaunchJobs) {
     JobSize size[kMaxLaunchJobs];
     job_sizes(a, n_jobs, size);
-    if (a.dev_ids == nullptr) order_jobs(a, n_jobs, size);
-    const int cus = workspace ? cu_count() : 0;
-    if (cus >= 64 && cus % kXcds == 0)
-      plan_tail(a, D, n_jobs, size, cus / kXcds, std::min(workspace_bytes, kWorkspaceBytes) / slot_bytes);
+    const int cus = cu_count();
+    const bool known = cus >= 64 && cus % kXcds == 0;
+    const TailPlan plan = plan_launch(a, D, n_jobs, size, known ? cus / kXcds : 0,
+                                      known && workspace ? std::min(workspace_bytes, kWorkspaceBytes) / slot_bytes : -1);
+    a.tail_items = plan.items;
+    a.part_ways = plan.ways;
+    a.row_split = plan.rows ? 1 : 0;
+    if (plan.items > 0) a.tail_start = n_jobs * a.per_xcd - plan.items;
   }
   const unsigned planes_x = (unsigned)a.per_xcd * kXcds;
   if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);

@@ -210,9 +210,12 @@ def test_tail_balancing_matches_plain_launch_and_oracle(hip, D, H, nq, lens, job
     (128, 5, 513, [1030, 1500, 64], [[2], [0, 1, 2]], torch.bfloat16), # jobs of 1 and 41 tiles: reordered, the short one's parts mostly empty
     (64, 7, 1030, [2100, 2090], [[0], [1]], torch.bfloat16),           # 35 items a job: not a multiple of 8
     (128, 37, 1900, [3000, 3000], [[0, 1], [1]], torch.bfloat16),      # 2 x 296 items, the shorter job's tail of a launch of several rounds
+    (64, 40, 1596, [1070, 3000, 2400], [[0], [1, 2]], torch.bfloat16), # the caller's order kept, the longer job's tail cut along the keys
+    (128, 33, 1100, [1270, 2500], [[0], [1]], torch.float16),          # reordered, the items counted whatever their length, cut along the rows
+    (64, 30, 1501, [2500, 1270], [[0], [1]], torch.bfloat16),          # longest first as given, likewise
 ])
 def test_split_launches_match_plain_launch_and_oracle(hip, D, H, Sq, lens, jobs, dtype):
-    """Launches of less than one round are split as a whole, jobs run longest first: every row of every state
+    """Launches of less than one round are split as a whole, jobs run in the order that takes least: every row of every state
     against the launch without a workspace.  P is rounded relative to another running maximum in a part, so a row differs
     by up to one rounding of P (2^-8 in bf16, weights summing to 1) and one of the output: 2^-7 of the largest value."""
     g = torch.Generator().manual_seed(D + Sq)
