@@ -457,8 +457,11 @@ void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, con
   REQUIRE(ids.scalar_type() == at::kInt && count.scalar_type() == at::kInt && ids.is_cuda() && count.is_cuda(),
           "schedule tensors must be int32 on the GPU");
   const int64_t per_row = ids.dim() > 1 ? ids.size(-1) : ids.numel(), per_count = count.dim() > 1 ? count.size(-1) : count.numel();
-  REQUIRE(ids.is_contiguous() && count.is_contiguous() && per_row >= max_jobs && per_count >= 1 && row >= 0 &&
-              (row + 1) * per_row <= ids.numel() && (row + 1) * per_count <= count.numel(),
+  // (row 0 is the tensors themselves: a list of any shape, a count that may be an element of a strided view)
+  REQUIRE(ids.is_contiguous() && count.numel() >= 1 &&
+              (row == 0 ? ids.numel() >= max_jobs
+                        : count.is_contiguous() && per_row >= max_jobs && row > 0 && (row + 1) * per_row <= ids.numel() &&
+                              (row + 1) * per_count <= count.numel()),
           "compute id list shorter than max_jobs");
   REQUIRE(slot_out.scalar_type() == q.scalar_type() && slot_out.is_contiguous() && slot_out.dim() == 5 &&
               slot_out.sizes().slice(1) == at::IntArrayRef({d.B, d.S, d.H, d.D}) && slot_out.size(0) >= table.n,

@@ -130,3 +130,19 @@ def test_threads_that_launch_on_one_stream_share_its_workspace(hip):
     for i in range(2):
         assert len(got[i]) == 150
         assert all(torch.equal(o, want[i][0]) and torch.equal(l, want[i][1]) for o, l in got[i])
+
+
+def test_a_schedule_of_its_own_may_be_a_strided_count_and_a_list_of_any_shape(hip):
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(1, 96, 2, 64, generator=g).bfloat16().cuda() for _ in range(3))
+    table = hip.ChunkTable([k, v, q], [v, k, q])
+    counts = torch.tensor([[2, 1], [0, 0]], dtype=torch.int32, device="cuda")
+    ids = torch.tensor([2, 0, -1], dtype=torch.int32, device="cuda")
+    states = []
+    for i, c in ((ids, counts[0, :1]), (ids, counts[:, 0]), (ids[:, None], counts[0, :1]), (ids[:2, None], counts)):
+        out, lse = torch.zeros(3, 1, 96, 2, 64, dtype=q.dtype, device="cuda"), torch.zeros(3, 1, 2, 96, device="cuda")
+        hip.attn_sched_fwd(q, table, i, c, 2, out, lse, -1, None, None)
+        states.append((out, lse))
+    for out, lse in states[1:]:
+        assert torch.equal(out, states[0][0]) and torch.equal(lse, states[0][1])
+    assert states[0][0][0].any() and states[0][0][2].any() and not states[0][0][1].any()
