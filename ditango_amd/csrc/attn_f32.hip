@@ -377,6 +377,10 @@ extern "C" int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32
   // the keys four ways fills it (12 heads x 2048 queries x 2 chunks, 1536 tiles: 270 instead of 346 us at d = 64, 479
   // instead of 601 at d = 128; 256 tiles: 40 instead of 110 us); from there on four query tiles that read the same keys
   // are the better neighbours in a workgroup (3072 tiles: 500 each at d = 64, 908 instead of 954 us at d = 128).
+  // The line holds for chunks of 256 keys and more.  A wavefront with a tile or less pays for the exchange of the parts without a
+  // shorter loop: 24 heads x 2048 queries x 512 keys 79 split, 96 us unsplit at d = 64, 153 and 165 at d = 128, but x 64 keys 27 and 21,
+  // 60 and 39.  Short chunks are launches of tens of us either way and up to 512 query tiles split well too (4 heads x 512 x 64 keys
+  // 6.8 and 10.7 us), so the number of keys is left out of the rule.
   const bool split = units * n_jobs < 3 * 1024;
   if (D == 128)
     return split ? launch_f32<128, 4>(a, n_jobs, (hipStream_t)stream) : launch_f32<128, 1>(a, n_jobs, (hipStream_t)stream);

@@ -385,12 +385,15 @@ __device__ __forceinline__ KeyRef key_ref(const JobView& v, int seg) {
   return r;
 }
 
-// Work items of fewer key tiles than this are never cut along the keys or the rows: there is next to nothing to gain (an
-// item costs about four tiles on top of its own), and a segment of a few padding tokens keeps the sums of one pass.
+// Work items of fewer key tiles than this are never cut along the keys or the rows: an item costs about four tiles on top of its
+// own, and a segment of a few padding tokens keeps the sums of one pass.  us per launch uncut -> cut, 4 heads x 512 queries at
+// D = 64 and 24 x 1000 at D = 128: 8 tiles 13.2 -> 10.7, 17.3 -> 15.3; 6 tiles 11.4 -> 9.7, 15.3 -> 13.8; up to 5 tiles the planner
+// does not cut.  Tiles of at most 128 rows (always cut from here on), 30 heads x 128, D = 128: 8 tiles 15.6 -> 14.1, 4 tiles 11.4 ->
+// 11.4, 2 tiles 9.3 -> 10.0.
 constexpr int kMinSplitTiles = 8;
 
 // Wavefronts per SIMD the register budget is set for.  D = 128: two (one workgroup per CU: its LDS
-// tiles fill the CU).  D = 64: four, i.e. TWO workgroups per CU (64 KB of LDS and at most 128
+// tiles fill the CU).  D = 64: four, i.e. TWO workgroups per CU (80 KB of LDS and at most 128
 // registers each): the second workgroup's wavefronts issue into the barrier waits, the start-up and
 // the epilogue of the first, which at 35 key tiles per work item are a tenth of its time (+10 %).
 constexpr int kWavesPerSimdD64 = 4;
@@ -433,7 +436,8 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   typedef typename E::x2 ex2;
   constexpr int kKeyBlocks = kSplitKeys ? 1 : 2;   // 32-key blocks of a tile that a wavefront works on
   // A reference of its own for every place that reads arguments, unrelated to the others as far as the compiler can see:
-  // it otherwise reads whole lines at the top and holds what later places need in 120 spilled scalar registers.
+  // it otherwise reads whole lines at the top and holds what later places need in spilled scalar registers (119 at D = 128 and
+  // 116 at D = 64 instead of 109 and 103).
   auto args = []() __attribute__((always_inline)) -> KernArgs& { return kernel_args(); };
   KernArgs& a = args();
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];

@@ -25,7 +25,7 @@ constexpr int kThreads = 256;
 // are 2.2 rounds of the chip).  HBM-bound; us per launch with 8 / 4 / 2 heads: 14882 x 24 heads of 128 41.7 / 39.5 / 41.3,
 // 12444 x 48 of 64 35.8 / 31.8 / 32.3, 9000 x 20 of 128 26.9 / 23.6 / 22.5, 119056 x 24 of 128 (6.0 TB/s) 262 / 260 / 278.
 constexpr int kHeads = 4;
-// 80 registers; 7 or 8 wavefronts would spill 24 or more of them.
+// 77 or 78 registers; 7 or 8 wavefronts would spill 24 or more of them.
 constexpr int kWavesPerSimd = 6;
 
 struct PrepArgs {
@@ -118,6 +118,8 @@ __device__ __forceinline__ float group_sum(float v) {
 // With the LDS butterfly and a root per row the kernel took as long for its arithmetic as for its bytes; us per launch before, with
 // the sums by DPP, and with the shared roots too: 14882 tokens x 24 heads of 128 35.2 / 34.5 / 34.1, 119056 x 24 256 / 245 / 240
 // (6.6 TB/s), 9000 x 20 20.3 / 19.6 / 19.3, 12444 x 48 of 64 with LayerNorm 30.0 / 28.9 / 28.7; 14882 x 24 without a norm 32.8.
+// Short launches, replayed from a graph, before and with both: 512 x 4 of 64 5.7 / 4.8, 2250 x 48 of 64 with LayerNorm 8.8 / 8.0, 8000 x
+// 3 of 128 5.7 / 5.5, 5000 x 10 9.1 / 8.1 (called one by one from Python the host is the limit there, 13 to 16 us).
 // (The sums come as values: from an array the compiler makes the choice one of addresses and the array a piece of LDS, which
 // costs every launch 8 us.)
 template <int D>
