@@ -62,6 +62,15 @@ _SIGNATURES = {
                                                     c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                                     c_i32, _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32),
                                                     _P(c_vp), _P(c_vp), c_f32, c_i32, c_vp]),
+    "dt_attn_merge_counters": (ctypes.c_int64, [c_i32, c_i32, c_i32]),
+    "dt_attn_jobs_merge_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
+                                              c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
+                                              c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_vp, c_f32, c_i32,
+                                              c_vp, c_i64, c_vp]),
+    "dt_attn_sched_merge_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
+                                               c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
+                                               c_vp, c_vp, c_i32, c_vp, c_i64, c_vp, c_i64, c_i32, c_vp, c_vp,
+                                               c_vp, c_f32, c_i32, c_vp, c_i64, c_vp]),
     "dt_attn_sched_seg_ws_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                                 c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                                 c_vp, c_vp, c_i32, c_vp, c_i64, c_vp, c_i64, c_i32, c_vp, c_vp,
@@ -271,9 +280,37 @@ def attn_workspace(device) -> torch.Tensor:
     return ws
 
 
+_counters: "dict" = {}     # as _workspaces
+KEPT_COUNTERS = 1 << 18    # words a kept set holds: launches of up to 32 512 query tiles
+
+
+def attn_counters(device, q: torch.Tensor) -> Optional[torch.Tensor]:
+    """The arrival counters of merging launches on ``q [B,Sq,H,D]`` made on the current stream of ``device``: int32, zero, and
+    left at zero by every launch.  One set per stream, kept and shared like the workspace; launches under capture get a set
+    of the graph's own pool, cleared by the graph.  ``None`` where a launch needs more than a kept set holds: it does not
+    merge then."""
+    B, Sq, H, _ = q.shape
+    need = int(load_library().dt_attn_merge_counters(B, Sq, H))
+    if need > KEPT_COUNTERS:
+        return None
+    dev = device if isinstance(device, torch.device) else torch.device(device)
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(need, dtype=torch.int32, device=dev).zero_()
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    key = (dev.type, index, _raw_stream(index))
+    c = _counters.pop(key, None)
+    if c is None:
+        while len(_counters) >= MAX_WORKSPACES:
+            _counters.pop(next(iter(_counters)))
+        c = torch.empty(KEPT_COUNTERS, dtype=torch.int32, device=dev).zero_()
+    _counters[key] = c
+    return c
+
+
 def release_workspaces() -> None:
     """Drop every attention workspace (they are re-created on demand)."""
     _workspaces.clear()
+    _counters.clear()
 
 
 class ChunkTable:
@@ -354,6 +391,27 @@ def attn_states(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Seq
     ``dev_segments``; rows outside every segment are left as they are.  ``convert`` as in ``ChunkTable``."""
     return _host().attn_states(q, k_chunks, v_chunks, jobs, max_chunks, cu_q, cu_kv, workspace, _attn_flags(q, q_prescaled),
                                None if dev_segments is None else dev_segments.native, convert, _stream())
+
+
+def attn_states_merge(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor],
+                      jobs: Sequence[Sequence[int]], max_chunks: int, outs: Sequence[torch.Tensor], lses: Sequence[torch.Tensor],
+                      which: Sequence[int], dst_dtype: torch.dtype, workspace: Optional[torch.Tensor] = None,
+                      q_prescaled: bool = False, cu_q: Optional[Sequence[int]] = None,
+                      cu_kv: Optional[Sequence[Sequence[int]]] = None, dev_segments: Optional[DeviceSegments] = None,
+                      convert=None):
+    """``attn_states``, and the merge of the given states and then ``states[which[..]]`` (``merge_states`` with a
+    ``[B,S,H,1]`` lse), in the same launch where it can.  Returns (states, out, lse)."""
+    return _host().attn_states_merge(q, k_chunks, v_chunks, jobs, max_chunks, cu_q, cu_kv, workspace, _attn_flags(q, q_prescaled),
+                                     None if dev_segments is None else dev_segments.native, convert, outs, lses, which, dst_dtype,
+                                     attn_counters(q.device, q), _stream())
+
+
+def attn_sched_merge(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor, max_jobs: int,
+                     slot_out: torch.Tensor, slot_lse: torch.Tensor, diag: int, diag_out: torch.Tensor, diag_lse: torch.Tensor,
+                     dst_dtype: torch.dtype, workspace: Optional[torch.Tensor] = None, q_prescaled: bool = False, row: int = 0):
+    """``attn_sched_fwd`` on whole queries and ``merge_arena``, in the same launch where it can.  Returns (out, lse)."""
+    return _host().attn_sched_merge(q, table.native, dev_compute_ids, dev_count, row, max_jobs, slot_out, slot_lse, diag, diag_out,
+                                    diag_lse, dst_dtype, workspace, attn_counters(q.device, q), _attn_flags(q, q_prescaled), _stream())
 
 
 def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor,

@@ -13,8 +13,8 @@ issues
 1. ONE attention launch that produces every state of the call (``dt_attn_jobs_fwd``:
    the local chunk, and the fresh state of the target block as a single multi-chunk
    job written straight into its cache tensors), and
-2. ONE fused N-way merge (``dt_merge_states``) over the cached states, the local
-   state and the fresh states.
+2. ONE N-way merge over the cached states, the local state and the fresh states: in the
+   same launch where it can (``dt_attn_jobs_merge_fwd``), else ``dt_merge_states``.
 
 Which chunk the ring would have delivered at each hop follows from tracking, as
 integers, the chunk id every ring position holds (``plan_call``); the chunk order, the reuse set, the cache writes and the pointer
@@ -387,15 +387,12 @@ class proAttention:
             else:
                 cu_q, cu_kv_of = segments
                 cu_kv = [cu_kv_of(c) for c in needed]
-        states = _hip.attn_states(query, [k for k, _ in kv], [v for _, v in kv], jobs, self._MAX_JOB_CHUNKS,
-                                  _hip.attn_workspace(query.device), self.q_prescaled, cu_q, cu_kv, dev_seg, _kernel_input)
+        states, out, lse = _hip.attn_states_merge(query, [k for k, _ in kv], [v for _, v in kv], jobs, self._MAX_JOB_CHUNKS,
+                                                  merge_outs, merge_lses, which, self.out_dtype, _hip.attn_workspace(query.device),
+                                                  self.q_prescaled, cu_q, cu_kv, dev_seg, _kernel_input)
         for job, i in zip(plan.jobs, which):
-            o, l = states[i]
             if job.store_slot is not None:
-                self.cache.store_block(job.store_slot, o, l)  # :207-211
-            merge_outs.append(o)
-            merge_lses.append(l)
-        out, lse = _hip.merge_states(merge_outs, merge_lses, dst_dtype=self.out_dtype, dst_lse_bsh=True)
+                self.cache.store_block(job.store_slot, *states[i])  # :207-211
         self.last_lse = lse
         return out
 
@@ -430,7 +427,13 @@ class proAttention:
                 seg_kv = [[(cu_kv_of(c)[i], cu_kv_of(c)[i + 1] - cu_kv_of(c)[i]) for i in range(len(cu_q) - 1)]
                           for c in range(C)]
         ws = _hip.attn_workspace(query.device)
-        if not rm.sched_windows:
+        out = None
+        if not rm.sched_windows and self._segments is None:
+            out, lse = _hip.attn_sched_merge(query, _hip.ChunkTable(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
+                                             rm.compute_counts[t][l], cache.arena_out, cache.arena_lse, diag, cache.diag_out,
+                                             cache.diag_lse, self.out_dtype, ws, self.q_prescaled,
+                                             (t % rm.num_timesteps) * rm.num_layers + l % rm.num_layers)
+        elif not rm.sched_windows:
             _hip.attn_sched_fwd(query, _hip.ChunkTable(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
                                 rm.compute_counts[t][l], cache.arena_out, cache.arena_lse, diag, cache.diag_out,
                                 cache.diag_lse, seg_q=seg_q, seg_kv=seg_kv, workspace=ws, q_prescaled=self.q_prescaled,
@@ -462,7 +465,8 @@ class proAttention:
         for c in range(C):
             if row[c] == 0 and c != diag:
                 valid[c] = True
-        out, lse = _hip.merge_arena(cache.arena_out, cache.arena_lse, diag, cache.diag_out, cache.diag_lse, self.out_dtype)
+        if out is None:
+            out, lse = _hip.merge_arena(cache.arena_out, cache.arena_lse, diag, cache.diag_out, cache.diag_lse, self.out_dtype)
         self.last_lse = lse
         rm.record_out_redundancy(timestep=t, layer_id=l, curr_out=out)
         return out

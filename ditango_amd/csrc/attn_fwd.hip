@@ -418,7 +418,176 @@ __device__ __forceinline__ void prefetch_args(uint64_t args) {
       : "memory");
 }
 
-// The work of one workgroup: query rows from row0 on of one job, batch and head.
+// ---- states that meet inside a launch ----------------------------------------------------------
+// What another workgroup of the launch reads (states and partial states of a merging launch) is stored and loaded with the
+// device-scope bit: past the L1 and the XCD's L2, so that behind the writer's s_waitcnt vmcnt(0) it is where every XCD finds
+// it.  The fences of an acquire and release at device scope do the same to whole caches: the invalidation alone, executed by
+// one wavefront per merge, took the keys and values of the XCD's other workgroups out of its L2 and cost 4 us per work
+// item (two samples of 24 heads x 1861 queries x 3 of 8 chunks 242 -> 261 us); counting and waiting cost nothing that shows.
+constexpr int kNt = 2, kDevice = 16, kDeviceNt = kDevice | kNt;   // cache-policy bits of a raw buffer access: nt, sc1
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc buffer_of(const void* base, uint32_t valid_bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, valid_bytes, kRsrcFlags);
+}
+__device__ __forceinline__ void store_device(float* p, float x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_device(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// This wavefront's contribution (device-scope stores) is complete: counts it.  True for the last of `expected`, whose
+// device-scope loads then see the contributions of the others, and for which the counter is back at zero.
+__device__ __forceinline__ bool arrive_last(uint32_t* counter, int expected) {
+  wait_tile_loads<0>();   // (stores as well)
+  if (expected > 1) {
+    uint32_t before = 0;
+    if ((threadIdx.x & 63) == 0) before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((int)__builtin_amdgcn_readfirstlane(before) + 1 != expected) return false;
+    if ((threadIdx.x & 63) == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  asm volatile("" ::: "memory");   // no load moves up in front of this
+  return true;
+}
+
+// Merges the states there are of the 32 query rows from row0 on (one batch and head): out = sum_i w_i out_i / sum_i w_i with
+// w_i = exp(lse_i - max), all in fp32.  One wavefront, which needs nobody else: `stage` is LDS of its own, 2 KB.
+//
+// HBM-bound: the workgroups of a launch run in step, so the last job's all merge at the end of a round, at 5.3 TB/s.  A
+// wavefront has two steps (8 states x 4 rows of a load instruction, D = 64: 4 x 8) in flight all the time, also across
+// the batches of states; three make no difference.  Against a merge kernel behind the launch: 24 heads x 119 056 queries, 3 of 32
+// chunks computed 17.79 -> 16.47 ms; 48 heads x 2222, D = 64, 5 of 8 340 -> 336 us; 4 heads x 512, D = 64, 2 of 4 19.4 -> 16.6;
+// two samples of 24 heads x 1861, 3 of 8 284 -> 284.  Tried without success: the jobs side by side, each some items
+// behind the one before it, so that a part of the workgroups merges while the others compute (they fall out of step and no
+// longer share keys and values in the L2: 24 heads x 14 882, 4 of 8 8.53 -> 8.75 ms); adjacent heads on the 8 XCDs (16.1 -> 16.6 ms).
+template <int D, bool kHalf>
+__device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row0) {
+  typedef Elem<kHalf> E;
+  constexpr int kBatch = D == 128 ? 8 : 4;   // states of a step (D = 64: half the registers)
+  constexpr int kRowLanes = D / 8;           // a lane holds 8 columns of a row
+  constexpr int kRowsPer = 64 / kRowLanes;   // rows of a load instruction
+  constexpr int kSteps = 32 / kRowsPer;      // steps of a batch of states
+  static_assert(kMergeBatch % kBatch == 0, "the lists are filled up to whole batches");
+  KernArgs& a = kernel_args();
+  typedef const AttnState __attribute__((address_space(4))) KernState;
+  KernState* states = a.dev_ids ? a.arena : a.state;
+  const int lane = threadIdx.x & 63, col = lane & 31;
+  const int n = a.merge_n, H = a.H, Sq = a.Sq;
+  const int rows = min(32, Sq - row0);
+  const int64_t lse_at = ((int64_t)b * H + h) * Sq + row0;
+  const int64_t out_at = (((int64_t)b * Sq + row0) * H + h) * D;
+  const uint32_t row_bytes = (uint32_t)H * D * 2u;
+  const uint32_t valid = (uint32_t)(rows - 1) * row_bytes + D * 2u;
+  const int my_row = min(col, rows - 1);
+  const uint32_t lane_off = (uint32_t)(lane / kRowLanes) * row_bytes + 16u * (uint32_t)(lane % kRowLanes);
+  // The batch under the load cursor.  States that are not there (behind the last one, and everything once i0 < 0) are empty
+  // descriptors: their loads touch no memory and return zeros.
+  int i0 = (n - 1) / kBatch * kBatch;
+  u32x4 r[kBatch];
+  auto open = [&]() __attribute__((always_inline)) {
+    KernState* st = states + max(i0, 0);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) r[j] = make_rsrc(st[j].out + out_at, i0 >= 0 && i0 + j < n ? valid : 0u);
+  };
+  u32x4 x[2][kBatch];
+  auto load = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j)
+      x[s & 1][j] = __builtin_amdgcn_raw_buffer_load_b128(
+          __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)r[j].y << 32 | r[j].x), 0, r[j].z, kRsrcFlags),
+          lane_off, (uint32_t)(s * kRowsPer) * row_bytes, kDeviceNt);
+  };
+  float l[kBatch];
+  auto load_lse = [&](int i0) __attribute__((always_inline)) {   // (the lists go on behind the last state with copies of it)
+    KernState* st = states + max(i0, 0);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) l[j] = load_device(st[j].lse + lse_at + my_row);
+  };
+  open();
+  load(0);
+  load(1);
+  float m = -INFINITY, den = 0.f;
+  for (int i = 0; i < n; i += kBatch) {   // (the last batch, which comes first below, stays in l)
+    load_lse(i);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) m = fmaxf(m, l[j]);
+  }
+  float acc[kSteps][8];
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[s][e] = 0.f;
+  float* weights = reinterpret_cast<float*>(stage);   // [32 rows][kBatch]
+  while (i0 >= 0) {
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      l[j] = i0 + j < n && m > -INFINITY ? __expf(l[j] - m) : 0.f;
+      den += l[j];
+    }
+#pragma unroll
+    for (int j = 0; j < kBatch; j += 4) *reinterpret_cast<f32x4*>(weights + col * kBatch + j) = f32x4{l[j], l[j + 1], l[j + 2], l[j + 3]};
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const float* ws = weights + (s * kRowsPer + lane / kRowLanes) * kBatch;
+      f32x4 wv[kBatch / 4];
+#pragma unroll
+      for (int j = 0; j < kBatch / 4; ++j) wv[j] = *reinterpret_cast<const f32x4*>(ws + 4 * j);
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x2 v = E::widen(x[s & 1][j][e]);
+          acc[s][2 * e] = __builtin_fmaf(wv[j / 4][j % 4], v.x, acc[s][2 * e]);
+          acc[s][2 * e + 1] = __builtin_fmaf(wv[j / 4][j % 4], v.y, acc[s][2 * e + 1]);
+        }
+      if (s + 2 == kSteps) {   // the next batch
+        i0 -= kBatch;
+        open();
+        load_lse(i0);
+      }
+      load((s + 2) % kSteps);
+      __builtin_amdgcn_sched_barrier(0);   // the loads stay behind the step that frees their registers
+    }
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  if (lane < rows) a.merge_lse[((int64_t)b * Sq + row0 + lane) * H + h] = den > 0.f ? m + __logf(den) : -INFINITY;
+  const bool wide = a.merge_dtype == DT_FP32;
+  const Rsrc dst = buffer_of(static_cast<uint8_t*>(a.merge_out) + out_at * (wide ? 4 : 2), wide ? 2 * valid : valid);
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s) {
+    const float f = __shfl(inv, s * kRowsPer + lane / kRowLanes);
+    // (rows whose states are all empty: 0, whatever the states hold)
+    const bool none = !(__shfl(m, s * kRowsPer + lane / kRowLanes) > -INFINITY);
+    float o[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = none ? 0.f : acc[s][e] * f;
+    if (wide) {
+      // A lane's 32 bytes as two stores would write every other 16 bytes of a line: through the LDS, so that a store covers
+      // whole rows (24 heads x 14 882 queries against one key tile, 8 states merged: 250 -> 232 us).
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        *reinterpret_cast<f32x4*>(stage + lane * 32 + 16 * q) = f32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(stage + q * 1024 + lane * 16);
+        const uint32_t row = (uint32_t)(s * kRowsPer + q * (kRowsPer / 2)) + (uint32_t)lane / (2 * kRowLanes);
+        __builtin_amdgcn_raw_buffer_store_b128(v, dst, 2 * row * row_bytes + 16u * ((uint32_t)lane % (2 * kRowLanes)), 0, kNt);
+      }
+    } else {
+      u32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f32x2 pair;
+        pair.x = o[2 * e];
+        pair.y = o[2 * e + 1];
+        v[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, typename E::x2));
+      }
+      __builtin_amdgcn_raw_buffer_store_b128(v, dst, lane_off + (uint32_t)(s * kRowsPer) * row_bytes, 0, kNt);
+    }
+  }
+}
+
+// The work of one workgroup: query rows from row0 on of one job, batch and head.  `slice` is
+// set to the 32-row slice of the tile whose rows this wavefront has stored, -1 for none.
 //
 // kSplitKeys: no more than half of the 256 rows exist, or another workgroup has the other half.  Wavefronts w and w + 4 --
 // one of either group -- then share 32 queries: the leading group's takes the first 32 keys of every tile, the trailing
@@ -427,8 +596,9 @@ __device__ __forceinline__ void prefetch_args(uint64_t args) {
 // time of a full one (one round of items of 32 key tiles: D = 128 79 -> 49 us, D = 64 87 -> 52), not half: the load
 // instructions and barriers stay.  That much is saved on the last query tile of a head where up to 128 of its rows exist
 // (24 heads x 1400 queries x 4 chunks, D = 128: 121 -> 118 us), and by cutting the items of the last round in two (plan_tail).
-template <int D, bool kPre, bool kHalf, bool kSplitKeys>
-__device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int row0, bool is_part, int part, int unit, int xcd) {
+template <int D, bool kPre, bool kHalf, bool kMerge, bool kSplitKeys>
+__device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int row0, bool is_part, int part, int unit, int xcd, int& slice) {
+  slice = -1;
   using T = Tile<D>;
   using E = Elem<kHalf>;
   typedef typename E::x8 ex8;
@@ -976,16 +1146,23 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
 
   // ---- epilogue -------------------------------------------------------------------------
   const float l_tot = l_run + __shfl_xor(l_run, 32);
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  const float lse = l_tot > 0.f ? (m_ref * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : -INFINITY;
+  float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  float lse = l_tot > 0.f ? (m_ref * c + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : -INFINITY;
   const int qrow = q0 + col;
   KernArgs& e = args();
   if (is_part) {
     // A part's state goes to the workspace as it lies in the registers, in fp32: whole kilobytes per store, no rounding.
-    const int64_t slot = ((int64_t)unit * kXcds + xcd) * e.part_ways + part;
+    const int ways = e.part_ways;
+    const int64_t item = (int64_t)unit * kXcds + xcd, slot = item * ways + part;
+    float* dst_lse = e.ws_lse + slot * kBQ + wave * 32 + col;
+    const uint32_t slice_bytes = 32 * D * 4;
+    float* dst = e.ws_out + (slot * kWaves + wave) * (32 * D);
     // (a NaN among the scores leaves no sum: the fold has to see that, an lse of -inf would be an empty part)
-    if (hh == 0) e.ws_lse[slot * kBQ + wave * 32 + col] = l_tot == l_tot ? lse : l_tot;
-    float* dst = e.ws_out + (slot * kWaves + wave) * (32 * D) + lane * 4;
+    const float part_lse = l_tot == l_tot ? lse : l_tot;
+    if (hh == 0) {
+      if constexpr (kMerge) store_device(dst_lse, part_lse);
+      else *dst_lse = part_lse;
+    }
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
@@ -993,11 +1170,49 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         f32x4 val;
 #pragma unroll
         for (int e = 0; e < 4; ++e) val[e] = o_acc[db][4 * g + e] * inv;
-        *reinterpret_cast<f32x4*>(dst + (4 * db + g) * 256) = val;
+        if constexpr (kMerge)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, val), buffer_of(dst, slice_bytes),
+                                                 (4 * db + g) * 1024 + lane * 16, 0, kDevice);
+        else *reinterpret_cast<f32x4*>(dst + (4 * db + g) * 256 + lane * 4) = val;
       }
-    return;
+    if constexpr (!kMerge) {
+      return;
+    } else {
+      // The wavefront that completes the last part of these 32 rows folds them all; the rest is as if it had computed the
+      // whole item.
+      if (!arrive_last(e.arrive + item * kWaves + wave, ways)) return;
+      const int64_t slot0 = item * ways;
+      const float* lses = e.ws_lse + slot0 * kBQ + wave * 32 + col;
+      const float* parts = e.ws_out + (slot0 * kWaves + wave) * (32 * D);
+      float m = -INFINITY, den = 0.f;
+      for (int p = 0; p < ways; ++p) m = fmaxf(m, load_device(lses + p * kBQ));
+#pragma unroll
+      for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.f;
+      for (int p = 0; p < ways; ++p) {
+        const Rsrc src = buffer_of(parts + (int64_t)p * (kBQ * D), slice_bytes);
+        f32x4 x[D / 8];
+#pragma unroll
+        for (int g = 0; g < D / 8; ++g)
+          x[g] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, g * 1024 + lane * 16, 0, kDevice));
+        const float l = load_device(lses + p * kBQ);
+        const float w = l == -INFINITY ? 0.f : __expf(l - m);   // (NaN stays NaN, and with it the row's sum)
+        den += w;
+#pragma unroll
+        for (int g = 0; g < D / 8; ++g)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) o_acc[g / 4][4 * (g % 4) + k] = __builtin_fmaf(w, x[g][k], o_acc[g / 4][4 * (g % 4) + k]);
+      }
+      inv = den > 0.f ? 1.f / den : 0.f;
+      lse = den > 0.f ? m + __logf(den) : -INFINITY;
+    }
   }
-  if (hh == 0 && qrow < q_end) view.lse[((int64_t)b * e.H + h) * e.Sq + qrow] = lse;
+  if (hh == 0 && qrow < q_end) {
+    float* dst = view.lse + ((int64_t)b * e.H + h) * e.Sq + qrow;
+    if constexpr (kMerge) store_device(dst, lse);
+    else *dst = lse;
+  }
 
   // O^T (registers, [d][query]) -> LDS [query][d] in the element type -> coalesced 16-byte stores, half of the columns at
   // a time through this wavefront's own staging rows.  No barrier: the staging rows are nobody else's and no part of the
@@ -1030,15 +1245,35 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
       const int qg = q0 + row;
       const u32x4 val = *reinterpret_cast<const u32x4*>(stage + row * D + ((cc ^ T::swz_o(row)) << 4));
       if (qg < q_end) {
-        uint16_t* dst = view.out + (((int64_t)b * e.Sq + qg) * e.H + h) * D + half * (D / 2) + cc * 8;
-        __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
+        if constexpr (kMerge) {
+          const Rsrc dst = buffer_of(view.out + (((int64_t)b * e.Sq + q0) * e.H + h) * D, 32u * D * 2u * (uint32_t)e.H);
+          __builtin_amdgcn_raw_buffer_store_b128(val, dst, (uint32_t)(row * e.H) * (D * 2u) + half * D + cc * 16, 0, kDeviceNt);
+        } else {
+          uint16_t* dst = view.out + (((int64_t)b * e.Sq + qg) * e.H + h) * D + half * (D / 2) + cc * 8;
+          __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
+        }
       }
     }
   }
+  slice = ((row0 & (kBQ - 1)) >> 5) + (kSplitKeys ? wave & 3 : wave);
 }
 
-template <int D, bool kPre, bool kHalf>
+// The work item (batch, head, query tile) of this workgroup, from its place in the grid alone.
+__device__ __forceinline__ int item_of_block(KernArgs& a) {
+  uint32_t x = blockIdx.x, y = blockIdx.y;
+  asm volatile("" : "+s"(x), "+s"(y));   // (worked out where it is needed, not kept from the start of the kernel)
+  int idx = x >> 3;
+  if ((int)y >= a.job_planes) {
+    const int unit = (((int)y - a.job_planes) * (int)(gridDim.x >> 3) + idx) / a.part_ways;
+    idx = (a.tail_start + unit) % a.per_xcd;
+  }
+  return (int)(x & (kXcds - 1)) * a.per_xcd + idx;
+}
+
+// kMerge: a launch that merges (see AttnArgs::arrive).
+template <int D, bool kPre, bool kHalf, bool kMerge>
 __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn_fwd_kernel(const AttnArgs args_by_value) {
+  static_assert(!(kMerge && kPre), "prescaled launches do not merge");
   static_assert(!(kPre && kHalf), "the prescaled softmax keeps probabilities up to 2^40: bf16 only");
   // The arguments are read where they arrive: in the kernarg segment (constant address space, scalar loads),
   // through its base pointer -- AttnArgs is the kernel's only parameter, so it sits at offset 0.  Going through the
@@ -1083,19 +1318,37 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   const int h = bh - b * a.H;
 
   JobView view;
-  if (!view_job(a, job, view)) return;
+  const bool there = view_job(a, job, view);
+  if (!kMerge && !there) return;
   row0 += qt * kBQ;
-  const int rows = view.q_end - view.q_begin - row0;
-  if (rows <= 0) return;  // the grid is sized for the longest job / segment
-  bool split_keys = false;
-  if (!kPre && !is_part && (half_rows || rows <= kBQ / 2)) {
-    int n_tiles = 0;
-    for (int s = view.seg_begin; s < view.seg_end; ++s) n_tiles += (key_ref(view, s).len + kBK - 1) / kBK;
-    split_keys = n_tiles >= kMinSplitTiles;
-    if (!split_keys && half_rows && part > 0) return;   // part 0 does the whole tile
+  // (the grid is sized for the longest job / segment; a launch that merges has whole jobs only)
+  const int rows = there ? view.q_end - view.q_begin - row0 : 0;
+  if (!kMerge && rows <= 0) return;
+  // what this wavefront stores; of a job that is not there, its first workgroup says that nothing will come
+  int slice = part > 0 ? -1 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (!kMerge || rows > 0) {
+    bool split_keys = false;
+    if (!kPre && !is_part && (half_rows || rows <= kBQ / 2)) {
+      int n_tiles = 0;
+      for (int s = view.seg_begin; s < view.seg_end; ++s) n_tiles += (key_ref(view, s).len + kBK - 1) / kBK;
+      split_keys = n_tiles >= kMinSplitTiles;
+      if (!split_keys && half_rows && part > 0) return;   // part 0 does the whole tile
+    }
+    if (split_keys) attn_item<D, kPre, kHalf, kMerge, !kPre>(view, b, h, row0, false, 0, 0, 0, slice);
+    else attn_item<D, kPre, kHalf, kMerge, false>(view, b, h, row0, is_part, part, unit, xcd, slice);
   }
-  if (split_keys) attn_item<D, kPre, kHalf, !kPre>(view, b, h, row0, false, 0, 0, 0);
-  else attn_item<D, kPre, kHalf, false>(view, b, h, row0, is_part, part, unit, xcd);
+  if constexpr (kMerge) {
+    slice = __builtin_amdgcn_readfirstlane(slice);   // uniform by construction
+    if (slice < 0) return;
+    KernArgs& m = kernel_args();
+    const int at = item_of_block(m);
+    const int bh = at / m.nqt;
+    const int first = (at - bh * m.nqt) * kBQ + 32 * slice;
+    if (first >= m.Sq || !arrive_last(m.arrive + kPartCounters + (int64_t)at * kWaves + slice, m.merge_jobs)) return;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int b = bh / m.H;
+    merge_rows<D, kHalf>(lds + Tile<D>::kLdsTiles + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * Tile<D>::kStageBytes, b, bh - b * m.H, first);
+  }
 }
 
 // Folds the part_ways partial states of every split item into the item's rows of its destination.  A workgroup takes 64
@@ -1211,34 +1464,31 @@ __global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const Attn
 static_assert(Tile<128>::kLdsBytes == kAttnLdsBytes128 && Tile<64>::kLdsBytes == kAttnLdsBytes64,
               "dt_common.h states the LDS footprint of the attention kernel");
 
-template <int D, bool kPre, bool kHalf>
+template <int D, bool kPre, bool kHalf, bool kMerge>
 static int launch_one(const AttnArgs& a, dim3 grid, hipStream_t stream) {
   // more than 64 KB of dynamic LDS has to be allowed once per kernel and device
   static thread_local int allowed_dev = -1;
   int dev = 0;
   if (int rc = hip_fail(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (allowed_dev != dev) {
-    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kPre, kHalf>),
+    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kPre, kHalf, kMerge>),
                                               hipFuncAttributeMaxDynamicSharedMemorySize, Tile<D>::kLdsBytes),
                           "hipFuncSetAttribute"))
       return rc;
     allowed_dev = dev;
   }
-  hipLaunchKernelGGL((attn_fwd_kernel<D, kPre, kHalf>), grid, dim3(kThreads), Tile<D>::kLdsBytes, stream, a);
+  hipLaunchKernelGGL((attn_fwd_kernel<D, kPre, kHalf, kMerge>), grid, dim3(kThreads), Tile<D>::kLdsBytes, stream, a);
   return hip_fail(hipGetLastError(), "attn_fwd launch");
 }
 
 static int launch_dim(const AttnArgs& a, int D, dim3 grid, hipStream_t stream) {
-  if (a.elem_f16) {
-    if (D == 128) return launch_one<128, false, true>(a, grid, stream);
-    return launch_one<64, false, true>(a, grid, stream);
+  if (a.arrive) {
+    if (a.elem_f16) return D == 128 ? launch_one<128, false, true, true>(a, grid, stream) : launch_one<64, false, true, true>(a, grid, stream);
+    return D == 128 ? launch_one<128, false, false, true>(a, grid, stream) : launch_one<64, false, false, true>(a, grid, stream);
   }
-  if (a.q_prescaled) {
-    if (D == 128) return launch_one<128, true, false>(a, grid, stream);
-    return launch_one<64, true, false>(a, grid, stream);
-  }
-  if (D == 128) return launch_one<128, false, false>(a, grid, stream);
-  return launch_one<64, false, false>(a, grid, stream);
+  if (a.elem_f16) return D == 128 ? launch_one<128, false, true, false>(a, grid, stream) : launch_one<64, false, true, false>(a, grid, stream);
+  if (a.q_prescaled) return D == 128 ? launch_one<128, true, false, false>(a, grid, stream) : launch_one<64, true, false, false>(a, grid, stream);
+  return D == 128 ? launch_one<128, false, false, false>(a, grid, stream) : launch_one<64, false, false, false>(a, grid, stream);
 }
 
 // Number of CUs of the current device (one workgroup of the attention kernel per CU at a time).
@@ -1530,6 +1780,10 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   const unsigned planes_x = (unsigned)a.per_xcd * kXcds;
   if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);
   const int64_t slots = (int64_t)a.tail_items * kXcds * a.part_ways;
+  if (a.arrive && !a.row_split && (int64_t)a.tail_items * kXcds * kWaves > kPartCounters) {
+    set_error("internal: %d split items per XCD exceed the part counters", a.tail_items);
+    return DT_ERR_INVALID;
+  }
   // (the planner only considers splits that fit, so this cannot fire; it guards later edits to it)
   if (!a.row_split && slots * slot_bytes > workspace_bytes) {
     set_error("internal: tail split of %lld parts needs %lld bytes of scratch, %lld are there", (long long)slots,
@@ -1547,7 +1801,7 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   // parts per XCD, spread over planes of per_xcd entries
   const int part_planes = (a.tail_items * a.part_ways + a.per_xcd - 1) / a.per_xcd;
   const dim3 grid(planes_x, (unsigned)(a.job_planes + part_planes), 1);
-  if (a.row_split) return launch_dim(a, D, grid, stream);
+  if (a.row_split || a.arrive) return launch_dim(a, D, grid, stream);   // (nothing to fold, or folded by the launch itself)
   std::lock_guard<std::mutex> pair(workspace_lock(workspace));
   if (int rc = launch_dim(a, D, grid, stream)) return rc;
   const dim3 fold_grid((unsigned)a.tail_items * kXcds * kWaves * (D / 64)), fold_block(kFoldThreads);

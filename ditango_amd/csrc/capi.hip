@@ -122,22 +122,58 @@ static int apply_flags(AttnArgs& a, int32_t flags) {
   return DT_OK;
 }
 
-extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
-                                       int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
-                                       const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
-                                       int64_t kv_ss, int64_t kv_sh, int32_t n_jobs, const int32_t* job_begin,
-                                       const int32_t* job_chunks, const int32_t* entry_kv_begin,
-                                       const int32_t* entry_kv_len, const int32_t* job_q_begin,
-                                       const int32_t* job_q_len, void* const* out_ptrs, float* const* lse_ptrs,
-                                       float softmax_scale, int32_t flags, void* workspace,
-                                       int64_t workspace_bytes, void* stream) {
+extern "C" int64_t dt_attn_merge_counters(int32_t B, int32_t Sq, int32_t H) {
+  return B <= 0 || Sq <= 0 || H <= 0 ? 0 : kPartCounters + 8ll * B * H * (((int64_t)Sq + 255) / 256);
+}
+
+// The merge of a launch's states, of which there are `n_states`.
+static int fill_merge(AttnArgs& a, const dt_merge_result* r, int32_t D, int32_t n_jobs, int32_t n_states) {
+  if (a.q_prescaled) {
+    set_error("launches on a prescaled q do not merge");
+    return DT_ERR_UNSUPPORTED;
+  }
+  if (n_jobs <= 0 || n_states <= 0) {
+    set_error("a merging launch needs at least one job and one state (got %d, %d)", n_jobs, n_states);
+    return DT_ERR_INVALID;
+  }
+  if (!r->out || !r->lse || !aligned16(r->out) || (r->dtype != DT_FP32 && r->dtype != (a.elem_f16 ? DT_FP16 : DT_BF16))) {
+    set_error("the merged result must be 16-byte aligned, in fp32 or in the dtype of the states, with an lse");
+    return DT_ERR_INVALID;
+  }
+  if (!r->counters || (reinterpret_cast<uintptr_t>(r->counters) & 3) || r->n_counters < dt_attn_merge_counters(a.B, a.Sq, a.H)) {
+    set_error("a merging launch needs %lld counters", (long long)dt_attn_merge_counters(a.B, a.Sq, a.H));
+    return DT_ERR_INVALID;
+  }
+  if ((int64_t)a.H * D * 32 * 4 >= (1ll << 31)) {
+    set_error("%d heads: 32 rows of the result span 2 GiB or more", a.H);
+    return DT_ERR_UNSUPPORTED;
+  }
+  // (the kernel reads the states in eights)
+  AttnState* states = a.dev_ids ? a.arena : a.state;
+  for (int i = n_states; i % kMergeBatch; ++i) states[i] = states[n_states - 1];
+  a.merge_n = n_states;
+  a.merge_jobs = n_jobs;
+  a.arrive = r->counters;
+  a.merge_out = r->out;
+  a.merge_lse = r->lse;
+  a.merge_dtype = r->dtype;
+  return DT_OK;
+}
+
+static int jobs_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb, int64_t q_ss, int64_t q_sh,
+                    int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs, const int32_t* kv_lens,
+                    const int64_t* kv_sb, int64_t kv_ss, int64_t kv_sh, int32_t n_jobs, const int32_t* job_begin,
+                    const int32_t* job_chunks, const int32_t* entry_kv_begin, const int32_t* entry_kv_len,
+                    const int32_t* job_q_begin, const int32_t* job_q_len, void* const* out_ptrs, float* const* lse_ptrs,
+                    const dt_merge_result* merge, float softmax_scale, int32_t flags, void* workspace,
+                    int64_t workspace_bytes, void* stream) {
   if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
   AttnArgs a{};
   if (int rc = fill_common(a, q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh,
                            softmax_scale))
     return rc;
   if (int rc = apply_flags(a, flags)) return rc;
-  if (n_jobs == 0) return DT_OK;
+  if (n_jobs == 0 && !merge) return DT_OK;
   if (n_jobs < 0 || n_jobs > DT_MAX_JOBS || !job_begin || !job_chunks || !out_ptrs || !lse_ptrs) {
     set_error("%d jobs: need 0..%d and non-null job tables", n_jobs, DT_MAX_JOBS);
     return DT_ERR_INVALID;
@@ -145,6 +181,21 @@ extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int
   if (job_begin[0] != 0 || job_begin[n_jobs] > DT_MAX_JOB_ENTRIES) {
     set_error("job_begin must start at 0 and end at most at %d", DT_MAX_JOB_ENTRIES);
     return DT_ERR_INVALID;
+  }
+  if (merge) {
+    if (merge->n_states < 0 || merge->n_states > DT_MAX_MERGE_LIST || !merge->state_outs || !merge->state_lses) {
+      set_error("%d states to merge: need 1..%d and non-null lists", merge->n_states, DT_MAX_MERGE_LIST);
+      return DT_ERR_INVALID;
+    }
+    for (int i = 0; i < merge->n_states; ++i) {
+      if (!merge->state_outs[i] || !merge->state_lses[i] || !aligned16(merge->state_outs[i])) {
+        set_error("state %d: null or misaligned", i);
+        return DT_ERR_INVALID;
+      }
+      a.state[i].out = static_cast<const uint16_t*>(merge->state_outs[i]);
+      a.state[i].lse = merge->state_lses[i];
+    }
+    if (int rc = fill_merge(a, merge, D, n_jobs, merge->n_states)) return rc;
   }
   if ((entry_kv_begin == nullptr) != (entry_kv_len == nullptr) || (job_q_begin == nullptr) != (job_q_len == nullptr)) {
     set_error("range arrays come in (begin, len) pairs");
@@ -195,6 +246,36 @@ extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int
   a.total = B * H * a.nqt;
   a.per_xcd = (a.total + 7) / 8;
   return launch_attn(a, D, n_jobs, (hipStream_t)stream, workspace, workspace_bytes);
+}
+
+extern "C" int dt_attn_seg_jobs_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+                                       int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
+                                       const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
+                                       int64_t kv_ss, int64_t kv_sh, int32_t n_jobs, const int32_t* job_begin,
+                                       const int32_t* job_chunks, const int32_t* entry_kv_begin,
+                                       const int32_t* entry_kv_len, const int32_t* job_q_begin,
+                                       const int32_t* job_q_len, void* const* out_ptrs, float* const* lse_ptrs,
+                                       float softmax_scale, int32_t flags, void* workspace,
+                                       int64_t workspace_bytes, void* stream) {
+  return jobs_fwd(q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh, n_jobs, job_begin,
+                  job_chunks, entry_kv_begin, entry_kv_len, job_q_begin, job_q_len, out_ptrs, lse_ptrs, nullptr, softmax_scale,
+                  flags, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dt_attn_jobs_merge_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+                                      int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
+                                      const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
+                                      int64_t kv_ss, int64_t kv_sh, int32_t n_jobs, const int32_t* job_begin,
+                                      const int32_t* job_chunks, void* const* out_ptrs, float* const* lse_ptrs,
+                                      const dt_merge_result* merge, float softmax_scale, int32_t flags, void* workspace,
+                                      int64_t workspace_bytes, void* stream) {
+  if (!merge) {
+    set_error("no result to merge into");
+    return DT_ERR_INVALID;
+  }
+  return jobs_fwd(q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh, n_jobs, job_begin,
+                  job_chunks, nullptr, nullptr, nullptr, nullptr, out_ptrs, lse_ptrs, merge, softmax_scale, flags, workspace,
+                  workspace_bytes, stream);
 }
 
 // Device-resident segment boundaries: shared checks of the two varlen entry points.
@@ -479,6 +560,36 @@ extern "C" int dt_attn_sched_seg_ws_fwd(const void* q, int32_t B, int32_t Sq, in
     jobs = max_jobs * n_seg;
   }
   return launch_attn(a, D, jobs, (hipStream_t)stream, workspace, workspace_bytes);
+}
+
+extern "C" int dt_attn_sched_merge_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,
+                                       int64_t q_ss, int64_t q_sh, int32_t n_chunks, const void* const* k_ptrs,
+                                       const void* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
+                                       int64_t kv_ss, int64_t kv_sh, const int32_t* dev_compute_ids,
+                                       const int32_t* dev_count, int32_t max_jobs, void* slot_out,
+                                       int64_t slot_out_stride, float* slot_lse, int64_t slot_lse_stride, int32_t diag,
+                                       void* diag_out, float* diag_lse, const dt_merge_result* merge,
+                                       float softmax_scale, int32_t flags, void* workspace, int64_t workspace_bytes,
+                                       void* stream) {
+  if (int rc = check_workspace(workspace, workspace_bytes)) return rc;
+  AttnArgs a{};
+  if (int rc = fill_common(a, q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh,
+                           softmax_scale))
+    return rc;
+  if (int rc = apply_flags(a, flags)) return rc;
+  if (int rc = fill_sched(a, n_chunks, k_ptrs, v_ptrs, kv_lens, dev_compute_ids, dev_count, max_jobs, slot_out,
+                          slot_out_stride, slot_lse, slot_lse_stride, diag, diag_out, diag_lse))
+    return rc;
+  if (!merge) {
+    set_error("no result to merge into");
+    return DT_ERR_INVALID;
+  }
+  for (int c = 0; c < n_chunks; ++c) {
+    a.arena[c].out = c == diag ? a.diag_out : a.slot_out + c * slot_out_stride;
+    a.arena[c].lse = c == diag ? diag_lse : slot_lse + c * slot_lse_stride;
+  }
+  if (int rc = fill_merge(a, merge, D, max_jobs, n_chunks)) return rc;
+  return launch_attn(a, D, max_jobs, (hipStream_t)stream, workspace, workspace_bytes);
 }
 
 extern "C" int dt_attn_sched_varlen_ws_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb,

@@ -30,6 +30,11 @@ struct AttnJob {
   int32_t q_begin, q_len;
 };
 
+struct AttnState {
+  const uint16_t* out;        // [B,Sq,H,D]
+  const float* lse;           // [B,H,Sq]
+};
+
 // Kernel arguments of the chunk-attention kernel.  Passed by value, so the
 // chunk and job tables travel in the kernarg segment: no device-side table,
 // no host-to-device copy per call.  q, K, V and the output states are 16-bit elements: bfloat16, or IEEE half when
@@ -76,17 +81,32 @@ struct AttnArgs {
   float* ws_out;    // [slot][8 wavefronts][D / 8 groups of 4 elements][64 lanes][4], the accumulators as they lie in registers
   float* ws_lse;    // [slot][256]
   int32_t row_split;    // the tail items are cut in two along the query rows instead of along the keys (no partial states)
+  // Launches that merge (arrive != nullptr): whoever completes the last of the launch's merge_jobs states of 32 query rows
+  // merges the merge_n states there are of these rows (`arena` or `state` below) into merge_out and merge_lse ([B,Sq,H]).
+  // The parts of a split item meet in the same way; there is no fold kernel.  Counters: kPartCounters for the parts, then 8 per work item of a job.
+  int32_t merge_n;
+  uint32_t* arrive;
+  void* merge_out;
+  float* merge_lse;
+  int32_t merge_jobs;
+  int32_t merge_dtype;  // DT_FP32, or the states' own 16-bit type
   // ---- the host's own
   int32_t B;
   int32_t q_prescaled;  // the caller folded scale_log2 into q: scores are already in log2 units
   int32_t elem_f16;     // the 16-bit tensors are IEEE half instead of bfloat16
   // ---- tables
-  AttnJob job[DT_MAX_JOBS];
+  union {
+    AttnJob job[DT_MAX_JOBS];
+    AttnState arena[DT_MAX_CHUNKS];       // merging launches with device-listed jobs: what they merge
+  };
   AttnChunk chunk[DT_MAX_CHUNKS];
   AttnEntry entry[DT_MAX_JOB_ENTRIES];
   int32_t seg_q_begin[DT_MAX_SEGMENTS];
   int32_t seg_q_len[DT_MAX_SEGMENTS];
-  const int32_t* cu_kv[DT_MAX_CHUNKS];
+  union {
+    const int32_t* cu_kv[DT_MAX_CHUNKS];
+    AttnState state[DT_MAX_MERGE_LIST];   // ... with host-listed jobs
+  };
 };
 
 // Dynamic LDS of one attention workgroup by head dimension (four 64-key buffers per operand and the epilogue's
@@ -107,9 +127,16 @@ static_assert(kWorkspaceBytes / partial_state_bytes(64) == 1536 && kWorkspaceByt
 // chunk, D = 128 2156 -> 2145 us; D = 64, 1008 parts, 1271 -> 1253).
 constexpr int64_t kStaticTailBytes = DT_NOALLOC_TAIL_SLOTS * partial_state_bytes(64);
 static_assert(kStaticTailBytes / partial_state_bytes(64) == 1024 && kStaticTailBytes / partial_state_bytes(128) == 515);
+// Arrival counters of the parts of split items in a merging launch: one per 32-row slice of an item; a launch splits fewer
+// items than the chip has CUs.
+constexpr int kPartCounters = 2048;
+
 // Device address and size of that array on the current device (looked up once per device).
 int static_tail_scratch(void** ptr, int64_t* bytes);
 
+constexpr int kMergeBatch = 8;   // the lists of states are filled up to multiples of this with the last one
+static_assert(DT_MAX_CHUNKS % kMergeBatch == 0 && DT_MAX_MERGE_LIST % kMergeBatch == 0, "filled lists stay in their place");
+static_assert(DT_MAX_MERGE_LIST * sizeof(AttnState) <= DT_MAX_CHUNKS * sizeof(int32_t*), "the list shares the boundaries' place");
 static_assert(sizeof(AttnArgs) <= 4096, "the kernel arguments travel in the 4 KB kernarg segment");
 
 int launch_attn(const AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace = nullptr,

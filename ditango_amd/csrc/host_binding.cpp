@@ -217,7 +217,7 @@ void attn_jobs(const Tensor& q, const ChunkTable& table, const std::vector<std::
                const std::optional<std::vector<Range>>& q_ranges,
                const std::optional<std::vector<std::vector<Range>>>& kv_ranges, const std::optional<Tensor>& workspace,
                int32_t flags, bool no_alloc, const Segments* seg, const std::optional<std::vector<int32_t>>& job_segments,
-               uint64_t stream) {
+               uint64_t stream, const dt_merge_result* merge = nullptr) {
   const Dims d = check_query(q, table);
   const size_t nj = jobs.size();
   REQUIRE(!(no_alloc && workspace), "no_alloc launches take no workspace");
@@ -296,7 +296,10 @@ void attn_jobs(const Tensor& q, const ChunkTable& table, const std::vector<std::
     }
     begin[n] = e;
     const auto sq = q.strides();
-    if (seg)
+    if (merge)   // (the caller has seen to it that there is one launch, without ranges)
+      CALL(dt_attn_jobs_merge_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss, table.sh, n,
+           begin, chunks, op, lp, merge, (float)scale, flags, ptr(workspace), bytes_of(workspace), stream_of(stream));
+    else if (seg)
       CALL(dt_attn_varlen_jobs_ws_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], nc, kp, vp, lens, sbs, table.ss,
            table.sh, n, begin, chunks, segs, seg->n_seg(), static_cast<const int32_t*>(ptr(seg->cu_q)), cu_kv,
            (int32_t)seg->max_q, op, lp, (float)scale, flags, ptr(workspace), bytes_of(workspace), stream_of(stream));
@@ -324,13 +327,32 @@ typedef std::vector<std::pair<Tensor, Tensor>> States;
 std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, std::optional<Tensor> dst_out,
                                 std::optional<Tensor> dst_lse, at::ScalarType dst_dtype, bool dst_bsh, uint64_t stream);
 
+// Whether a launch can merge into a state of dst_dtype (see dt_merge_result).
+bool can_merge(const Tensor& q, const Dims& d, at::ScalarType dst_dtype, int32_t flags, const std::optional<Tensor>& counters) {
+  if (!counters || (flags & DT_ATTN_Q_PRESCALED) || (dst_dtype != at::kFloat && dst_dtype != q.scalar_type())) return false;
+  REQUIRE(counters->is_cuda() && counters->scalar_type() == at::kInt && counters->is_contiguous(), "counters must be int32 on the GPU");
+  return d.H * d.D * 32 * 4 < (1ll << 31);   // (the number of counters is checked with the launch)
+}
+dt_merge_result merge_into(const Tensor& out, const Tensor& lse, const Tensor& counters) {
+  return {ptr(out), static_cast<float*>(ptr(lse)), dtype_code(out), 0, nullptr, nullptr, static_cast<uint32_t*>(ptr(counters)), counters.numel()};
+}
+
+// What attn_states merges behind its launch, or with it: `outs`, `lses` and then states[which[..]].
+struct StatesMerge {
+  std::vector<Tensor> outs, lses;
+  std::vector<int32_t> which;
+  at::ScalarType dtype;
+  std::optional<Tensor> counters;
+  std::pair<Tensor, Tensor> result;
+};
+
 // The fresh states (out in q's dtype, lse [B,H,Sq]) of q against the concatenations of the chunks jobs[j]
 // (ditango_amd._hip.attn_states): one launch, unless the jobs exceed its limits; a job of more than max_chunks chunks is
 // computed in pieces that are folded into its state.
 States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs,
                    const std::vector<std::vector<int32_t>>& jobs, int64_t max_chunks, const std::optional<std::vector<int32_t>>& cu_q,
                    const std::optional<std::vector<std::vector<int32_t>>>& cu_kv, const std::optional<Tensor>& workspace,
-                   int32_t flags, const Segments* seg, const py::object& convert, uint64_t stream) {
+                   int32_t flags, const Segments* seg, const py::object& convert, uint64_t stream, StatesMerge* m = nullptr) {
   REQUIRE(q.dim() == 4, "q must be [B,S,H,D] with contiguous D");
   const Dims d{q.size(0), q.size(1), q.size(2), q.size(3)};
   const ChunkTable table(ks, vs, d.B, convert);
@@ -370,8 +392,38 @@ States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::ve
     }
     if (pieces.size() - first > 1) folds.emplace_back(first, pieces.size() - first);
   }
-  if (lists.empty()) return states;
-  attn_jobs(q, table, lists, outs, lses, 0.0, cu_q ? std::optional(std::move(q_ranges)) : std::nullopt,
+  if (m) {
+    for (int32_t i : m->which) {
+      REQUIRE(i >= 0 && (size_t)i < states.size(), "merge of a state that is not computed");
+      m->outs.push_back(states[i].first);
+      m->lses.push_back(states[i].second);
+    }
+    // one launch of whole jobs, and states in the form that it reads
+    size_t entries = 0;
+    for (const auto& list : lists) entries += list.size();
+    bool whole = !seg && !cu_q && folds.empty() && !lists.empty() && lists.size() <= DT_MAX_JOBS && entries <= DT_MAX_JOB_ENTRIES &&
+                 table.n <= DT_MAX_CHUNKS && m->outs.size() <= DT_MAX_MERGE_LIST && can_merge(q, d, m->dtype, flags, m->counters);
+    const void* state_outs[DT_MAX_MERGE_LIST];
+    const float* state_lses[DT_MAX_MERGE_LIST];
+    for (size_t i = 0; whole && i < m->outs.size(); ++i) {
+      const Tensor &o = m->outs[i], &l = m->lses[i];
+      whole = o.scalar_type() == q.scalar_type() && o.is_cuda() && o.is_contiguous() && shape_is(o, {d.B, d.S, d.H, d.D}) &&
+              lse_layout(l, d.B, d.S, d.H) == DT_LSE_BHS && (reinterpret_cast<uintptr_t>(ptr(o)) & 15) == 0;
+      state_outs[i] = ptr(o);
+      state_lses[i] = static_cast<const float*>(ptr(l));
+    }
+    if (whole) {
+      m->result = {new_out(d, m->dtype, q), new_lse(d, true, q)};
+      dt_merge_result into = merge_into(m->result.first, m->result.second, *m->counters);
+      into.n_states = (int32_t)m->outs.size();
+      into.state_outs = state_outs;
+      into.state_lses = state_lses;
+      attn_jobs(q, table, lists, outs, lses, 0.0, std::nullopt, std::nullopt, workspace, flags, false, nullptr, std::nullopt, stream, &into);
+      return states;
+    }
+  }
+  if (lists.empty() && !m) return states;
+  if (!lists.empty()) attn_jobs(q, table, lists, outs, lses, 0.0, cu_q ? std::optional(std::move(q_ranges)) : std::nullopt,
             cu_q ? std::optional(std::move(kv_ranges)) : std::nullopt, workspace, flags, false, seg,
             seg ? std::optional(std::move(segs)) : std::nullopt, stream);
   for (const auto& [first, n] : folds) {
@@ -382,7 +434,21 @@ States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::ve
     }
     merge(o, l, o[0], l[0], q.scalar_type(), false, stream);
   }
+  if (m) m->result = merge(m->outs, m->lses, std::nullopt, std::nullopt, m->dtype, true, stream);
   return states;
+}
+
+// attn_states, and the merge of (outs, lses) and states[which[..]], in the same launch where it can (ditango_amd._hip.attn_states_merge).
+std::tuple<States, Tensor, Tensor> attn_states_merge(
+    const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs, const std::vector<std::vector<int32_t>>& jobs,
+    int64_t max_chunks, const std::optional<std::vector<int32_t>>& cu_q, const std::optional<std::vector<std::vector<int32_t>>>& cu_kv,
+    const std::optional<Tensor>& workspace, int32_t flags, const Segments* seg, const py::object& convert, std::vector<Tensor> outs,
+    std::vector<Tensor> lses, std::vector<int32_t> which, at::ScalarType dst_dtype, const std::optional<Tensor>& counters,
+    uint64_t stream) {
+  REQUIRE(outs.size() == lses.size(), "one lse per state");
+  StatesMerge m{std::move(outs), std::move(lses), std::move(which), dst_dtype, counters, {}};
+  States states = attn_states(q, ks, vs, jobs, max_chunks, cu_q, cu_kv, workspace, flags, seg, convert, stream, &m);
+  return {std::move(states), m.result.first, m.result.second};
 }
 
 // The fp32 states of fp32 q against the concatenations of the fp32 chunks jobs[j] (ditango_amd._hip.attn_jobs_f32_fwd); every
@@ -450,7 +516,7 @@ void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, con
                 const Tensor& slot_out, const Tensor& slot_lse, int32_t diag, const std::optional<Tensor>& diag_out,
                 const std::optional<Tensor>& diag_lse, double scale, const std::optional<std::vector<Range>>& seg_q,
                 const std::optional<std::vector<std::vector<Range>>>& seg_kv, const std::optional<Tensor>& workspace,
-                int32_t flags, const Segments* seg, uint64_t stream) {
+                int32_t flags, const Segments* seg, uint64_t stream, const dt_merge_result* merge = nullptr) {
   const Dims d = check_query(q, table);
   REQUIRE(table.n <= DT_MAX_CHUNKS, "the table holds ", std::to_string(table.n), " chunks, one launch addresses ",
           std::to_string(DT_MAX_CHUNKS));
@@ -478,6 +544,13 @@ void attn_sched(const Tensor& q, const ChunkTable& table, const Tensor& ids, con
   const int32_t* dev_count = static_cast<const int32_t*>(ptr(count)) + row * per_count;
   float* sl = static_cast<float*>(ptr(slot_lse));
   float* dl = static_cast<float*>(ptr(diag_lse));
+  if (merge) {   // (whole queries)
+    CALL(dt_attn_sched_merge_fwd, ptr(q), d.B, d.S, d.H, d.D, sq[0], sq[1], sq[2], (int32_t)table.n, table.k.data(),
+         table.v.data(), table.len.data(), table.sb.data(), table.ss, table.sh, dev_ids, dev_count, max_jobs, ptr(slot_out),
+         slot_out.stride(0), sl, slot_lse.stride(0), diag, ptr(diag_out), dl, merge, (float)scale, flags, ptr(workspace),
+         bytes_of(workspace), stream_of(stream));
+    return;
+  }
   if (seg) {
     REQUIRE(!seg_q && !seg_kv, "device segment boundaries replace the host ranges");
     REQUIRE((int64_t)seg->cu_kv.size() == table.n, "one cu_seqlens_kv per chunk of the table");
@@ -591,6 +664,25 @@ std::pair<Tensor, Tensor> merge_arena(const Tensor& arena_out, const Tensor& are
   return {dst_out, dst_lse};
 }
 
+// attn_sched on whole queries and the merge of the arena, in the same launch where it can (ditango_amd._hip.attn_sched_merge).
+std::pair<Tensor, Tensor> attn_sched_merge(const Tensor& q, const ChunkTable& table, const Tensor& ids, const Tensor& count, int64_t row,
+                                           int32_t max_jobs, const Tensor& slot_out, const Tensor& slot_lse, int32_t diag,
+                                           const Tensor& diag_out, const Tensor& diag_lse, at::ScalarType dst_dtype,
+                                           const std::optional<Tensor>& workspace, const std::optional<Tensor>& counters,
+                                           int32_t flags, uint64_t stream) {
+  const Dims d = check_query(q, table);
+  if (max_jobs > 0 && slot_out.dim() == 5 && slot_out.size(0) == table.n && can_merge(q, d, dst_dtype, flags, counters)) {
+    const Tensor out = new_out(d, dst_dtype, q), lse = new_lse(d, true, q);
+    const dt_merge_result into = merge_into(out, lse, *counters);
+    attn_sched(q, table, ids, count, row, max_jobs, slot_out, slot_lse, diag, diag_out, diag_lse, 0.0, std::nullopt, std::nullopt,
+               workspace, flags, nullptr, stream, &into);
+    return {out, lse};
+  }
+  attn_sched(q, table, ids, count, row, max_jobs, slot_out, slot_lse, diag, diag_out, diag_lse, 0.0, std::nullopt, std::nullopt,
+             workspace, flags, nullptr, stream);
+  return merge_arena(slot_out, slot_lse, diag, diag_out, diag_lse, dst_dtype, stream);
+}
+
 // One pass from (src_out, src_lse) into (dst_out, dst_lse), any dtypes and lse layouts.
 void copy_state(const Tensor& src_out, const Tensor& src_lse, const Tensor& dst_out, const Tensor& dst_lse, uint64_t stream) {
   REQUIRE(src_out.dim() == 4 && src_out.is_cuda() && src_out.is_contiguous(), "the source must be contiguous [B,Sq,H,D] on the GPU");
@@ -648,10 +740,30 @@ PYBIND11_MODULE(_ditango_host, m) {
         return py::make_tuple(k, v, t.len, t.sb);
       });
   py::class_<Segments>(m, "Segments").def(py::init(&make_segments)).def_property_readonly("n_seg", &Segments::n_seg);
-  m.def("attn_jobs", &attn_jobs);
-  m.def("attn_states", &attn_states);
+  m.def("attn_jobs", [](const Tensor& q, const ChunkTable& table, const std::vector<std::vector<int32_t>>& jobs,
+                        const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, double scale,
+                        const std::optional<std::vector<Range>>& q_ranges, const std::optional<std::vector<std::vector<Range>>>& kv_ranges,
+                        const std::optional<Tensor>& workspace, int32_t flags, bool no_alloc, const Segments* seg,
+                        const std::optional<std::vector<int32_t>>& job_segments, uint64_t stream) {
+    attn_jobs(q, table, jobs, outs, lses, scale, q_ranges, kv_ranges, workspace, flags, no_alloc, seg, job_segments, stream);
+  });
+  m.def("attn_states", [](const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs,
+                          const std::vector<std::vector<int32_t>>& jobs, int64_t max_chunks, const std::optional<std::vector<int32_t>>& cu_q,
+                          const std::optional<std::vector<std::vector<int32_t>>>& cu_kv, const std::optional<Tensor>& workspace,
+                          int32_t flags, const Segments* seg, const py::object& convert, uint64_t stream) {
+    return attn_states(q, ks, vs, jobs, max_chunks, cu_q, cu_kv, workspace, flags, seg, convert, stream);
+  });
+  m.def("attn_states_merge", &attn_states_merge);
   m.def("attn_states_f32", &attn_states_f32);
-  m.def("attn_sched", &attn_sched);
+  m.def("attn_sched", [](const Tensor& q, const ChunkTable& table, const Tensor& ids, const Tensor& count, int64_t row, int32_t max_jobs,
+                         const Tensor& slot_out, const Tensor& slot_lse, int32_t diag, const std::optional<Tensor>& diag_out,
+                         const std::optional<Tensor>& diag_lse, double scale, const std::optional<std::vector<Range>>& seg_q,
+                         const std::optional<std::vector<std::vector<Range>>>& seg_kv, const std::optional<Tensor>& workspace,
+                         int32_t flags, const Segments* seg, uint64_t stream) {
+    attn_sched(q, table, ids, count, row, max_jobs, slot_out, slot_lse, diag, diag_out, diag_lse, scale, seg_q, seg_kv, workspace, flags,
+               seg, stream);
+  });
+  m.def("attn_sched_merge", &attn_sched_merge);
   m.def("merge", &merge);
   m.def("merge_arena", &merge_arena);
   m.def("cache_store", &cache_store);

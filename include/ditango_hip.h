@@ -353,6 +353,53 @@ int dt_attn_seg_jobs_noalloc_fwd(const void* q, int32_t B, int32_t Sq, int32_t H
                                  float softmax_scale, int32_t flags, void* stream);
 
 /*
+ * An attention launch that also merges: dt_attn_jobs_fwd / dt_attn_sched_fwd followed by dt_merge_states, in one kernel.
+ * Whoever completes the last of the launch's states of 32 query rows merges the states there are of these rows, while other
+ * workgroups still compute: the launch sequence of one layer call (core/attention.py:110-216) without the pass
+ * over the states behind it.  The parts of a split tail (dt_attn_seg_jobs_ws_fwd) are folded in the same way.
+ *   out, dtype  the merged state [B,Sq,H,D], 16-byte aligned, DT_FP32 or the dtype of q
+ *   lse         fp32 [B,Sq,H]
+ *   counters    device memory, dt_attn_merge_counters(B, Sq, H) words that are zero; every launch leaves them at zero.
+ *               Launches that share them must not overlap on the GPU, like launches that share a workspace
+ *   state_outs, state_lses   (dt_attn_jobs_merge_fwd) HOST arrays of the n_states states to merge, [B,Sq,H,D] contiguous in the
+ *               dtype of q with lse [B,H,Sq]: destinations of the launch's jobs, cached states, in any order; one may
+ *               appear more than once.  dt_attn_sched_merge_fwd merges every slot 0 .. n_chunks - 1 of the
+ *               arena, slot `diag` replaced by (diag_out, diag_lse), and does not read the lists
+ * Not with DT_ATTN_Q_PRESCALED (DT_ERR_UNSUPPORTED); at least one job.  A workspace as for dt_attn_seg_jobs_ws_fwd.
+ */
+#define DT_MAX_MERGE_LIST 16
+typedef struct dt_merge_result {
+  void* out;
+  float* lse;
+  int32_t dtype;
+  int32_t n_states;
+  const void* const* state_outs;
+  const float* const* state_lses;
+  uint32_t* counters;
+  int64_t n_counters;
+} dt_merge_result;
+int64_t dt_attn_merge_counters(int32_t B, int32_t Sq, int32_t H);
+int dt_attn_jobs_merge_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
+                           int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                           int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,
+                           const int32_t* kv_lens, const int64_t* kv_stride_b,
+                           int64_t kv_stride_s, int64_t kv_stride_h,
+                           int32_t n_jobs, const int32_t* job_begin, const int32_t* job_chunks,
+                           void* const* out_ptrs, float* const* lse_ptrs, const dt_merge_result* merge,
+                           float softmax_scale, int32_t flags, void* workspace, int64_t workspace_bytes,
+                           void* stream);
+int dt_attn_sched_merge_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
+                            int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                            int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,
+                            const int32_t* kv_lens, const int64_t* kv_stride_b,
+                            int64_t kv_stride_s, int64_t kv_stride_h,
+                            const int32_t* dev_compute_ids, const int32_t* dev_count, int32_t max_jobs,
+                            void* slot_out, int64_t slot_out_stride, float* slot_lse, int64_t slot_lse_stride,
+                            int32_t diag, void* diag_out, float* diag_lse, const dt_merge_result* merge,
+                            float softmax_scale, int32_t flags, void* workspace, int64_t workspace_bytes,
+                            void* stream);
+
+/*
  * N-way LSE merge: lse = logsumexp_i lse_i, out = sum_i exp(lse_i - lse) out_i.
  * Replaces the chain of update_out_and_lse / _update_out_and_lse calls
  * (utils.py:24-84; called at core/attention.py:116,144,194,196,213 and

@@ -1,0 +1,136 @@
+"""Launches that merge (``dt_attn_sched_merge_fwd``, ``dt_attn_jobs_merge_fwd``) against the same launch without a merge and
+the merge kernel behind it: the two compute one thing, in fp32 from the same 16-bit states."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from ditango_amd import _hip
+    _hip.load_library()
+    return _hip
+
+
+def _inputs(B, Sq, H, D, lens, dtype, strided=False):
+    g = torch.Generator(device="cuda").manual_seed(Sq * 131 + H * 7 + D)
+
+    def make(n):
+        if strided:   # slices of a fused projection
+            return torch.randn(B, n, 3, H, D, generator=g, device="cuda").to(dtype)[:, :, 1]
+        return torch.randn(B, n, H, D, generator=g, device="cuda").to(dtype)
+
+    return make(Sq), [make(n) for n in lens], [make(n) for n in lens]
+
+
+def _close(got, want, dtype, what):
+    """fp32 results of the same states: products and sums of n terms in another order and another exp's last bits, 2^-20 of the
+    largest value here.  A 16-bit result, or states that were folded from parts (another order under their rounding), may differ by one
+    rounding of a state: 2^-8 (bf16) or 2^-11 (fp16) of the value's binade."""
+    tol = {torch.float32: 2.0 ** -20, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    scale = max(1.0, want.float().abs().max().item())
+    assert (got.float() - want.float()).abs().max().item() <= tol * scale, what
+    assert torch.isfinite(got.float()).all(), what
+
+
+# rows: one, the edges of a 32-row slice, of half a tile and of a tile, several tiles; chunks without keys, of less than a key
+# tile, of the sizes at which a launch is cut along its rows (8 key tiles) and along its keys (16 and more)
+SHAPES = [
+    (1, 1, 3, 64, (40, 0, 64), (0, 2)), (1, 31, 2, 128, (64, 65, 1), (0, 1, 2)), (2, 33, 3, 64, (200, 130), (1,)),
+    (1, 127, 4, 128, (512, 512, 512), (0, 2)), (1, 129, 4, 64, (512, 512, 512), (0, 2)), (1, 512, 4, 64, (512,) * 4, (0, 3)),
+    (1, 255, 2, 128, (1500, 700), (0, 1)), (2, 257, 3, 64, (2000, 1999, 2000), (0, 1)), (1, 300, 2, 64, (4000, 4000), (0,)),
+    (1, 700, 5, 128, (1100,) * 11, (0, 4, 10)), (1, 1861, 6, 64, (1861,) * 3 + (1860,) * 2, (0, 3)), (1, 96, 1, 128, (96,) * 40, (7,)),
+]
+
+
+@pytest.mark.parametrize("B,Sq,H,D,lens,computed", SHAPES)
+@pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_scheduled_launch_that_merges(hip, B, Sq, H, D, lens, computed, dtype, out):
+    q, ks, vs = _inputs(B, Sq, H, D, lens, dtype, strided=Sq % 2 == 1)
+    C, diag = len(lens), computed[0]
+    table = hip.ChunkTable(ks, vs)
+    ids = torch.tensor(list(computed) + [-1] * (C - len(computed)), dtype=torch.int32, device="cuda")
+    count = torch.tensor([len(computed), 0], dtype=torch.int32, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(5)
+    slots = torch.randn(C, B, Sq, H, D, generator=g, device="cuda").to(dtype)
+    lses = 2 * torch.randn(C, B, H, Sq, generator=g, device="cuda")
+    ws = hip.attn_workspace("cuda")
+
+    def run(merging):
+        so, sl = slots.clone(), lses.clone()
+        do, dl = torch.zeros_like(so[0]), torch.zeros_like(sl[0])
+        args = (q, table, ids, count, C, so, sl, diag, do, dl)   # (more jobs than the schedule lists)
+        if merging:
+            return (*hip.attn_sched_merge(*args, out, ws), so, sl, do, dl)
+        hip.attn_sched_fwd(*args, workspace=ws)
+        return (*hip.merge_arena(so, sl, diag, do, dl, out), so, sl, do, dl)
+
+    want, got, again = run(False), run(True), run(True)
+    split = len(computed) * max(lens) >= 16 * 64 * len(computed)
+    for i, name in enumerate(("out", "lse", "slots", "slot lse", "local", "local lse")):
+        assert torch.equal(got[i], again[i]), name
+        loose = dtype if i in (2, 4) or (i == 0 and (split or out != torch.float32)) else torch.float32
+        _close(got[i], want[i], loose, name)
+    assert not hip.attn_counters("cuda", q).any()
+
+
+@pytest.mark.parametrize("B,Sq,H,D,lens,jobs,cached", [
+    (1, 65, 3, 64, (100, 100), [[0], [1]], 0), (1, 512, 4, 128, (512,) * 4, [[2], [0, 1, 3]], 3), (2, 333, 2, 64, (900, 1700, 64), [[0, 1, 2]], 1),
+    (1, 288, 5, 128, (2300, 1), [[0], [1], [0, 1]], 14),
+])
+def test_jobs_that_merge_with_cached_states(hip, B, Sq, H, D, lens, jobs, cached):
+    dtype = torch.bfloat16
+    q, ks, vs = _inputs(B, Sq, H, D, lens, dtype)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    outs = [torch.randn(B, Sq, H, D, generator=g, device="cuda").to(dtype) for _ in range(cached)]
+    lses = [2 * torch.randn(B, H, Sq, generator=g, device="cuda") for _ in range(cached)]
+    which = list(range(len(jobs))) + [0]   # (a state may be merged twice)
+    if cached + len(which) > 16:
+        which = which[:2]
+    ws = hip.attn_workspace("cuda")
+    states, out, lse = hip.attn_states_merge(q, ks, vs, jobs, 32, outs, lses, which, torch.float32, ws)
+    plain = hip.attn_states(q, ks, vs, jobs, 32, ws)
+    for (o, l), (po, pl) in zip(states, plain):
+        _close(o, po, dtype, "state")
+        _close(l, pl, torch.float32, "state lse")
+    want, want_lse = hip.merge_states(outs + [states[i][0] for i in which], lses + [states[i][1] for i in which], dst_lse_bsh=True)
+    _close(out, want, torch.float32, "out")
+    _close(lse, want_lse, torch.float32, "lse")
+    assert not hip.attn_counters("cuda", q).any()
+
+
+def test_rows_without_any_state_and_infinite_values(hip):
+    """A row whose states are all empty is 0 with lse -inf; an infinity in a state of weight is one in the result."""
+    q, ks, vs = _inputs(1, 40, 2, 64, (64, 64), torch.bfloat16)
+    so = torch.randn(2, 1, 40, 2, 64, device="cuda").bfloat16()
+    sl = torch.full((2, 1, 2, 40), float("-inf"), device="cuda")
+    ids = torch.zeros(2, dtype=torch.int32, device="cuda")
+    none = torch.zeros(2, dtype=torch.int32, device="cuda")
+    table = hip.ChunkTable(ks, vs)
+    out, lse = hip.attn_sched_merge(q, table, ids, none, 1, so, sl, -1, so[0], sl[0], torch.float32)
+    assert (out == 0).all() and (lse == float("-inf")).all()
+    sl.fill_(0.5)
+    so[1, 0, 7, 1, 3] = float("inf")
+    out, lse = hip.attn_sched_merge(q, table, ids, none, 1, so, sl, -1, so[0], sl[0], torch.float32)
+    assert out[0, 7, 1, 3] == float("inf") and torch.isinf(out).sum() == 1
+    _close(lse, torch.full_like(lse, 0.5 + 0.6931472), torch.float32, "lse")
+
+
+def test_merging_launch_replays_in_a_graph(hip):
+    q, ks, vs = _inputs(1, 600, 3, 64, (1500, 1500), torch.bfloat16)
+    run = lambda: hip.attn_states_merge(q, ks, vs, [[0], [1]], 32, [], [], [0, 1], torch.float32, hip.attn_workspace("cuda"))[1:]
+    want = run()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        run()
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            got = run()
+    for _ in range(4):
+        q.copy_(torch.randn(q.shape, device="cuda").bfloat16())
+        graph.replay()
+        want = run()
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
