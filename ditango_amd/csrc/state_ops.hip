@@ -442,6 +442,80 @@ __global__ __launch_bounds__(kThreads) void merge_states_kernel(const MergeArgs 
   }
 }
 
+// ---- the running state of a ring loop ----------------------------------------------------------
+// A 16-bit block state merged into an fp32 running state.  HBM-bound, 40 bytes an element and 2 of every 5 of them written.  As in
+// flat_copy_kernel below, a lane moves 16 bytes of the running state (and 8 of the block) and nothing else: the fewer
+// loads a wavefront has in flight, the faster such a mix of reads and writes runs here.  us per launch, lane groups of
+// merge_states_kernel (32 and 16 bytes a lane) -> here: 6851 x 48 heads, D = 128 77.6 -> 67.1 (6.3 TB/s), 14 882 x 24 83 -> 72.4,
+// D = 64 48.2 -> 38.0, 2222 x 48, D = 64 17.5 -> 13.1.  Workgroups of 512 and 1024 lanes 68.6 and 68.8.  One block
+// state alone (the first of a loop) is 24 bytes an element and bound by the instructions of so many lanes: it stays there (43.4;
+// 57 here).
+struct UpdateArgs {
+  const float* run;
+  const float* run_lse;
+  const uint16_t* blk;
+  const float* blk_lse;
+  float* dst;
+  float* dst_lse;         // may be null
+  int32_t Sq, H;
+  uint32_t rows;          // B * Sq * H
+  int32_t run_bsh, blk_bsh, dst_bsh;
+  uint32_t mul_h, mul_s;  // n / H and n / Sq for n < 2^31 (see quotient)
+  int32_t shift_h, shift_s;
+};
+constexpr int kUpdateThreads = 256;
+constexpr int kUpdateGroup = 64;   // workgroups that follow each other on one XCD (1: 3 % slower, 8: the same)
+
+// n / d for n < 2^31, with mul = ceil(2^(31 + L) / d) and shift = L - 1 for the smallest L with d <= 2^L: the error of mul, less
+// than d, times n stays below 2^(31 + L).  d = 1: shift -1.
+__device__ __forceinline__ uint32_t quotient(uint32_t n, uint32_t mul, int shift) {
+  return shift < 0 ? n : __umulhi(n, mul) >> shift;
+}
+static void set_quotient(int32_t d, uint32_t& mul, int32_t& shift) {
+  int L = 0;
+  while ((1ll << L) < d) ++L;
+  mul = L == 0 ? 0u : (uint32_t)(((1ull << (31 + L)) + (uint64_t)d - 1) / (uint64_t)d);
+  shift = L - 1;
+}
+
+template <int D, bool kF16>
+__global__ __launch_bounds__(kUpdateThreads) void merge_update_kernel(const UpdateArgs a) {
+  // The lse of consecutive queries share a line of the [B,H,Sq] layout; workgroups go to the 8 XCDs in turn.  So that a line
+  // is read into one L2 only, 64 workgroups that follow each other in memory are 64 of one XCD.
+  uint32_t wg = blockIdx.x;
+  constexpr uint32_t kSpan = 8 * kUpdateGroup;
+  if ((wg / kSpan + 1) * kSpan <= gridDim.x) wg = wg / kSpan * kSpan + (wg & 7u) * kUpdateGroup + (wg % kSpan >> 3);
+  const int64_t elem = ((int64_t)wg * kUpdateThreads + threadIdx.x) * 4;
+  const int64_t row64 = elem / D;
+  if (row64 >= a.rows) return;
+  const uint32_t row = (uint32_t)row64;   // ((b * Sq) + s) * H + h
+  uint32_t bhs = row;
+  if (!a.blk_bsh || !a.run_bsh || !a.dst_bsh) {
+    const uint32_t bs = quotient(row, a.mul_h, a.shift_h), h = row - bs * (uint32_t)a.H;
+    const uint32_t b = quotient(bs, a.mul_s, a.shift_s), q = bs - b * (uint32_t)a.Sq;
+    bhs = (b * (uint32_t)a.H + h) * (uint32_t)a.Sq + q;
+  }
+  const f32x4 x0 = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(a.run + elem));
+  const float l0 = a.run_lse[a.run_bsh ? row : bhs];
+  const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(a.blk + elem));
+  const float l1 = a.blk_lse[a.blk_bsh ? row : bhs];
+  float x1[4];
+  widen16x2(w.x, kF16, x1[0], x1[1]);
+  widen16x2(w.y, kF16, x1[2], x1[3]);
+  const float m = fmaxf(l0, l1);
+  f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+  if (m > -INFINITY) {
+    const float w0 = __expf(l0 - m), w1 = __expf(l1 - m);
+    den = w0 + w1;
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = __builtin_fmaf(w1, x1[e], w0 * x0[e]) * inv;
+  }
+  __builtin_nontemporal_store(y, reinterpret_cast<f32x4*>(a.dst + elem));
+  if (a.dst_lse != nullptr && elem % D == 0) a.dst_lse[a.dst_bsh ? row : bhs] = den > 0.f ? m + __logf(den) : -INFINITY;
+}
+
 struct CopyArgs {
   const void* src_out;
   const float* src_lse;
@@ -782,11 +856,46 @@ static void launch_merge_d(const MergeArgs& a, bool tiled, int passes, unsigned 
   }
 }
 
+// The launches of merge_update_kernel: an fp32 state and a 16-bit one behind it, into fp32.
+static bool is_update(const MergeArgs& a) {
+  return a.n == 2 && a.dst_dtype == DT_FP32 && a.fp32_mask == 1u && (int64_t)a.B * a.Sq * a.H < (1ll << 31);
+}
+
+static int launch_update(const MergeArgs& a, int D, hipStream_t stream) {
+  UpdateArgs u{};
+  u.run = static_cast<const float*>(a.out[0]);
+  u.run_lse = a.lse[0];
+  u.blk = static_cast<const uint16_t*>(a.out[1]);
+  u.blk_lse = a.lse[1];
+  u.dst = static_cast<float*>(a.dst_out);
+  u.dst_lse = a.dst_lse;
+  u.Sq = a.Sq;
+  u.H = a.H;
+  u.rows = (uint32_t)((int64_t)a.B * a.Sq * a.H);
+  u.run_bsh = (int32_t)(a.bsh_mask & 1);
+  u.blk_bsh = (int32_t)((a.bsh_mask >> 1) & 1);
+  u.dst_bsh = a.dst_bsh;
+  set_quotient(a.H, u.mul_h, u.shift_h);
+  set_quotient(a.Sq, u.mul_s, u.shift_s);
+  const int64_t lanes = (int64_t)u.rows * (D / 4);
+  const dim3 grid((unsigned)((lanes + kUpdateThreads - 1) / kUpdateThreads)), block(kUpdateThreads);
+  const bool f16 = (a.f16_mask >> 1) & 1;
+  if (D == 128) {
+    if (f16) hipLaunchKernelGGL((merge_update_kernel<128, true>), grid, block, 0, stream, u);
+    else hipLaunchKernelGGL((merge_update_kernel<128, false>), grid, block, 0, stream, u);
+  } else {
+    if (f16) hipLaunchKernelGGL((merge_update_kernel<64, true>), grid, block, 0, stream, u);
+    else hipLaunchKernelGGL((merge_update_kernel<64, false>), grid, block, 0, stream, u);
+  }
+  return hip_fail(hipGetLastError(), "merge_update launch");
+}
+
 int launch_merge(const MergeArgs& a, int D, hipStream_t stream) {
   if (D != 128 && D != 64) {
     set_error("head dim %d not built (64 and 128 are)", D);
     return DT_ERR_UNSUPPORTED;
   }
+  if (is_update(a)) return launch_update(a, D, stream);
   const int R = 128 / D;   // rows per unit
   const int64_t units = ((int64_t)a.B * a.Sq * a.H + R - 1) / R;
   const bool tiled = unit_tiles_fit(a.H, D);

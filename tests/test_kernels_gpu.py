@@ -622,3 +622,32 @@ def test_running_state_from_one_row_to_256_mib(hip, rows):
     ref = blocks[0][0].float() * (1 - w) + blocks[1][0].float() * w
     torch.testing.assert_close(out, ref, rtol=2e-6, atol=4e-6)   # the weights carry a few ulp, the terms are below 6
     torch.testing.assert_close(lse[..., 0], torch.logaddexp(blocks[0][1], blocks[1][1]).transpose(1, 2), rtol=0, atol=2e-6)
+
+
+@pytest.mark.parametrize("B,Sq,H,D", [(1, 1, 1, 64), (1, 1, 1, 128), (3, 7, 1, 64), (1, 1, 37, 128), (2, 5, 3, 128), (1, 300, 7, 64),
+                                      (1, 523, 24, 128), (2, 1031, 48, 64)])
+@pytest.mark.parametrize("layouts", [(1, 0, 1), (0, 1, 0), (1, 1, 1)])
+def test_running_state_and_a_block(hip, B, Sq, H, D, layouts):
+    """The update of an fp32 running state has a kernel of its own: one row, one head, one query, odd counts, enough workgroups
+    for their reordering and a remainder behind it; every lse layout; empty rows on either side and on both; in place.
+    Against the closed form in 64 bits: three roundings of fp32 an element (2^-22 of the largest, here below 8) and the exp's."""
+    gen = torch.Generator().manual_seed(B + Sq * 3 + H * 5 + D)
+    for dtype in (torch.bfloat16, torch.float16):
+        run, blk = torch.randn(B, Sq, H, D, generator=gen), torch.randn(B, Sq, H, D, generator=gen).to(dtype)
+        lses = [4 * torch.randn(B, H, Sq, generator=gen) for _ in range(2)]
+        lses[0][:, :, ::3] = -math.inf
+        lses[1][:, :, ::2] = -math.inf
+        store = lambda l, bsh: (l.transpose(1, 2).contiguous().unsqueeze(-1) if bsh else l).cuda()
+        w = torch.stack(lses).double()
+        ref_lse = torch.logsumexp(w, 0)
+        p = torch.nan_to_num(torch.exp(w - ref_lse)).permute(0, 1, 3, 2).unsqueeze(-1)
+        ref = p[0] * run.double() + p[1] * blk.double()
+        for in_place in (False, True):
+            d_run, d_lse = run.cuda(), store(lses[0], layouts[0])
+            out, lse = (d_run, d_lse) if in_place else (torch.full_like(d_run, math.nan), store(torch.zeros(B, H, Sq), layouts[2]))
+            hip.merge_states([d_run, blk.cuda()], [d_lse, store(lses[1], layouts[1])], dst_out=out, dst_lse=lse)
+            got = (lse.squeeze(-1).transpose(1, 2) if lse.dim() == 4 else lse).cpu().double()
+            assert (out.cpu().double() - ref).abs().max() <= 4e-6
+            none = torch.isinf(ref_lse)
+            assert (got[none] == -math.inf).all()
+            assert torch.where(none, 0.0, got - ref_lse).abs().max() <= 4e-6
