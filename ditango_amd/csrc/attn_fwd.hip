@@ -450,23 +450,34 @@ __device__ __forceinline__ bool arrive_last(uint32_t* counter, int expected) {
 }
 
 // Merges the states there are of the 32 query rows from row0 on (one batch and head): out = sum_i w_i out_i / sum_i w_i with
-// w_i = exp(lse_i - max), all in fp32.  One wavefront, which needs nobody else: `stage` is LDS of its own, 2 KB.
+// w_i = exp(lse_i - max), all in fp32.  One wavefront, which needs nobody else: `stage` is LDS of its own.
 //
-// HBM-bound: the workgroups of a launch run in step, so the last job's all merge at the end of a round, at 5.3 TB/s.  A
-// wavefront has two steps (8 states x 4 rows of a load instruction, D = 64: 4 x 8) in flight all the time, also across
-// the batches of states; three make no difference.  Against a merge kernel behind the launch: 24 heads x 119 056 queries, 3 of 32
-// chunks computed 17.79 -> 16.47 ms; 48 heads x 2222, D = 64, 5 of 8 340 -> 336 us; 4 heads x 512, D = 64, 2 of 4 19.4 -> 16.6;
-// two samples of 24 heads x 1861, 3 of 8 284 -> 284.  Tried without success: the jobs side by side, each some items
-// behind the one before it, so that a part of the workgroups merges while the others compute (they fall out of step and no
-// longer share keys and values in the L2: 24 heads x 14 882, 4 of 8 8.53 -> 8.75 ms); adjacent heads on the 8 XCDs (16.1 -> 16.6 ms).
-template <int D, bool kHalf>
+// HBM-bound in large launches: the workgroups run in step, so the last job's all merge at the end of a round, at 5.3 TB/s.
+// Against a merge kernel behind the launch: 24 heads x 119 056 queries, 3 of 32 chunks computed 17.79 -> 16.07 ms; 48 heads x
+// 2222, D = 64, 5 of 8 340 -> 336 us; 4 heads x 512, D = 64, 2 of 4 19.1 -> 15.6.  Tried without success: the jobs side by side,
+// each some items behind the one before it, so that a part of the workgroups merges while the others compute (they fall out of
+// step and no longer share keys and values in the L2: 24 heads x 14 882, 4 of 8 8.53 -> 8.75 ms); adjacent heads on the 8 XCDs
+// (16.1 -> 16.6 ms).
+//
+// In small ones a chain of waits at the end of the launch: one wavefront reads 32 rows of all states.  Up to 8 states
+// (kOneBatch) every weight is known before the first row, so rows are finished one after the other, without accumulators for
+// all of them, and the registers hold loads instead: 128 at D = 128 (4 steps of 8 states or all 8 steps of 4), 64 at D = 64.
+// us per call, two steps in flight -> this: 24 heads x 200 queries, D = 128, 1 of 2 chunks 22.8 -> 19.9, 4 of 8 27.1 -> 26.7; 40
+// heads x 2222, D = 128, 2 of 4 221 -> 217; 12 heads x 700, D = 64, 1 of 2 17.4 -> 16.9.  More states keep 32 rows of sums in
+// registers and two steps in flight (three make no difference to 29 states of 743 MB; four at D = 64 cost 24 heads x 200
+// queries, 16 states 1.5 us).
+template <int D, bool kHalf, int kStates, bool kOneBatch>
 __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row0) {
   typedef Elem<kHalf> E;
-  constexpr int kBatch = D == 128 ? 8 : 4;   // states of a step (D = 64: half the registers)
-  constexpr int kRowLanes = D / 8;           // a lane holds 8 columns of a row
-  constexpr int kRowsPer = 64 / kRowLanes;   // rows of a load instruction
-  constexpr int kSteps = 32 / kRowsPer;      // steps of a batch of states
-  static_assert(kMergeBatch % kBatch == 0, "the lists are filled up to whole batches");
+  constexpr int kLoads = D == 128 ? kStates : 4;        // states of a step
+  constexpr int kParts = kStates / kLoads;              // steps of the same rows
+  constexpr int kDepth = (kOneBatch ? D / 4 : D / 8) / kLoads;   // steps in flight
+  constexpr int kRowLanes = D / 8;                      // a lane holds 8 columns of a row
+  constexpr int kRowsPer = 64 / kRowLanes;              // rows of a load instruction
+  constexpr int kRowSteps = 32 / kRowsPer;
+  constexpr int kSteps = kRowSteps * kParts;            // steps of a batch of states
+  static_assert(kMergeBatch % kStates == 0, "the lists are filled up to whole batches");
+  static_assert(kSteps % kDepth == 0, "a step's registers are known at compile time");
   KernArgs& a = kernel_args();
   typedef const AttnState __attribute__((address_space(4))) KernState;
   KernState* states = a.dev_ids ? a.arena : a.state;
@@ -481,95 +492,72 @@ __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row
   const uint32_t lane_off = (uint32_t)(lane / kRowLanes) * row_bytes + 16u * (uint32_t)(lane % kRowLanes);
   // The batch under the load cursor.  States that are not there (behind the last one, and everything once i0 < 0) are empty
   // descriptors: their loads touch no memory and return zeros.
-  int i0 = (n - 1) / kBatch * kBatch;
-  u32x4 r[kBatch];
+  int i0 = (n - 1) / kStates * kStates;
+  u32x4 r[kStates];
   auto open = [&]() __attribute__((always_inline)) {
     KernState* st = states + max(i0, 0);
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) r[j] = make_rsrc(st[j].out + out_at, i0 >= 0 && i0 + j < n ? valid : 0u);
+    for (int j = 0; j < kStates; ++j) r[j] = make_rsrc(st[j].out + out_at, i0 >= 0 && i0 + j < n ? valid : 0u);
   };
-  u32x4 x[2][kBatch];
+  u32x4 x[kDepth][kLoads];
   auto load = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j)
-      x[s & 1][j] = __builtin_amdgcn_raw_buffer_load_b128(
-          __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)r[j].y << 32 | r[j].x), 0, r[j].z, kRsrcFlags),
-          lane_off, (uint32_t)(s * kRowsPer) * row_bytes, kDeviceNt);
+    for (int j = 0; j < kLoads; ++j) {
+      const u32x4& d = r[s % kParts * kLoads + j];
+      x[s % kDepth][j] = __builtin_amdgcn_raw_buffer_load_b128(
+          __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)d.y << 32 | d.x), 0, d.z, kRsrcFlags),
+          lane_off, (uint32_t)(s / kParts * kRowsPer) * row_bytes, kDeviceNt);
+    }
   };
-  float l[kBatch];
+  float l[kStates];
   auto load_lse = [&](int i0) __attribute__((always_inline)) {   // (the lists go on behind the last state with copies of it)
     KernState* st = states + max(i0, 0);
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) l[j] = load_device(st[j].lse + lse_at + my_row);
+    for (int j = 0; j < kStates; ++j) l[j] = load_device(st[j].lse + lse_at + my_row);
   };
+  if (kOneBatch) load_lse(0);
   open();
-  load(0);
-  load(1);
+#pragma unroll
+  for (int s = 0; s < kDepth; ++s) load(s);
   float m = -INFINITY, den = 0.f;
-  for (int i = 0; i < n; i += kBatch) {   // (the last batch, which comes first below, stays in l)
-    load_lse(i);
+  for (int i = 0; i < n; i += kStates) {   // (the last batch, which comes first below, stays in l)
+    if (!kOneBatch) load_lse(i);
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) m = fmaxf(m, l[j]);
+    for (int j = 0; j < kStates; ++j) m = fmaxf(m, l[j]);
+    if (kOneBatch) break;
   }
-  float acc[kSteps][8];
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[s][e] = 0.f;
-  float* weights = reinterpret_cast<float*>(stage);   // [32 rows][kBatch]
-  while (i0 >= 0) {
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      l[j] = i0 + j < n && m > -INFINITY ? __expf(l[j] - m) : 0.f;
-      den += l[j];
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; j += 4) *reinterpret_cast<f32x4*>(weights + col * kBatch + j) = f32x4{l[j], l[j + 1], l[j + 2], l[j + 3]};
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const float* ws = weights + (s * kRowsPer + lane / kRowLanes) * kBatch;
-      f32x4 wv[kBatch / 4];
-#pragma unroll
-      for (int j = 0; j < kBatch / 4; ++j) wv[j] = *reinterpret_cast<const f32x4*>(ws + 4 * j);
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const f32x2 v = E::widen(x[s & 1][j][e]);
-          acc[s][2 * e] = __builtin_fmaf(wv[j / 4][j % 4], v.x, acc[s][2 * e]);
-          acc[s][2 * e + 1] = __builtin_fmaf(wv[j / 4][j % 4], v.y, acc[s][2 * e + 1]);
-        }
-      if (s + 2 == kSteps) {   // the next batch
-        i0 -= kBatch;
-        open();
-        load_lse(i0);
-      }
-      load((s + 2) % kSteps);
-      __builtin_amdgcn_sched_barrier(0);   // the loads stay behind the step that frees their registers
-    }
-  }
-  const float inv = den > 0.f ? 1.f / den : 0.f;
-  if (lane < rows) a.merge_lse[((int64_t)b * Sq + row0 + lane) * H + h] = den > 0.f ? m + __logf(den) : -INFINITY;
   const bool wide = a.merge_dtype == DT_FP32;
   const Rsrc dst = buffer_of(static_cast<uint8_t*>(a.merge_out) + out_at * (wide ? 4 : 2), wide ? 2 * valid : valid);
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    const float f = __shfl(inv, s * kRowsPer + lane / kRowLanes);
-    // (rows whose states are all empty: 0, whatever the states hold)
-    const bool none = !(__shfl(m, s * kRowsPer + lane / kRowLanes) > -INFINITY);
+  // 1 / sum of the weights of row `col`; -1 for a row whose states are all empty, whose result is 0, whatever the states hold
+  float norm;
+  auto finish_row = [&]() __attribute__((always_inline)) {
+    norm = !(m > -INFINITY) ? -1.f : den > 0.f ? 1.f / den : 0.f;
+    if (lane < rows) a.merge_lse[((int64_t)b * Sq + row0 + lane) * H + h] = den > 0.f ? m + __logf(den) : -INFINITY;
+  };
+  float* weights = reinterpret_cast<float*>(stage);   // [32 rows][kStates]
+  auto store_rows = [&](int rs, float f, const float (&sum)[8]) __attribute__((always_inline)) {
     float o[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = none ? 0.f : acc[s][e] * f;
+    for (int e = 0; e < 8; ++e) o[e] = f < 0.f ? 0.f : sum[e] * f;
     if (wide) {
       // A lane's 32 bytes as two stores would write every other 16 bytes of a line: through the LDS, so that a store covers
-      // whole rows (24 heads x 14 882 queries against one key tile, 8 states merged: 250 -> 232 us).
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        *reinterpret_cast<f32x4*>(stage + lane * 32 + 16 * q) = f32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
+      // whole rows (24 heads x 14 882 queries against one key tile, 8 states merged: 250 -> 232 us; stores of half lines, exchanged
+      // in the registers of four lanes, lose as much).
+      constexpr int kWeightBytes = kOneBatch ? 32 * kStates * 4 : 0;
+      constexpr int kTurns = kWeightBytes + 2048 <= Tile<D>::kStageBytes ? 1 : 2;   // all rows at once, or half of them
+      static_assert(kWeightBytes + 2048 / kTurns <= Tile<D>::kStageBytes, "a wavefront's own staging rows");
+      uint8_t* rows_at = stage + kWeightBytes;
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(stage + q * 1024 + lane * 16);
-        const uint32_t row = (uint32_t)(s * kRowsPer + q * (kRowsPer / 2)) + (uint32_t)lane / (2 * kRowLanes);
+        if (kTurns == 1 ? q == 0 : lane / 32 == q) {
+#pragma unroll
+          for (int e = 0; e < 8; e += 4)
+            *reinterpret_cast<f32x4*>(rows_at + (kTurns == 1 ? lane : col) * 32 + 4 * e) = f32x4{o[e], o[e + 1], o[e + 2], o[e + 3]};
+        }
+        asm volatile("" ::: "memory");   // (a lane that stores nothing would keep what it has read before)
+        const u32x4 v = *reinterpret_cast<const u32x4*>(rows_at + (kTurns == 1 ? q * 1024 : 0) + lane * 16);
+        asm volatile("" ::: "memory");
+        const uint32_t row = (uint32_t)(rs * kRowsPer + q * (kRowsPer / 2)) + (uint32_t)lane / (2 * kRowLanes);
         __builtin_amdgcn_raw_buffer_store_b128(v, dst, 2 * row * row_bytes + 16u * ((uint32_t)lane % (2 * kRowLanes)), 0, kNt);
       }
     } else {
@@ -581,8 +569,61 @@ __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row
         pair.y = o[2 * e + 1];
         v[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, typename E::x2));
       }
-      __builtin_amdgcn_raw_buffer_store_b128(v, dst, lane_off + (uint32_t)(s * kRowsPer) * row_bytes, 0, kNt);
+      __builtin_amdgcn_raw_buffer_store_b128(v, dst, lane_off + (uint32_t)(rs * kRowsPer) * row_bytes, 0, kNt);
     }
+  };
+  float acc[kOneBatch ? 1 : kRowSteps][8];
+#pragma unroll
+  for (auto& row : acc)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) row[e] = 0.f;
+  while (i0 >= 0) {
+#pragma unroll
+    for (int j = 0; j < kStates; ++j) {
+      l[j] = i0 + j < n && m > -INFINITY ? __expf(l[j] - m) : 0.f;
+      den += l[j];
+    }
+    if constexpr (kOneBatch) finish_row();
+#pragma unroll
+    for (int j = 0; j < kStates; j += 4) *reinterpret_cast<f32x4*>(weights + col * kStates + j) = f32x4{l[j], l[j + 1], l[j + 2], l[j + 3]};
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+      const int rs = s / kParts;
+      float (&sum)[8] = acc[kOneBatch ? 0 : rs];
+      float f = 0.f;
+      if (kOneBatch && s % kParts == kParts - 1) f = __shfl(norm, rs * kRowsPer + lane / kRowLanes);
+      const float* ws = weights + (rs * kRowsPer + lane / kRowLanes) * kStates + s % kParts * kLoads;
+      f32x4 wv[kLoads / 4];
+#pragma unroll
+      for (int j = 0; j < kLoads / 4; ++j) wv[j] = *reinterpret_cast<const f32x4*>(ws + 4 * j);
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x2 v = E::widen(x[s % kDepth][j][e]);
+          sum[2 * e] = __builtin_fmaf(wv[j / 4][j % 4], v.x, sum[2 * e]);
+          sum[2 * e + 1] = __builtin_fmaf(wv[j / 4][j % 4], v.y, sum[2 * e + 1]);
+        }
+      if (!kOneBatch && s + kDepth == kSteps) {   // the next batch
+        i0 -= kStates;
+        open();
+        load_lse(i0);
+      }
+      if (!kOneBatch || s + kDepth < kSteps) load((s + kDepth) % kSteps);
+      __builtin_amdgcn_sched_barrier(0);   // the loads stay behind the step that frees their registers
+      if (kOneBatch && s % kParts == kParts - 1) {
+        store_rows(rs, f, sum);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (kOneBatch) return;
+  }
+  finish_row();
+  if constexpr (!kOneBatch) {
+#pragma unroll
+    for (int s = 0; s < kRowSteps; ++s) store_rows(s, __shfl(norm, s * kRowsPer + lane / kRowLanes), acc[s]);
   }
 }
 
@@ -1184,25 +1225,45 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
       const int64_t slot0 = item * ways;
       const float* lses = e.ws_lse + slot0 * kBQ + wave * 32 + col;
       const float* parts = e.ws_out + (slot0 * kWaves + wave) * (32 * D);
+      // A chain of waits: two parts are under way while one is added (behind the last one, empty descriptors: no memory is
+      // touched).  One after the other, 2 heads x 4000 queries, D = 128, 4 of 8 chunks took 80.8 us instead of 75.6 and 24 heads x
+      // 1000 76.8 instead of 70.7.
+      f32x4 x[2][D / 8];
+      float l[2];
+      auto load = [&](int p, int buf) __attribute__((always_inline)) {
+        const int at = min(p, ways - 1);
+        const Rsrc src = buffer_of(parts + (int64_t)at * (kBQ * D), p < ways ? slice_bytes : 0u);
+        l[buf] = load_device(lses + at * kBQ);
+#pragma unroll
+        for (int g = 0; g < D / 8; ++g)
+          x[buf][g] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, g * 1024 + lane * 16, 0, kDevice));
+      };
+      load(0, 0);
+      load(1, 1);
       float m = -INFINITY, den = 0.f;
-      for (int p = 0; p < ways; ++p) m = fmaxf(m, load_device(lses + p * kBQ));
+      for (int p = 0; p < ways; p += 8) {
+        float some[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) some[j] = load_device(lses + min(p + j, ways - 1) * kBQ);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m = fmaxf(m, some[j]);
+      }
 #pragma unroll
       for (int i = 0; i < D / 32; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.f;
-      for (int p = 0; p < ways; ++p) {
-        const Rsrc src = buffer_of(parts + (int64_t)p * (kBQ * D), slice_bytes);
-        f32x4 x[D / 8];
+      for (int p0 = 0; p0 < ways; p0 += 2) {
 #pragma unroll
-        for (int g = 0; g < D / 8; ++g)
-          x[g] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, g * 1024 + lane * 16, 0, kDevice));
-        const float l = load_device(lses + p * kBQ);
-        const float w = l == -INFINITY ? 0.f : __expf(l - m);   // (NaN stays NaN, and with it the row's sum)
-        den += w;
+        for (int j = 0; j < 2; ++j) {
+          const float w = p0 + j >= ways || l[j] == -INFINITY ? 0.f : __expf(l[j] - m);   // (NaN stays NaN, and with it the row's sum)
+          den += w;
 #pragma unroll
-        for (int g = 0; g < D / 8; ++g)
+          for (int g = 0; g < D / 8; ++g)
 #pragma unroll
-          for (int k = 0; k < 4; ++k) o_acc[g / 4][4 * (g % 4) + k] = __builtin_fmaf(w, x[g][k], o_acc[g / 4][4 * (g % 4) + k]);
+            for (int k = 0; k < 4; ++k) o_acc[g / 4][4 * (g % 4) + k] = __builtin_fmaf(w, x[j][g][k], o_acc[g / 4][4 * (g % 4) + k]);
+          load(p0 + j + 2, j);
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       inv = den > 0.f ? 1.f / den : 0.f;
       lse = den > 0.f ? m + __logf(den) : -INFINITY;
@@ -1347,7 +1408,11 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     if (first >= m.Sq || !arrive_last(m.arrive + kPartCounters + (int64_t)at * kWaves + slice, m.merge_jobs)) return;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int b = bh / m.H;
-    merge_rows<D, kHalf>(lds + Tile<D>::kLdsTiles + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * Tile<D>::kStageBytes, b, bh - b * m.H, first);
+    uint8_t* stage = lds + Tile<D>::kLdsTiles + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * Tile<D>::kStageBytes;
+    const int n = m.merge_n;
+    if (n <= 4) merge_rows<D, kHalf, 4, true>(stage, b, bh - b * m.H, first);
+    else if (n <= kMergeBatch) merge_rows<D, kHalf, kMergeBatch, true>(stage, b, bh - b * m.H, first);
+    else merge_rows<D, kHalf, D == 128 ? 8 : 4, false>(stage, b, bh - b * m.H, first);
   }
 }
 

@@ -75,6 +75,15 @@ def test_scheduled_launch_that_merges(hip, B, Sq, H, D, lens, computed, dtype, o
     assert not hip.attn_counters("cuda", q).any()
 
 
+
+@pytest.mark.parametrize("n", [1, 4, 5, 8, 9, 16, 17])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+def test_numbers_of_states_that_merge(hip, n, D, dtype, out):
+    """The edges of the merge's batches of states, on rows that end in the middle of a load instruction's."""
+    test_scheduled_launch_that_merges(hip, 1, 70, 3, D, (90,) * n, (n // 2,), dtype, out)
+
+
 @pytest.mark.parametrize("B,Sq,H,D,lens,jobs,cached", [
     (1, 65, 3, 64, (100, 100), [[0], [1]], 0), (1, 512, 4, 128, (512,) * 4, [[2], [0, 1, 3]], 3), (2, 333, 2, 64, (900, 1700, 64), [[0, 1, 2]], 1),
     (1, 288, 5, 128, (2300, 1), [[0], [1], [0, 1]], 14),
