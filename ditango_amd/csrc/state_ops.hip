@@ -856,9 +856,10 @@ static void launch_merge_d(const MergeArgs& a, bool tiled, int passes, unsigned 
   }
 }
 
-// The launches of merge_update_kernel: an fp32 state and a 16-bit one behind it, into fp32.
-static bool is_update(const MergeArgs& a) {
-  return a.n == 2 && a.dst_dtype == DT_FP32 && a.fp32_mask == 1u && (int64_t)a.B * a.Sq * a.H < (1ll << 31);
+// The launches of merge_update_kernel: an fp32 state and a 16-bit one behind it, into fp32.  A grid holds fewer than 2^32 lanes, and a
+// row takes D / 4 of them, twice what the lane groups of merge_states_kernel take at D = 128: states of 64 GiB and more go there.
+static bool is_update(const MergeArgs& a, int D) {
+  return a.n == 2 && a.dst_dtype == DT_FP32 && a.fp32_mask == 1u && (int64_t)a.B * a.Sq * a.H * (D / 4) <= (1ll << 32) - kUpdateThreads;
 }
 
 static int launch_update(const MergeArgs& a, int D, hipStream_t stream) {
@@ -895,7 +896,7 @@ int launch_merge(const MergeArgs& a, int D, hipStream_t stream) {
     set_error("head dim %d not built (64 and 128 are)", D);
     return DT_ERR_UNSUPPORTED;
   }
-  if (is_update(a)) return launch_update(a, D, stream);
+  if (is_update(a, D)) return launch_update(a, D, stream);
   const int R = 128 / D;   // rows per unit
   const int64_t units = ((int64_t)a.B * a.Sq * a.H + R - 1) / R;
   const bool tiled = unit_tiles_fit(a.H, D);

@@ -651,3 +651,24 @@ def test_running_state_and_a_block(hip, B, Sq, H, D, layouts):
             none = torch.isinf(ref_lse)
             assert (got[none] == -math.inf).all()
             assert torch.where(none, 0.0, got - ref_lse).abs().max() <= 4e-6
+
+
+@pytest.mark.parametrize("rows_less", [0, 8])
+def test_running_state_of_64_gib(hip, rows_less):
+    """The largest state that the update's own kernel has lanes for, and the first that goes to the general one, in place.
+    Constant values: both weights are 1/2 to the last bits, the result is 1.5."""
+    H, D, Sq = 1, 128, (1 << 27) - rows_less
+    need = Sq * (6 * D + 8)
+    if torch.cuda.mem_get_info()[0] < need + (4 << 30):
+        torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < need + (4 << 30):
+        pytest.skip("needs 104 GiB of free GPU memory")
+    run = torch.full((1, Sq, H, D), 1.0, device="cuda")
+    blk = torch.full((1, Sq, H, D), 2.0, dtype=torch.bfloat16, device="cuda")
+    run_lse = torch.zeros(1, Sq, H, 1, device="cuda")
+    blk_lse = torch.zeros(1, H, Sq, device="cuda")
+    hip.merge_states([run, blk], [run_lse, blk_lse], dst_out=run, dst_lse=run_lse)
+    for got, want in ((run, 1.5), (run_lse, 0.6931472)):
+        assert abs(got.amin().item() - want) <= 1e-6 and abs(got.amax().item() - want) <= 1e-6
+    del run, blk
+    torch.cuda.empty_cache()
