@@ -450,6 +450,12 @@ __global__ __launch_bounds__(kThreads) void merge_states_kernel(const MergeArgs 
 // D = 64 48.2 -> 38.0, 2222 x 48, D = 64 17.5 -> 13.1.  Workgroups of 512 and 1024 lanes 68.6 and 68.8.  One block
 // state alone (the first of a loop) is 24 bytes an element and bound by the instructions of so many lanes: it stays there (43.4;
 // 57 here).
+struct RowIndex {         // row ((b * Sq) + s) * H + h of B * Sq * H < 2^31 -> its place in the [B,H,Sq] layout
+  int32_t Sq, H;
+  uint32_t rows;          // B * Sq * H
+  uint32_t mul_h, mul_s;  // n / H and n / Sq for n < 2^31 (see quotient)
+  int32_t shift_h, shift_s;
+};
 struct UpdateArgs {
   const float* run;
   const float* run_lse;
@@ -457,11 +463,8 @@ struct UpdateArgs {
   const float* blk_lse;
   float* dst;
   float* dst_lse;         // may be null
-  int32_t Sq, H;
-  uint32_t rows;          // B * Sq * H
+  RowIndex at;
   int32_t run_bsh, blk_bsh, dst_bsh;
-  uint32_t mul_h, mul_s;  // n / H and n / Sq for n < 2^31 (see quotient)
-  int32_t shift_h, shift_s;
 };
 constexpr int kUpdateThreads = 256;
 constexpr int kUpdateGroup = 64;   // workgroups that follow each other on one XCD (1: 3 % slower, 8: the same)
@@ -477,24 +480,41 @@ static void set_quotient(int32_t d, uint32_t& mul, int32_t& shift) {
   mul = L == 0 ? 0u : (uint32_t)(((1ull << (31 + L)) + (uint64_t)d - 1) / (uint64_t)d);
   shift = L - 1;
 }
+__device__ __forceinline__ uint32_t bhs_of(const RowIndex& at, uint32_t row) {
+  const uint32_t bs = quotient(row, at.mul_h, at.shift_h), h = row - bs * (uint32_t)at.H;
+  const uint32_t b = quotient(bs, at.mul_s, at.shift_s), q = bs - b * (uint32_t)at.Sq;
+  return (b * (uint32_t)at.H + h) * (uint32_t)at.Sq + q;
+}
+static RowIndex row_index(int B, int Sq, int H) {
+  RowIndex at{};
+  at.Sq = Sq;
+  at.H = H;
+  at.rows = (uint32_t)((int64_t)B * Sq * H);
+  set_quotient(H, at.mul_h, at.shift_h);
+  set_quotient(Sq, at.mul_s, at.shift_s);
+  return at;
+}
+// A grid holds fewer than 2^32 lanes, and these kernels take D / 4 of them a row.
+static bool lanes_fit(int B, int Sq, int H, int D) { return (int64_t)B * Sq * H * (D / 4) <= (1ll << 32) - kUpdateThreads; }
+static dim3 lane_grid(const RowIndex& at, int D) {
+  return dim3((unsigned)(((int64_t)at.rows * (D / 4) + kUpdateThreads - 1) / kUpdateThreads));
+}
 
-template <int D, bool kF16>
-__global__ __launch_bounds__(kUpdateThreads) void merge_update_kernel(const UpdateArgs a) {
-  // The lse of consecutive queries share a line of the [B,H,Sq] layout; workgroups go to the 8 XCDs in turn.  So that a line
-  // is read into one L2 only, 64 workgroups that follow each other in memory are 64 of one XCD.
+// The first element of this lane.  The lse of consecutive queries share a line of the [B,H,Sq] layout; workgroups go to the 8 XCDs
+// in turn.  So that a line is read into one L2 only, 64 workgroups that follow each other in memory are 64 of one XCD.
+__device__ __forceinline__ int64_t lane_elem() {
   uint32_t wg = blockIdx.x;
   constexpr uint32_t kSpan = 8 * kUpdateGroup;
   if ((wg / kSpan + 1) * kSpan <= gridDim.x) wg = wg / kSpan * kSpan + (wg & 7u) * kUpdateGroup + (wg % kSpan >> 3);
-  const int64_t elem = ((int64_t)wg * kUpdateThreads + threadIdx.x) * 4;
-  const int64_t row64 = elem / D;
-  if (row64 >= a.rows) return;
-  const uint32_t row = (uint32_t)row64;   // ((b * Sq) + s) * H + h
-  uint32_t bhs = row;
-  if (!a.blk_bsh || !a.run_bsh || !a.dst_bsh) {
-    const uint32_t bs = quotient(row, a.mul_h, a.shift_h), h = row - bs * (uint32_t)a.H;
-    const uint32_t b = quotient(bs, a.mul_s, a.shift_s), q = bs - b * (uint32_t)a.Sq;
-    bhs = (b * (uint32_t)a.H + h) * (uint32_t)a.Sq + q;
-  }
+  return ((int64_t)wg * kUpdateThreads + threadIdx.x) * 4;
+}
+
+template <int D, bool kF16>
+__global__ __launch_bounds__(kUpdateThreads) void merge_update_kernel(const UpdateArgs a) {
+  const int64_t elem = lane_elem(), row64 = elem / D;
+  if (row64 >= a.at.rows) return;
+  const uint32_t row = (uint32_t)row64;
+  const uint32_t bhs = !a.blk_bsh || !a.run_bsh || !a.dst_bsh ? bhs_of(a.at, row) : row;
   const f32x4 x0 = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(a.run + elem));
   const float l0 = a.run_lse[a.run_bsh ? row : bhs];
   const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(a.blk + elem));
@@ -524,6 +544,43 @@ struct CopyArgs {
   int32_t B, Sq, H;
   int32_t src_dtype, src_bsh, dst_dtype, dst_bsh;   // DT_BF16 / DT_FP32 / DT_FP16
 };
+
+// An fp32 state rounded to a 16-bit one (a cache store) or a 16-bit one widened (a load): a lane moves 4 elements, as in
+// merge_update_kernel above, and the first lane of a row its lse.  A short launch is bound by its start and its last workgroups'
+// waits, of which this has two, one behind the other.  us per launch, the kernels below -> this, for stores at D = 64 2222 x 48
+// heads 10.3 -> 9.7, 6001 x 7 5.3 -> 4.9, 14 882 x 24 26.3 -> 25.5, 14 882 x 48 48.3 -> 47.6; for loads of less than 2^16 rows 2001
+// x 30 heads, D = 64 7.7 -> 6.1, D = 128 10.4 -> 10.1, 6001 x 7, D = 64 5.4 -> 4.7, 300 x 5, D = 128 2.7 -> 2.4.
+template <int D, int SRC, int DST>
+__global__ __launch_bounds__(kUpdateThreads) void state_convert_kernel(const CopyArgs a, const RowIndex at) {
+  static_assert((SRC == DT_FP32) != (DST == DT_FP32), "fp32 on one side");
+  const int64_t elem = lane_elem(), row64 = elem / D;
+  if (row64 >= at.rows) return;
+  const bool my_lse = a.dst_lse != nullptr && a.src_lse != nullptr && elem % D == 0;
+  uint32_t row = 0, bhs = 0;
+  float l = 0.f;
+  u32x4 w;
+  u32x2 n;
+  if (SRC == DT_FP32) w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const float*>(a.src_out) + elem));
+  else n = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(a.src_out) + elem));
+  if (my_lse) {
+    row = (uint32_t)row64;
+    bhs = !a.src_bsh || !a.dst_bsh ? bhs_of(at, row) : row;
+    l = a.src_lse[a.src_bsh ? row : bhs];
+  }
+  if (SRC == DT_FP32) {
+    n.x = pack16x2(__uint_as_float(w[0]), __uint_as_float(w[1]), DST == DT_FP16);
+    n.y = pack16x2(__uint_as_float(w[2]), __uint_as_float(w[3]), DST == DT_FP16);
+    __builtin_nontemporal_store(n, reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.dst_out) + elem));
+  } else {
+    float x[4];
+    widen16x2(n.x, SRC == DT_FP16, x[0], x[1]);
+    widen16x2(n.y, SRC == DT_FP16, x[2], x[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = __float_as_uint(x[i]);
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<float*>(a.dst_out) + elem));
+  }
+  if (my_lse) a.dst_lse[a.dst_bsh ? row : bhs] = l;
+}
 
 
 constexpr int kCopyRows = 1;  // rows per lane group (2 and 4 measured: -6 % and -12 %)
@@ -856,10 +913,10 @@ static void launch_merge_d(const MergeArgs& a, bool tiled, int passes, unsigned 
   }
 }
 
-// The launches of merge_update_kernel: an fp32 state and a 16-bit one behind it, into fp32.  A grid holds fewer than 2^32 lanes, and a
-// row takes D / 4 of them, twice what the lane groups of merge_states_kernel take at D = 128: states of 64 GiB and more go there.
+// The launches of merge_update_kernel: an fp32 state and a 16-bit one behind it, into fp32.  (The lane groups of
+// merge_states_kernel are half as many lanes: states of 64 GiB and more go there.)
 static bool is_update(const MergeArgs& a, int D) {
-  return a.n == 2 && a.dst_dtype == DT_FP32 && a.fp32_mask == 1u && (int64_t)a.B * a.Sq * a.H * (D / 4) <= (1ll << 32) - kUpdateThreads;
+  return a.n == 2 && a.dst_dtype == DT_FP32 && a.fp32_mask == 1u && lanes_fit(a.B, a.Sq, a.H, D);
 }
 
 static int launch_update(const MergeArgs& a, int D, hipStream_t stream) {
@@ -870,16 +927,11 @@ static int launch_update(const MergeArgs& a, int D, hipStream_t stream) {
   u.blk_lse = a.lse[1];
   u.dst = static_cast<float*>(a.dst_out);
   u.dst_lse = a.dst_lse;
-  u.Sq = a.Sq;
-  u.H = a.H;
-  u.rows = (uint32_t)((int64_t)a.B * a.Sq * a.H);
+  u.at = row_index(a.B, a.Sq, a.H);
   u.run_bsh = (int32_t)(a.bsh_mask & 1);
   u.blk_bsh = (int32_t)((a.bsh_mask >> 1) & 1);
   u.dst_bsh = a.dst_bsh;
-  set_quotient(a.H, u.mul_h, u.shift_h);
-  set_quotient(a.Sq, u.mul_s, u.shift_s);
-  const int64_t lanes = (int64_t)u.rows * (D / 4);
-  const dim3 grid((unsigned)((lanes + kUpdateThreads - 1) / kUpdateThreads)), block(kUpdateThreads);
+  const dim3 grid = lane_grid(u.at, D), block(kUpdateThreads);
   const bool f16 = (a.f16_mask >> 1) & 1;
   if (D == 128) {
     if (f16) hipLaunchKernelGGL((merge_update_kernel<128, true>), grid, block, 0, stream, u);
@@ -943,6 +995,26 @@ struct LaunchCopyRows64 {
   }
 };
 
+// The launches of state_convert_kernel.  Stores: D = 64 (D = 128, row-mapped kernel -> this: 1000 x 40 heads 7.7 -> 7.6 us, but 2001 x
+// 30 10.1 -> 10.4 and 14 882 x 24 43.5 -> 46.8).  Loads: below 2^16 rows (2222 x 48, D = 64, state_widen_kernel -> this: 9.5 -> 9.8,
+// 6851 x 48, D = 128 41.5 -> 42.1).
+static bool is_convert(const CopyArgs& a, int D) {
+  if ((a.src_dtype == DT_FP32) == (a.dst_dtype == DT_FP32) || !lanes_fit(a.B, a.Sq, a.H, D)) return false;
+  return a.src_dtype == DT_FP32 ? D == 64 : (int64_t)a.B * a.Sq * a.H < (1 << 16);
+}
+
+static int launch_convert(const CopyArgs& a, int D, hipStream_t stream) {
+  const RowIndex at = row_index(a.B, a.Sq, a.H);
+  const dim3 grid = lane_grid(at, D), block(kUpdateThreads);
+  if (a.dst_dtype == DT_BF16) hipLaunchKernelGGL((state_convert_kernel<64, DT_FP32, DT_BF16>), grid, block, 0, stream, a, at);
+  else if (a.dst_dtype == DT_FP16) hipLaunchKernelGGL((state_convert_kernel<64, DT_FP32, DT_FP16>), grid, block, 0, stream, a, at);
+  else if (D == 64 && a.src_dtype == DT_BF16) hipLaunchKernelGGL((state_convert_kernel<64, DT_BF16, DT_FP32>), grid, block, 0, stream, a, at);
+  else if (D == 64) hipLaunchKernelGGL((state_convert_kernel<64, DT_FP16, DT_FP32>), grid, block, 0, stream, a, at);
+  else if (a.src_dtype == DT_BF16) hipLaunchKernelGGL((state_convert_kernel<128, DT_BF16, DT_FP32>), grid, block, 0, stream, a, at);
+  else hipLaunchKernelGGL((state_convert_kernel<128, DT_FP16, DT_FP32>), grid, block, 0, stream, a, at);
+  return hip_fail(hipGetLastError(), "state_convert launch");
+}
+
 int launch_copy(const CopyArgs& a, int D, hipStream_t stream) {
   const bool with_lse = a.dst_lse != nullptr && a.src_lse != nullptr;
   if (a.src_dtype == a.dst_dtype && (!with_lse || a.src_bsh == a.dst_bsh) && (D == 64 || D == 128)) {
@@ -967,6 +1039,7 @@ int launch_copy(const CopyArgs& a, int D, hipStream_t stream) {
     set_error("head dim %d not built (64 and 128 are)", D);
     return DT_ERR_UNSUPPORTED;
   }
+  if (is_convert(a, D)) return launch_convert(a, D, stream);
   if (a.src_dtype != DT_FP32 && a.dst_dtype == DT_FP32) {
     const int64_t rows = (int64_t)a.B * a.Sq * a.H;
     const int64_t groups = rows * D / 4;
@@ -988,8 +1061,9 @@ int launch_copy(const CopyArgs& a, int D, hipStream_t stream) {
     return hip_fail(hipGetLastError(), "state_widen launch");
   }
   if (D == 64 && unit_tiles_fit(a.H, D)) {
-    // two neighbouring rows per lane group, query x head tiles (fp32 -> slot at 714 336 rows: 5.70 against 5.44 TB/s
-    // for the row mapping; at D = 128 the row mapping with its contiguous lse runs is the faster one, 6.3 against 6.0)
+    // one 16-bit type into another, or another lse layout: two neighbouring rows per lane group, query x head tiles (fp32 -> slot
+    // at 714 336 rows, which is state_convert_kernel's now: 5.70 against 5.44 TB/s for the row mapping; at D = 128 the row mapping
+    // with its contiguous lse runs is the faster one, 6.3 against 6.0)
     const int64_t wgs = unit_grid(a.B, a.Sq, a.H, D, true, 1);
     if (wgs <= 0) return DT_OK;
     if (wgs > 0x7fffffffLL) {

@@ -672,3 +672,22 @@ def test_running_state_of_64_gib(hip, rows_less):
         assert abs(got.amin().item() - want) <= 1e-6 and abs(got.amax().item() - want) <= 1e-6
     del run, blk
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("B,Sq,H,D", [(1, 1, 1, 64), (1, 1, 1, 128), (3, 7, 1, 64), (1, 1, 37, 128), (2, 5, 3, 128), (1, 300, 7, 64),
+                                      (1, 2185, 30, 128), (1, 4369, 15, 64), (2, 2048, 16, 64), (1, 4096, 16, 128)])
+@pytest.mark.parametrize("bsh", [True, False])
+def test_states_convert_exactly(hip, B, Sq, H, D, bsh):
+    """fp32 states rounded and 16-bit ones widened, either lse layout outside the cache: one row, one head, one query, odd counts, the last sizes of
+    short loads (65 535 rows) and the first of longer ones.  One rounding to nearest, and exact widening: bits as torch's."""
+    gen = torch.Generator().manual_seed(B + Sq * 3 + H * 5 + D)
+    store = lambda l, bsh: (l.transpose(1, 2).contiguous().unsqueeze(-1) if bsh else l).cuda()
+    wide, lse = torch.randn(B, Sq, H, D, generator=gen), 4 * torch.randn(B, H, Sq, generator=gen)
+    lse[:, :, ::3] = -math.inf
+    wide.view(-1)[::53] = math.inf
+    for dtype in (torch.bfloat16, torch.float16):
+        slot, slot_lse = torch.full((B, Sq, H, D), math.nan, dtype=dtype, device="cuda"), torch.zeros(B, H, Sq, device="cuda")
+        hip.cache_store(wide.cuda(), store(lse, bsh), slot, slot_lse)
+        assert torch.equal(slot.cpu(), wide.to(dtype)) and torch.equal(slot_lse.cpu(), lse)
+        back, back_lse = hip.cache_load(slot, slot_lse, torch.float32, dst_lse_bsh=bsh)
+        assert torch.equal(back.cpu(), wide.to(dtype).float()) and torch.equal(back_lse.cpu(), store(lse, bsh).cpu())
