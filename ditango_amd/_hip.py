@@ -286,16 +286,16 @@ KEPT_COUNTERS = 1 << 18    # words a kept set holds: launches of up to 32 512 qu
 
 def attn_counters(device, q: torch.Tensor) -> Optional[torch.Tensor]:
     """The arrival counters of merging launches on ``q [B,Sq,H,D]`` made on the current stream of ``device``: int32, zero, and
-    left at zero by every launch.  One set per stream, kept and shared like the workspace; launches under capture get a set
-    of the graph's own pool, cleared by the graph.  ``None`` where a launch needs more than a kept set holds: it does not
-    merge then."""
+    left at zero by every launch.  One set per stream, kept and shared like the workspace.  ``None``, and the launch does not
+    merge, where it needs more than a kept set holds, and under capture: a graph's set would have to be cleared by every replay, a
+    launch more than the merge saves."""
     B, Sq, H, _ = q.shape
     need = int(load_library().dt_attn_merge_counters(B, Sq, H))
     if need > KEPT_COUNTERS:
         return None
-    dev = device if isinstance(device, torch.device) else torch.device(device)
     if torch.cuda.is_current_stream_capturing():
-        return torch.empty(need, dtype=torch.int32, device=dev).zero_()
+        return None
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (dev.type, index, _raw_stream(index))
     c = _counters.pop(key, None)

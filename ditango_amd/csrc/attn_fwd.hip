@@ -1812,36 +1812,9 @@ static std::mutex& workspace_lock(const void* workspace) {
   return locks[(reinterpret_cast<uintptr_t>(workspace) >> 4) * 0x9e3779b97f4a7c15ull >> (64 - kBits)];
 }
 
-int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
-  if (n_jobs <= 0 || a_in.total <= 0) return DT_OK;
-  if (D != 128 && D != 64) {
-    set_error("head dim %d not built (64 and 128 are)", D);
-    return DT_ERR_UNSUPPORTED;
-  }
-  if (a_in.elem_f16 && a_in.q_prescaled) {
-    set_error("fp16 tensors and a prescaled q do not combine (the prescaled softmax keeps probabilities beyond fp16's range)");
-    return DT_ERR_UNSUPPORTED;
-  }
-  AttnArgs a = a_in;
-  a.job_planes = n_jobs;
-  a.tail_start = INT32_MAX;
-  a.tail_items = 0;
-  a.part_ways = 0;
-  a.row_split = 0;
-  constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
+// The launch as it is planned (and the fold kernel behind it).
+static int launch_planned(AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
   const int64_t slot_bytes = partial_state_bytes(D);
-  if (n_jobs <= kMaxLaunchJobs) {
-    JobSize size[kMaxLaunchJobs];
-    job_sizes(a, n_jobs, size);
-    const int cus = cu_count();
-    const bool known = cus >= 64 && cus % kXcds == 0;
-    const TailPlan plan = plan_launch(a, D, n_jobs, size, known ? cus / kXcds : 0,
-                                      known && workspace ? std::min(workspace_bytes, kWorkspaceBytes) / slot_bytes : -1);
-    a.tail_items = plan.items;
-    a.part_ways = plan.ways;
-    a.row_split = plan.rows ? 1 : 0;
-    if (plan.items > 0) a.tail_start = n_jobs * a.per_xcd - plan.items;
-  }
   const unsigned planes_x = (unsigned)a.per_xcd * kXcds;
   if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);
   const int64_t slots = (int64_t)a.tail_items * kXcds * a.part_ways;
@@ -1878,6 +1851,80 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
     else hipLaunchKernelGGL((attn_tail_fold_kernel<64, false>), fold_grid, fold_block, 0, stream, a);
   }
   return hip_fail(hipGetLastError(), "attn tail fold launch");
+}
+
+// Whether a launch that merges does so itself, or the fold and merge kernels behind it; `tiles` is the key tiles of the
+// longest item.  In 8 rounds and more the merge of one round runs beside the keys of another: 24 heads x 119 056 queries, 3 of 32
+// chunks 17.2 -> 15.9 ms, 24 x 14 882, 4 of 8 8348 -> 8306 us.  In shorter ones it is one wavefront's chain of waits per 32 rows, against
+// kernels that spread over the chip, and a launch less for the host (us per call with the GPU kept busy, kernels behind -> own):
+//   * items in three parts and more are folded one part after the other: 4 heads x 1244 queries, two chunks, D = 128 27 -> 34,
+//     16 x 2075, two states 92 -> 99, 16 x 2177, D = 64 59 -> 63; two parts 16 x 1331, D = 128 46.4 -> 45.6, 4 x 3026, D = 64 39.5 -> 37.8;
+//   * D = 64 otherwise gains: 30 x 630, 4 states 18.6 -> 16.5, 30 x 1513 53.4 -> 51.3, 48 x 143 13.2 -> 12.9 (of 60 launches the
+//     worst 38.7 -> 39.6, 40 x 1010);
+//   * D = 128 does not: 40 x 274, 4 states 20 -> 24, 24 x 418 20 -> 23, 40 x 959 34.6 -> 35.3, 48 x 1452 87.6 -> 89.7.  Only where an item is
+//     over before the host has the next call ready (4 key tiles) does the launch less count for more: 24 x 200 22.8 -> 19.9 in a loop of
+//     calls, 15 -> 16.5 with the GPU kept busy.
+static bool merges_in_launch(const AttnArgs& a, int D, int n_jobs, int tiles, int cus, const TailPlan& plan) {
+  if (cus > 0 && (int64_t)n_jobs * a.per_xcd >= 8 * cus) return true;
+  if (plan.items > 0 && !plan.rows && plan.ways > 2) return false;
+  return D == 64 || tiles <= 4;
+}
+
+// The merge of such a launch, by the merge kernel.
+static int merge_behind(const AttnArgs& a, int D, hipStream_t stream) {
+  const AttnState* states = a.dev_ids ? a.arena : a.state;
+  const void* outs[DT_MAX_CHUNKS];
+  const float* lses[DT_MAX_CHUNKS];
+  int32_t dtypes[DT_MAX_CHUNKS];
+  for (int i = 0; i < a.merge_n; ++i) {
+    outs[i] = states[i].out;
+    lses[i] = states[i].lse;
+    dtypes[i] = a.elem_f16 ? DT_FP16 : DT_BF16;
+  }
+  return dt_merge_states(a.merge_n, outs, lses, dtypes, nullptr, a.merge_out, a.merge_dtype, a.merge_lse, DT_LSE_BSH, a.B, a.Sq, a.H,
+                         D, stream);
+}
+static_assert(DT_MAX_MERGE_LIST <= DT_MAX_CHUNKS && DT_MAX_CHUNKS <= DT_MAX_MERGE, "any list of states is one merge launch");
+
+int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
+  if (n_jobs <= 0 || a_in.total <= 0) return DT_OK;
+  if (D != 128 && D != 64) {
+    set_error("head dim %d not built (64 and 128 are)", D);
+    return DT_ERR_UNSUPPORTED;
+  }
+  if (a_in.elem_f16 && a_in.q_prescaled) {
+    set_error("fp16 tensors and a prescaled q do not combine (the prescaled softmax keeps probabilities beyond fp16's range)");
+    return DT_ERR_UNSUPPORTED;
+  }
+  AttnArgs a = a_in;
+  a.job_planes = n_jobs;
+  a.tail_start = INT32_MAX;
+  a.tail_items = 0;
+  a.part_ways = 0;
+  a.row_split = 0;
+  constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
+  bool merge_after = false;
+  if (n_jobs <= kMaxLaunchJobs) {
+    JobSize size[kMaxLaunchJobs];
+    job_sizes(a, n_jobs, size);
+    const int cus = cu_count();
+    const bool known = cus >= 64 && cus % kXcds == 0;
+    const TailPlan plan = plan_launch(a, D, n_jobs, size, known ? cus / kXcds : 0,
+                                      known && workspace ? std::min(workspace_bytes, kWorkspaceBytes) / partial_state_bytes(D) : -1);
+    a.tail_items = plan.items;
+    a.part_ways = plan.ways;
+    a.row_split = plan.rows ? 1 : 0;
+    if (plan.items > 0) a.tail_start = n_jobs * a.per_xcd - plan.items;
+    if (a.arrive) {
+      int longest = 0;
+      for (int j = 0; j < n_jobs; ++j) longest = std::max(longest, size[j].tiles);
+      merge_after = !merges_in_launch(a, D, n_jobs, longest, known ? cus / kXcds : 0, plan);
+    }
+  }
+  if (!merge_after) return launch_planned(a, D, n_jobs, stream, workspace, workspace_bytes);
+  a.arrive = nullptr;
+  if (int rc = launch_planned(a, D, n_jobs, stream, workspace, workspace_bytes)) return rc;
+  return merge_behind(a, D, stream);
 }
 
 }  // namespace dt

@@ -353,7 +353,8 @@ int dt_attn_seg_jobs_noalloc_fwd(const void* q, int32_t B, int32_t Sq, int32_t H
                                  float softmax_scale, int32_t flags, void* stream);
 
 /*
- * An attention launch that also merges: dt_attn_jobs_fwd / dt_attn_sched_fwd followed by dt_merge_states, in one kernel.
+ * An attention launch that also merges: dt_attn_jobs_fwd / dt_attn_sched_fwd followed by dt_merge_states, in one kernel where
+ * that is the faster form for the sizes of the launch, else in kernels one behind the other.
  * Whoever completes the last of the launch's states of 32 query rows merges the states there are of these rows, while other
  * workgroups still compute: the launch sequence of one layer call (core/attention.py:110-216) without the pass
  * over the states behind it.  The parts of a split tail (dt_attn_seg_jobs_ws_fwd) are folded in the same way.

@@ -40,6 +40,7 @@ SHAPES = [
     (1, 1, 3, 64, (40, 0, 64), (0, 2)), (1, 31, 2, 128, (64, 65, 1), (0, 1, 2)), (2, 33, 3, 64, (200, 130), (1,)),
     (1, 127, 4, 128, (512, 512, 512), (0, 2)), (1, 129, 4, 64, (512, 512, 512), (0, 2)), (1, 512, 4, 64, (512,) * 4, (0, 3)),
     (1, 255, 2, 128, (1500, 700), (0, 1)), (2, 257, 3, 64, (2000, 1999, 2000), (0, 1)), (1, 300, 2, 64, (4000, 4000), (0,)),
+    (2, 100, 516, 64, (2560, 2500), (0, 1)), (2, 100, 516, 128, (1700, 1600), (1, 0)),   # long enough to merge and fold items of several parts
     (1, 700, 5, 128, (1100,) * 11, (0, 4, 10)), (1, 1861, 6, 64, (1861,) * 3 + (1860,) * 2, (0, 3)), (1, 96, 1, 128, (96,) * 40, (7,)),
 ]
 
