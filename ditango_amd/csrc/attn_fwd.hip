@@ -462,8 +462,9 @@ __device__ __forceinline__ bool arrive_last(uint32_t* counter, int expected) {
 // In small ones a chain of waits at the end of the launch: one wavefront reads 32 rows of all states.  Up to 8 states
 // (kOneBatch) every weight is known before the first row, so rows are finished one after the other, without accumulators for
 // all of them, and the registers hold loads instead: 128 at D = 128 (4 steps of 8 states or all 8 steps of 4), 64 at D = 64.
-// us per call, two steps in flight -> this: 24 heads x 200 queries, D = 128, 1 of 2 chunks 22.8 -> 19.9, 4 of 8 27.1 -> 26.7; 40
-// heads x 2222, D = 128, 2 of 4 221 -> 217; 12 heads x 700, D = 64, 1 of 2 17.4 -> 16.9.  More states keep 32 rows of sums in
+// us per call, two steps in flight -> this: 24 heads x 200 queries, D = 128, 1 of 2 chunks 22.8 -> 19.9, 4 of 8 27.1 -> 26.7;
+// 12 heads x 700, D = 64, 1 of 2 17.4 -> 16.9 (and 40 x 2222, D = 128, 2 of 4 221 -> 217, which merges_in_launch leaves to the merge
+// kernel).  More states keep 32 rows of sums in
 // registers and two steps in flight (three make no difference to 29 states of 743 MB; four at D = 64 cost 24 heads x 200
 // queries, 16 states 1.5 us).
 template <int D, bool kHalf, int kStates, bool kOneBatch>
@@ -1227,7 +1228,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
       const float* parts = e.ws_out + (slot0 * kWaves + wave) * (32 * D);
       // A chain of waits: two parts are under way while one is added (behind the last one, empty descriptors: no memory is
       // touched).  One after the other, 2 heads x 4000 queries, D = 128, 4 of 8 chunks took 80.8 us instead of 75.6 and 24 heads x
-      // 1000 76.8 instead of 70.7.
+      // 1000 76.8 instead of 70.7; such short launches of many parts are the fold kernel's again (merges_in_launch).
       f32x4 x[2][D / 8];
       float l[2];
       auto load = [&](int p, int buf) __attribute__((always_inline)) {
