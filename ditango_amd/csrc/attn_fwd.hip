@@ -1860,6 +1860,8 @@ static int launch_planned(AttnArgs& a, int D, int n_jobs, hipStream_t stream, vo
 // kernels that spread over the chip, and a launch less for the host (us per call with the GPU kept busy, kernels behind -> own):
 //   * items in three parts and more are folded one part after the other: 4 heads x 1244 queries, two chunks, D = 128 27 -> 34,
 //     16 x 2075, two states 92 -> 99, 16 x 2177, D = 64 59 -> 63; two parts 16 x 1331, D = 128 46.4 -> 45.6, 4 x 3026, D = 64 39.5 -> 37.8;
+//   * 8 states in place of 2 are four times the loads of that chain: D = 64 24 x 269 17.0 -> 21.7, 24 x 1423 38.7 -> 40.7, 48 x 160 15.2
+//     -> 17.6, D = 128 20 x 200 19 -> 25; 4 are the most that gain at D = 64;
 //   * D = 64 otherwise gains: 30 x 630, 4 states 18.6 -> 16.5, 30 x 1513 53.4 -> 51.3, 48 x 143 13.2 -> 12.9 (of 60 launches the
 //     worst 38.7 -> 39.6, 40 x 1010);
 //   * D = 128 does not: 40 x 274, 4 states 20 -> 24, 24 x 418 20 -> 23, 40 x 959 34.6 -> 35.3, 48 x 1452 87.6 -> 89.7.  Only where an item is
@@ -1867,7 +1869,7 @@ static int launch_planned(AttnArgs& a, int D, int n_jobs, hipStream_t stream, vo
 //     calls, 15 -> 16.5 with the GPU kept busy.
 static bool merges_in_launch(const AttnArgs& a, int D, int n_jobs, int tiles, int cus, const TailPlan& plan) {
   if (cus > 0 && (int64_t)n_jobs * a.per_xcd >= 8 * cus) return true;
-  if (plan.items > 0 && !plan.rows && plan.ways > 2) return false;
+  if (a.merge_n > 4 || (plan.items > 0 && !plan.rows && plan.ways > 2)) return false;
   return D == 64 || tiles <= 4;
 }
 

@@ -81,8 +81,9 @@ def test_scheduled_launch_that_merges(hip, B, Sq, H, D, lens, computed, dtype, o
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 def test_numbers_of_states_that_merge(hip, n, D, dtype, out):
-    """The edges of the merge's batches of states, on rows that end in the middle of a load instruction's."""
-    test_scheduled_launch_that_merges(hip, 1, 70, 3, D, (90,) * n, (n // 2,), dtype, out)
+    """The edges of the merge's batches of states, on rows that end in the middle of a load instruction's (with heads enough that
+    a launch of more than 4 states merges)."""
+    test_scheduled_launch_that_merges(hip, 1, 70, 520, D, (90,) * n, (n // 2,), dtype, out)
 
 
 @pytest.mark.parametrize("B,Sq,H,D,lens,jobs,cached", [
