@@ -1804,9 +1804,9 @@ static TailPlan plan_launch(AttnArgs& a, int D, int n_jobs, JobSize* size, int c
   return best;
 }
 
-// Held while a split launch and its fold kernel go into the queue: two threads may launch on one stream, with the workspace
-// that belongs to it, and nothing of the other's may come between the parts and their fold.  (One of a few locks, chosen by the
-// workspace: a thread that waits for room in its stream's queue holds up few others.)
+// Held while a launch that writes partial states, and the fold kernel where there is one, go into the queue: two threads may
+// launch on one stream, with the workspace that belongs to it, and no parts of the other's may come between the parts and their
+// fold.  (One of a few locks, chosen by the workspace: a thread that waits for room in its stream's queue holds up few others.)
 static std::mutex& workspace_lock(const void* workspace) {
   constexpr int kBits = 6;
   static std::mutex locks[1 << kBits];
@@ -1840,9 +1840,10 @@ static int launch_planned(AttnArgs& a, int D, int n_jobs, hipStream_t stream, vo
   // parts per XCD, spread over planes of per_xcd entries
   const int part_planes = (a.tail_items * a.part_ways + a.per_xcd - 1) / a.per_xcd;
   const dim3 grid(planes_x, (unsigned)(a.job_planes + part_planes), 1);
-  if (a.row_split || a.arrive) return launch_dim(a, D, grid, stream);   // (nothing to fold, or folded by the launch itself)
+  if (a.row_split) return launch_dim(a, D, grid, stream);   // (no partial states)
   std::lock_guard<std::mutex> pair(workspace_lock(workspace));
   if (int rc = launch_dim(a, D, grid, stream)) return rc;
+  if (a.arrive) return DT_OK;   // folded by the launch itself
   const dim3 fold_grid((unsigned)a.tail_items * kXcds * kWaves * (D / 64)), fold_block(kFoldThreads);
   if (D == 128) {
     if (a.elem_f16) hipLaunchKernelGGL((attn_tail_fold_kernel<128, true>), fold_grid, fold_block, 0, stream, a);

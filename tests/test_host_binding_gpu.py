@@ -132,6 +132,39 @@ def test_threads_that_launch_on_one_stream_share_its_workspace(hip):
         assert all(torch.equal(o, want[i][0]) and torch.equal(l, want[i][1]) for o, l in got[i])
 
 
+def test_a_launch_that_folds_its_own_parts_shares_the_workspace_too(hip):
+    """As above, the second thread's launches merging their states and folding their parts themselves (tests/test_launch_order.py
+    has the order of the launches)."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda", dtype=torch.bfloat16)
+    q, k, v = rnd(1, 900, 2, 128), rnd(1, 2600, 2, 128), rnd(1, 2600, 2, 128)
+    q2, ks, vs = rnd(2, 100, 516, 64), [rnd(2, n, 516, 64) for n in (2560, 2500)], [rnd(2, n, 516, 64) for n in (2560, 2500)]
+    runs = [lambda: hip.attn_states(q, [k], [v], [[0]], 32, hip.attn_workspace("cuda"))[0],
+            lambda: hip.attn_states_merge(q2, ks, vs, [[0], [1]], 32, [], [], [0, 1], torch.float32, hip.attn_workspace("cuda"))[1:]]
+    want = [run() for run in runs]
+    plain = hip.attn_states(q, [k], [v], [[0]], 32, None)[0]
+    assert not torch.equal(want[0][0], plain[0])   # it is split
+    torch.cuda.synchronize()
+    errors = []
+    start = threading.Barrier(2)
+
+    def work(i):
+        try:
+            start.wait()
+            for _ in range(60):
+                out, lse = runs[i]()
+                assert torch.equal(out, want[i][0]) and torch.equal(lse, want[i][1])
+        except BaseException as e:   # noqa: BLE001 (reported by the assertion below)
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+
+
 def test_a_schedule_of_its_own_may_be_a_strided_count_and_a_list_of_any_shape(hip):
     g = torch.Generator().manual_seed(7)
     q, k, v = (torch.randn(1, 96, 2, 64, generator=g).bfloat16().cuda() for _ in range(3))
