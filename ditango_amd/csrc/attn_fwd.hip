@@ -492,7 +492,8 @@ __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row
   const int my_row = min(col, rows - 1);
   const uint32_t lane_off = (uint32_t)(lane / kRowLanes) * row_bytes + 16u * (uint32_t)(lane % kRowLanes);
   // The batch under the load cursor.  States that are not there (behind the last one, and everything once i0 < 0) are empty
-  // descriptors: their loads touch no memory and return zeros.
+  // descriptors: their loads touch no memory and return zeros.  So do those of rows that are not there.  (The row is part of the
+  // lane's offset, as in the stores: the scalar offset stays 0, below the length of every descriptor that is not empty.)
   int i0 = (n - 1) / kStates * kStates;
   u32x4 r[kStates];
   auto open = [&]() __attribute__((always_inline)) {
@@ -502,12 +503,12 @@ __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row
   };
   u32x4 x[kDepth][kLoads];
   auto load = [&](int s) __attribute__((always_inline)) {
+    const uint32_t off = lane_off + (uint32_t)(s / kParts * kRowsPer) * row_bytes;
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const u32x4& d = r[s % kParts * kLoads + j];
       x[s % kDepth][j] = __builtin_amdgcn_raw_buffer_load_b128(
-          __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)d.y << 32 | d.x), 0, d.z, kRsrcFlags),
-          lane_off, (uint32_t)(s / kParts * kRowsPer) * row_bytes, kDeviceNt);
+          __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)d.y << 32 | d.x), 0, d.z, kRsrcFlags), off, 0, kDeviceNt);
     }
   };
   float l[kStates];

@@ -128,6 +128,28 @@ def test_rows_without_any_state_and_infinite_values(hip):
     _close(lse, torch.full_like(lse, 0.5 + 0.6931472), torch.float32, "lse")
 
 
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 9])
+@pytest.mark.parametrize("D", [64, 128])
+def test_infinities_of_the_last_state(hip, n, D):
+    """The lists of states go on behind the last one with copies of it that are not to be read: an infinity of its own, in every
+    row, is one in the result, and nothing else is.  (Heads enough that a launch of one job merges itself; 32 rows and 8.)"""
+    Sq, H = 40, 2048
+    q, ks, vs = _inputs(1, Sq, H, D, (64,) * n, torch.bfloat16)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    so = torch.randn(n, 1, Sq, H, D, generator=g, device="cuda").bfloat16()
+    sl = 2 * torch.randn(n, 1, H, Sq, generator=g, device="cuda")
+    col = ((5 * torch.arange(Sq, device="cuda")[:, None] + 3 * torch.arange(H, device="cuda")) % D)[None, :, :, None]
+    so[-1].scatter_(-1, col, float("inf"))
+    ids = torch.zeros(n, dtype=torch.int32, device="cuda")
+    out, lse = hip.attn_sched_merge(q, hip.ChunkTable(ks, vs), ids, ids[:1].clone(), 1, so, sl, -1, so[0], sl[0], torch.float32)
+    assert not torch.isnan(out).any()
+    assert torch.equal(torch.isinf(out), torch.zeros_like(out, dtype=torch.bool).scatter_(-1, col, True))
+    want, want_lse = hip.merge_arena(so, sl, -1, so[0], sl[0])
+    finite = ~torch.isinf(out)
+    _close(out[finite], want[finite], torch.float32, "out")
+    _close(lse, want_lse, torch.float32, "lse")
+
+
 def test_merging_launch_replays_in_a_graph(hip):
     q, ks, vs = _inputs(1, 600, 3, 64, (1500, 1500), torch.bfloat16)
     run = lambda: hip.attn_states_merge(q, ks, vs, [[0], [1]], 32, [], [], [0, 1], torch.float32, hip.attn_workspace("cuda"))[1:]
