@@ -1856,23 +1856,43 @@ static int launch_planned(AttnArgs& a, int D, int n_jobs, hipStream_t stream, vo
   return hip_fail(hipGetLastError(), "attn tail fold launch");
 }
 
-// Whether a launch that merges does so itself, or the fold and merge kernels behind it; `tiles` is the key tiles of the
-// longest item.  In 8 rounds and more the merge of one round runs beside the keys of another: 24 heads x 119 056 queries, 3 of 32
-// chunks 17.2 -> 15.9 ms, 24 x 14 882, 4 of 8 8348 -> 8306 us.  In shorter ones it is one wavefront's chain of waits per 32 rows, against
-// kernels that spread over the chip, and a launch less for the host (us per call with the GPU kept busy, kernels behind -> own):
-//   * items in three parts and more are folded one part after the other: 4 heads x 1244 queries, two chunks, D = 128 27 -> 34,
-//     16 x 2075, two states 92 -> 99, 16 x 2177, D = 64 59 -> 63; two parts 16 x 1331, D = 128 46.4 -> 45.6, 4 x 3026, D = 64 39.5 -> 37.8;
-//   * 8 states in place of 2 are four times the loads of that chain: D = 64 24 x 269 17.0 -> 21.7, 24 x 1423 38.7 -> 40.7, 48 x 160 15.2
-//     -> 17.6, D = 128 20 x 200 19 -> 25; 4 are the most that gain at D = 64;
-//   * D = 64 otherwise gains: 30 x 630, 4 states 18.6 -> 16.5, 30 x 1513 53.4 -> 51.3, 48 x 143 13.2 -> 12.9 (of 60 launches the
-//     worst 38.7 -> 39.6, 40 x 1010);
-//   * D = 128 does not: 40 x 274, 4 states 20 -> 24, 24 x 418 20 -> 23, 40 x 959 34.6 -> 35.3, 48 x 1452 87.6 -> 89.7.  Only where an item is
-//     over before the host has the next call ready (4 key tiles) does the launch less count for more: 24 x 200 22.8 -> 19.9 in a loop of
-//     calls, 15 -> 16.5 with the GPU kept busy.
+// Whether a launch that merges does so itself, or the fold and merge kernels behind it; `tiles` is the key tiles of the longest
+// item, `cus` the CUs of an XCD.  What an item pays is its states' way past the L2, the wait for them and the count; what the
+// launch gains is the merge of one round beside the keys of another.  us per call through proAttention.attn, kernels behind -> own:
+//   * only the last job's items merge, so there have to be more of them than run at a time, 1.5 a CU: D = 128 24 heads x 1861 queries, 15 of 16
+//     chunks computed (24 a XCD) 643 -> 664, 24 x 4000, 3 of 8 (48) 543 -> 536; D = 64 24 x 1861 377 -> 382, 24 x 4000, 15 of 16 1463 ->
+//     1450;
+//   * an item has to be long beside what it pays, 10 key tiles at D = 64 (24 x 6000 against chunks of 6 tiles 229 -> 246, 16 x 8000, 8 tiles
+//     142 -> 142, 32 x 5157, 11 tiles 318 -> 311) and 20 at D = 128, whose states are twice the bytes (24 x 6000, 6 tiles 429 -> 449, 16 x
+//     8000, 8 tiles 266 -> 281, 24 x 6510, 13 tiles 605 -> 605, 32 x 8979, 24 tiles 1292 -> 1281);
+//   * with 8 items a CU in all both head dimensions gain or are even (24 x 119 056, 3 of 32 17.2 -> 15.9 ms, 30 x 8713, 2 of 3 1877 -> 1863); with
+//     fewer D = 128 may lose (48 x 2222, 1 of 8, 1.7 a CU 162 -> 167; 4 of 16, 6.8 a CU 512 -> 514), D = 64 does not (101 -> 102, 301 -> 295).
+static bool long_launch_merges(int D, int n_jobs, int per_xcd, int tiles, int cus) {
+  return cus > 0 && (int64_t)n_jobs * per_xcd >= 8 * cus && 2 * per_xcd >= 3 * cus && tiles >= (D == 64 ? 10 : 20);
+}
+// In a short launch the merge is one wavefront's chain of waits per 32 rows, against kernels that spread over the chip, and the GPU mostly
+// loses by it; what is gained is one launch less for the host, whose share of a call is 16 us (18.5 with the merge kernel).  So a
+// launch that is over by then merges itself (us per call in a loop of calls, kernels behind -> own; in brackets the same with the GPU kept
+// busy):
+//   * D = 64 up to 128 queries (24 x 96, 2 states 18.7 -> 15.9 [13.3 -> 12.9]) and beyond them up to 12 items an XCD (4 x 512, 2 of 4
+//     19.0 -> 16.3 [16.4 -> 15.8], 24 x 200 18.4 -> 17.0 [15.7 -> 16.9]); 24 items are too many (48 x 512, two states 20.5 -> 23.0 [22.0 ->
+//     24.3], 24 x 512, 4 states 20.6 -> 23.4).  From an item a CU of one job, of 10 key tiles, it gains in fewer rounds than the rule above asks
+//     for (12 x 7732, steps of up to 4 chunks 2964 -> 2941, 48 x 2222 148 -> 146, two samples of 24 x 1639 1.02; 16 x 1968, 11 tiles 1.00);
+//     24 x 1735 and 48 x 1000 lose 2 and 4 %;
+//   * D = 128 up to 12 items and either 128 queries and 4 key tiles (24 x 96, 2 states 18.7 -> 16.7 [14.3 -> 15.7]; 30 x 99, 4 tiles 1.00) or
+//     160 and 2 (8 x 147, 2 tiles 1.16, 20 x 156, one 1.11); 48 x 119, 18 items 0.95, 24 x 103, 7 tiles 0.94, 12 x 200, 4 tiles 18.4 -> 20.8
+//     [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94;
+//   * up to 4 states: 8 are twice the loads of the chain (D = 64 24 x 269 17.0 -> 21.7, D = 128 20 x 200 19 -> 25);
+//   * items in up to two parts: three and more are folded one after the other (3 x 1706, D = 64, 4 parts 0.91).
+static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, int per_xcd, int tiles, int cus) {
+  const bool few = (int64_t)n_jobs * per_xcd <= 12, small = Sq <= kBQ / 2;
+  if (n_states > 4) return false;
+  if (D == 64) return small || few || (cus > 0 && per_xcd >= cus && tiles >= 10);
+  return few && (small ? tiles <= 4 : Sq <= 160 && tiles <= 2);
+}
 static bool merges_in_launch(const AttnArgs& a, int D, int n_jobs, int tiles, int cus, const TailPlan& plan) {
-  if (cus > 0 && (int64_t)n_jobs * a.per_xcd >= 8 * cus) return true;
-  if (a.merge_n > 4 || (plan.items > 0 && !plan.rows && plan.ways > 2)) return false;
-  return D == 64 || tiles <= 4;
+  if (long_launch_merges(D, n_jobs, a.per_xcd, tiles, cus)) return true;
+  return short_launch_merges(D, a.Sq, a.merge_n, n_jobs, a.per_xcd, tiles, cus) && (plan.items == 0 || plan.rows || plan.ways <= 2);
 }
 
 // The merge of such a launch, by the merge kernel.
