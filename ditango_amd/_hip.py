@@ -63,6 +63,7 @@ _SIGNATURES = {
                                                     c_i32, _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32),
                                                     _P(c_vp), _P(c_vp), c_f32, c_i32, c_vp]),
     "dt_attn_merge_counters": (ctypes.c_int64, [c_i32, c_i32, c_i32]),
+    "dt_attn_merges_in_launch": (ctypes.c_int, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
     "dt_attn_jobs_merge_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                               c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                               c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_vp, c_f32, c_i32,
@@ -290,12 +291,14 @@ def attn_counters(device, q: torch.Tensor) -> Optional[torch.Tensor]:
     merge, where it needs more than a kept set holds, and under capture: a graph's set would have to be cleared by every replay, a
     launch more than the merge saves."""
     B, Sq, H, _ = q.shape
-    need = int(load_library().dt_attn_merge_counters(B, Sq, H))
-    if need > KEPT_COUNTERS:
-        return None
-    if torch.cuda.is_current_stream_capturing():
-        return None
     dev = device if isinstance(device, torch.device) else torch.device(device)
+    return _stream_counters(dev, int(load_library().dt_attn_merge_counters(B, Sq, H)))
+
+
+def _stream_counters(dev: torch.device, need: int) -> Optional[torch.Tensor]:
+    """``attn_counters`` for a launch that needs ``need`` of them: what the native side calls when it is about to merge."""
+    if need > KEPT_COUNTERS or torch.cuda.is_current_stream_capturing():
+        return None
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     key = (dev.type, index, _raw_stream(index))
     c = _counters.pop(key, None)
@@ -403,7 +406,7 @@ def attn_states_merge(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunk
     ``[B,S,H,1]`` lse), in the same launch where it can.  Returns (states, out, lse)."""
     return _host().attn_states_merge(q, k_chunks, v_chunks, jobs, max_chunks, cu_q, cu_kv, workspace, _attn_flags(q, q_prescaled),
                                      None if dev_segments is None else dev_segments.native, convert, outs, lses, which, dst_dtype,
-                                     attn_counters(q.device, q), _stream())
+                                     lambda need: _stream_counters(q.device, need), _stream())
 
 
 def attn_sched_merge(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor, max_jobs: int,
@@ -411,7 +414,8 @@ def attn_sched_merge(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.
                      dst_dtype: torch.dtype, workspace: Optional[torch.Tensor] = None, q_prescaled: bool = False, row: int = 0):
     """``attn_sched_fwd`` on whole queries and ``merge_arena``, in the same launch where it can.  Returns (out, lse)."""
     return _host().attn_sched_merge(q, table.native, dev_compute_ids, dev_count, row, max_jobs, slot_out, slot_lse, diag, diag_out,
-                                    diag_lse, dst_dtype, workspace, attn_counters(q.device, q), _attn_flags(q, q_prescaled), _stream())
+                                    diag_lse, dst_dtype, workspace,
+                                    lambda need: _stream_counters(q.device, need), _attn_flags(q, q_prescaled), _stream())
 
 
 def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor,

@@ -1890,6 +1890,15 @@ static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, int per
   if (D == 64) return small || few || (cus > 0 && per_xcd >= cus && tiles >= 10);
   return few && (small ? tiles <= 4 : Sq <= 160 && tiles <= 2);
 }
+// CUs of an XCD of the current device; 0: not known.
+static int xcd_cus() {
+  const int cus = cu_count();
+  return cus >= 64 && cus % kXcds == 0 ? cus / kXcds : 0;
+}
+bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, int per_xcd, int tiles) {
+  const int cus = xcd_cus();
+  return long_launch_merges(D, n_jobs, per_xcd, tiles, cus) || short_launch_merges(D, Sq, n_states, n_jobs, per_xcd, tiles, cus);
+}
 static bool merges_in_launch(const AttnArgs& a, int D, int n_jobs, int tiles, int cus, const TailPlan& plan) {
   if (long_launch_merges(D, n_jobs, a.per_xcd, tiles, cus)) return true;
   return short_launch_merges(D, a.Sq, a.merge_n, n_jobs, a.per_xcd, tiles, cus) && (plan.items == 0 || plan.rows || plan.ways <= 2);
@@ -1932,10 +1941,9 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   if (n_jobs <= kMaxLaunchJobs) {
     JobSize size[kMaxLaunchJobs];
     job_sizes(a, n_jobs, size);
-    const int cus = cu_count();
-    const bool known = cus >= 64 && cus % kXcds == 0;
-    const TailPlan plan = plan_launch(a, D, n_jobs, size, known ? cus / kXcds : 0,
-                                      known && workspace ? std::min(workspace_bytes, kWorkspaceBytes) / partial_state_bytes(D) : -1);
+    const int cus = xcd_cus();
+    const TailPlan plan = plan_launch(a, D, n_jobs, size, cus,
+                                      cus > 0 && workspace ? std::min(workspace_bytes, kWorkspaceBytes) / partial_state_bytes(D) : -1);
     a.tail_items = plan.items;
     a.part_ways = plan.ways;
     a.row_split = plan.rows ? 1 : 0;
@@ -1943,7 +1951,7 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
     if (a.arrive) {
       int longest = 0;
       for (int j = 0; j < n_jobs; ++j) longest = std::max(longest, size[j].tiles);
-      merge_after = !merges_in_launch(a, D, n_jobs, longest, known ? cus / kXcds : 0, plan);
+      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan);
     }
   }
   if (!merge_after) return launch_planned(a, D, n_jobs, stream, workspace, workspace_bytes);

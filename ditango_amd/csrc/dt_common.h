@@ -139,6 +139,8 @@ static_assert(DT_MAX_CHUNKS % kMergeBatch == 0 && DT_MAX_MERGE_LIST % kMergeBatc
 static_assert(DT_MAX_MERGE_LIST * sizeof(AttnState) <= DT_MAX_CHUNKS * sizeof(int32_t*), "the list shares the boundaries' place");
 static_assert(sizeof(AttnArgs) <= 4096, "the kernel arguments travel in the 4 KB kernarg segment");
 
+// Whether a merging launch of these sizes may merge itself (see merges_in_launch).
+bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, int per_xcd, int tiles);
 int launch_attn(const AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace = nullptr,
                 int64_t workspace_bytes = 0);
 

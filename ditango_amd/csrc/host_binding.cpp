@@ -327,12 +327,21 @@ typedef std::vector<std::pair<Tensor, Tensor>> States;
 std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vector<Tensor>& lses, std::optional<Tensor> dst_out,
                                 std::optional<Tensor> dst_lse, at::ScalarType dst_dtype, bool dst_bsh, uint64_t stream);
 
-// Whether a launch can merge into a state of dst_dtype (see dt_merge_result).
-bool can_merge(const Tensor& q, const Dims& d, at::ScalarType dst_dtype, int32_t flags, const std::optional<Tensor>& counters) {
-  if (!counters || (flags & DT_ATTN_Q_PRESCALED) || (dst_dtype != at::kFloat && dst_dtype != q.scalar_type())) return false;
-  REQUIRE(counters->is_cuda() && counters->scalar_type() == at::kInt && counters->is_contiguous(), "counters must be int32 on the GPU");
-  return d.H * d.D * 32 * 4 < (1ll << 31);   // (the number of counters is checked with the launch)
+// The counters of a launch that merges n_states states into one of dst_dtype (see dt_merge_result); none where it cannot, or where its
+// sizes are better served by the merge kernel behind it.  Only a launch that merges asks for them, with counters(how many): host work, and
+// memory of the stream's.
+std::optional<Tensor> merge_counters(const Tensor& q, const Dims& d, at::ScalarType dst_dtype, int32_t flags, int64_t n_jobs,
+                                     int64_t key_tiles, int64_t n_states, const py::object& counters) {
+  if (counters.is_none() || (flags & DT_ATTN_Q_PRESCALED) || (dst_dtype != at::kFloat && dst_dtype != q.scalar_type()) ||
+      d.H * d.D * 32 * 4 >= (1ll << 31))
+    return std::nullopt;
+  const int need = dt_attn_merges_in_launch(d.B, d.S, d.H, d.D, n_jobs, key_tiles, n_states);
+  if (need == 0) return std::nullopt;
+  auto c = py::cast<std::optional<Tensor>>(counters(need));
+  REQUIRE(!c || (c->is_cuda() && c->scalar_type() == at::kInt && c->is_contiguous()), "counters must be int32 on the GPU");
+  return c;   // (their number is checked with the launch)
 }
+int64_t tiles_of(const ChunkTable& table, int32_t c) { return (table.len[c] + 63) / 64; }
 dt_merge_result merge_into(const Tensor& out, const Tensor& lse, const Tensor& counters) {
   return {ptr(out), static_cast<float*>(ptr(lse)), dtype_code(out), 0, nullptr, nullptr, static_cast<uint32_t*>(ptr(counters)), counters.numel()};
 }
@@ -342,7 +351,7 @@ struct StatesMerge {
   std::vector<Tensor> outs, lses;
   std::vector<int32_t> which;
   at::ScalarType dtype;
-  std::optional<Tensor> counters;
+  py::object counters;
   std::pair<Tensor, Tensor> result;
 };
 
@@ -402,7 +411,7 @@ States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::ve
     size_t entries = 0;
     for (const auto& list : lists) entries += list.size();
     bool whole = !seg && !cu_q && folds.empty() && !lists.empty() && lists.size() <= DT_MAX_JOBS && entries <= DT_MAX_JOB_ENTRIES &&
-                 table.n <= DT_MAX_CHUNKS && m->outs.size() <= DT_MAX_MERGE_LIST && can_merge(q, d, m->dtype, flags, m->counters);
+                 table.n <= DT_MAX_CHUNKS && m->outs.size() <= DT_MAX_MERGE_LIST;
     const void* state_outs[DT_MAX_MERGE_LIST];
     const float* state_lses[DT_MAX_MERGE_LIST];
     for (size_t i = 0; whole && i < m->outs.size(); ++i) {
@@ -412,9 +421,19 @@ States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::ve
       state_outs[i] = ptr(o);
       state_lses[i] = static_cast<const float*>(ptr(l));
     }
+    std::optional<Tensor> counters;
     if (whole) {
+      int64_t longest = 0;
+      for (const auto& list : lists) {
+        int64_t tiles = 0;
+        for (int32_t c : list) tiles += tiles_of(table, c);
+        longest = std::max(longest, tiles);
+      }
+      counters = merge_counters(q, d, m->dtype, flags, (int64_t)lists.size(), longest, (int64_t)m->outs.size(), m->counters);
+    }
+    if (counters) {
       m->result = {new_out(d, m->dtype, q), new_lse(d, true, q)};
-      dt_merge_result into = merge_into(m->result.first, m->result.second, *m->counters);
+      dt_merge_result into = merge_into(m->result.first, m->result.second, *counters);
       into.n_states = (int32_t)m->outs.size();
       into.state_outs = state_outs;
       into.state_lses = state_lses;
@@ -443,8 +462,7 @@ std::tuple<States, Tensor, Tensor> attn_states_merge(
     const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs, const std::vector<std::vector<int32_t>>& jobs,
     int64_t max_chunks, const std::optional<std::vector<int32_t>>& cu_q, const std::optional<std::vector<std::vector<int32_t>>>& cu_kv,
     const std::optional<Tensor>& workspace, int32_t flags, const Segments* seg, const py::object& convert, std::vector<Tensor> outs,
-    std::vector<Tensor> lses, std::vector<int32_t> which, at::ScalarType dst_dtype, const std::optional<Tensor>& counters,
-    uint64_t stream) {
+    std::vector<Tensor> lses, std::vector<int32_t> which, at::ScalarType dst_dtype, const py::object& counters, uint64_t stream) {
   REQUIRE(outs.size() == lses.size(), "one lse per state");
   StatesMerge m{std::move(outs), std::move(lses), std::move(which), dst_dtype, counters, {}};
   States states = attn_states(q, ks, vs, jobs, max_chunks, cu_q, cu_kv, workspace, flags, seg, convert, stream, &m);
@@ -668,12 +686,18 @@ std::pair<Tensor, Tensor> merge_arena(const Tensor& arena_out, const Tensor& are
 std::pair<Tensor, Tensor> attn_sched_merge(const Tensor& q, const ChunkTable& table, const Tensor& ids, const Tensor& count, int64_t row,
                                            int32_t max_jobs, const Tensor& slot_out, const Tensor& slot_lse, int32_t diag,
                                            const Tensor& diag_out, const Tensor& diag_lse, at::ScalarType dst_dtype,
-                                           const std::optional<Tensor>& workspace, const std::optional<Tensor>& counters,
+                                           const std::optional<Tensor>& workspace, const py::object& counters,
                                            int32_t flags, uint64_t stream) {
   const Dims d = check_query(q, table);
-  if (max_jobs > 0 && slot_out.dim() == 5 && slot_out.size(0) == table.n && can_merge(q, d, dst_dtype, flags, counters)) {
+  std::optional<Tensor> arrive;
+  if (max_jobs > 0 && slot_out.dim() == 5 && slot_out.size(0) == table.n) {
+    int64_t longest = 0;
+    for (int32_t c = 0; c < table.n; ++c) longest = std::max(longest, tiles_of(table, c));
+    arrive = merge_counters(q, d, dst_dtype, flags, max_jobs, longest, table.n, counters);
+  }
+  if (arrive) {
     const Tensor out = new_out(d, dst_dtype, q), lse = new_lse(d, true, q);
-    const dt_merge_result into = merge_into(out, lse, *counters);
+    const dt_merge_result into = merge_into(out, lse, *arrive);
     attn_sched(q, table, ids, count, row, max_jobs, slot_out, slot_lse, diag, diag_out, diag_lse, 0.0, std::nullopt, std::nullopt,
                workspace, flags, nullptr, stream, &into);
     return {out, lse};

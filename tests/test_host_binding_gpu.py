@@ -179,3 +179,40 @@ def test_a_schedule_of_its_own_may_be_a_strided_count_and_a_list_of_any_shape(hi
     for out, lse in states[1:]:
         assert torch.equal(out, states[0][0]) and torch.equal(lse, states[0][1])
     assert states[0][0][0].any() and states[0][0][2].any() and not states[0][0][1].any()
+
+
+def test_counters_are_asked_for_by_launches_that_merge_only(hip, monkeypatch):
+    """The counters of a merging launch are host work, and memory of the stream's: calls that cannot merge (segments, a prescaled q,
+    states of another type) and calls whose sizes go to the merge kernel never ask for them."""
+    asked = []
+    counters = hip._stream_counters
+    monkeypatch.setattr(hip, "_stream_counters", lambda *a: asked.append(a) or counters(*a))
+    rnd = lambda *s, dtype=torch.bfloat16: torch.randn(*s, device="cuda").to(dtype)
+
+    def call(Sq, D, states=(), **k):
+        q, ks, vs = rnd(1, Sq, 2, D), [rnd(1, 300, 2, D)] * 2, [rnd(1, 300, 2, D)] * 2
+        outs, lses = [s[0] for s in states], [s[1] for s in states]
+        asked.clear()
+        _, out, _ = hip.attn_states_merge(q, ks, vs, [[0], [1]], 32, outs, lses, [0, 1], torch.float32, hip.attn_workspace("cuda"), **k)
+        assert torch.isfinite(out).all()
+        return len(asked)
+
+    state = lambda dtype: (rnd(1, 200, 2, 64, dtype=dtype), rnd(1, 2, 200, dtype=torch.float32))
+    assert call(200, 64) == 1 and call(200, 64, [state(torch.bfloat16)]) == 1
+    assert call(200, 64, [state(torch.float32)]) == 0
+    assert call(200, 64, [state(torch.bfloat16)] * 3) == 0      # 5 states
+    assert call(200, 128) == 0
+    assert call(200, 64, q_prescaled=True) == 0
+    assert call(200, 64, cu_q=[0, 200], cu_kv=[[0, 300]] * 2) == 0
+    cu, cu_kv = torch.tensor([0, 200], dtype=torch.int32, device="cuda"), torch.tensor([0, 300], dtype=torch.int32, device="cuda")
+    assert call(200, 64, dev_segments=hip.DeviceSegments(cu, [cu_kv] * 2, 200)) == 0
+
+    def scheduled(Sq, D, **k):
+        q, ks = rnd(1, Sq, 2, D), [rnd(1, 300, 2, D)] * 2
+        so, sl = rnd(2, 1, Sq, 2, D), rnd(2, 1, 2, Sq, dtype=torch.float32)
+        ids = torch.tensor([0, 1], dtype=torch.int32, device="cuda")
+        asked.clear()
+        hip.attn_sched_merge(q, hip.ChunkTable(ks, ks), ids, ids[1:], 1, so, sl, -1, so[0], sl[0], torch.float32, hip.attn_workspace("cuda"), **k)
+        return len(asked)
+
+    assert scheduled(200, 64) == 1 and scheduled(200, 128) == 0 and scheduled(200, 64, q_prescaled=True) == 0
