@@ -2,6 +2,7 @@
 import pytest
 
 from tests.launch_log import record
+from tests.test_merge_launch_gpu import MERGING
 
 # launches in several parts with a fold kernel behind, and with the fold in a launch that merges
 SPLIT = dict(B=1, Sq=900, H=2, D=128, lens=[2600], jobs=[[0]], merged=0)
@@ -46,6 +47,11 @@ MERGES = [
     (_masked(48, 128, 128, 3, 3), False), (_masked(3, 128, 128, 2, 2, 256), True), (_masked(3, 128, 128, 2, 2, 257), False),
     (_masked(4, 96, 64, 4, 1), True), (_masked(4, 96, 64, 5, 1), False), (_masked(3, 1706, 64, 3, 1), False),
 ]
+
+
+def test_the_gpu_tests_of_merging_launches_merge(tmp_path):
+    for call, kernels in zip(MERGING, record(tmp_path, MERGING)):
+        assert len(kernels) == 1, call
 
 
 def test_which_launches_merge_their_states(tmp_path):

@@ -1,5 +1,7 @@
 """Launches that merge (``dt_attn_sched_merge_fwd``, ``dt_attn_jobs_merge_fwd``) against the same launch without a merge and
-the merge kernel behind it: the two compute one thing, in fp32 from the same 16-bit states."""
+the merge kernel behind it: the two compute one thing, in fp32 from the same 16-bit states.  Such a call merges in the launch for some
+sizes and in a kernel behind it for others; tests/test_launch_order.py checks, without a GPU, that those of ``MERGING`` below are
+of the first kind."""
 import pytest
 import torch
 
@@ -29,13 +31,15 @@ def _close(got, want, dtype, what):
     largest value here.  A 16-bit result, or states that were folded from parts (another order under their rounding), may differ by one
     rounding of a state: 2^-8 (bf16) or 2^-11 (fp16) of the value's binade."""
     tol = {torch.float32: 2.0 ** -20, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
-    scale = max(1.0, want.float().abs().max().item())
-    assert (got.float() - want.float()).abs().max().item() <= tol * scale, what
-    assert torch.isfinite(got.float()).all(), what
+    got, want = got.float(), want.float()
+    got, want = got.masked_fill(got == want, 0.0), want.masked_fill(got == want, 0.0)   # (the lse of a chunk without keys: -inf in both)
+    assert torch.isfinite(got).all(), what
+    err, scale = (got - want).abs().max().item(), max(1.0, want.abs().max().item())
+    assert err <= tol * scale, what
 
 
 # rows: one, the edges of a 32-row slice, of half a tile and of a tile, several tiles; chunks without keys, of less than a key
-# tile, of the sizes at which a launch is cut along its rows (8 key tiles) and along its keys (16 and more)
+# tile, of the sizes at which a launch is cut along its rows (8 key tiles) and along its keys (16 and more); some of them merge
 SHAPES = [
     (1, 1, 3, 64, (40, 0, 64), (0, 2)), (1, 31, 2, 128, (64, 65, 1), (0, 1, 2)), (2, 33, 3, 64, (200, 130), (1,)),
     (1, 127, 4, 128, (512, 512, 512), (0, 2)), (1, 129, 4, 64, (512, 512, 512), (0, 2)), (1, 512, 4, 64, (512,) * 4, (0, 3)),
@@ -45,7 +49,19 @@ SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("B,Sq,H,D,lens,computed", SHAPES)
+# launches that merge: short ones, one job a chunk, and ...
+SHORT = [SHAPES[i] for i in (0, 1, 2, 4, 5)] + [(1, 128, 6, 128, (250, 30), (0, 1)), (1, 700, 3, 64, (700, 650), (1, 0))]   # (the last along its rows)
+# ... long ones, of enough items and key tiles: whole items of one, several and many tiles, items cut in two along the rows, and in 2, 4 and 5
+# parts along the keys; 2 ... 6 states; the last in few rounds
+LONG = [
+    (1, 31, 1040, 128, (1290, 90), (0, 1)), (1, 300, 560, 128, (1300, 90), (1, 0)), (1, 1861, 66, 128, (1300, 90, 64, 0), (0, 2, 3)),
+    (1, 300, 528, 128, (1300, 90), (0, 1)), (1, 300, 540, 64, (700, 90), (0,)), (1, 100, 1080, 128, (2600, 90), (0, 1)),
+    (1, 300, 352, 128, (2600, 90, 90), (0, 1, 2)), (2, 300, 262, 64, (2600, 90), (0, 1)), (1, 289, 200, 64, (700, 90, 90, 1, 90, 0), (0, 4)),
+    (1, 300, 130, 64, (700, 600), (0, 1)),
+]
+
+
+@pytest.mark.parametrize("B,Sq,H,D,lens,computed", SHAPES + SHORT[-2:] + LONG)
 @pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 def test_scheduled_launch_that_merges(hip, B, Sq, H, D, lens, computed, dtype, out):
     q, ks, vs = _inputs(B, Sq, H, D, lens, dtype, strided=Sq % 2 == 1)
@@ -77,28 +93,44 @@ def test_scheduled_launch_that_merges(hip, B, Sq, H, D, lens, computed, dtype, o
 
 
 
-@pytest.mark.parametrize("n", [1, 4, 5, 8, 9, 16, 17])
+NUMBERS = [1, 4, 5, 8, 9, 16, 17]
+
+
+def _of_states(n, D):
+    """Rows that end in the middle of a load instruction's; heads and keys enough that the launch merges any number of states."""
+    return 1, 70, 520 if n >= 5 else 2080, D, (1290 if D == 128 else 650,) + (90,) * (n - 1), (n // 2,)
+
+
+@pytest.mark.parametrize("n", NUMBERS)
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("dtype,out", [(torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 def test_numbers_of_states_that_merge(hip, n, D, dtype, out):
-    """The edges of the merge's batches of states, on rows that end in the middle of a load instruction's (with heads enough that
-    a launch of more than 4 states merges)."""
-    test_scheduled_launch_that_merges(hip, 1, 70, 520, D, (90,) * n, (n // 2,), dtype, out)
+    """The edges of the merge's batches of states."""
+    test_scheduled_launch_that_merges(hip, *_of_states(n, D), dtype, out)
 
 
-@pytest.mark.parametrize("B,Sq,H,D,lens,jobs,cached", [
+# host-listed jobs and cached states; those from the fifth on merge 2, 6, 9, 16, 5 and 3 states in the launch
+JOBS = [
     (1, 65, 3, 64, (100, 100), [[0], [1]], 0), (1, 512, 4, 128, (512,) * 4, [[2], [0, 1, 3]], 3), (2, 333, 2, 64, (900, 1700, 64), [[0, 1, 2]], 1),
     (1, 288, 5, 128, (2300, 1), [[0], [1], [0, 1]], 14),
-])
+    (1, 600, 3, 64, (500, 200), [[0, 1]], 0), (1, 288, 352, 128, (700, 600, 64), [[0, 1], [2], [1]], 2), (1, 70, 800, 64, (650, 90), [[1, 0], [0], [1]], 5),
+    (1, 300, 352, 128, (1300, 1), [[0], [1], [0, 1]], 14), (1, 100, 1080, 64, (2600, 90), [[0], [1]], 2), (1, 128, 5, 128, (190, 56), [[0, 1]], 1),
+]
+
+
+def _merged_jobs(jobs, cached):
+    which = list(range(len(jobs))) + [0]   # (a state may be merged twice)
+    return which[:2] if cached + len(which) > 16 else which
+
+
+@pytest.mark.parametrize("B,Sq,H,D,lens,jobs,cached", JOBS)
 def test_jobs_that_merge_with_cached_states(hip, B, Sq, H, D, lens, jobs, cached):
     dtype = torch.bfloat16
     q, ks, vs = _inputs(B, Sq, H, D, lens, dtype)
     g = torch.Generator(device="cuda").manual_seed(9)
     outs = [torch.randn(B, Sq, H, D, generator=g, device="cuda").to(dtype) for _ in range(cached)]
     lses = [2 * torch.randn(B, H, Sq, generator=g, device="cuda") for _ in range(cached)]
-    which = list(range(len(jobs))) + [0]   # (a state may be merged twice)
-    if cached + len(which) > 16:
-        which = which[:2]
+    which = _merged_jobs(jobs, cached)
     ws = hip.attn_workspace("cuda")
     states, out, lse = hip.attn_states_merge(q, ks, vs, jobs, 32, outs, lses, which, torch.float32, ws)
     plain = hip.attn_states(q, ks, vs, jobs, 32, ws)
@@ -128,13 +160,18 @@ def test_rows_without_any_state_and_infinite_values(hip):
     _close(lse, torch.full_like(lse, 0.5 + 0.6931472), torch.float32, "lse")
 
 
+def _infinite(n, D):
+    """One job, with heads and keys enough that its launch merges; 32 rows and 8."""
+    return 1, 40, 2048, D, (1290 if D == 128 else 650,) + (64,) * (n - 1)
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 9])
 @pytest.mark.parametrize("D", [64, 128])
 def test_infinities_of_the_last_state(hip, n, D):
     """The lists of states go on behind the last one with copies of it that are not to be read: an infinity of its own, in every
-    row, is one in the result, and nothing else is.  (Heads enough that a launch of one job merges itself; 32 rows and 8.)"""
-    Sq, H = 40, 2048
-    q, ks, vs = _inputs(1, Sq, H, D, (64,) * n, torch.bfloat16)
+    row, is one in the result, and nothing else is."""
+    B, Sq, H, D, lens = _infinite(n, D)
+    q, ks, vs = _inputs(B, Sq, H, D, lens, torch.bfloat16)
     g = torch.Generator(device="cuda").manual_seed(n)
     so = torch.randn(n, 1, Sq, H, D, generator=g, device="cuda").bfloat16()
     sl = 2 * torch.randn(n, 1, H, Sq, generator=g, device="cuda")
@@ -150,7 +187,60 @@ def test_infinities_of_the_last_state(hip, n, D):
     _close(lse, want_lse, torch.float32, "lse")
 
 
-def test_merging_launch_replays_in_a_graph(hip):
+def _call(B, Sq, H, D, lens, states, jobs=None, max_jobs=0, **k):
+    """The arguments of ``record`` in tests/launch_log.py."""
+    return dict(B=B, Sq=Sq, H=H, D=D, lens=list(lens), jobs=jobs, max_jobs=max_jobs, merged=states)
+
+
+GRAPH = (1, 129, 4, 64, (512,) * 3)
+MERGING = [_call(B, Sq, H, D, lens, len(lens), max_jobs=len(lens)) for B, Sq, H, D, lens, _ in
+           SHORT + LONG + [_of_states(n, D) for n in NUMBERS for D in (64, 128)] + [(*GRAPH, ())]]
+MERGING += [_call(*_infinite(n, D), n, max_jobs=1) for n in (1, 2, 3, 5, 9) for D in (64, 128)]
+MERGING += [_call(B, Sq, H, D, lens, cached + len(_merged_jobs(jobs, cached)), jobs) for B, Sq, H, D, lens, jobs, cached in JOBS[:1] + JOBS[4:]]
+
+
+def test_captured_merging_launch_replays(hip):
+    """A launch that merges, captured with counters of the graph's own: they are at zero after every replay, with eager launches that
+    have theirs in between.  (A layer call under capture runs the merge kernel: its counters would have to be cleared by the graph.)"""
+    B, Sq, H, D, lens = GRAPH
+    q, ks, vs = _inputs(B, Sq, H, D, lens, torch.bfloat16)
+    table = hip.ChunkTable(ks, vs)
+    ids, count = torch.tensor([2, 0, 1], dtype=torch.int32, device="cuda"), torch.tensor([2], dtype=torch.int32, device="cuda")
+    ws = hip.attn_workspace("cuda").clone()
+    own = torch.zeros(hip.attn_counters("cuda", q).numel(), dtype=torch.int32, device="cuda")
+    asked = []
+
+    def run(counters, workspace, so, sl):
+        return hip._host().attn_sched_merge(q, table.native, ids, count, 0, 3, so, sl, -1, so[0], sl[0], torch.float32, workspace, counters,
+                                            0, hip._stream())
+
+    g = torch.Generator(device="cuda").manual_seed(3)
+    states = lambda: (torch.randn(3, B, Sq, H, D, generator=g, device="cuda").bfloat16(), torch.randn(3, B, H, Sq, generator=g, device="cuda"))
+    slots, eager_slots = states(), states()
+    eager = lambda: run(lambda need: hip.attn_counters("cuda", q), hip.attn_workspace("cuda"), *eager_slots)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        run(lambda need: own, ws, *slots)
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            got = run(lambda need: asked.append(need) or own, ws, *slots)
+    assert asked and asked[0] <= own.numel()
+    for _ in range(5):
+        q.copy_(torch.randn(q.shape, generator=g, device="cuda").bfloat16())
+        for mine, others in zip(slots, eager_slots):
+            mine.copy_(torch.randn(mine.shape, generator=g, device="cuda").to(mine.dtype))
+            others.copy_(mine)
+        graph.replay()
+        want = eager()
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        assert all(torch.equal(mine, others) for mine, others in zip(slots, eager_slots))
+        assert not own.any() and not hip.attn_counters("cuda", q).any()
+
+
+def test_layer_call_replays_in_a_graph(hip):
+    """Under capture the states are merged by the kernel behind the launch."""
     q, ks, vs = _inputs(1, 600, 3, 64, (1500, 1500), torch.bfloat16)
     run = lambda: hip.attn_states_merge(q, ks, vs, [[0], [1]], 32, [], [], [0, 1], torch.float32, hip.attn_workspace("cuda"))[1:]
     want = run()
