@@ -63,7 +63,7 @@ _SIGNATURES = {
                                                     c_i32, _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32), _P(c_i32),
                                                     _P(c_vp), _P(c_vp), c_f32, c_i32, c_vp]),
     "dt_attn_merge_counters": (ctypes.c_int64, [c_i32, c_i32, c_i32]),
-    "dt_attn_merges_in_launch": (ctypes.c_int, [c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32]),
+    "dt_attn_merges_in_launch": (ctypes.c_int, [c_i32] * 8),
     "dt_attn_jobs_merge_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                               c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                               c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_vp, c_f32, c_i32,

@@ -454,7 +454,7 @@ __device__ __forceinline__ bool arrive_last(uint32_t* counter, int expected) {
 //
 // HBM-bound in large launches: the workgroups run in step, so the last job's all merge at the end of a round, at 5.3 TB/s.
 // Against a merge kernel behind the launch: 24 heads x 119 056 queries, 3 of 32 chunks computed 17.79 -> 16.07 ms; 48 heads x
-// 2222, D = 64, 5 of 8 340 -> 336 us; 4 heads x 512, D = 64, 2 of 4 19.1 -> 15.6.  Tried without success: the jobs side by side,
+// 2222, D = 64, 5 of 8 340 -> 336 us; 4 heads x 512, D = 64, 2 of 4 19.0 -> 16.3.  Tried without success: the jobs side by side,
 // each some items behind the one before it, so that a part of the workgroups merges while the others compute (they fall out of
 // step and no longer share keys and values in the L2: 24 heads x 14 882, 4 of 8 8.53 -> 8.75 ms); adjacent heads on the 8 XCDs
 // (16.1 -> 16.6 ms).
@@ -462,11 +462,10 @@ __device__ __forceinline__ bool arrive_last(uint32_t* counter, int expected) {
 // In small ones a chain of waits at the end of the launch: one wavefront reads 32 rows of all states.  Up to 8 states
 // (kOneBatch) every weight is known before the first row, so rows are finished one after the other, without accumulators for
 // all of them, and the registers hold loads instead: 128 at D = 128 (4 steps of 8 states or all 8 steps of 4), 64 at D = 64.
-// us per call, two steps in flight -> this: 24 heads x 200 queries, D = 128, 1 of 2 chunks 22.8 -> 19.9, 4 of 8 27.1 -> 26.7;
-// 12 heads x 700, D = 64, 1 of 2 17.4 -> 16.9 (and 40 x 2222, D = 128, 2 of 4 221 -> 217, which merges_in_launch leaves to the merge
-// kernel).  More states keep 32 rows of sums in
-// registers and two steps in flight (three make no difference to 29 states of 743 MB; four at D = 64 cost 24 heads x 200
-// queries, 16 states 1.5 us).
+// How many steps are in flight decides little at the sizes that merge here (us per call with the GPU kept busy, two -> this: 24
+// heads x 96 queries, two states, D = 64 12.8 -> 12.6, D = 128 15.3 -> 15.2, 4 states 15.9 -> 16.4; 12 x 700, D = 64 17.3 -> 17.2; 24 x 4000,
+// 3 of 8 chunks 540 -> 540).  More states keep 32 rows of sums in registers and two steps in flight (three make no difference to 29
+// states of 743 MB).
 template <int D, bool kHalf, int kStates, bool kOneBatch>
 __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row0) {
   typedef Elem<kHalf> E;
@@ -1227,9 +1226,9 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
       const int64_t slot0 = item * ways;
       const float* lses = e.ws_lse + slot0 * kBQ + wave * 32 + col;
       const float* parts = e.ws_out + (slot0 * kWaves + wave) * (32 * D);
-      // A chain of waits: two parts are under way while one is added (behind the last one, empty descriptors: no memory is
-      // touched).  One after the other, 2 heads x 4000 queries, D = 128, 4 of 8 chunks took 80.8 us instead of 75.6 and 24 heads x
-      // 1000 76.8 instead of 70.7; such short launches of many parts are the fold kernel's again (merges_in_launch).
+      // Two parts are under way while one is added (behind the last one, empty descriptors: no memory is touched).  At the sizes that
+      // fold themselves -- long launches, and short ones in two parts -- it decides little (us per call, one after the other -> this: D =
+      // 128 24 heads x 8903 queries, 4 of 8 chunks, 8 parts 3050 -> 3043; D = 64 12 x 7844, 10 of 16, 16 parts 3433 -> 3442).
       f32x4 x[2][D / 8];
       float l[2];
       auto load = [&](int p, int buf) __attribute__((always_inline)) {
@@ -1871,37 +1870,42 @@ static bool long_launch_merges(int D, int n_jobs, int per_xcd, int tiles, int cu
   return cus > 0 && (int64_t)n_jobs * per_xcd >= 8 * cus && 2 * per_xcd >= 3 * cus && tiles >= (D == 64 ? 10 : 20);
 }
 // In a short launch the merge is one wavefront's chain of waits per 32 rows, against kernels that spread over the chip, and the GPU mostly
-// loses by it; what is gained is one launch less for the host, whose share of a call is 16 us (18.5 with the merge kernel).  So a
-// launch that is over by then merges itself (us per call in a loop of calls, kernels behind -> own; in brackets the same with the GPU kept
-// busy):
+// loses by it; what is gained is one launch less for the host, 2.5 us.  Through proAttention.attn a call whose jobs are listed on the device
+// (reuse mask) takes the host 16 us, one with jobs listed by the host (stride schedule) 30; a launch that is over by then merges itself
+// (us per call in a loop of calls, kernels behind -> own; in brackets the same with the GPU kept busy):
 //   * D = 64 up to 128 queries (24 x 96, 2 states 18.7 -> 15.9 [13.3 -> 12.9]) and beyond them up to 12 items an XCD (4 x 512, 2 of 4
-//     19.0 -> 16.3 [16.4 -> 15.8], 24 x 200 18.4 -> 17.0 [15.7 -> 16.9]); 24 items are too many (48 x 512, two states 20.5 -> 23.0 [22.0 ->
-//     24.3], 24 x 512, 4 states 20.6 -> 23.4).  From an item a CU of one job, of 10 key tiles, it gains in fewer rounds than the rule above asks
-//     for (12 x 7732, steps of up to 4 chunks 2964 -> 2941, 48 x 2222 148 -> 146, two samples of 24 x 1639 1.02; 16 x 1968, 11 tiles 1.00);
-//     24 x 1735 and 48 x 1000 lose 2 and 4 %;
+//     19.0 -> 16.3 [16.4 -> 15.8], 24 x 200 18.4 -> 17.0 [15.7 -> 16.9]), 48 where the host lists the jobs (48 x 400, steps of 1 and 4 chunks
+//     33.0 -> 30.4 [25.0 -> 26.1]); 24 items on the device's list are too many (48 x 512, two states 20.5 -> 23.0 [22.0 -> 24.3], 24 x 512, 4
+//     states 20.6 -> 23.4) and 72 on the host's (48 x 600, 2 chunks 36.2 -> 37.9);
+//   * D = 64 in launches that the GPU gains by: one job of 24 key tiles and more, whose items all merge (30 x 1952, 1 of 3 1.06, 12 x 4154, 1 of 4 77.5
+//     -> 75.4; 32 x 1479, 24 tiles 1.00, 32 x 1068, 5 tiles 0.96), and an item a CU of one job, of 10 key tiles (12 x 7732, steps of up to 4
+//     chunks 2964 -> 2941, 48 x 2222 148 -> 146; 16 x 1968, 11 tiles 1.00; 24 x 1735 and 48 x 1000, 0.7 a CU, 0.98 and 0.96);
 //   * D = 128 up to 12 items and either 128 queries and 4 key tiles (24 x 96, 2 states 18.7 -> 16.7 [14.3 -> 15.7]; 30 x 99, 4 tiles 1.00) or
 //     160 and 2 (8 x 147, 2 tiles 1.16, 20 x 156, one 1.11); 48 x 119, 18 items 0.95, 24 x 103, 7 tiles 0.94, 12 x 200, 4 tiles 18.4 -> 20.8
-//     [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94;
+//     [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94.  With the host's list up to 24 items of 4 key tiles (48 x 254, 24
+//     items 32.1 -> 29.8 [20.8 -> 25.0]; 48 x 400, 48 items 32.3 -> 36.4);
 //   * up to 4 states: 8 are twice the loads of the chain (D = 64 24 x 269 17.0 -> 21.7, D = 128 20 x 200 19 -> 25);
 //   * items in up to two parts: three and more are folded one after the other (3 x 1706, D = 64, 4 parts 0.91).
-static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, int per_xcd, int tiles, int cus) {
-  const bool few = (int64_t)n_jobs * per_xcd <= 12, small = Sq <= kBQ / 2;
+static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles, int cus) {
+  const int64_t items = (int64_t)n_jobs * per_xcd;
+  const bool small = Sq <= kBQ / 2;
   if (n_states > 4) return false;
-  if (D == 64) return small || few || (cus > 0 && per_xcd >= cus && tiles >= 10);
-  return few && (small ? tiles <= 4 : Sq <= 160 && tiles <= 2);
+  if (D == 64) return small || items <= (host_listed ? 48 : 12) || (n_jobs == 1 && tiles >= 24) || (cus > 0 && per_xcd >= cus && tiles >= 10);
+  return (items <= (host_listed ? 24 : 12) && (small || host_listed) && tiles <= 4) || (items <= 12 && Sq <= 160 && tiles <= 2);
 }
 // CUs of an XCD of the current device; 0: not known.
 static int xcd_cus() {
   const int cus = cu_count();
   return cus >= 64 && cus % kXcds == 0 ? cus / kXcds : 0;
 }
-bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, int per_xcd, int tiles) {
+bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles) {
   const int cus = xcd_cus();
-  return long_launch_merges(D, n_jobs, per_xcd, tiles, cus) || short_launch_merges(D, Sq, n_states, n_jobs, per_xcd, tiles, cus);
+  return long_launch_merges(D, n_jobs, per_xcd, tiles, cus) || short_launch_merges(D, Sq, n_states, n_jobs, host_listed, per_xcd, tiles, cus);
 }
 static bool merges_in_launch(const AttnArgs& a, int D, int n_jobs, int tiles, int cus, const TailPlan& plan) {
   if (long_launch_merges(D, n_jobs, a.per_xcd, tiles, cus)) return true;
-  return short_launch_merges(D, a.Sq, a.merge_n, n_jobs, a.per_xcd, tiles, cus) && (plan.items == 0 || plan.rows || plan.ways <= 2);
+  return short_launch_merges(D, a.Sq, a.merge_n, n_jobs, a.dev_ids == nullptr, a.per_xcd, tiles, cus) &&
+         (plan.items == 0 || plan.rows || plan.ways <= 2);
 }
 
 // The merge of such a launch, by the merge kernel.

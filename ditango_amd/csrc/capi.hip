@@ -126,11 +126,12 @@ extern "C" int64_t dt_attn_merge_counters(int32_t B, int32_t Sq, int32_t H) {
   return B <= 0 || Sq <= 0 || H <= 0 ? 0 : kPartCounters + 8ll * B * H * (((int64_t)Sq + 255) / 256);
 }
 
-extern "C" int dt_attn_merges_in_launch(int32_t B, int32_t Sq, int32_t H, int32_t D, int32_t n_jobs, int32_t key_tiles, int32_t n_states) {
+extern "C" int dt_attn_merges_in_launch(int32_t B, int32_t Sq, int32_t H, int32_t D, int32_t n_jobs, int32_t host_listed, int32_t key_tiles,
+                                        int32_t n_states) {
   if (B <= 0 || Sq <= 0 || H <= 0 || n_jobs <= 0 || n_states <= 0) return 0;
   const int64_t total = (int64_t)B * H * (((int64_t)Sq + 255) / 256);
   const int64_t counters = dt_attn_merge_counters(B, Sq, H);
-  if (counters > INT32_MAX || !may_merge_in_launch(D, Sq, n_states, n_jobs, (int32_t)((total + 7) / 8), key_tiles)) return 0;
+  if (counters > INT32_MAX || !may_merge_in_launch(D, Sq, n_states, n_jobs, host_listed != 0, (int32_t)((total + 7) / 8), key_tiles)) return 0;
   return (int)counters;
 }
 

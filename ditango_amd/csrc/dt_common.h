@@ -140,7 +140,7 @@ static_assert(DT_MAX_MERGE_LIST * sizeof(AttnState) <= DT_MAX_CHUNKS * sizeof(in
 static_assert(sizeof(AttnArgs) <= 4096, "the kernel arguments travel in the 4 KB kernarg segment");
 
 // Whether a merging launch of these sizes may merge itself (see merges_in_launch).
-bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, int per_xcd, int tiles);
+bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles);
 int launch_attn(const AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace = nullptr,
                 int64_t workspace_bytes = 0);
 

@@ -331,11 +331,11 @@ std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vect
 // sizes are better served by the merge kernel behind it.  Only a launch that merges asks for them, with counters(how many): host work, and
 // memory of the stream's.
 std::optional<Tensor> merge_counters(const Tensor& q, const Dims& d, at::ScalarType dst_dtype, int32_t flags, int64_t n_jobs,
-                                     int64_t key_tiles, int64_t n_states, const py::object& counters) {
+                                     bool host_listed, int64_t key_tiles, int64_t n_states, const py::object& counters) {
   if (counters.is_none() || (flags & DT_ATTN_Q_PRESCALED) || (dst_dtype != at::kFloat && dst_dtype != q.scalar_type()) ||
       d.H * d.D * 32 * 4 >= (1ll << 31))
     return std::nullopt;
-  const int need = dt_attn_merges_in_launch(d.B, d.S, d.H, d.D, n_jobs, key_tiles, n_states);
+  const int need = dt_attn_merges_in_launch(d.B, d.S, d.H, d.D, n_jobs, host_listed, key_tiles, n_states);
   if (need == 0) return std::nullopt;
   auto c = py::cast<std::optional<Tensor>>(counters(need));
   REQUIRE(!c || (c->is_cuda() && c->scalar_type() == at::kInt && c->is_contiguous()), "counters must be int32 on the GPU");
@@ -429,7 +429,7 @@ States attn_states(const Tensor& q, const std::vector<Tensor>& ks, const std::ve
         for (int32_t c : list) tiles += tiles_of(table, c);
         longest = std::max(longest, tiles);
       }
-      counters = merge_counters(q, d, m->dtype, flags, (int64_t)lists.size(), longest, (int64_t)m->outs.size(), m->counters);
+      counters = merge_counters(q, d, m->dtype, flags, (int64_t)lists.size(), true, longest, (int64_t)m->outs.size(), m->counters);
     }
     if (counters) {
       m->result = {new_out(d, m->dtype, q), new_lse(d, true, q)};
@@ -693,7 +693,7 @@ std::pair<Tensor, Tensor> attn_sched_merge(const Tensor& q, const ChunkTable& ta
   if (max_jobs > 0 && slot_out.dim() == 5 && slot_out.size(0) == table.n) {
     int64_t longest = 0;
     for (int32_t c = 0; c < table.n; ++c) longest = std::max(longest, tiles_of(table, c));
-    arrive = merge_counters(q, d, dst_dtype, flags, max_jobs, longest, table.n, counters);
+    arrive = merge_counters(q, d, dst_dtype, flags, max_jobs, false, longest, table.n, counters);
   }
   if (arrive) {
     const Tensor out = new_out(d, dst_dtype, q), lse = new_lse(d, true, q);

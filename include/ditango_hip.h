@@ -371,6 +371,7 @@ int dt_attn_seg_jobs_noalloc_fwd(const void* q, int32_t B, int32_t Sq, int32_t H
  * dt_attn_merges_in_launch is 0 where a launch of these sizes runs the merge kernel behind the attention kernel whatever its split: a
  * caller may then make the two calls itself and needs no counters.  Else it is the number of counters.  Host work only.
  *   n_jobs      jobs of the launch (dt_attn_sched_merge_fwd: max_jobs)
+ *   host_listed 1: dt_attn_jobs_merge_fwd, 0: dt_attn_sched_merge_fwd
  *   key_tiles   of the longest job: sum over its chunks of ceil(length / 64) (dt_attn_sched_merge_fwd: of the longest chunk)
  *   n_states    states to merge
  */
@@ -386,7 +387,8 @@ typedef struct dt_merge_result {
   int64_t n_counters;
 } dt_merge_result;
 int64_t dt_attn_merge_counters(int32_t B, int32_t Sq, int32_t H);
-int dt_attn_merges_in_launch(int32_t B, int32_t Sq, int32_t H, int32_t D, int32_t n_jobs, int32_t key_tiles, int32_t n_states);
+int dt_attn_merges_in_launch(int32_t B, int32_t Sq, int32_t H, int32_t D, int32_t n_jobs, int32_t host_listed, int32_t key_tiles,
+                             int32_t n_states);
 int dt_attn_jobs_merge_fwd(const void* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
                            int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
                            int32_t n_chunks, const void* const* k_ptrs, const void* const* v_ptrs,

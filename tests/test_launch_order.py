@@ -29,6 +29,11 @@ def _masked(H, Sq, D, states, jobs, keys=None, B=1):
     return dict(B=B, Sq=Sq, H=H, D=D, lens=[keys or Sq] * states, jobs=None, max_jobs=jobs, merged=states)
 
 
+def _listed(H, Sq, D, states, jobs, keys=None, B=1):
+    """The same with jobs of one chunk each that the host lists."""
+    return dict(_masked(H, Sq, D, max(states, jobs), 0, keys, B), jobs=[[j] for j in range(jobs)], merged=states)
+
+
 # both sides of every line of the rule: whether the launch merges the states itself
 MERGES = [
     # items of one job: 24 and 48 an XCD; items in all: 216 and 270
@@ -46,6 +51,12 @@ MERGES = [
     (_masked(24, 161, 128, 2, 2, 128), False), (_masked(48, 128, 128, 3, 2), True),
     (_masked(48, 128, 128, 3, 3), False), (_masked(3, 128, 128, 2, 2, 256), True), (_masked(3, 128, 128, 2, 2, 257), False),
     (_masked(4, 96, 64, 4, 1), True), (_masked(4, 96, 64, 5, 1), False), (_masked(3, 1706, 64, 3, 1), False),
+    # one job whose items all merge
+    (_masked(32, 1479, 64, 2, 1), True), (_masked(32, 1479, 64, 2, 1, 23 * 64), False), (_masked(32, 1479, 64, 2, 2), False),
+    # the host's list: items, key tiles
+    (_listed(48, 400, 64, 4, 4), True), (_listed(48, 600, 64, 4, 3), False), (_listed(48, 254, 128, 4, 4), True),
+    (_listed(48, 254, 128, 3, 3, B=2), False), (_listed(24, 256, 128, 2, 2), True), (_listed(24, 257, 128, 2, 2), False),
+    (_listed(12, 300, 64, 5, 2), False),
 ]
 
 
