@@ -1877,13 +1877,13 @@ static bool long_launch_merges(int D, int n_jobs, int per_xcd, int tiles, int cu
 //     19.0 -> 16.3 [16.4 -> 15.8], 24 x 200 18.4 -> 17.0 [15.7 -> 16.9]), 48 where the host lists the jobs (48 x 400, steps of 1 and 4 chunks
 //     33.0 -> 30.4 [25.0 -> 26.1]); 24 items on the device's list are too many (48 x 512, two states 20.5 -> 23.0 [22.0 -> 24.3], 24 x 512, 4
 //     states 20.6 -> 23.4) and 72 on the host's (48 x 600, 2 chunks 36.2 -> 37.9);
-//   * D = 64 in launches that the GPU gains by: one job of 24 key tiles and more, whose items all merge (30 x 1952, 1 of 3 1.06, 12 x 4154, 1 of 4 77.5
-//     -> 75.4; 32 x 1479, 24 tiles 1.00, 32 x 1068, 5 tiles 0.96), and an item a CU of one job, of 10 key tiles (12 x 7732, steps of up to 4
-//     chunks 2964 -> 2941, 48 x 2222 148 -> 146; 16 x 1968, 11 tiles 1.00; 24 x 1735 and 48 x 1000, 0.7 a CU, 0.98 and 0.96);
+//   * D = 64 in launches that the GPU gains by: one job of 24 key tiles and more, whose items all merge (30 x 1952, 1 of 3 1.06, 12 x 4154,
+//     1 of 4 77.5 -> 75.4; 32 x 1479, 24 tiles 1.00, 32 x 1068, 5 tiles 0.96), and an item a CU of one job, of 10 key tiles (12 x 7732,
+//     steps of up to 4 chunks 2964 -> 2941, 48 x 2222 148 -> 146; 16 x 1968, 11 tiles 1.00; 24 x 1735 and 48 x 1000, 0.7 a CU, 0.98, 0.96);
 //   * D = 128 up to 12 items and either 128 queries and 4 key tiles (24 x 96, 2 states 18.7 -> 16.7 [14.3 -> 15.7]; 30 x 99, 4 tiles 1.00) or
-//     160 and 2 (8 x 147, 2 tiles 1.16, 20 x 156, one 1.11; 3 tiles are even: 12 x 142 1.01, 24 x 156 0.95); 48 x 119, 18 items 0.95, 24 x 103, 7 tiles 0.94, 12 x 200, 4 tiles 18.4 -> 20.8
-//     [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94.  With the host's list up to 24 items of 4 key tiles (48 x 254, 24
-//     items 32.1 -> 29.8 [20.8 -> 25.0]; 48 x 400, 48 items 32.3 -> 36.4);
+//     160 and 2 (8 x 147, 2 tiles 1.16, 20 x 156, one 1.11; 3 tiles are even: 12 x 142 1.01, 24 x 156 0.95); 48 x 119, 18 items 0.95, 24 x
+//     103, 7 tiles 0.94, 12 x 200, 4 tiles 18.4 -> 20.8 [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94.  With the host's
+//     list up to 24 items of 4 key tiles (48 x 254, 24 items 32.1 -> 29.8 [20.8 -> 25.0]; 48 x 400, 48 items 32.3 -> 36.4);
 //   * up to 4 states: 8 are twice the loads of the chain (D = 64 24 x 269 17.0 -> 21.7, D = 128 20 x 200 19 -> 25);
 //   * items in up to two parts: three and more are folded one after the other (3 x 1706, D = 64, 4 parts 0.91).
 static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles, int cus) {

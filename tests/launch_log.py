@@ -97,6 +97,12 @@ for calls in asked["in turn"]:
     runtime.log_clear()
     call(**calls)
     answer.append([line.split(" ", 1) for line in runtime.log_text().decode().splitlines()])
+    if calls["merged"]:   # what the library says of such a call beforehand
+        B, Sq, H, D, jobs = (calls[k] for k in ("B", "Sq", "H", "D", "jobs"))
+        tiles = lambda c: (calls["lens"][c] + 63) // 64
+        longest = max(map(tiles, range(len(calls["lens"])))) if jobs is None else max(sum(map(tiles, job)) for job in jobs)
+        need = lib.dt_attn_merges_in_launch(B, Sq, H, D, calls["max_jobs"] if jobs is None else len(jobs), int(jobs is not None), longest, calls["merged"])
+        assert need == lib.dt_attn_merge_counters(B, Sq, H) if len(answer[-1]) == 1 else need in (0, lib.dt_attn_merge_counters(B, Sq, H)), calls
 if asked["together"]:
     runtime.log_clear()
     runtime.log_wait(2000)
@@ -115,7 +121,7 @@ print(json.dumps(answer))
 def record(tmp_path, in_turn=(), together=(), times=0):
     """The launches, (thread, kernel) in the order in which they enter the queue, of every call of ``in_turn`` and then of the calls
     of ``together``, each made ``times`` times by a thread of its own while a launch takes 2 ms.  A call is the arguments of
-    ``call`` above."""
+    ``call`` above; one of ``in_turn`` that merges in its launch has to be one of which ``dt_attn_merges_in_launch`` says so."""
     source, runtime = tmp_path / "runtime.cpp", tmp_path / "runtime.so"
     source.write_text(_RUNTIME)
     subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-o", str(runtime), str(source)], check=True)
