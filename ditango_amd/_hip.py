@@ -46,6 +46,10 @@ _SIGNATURES = {
     "dt_attn_jobs_f32_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                             c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), _P(c_i64), _P(c_i64),
                                             c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_f32, c_vp]),
+    "dt_attn_jobs_f32_ws_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
+                                               c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), _P(c_i64), _P(c_i64),
+                                               c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_i32, c_f32, c_vp, c_i64, c_vp, c_i64,
+                                               c_vp]),
     "dt_attn_jobs_fwd": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i64, c_i64, c_i64,
                                         c_i32, _P(c_vp), _P(c_vp), _P(c_i32), _P(c_i64), c_i64, c_i64,
                                         c_i32, _P(c_i32), _P(c_i32), _P(c_vp), _P(c_vp), c_f32, c_vp]),
@@ -247,11 +251,17 @@ def attn_chunk_f32_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, softma
 
 
 def attn_jobs_f32_fwd(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor],
-                      jobs: Sequence[Sequence[int]], softmax_scale: float = 0.0) -> List[Tuple[torch.Tensor, torch.Tensor]]:
-    """One launch: the fp32 states (out [B,Sq,H,D], lse [B,H,Sq]) of fp32 q against the concatenations of the fp32
-    chunks ``jobs[j]``.  Each chunk may have strides of its own.  More jobs or chunks than one launch addresses run in
-    several."""
-    return _host().attn_states_f32(q, k_chunks, v_chunks, jobs, softmax_scale, _stream())
+                      jobs: Sequence[Sequence[int]], softmax_scale: float = 0.0, lse_bsh: bool = False) -> List[Tuple[torch.Tensor, torch.Tensor]]:
+    """One launch: the fp32 states (out [B,Sq,H,D], lse [B,H,Sq] or, with ``lse_bsh``, [B,Sq,H,1]) of fp32 q against the
+    concatenations of the fp32 chunks ``jobs[j]``.  Each chunk may have strides of its own.  More jobs or chunks than one
+    launch addresses run in several.  Under graph capture workspace and counters come from the graph's pool, and every replay clears the
+    counters."""
+    _require(q.is_cuda and q.dim() == 4, "q must be fp32 [B,S,H,D] on the GPU with contiguous D")
+    B, Sq, H, _ = q.shape
+    need = len(jobs) * B * H * (-(-Sq // 64))
+    counters = torch.zeros(need, dtype=torch.int32, device=q.device) if torch.cuda.is_current_stream_capturing() \
+        else _stream_counters(q.device, need)
+    return _host().attn_states_f32(q, k_chunks, v_chunks, jobs, softmax_scale, _stream(), lse_bsh, attn_workspace(q.device), counters)
 
 
 _workspaces: "dict" = {}   # (device type, index, stream handle) -> tensor, in order of last use

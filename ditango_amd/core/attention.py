@@ -233,8 +233,7 @@ class proAttention:
         self.q_prescaled = False
         # What happens to fp32 inputs (flash_attn_func takes none; the reference's CPU-runnable configuration is
         # stated in fp32): "round" = rounded to bf16 at the kernel boundary, the bf16 MFMA kernels run;
-        # "exact" = every fresh state is computed in fp32 from the fp32 tensors (dt_attn_jobs_f32_fwd, fp32
-        # matrix instructions) and only cached states are rounded to bf16.
+        # "exact" = every fresh state is computed in fp32 from the fp32 tensors (dt_attn_jobs_f32_ws_fwd) and only cached states are rounded to bf16.
         self.fp32_inputs = "round"
         self._exact_f32 = False
         # while a variable-length call runs: (cu_seqlens_q, chunk -> cu_seqlens_kv) as host lists, or a
@@ -360,9 +359,23 @@ class proAttention:
             result.append(parts[0])
         return result
 
+    def _result_f32(self, query, chunks, key, value):
+        """fp32 (out, lse [B,S,H,1]) of ``query`` against the concatenation of ``chunks``, computed in fp32."""
+        if self._segments is not None:
+            raise NotImplementedError("fp32_inputs = 'exact' does not cover variable-length calls")
+        needed = list(dict.fromkeys(chunks))
+        kv = [self._chunk_f32(c, key, value, query.shape[0]) for c in needed]
+        index = {c: i for i, c in enumerate(needed)}
+        return _hip.attn_jobs_f32_fwd(query, [k for k, _ in kv], [v for _, v in kv], [[index[c] for c in chunks]], lse_bsh=True)[0]
+
     def _execute(self, plan: CallPlan, query, key, value, merge_outs, merge_lses, segments=None) -> torch.Tensor:
         r = self.local_chunk_id
         if self._exact_f32:
+            if not merge_outs and self.out_dtype is torch.float32 and len(plan.computed) <= self._MAX_JOB_CHUNKS \
+                    and all(job.store_slot is None for job in plan.jobs):
+                # nothing is kept and nothing is reused: the result is the attention over all chunks of the call
+                out, self.last_lse = self._result_f32(query, [c for job in plan.jobs for c in job.chunks], key, value)
+                return out
             distinct = list(dict.fromkeys(job.chunks for job in plan.jobs))
             seen = dict(zip(distinct, self._job_states_f32(query, distinct, key, value)))
             for job in plan.jobs:

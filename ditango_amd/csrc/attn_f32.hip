@@ -4,29 +4,36 @@
 // for callers that hold fp32 tensors and want the attention of THOSE numbers, not of their bf16
 // roundings -- the reference's CPU-runnable configuration (fp32, 512 queries x 4 chunks of 512 keys,
 // 4 heads, d = 64, which the reference runs on its torch math path because flash_attn_func takes no
-// fp32).  Products and sums are fp32 throughout (v_mfma_f32_32x32x2_f32 multiplies and adds in fp32), so
-// results agree with an fp32 or fp64 closed form to rounding error.
+// fp32).
 //
-// What bounds it: the fp32 matrix pipe, 64 cycles per v_mfma_f32_32x32x2_f32 = 157 TFLOP/s.  In that time a
-// wavefront only needs one new value per lane of the A operand, so the operands come straight from global
-// memory (L1 / L2) into registers: no LDS, no barrier, every wavefront runs on its own.
-//   * A wavefront owns 32 queries and walks key tiles of 32.  Scores are computed transposed, S^T = K Q^T: a
-//     lane owns ONE query (column lane % 32) and 16 of the tile's keys, so the row maximum is an in-register
-//     reduction plus one exchange with lane ^ 32.
-//   * An MFMA contracts two values, one per half of the wavefront.  Which two is free as long as both operands
-//     agree: halves 0 and 1 take d = 8 j + t and 8 j + 4 + t, so one 16-byte load of K (and of Q) feeds four
-//     MFMAs; for O^T += V^T P^T the pair is the two keys whose probabilities the two halves already hold in the
-//     same accumulator register, so P goes from the softmax into the MFMA without moving.  The rows of V^T are
-//     permuted (row i of block b is d = i * D/32 + b), so one load of V feeds D / 32 MFMAs.
-//   * One tile's V is loaded before the score MFMAs, the next tile's K before the P V ones: each has the other
-//     product's time (64 to 128 MFMAs) to arrive, with single buffers.
-//   * The four wavefronts of a workgroup are four query tiles (KW = 1) or split the keys of one (KW = 4, every
-//     fourth tile each, folded through the LDS at the end).
-//   * Measured: 12 heads x 2048 queries x 4 chunks of 2048 keys 103 TFLOP/s at d = 64 and 114 at d = 128 (a plain
-//     fp32 library GEMM of 8192^3 reaches 154 on the same part); the configuration above, one launch for its four
-//     chunks: 18 us against 4 x 220 us on the vector ALU (1.2 TFLOP/s).
+// The products run on the bf16 matrix pipe, 16 times the rate of the fp32 one: every fp32 operand is split into three bf16 values h + m +
+// l, 3 x 8 bits, which leaves nothing out, and a product is the sum of the six terms hh, hm, mh, mm, hl, lh; what is dropped (ml, lm, ll) is
+// below 2^-25 of the product, less than the one rounding of an fp32 multiply-add.  Small terms are added first, and a tile's share of O^T is
+// summed for itself and then added once.  Against fp64, over 22 launches of 96 ... 1680 queries x 190 ... 9560 keys: relative error (2-norm)
+// 1.6 ... 2.4e-7, where v_mfma_f32_32x32x2_f32 (64 cycles for two values a lane) gave 2.9 ... 4.6e-7 of the same numbers.
+// Numbers that do not split -- infinities, NaN, what ends below the exponent range -- show in the result (NaN, or less than 2^-100);
+// a wavefront that sees them walks its keys once more with fp32 products and takes the elements or rows concerned from there.
+//
+// What bounds it: a wavefront issues in order, and an MFMA holds it up (24 MFMAs with 88 vector instructions between them take as long as
+// one behind the other), so a tile takes 48 MFMAs x 32 cycles + 330 vector instructions x 4 at d = 64 (twice the MFMAs at 128), less what
+// the other wavefront of the SIMD hides of it: counters of 8 heads x 1195 queries x 9560 keys, MFMA pipe busy 41 % of the SIMDs' cycles, vector
+// ALU 37 %.  So the split of K and V, half of the vector instructions where every wavefront does its own, is shared:
+//   * QW (2 or 4) wavefronts of a workgroup own 32 queries each and walk the same key tiles of 32.  Each loads its share of a tile in whole
+//     lines, a turn ahead, splits it and puts the three parts into the LDS, from where all read operands (16-byte reads of K,
+//     transposing reads of V, as in attn_fwd.hip).  The KW = 4 / QW groups of a workgroup take every KW-th tile.
+//   * Scores are computed transposed, S^T = K Q^T: a lane owns ONE query (column lane % 32) and 16 of the tile's keys, the row maximum is an
+//     in-register reduction plus one exchange with lane ^ 32, and with the rows of K permuted the probabilities are where the
+//     second product needs them.
+//   * Where the queries alone leave the chip idle, `parts` workgroups share the keys of a work item (plan_f32).
+//   * Measured (us per call with the GPU kept busy, kernel of fp32 products and merge kernel behind it -> this, which needs no other):
+//     4 heads x 512 queries x 2048 keys, d = 64 30 -> 21; 12 x 1053 x 4212 163 -> 101; 8 x 1195 x 9560 258 -> 154 (157 TFLOP/s, as much as
+//     the fp32 pipe has); d = 128 12 x 355 x 2840 107 -> 71, 10 x 847 x 1694 120 -> 73.
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <cstddef>
+#include <mutex>
+#include <type_traits>
 
 #include "dt_common.h"
 
@@ -36,60 +43,302 @@ namespace {
 constexpr int kThreadsF32 = 256;
 constexpr int kWavesF32 = kThreadsF32 / 64;
 constexpr int kTile = 32;   // queries per wavefront, keys per tile
+constexpr int kMaxParts = 16;   // workgroups that share the key tiles of a work item
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 // rows need no more than the 4-byte alignment of their elements
 typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
 
+constexpr int kDevice = 16;   // cache-policy bit of a raw buffer access: device scope (sc1)
+typedef __amdgpu_buffer_rsrc_t Rsrc;
+__device__ __forceinline__ Rsrc buffer_of(const void* base, uint32_t valid_bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, valid_bytes, 0x00020000);
+}
+__device__ __forceinline__ f32x4 load4(Rsrc r, uint32_t off, uint32_t uniform_off) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, uniform_off, 0));
+}
+__device__ __forceinline__ f32x2 load2(Rsrc r, uint32_t off, uint32_t uniform_off) {
+  return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, uniform_off, 0));
+}
+
 // What stands in for a row of V past the end of a chunk.
 __device__ const float kZeroRow[4] = {};
 
+struct F32Chunk {
+  const float *k, *v;
+  int64_t sb, ss, sh;   // element strides
+  int64_t len;
+};
+struct F32Job {
+  float *out, *lse;
+  int32_t begin, end;
+};
 struct AttnF32Args {
   const float* q;
   int64_t q_sb, q_ss, q_sh;
-  int32_t B, H, Sq;
+  int32_t B, H, Sq, D;
+  int32_t parts;     // workgroups that share the key tiles of a work item
+  int32_t lse_bsh;   // lse as [B,Sq,H] instead of [B,H,Sq]
+  // parts > 1: sums, relative to the part's maximum, [part][job][item][32 QW queries][D], and behind them (maximum, sum of weights) of
+  // every query; arrival counters, one per job and item, zero between launches
+  float* ws;
+  uint32_t* arrive;
   int32_t n_qg;      // query groups (workgroups) per (batch, head)
   int32_t total;     // B * H * n_qg
   int32_t per_xcd;
   float scale, scale_log2;
-  // job j attends to the concatenation of the chunks job_chunks[job_begin[j] .. job_begin[j + 1])
-  const float* k[DT_MAX_CHUNKS];
-  const float* v[DT_MAX_CHUNKS];
-  int64_t kv_sb[DT_MAX_CHUNKS], kv_ss[DT_MAX_CHUNKS], kv_sh[DT_MAX_CHUNKS];
-  int32_t kv_len[DT_MAX_CHUNKS];
-  float* out[DT_MAX_JOBS];
-  float* lse[DT_MAX_JOBS];
-  int32_t job_begin[DT_MAX_JOBS + 1];
-  int32_t job_chunks[DT_MAX_JOB_ENTRIES];
+  float grid, inv_grid;
+  // job j attends to the concatenation of the chunks refs[job[j].begin .. job[j].end)
+  int32_t refs[DT_MAX_JOB_ENTRIES];
+  F32Job job[DT_MAX_JOBS];
+  F32Chunk chunk[DT_MAX_CHUNKS];
 };
 static_assert(sizeof(AttnF32Args) <= 4096, "the kernel arguments travel in the 4 KB kernarg segment");
 
-template <int D>
+typedef const AttnF32Args __attribute__((address_space(4))) KernArgsF32;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kJob = (int)offsetof(AttnF32Args, job), kChunk = (int)offsetof(AttnF32Args, chunk), kRefs = (int)offsetof(AttnF32Args, refs);
+// Brings the argument lines that a workgroup is about to read into the scalar cache, all at once (see attn_fwd.hip).
+__device__ __forceinline__ void prefetch_args(uint64_t args) {
+  uint32_t t0, t1, t2, t3, t4, t5, t6, t7, t8, t9, t10;
+  asm volatile(
+      "s_load_dword %0, %11, 0x0\n\ts_load_dword %1, %11, 0x40\n\ts_load_dword %2, %11, %12\n\ts_load_dword %3, %11, %13\n\t"
+      "s_load_dword %4, %11, %14\n\ts_load_dword %5, %11, %15\n\ts_load_dword %6, %11, %16\n\ts_load_dword %7, %11, %17\n\t"
+      "s_load_dword %8, %11, %18\n\ts_load_dword %9, %11, %19\n\ts_load_dword %10, %11, %20\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8), "=&s"(t9), "=&s"(t10)
+      : "s"(args), "i"(kRefs), "i"(kRefs + 64), "i"(kJob), "i"(kJob + 64), "i"(kChunk), "i"(kChunk + 64), "i"(kChunk + 128),
+        "i"(kChunk + 192), "i"(kChunk + 256)
+      : "memory");
+}
+
+template <int D, int QW>
 struct F32Lds {
+  // while the keys are walked: three parts of K and of V per group of wavefronts, [32 keys][D] of 16 bits each
+  static constexpr int kPlane = kTile * D * 2;
+  static constexpr int kGroupBytes = 6 * kPlane;
+  __device__ static constexpr int swz_k(int row) { return D == 128 ? (row & 15) : ((row >> 1) & 7); }
+  __device__ static constexpr int swz_v(int row) { return D == 128 ? (row & 3) : ((row >> 1) & 1); }
+  // behind that: the output rows of every wavefront
   static constexpr int kPitch = D + 4;             // floats per query row of a wavefront's partial output
   static constexpr int kFloatsPerWave = kTile * kPitch + 2 * kTile;   // + maximum and sum of every query
-  static constexpr int kBytes = kWavesF32 * kFloatsPerWave * 4;
+  static constexpr int kWalk = kWavesF32 / QW * kGroupBytes, kEnd = kWavesF32 * kFloatsPerWave * 4;
+  static constexpr int kBytes = kWalk > kEnd ? kWalk : kEnd;
+};
+// Transposing LDS read, see attn_fwd.hip.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ s16x4 lds_read_tr(const uint8_t* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(p));
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float pair32 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+
+// Two fp32 values as the sum of three bf16 ones each: h, the 8 leading bits of the significand rounded to nearest, m the same of
+// what is left, l the rest.  24 bits are three times 8: nothing is left behind l.
+struct Split2 {
+  uint32_t h, m, l;
+};
+__device__ __forceinline__ Split2 split2(float a, float b) {
+  auto round = [](pair32 r) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2)); };
+  auto less = [](pair32 r, uint32_t w) {
+    return pair32{r.x - __builtin_bit_cast(float, w << 16), r.y - __builtin_bit_cast(float, w & 0xffff0000u)};
+  };
+  Split2 s;
+  pair32 r = {a, b};
+  s.h = round(r);
+  r = less(r, s.h);
+  s.m = round(r);
+  r = less(r, s.m);
+  s.l = round(r);
+  return s;
+}
+// Eight values, as an operand of the MFMA.
+struct Split8 {
+  bf16x8 h, m, l;
+};
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+  u32x4 h, m, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const Split2 s = split2(x[2 * i], x[2 * i + 1]);
+    h[i] = s.h; m[i] = s.m; l[i] = s.l;
+  }
+  return {__builtin_bit_cast(bf16x8, h), __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l)};
+}
+__device__ __forceinline__ f32x16 mfma16(const bf16x8& a, const bf16x8& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Workgroup barrier that waits for this wavefront's LDS traffic only: loads of later tiles stay in flight across it.
+__device__ __forceinline__ void tile_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Magnitudes of a row of Q for which three bf16 values hold what counts of an fp32 one: below 2^-110 the last of them loses bits to
+// the end of the exponent range, which 2^90 times as large a K would bring back.
+constexpr uint32_t kTiny = (uint32_t)(127 - 100) << 23, kHuge = (uint32_t)(127 + 90) << 23;
+// Whether an element of O^T is one that the split products may have got wrong: not finite (an infinity leaves NaN behind where
+// it is split), or so small that its terms ended below the exponent range (or zero, which is as rare).
+constexpr uint32_t kOddFrom = 0xff000000u - 2 * kTiny;
+__device__ __forceinline__ uint32_t oddity(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 2 * kTiny; }
+
+// m scale + log(den), rounded about once: the logarithm of den's exponent and of its significand, and the two large terms' sum
+// with its error.  (Plainly, the rounding of a logarithm of 2 to 5 comes on top: 2-norm error of the lse against fp64, 4 heads x 512
+// queries x 2048 keys, 5.2e-8 -> 3.44e-8; the rounding of the exact value to fp32 alone is 3.38e-8.)
+__device__ __forceinline__ float lse_of(float m, float den, float scale) {
+  if (!(den > 0.f)) return -INFINITY;
+  float f = __builtin_amdgcn_frexp_mantf(den);
+  float k = (float)__builtin_amdgcn_frexp_expf(den);
+  if (f < 0.70710678f) {
+    f *= 2.f;
+    k -= 1.f;
+  }
+  constexpr float kLn2Hi = 0.693359375f, kLn2Lo = -2.12194440e-4f;   // (10 bits: k kLn2Hi is exact)
+  const float a = m * scale, b = k * kLn2Hi, sum = a + b;
+  if (!(__builtin_fabsf(sum) < INFINITY)) return sum;
+  const float back = sum - a;
+  const float rest = __builtin_fmaf(m, scale, -a) + ((a - (sum - back)) + (b - back));
+  return sum + (rest + __builtin_fmaf(k, kLn2Lo, logf(f)));
+}
+
+// The walk through the key tiles of a job that one group of wavefronts works on: `left` tiles, counted through the job's chunks.
+template <bool kFar>
+struct Cursor {
+  int seg, seg_end, left;
+  int k0 = 0, len = 0;          // first key of the tile, keys of the chunk
+  const float *kb = nullptr, *vb = nullptr;   // K / V of the chunk for this batch and head
+  int64_t ss = 0;               // its token stride
+  uint32_t plane = 0;           // (!kFar) bytes of the chunk's K (and V) as a buffer, behind which keys read as zeros
+
+  __device__ __forceinline__ Cursor(KernArgsF32& a, int job, int n) : seg(a.job[job].begin - 1), seg_end(a.job[job].end), left(n) {}
+  // False behind the last tile: the buffers are then empty, loads touch no memory and return zeros.
+  __device__ __forceinline__ bool advance(KernArgsF32& a, int b, int h, int tiles) {
+    if (--left < 0) {
+      k0 = len = 0;
+      plane = 0;
+      return false;
+    }
+    k0 += tiles * kTile;
+    while (k0 >= len) {
+      int cid = 0, n = 0;
+      while (n == 0 && ++seg < seg_end) {   // (there is a chunk: `left` tiles are)
+        cid = a.refs[seg];
+        n = (int)a.chunk[cid].len;
+      }
+      k0 -= (len + kTile - 1) / kTile * kTile;   // tiles that reach into this chunk
+      len = n;
+      const auto& chunk = a.chunk[cid];
+      const int64_t off = (int64_t)b * chunk.sb + (int64_t)h * chunk.sh;
+      kb = chunk.k + off;
+      vb = chunk.v + off;
+      ss = chunk.ss;
+      plane = ((uint32_t)(n - 1) * (uint32_t)ss + (uint32_t)a.D) * 4u;
+    }
+    return true;
+  }
 };
 
-// D = 64: two wavefronts per SIMD.  D = 128: the operands of a tile (K, V, Q, O: 64
-// registers each) leave room for one.
-template <int D, int KW>
-__global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(const AttnF32Args args_by_value) {
-  using L = F32Lds<D>;
-  constexpr int kNB = D / 32;      // blocks of 32 output elements
+// O^T of 32 queries against the cursor's tiles with fp32 products (v_mfma_f32_32x32x2_f32), straight from global memory: for the few
+// wavefronts whose numbers do not split.  An MFMA contracts two values, one per half of the wavefront; which two is free as long
+// as both operands agree: halves 0 and 1 take d = 8 j + t and 8 j + 4 + t, and of P V the two keys whose probabilities they hold in
+// the same accumulator register.  Register r of block i is d = (8 (r / 4) + 4 hh + r % 4) D/32 + i.
+template <int D, bool kFar>
+__device__ __forceinline__ void walk_fp32(KernArgsF32& a, int b, int h, int job, int q0, int first, int step, int n, f32x16 (&o)[D / 32],
+                                          float& m, float& l) {
+  constexpr int kNB = D / 32;
   constexpr int kKL = D / 8;       // 16-byte K loads of a lane per tile
   typedef float vvec __attribute__((ext_vector_type(kNB), aligned(4)));
+  const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5;
+  const float c = a.scale_log2;
+  f32x4 qf[kKL];
+  const float* qp = a.q + (int64_t)b * a.q_sb + (int64_t)min(q0 + col, a.Sq - 1) * a.q_ss + (int64_t)h * a.q_sh + 4 * hh;
+#pragma unroll
+  for (int j = 0; j < kKL; ++j) qf[j] = *reinterpret_cast<const f32x4*>(qp + 8 * j);
+#pragma unroll
+  for (int i = 0; i < kNB; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+  m = -FLT_MAX;
+  l = 0.f;
+  Cursor<kFar> at(a, job, n);
+  for (bool more = at.advance(a, b, h, first); more; more = at.advance(a, b, h, step)) {
+    f32x16 s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+    const float* p = at.kb + (int64_t)min(at.k0 + col, at.len - 1) * at.ss + 4 * hh;
+#pragma unroll
+    for (int j = 0; j < kKL; ++j) {
+      const f32x4 k = *reinterpret_cast<const f32x4*>(p + 8 * j);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[t], qf[j][t], s, 0, 0, 0);
+    }
+    const int valid = at.len - at.k0;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      if (8 * (r >> 2) + 4 * hh + (r & 3) >= valid) s[r] = -INFINITY;
+      mx = fmaxf(mx, s[r]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m, mx);
+    const float alpha = __builtin_amdgcn_exp2f((m - m_new) * c);
+    l *= alpha;
+    m = m_new;
+#pragma unroll
+    for (int i = 0; i < kNB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f((s[r] - m) * c);
+      l += s[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      // (past the end zeros, not some key: 0 times an infinity would be NaN)
+      const int key = at.k0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+      vvec v = *reinterpret_cast<const vvec*>(at.vb + (int64_t)min(key, at.len - 1) * at.ss + kNB * col);
+      if (key >= at.len) v = 0.f;
+#pragma unroll
+      for (int i = 0; i < kNB; ++i) {
+        float vi;
+        if constexpr (kNB == 2) vi = i == 0 ? v.x : v.y;
+        else vi = v[i];
+        o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vi, s[r], o[i], 0, 0, 0);
+      }
+    }
+  }
+  l += __shfl_xor(l, 32);
+}
+
+// QW query tiles of 32 and KW groups of key tiles: wavefront w works on query tile w % QW of the workgroup and on every KW-th key
+// tile of the workgroup's part.  The QW wavefronts of a group share what they split.
+template <int D, int QW, bool kFar>
+__global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(const AttnF32Args args_by_value) {
+  constexpr int KW = kWavesF32 / QW;
+  using L = F32Lds<D, QW>;
+  constexpr int kNB = D / 32;                 // blocks of 32 output elements
+  constexpr int kRowLanes = D / 4;            // lanes that load a key, 16 bytes each
+  constexpr int kRowsPer = 64 / kRowLanes;    // keys of a load instruction
+  constexpr int kLoads = kTile / (kRowsPer * QW);   // loads of a wavefront per tile and operand
   // read in place, in the kernarg segment (the struct is the only parameter)
-  typedef const AttnF32Args __attribute__((address_space(4))) KernArgs;
-  KernArgs& a = *(KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  KernArgsF32& a = *(KernArgsF32*)__builtin_amdgcn_kernarg_segment_ptr();
   (void)args_by_value;
-  extern __shared__ __attribute__((aligned(16))) float lds_f32[];
+  prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_f32[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int member = wave % QW, group = wave / QW;
   const int col = lane & 31, hh = lane >> 5;
-  const int job = blockIdx.y;
+  const int job = blockIdx.y / a.parts, part = blockIdx.y - job * a.parts;
   // every XCD works through a contiguous range of heads: its L2 then holds few K / V streams
   const int idx = blockIdx.x >> 3;
   const int item = (int)(blockIdx.x & 7) * a.per_xcd + idx;
@@ -97,155 +346,270 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   const int bh = item / a.n_qg;
   const int qg = item - bh * a.n_qg;
   const int b = bh / a.H, h = bh - b * a.H;
-  const int q0 = (qg * (kWavesF32 / KW) + wave / KW) * kTile;
-  const int kpart = wave % KW;
-  if (KW == 1 && q0 >= a.Sq) return;   // (no barrier follows in this variant)
+  const int q0 = (qg * QW + member) * kTile;
+  const float c = a.scale_log2;
 
-  // Q: B operand, d = 8 j + 4 hh + t (rows past Sq repeat the last one; their results are not stored)
-  f32x4 qf[kKL];
-  {
-    const float* qp = a.q + (int64_t)b * a.q_sb + (int64_t)min(q0 + col, a.Sq - 1) * a.q_ss + (int64_t)h * a.q_sh + 4 * hh;
+  // key tiles of the job, of which this workgroup takes `turns` times KW from `first` on (the groups in turn)
+  int tiles = 0;
+  for (int s = a.job[job].begin; s < a.job[job].end; ++s) tiles += ((int)a.chunk[a.refs[s]].len + kTile - 1) / kTile;
+  const int per_part = (tiles + a.parts * KW - 1) / (a.parts * KW);
+  const int begin = part * per_part * KW, mine_of = min(tiles, begin + per_part * KW) - begin;
+  const int turns = mine_of > 0 ? (mine_of + KW - 1) / KW : 0;
+  const int n_tiles = mine_of > group ? (mine_of - group + KW - 1) / KW : 0;
+
+  // ---- K and V: a wavefront loads its share of a tile with whole lines, splits it and puts the three parts into the LDS
+  Cursor<kFar> at_k(a, job, n_tiles), at_v(a, job, n_tiles);   // K runs two tiles ahead, V one: a load has a whole turn to arrive
+  const int d_mine = 4 * (lane % kRowLanes);
+  auto row_mine = [&](int i) { return (i * QW + member) * kRowsPer + lane / kRowLanes; };
+  f32x4 kreg[kLoads], vreg[kLoads];
+  auto load_tile = [&](const Cursor<kFar>& at, const float* base, f32x4 (&reg)[kLoads]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kKL; ++j) qf[j] = *reinterpret_cast<const f32x4*>(qp + 8 * j);
+    for (int i = 0; i < kLoads; ++i) {
+      if constexpr (kFar) {
+        reg[i] = 0.f;
+        const int key = at.k0 + row_mine(i);
+        if (key < at.len) reg[i] = *reinterpret_cast<const f32x4*>(base + (int64_t)key * at.ss + d_mine);
+      } else {
+        // (the tile's offset is the scalar one: inside the buffer, as the range check subtracts it from the length)
+        reg[i] = load4(buffer_of(base, at.plane), ((uint32_t)row_mine(i) * (uint32_t)at.ss + d_mine) * 4u, (uint32_t)at.k0 * (uint32_t)at.ss * 4u);
+      }
+    }
+  };
+  uint8_t* planes = lds_f32 + group * L::kGroupBytes;
+  auto put = [&](uint8_t* to, const f32x4& x) __attribute__((always_inline)) {
+    const Split2 lo = split2(x[0], x[1]), hi = split2(x[2], x[3]);
+    *reinterpret_cast<u32x2*>(to) = u32x2{lo.h, hi.h};
+    *reinterpret_cast<u32x2*>(to + L::kPlane) = u32x2{lo.m, hi.m};
+    *reinterpret_cast<u32x2*>(to + 2 * L::kPlane) = u32x2{lo.l, hi.l};
+  };
+  // rows of 16-bit elements; 16-byte chunks (K) and 64-byte segments (V) are stored permuted by the row, so that neither the reads of
+  // 16 bytes a row nor the transposing ones meet in a bank
+  auto put_k = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int r = row_mine(i);
+      put(planes + r * (2 * D) + 16 * ((d_mine >> 3) ^ L::swz_k(r)) + 2 * (d_mine & 7), kreg[i]);
+    }
+  };
+  auto put_v = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int r = row_mine(i);
+      put(planes + 3 * L::kPlane + r * (2 * D) + 64 * ((d_mine >> 5) ^ L::swz_v(r)) + 2 * (d_mine & 31), vreg[i]);
+    }
+  };
+  const int krow = (col & 19) | ((col & 4) << 1) | ((col & 8) >> 1);
+  auto k_frag = [&](int plane, int s) __attribute__((always_inline)) {
+    return *reinterpret_cast<const bf16x8*>(planes + plane * L::kPlane + krow * (2 * D) + 16 * ((2 * s + hh) ^ L::swz_k(krow)));
+  };
+  const int vrow = 8 * hh + ((lane & 15) >> 2);
+  auto v_frag = [&](int plane, int i, int half) __attribute__((always_inline)) {
+    const uint8_t* p = planes + (3 + plane) * L::kPlane + (vrow + 16 * half) * (2 * D) + 64 * (i ^ L::swz_v(vrow)) +
+                       (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+    const s16x4 lo = lds_read_tr(p), hi = lds_read_tr(p + 4 * (2 * D));
+    return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+
+  // The instructions that split the next operand go between the MFMAs, which are then the longer of the two.
+  auto interleave = [](auto reads, auto products) __attribute__((always_inline)) {
+    constexpr int kValu = (44 * kLoads / 2 + decltype(products)::value - 1) / decltype(products)::value;
+    __builtin_amdgcn_sched_group_barrier(0x100, decltype(reads)::value, 0);
+#pragma unroll
+    for (int i = 0; i < decltype(products)::value; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+    }
+  };
+
+  const bool any = at_k.advance(a, b, h, begin + group);
+  bool more = at_v.advance(a, b, h, begin + group);
+  load_tile(at_k, at_k.kb, kreg);
+  load_tile(at_v, at_v.vb, vreg);
+
+  // Q: B operand, d = 16 s + 8 hh + e (rows past Sq repeat the last one; their results are not stored)
+  Split8 qs[D / 16];
+  bool odd_q;   // a row of Q outside the magnitudes that can be split
+  {
+    // Whole rows through the LDS (the output rows' place): as loads of 16 bytes of 32 different rows 0.2 to 1 us longer (us per call, 12 heads
+    // x 280 queries x 560 keys, d = 128 27.9 -> 26.9, 10 x 114 x 456 22.7 -> 22.3; 4 x 512 x 2048, d = 64 21.7 -> 21.4).
+    const float* qp = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + d_mine;
+    float* rows = reinterpret_cast<float*>(lds_f32) + wave * L::kFloatsPerWave;
+    f32x4 qv[kTile / kRowsPer];
+#pragma unroll
+    for (int i = 0; i < kTile / kRowsPer; ++i)
+      qv[i] = *reinterpret_cast<const f32x4*>(qp + (int64_t)min(q0 + i * kRowsPer + lane / kRowLanes, a.Sq - 1) * a.q_ss);
+#pragma unroll
+    for (int i = 0; i < kTile / kRowsPer; ++i)
+      *reinterpret_cast<f32x4*>(rows + (i * kRowsPer + lane / kRowLanes) * L::kPitch + d_mine) = qv[i];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) qv[i] = *reinterpret_cast<const f32x4*>(rows + col * L::kPitch + 16 * (i >> 1) + 8 * hh + 4 * (i & 1));
+    float big = 0.f;
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) {
+      float x[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        x[t] = qv[2 * s + (t >> 2)][t & 3];
+        big = fmaxf(big, __builtin_fabsf(x[t]));
+      }
+      qs[s] = split8(x);
+    }
+    big = fmaxf(big, __shfl_xor(big, 32));
+    odd_q = __builtin_bit_cast(uint32_t, big) - kTiny > kHuge - kTiny;
   }
 
-  f32x16 o[kNB];
+  f32x16 o[kNB];   // O^T: register r of block i is d = 32 i + 8 (r / 4) + 4 hh + r % 4
 #pragma unroll
   for (int i = 0; i < kNB; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
   // The maximum starts at the lowest finite value: a row that has met nothing but scores of -inf then gets weights of
-  // exp2(-inf) = 0 and no sum, without a test for it (a test per tile: +1 % at d = 128).
+  // exp2(-inf) = 0 and no sum, without a test for it.
   float m = -FLT_MAX, l = 0.f;
-  const float c = a.scale_log2;
 
-  // The cursor: this wavefront's tiles are every KW-th of the job's, counted through its chunks.  Behind the last
-  // tile it stays on a chunk with keys, so that the loads below need no branch.
-  int seg = a.job_begin[job] - 1;
-  const int seg_end = a.job_begin[job + 1];
-  int k0 = 0, len = 0;          // first key of the tile, keys of the chunk
-  const float *kb = nullptr, *vb = nullptr;   // K / V of the chunk for this batch and head
-  int64_t ss = 0;               // its token stride
-  int whole = 0;                // its keys, where a lane's offset in a tile of V fits 32 bits
-  auto advance = [&](int tiles) __attribute__((always_inline)) -> bool {
-    k0 += tiles * kTile;
-    while (k0 >= len) {
-      int cid = 0, n = 0;
-      while (n == 0) {
-        if (++seg >= seg_end) return false;
-        cid = a.job_chunks[seg];
-        n = a.kv_len[cid];
-      }
-      k0 -= (len + kTile - 1) / kTile * kTile;   // tiles that reach into this chunk
-      len = n;
-      const int64_t off = (int64_t)b * a.kv_sb[cid] + (int64_t)h * a.kv_sh[cid];
-      kb = a.k[cid] + off;
-      vb = a.v[cid] + off;
-      ss = a.kv_ss[cid];
-      whole = (uint64_t)ss < (1u << 28) ? n : 0;
-    }
-    return true;
-  };
-
-  f32x4 kf[kKL];
-  vvec vf[16];
-  auto load_k = [&]() __attribute__((always_inline)) {
-    const float* p = kb + (int64_t)min(k0 + col, len - 1) * ss + 4 * hh;
+  tile_barrier();   // (everybody has Q)
+  if (turns > 0) {
+    put_k();
+    at_k.advance(a, b, h, KW);
+    load_tile(at_k, at_k.kb, kreg);
+  }
+  tile_barrier();
+  for (int turn = 0; turn < turns; ++turn) {
+    // K of this tile is in the LDS
+    const int valid = more ? at_v.len - at_v.k0 : 0;   // (none: the group's tiles are over, another's are not)
+    bf16x8 kf[D / 16][3];   // read before the split of V, whose instructions hide the wait for them
 #pragma unroll
-    for (int j = 0; j < kKL; ++j) kf[j] = *reinterpret_cast<const f32x4*>(p + 8 * j);
-  };
-  // Keys 8 (r / 4) + 4 hh + r % 4 of the tile; past the end zeros, not some key: their probability is 0, and 0 times an
-  // infinity would be NaN.  The zeros are loaded, and chunks of a larger stride take the branch of 64-bit offsets: with the
-  // loaded rows zeroed behind a test, or 64-bit offsets in whole tiles, every tile takes 1 to 4 % longer (12 heads x 1742 queries
-  // x 3484 keys: 405 us at d = 128 and 218 at d = 64 with both, 402 and 211 as it is, and with neither zeros nor large strides).
-  auto load_v = [&]() __attribute__((always_inline)) {
-    if (k0 + kTile <= whole) {
-      const float* p = vb + (int64_t)k0 * ss;
-      const uint32_t lane_off = (uint32_t)(4 * hh) * (uint32_t)ss + (uint32_t)(kNB * col);
+    for (int j = 0; j < D / 16; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) kf[j][p] = k_frag(p, j);
+    put_v();
+    f32x16 s, small;   // (the small terms for themselves: D / 16 sums at the magnitude of the score are rounded, not six times as many)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = small[r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) {
+      const bf16x8 kh = kf[j][0], km = kf[j][1], kl = kf[j][2];
+      small = mfma16(kl, qs[j].h, small);
+      small = mfma16(kh, qs[j].l, small);
+      small = mfma16(km, qs[j].m, small);
+      small = mfma16(km, qs[j].h, small);
+      small = mfma16(kh, qs[j].m, small);
+      s = mfma16(kh, qs[j].h, s);
+    }
+    interleave(std::integral_constant<int, 3 * D / 16>(), std::integral_constant<int, 6 * D / 16>());
+    more = at_v.advance(a, b, h, KW);
+    load_tile(at_v, at_v.vb, vreg);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] += small[r];
+    if (__builtin_expect(valid < kTile, 0)) {
+      asm volatile("" ::: "memory");   // keeps this a real branch
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        vf[r] = *reinterpret_cast<const vvec*>(p + (int64_t)(8 * (r >> 2) + (r & 3)) * ss + lane_off);
-    } else {
-      // (both pointers in the global address space, or the loads become flat ones)
-      typedef const __attribute__((address_space(1))) vvec* Row;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = k0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-        const Row row = (Row)(vb + (int64_t)min(key, len - 1) * ss + kNB * col);
-        vf[r] = *(key < len ? row : (Row)kZeroRow);
-      }
-    }
-  };
-
-  bool more = advance(kpart);
-  if (more) load_k();
-  while (more) {
-    load_v();
-    __builtin_amdgcn_sched_barrier(0);   // V is on its way before the score MFMAs start
-    const int valid = len - k0;
-    f32x16 s, s_odd;   // two chains: an MFMA that waits for the one before it leaves the pipe idle (D = 64: +12 %)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = s_odd[r] = 0.f;
-#pragma unroll
-    for (int j = 0; j < kKL; ++j)
-#pragma unroll
-      for (int t = 0; t < 4; t += 2) {
-        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][t], qf[j][t], s, 0, 0, 0);
-        s_odd = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][t + 1], qf[j][t + 1], s_odd, 0, 0, 0);
-      }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] += s_odd[r];
-    __builtin_amdgcn_sched_barrier(0);
-    more = advance(KW);
-    // The next tile's K is on its way before the P V MFMAs (behind the last tile: some K again).  Without a branch:
-    // with one, V could only be awaited together with this K.
-    load_k();
-    __builtin_amdgcn_sched_barrier(0);
-    if (valid < kTile) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + 4 * hh + (r & 3) >= valid) s[r] = -INFINITY;
+        if (16 * (r >> 3) + 8 * hh + (r & 7) >= valid) s[r] = -INFINITY;
     }
     float mx = s[0];
 #pragma unroll
     for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mx, __shfl_xor(mx, 32));
-    if (__any(mx > m)) {
-      const float m_new = fmaxf(m, mx);
-      const float alpha = __builtin_amdgcn_exp2f((m - m_new) * c);   // (0 on the first tile, or 1 with nothing to rescale)
-      l *= alpha;
-#pragma unroll
-      for (int i = 0; i < kNB; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
-      m = m_new;
-    }
+    // The reference is the next multiple of a.grid (a power of two, 2 to 4 in the exponent): rows, groups and parts of one magnitude have
+    // the same one, and their sums meet with weights that are exactly 1.
+    const float m_new = fmaxf(m, ceilf(mx * a.inv_grid) * a.grid);
+    const float alpha = __builtin_amdgcn_exp2f((m - m_new) * c);   // (0 on the first tile, or 1 with nothing to rescale)
+    m = m_new;
     // the difference first, then the scale: the exponent is exact to its own rounding however large the scores are
+    float sum[2] = {0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       s[r] = __builtin_amdgcn_exp2f((s[r] - m) * c);
-      l += s[r];
+      sum[r & 1] += s[r];
     }
+    l = fmaf(l, alpha, sum[0] + sum[1]);
+    Split8 ps[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float p[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = s[8 * g + e];
+      ps[g] = split8(p);
+    }
+    tile_barrier();
+    // V of this tile is in the LDS, and nobody reads its K any more
+    // The tile's share of O^T is summed for itself, the small terms first: one rounding at the magnitude of O^T per tile.
+#pragma unroll
+    for (int i = 0; i < kNB; i += 2) {
+      bf16x8 vf[3][2][2];   // (as K: before the split of the next K)
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) vf[p][g][e] = v_frag(p, i + e, g);
+      if (i == 0) put_k();
+      f32x16 t[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t[0][r] = t[1][r] = 0.f;
+      auto term = [&](int plane, const bf16x8 (&p)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) t[e] = mfma16(vf[plane][g][e], p[g], t[e]);
+      };
+      const bf16x8 ph[2] = {ps[0].h, ps[1].h}, pm[2] = {ps[0].m, ps[1].m}, pl[2] = {ps[0].l, ps[1].l};
+      term(2, ph);
+      term(0, pl);
+      term(1, pm);
+      term(1, ph);
+      term(0, pm);
+      term(0, ph);
+      if (i == 0) interleave(std::integral_constant<int, 24>(), std::integral_constant<int, 24>());
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i + e][r] = fmaf(o[i + e][r], alpha, t[e][r]);
+    }
+    at_k.advance(a, b, h, KW);
+    load_tile(at_k, at_k.kb, kreg);
+    tile_barrier();
+  }
+  l += __shfl_xor(l, 32);
+
+  // ---- epilogue: O^T -> LDS as [query][d] (the tiles' place), then whole rows to memory; the groups are folded on the way
+  float* mine = reinterpret_cast<float*>(lds_f32) + wave * L::kFloatsPerWave;
+  uint32_t worst = 0;
+#pragma unroll
+  for (int i = 0; i < kNB; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = o[i][4 * g + e];
+        worst = max(worst, oddity(x[e]));
+      }
+      *reinterpret_cast<f32x4*>(mine + col * L::kPitch + 32 * i + 8 * g + 4 * hh) = x;
+    }
+  const bool odd_row = odd_q || !(l < INFINITY);
+  if (__builtin_expect(any && __any(odd_row || worst >= kOddFrom), 0)) {
+    // Once more with fp32 products, for the elements and rows that need it; the others stay what they are.
+    float m2, l2;
+    walk_fp32<D, kFar>(a, b, h, job, q0, begin + group, KW, n_tiles, o, m2, l2);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const bool whole_row = odd_row || __shfl_xor((int)odd_row, 32) != 0;
+    const float f = __builtin_amdgcn_exp2f((m2 - m) * c);
 #pragma unroll
     for (int r = 0; r < 16; ++r)
 #pragma unroll
       for (int i = 0; i < kNB; ++i) {
-        float vi;
-        if constexpr (kNB == 2) vi = i == 0 ? vf[r].x : vf[r].y;
-        else vi = vf[r][i];
-        o[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(vi, s[r], o[i], 0, 0, 0);
+        float* x = mine + col * L::kPitch + (8 * (r >> 2) + 4 * hh + (r & 3)) * kNB + i;
+        if (whole_row) *x = o[i][r];
+        else if (oddity(*x) >= kOddFrom) *x = o[i][r] * f;
       }
-  }
-  l += __shfl_xor(l, 32);
-
-  // ---- epilogue: O^T -> LDS as [query][d], then whole rows to memory; with KW > 1 the parts are folded on the way
-  float* mine = lds_f32 + wave * L::kFloatsPerWave;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    vvec row;
-#pragma unroll
-    for (int i = 0; i < kNB; ++i) row[i] = o[i][r];
-    *reinterpret_cast<vvec*>(mine + col * L::kPitch + (8 * (r >> 2) + 4 * hh + (r & 3)) * kNB) = row;
+    if (whole_row) {
+      m = m2;
+      l = l2;
+    }
   }
   if (hh == 0) {
     mine[kTile * L::kPitch + col] = m;
@@ -253,62 +617,189 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   }
   if constexpr (KW > 1) __syncthreads();
   else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // a wavefront reads back only what it wrote itself
-  const float* parts = lds_f32 + (wave - kpart) * L::kFloatsPerWave;
-  constexpr int kLanesPerRow = D / 4;
-  constexpr int kRowsPerPass = 64 / kLanesPerRow;
+  const float* halves = reinterpret_cast<float*>(lds_f32) + member * L::kFloatsPerWave;   // group g: QW wavefronts on
   constexpr int kRowsPerWave = kTile / KW;
-  float* out = a.out[job];
-  float* lse = a.lse[job];
+  // `row` of the workgroup's 32 QW
+  auto store_row = [&](int row, const float (&acc)[4], float den, float mm) __attribute__((always_inline)) {
+    const int q = qg * QW * kTile + row;
+    if (q >= a.Sq) return;
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+    f32x4 y;
 #pragma unroll
-  for (int p = 0; p < kRowsPerWave; p += kRowsPerPass) {
-    const int row = kpart * kRowsPerWave + p + lane / kLanesPerRow;
-    const int d = (lane % kLanesPerRow) * 4;
+    for (int e = 0; e < 4; ++e) y[e] = acc[e] * inv;
+    *reinterpret_cast<f32x4*>(a.job[job].out + (((int64_t)b * a.Sq + q) * a.H + h) * D + d_mine) = y;
+    if (d_mine == 0)
+      a.job[job].lse[a.lse_bsh ? ((int64_t)b * a.Sq + q) * a.H + h : ((int64_t)b * a.H + h) * a.Sq + q] =
+          lse_of(mm, den, a.scale);
+  };
+  const int64_t n_rows = (int64_t)(gridDim.y / a.parts) * a.total * (QW * kTile);   // of a part, all jobs
+  const int64_t sums = n_rows * a.parts * D;
+  auto part_row = [&](int p) { return p * n_rows + ((int64_t)job * a.total + item) * (QW * kTile); };
+#pragma unroll 1
+  for (int p = 0; p < kRowsPerWave; p += kRowsPer) {
+    const int row = group * kRowsPerWave + p + lane / kRowLanes;
     float mm = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < KW; ++w) mm = fmaxf(mm, parts[w * L::kFloatsPerWave + kTile * L::kPitch + row]);
+    for (int w = 0; w < KW; ++w) mm = fmaxf(mm, halves[w * QW * L::kFloatsPerWave + kTile * L::kPitch + row]);
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     float den = 0.f;
 #pragma unroll
     for (int w = 0; w < KW; ++w) {
-      const float* pw = parts + w * L::kFloatsPerWave;
+      const float* pw = halves + w * QW * L::kFloatsPerWave;
       const float lw = pw[kTile * L::kPitch + kTile + row];
       const float ww = KW == 1 ? 1.f : (lw == 0.f ? 0.f : __builtin_amdgcn_exp2f((pw[kTile * L::kPitch + row] - mm) * c));
-      const f32x4 x = *reinterpret_cast<const f32x4*>(pw + row * L::kPitch + d);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(pw + row * L::kPitch + d_mine);
       den = fmaf(ww, lw, den);
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] = fmaf(ww, x[e], acc[e]);
     }
-    if (q0 + row < a.Sq) {
-      const float inv = den > 0.f ? 1.f / den : 0.f;
-      f32x4 y;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) y[e] = acc[e] * inv;
-      *reinterpret_cast<f32x4*>(out + (((int64_t)b * a.Sq + q0 + row) * a.H + h) * D + d) = y;
-      if (d == 0) lse[((int64_t)b * a.H + h) * a.Sq + q0 + row] = den > 0.f ? mm * a.scale + logf(den) : -INFINITY;
+    if (a.parts == 1) {
+      store_row(row + member * kTile, acc, den, mm);
+    } else {
+      // past the L2, for the workgroup that folds (see attn_fwd.hip, "states that meet inside a launch")
+      const int at = member * kTile + row;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{acc[0], acc[1], acc[2], acc[3]}),
+                                             buffer_of(a.ws + part_row(part) * D, QW * kTile * D * 4), (at * D + d_mine) * 4, 0, kDevice);
+      if (d_mine == 0) {
+        float* ml = a.ws + sums + 2 * (part_row(part) + at);
+        __hip_atomic_store(ml, mm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(ml + 1, den, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
   }
+  if (a.parts == 1) return;
+
+  // ---- the workgroup that is the last of its item to get here folds the parts
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  uint32_t* last = reinterpret_cast<uint32_t*>(lds_f32);
+  if (threadIdx.x == 0) {
+    uint32_t* counter = a.arrive + (int64_t)job * a.total + item;
+    const bool mine_is = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (uint32_t)a.parts;
+    if (mine_is) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *last = mine_is;
+  }
+  __syncthreads();
+  if (*last == 0) return;
+  __syncthreads();
+  constexpr int kRows = kTile * QW;
+  constexpr int kSteps = kRows / (kWavesF32 * kRowsPer);   // rows of a lane
+  constexpr int kBatch = 16 / kSteps;                      // parts whose sums are on their way together
+  auto row_of = [&](int i) { return (i * kWavesF32 + wave) * kRowsPer + lane / kRowLanes; };
+  f32x4 x[kBatch][kSteps];
+  auto load_sums = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      // (behind the last part an empty buffer: zeros, no memory is touched)
+      const Rsrc src = buffer_of(a.ws + part_row(min(p + j, a.parts - 1)) * D, p + j < a.parts ? kRows * D * 4 : 0);
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i)
+        x[j][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(src, (row_of(i) * D + d_mine) * 4, 0, kDevice));
+    }
+  };
+  float* weights = reinterpret_cast<float*>(lds_f32) + 2 * kRows;   // [part][query]; in front of them (maximum, sum) of every query
+  load_sums(0);
+  if (threadIdx.x < kRows) {   // a thread, a query
+    f32x2 ml[kMaxParts];
+#pragma unroll
+    for (int p = 0; p < kMaxParts; ++p)
+      ml[p] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                                            buffer_of(a.ws + sums + 2 * part_row(min(p, a.parts - 1)), p < a.parts ? kRows * 8 : 0),
+                                            threadIdx.x * 8, 0, kDevice));
+    float mm = -INFINITY, den = 0.f;
+#pragma unroll
+    for (int p = 0; p < kMaxParts; ++p) mm = p < a.parts ? fmaxf(mm, ml[p].x) : mm;
+#pragma unroll
+    for (int p = 0; p < kMaxParts; ++p) {
+      const float w = ml[p].y == 0.f ? 0.f : __builtin_amdgcn_exp2f((ml[p].x - mm) * c);   // (no part, no sum)
+      den = fmaf(w, ml[p].y, den);
+      weights[p * kRows + threadIdx.x] = w;
+    }
+    weights[(int)threadIdx.x - 2 * kRows] = mm;
+    weights[(int)threadIdx.x - kRows] = den;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  float acc[kSteps][4];
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i) acc[i][0] = acc[i][1] = acc[i][2] = acc[i][3] = 0.f;
+  for (int p = 0; p < a.parts; p += kBatch) {
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j)
+#pragma unroll
+      for (int i = 0; i < kSteps; ++i) {
+        const float w = weights[(p + j) * kRows + row_of(i)];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(w, x[j][i][e], acc[i][e]);
+      }
+    if (p + kBatch < a.parts) load_sums(p + kBatch);
+  }
+#pragma unroll
+  for (int i = 0; i < kSteps; ++i)
+    store_row(row_of(i), acc[i], weights[row_of(i) - kRows], weights[row_of(i) - 2 * kRows]);
 }
 
-template <int D, int KW>
+template <int D, int QW, bool kFar>
 int launch_f32(AttnF32Args& a, int n_jobs, hipStream_t stream) {
   // more than 64 KB of dynamic LDS has to be allowed once per kernel and device
   static thread_local int allowed_dev = -1;
+  constexpr int kLds = F32Lds<D, QW>::kBytes;
   int dev = 0;
   if (int rc = hip_fail(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (allowed_dev != dev) {
-    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<D, KW>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, F32Lds<D>::kBytes),
+    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_f32_kernel<D, QW, kFar>),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
                           "hipFuncSetAttribute"))
       return rc;
     allowed_dev = dev;
   }
-  constexpr int kQueries = kTile * kWavesF32 / KW;
-  a.n_qg = (a.Sq + kQueries - 1) / kQueries;
-  a.total = a.B * a.H * a.n_qg;
-  a.per_xcd = (a.total + 7) / 8;
-  hipLaunchKernelGGL((attn_f32_kernel<D, KW>), dim3((unsigned)a.per_xcd * 8u, (unsigned)n_jobs, 1), dim3(kThreadsF32),
-                     F32Lds<D>::kBytes, stream, a);
+  hipLaunchKernelGGL((attn_f32_kernel<D, QW, kFar>), dim3((unsigned)a.per_xcd * 8u, (unsigned)(n_jobs * a.parts), 1), dim3(kThreadsF32),
+                     kLds, stream, a);
   return hip_fail(hipGetLastError(), "attn_f32 launch");
+}
+
+// Query tiles of a workgroup and workgroups that share the keys of a work item.  What a launch takes, in us: its rounds of workgroups
+// times the turns of one times what a turn takes (one workgroup on a CU, and at d = 64 two), and what a workgroup costs on top: start, end,
+// and the fold of the parts.  Four query tiles a workgroup split K and V half as often as two, but fold twice the bytes and leave a
+// small launch fewer workgroups.  The constants are fitted to 22 launches of 1 ... 12 heads x 96 ... 1680 queries against 2 ... 8
+// chunks of as many keys, in every split up to 16 (300 timings): the plan takes at most 2.8 % more than the best of them, 0.3 % on average.
+// us unsplit, -> as planned: 4 heads x 512 queries x 2048 keys, d = 64 67 -> 21 (8 parts); 12 x 1680 x 3360, d = 64 168 -> 111 (3 parts
+// of 4 query tiles); 10 x 847 x 1694, d = 128 111 -> 73 (3 of 4); 2 x 553 x 4424, d = 128 152 -> 53 (8).
+struct F32Plan {
+  int qw = 2, parts = 1;
+};
+struct F32Cost {
+  double one, two, base, fold;   // a turn alone, beside another workgroup's; a launch; a part
+};
+F32Plan plan_f32(int D, int heads, int Sq, int n_jobs, int tiles, int64_t workspace_bytes, int64_t n_counters) {
+  constexpr F32Cost kCost[2][2] = {{{1.45, 3.15, 14.0, 0.15}, {1.4, 2.66, 14.5, 0.5}}, {{3.15, 0, 17.0, 0.3}, {2.6, 0, 23.0, 0.6}}};
+  constexpr int64_t kCus = 32;   // of an XCD
+  F32Plan best;
+  double least = 1e30;
+  for (int qw = 2; qw <= 4; qw += 2) {
+    const F32Cost& t = kCost[D == 128][qw == 4];
+    const int64_t items = (int64_t)heads * ((Sq + kTile * qw - 1) / (kTile * qw)) * n_jobs, per_xcd = (items + 7) / 8;
+    const int kw = kWavesF32 / qw;
+    for (int parts = 1; parts <= kMaxParts; ++parts) {
+      if (parts > 1 && (parts * kw > tiles || items > n_counters || items * parts * (kTile * qw) * (D + 2) * 4 > workspace_bytes)) break;
+      const double turns = (tiles + kw * parts - 1) / (kw * parts);
+      const int64_t groups = per_xcd * parts;
+      double time = t.base + (parts > 1 ? 1.0 + t.fold * parts : 0.0);
+      if (D == 128) {
+        const int64_t rounds = (groups + kCus - 1) / kCus;
+        time += rounds * turns * t.one + (rounds - 1) * 7.0;
+      } else {
+        const int64_t full = groups / (2 * kCus), rest = groups % (2 * kCus);
+        time += full * turns * t.two + (rest == 0 ? 0.0 : rest <= kCus ? turns * t.one : turns * t.two);
+        time += (full + (rest > 0) - 1) * 2.5;
+      }
+      if (time < least) {
+        least = time;
+        best.qw = qw;
+        best.parts = parts;
+      }
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -316,12 +807,13 @@ int launch_f32(AttnF32Args& a, int n_jobs, hipStream_t stream) {
 
 using namespace dt;
 
-extern "C" int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb, int64_t q_ss,
+extern "C" int dt_attn_jobs_f32_ws_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb, int64_t q_ss,
                                     int64_t q_sh, int32_t n_chunks, const float* const* k_ptrs,
                                     const float* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
                                     const int64_t* kv_ss, const int64_t* kv_sh, int32_t n_jobs, const int32_t* job_begin,
                                     const int32_t* job_chunks, float* const* out_ptrs, float* const* lse_ptrs,
-                                    float softmax_scale, void* stream) {
+                                    int32_t lse_layout, float softmax_scale, void* workspace, int64_t workspace_bytes, uint32_t* counters,
+                                    int64_t n_counters, void* stream) {
   if (B <= 0 || Sq <= 0 || H <= 0) {
     set_error("B, Sq, H must be positive (got %d, %d, %d)", B, Sq, H);
     return DT_ERR_INVALID;
@@ -347,16 +839,21 @@ extern "C" int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32
   AttnF32Args a{};
   a.q = q;
   a.q_sb = q_sb; a.q_ss = q_ss; a.q_sh = q_sh;
-  a.B = B; a.H = H; a.Sq = Sq;
+  a.B = B; a.H = H; a.Sq = Sq; a.D = D;
+  a.parts = 1;
   a.scale = softmax_scale > 0.f ? softmax_scale : 1.0f / std::sqrt((float)D);
   a.scale_log2 = a.scale * 1.4426950408889634f;
+  a.grid = std::exp2(std::floor(std::log2(4.f / a.scale_log2)));
+  a.inv_grid = 1.f / a.grid;
+  bool far = false;
   for (int i = 0; i < n_chunks; ++i) {
     if (kv_lens[i] < 0 || (kv_lens[i] > 0 && (!k_ptrs[i] || !v_ptrs[i]))) {
       set_error("chunk %d: negative length or null k/v", i);
       return DT_ERR_INVALID;
     }
-    a.k[i] = k_ptrs[i]; a.v[i] = v_ptrs[i];
-    a.kv_len[i] = kv_lens[i]; a.kv_sb[i] = kv_sb[i]; a.kv_ss[i] = kv_ss[i]; a.kv_sh[i] = kv_sh[i];
+    a.chunk[i] = {k_ptrs[i], v_ptrs[i], kv_sb[i], kv_ss[i], kv_sh[i], kv_lens[i]};
+    // (a chunk's keys of one batch and head beyond 2 GiB, or in falling order: 64-bit offsets, slower)
+    far = far || kv_ss[i] < 0 || (kv_lens[i] > 0 && (uint64_t)kv_ss[i] > (1ull << 29) / ((uint64_t)kv_lens[i] + kTile));
   }
   if (job_begin[0] != 0) {
     set_error("job_begin must start at 0");
@@ -371,29 +868,51 @@ extern "C" int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32
       set_error("job %d: null destination", j);
       return DT_ERR_INVALID;
     }
-    a.out[j] = out_ptrs[j]; a.lse[j] = lse_ptrs[j];
-    a.job_begin[j] = job_begin[j];
+    a.job[j] = {out_ptrs[j], lse_ptrs[j], job_begin[j], job_begin[j + 1]};
   }
-  a.job_begin[n_jobs] = job_begin[n_jobs];
   for (int e = 0; e < job_begin[n_jobs]; ++e) {
     if (job_chunks[e] < 0 || job_chunks[e] >= n_chunks) {
       set_error("job chunk reference %d is outside the chunk table", job_chunks[e]);
       return DT_ERR_INVALID;
     }
-    a.job_chunks[e] = job_chunks[e];
+    a.refs[e] = job_chunks[e];
   }
-  // One wavefront per SIMD takes 1024 query tiles.  Below three such rounds the last one is rarely full and splitting
-  // the keys four ways fills it (12 heads x 2048 queries x 2 chunks, 1536 tiles: 270 instead of 346 us at d = 64, 479
-  // instead of 601 at d = 128; 256 tiles: 40 instead of 110 us); from there on four query tiles that read the same keys
-  // are the better neighbours in a workgroup (3072 tiles: 500 each at d = 64, 908 instead of 954 us at d = 128).
-  // The line holds for chunks of 256 keys and more.  A wavefront with a tile or less pays for the exchange of the parts without a
-  // shorter loop: 24 heads x 2048 queries x 512 keys 79 split, 96 us unsplit at d = 64, 153 and 165 at d = 128, but x 64 keys 27 and 21,
-  // 60 and 39.  Short chunks are launches of tens of us either way and up to 512 query tiles split well too (4 heads x 512 x 64 keys
-  // 6.8 and 10.7 us), so the number of keys is left out of the rule.
-  const bool split = units * n_jobs < 3 * 1024;
-  if (D == 128)
-    return split ? launch_f32<128, 4>(a, n_jobs, (hipStream_t)stream) : launch_f32<128, 1>(a, n_jobs, (hipStream_t)stream);
-  return split ? launch_f32<64, 4>(a, n_jobs, (hipStream_t)stream) : launch_f32<64, 1>(a, n_jobs, (hipStream_t)stream);
+  if (lse_layout != DT_LSE_BHS && lse_layout != DT_LSE_BSH) {
+    set_error("unknown lse layout %d", lse_layout);
+    return DT_ERR_INVALID;
+  }
+  a.lse_bsh = lse_layout == DT_LSE_BSH;
+  int tiles = 0;
+  for (int j = 0; j < n_jobs; ++j) {
+    int64_t n = 0;
+    for (int e = job_begin[j]; e < job_begin[j + 1]; ++e) n += ((int64_t)kv_lens[job_chunks[e]] + kTile - 1) / kTile;
+    tiles = std::max(tiles, (int)std::min<int64_t>(n, INT32_MAX / 2));
+  }
+  const bool scratch = workspace && counters && !far;
+  const F32Plan plan = plan_f32(D, B * H, Sq, n_jobs, tiles, scratch ? workspace_bytes : 0, scratch ? n_counters : 0);
+  const int qw = far ? 2 : plan.qw;
+  a.parts = plan.parts;
+  a.n_qg = (Sq + kTile * qw - 1) / (kTile * qw);
+  a.total = B * H * a.n_qg;
+  a.per_xcd = (a.total + 7) / 8;
+  a.ws = static_cast<float*>(workspace);
+  a.arrive = counters;
+  hipStream_t s = (hipStream_t)stream;
+  std::unique_lock<std::mutex> lock;   // (another thread's parts, on the same stream and workspace, may wait for a fold kernel)
+  if (a.parts > 1) lock = std::unique_lock<std::mutex>(workspace_lock(workspace));
+  if (far) return D == 128 ? launch_f32<128, 2, true>(a, n_jobs, s) : launch_f32<64, 2, true>(a, n_jobs, s);
+  if (D == 128) return qw == 2 ? launch_f32<128, 2, false>(a, n_jobs, s) : launch_f32<128, 4, false>(a, n_jobs, s);
+  return qw == 2 ? launch_f32<64, 2, false>(a, n_jobs, s) : launch_f32<64, 4, false>(a, n_jobs, s);
+}
+
+extern "C" int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb, int64_t q_ss,
+                                    int64_t q_sh, int32_t n_chunks, const float* const* k_ptrs,
+                                    const float* const* v_ptrs, const int32_t* kv_lens, const int64_t* kv_sb,
+                                    const int64_t* kv_ss, const int64_t* kv_sh, int32_t n_jobs, const int32_t* job_begin,
+                                    const int32_t* job_chunks, float* const* out_ptrs, float* const* lse_ptrs,
+                                    float softmax_scale, void* stream) {
+  return dt_attn_jobs_f32_ws_fwd(q, B, Sq, H, D, q_sb, q_ss, q_sh, n_chunks, k_ptrs, v_ptrs, kv_lens, kv_sb, kv_ss, kv_sh, n_jobs, job_begin,
+                                 job_chunks, out_ptrs, lse_ptrs, DT_LSE_BHS, softmax_scale, nullptr, 0, nullptr, 0, stream);
 }
 
 extern "C" int dt_attn_chunk_f32_fwd(const float* q, const float* k, const float* v, float* out, float* lse, int32_t B,

@@ -1804,10 +1804,7 @@ static TailPlan plan_launch(AttnArgs& a, int D, int n_jobs, JobSize* size, int c
   return best;
 }
 
-// Held while a launch that writes partial states, and the fold kernel where there is one, go into the queue: two threads may
-// launch on one stream, with the workspace that belongs to it, and no parts of the other's may come between the parts and their
-// fold.  (One of a few locks, chosen by the workspace: a thread that waits for room in its stream's queue holds up few others.)
-static std::mutex& workspace_lock(const void* workspace) {
+std::mutex& workspace_lock(const void* workspace) {
   constexpr int kBits = 6;
   static std::mutex locks[1 << kBits];
   return locks[(reinterpret_cast<uintptr_t>(workspace) >> 4) * 0x9e3779b97f4a7c15ull >> (64 - kBits)];

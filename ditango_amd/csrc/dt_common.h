@@ -4,6 +4,8 @@
 #include <stdint.h>
 #include "ditango_hip.h"
 
+#include <mutex>
+
 namespace dt {
 
 void set_error(const char* fmt, ...);
@@ -139,6 +141,10 @@ static_assert(DT_MAX_CHUNKS % kMergeBatch == 0 && DT_MAX_MERGE_LIST % kMergeBatc
 static_assert(DT_MAX_MERGE_LIST * sizeof(AttnState) <= DT_MAX_CHUNKS * sizeof(int32_t*), "the list shares the boundaries' place");
 static_assert(sizeof(AttnArgs) <= 4096, "the kernel arguments travel in the 4 KB kernarg segment");
 
+// Held while a launch that writes partial states, and the fold kernel where there is one, go into the queue: two threads may
+// launch on one stream, with the workspace that belongs to it, and no parts of the other's may come between the parts and their
+// fold.  (One of a few locks, chosen by the workspace: a thread that waits for room in its stream's queue holds up few others.)
+std::mutex& workspace_lock(const void* workspace);
 // Whether a merging launch of these sizes may merge itself (see merges_in_launch).
 bool may_merge_in_launch(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles);
 int launch_attn(const AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace = nullptr,

@@ -470,9 +470,12 @@ std::tuple<States, Tensor, Tensor> attn_states_merge(
 }
 
 // The fp32 states of fp32 q against the concatenations of the fp32 chunks jobs[j] (ditango_amd._hip.attn_jobs_f32_fwd); every
-// chunk may have strides of its own.
+// chunk may have strides of its own.  bsh: lse as [B,Sq,H,1].
 States attn_states_f32(const Tensor& q, const std::vector<Tensor>& ks, const std::vector<Tensor>& vs,
-                       const std::vector<std::vector<int32_t>>& jobs, double scale, uint64_t stream) {
+                       const std::vector<std::vector<int32_t>>& jobs, double scale, uint64_t stream, bool bsh,
+                       const std::optional<Tensor>& workspace, const std::optional<Tensor>& counters) {
+  REQUIRE(!counters || (counters->is_cuda() && counters->scalar_type() == at::kInt && counters->is_contiguous()),
+          "counters must be int32 on the GPU");
   auto check_f32 = [](const Tensor& t, const Name& name) {
     REQUIRE(t.is_cuda() && t.scalar_type() == at::kFloat && t.dim() == 4 && t.stride(3) == 1, name.str(),
             " must be fp32 [B,S,H,D] on the GPU with contiguous D");
@@ -488,7 +491,7 @@ States attn_states_f32(const Tensor& q, const std::vector<Tensor>& ks, const std
   }
   States states;
   for (size_t j = 0; j < jobs.size(); ++j) {
-    states.emplace_back(new_out(d, at::kFloat, q), new_lse(d, false, q));
+    states.emplace_back(new_out(d, at::kFloat, q), new_lse(d, bsh, q));
     for (int32_t c : jobs[j]) REQUIRE(c >= 0 && (size_t)c < ks.size(), "job ", std::to_string(j), " references a chunk outside the table");
   }
   for (size_t start = 0; start < jobs.size();) {
@@ -521,8 +524,9 @@ States attn_states_f32(const Tensor& q, const std::vector<Tensor>& ks, const std
       lp[n] = static_cast<float*>(ptr(states[start + n].second));
     }
     REQUIRE(n > 0, "job ", std::to_string(start), " references more chunks than one launch addresses: split it and merge the parts");
-    CALL(dt_attn_jobs_f32_fwd, static_cast<const float*>(ptr(q)), d.B, d.S, d.H, d.D, q.stride(0), q.stride(1), q.stride(2),
-         nc, kp, vp, lens, sb, ss, sh, n, begin, chunks, op, lp, (float)scale, stream_of(stream));
+    CALL(dt_attn_jobs_f32_ws_fwd, static_cast<const float*>(ptr(q)), d.B, d.S, d.H, d.D, q.stride(0), q.stride(1), q.stride(2),
+         nc, kp, vp, lens, sb, ss, sh, n, begin, chunks, op, lp, bsh ? DT_LSE_BSH : DT_LSE_BHS, (float)scale, ptr(workspace),
+         bytes_of(workspace), static_cast<uint32_t*>(ptr(counters)), counters ? counters->numel() : 0, stream_of(stream));
     start += n;
   }
   return states;
@@ -778,7 +782,8 @@ PYBIND11_MODULE(_ditango_host, m) {
     return attn_states(q, ks, vs, jobs, max_chunks, cu_q, cu_kv, workspace, flags, seg, convert, stream);
   });
   m.def("attn_states_merge", &attn_states_merge);
-  m.def("attn_states_f32", &attn_states_f32);
+  m.def("attn_states_f32", &attn_states_f32, py::arg("q"), py::arg("ks"), py::arg("vs"), py::arg("jobs"), py::arg("scale"), py::arg("stream"),
+        py::arg("bsh") = false, py::arg("workspace") = py::none(), py::arg("counters") = py::none());
   m.def("attn_sched", [](const Tensor& q, const ChunkTable& table, const Tensor& ids, const Tensor& count, int64_t row, int32_t max_jobs,
                          const Tensor& slot_out, const Tensor& slot_lse, int32_t diag, const std::optional<Tensor>& diag_out,
                          const std::optional<Tensor>& diag_lse, double scale, const std::optional<std::vector<Range>>& seg_q,

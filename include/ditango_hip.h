@@ -91,8 +91,8 @@ int dt_attn_chunk_f16_fwd(const void* q, const void* k, const void* v, void* out
                           float softmax_scale, void* stream);
 
 /*
- * The same call site (core/attention.py:185-191) for fp32 tensors, computed in fp32 throughout (fp32 matrix
- * instructions, fp32 exponentials): the attention of the fp32 numbers themselves, not of their bf16 roundings.
+ * The same call site (core/attention.py:185-191) for fp32 tensors, computed to fp32 throughout (products exact to fp32 rounding,
+ * fp32 sums and exponentials): the attention of the fp32 numbers themselves, not of their bf16 roundings.
  * flash_attn_func takes no fp32; the
  * reference runs its CPU-runnable configuration (fp32, B=1, H=4, d=64, 512 queries x 4 chunks of
  * 512 keys) on its torch math path, and this entry point is that path's counterpart here.  q / k / v
@@ -118,6 +118,23 @@ int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32
                          const int64_t* kv_stride_h, int32_t n_jobs, const int32_t* job_begin,
                          const int32_t* job_chunks, float* const* out_ptrs, float* const* lse_ptrs,
                          float softmax_scale, void* stream);
+
+/*
+ * dt_attn_jobs_f32_fwd with lse in a layout of choice (DT_LSE_BHS, or DT_LSE_BSH: the running layout [B,Sq,H,1] of
+ * utils.py:49, so that a job over all chunks of a call is the call's result, core/attention.py:185-196) and with scratch: where
+ * the queries alone leave the GPU idle, the key tiles of a job are shared by several workgroups, which put partial sums into the
+ * workspace; the last one folds them.  workspace: device memory, 16-byte aligned, used up to workspace_bytes.  counters: n_counters words of
+ * device memory that are zero; every launch leaves them at zero.  Launches that share either must not overlap on the GPU.
+ * Without them, or where they are too few, as dt_attn_jobs_f32_fwd.
+ */
+int dt_attn_jobs_f32_ws_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
+                            int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
+                            int32_t n_chunks, const float* const* k_ptrs, const float* const* v_ptrs,
+                            const int32_t* kv_lens, const int64_t* kv_stride_b, const int64_t* kv_stride_s,
+                            const int64_t* kv_stride_h, int32_t n_jobs, const int32_t* job_begin,
+                            const int32_t* job_chunks, float* const* out_ptrs, float* const* lse_ptrs,
+                            int32_t lse_layout, float softmax_scale, void* workspace, int64_t workspace_bytes,
+                            uint32_t* counters, int64_t n_counters, void* stream);
 
 /*
  * Several attention states in one launch.  Job j attends q to the

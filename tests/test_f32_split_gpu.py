@@ -1,0 +1,86 @@
+"""fp32 attention on the bf16 matrix pipe: both widths of a workgroup, keys shared by several workgroups, numbers that do not split."""
+import pytest
+import torch
+
+from oracle import attention_math as om
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(hip, q, ks, vs, jobs, bsh, bound=1e-5):
+    """Against the closed form in fp64, 1e-5 as for the other fp32 tests: sums of at most some thousand terms in fp32."""
+    got = hip.attn_jobs_f32_fwd(q.cuda(), [k.cuda() for k in ks], [v.cuda() for v in vs], jobs, lse_bsh=bsh)
+    torch.cuda.synchronize()
+    for job, (out, lse) in zip(jobs, got):
+        k, v = (torch.cat([t[c] for c in job] or [t[0][:, :0]], 1) for t in (ks, vs))
+        lse = lse.squeeze(-1).transpose(1, 2) if bsh else lse
+        if k.shape[1] == 0:
+            assert (out == 0).all() and torch.isneginf(lse).all()
+            continue
+        ref_out, ref_lse = om.chunk_attention(q, k, v, compute_dtype=torch.float64)
+        scale = v.abs().max().item()
+        assert (out.double().cpu() - ref_out).abs().max().item() <= bound * scale, job
+        assert (lse.double().cpu() - ref_lse).abs().max().item() <= bound, job
+    return got
+
+
+@pytest.mark.parametrize("B,Sq,H,D,lens,jobs,bsh", [
+    (1, 1, 1, 64, [1], [[0]], True),                                   # one query, one key
+    (1, 65, 2, 64, [31, 0, 33, 70, 1], [[0, 1, 2, 3, 4, 0]], True),    # chunks that end inside tiles, an empty one, one twice
+    (1, 33, 1, 128, [1030], [[0]], True),                              # 33 tiles in parts that do not divide them
+    (2, 129, 3, 128, [64, 65], [[0, 1], [1], []], False),              # jobs of unequal length, one without keys
+    (1, 512, 4, 64, [512, 512, 512, 512], [[0, 1, 2, 3]], True),       # 8 parts
+    (1, 700, 12, 64, [700, 701], [[0, 1]], True),                      # four query tiles a workgroup
+    (1, 847, 10, 128, [847, 846], [[0, 1]], False),
+])
+def test_split_products_match_fp64_closed_form(hip, B, Sq, H, D, lens, jobs, bsh):
+    g = torch.Generator().manual_seed(Sq + D)
+    q = torch.randn(B, Sq, H, D, generator=g)
+    ks, vs = ([torch.randn(B, n, H, D, generator=g) for n in lens] for _ in range(2))
+    _check(hip, q, ks, vs, jobs, bsh)
+
+
+@pytest.mark.parametrize("D,q_scale,k_scale,v_scale", [
+    (64, 2.0 ** 100, 2.0 ** -100, 1.0),      # the low parts of K end below the exponent range
+    (128, 2.0 ** -110, 2.0 ** 110, 1.0),     # ... of Q
+    (64, 1.0, 1.0, 2.0 ** -118),             # ... of V, and the result is as small
+    (128, 1.0, 1.0, 2.0 ** 100),
+    (64, 1.0, 1.0, 0.0),
+])
+def test_magnitudes_at_the_ends_of_the_range(hip, D, q_scale, k_scale, v_scale):
+    g = torch.Generator().manual_seed(D)
+    q = torch.randn(1, 70, 2, D, generator=g) * q_scale
+    ks, vs = ([torch.randn(1, 300, 2, D, generator=g) * s] for s in (k_scale, v_scale))
+    _check(hip, q, ks, vs, [[0]], True)
+
+
+def test_infinities_in_one_part_of_the_keys(hip):
+    """An infinity of V leaves the other columns, and a key of infinite score the other rows, bit for bit what they are."""
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(1, 96, 2, 64, generator=g)
+    k, v = (torch.randn(1, 1500, 2, 64, generator=g) for _ in range(2))
+    [(want, want_lse)] = hip.attn_jobs_f32_fwd(q.cuda(), [k.cuda()], [v.cuda()], [[0]])
+    v2 = v.clone()
+    v2[0, 1300, 1, 7] = float("-inf")
+    [(out, lse)] = hip.attn_jobs_f32_fwd(q.cuda(), [k.cuda()], [v2.cuda()], [[0]])
+    want = want.clone()
+    want[:, :, 1, 7] = float("-inf")
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+
+
+def test_result_under_graph_capture(hip):
+    """Parts, counters and all: every replay equals the eager call, with other launches of the stream between them."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v = (torch.randn(1, n, 4, 64, generator=g, device="cuda") for n in (200, 2000, 2000))
+    run = lambda: hip.attn_jobs_f32_fwd(q, [k], [v], [[0]], lse_bsh=True)[0]
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, lse = run()
+    for i in range(4):
+        q.copy_(torch.randn(q.shape, generator=g, device="cuda"))
+        graph.replay()
+        want, want_lse = run()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(lse, want_lse), i
