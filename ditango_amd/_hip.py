@@ -333,10 +333,14 @@ class ChunkTable:
     ``convert`` is called on chunks that are neither bf16 nor fp16."""
 
     def __init__(self, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor], batch: int = 0, convert=None):
-        self.native = _host().ChunkTable(list(k_chunks), list(v_chunks), batch, convert)
+        self.native = _host().ChunkTable(k_chunks, v_chunks, batch, convert)
 
-        t = self.native
-        self.n, self.B, self.H, self.D, self.ss, self.sh = t.n, t.B, t.H, t.D, t.ss, t.sh
+    n = property(lambda self: self.native.n)
+    B = property(lambda self: self.native.B)
+    H = property(lambda self: self.native.H)
+    D = property(lambda self: self.native.D)
+    ss = property(lambda self: self.native.ss)
+    sh = property(lambda self: self.native.sh)
 
     def whole(self):
         """ctypes arrays (k_ptrs, v_ptrs, lens, batch strides) of the whole table, for callers of the C ABI."""
@@ -532,37 +536,5 @@ def qk_norm_rope(x: torch.Tensor, *, norm: int = DT_NORM_NONE, weight: Optional[
     ``[rope_end-rope_begin, D]`` or ``[B, rope_end-rope_begin, D]``.  ``out_scale`` multiplies the result
     before its rounding to the output dtype; the ``DT_ROUND_*`` bits round to x's dtype.  weight / bias are fp32, or
     with ``DT_WEIGHTS_16`` in ``rounding`` of x's dtype."""
-    lib = load_library()
-    _require(x.is_cuda and x.dtype in HALF_DTYPES and x.dim() == 4 and x.stride(3) == 1, "x must be bf16 or fp16 [B,S,H,D] on the GPU")
-    B, S, H, D = x.shape
-    if out is None:
-        out = torch.empty((B, S, H, D), dtype=x.dtype, device=x.device)
-    _require(out.is_cuda and out.dtype == x.dtype and out.is_contiguous() and tuple(out.shape) == (B, S, H, D),
-             "out must be a contiguous [B,S,H,D] in x's dtype")
-    rounding = int(rounding) | (DT_IO_FP16 if x.dtype == torch.float16 else 0)
-    w_dtype = x.dtype if rounding & DT_WEIGHTS_16 else torch.float32
-    for name, t in (("weight", weight), ("bias", bias)):
-        _require(t is None or (t.is_cuda and t.dtype == w_dtype and t.is_contiguous() and t.numel() == D),
-                 f"{name} must be {'of the dtype of x' if rounding & DT_WEIGHTS_16 else 'fp32'}, [D] on the GPU")
-    if rope_end is None:
-        rope_end = S
-    tab_sb = 0
-    if rope != DT_ROPE_NONE and rope_end > rope_begin:
-        rows = rope_end - rope_begin
-        for name, t in (("cos", cos), ("sin", sin)):
-            _require(t is not None and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
-                     and t.shape[-1] == D and t.shape[-2] == rows and t.dim() in (2, 3),
-                     f"{name} must be a contiguous fp32 [rows, D] or [B, rows, D] table on the GPU")
-        _require(cos.shape == sin.shape, "cos and sin must have one shape")
-        if cos.dim() == 3:
-            _require(cos.shape[0] == B, "batched tables need B leading entries")
-            tab_sb = rows * D
-    sec = (c_i32 * max(1, len(sections)))(*[int(v) for v in sections])
-    rc = lib.dt_qk_norm_rope(x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), out.data_ptr(), B, S, H, D,
-                             int(norm), weight.data_ptr() if weight is not None else None,
-                             bias.data_ptr() if bias is not None else None, float(eps), int(rope),
-                             cos.data_ptr() if cos is not None else None, sin.data_ptr() if sin is not None else None,
-                             tab_sb, int(rope_begin), int(rope_end), sec, len(sections), int(rounding), float(out_scale),
-                             _stream())
-    _check(rc, "dt_qk_norm_rope")
-    return out
+    return _host().qk_norm_rope(x, norm, weight, bias, eps, rope, cos, sin, rope_begin, rope_end, sections, rounding, out, out_scale,
+                                _stream())

@@ -246,8 +246,7 @@ class proAttention:
 
     # ---- stride mode ------------------------------------------------------------------------------
     def _strides(self, timestep: int) -> Tuple[int, int]:
-        rm = get_redundancy_map()
-        return rm.get_curr_isp_stride(timestep, self.layer_id), rm.get_next_isp_stride(timestep, self.layer_id)
+        return get_redundancy_map().get_isp_strides(timestep, self.layer_id)
 
     @get_timer("oAttn")
     def attn(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> Optional[torch.Tensor]:
@@ -575,6 +574,18 @@ class proAttention:
             logger.warning("cu_seqlens_q not provided, using normal attention instead.")
             return self.attn(query, key, value)
         total_q, H, D = query.shape
+        out = self._varlen(query.view(1, total_q, H, D), key.view(1, key.shape[0], H, D), value.view(1, value.shape[0], H, D),
+                           cu_seqlens_q, cu_seqlens_kv, max_seqlen_q)
+        return out.view(total_q, H, D)
+
+    @get_timer("varlen oAttn")
+    def varlen_sample(self, query, key, value, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q):
+        """``varlen_attn`` on one packed batch that still has its batch dimension, ``[1, total, H, D]`` in and out: what a model
+        holds, without the six views (1.3 us each) that flattening it takes."""
+        return self._varlen(query, key, value, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q)
+
+    def _varlen(self, query, key, value, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q):
+        total_q, H, D = query.shape[1:]
         r = self.local_chunk_id
         on_device = torch.is_tensor(cu_seqlens_q) and cu_seqlens_q.is_cuda
         if on_device and not self.dry_run:
@@ -596,8 +607,7 @@ class proAttention:
 
             self._segments = (cu_q, cu_kv_of)
         try:
-            out = self.attn(query.view(1, total_q, H, D), key.view(1, key.shape[0], H, D),
-                            value.view(1, value.shape[0], H, D))
+            out = self.attn(query, key, value)
         finally:
             self._segments = None
         # rows outside every segment: flash_attn_varlen_func leaves zeros
@@ -605,7 +615,7 @@ class proAttention:
             _hip.zero_rows_from(out.view(total_q, H * D), cu_seqlens_q[-1:])
         elif cu_q[-1] < total_q:
             out[:, cu_q[-1]:] = 0
-        return out.view(total_q, H, D)
+        return out
 
 
 def _int32(t: torch.Tensor) -> torch.Tensor:

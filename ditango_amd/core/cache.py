@@ -28,8 +28,7 @@ logger = init_logger(__name__)
 
 def _allocated_mb() -> float:
     """``torch.cuda.memory_allocated()`` in MB; that function flattens and sorts every statistic first, 80 us a call."""
-    stats = torch.cuda.memory_stats_as_nested_dict()
-    return stats["allocated_bytes"]["all"]["current"] / (1024 * 1024) if stats else 0.0
+    return _hip._host().allocated_bytes(torch.cuda.current_device()) / (1024 * 1024) if torch.cuda.is_initialized() else 0.0
 
 
 class proCache:

@@ -83,6 +83,14 @@ class RedundancyMap:
             return self.base_weight
         return self._stride_of(int(self.divider_map[timestep + 1, layer_id].item()))
 
+    def get_isp_strides(self, timestep: int, layer_id: int):
+        """(``get_curr_isp_stride``, ``get_next_isp_stride``), the map read once."""
+        if not self.auto_setting and timestep != self.num_timesteps - 1:
+            both = _hip._host().two_rows(self.divider_map, timestep, layer_id)
+            if both is not None:
+                return self._stride_of(both[0]), self._stride_of(both[1])
+        return self.get_curr_isp_stride(timestep, layer_id), self.get_next_isp_stride(timestep, layer_id)
+
     def set_pattern_for_row(self, row_idx: int, split_list: Sequence[int], pattern_list: Sequence[int]) -> None:
         """:90-119 -- piecewise-constant dividers over the layers of one step."""
         if row_idx >= self.num_timesteps:

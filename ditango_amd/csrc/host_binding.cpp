@@ -9,6 +9,7 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/CachingDeviceAllocator.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <algorithm>
@@ -746,6 +747,57 @@ void zero_rows_from(const Tensor& t, const Tensor& first_row, uint64_t stream) {
        static_cast<const int32_t*>(ptr(first_row)), stream_of(stream));
 }
 
+// ---- producer ------------------------------------------------------------------------------------------------
+
+// ditango_amd._hip.qk_norm_rope
+Tensor qk_norm_rope(const Tensor& x, int32_t norm, const std::optional<Tensor>& weight, const std::optional<Tensor>& bias, double eps,
+                    int32_t rope, const std::optional<Tensor>& cos, const std::optional<Tensor>& sin, int32_t rope_begin,
+                    std::optional<int32_t> rope_end, const std::vector<int32_t>& sections, int32_t rounding, std::optional<Tensor> out,
+                    double out_scale, uint64_t stream) {
+  REQUIRE(x.is_cuda() && is_half(x) && x.dim() == 4 && x.stride(3) == 1, "x must be bf16 or fp16 [B,S,H,D] on the GPU");
+  const Dims d{x.size(0), x.size(1), x.size(2), x.size(3)};
+  if (!out) out = new_out(d, x.scalar_type(), x);
+  REQUIRE(out->is_cuda() && out->scalar_type() == x.scalar_type() && out->is_contiguous() && shape_is(*out, {d.B, d.S, d.H, d.D}),
+          "out must be a contiguous [B,S,H,D] in x's dtype");
+  if (x.scalar_type() == at::kHalf) rounding |= DT_IO_FP16;
+  const bool narrow = rounding & DT_WEIGHTS_16;
+  for (const auto* t : {&weight, &bias})
+    REQUIRE(!*t || ((*t)->is_cuda() && (*t)->scalar_type() == (narrow ? x.scalar_type() : at::kFloat) && (*t)->is_contiguous() &&
+                    (*t)->numel() == d.D),
+            t == &weight ? "weight" : "bias", " must be ", narrow ? "of the dtype of x" : "fp32", ", [D] on the GPU");
+  const int64_t end = rope_end ? *rope_end : d.S, rows = end - rope_begin;
+  int64_t table_stride = 0;
+  if (rope != DT_ROPE_NONE && rows > 0) {
+    for (const auto* t : {&cos, &sin})
+      REQUIRE(*t && (*t)->is_cuda() && (*t)->scalar_type() == at::kFloat && (*t)->is_contiguous() && ((*t)->dim() == 2 || (*t)->dim() == 3) &&
+                  (*t)->size(-1) == d.D && (*t)->size(-2) == rows,
+              t == &cos ? "cos" : "sin", " must be a contiguous fp32 [rows, D] or [B, rows, D] table on the GPU");
+    REQUIRE(cos->sizes() == sin->sizes(), "cos and sin must have one shape");
+    if (cos->dim() == 3) {
+      REQUIRE(cos->size(0) == d.B, "batched tables need B leading entries");
+      table_stride = rows * d.D;
+    }
+  }
+  CALL(dt_qk_norm_rope, ptr(x), x.stride(0), x.stride(1), x.stride(2), ptr(*out), d.B, d.S, d.H, d.D, norm, ptr(weight), ptr(bias), (float)eps,
+       rope, static_cast<const float*>(ptr(cos)), static_cast<const float*>(ptr(sin)), table_stride, rope_begin, (int32_t)end,
+       sections.data(), (int32_t)sections.size(), rounding, (float)out_scale, stream_of(stream));
+  return *out;
+}
+
+// ---- host state of a call -------------------------------------------------------------------------------------
+
+// Elements [row, col] and [row + 1, col] of a 2-D int64 CPU tensor, or nothing where it is another one or a row or column is not there.
+std::optional<std::pair<int64_t, int64_t>> two_rows(const Tensor& t, int64_t row, int64_t col) {
+  if (t.is_cuda() || t.scalar_type() != at::kLong || t.dim() != 2 || row < 0 || row + 1 >= t.size(0) || col < 0 || col >= t.size(1))
+    return std::nullopt;
+  const int64_t* at = t.const_data_ptr<int64_t>() + row * t.stride(0) + col * t.stride(1);
+  return std::make_pair(at[0], at[t.stride(0)]);
+}
+// Bytes that PyTorch's allocator has handed out on a device.
+int64_t allocated_bytes(int64_t device) {
+  return c10::getDeviceAllocator(at::kCUDA)->getDeviceStats((c10::DeviceIndex)device).allocated_bytes[0].current;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_ditango_host, m) {
@@ -798,4 +850,7 @@ PYBIND11_MODULE(_ditango_host, m) {
   m.def("cache_store", &cache_store);
   m.def("cache_load", &cache_load);
   m.def("zero_rows_from", &zero_rows_from);
+  m.def("qk_norm_rope", &qk_norm_rope);
+  m.def("two_rows", &two_rows);
+  m.def("allocated_bytes", &allocated_bytes);
 }

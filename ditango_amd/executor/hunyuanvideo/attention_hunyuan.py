@@ -25,6 +25,9 @@ class Hunyuan_DiTangoProcessor:
 
     def ringfusion_attn(self, q, k, v, drop_rate=0, attn_mask=None, causal=False, cu_seqlens_q=None, cu_seqlens_kv=None,
                         max_seqlen_q=None, max_seqlen_kv=None, batch_size=1):
+        if cu_seqlens_q is not None and q.shape[0] == k.shape[0] == v.shape[0] == 1:
+            x = self.oAttn.varlen_sample(q, k, v, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q)
+            return x.view(batch_size, max_seqlen_q, x.shape[2] * x.shape[3])
         pre_attn_layout, post_attn_layout = MEMORY_LAYOUT["flash"]
         q, k, v = pre_attn_layout(q), pre_attn_layout(k), pre_attn_layout(v)
         x = self.varlen_Attn(q, k, v, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q, max_seqlen_kv)

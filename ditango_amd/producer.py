@@ -28,16 +28,19 @@ _ROPES = {None: _hip.DT_ROPE_NONE, "none": _hip.DT_ROPE_NONE, "interleaved": _hi
 
 
 def _f32(t: Optional[torch.Tensor], device) -> Optional[torch.Tensor]:
-    if t is None:
-        return None
+    if t is None or (t.dtype is torch.float32 and t.device == device and t.is_contiguous()):
+        return t
     return t.detach().to(device=device, dtype=torch.float32).contiguous()
 
 
 def _read_in_place(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor]) -> bool:
     """Norm parameters in x's own 16-bit type, as a model's modules hold them, are widened by the kernel as it reads them
     (two conversion launches a call less); any other dtype, place or alignment goes through an fp32 copy."""
-    return all(t is None or (t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0)
-               for t in (weight, bias)) and x.dtype in _hip.HALF_DTYPES
+    dtype = x.dtype
+    for t in (weight, bias):
+        if t is not None and not (t.dtype is dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            return False
+    return dtype in _hip.HALF_DTYPES
 
 
 def prepare_qk(x: torch.Tensor, *, norm: Optional[str] = None, weight: Optional[torch.Tensor] = None,
@@ -72,7 +75,6 @@ def prepare_qk(x: torch.Tensor, *, norm: Optional[str] = None, weight: Optional[
     rounding = (_hip.DT_ROUND_NORM_BF16 if match_eager_rounding else 0) | (_hip.DT_ROUND_ROPE_BF16 if bf16_rope_math else 0)
     if (weight is not None or bias is not None) and _read_in_place(x, weight, bias):
         rounding |= _hip.DT_WEIGHTS_16
-        weight, bias = (t.detach() if t is not None else None for t in (weight, bias))
     else:
         weight, bias = _f32(weight, x.device), _f32(bias, x.device)
     return _hip.qk_norm_rope(x, norm=_NORMS[norm], weight=weight, bias=bias, eps=eps,

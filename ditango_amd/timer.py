@@ -4,6 +4,7 @@ entry and exit when timing is enabled and costs nothing when it is not (the
 reference enables it from denoise step 2 on)."""
 import time
 from contextlib import ContextDecorator
+from functools import wraps
 from typing import Dict, List
 
 import torch
@@ -36,6 +37,14 @@ class _Timer(ContextDecorator):
     def __init__(self, name: str):
         self.name = name
         self._t0 = None
+
+    def __call__(self, func):
+        timed = super().__call__(func)
+
+        @wraps(func)
+        def call(*args, **kwargs):
+            return timed(*args, **kwargs) if _ENABLED else func(*args, **kwargs)
+        return call
 
     def __enter__(self):
         if _ENABLED:
