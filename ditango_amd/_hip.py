@@ -114,6 +114,8 @@ _SIGNATURES = {
     "dt_build_schedule": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp]),
     "dt_build_schedule_table": (ctypes.c_int, [c_vp, c_i32, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp]),
     "dt_rel_l1_sums": (ctypes.c_int, [c_vp, c_vp, c_i64, c_vp, c_vp]),
+    "dt_qkv_project": (ctypes.c_int, [c_vp, c_i64, c_i64, c_i32, c_vp, c_i64, c_i64, c_i32, c_i32, c_i32, c_i32, c_i32, c_vp, c_vp, c_vp,
+                                      c_i32, c_vp]),
     "dt_qk_norm_rope": (ctypes.c_int, [c_vp, c_i64, c_i64, c_i64, c_vp, c_i32, c_i32, c_i32, c_i32,
                                        c_i32, c_vp, c_vp, c_f32, c_i32, c_vp, c_vp, c_i64, c_i32, c_i32,
                                        _P(c_i32), c_i32, c_i32, c_f32, c_vp]),
@@ -538,3 +540,10 @@ def qk_norm_rope(x: torch.Tensor, *, norm: int = DT_NORM_NONE, weight: Optional[
     with ``DT_WEIGHTS_16`` in ``rounding`` of x's dtype."""
     return _host().qk_norm_rope(x, norm, weight, bias, eps, rope, cos, sin, rope_begin, rope_end, sections, rounding, out, out_scale,
                                 _stream())
+
+
+def qkv_project(text: torch.Tensor, video: torch.Tensor, heads: int, projections, cos: Optional[torch.Tensor] = None,
+                sin: Optional[torch.Tensor] = None):
+    """q, k and v ``[B,T+V,heads,64]`` of ``text`` ``[B,T,K]`` and ``video`` ``[B,V,K]`` in one launch.  ``projections``: three of
+    ``(weight, bias, norm, norm_weight, norm_bias, eps, rope)``; cos/sin fp32 ``[V,64]`` for those with ``rope``."""
+    return _host().qkv_project(text, video, heads, projections, cos, sin, _stream())

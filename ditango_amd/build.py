@@ -28,7 +28,7 @@ HOST_PATH = LIB_DIR / "_ditango_host.so"             # Python extension: the hos
 PROBES_PATH = LIB_DIR / "libditango_probes.so"
 DEMO_PATH = LIB_DIR / "dt_capi_demo"
 RESOURCES_PATH = LIB_DIR / "kernel_resources.json"   # per-kernel registers / scratch / occupancy of the last build
-SOURCES = ["attn_fwd.hip", "attn_f32.hip", "state_ops.hip", "producer.hip", "capi.hip"]
+SOURCES = ["attn_fwd.hip", "attn_f32.hip", "state_ops.hip", "producer.hip", "qkv.hip", "capi.hip"]
 PROBE_SOURCES = ["probes.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

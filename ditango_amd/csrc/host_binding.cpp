@@ -784,6 +784,41 @@ Tensor qk_norm_rope(const Tensor& x, int32_t norm, const std::optional<Tensor>& 
   return *out;
 }
 
+// ditango_amd._hip.qkv_project.  A projection: (weight, bias, norm, norm weight, norm bias, eps, rope).
+using Projection = std::tuple<Tensor, std::optional<Tensor>, int32_t, std::optional<Tensor>, std::optional<Tensor>, double, bool>;
+std::vector<Tensor> qkv_project(const Tensor& text_rows, const Tensor& video, int64_t heads, const std::vector<Projection>& projections,
+                                const std::optional<Tensor>& cos, const std::optional<Tensor>& sin, uint64_t stream) {
+  for (const auto* t : {&text_rows, &video})
+    REQUIRE(t->is_cuda() && is_half(*t) && t->dim() == 3 && t->stride(2) == 1 && t->scalar_type() == video.scalar_type() && t->size(0) == video.size(0) &&
+                t->size(2) == video.size(2),
+            "text and video must be bf16 or fp16 [B,tokens,channels] on the GPU, of one dtype");
+  REQUIRE(projections.size() == 3 && heads > 0, "three projections and a positive number of heads are needed");
+  const int64_t B = video.size(0), T = text_rows.size(1), V = video.size(1), K = video.size(2), D = std::get<0>(projections[0]).size(0) / heads;
+  dt_projection table[3] = {};
+  std::vector<Tensor> outs;
+  for (int i = 0; i < 3; ++i) {
+    const auto& [w, bias, norm, norm_w, norm_b, eps, rope] = projections[i];
+    REQUIRE(w.is_cuda() && w.scalar_type() == video.scalar_type() && w.is_contiguous() && shape_is(w, {heads * D, K}),
+            "weights must be contiguous [heads D, channels] in the tokens' dtype");
+    REQUIRE(!bias || (bias->is_cuda() && bias->scalar_type() == video.scalar_type() && bias->is_contiguous() && bias->numel() == heads * D),
+            "biases must be [heads D] in the tokens' dtype");
+    for (const auto* t : {&norm_w, &norm_b})
+      REQUIRE(!*t || ((*t)->is_cuda() && (*t)->scalar_type() == video.scalar_type() && (*t)->is_contiguous() && (*t)->numel() == D),
+              "norm parameters must be [D] in the tokens' dtype");
+    if (rope)
+      for (const auto* t : {&cos, &sin})
+        REQUIRE(*t && (*t)->is_cuda() && (*t)->scalar_type() == at::kFloat && (*t)->is_contiguous() && shape_is(**t, {V, D}),
+                "cos and sin must be contiguous fp32 [video tokens, D] tables on the GPU");
+    outs.push_back(new_out(Dims{B, T + V, heads, D}, video.scalar_type(), video));
+    table[i] = {ptr(w), ptr(bias), ptr(outs.back()), ptr(norm_w), ptr(norm_b), norm, rope, (float)eps};
+  }
+  const int32_t rounding = video.scalar_type() == at::kHalf ? DT_IO_FP16 : 0;
+  CALL(dt_qkv_project, ptr(text_rows), text_rows.stride(0), text_rows.stride(1), (int32_t)T, ptr(video), video.stride(0), video.stride(1), (int32_t)V, (int32_t)B,
+       (int32_t)K, (int32_t)heads, (int32_t)D, table, static_cast<const float*>(ptr(cos)), static_cast<const float*>(ptr(sin)), rounding,
+       stream_of(stream));
+  return outs;
+}
+
 // ---- host state of a call -------------------------------------------------------------------------------------
 
 // Elements [row, col] and [row + 1, col] of a 2-D int64 CPU tensor, or nothing where it is another one or a row or column is not there.
@@ -851,6 +886,7 @@ PYBIND11_MODULE(_ditango_host, m) {
   m.def("cache_load", &cache_load);
   m.def("zero_rows_from", &zero_rows_from);
   m.def("qk_norm_rope", &qk_norm_rope);
+  m.def("qkv_project", &qkv_project);
   m.def("two_rows", &two_rows);
   m.def("allocated_bytes", &allocated_bytes);
 }

@@ -1,0 +1,419 @@
+// The q, k and v of a layer in one launch: three linear projections of the text and video tokens, with LayerNorm over the head
+// dimension and interleaved RoPE on q and k before they are written, as the [B,S,H,64] tensors the attention kernel reads.
+// Replaces the concatenation, the three library products and the two producer launches of
+// executor/cogvideox/attention_processor.py:39-71.
+//
+// What bounds it: the matrix pipe and, behind it, LDS reads (70 % of the LDS cycles at 160 x 512) and the loads.  48 heads x 2222 tokens
+// x 3072 channels, 126 GFLOP: 130 us, 970 TFLOP/s, against 126 in three library products and 33 in the three launches around them (us
+// between events around a loop, both sides: 153 -> 130); 16 heads x 602 x 1024 42 -> 18.  Twice the products of the former the
+// library's kernels do faster (48 x 3358 198 -> 218), so the adapter asks for no more than 150 GFLOP here.
+// out^T = W X^T with v_mfma_f32_32x32x16, accumulated in fp32.  A wavefront owns one head (64 output columns) of 32 MB tokens; with
+// the product transposed a lane holds 32 of the 64 columns of ONE token, so the statistics of a row are sums in registers and one
+// exchange with lane ^ 32, and the rotated pairs are neighbouring registers.
+//   * A workgroup of 8 wavefronts takes BM = 32 MB WM tokens x BN = 64 (8 / WM) columns of the three outputs side by side.
+//   * Steps of 32 input channels, three LDS buffers: tiles go from memory straight into the LDS (global_load_lds, two steps ahead) as
+//     rows of 64 bytes, their four 16-byte pieces permuted by the row so that operand reads meet in no bank.
+//   * The two wavefronts of a SIMD issue their loads at different halves of the step (an M0 write and a load each 20 cycles or so,
+//     in which a wavefront issues no MFMA): 48 heads x 2222 tokens 140 -> 128 us together with the epilogue's tables through the LDS.
+//   * One barrier a step, in its middle: in front of it a wavefront has read the last operands it needs of the step's buffer and
+//     waited for its own loads of the next one; behind it come the first operands of the next step, half a step before the MFMAs
+//     that take them.
+#include <algorithm>
+#include <type_traits>
+
+#include "dt_common.h"
+
+namespace dt {
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kThreads = 512;
+constexpr int kWaves = 8;
+constexpr int kHead = 64;
+constexpr int kXcds = 8;
+constexpr int kStageBytes = kWaves * 32 * kHead * 2;   // output rows on their way
+
+struct QkvProj {
+  const uint16_t* w;          // [N, K]
+  const uint16_t* bias;       // [N] or null
+  uint16_t* y;                // [M, N]
+  const uint16_t *nw, *nb;    // LayerNorm weight and bias over the head dimension, or null
+  int32_t norm, rope;
+  float eps;
+};
+struct QkvArgs {
+  const uint16_t *text, *video;
+  int64_t text_sb, text_ss, video_sb, video_ss;   // elements
+  int32_t T, S, M;            // text tokens, all tokens of a sample, of the batch
+  int32_t N, K;               // output columns of one projection, input channels
+  int32_t m_tiles, tiles, per_xcd;
+  const float *cos, *sin;     // [S - T, 64]
+  QkvProj proj[3];
+};
+typedef const QkvArgs __attribute__((address_space(4))) KernArgs;
+
+template <bool kHalf>
+struct Elem {
+  typedef bf16x8 x8;
+  typedef bf16x2 x2;
+  __device__ static __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+};
+template <>
+struct Elem<true> {
+  typedef f16x8 x8;
+  typedef f16x2 x2;
+  __device__ static __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+};
+template <bool kHalf>
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  f32x2 f = {lo, hi};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, typename Elem<kHalf>::x2));
+}
+template <bool kHalf>
+__device__ __forceinline__ f32x2 unpack2(uint32_t w) {
+  if constexpr (kHalf) return __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2);
+  else return f32x2{__builtin_bit_cast(float, w << 16), __builtin_bit_cast(float, w & 0xffff0000u)};
+}
+// 64 x 16 bytes from the lanes' addresses to consecutive LDS bytes (see load_block_to_lds in attn_fwd.hip for why in assembly).
+__device__ __forceinline__ void load_block_to_lds(const uint16_t* from, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :
+               : "v"(from), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
+               : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N >= 0 && N <= 63, "an immediate of the wait");
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
+}
+__device__ __forceinline__ void step_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int MB, int WM, int KH, int NBUF, bool kHalf>
+__global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_value) {
+  typedef Elem<kHalf> E;
+  constexpr int WN = kWaves / WM;
+  constexpr int BM = 32 * MB * WM, BN = kHead * WN;
+  constexpr int kStep = 16 * KH, kRowBytes = kStep * 2;   // input channels of a step
+  constexpr int kPieces = kRowBytes / 16, kRowsPer = 64 / kPieces;   // 16-byte pieces of a row, rows of a load
+  constexpr int kSwzShift = KH == 2 ? 2 : 1;
+  constexpr int kGroups = (BM + BN) / kRowsPer;           // 1 KB loads of a step
+  constexpr int kMost = (kGroups + kWaves - 1) / kWaves;  // of a wavefront
+  constexpr int kFull = kGroups % kWaves ? kGroups % kWaves : kWaves;   // wavefronts that have so many; the others one less
+  constexpr int kBufBytes = (BM + BN) * kRowBytes;
+  KernArgs& a = *(KernArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  (void)args_by_value;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((uint8_t __attribute__((address_space(3)))*)lds);
+
+  // tiles of an XCD are neighbours: all token tiles of a column tile, then the next column tile
+  const int idx = blockIdx.x >> 3;
+  const int tile = (int)(blockIdx.x & (kXcds - 1)) * a.per_xcd + idx;
+  if (idx >= a.per_xcd || tile >= a.tiles) return;
+  const int n_tile = tile / a.m_tiles;
+  const int m0 = (tile - n_tile * a.m_tiles) * BM, n0 = n_tile * BN;
+  const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wm = wave / WN, wn = wave - wm * WN;
+  const int steps = a.K / kStep;
+
+  // ---- this lane's place in the tiles it loads: rows past the end are the last one's again
+  const uint16_t* from[kMost];
+#pragma unroll
+  for (int i = 0; i < kMost; ++i) {
+    const int row = (i * kWaves + wave) * kRowsPer + lane / kPieces;
+    const int piece = (lane % kPieces) ^ ((row >> kSwzShift) & (kPieces - 1));
+    if (row < BM) {
+      const int m = min(m0 + row, a.M - 1), b = m / a.S, s = m - b * a.S;
+      from[i] = s < a.T ? a.text + b * a.text_sb + s * a.text_ss : a.video + b * a.video_sb + (int64_t)(s - a.T) * a.video_ss;
+    } else {
+      const int n = min(n0 + row - BM, 3 * a.N - 1), p = n / a.N;
+      const uint16_t* w = p == 0 ? a.proj[0].w : p == 1 ? a.proj[1].w : a.proj[2].w;
+      from[i] = w + (int64_t)(n - p * a.N) * a.K;
+    }
+    from[i] += 8 * piece;
+  }
+  auto load_step = [&](int buffer) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kMost; ++i) {
+      if (i + 1 < kMost || wave < kFull) load_block_to_lds(from[i], lds0 + buffer * kBufBytes + (i * kWaves + wave) * 1024);
+      from[i] += kStep;
+    }
+  };
+  // all but the loads of the kAhead newest steps
+  auto wait_steps = [&](auto ahead) __attribute__((always_inline)) {
+    constexpr int kAhead = decltype(ahead)::value;
+    if constexpr (kFull == kWaves || kAhead == 0) wait_loads<kAhead * kMost>();
+    else if (wave < kFull) wait_loads<kAhead * kMost>();
+    else wait_loads<kAhead * (kMost - 1)>();
+  };
+
+  f32x16 acc[2][MB];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.f;
+
+  struct Operands {
+    typename E::x8 w[2], x[MB];
+  };
+  // operands of half a step: 16 input channels
+  auto read = [&](Operands& o, int buffer, int half) __attribute__((always_inline)) {
+    const uint8_t* at = lds + buffer * kBufBytes + col * kRowBytes + (((2 * half + hh) ^ ((col >> kSwzShift) & (kPieces - 1))) << 4);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) o.w[j] = *reinterpret_cast<const typename E::x8*>(at + (BM + wn * kHead + 32 * j) * kRowBytes);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) o.x[i] = *reinterpret_cast<const typename E::x8*>(at + (wm * 32 * MB + 32 * i) * kRowBytes);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[j][i] = E::mfma(o.w[j], o.x[i], acc[j][i]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  load_step(0);
+#pragma unroll
+  for (int t = 1; t < NBUF; ++t)
+    if (t < steps) load_step(t);
+  if (steps >= NBUF) wait_steps(std::integral_constant<int, NBUF - 1>());
+  else wait_steps(std::integral_constant<int, 0>());
+  step_barrier();
+  Operands operands[2];
+  read(operands[0], 0, 0);
+  int buffer = 0;
+  const bool late = wave >= kWaves / 2;
+  for (int t = 0; t < steps; ++t) {
+    if (late && t > 0 && t + NBUF - 1 < steps) load_step(buffer == 0 ? NBUF - 1 : buffer - 1);
+#pragma unroll
+    for (int h = 0; h < KH - 1; ++h) {
+      read(operands[(h + 1) & 1], buffer, h + 1);
+      multiply(operands[h & 1]);
+    }
+    // the next step's tile has landed, for everybody; nobody reads this one's any more
+    if (t + NBUF - 1 < steps) wait_steps(std::integral_constant<int, NBUF - 2>());
+    else wait_steps(std::integral_constant<int, 0>());
+    step_barrier();
+    if (!late && t + NBUF < steps) load_step(buffer);
+    buffer = buffer == NBUF - 1 ? 0 : buffer + 1;
+    read(operands[0], buffer, 0);   // (behind the last step: some operands nobody uses)
+    multiply(operands[(KH - 1) & 1]);
+  }
+
+  // ---- bias, LayerNorm, RoPE; a wavefront's rows go through LDS of its own, so that stores are whole rows.  The tables of the
+  // workgroup's tokens come into the LDS once for all of its heads (from memory for each, the launch took 25 us longer).
+  constexpr int kTable = BM * kHead * 4;
+  float* tables = reinterpret_cast<float*>(lds + kStageBytes);
+  if (n0 < 2 * a.N && (a.proj[0].rope || a.proj[1].rope)) {
+#pragma unroll
+    for (int i = 0; i < BM / 32; ++i) {
+      const int row = (i * kWaves + wave) * 4 + (lane >> 4), s = min(m0 + row, a.M - 1) % a.S;
+      const int64_t at = (int64_t)max(s - a.T, 0) * kHead + 4 * (lane & 15);
+      const uint32_t to = lds0 + kStageBytes + (i * kWaves + wave) * 1024;
+      load_block_to_lds(reinterpret_cast<const uint16_t*>(a.cos + at), to);
+      load_block_to_lds(reinterpret_cast<const uint16_t*>(a.sin + at), to + kTable);
+    }
+  }
+  const int n_wave = n0 + wn * kHead;
+  const bool mine = n_wave < 3 * a.N;
+  const int p = mine ? n_wave / a.N : 0, n_proj = mine ? n_wave - p * a.N : 0;
+  const auto& pr = a.proj[p];
+  u32x2 bias[2][4], nw[2][4], nb[2][4];   // zero, one and zero where there are none
+  const uint32_t one = pack2<kHalf>(1.f, 1.f);
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = 32 * j + 8 * g + 4 * hh;
+      bias[j][g] = pr.bias ? *reinterpret_cast<const u32x2*>(pr.bias + n_proj + d) : u32x2{0, 0};
+      nw[j][g] = pr.nw ? *reinterpret_cast<const u32x2*>(pr.nw + d) : u32x2{one, one};
+      nb[j][g] = pr.nb ? *reinterpret_cast<const u32x2*>(pr.nb + d) : u32x2{0, 0};
+    }
+  wait_loads<0>();
+  step_barrier();
+  if (!mine) return;
+  uint8_t* stage = lds + wave * (32 * kHead * 2);
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    const int block = (wm * MB + i) * 32, m_first = m0 + block;
+    if (m_first >= a.M) break;
+    float v[32];
+#pragma unroll
+    for (int e = 0; e < 32; e += 2) {   // rounded as the projection's output is
+      const f32x2 b = unpack2<kHalf>(bias[e >> 4][(e >> 2) & 3][(e >> 1) & 1]);
+      const f32x2 r = unpack2<kHalf>(pack2<kHalf>(acc[e >> 4][i][e & 15] + b.x, acc[e >> 4][i][(e & 15) + 1] + b.y));
+      v[e] = r.x;
+      v[e + 1] = r.y;
+    }
+    if (pr.norm != DT_NORM_NONE) {
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) sum += v[e];
+      sum += __shfl_xor(sum, 32);
+      const float mean = sum * (1.0f / kHead);
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) ss += (v[e] - mean) * (v[e] - mean);
+      ss += __shfl_xor(ss, 32);
+      const float rs = 1.0f / sqrtf(ss * (1.0f / kHead) + pr.eps);
+#pragma unroll
+      for (int e = 0; e < 32; e += 2) {
+        const f32x2 w = unpack2<kHalf>(nw[e >> 4][(e >> 2) & 3][(e >> 1) & 1]), b = unpack2<kHalf>(nb[e >> 4][(e >> 2) & 3][(e >> 1) & 1]);
+        v[e] = (v[e] - mean) * rs * w.x + b.x;
+        v[e + 1] = (v[e + 1] - mean) * rs * w.y + b.y;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {   // rounded as the norm's output is
+        const float* x = v + 16 * j + 4 * g;
+        *reinterpret_cast<u32x2*>(stage + col * (kHead * 2) + (((4 * j + g) ^ ((col >> 1) & 7)) << 4) + 8 * hh) =
+            u32x2{pack2<kHalf>(x[0], x[1]), pack2<kHalf>(x[2], x[3])};
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 8 * r + (lane >> 3), d = 8 * (lane & 7);
+      u32x4 x = *reinterpret_cast<const u32x4*>(stage + row * (kHead * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+      const int m = m_first + row;
+      if (pr.rope) {
+        const float* c = tables + (block + row) * kHead + d;
+        const bool video = m % a.S >= a.T;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const f32x2 z = unpack2<kHalf>(x[e]);
+          const f32x2 cs = *reinterpret_cast<const f32x2*>(c + 2 * e), sn = *reinterpret_cast<const f32x2*>(c + kTable / 4 + 2 * e);
+          const uint32_t y = pack2<kHalf>(z.x * cs.x + -z.y * sn.x, z.y * cs.y + z.x * sn.y);
+          x[e] = video ? y : x[e];
+        }
+      }
+      if (m < a.M) *reinterpret_cast<u32x4*>(pr.y + (int64_t)m * a.N + n_proj + d) = x;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
+template <int MB, int WM, int KH, int NBUF>
+constexpr int lds_bytes() { return std::max(NBUF * (32 * MB * WM + kHead * (kWaves / WM)) * KH * 32, kStageBytes + 2 * 32 * MB * WM * kHead * 4); }
+
+template <int MB, int WM, int KH, int NBUF, bool kHalf>
+int launch_t(QkvArgs& a, hipStream_t stream) {
+  constexpr int BM = 32 * MB * WM, BN = kHead * (kWaves / WM), kLds = lds_bytes<MB, WM, KH, NBUF>();
+  static_assert(kLds <= 163840, "the LDS of a CU");
+  static thread_local int allowed_dev = -1;   // more than 64 KB of dynamic LDS has to be allowed once per kernel and device
+  int dev = 0;
+  if (int rc = hip_fail(hipGetDevice(&dev), "hipGetDevice")) return rc;
+  if (allowed_dev != dev) {
+    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&qkv_kernel<MB, WM, KH, NBUF, kHalf>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+                          "hipFuncSetAttribute"))
+      return rc;
+    allowed_dev = dev;
+  }
+  a.m_tiles = (a.M + BM - 1) / BM;
+  a.tiles = a.m_tiles * ((3 * a.N + BN - 1) / BN);
+  a.per_xcd = (a.tiles + kXcds - 1) / kXcds;
+  hipLaunchKernelGGL((qkv_kernel<MB, WM, KH, NBUF, kHalf>), dim3((unsigned)a.per_xcd * kXcds), dim3(kThreads), kLds, stream, a);
+  return hip_fail(hipGetLastError(), "qkv launch");
+}
+template <int MB, int WM, int KH, int NBUF>
+int launch(QkvArgs& a, bool half, hipStream_t stream) {
+  return half ? launch_t<MB, WM, KH, NBUF, true>(a, stream) : launch_t<MB, WM, KH, NBUF, false>(a, stream);
+}
+
+// Which tile a launch takes: 64 x 256, two workgroups a CU, 192 x 256 or 160 x 512.  The time of each in us is its rounds of the 256 CUs
+// times the 64-channel steps of one, and what a round and the launch cost on top; constants fitted to 70 launches of 8 ... 48 heads (8 ... 48
+// steps) x 280 ... 12 000 tokens (errors 4 to 5 %; the choice takes 0.7 % more than the best of the three on average).  us, modules and producer -> 64
+// x 256 / 192 x 256 / 160 x 512: 16 heads x 602 tokens 42 -> 18 / 34 / 49; 48 x 1440 132 -> 125 / 118 / 135 (with 192 x 256 two rounds, one
+// of which is half empty with 160 x 512); 24 x 4330 108 -> 97 / 77 / 90; 48 x 2222 153 -> 166 / 139 / 130 (252 workgroups of 160 x 512, one round).
+enum Tiles { kFew, kSome, kMany };
+Tiles plan(int M, int N, int K) {
+  constexpr int kCus = 32;   // of an XCD
+  const double steps = K / 64.0;
+  auto per_xcd = [&](int bm, int bn) { return (int64_t)(((int64_t)((M + bm - 1) / bm) * ((3 * N + bn - 1) / bn) + kXcds - 1) / kXcds); };
+  auto rounds = [&](int bm, int bn) { return (double)((per_xcd(bm, bn) + kCus - 1) / kCus); };
+  const int64_t pairs = per_xcd(64, 256) / (2 * kCus), rest = per_xcd(64, 256) % (2 * kCus);
+  const double shared = pairs + (rest > kCus ? 1 : 0), alone = rest > 0 && rest <= kCus ? 1 : 0;
+  const double few = 4.2 + alone * (2.7 + 0.80 * steps) + shared * (9.1 + 1.08 * steps);
+  const double some = 15.4 + rounds(192, 256) * 1.18 * steps + (rounds(192, 256) - 1) * 16.0;
+  const double many = 19.8 + rounds(160, 512) * 1.96 * steps + (rounds(160, 512) - 1) * 24.9;
+  return few <= some && few <= many ? kFew : some <= many ? kSome : kMany;
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+}  // namespace
+}  // namespace dt
+
+using namespace dt;
+
+extern "C" int dt_qkv_project(const void* text, int64_t text_stride_b, int64_t text_stride_s, int32_t T, const void* video,
+                              int64_t video_stride_b, int64_t video_stride_s, int32_t V, int32_t B, int32_t K, int32_t H, int32_t D,
+                              const dt_projection* proj, const float* cos, const float* sin, int32_t rounding, void* stream) {
+  if (B <= 0 || T < 0 || V < 0 || T > INT32_MAX - V || T + V <= 0 || H <= 0 || K <= 0) {
+    set_error("B, T + V, H and K must be positive (got %d, %d + %d, %d, %d)", B, T, V, H, K);
+    return DT_ERR_INVALID;
+  }
+  if (D != kHead || K % 64) {
+    set_error("head dim %d and %d input channels not built (64, and multiples of 64, are)", D, K);
+    return DT_ERR_UNSUPPORTED;
+  }
+  if ((int64_t)B * (T + V) > (1 << 24) || H > (1 << 16) || K > (1 << 20)) {
+    set_error("too many tokens, heads or channels (%lld, %d, %d)", (long long)B * (T + V), H, K);
+    return DT_ERR_INVALID;
+  }
+  if ((T > 0 && (!text || !aligned16(text))) || (V > 0 && (!video || !aligned16(video))) || (text_stride_b & 7) || (text_stride_s & 7) ||
+      (video_stride_b & 7) || (video_stride_s & 7) || !proj) {
+    set_error("tokens must be non-null, 16-byte aligned, with strides that are multiples of 8 elements; three projections are needed");
+    return DT_ERR_INVALID;
+  }
+  if (rounding & ~DT_IO_FP16) {
+    set_error("bad rounding code %d", rounding);
+    return DT_ERR_INVALID;
+  }
+  QkvArgs a{};
+  a.text = static_cast<const uint16_t*>(text); a.video = static_cast<const uint16_t*>(video);
+  a.text_sb = text_stride_b; a.text_ss = text_stride_s; a.video_sb = video_stride_b; a.video_ss = video_stride_s;
+  a.T = T; a.S = T + V; a.M = B * (T + V);
+  a.N = H * kHead; a.K = K;
+  a.cos = cos; a.sin = sin;
+  for (int i = 0; i < 3; ++i) {
+    const dt_projection& p = proj[i];
+    if (!p.weight || !p.out || !aligned16(p.weight) || !aligned16(p.out) || !aligned16(p.bias) || !aligned16(p.norm_weight) || !aligned16(p.norm_bias)) {
+      set_error("projection %d: null weight or output, or a pointer that is not 16-byte aligned", i);
+      return DT_ERR_INVALID;
+    }
+    if (p.norm != DT_NORM_NONE && p.norm != DT_NORM_LAYER) {
+      set_error("projection %d: bad norm code %d", i, p.norm);
+      return DT_ERR_INVALID;
+    }
+    if (p.rope && V > 0 && (!cos || !sin || !aligned16(cos) || !aligned16(sin))) {
+      set_error("cos/sin tables must be non-null and 16-byte aligned");
+      return DT_ERR_INVALID;
+    }
+    a.proj[i] = {static_cast<const uint16_t*>(p.weight), static_cast<const uint16_t*>(p.bias), static_cast<uint16_t*>(p.out),
+                 static_cast<const uint16_t*>(p.norm_weight), static_cast<const uint16_t*>(p.norm_bias), p.norm, p.rope != 0 && V > 0, p.eps};
+  }
+  const bool half = (rounding & DT_IO_FP16) != 0;
+  const hipStream_t s = (hipStream_t)stream;
+  switch (plan(a.M, a.N, K)) {
+    case kFew: return launch<1, 2, 4, 2>(a, half, s);
+    case kSome: return launch<3, 2, 4, 2>(a, half, s);
+    default: return launch<5, 1, 2, 3>(a, half, s);
+  }
+}

@@ -8,7 +8,8 @@ What differs from the reference is how the stretch between the projections and t
 reference transposes to ``[B,H,S,D]``, applies the norm modules and ``apply_rotary_emb`` as eager ops on the
 video tokens, and transposes back with ``.contiguous()`` (:48-71) -- six passes over q and k.  Here the
 projection output is viewed as ``[B,S,H,D]`` (what the kernels read; no transposition at all) and LayerNorm +
-RoPE on the rows behind the text tokens are ONE pass each for q and k (``dt_qk_norm_rope``); the attention
+RoPE on the rows behind the text tokens are ONE pass each for q and k (``dt_qk_norm_rope``) -- or, with heads of 64 and plain
+``nn.Linear`` projections, the end of one launch that makes q, k and v from the two token streams (``.projection``); the attention
 writes the activation dtype directly (``proAttention.out_dtype``), so the cast of :80 is no pass either.
 """
 from __future__ import annotations
@@ -22,6 +23,7 @@ from ...core.parallel_state import get_isp_group
 from ...core.redundancy_map import get_redundancy_map
 from ...logger import init_logger
 from ...producer import prepare_qk
+from .projection import project_qkv
 
 logger = init_logger(__name__)
 
@@ -43,6 +45,9 @@ class CVX_oCacheAttnProcessor:
         """(query, key, value) of this rank's token shard, text tokens first, as ``[B,S,H,D]`` (bf16 or fp16, the model's dtype) in the layout
         the attention reads (:39-71 of the reference, without its transposes).  Also what a test or a ring
         stand-in calls to produce the K/V another rank would send."""
+        fused = project_qkv(attn, encoder_hidden_states, hidden_states, image_rotary_emb)
+        if fused is not None:
+            return fused
         text_seqlen = encoder_hidden_states.size(1)
         batch_size = hidden_states.shape[0]
         x = torch.cat([encoder_hidden_states, hidden_states], dim=1)

@@ -525,6 +525,28 @@ int dt_qk_norm_rope(const void* x, int64_t x_stride_b, int64_t x_stride_s, int64
                     int32_t rope_begin, int32_t rope_end, const int32_t* sections, int32_t n_sections,
                     int32_t rounding, float out_scale, void* stream);
 
+typedef struct {
+  const void* weight;
+  const void* bias;
+  void* out;
+  const void* norm_weight;
+  const void* norm_bias;
+  int32_t norm, rope;
+  float eps;
+} dt_projection;
+/*
+ * The producer with the projections in front of it: q, k and v of `text` ([B,T,K]) and, behind it, `video` ([B,V,K]) tokens in one
+ * launch -- executor/cogvideox/attention_processor.py:39-71.  proj[0..2] are q, k and v: out[b,s] = x[b,s] weight^T + bias, rounded to the
+ * tensors' type, then LayerNorm over each head (norm = DT_NORM_LAYER) and interleaved RoPE of the video tokens (rope != 0; cos and sin
+ * are fp32 [V, D]), rounded after each, and written as [B,T+V,H,D].
+ * 16-bit tensors (bfloat16, with rounding = DT_IO_FP16 IEEE half), parameters among them: weight [H D, K] contiguous, bias [H D] or NULL,
+ * norm_weight and norm_bias [D] or NULL; token rows contiguous, 16-byte aligned; D = 64, K a multiple of 64.
+ */
+int dt_qkv_project(const void* text, int64_t text_stride_b, int64_t text_stride_s, int32_t T,
+                   const void* video, int64_t video_stride_b, int64_t video_stride_s, int32_t V,
+                   int32_t B, int32_t K, int32_t H, int32_t D, const dt_projection* proj,
+                   const float* cos, const float* sin, int32_t rounding, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
