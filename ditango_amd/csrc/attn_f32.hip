@@ -590,7 +590,7 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
       }
       *reinterpret_cast<f32x4*>(mine + col * L::kPitch + 32 * i + 8 * g + 4 * hh) = x;
     }
-  const bool odd_row = odd_q || !(l < INFINITY);
+  const bool odd_row = odd_q || !(l > 0.f && l < INFINITY);   // (no sum: a maximum whose reference is past the exponent range, or scores of -inf only)
   if (__builtin_expect(any && __any(odd_row || worst >= kOddFrom), 0)) {
     // Once more with fp32 products, for the elements and rows that need it; the others stay what they are.
     float m2, l2;

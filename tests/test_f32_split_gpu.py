@@ -68,6 +68,16 @@ def test_infinities_in_one_part_of_the_keys(hip):
     assert torch.equal(out, want) and torch.equal(lse, want_lse)
 
 
+def test_scores_whose_reference_leaves_the_range(hip):
+    """The largest score is finite and the next multiple of the grid above it is not: one key has all the weight."""
+    q, k = torch.zeros(1, 40, 1, 64), torch.zeros(1, 70, 1, 64)
+    q[..., 3] = 2.0 ** 63
+    k[0, 50, 0, 3] = 1.75 * 2.0 ** 63
+    v = torch.randn(1, 70, 1, 64, generator=torch.Generator().manual_seed(8))
+    [(out, _)] = hip.attn_jobs_f32_fwd(q.cuda(), [k.cuda()], [v.cuda()], [[0]], softmax_scale=8.0)
+    assert torch.equal(out.cpu(), v[:, 50:51].expand_as(out))
+
+
 def test_result_under_graph_capture(hip):
     """Parts, counters and all: every replay equals the eager call, with other launches of the stream between them."""
     g = torch.Generator(device="cuda").manual_seed(6)
