@@ -3,16 +3,17 @@
 // Replaces the concatenation, the three library products and the two producer launches of
 // executor/cogvideox/attention_processor.py:39-71.
 //
-// What bounds it: the matrix pipe and, behind it, LDS reads (70 % of the LDS cycles at 160 x 512) and the loads.  48 heads x 2222 tokens
-// x 3072 channels, 126 GFLOP: 130 us, 970 TFLOP/s, against 126 in three library products and 33 in the three launches around them (us
-// between events around a loop, both sides: 153 -> 130); 16 heads x 602 x 1024 42 -> 18.  Twice the products of the former the
-// library's kernels do faster (48 x 3358 198 -> 218), so the adapter asks for no more than 150 GFLOP here.
+// What bounds it: the matrix pipe, with LDS reads behind it (70 to 85 % as many cycles as the MFMAs); of 141 us for 48 heads x 2222
+// tokens x 3072 channels (126 GFLOP) 28 are the loads of the tiles, 18 of those their issue (timed with loads left out, and with
+// loads of one place), 18 start and end.  In a loop of calls, modules and producer -> this: the same 153 -> 130 us (970 TFLOP/s), 16 heads x 602
+// x 1024 42 -> 18.  From 200 GFLOP on the library's products take less (48 x 8016 429 -> 458), and the adapter calls the modules.
 // out^T = W X^T with v_mfma_f32_32x32x16, accumulated in fp32.  A wavefront owns one head (64 output columns) of 32 MB tokens; with
 // the product transposed a lane holds 32 of the 64 columns of ONE token, so the statistics of a row are sums in registers and one
 // exchange with lane ^ 32, and the rotated pairs are neighbouring registers.
 //   * A workgroup of 8 wavefronts takes BM = 32 MB WM tokens x BN = 64 (8 / WM) columns of the three outputs side by side.
-//   * Steps of 32 input channels, three LDS buffers: tiles go from memory straight into the LDS (global_load_lds, two steps ahead) as
-//     rows of 64 bytes, their four 16-byte pieces permuted by the row so that operand reads meet in no bank.
+//   * Steps of 64 input channels with two LDS buffers, of 32 with three where the tile is 160 x 512: tiles go from memory straight into the
+//     LDS (global_load_lds, one or two steps ahead) as rows of 128 or 64 bytes, their 16-byte pieces permuted by the row so that operand
+//     reads meet in no bank.
 //   * The two wavefronts of a SIMD issue their loads at different halves of the step (an M0 write and a load each 20 cycles or so,
 //     in which a wavefront issues no MFMA): 48 heads x 2222 tokens 140 -> 128 us together with the epilogue's tables through the LDS.
 //   * One barrier a step, in its middle: in front of it a wavefront has read the last operands it needs of the step's buffer and
@@ -336,23 +337,25 @@ int launch(QkvArgs& a, bool half, hipStream_t stream) {
   return half ? launch_t<MB, WM, KH, NBUF, true>(a, stream) : launch_t<MB, WM, KH, NBUF, false>(a, stream);
 }
 
-// Which tile a launch takes: 64 x 256, two workgroups a CU, 192 x 256 or 160 x 512.  The time of each in us is its rounds of the 256 CUs
-// times the 64-channel steps of one, and what a round and the launch cost on top; constants fitted to 70 launches of 8 ... 48 heads (8 ... 48
-// steps) x 280 ... 12 000 tokens (errors 4 to 5 %; the choice takes 0.7 % more than the best of the three on average).  us, modules and producer -> 64
-// x 256 / 192 x 256 / 160 x 512: 16 heads x 602 tokens 42 -> 18 / 34 / 49; 48 x 1440 132 -> 125 / 118 / 135 (with 192 x 256 two rounds, one
-// of which is half empty with 160 x 512); 24 x 4330 108 -> 97 / 77 / 90; 48 x 2222 153 -> 166 / 139 / 130 (252 workgroups of 160 x 512, one round).
-enum Tiles { kFew, kSome, kMany };
+// Which tile a launch takes: 64 x 256, two workgroups a CU, 192 x 256, 256 x 256 or 160 x 512.  The time of each in us is its rounds of the
+// 256 CUs times the 64-channel steps of one, and what a round and the launch cost on top; constants fitted to 70 launches of 8 ... 48 heads
+// (8 ... 48 steps) x 280 ... 12 000 tokens (errors 4 to 5 %; the choice takes 0.9 % more than the best on average).  us, modules and producer ->
+// 64 x 256 / 192 x 256 / 256 x 256 / 160 x 512: 16 heads x 602 tokens 42 -> 18 / 34 / 39 / 49; 24 x 4330 108 -> 94 / 87 / 105 / 78; 48 x 2222
+// 153 -> 167 / 141 / 171 / 130 (252 workgroups of 160 x 512, one round); 48 x 3328 198 -> 248 / 214 / 186 / 235 (468 of 256 x 256, two).
+enum Tiles { kFew, kSome, kMost, kMany };
 Tiles plan(int M, int N, int K) {
   constexpr int kCus = 32;   // of an XCD
   const double steps = K / 64.0;
-  auto per_xcd = [&](int bm, int bn) { return (int64_t)(((int64_t)((M + bm - 1) / bm) * ((3 * N + bn - 1) / bn) + kXcds - 1) / kXcds); };
-  auto rounds = [&](int bm, int bn) { return (double)((per_xcd(bm, bn) + kCus - 1) / kCus); };
+  auto per_xcd = [&](int bm, int bn) { return ((int64_t)((M + bm - 1) / bm) * ((3 * N + bn - 1) / bn) + kXcds - 1) / kXcds; };
+  auto time = [&](int bm, int bn, double launch, double step, double round) {
+    const double rounds = (double)((per_xcd(bm, bn) + kCus - 1) / kCus);
+    return launch + rounds * step * steps + (rounds - 1) * round;
+  };
   const int64_t pairs = per_xcd(64, 256) / (2 * kCus), rest = per_xcd(64, 256) % (2 * kCus);
-  const double shared = pairs + (rest > kCus ? 1 : 0), alone = rest > 0 && rest <= kCus ? 1 : 0;
-  const double few = 4.2 + alone * (2.7 + 0.80 * steps) + shared * (9.1 + 1.08 * steps);
-  const double some = 15.4 + rounds(192, 256) * 1.18 * steps + (rounds(192, 256) - 1) * 16.0;
-  const double many = 19.8 + rounds(160, 512) * 1.96 * steps + (rounds(160, 512) - 1) * 24.9;
-  return few <= some && few <= many ? kFew : some <= many ? kSome : kMany;
+  const double shared = (double)(pairs + (rest > kCus ? 1 : 0)), alone = rest > 0 && rest <= kCus ? 1 : 0;
+  const double of[4] = {4.2 + alone * (2.7 + 0.80 * steps) + shared * (9.1 + 1.08 * steps), time(192, 256, 15.4, 1.18, 16.0),
+                        time(256, 256, 17.0, 1.45, 16.0), time(160, 512, 19.8, 1.96, 24.9)};
+  return (Tiles)(std::min_element(of, of + 4) - of);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -414,6 +417,7 @@ extern "C" int dt_qkv_project(const void* text, int64_t text_stride_b, int64_t t
   switch (plan(a.M, a.N, K)) {
     case kFew: return launch<1, 2, 4, 2>(a, half, s);
     case kSome: return launch<3, 2, 4, 2>(a, half, s);
+    case kMost: return launch<4, 2, 4, 2>(a, half, s);
     default: return launch<5, 1, 2, 3>(a, half, s);
   }
 }

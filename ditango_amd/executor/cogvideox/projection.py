@@ -9,9 +9,9 @@ from ... import _hip
 from ...producer import _f32
 
 HEAD_DIM = 64
-# Operations beyond which the library's products are faster, the launches around them included (us, modules -> one launch): 48 heads x 2222
-# tokens x 3072 channels, 126 GFLOP, 153 -> 130; 2951 tokens, 167 GFLOP, 211 -> 210; 3358, 190 GFLOP, 198 -> 218.
-MOST_FLOPS = 1.5e11
+# Operations beyond which the library's products may be faster, the launches around them included (us, modules -> one launch): 48 heads x
+# 2222 tokens x 3072 channels, 126 GFLOP, 153 -> 130; 3328 tokens, 188 GFLOP, 198 -> 186; 4454, 252 GFLOP, 239 -> 253; 8016 429 -> 458.
+MOST_FLOPS = 2.0e11
 
 
 def _only_arithmetic() -> bool:

@@ -71,7 +71,8 @@ def _check(got, want, dtype):
     (1, 28, 37, 8, 192, torch.bfloat16),       # one row more than a tile of 64
     (3, 5, 300, 5, 320, torch.bfloat16),       # rows of three samples in one tile
     (1, 113, 2500, 24, 1536, torch.bfloat16),  # 192 x 256
-    (1, 28, 2213, 48, 3072, torch.float16),    # 160 x 512, one row more than 14 tiles
+    (1, 28, 2212, 48, 3072, torch.float16),    # 160 x 512, 14 full tiles of rows
+    (1, 28, 3301, 48, 3072, torch.bfloat16),   # 256 x 256, one row more than 13 tiles
 ])
 @pytest.mark.parametrize("bias,rotated", [(True, True), (False, False)])
 def test_projections_match_fp64(hip, B, T, V, H, K, dtype, bias, rotated):
