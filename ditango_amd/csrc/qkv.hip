@@ -8,8 +8,7 @@
 // loads of one place), 18 start and end.  In a loop of calls, modules and producer -> this: the same 153 -> 130 us (970 TFLOP/s), 16 heads x 602
 // x 1024 42 -> 18.  From 200 GFLOP on the library's products take less (48 x 8016 429 -> 458), and the adapter calls the modules.
 // out^T = W X^T with v_mfma_f32_32x32x16, accumulated in fp32.  A wavefront owns one head (64 output columns) of 32 MB tokens; with
-// the product transposed a lane holds 32 of the 64 columns of ONE token, so the statistics of a row are sums in registers and one
-// exchange with lane ^ 32, and the rotated pairs are neighbouring registers.
+// the product transposed a lane holds 32 of the 64 columns of ONE token, four neighbouring ones at a time.
 //   * A workgroup of 8 wavefronts takes BM = 32 MB WM tokens x BN = 64 (8 / WM) columns of the three outputs side by side.
 //   * Steps of 64 input channels with two LDS buffers, of 32 with three where the tile is 160 x 512: tiles go from memory straight into the
 //     LDS (global_load_lds, one or two steps ahead) as rows of 128 or 64 bytes, their 16-byte pieces permuted by the row so that operand
@@ -19,23 +18,22 @@
 //   * One barrier a step, in its middle: in front of it a wavefront has read the last operands it needs of the step's buffer and
 //     waited for its own loads of the next one; behind it come the first operands of the next step, half a step before the MFMAs
 //     that take them.
+//   * The accumulators go through the LDS as rows of 16-bit projections, and norm and rotation follow with eight lanes a row, in the order
+//     of sums of qk_norm_rope_kernel: q, k and v are bit for bit those of the modules and the producer wherever the library adds up a
+//     product in one chain.
 #include <algorithm>
 #include <type_traits>
 
-#include "dt_common.h"
+#include "producer_math.h"
 
 namespace dt {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 512;
 constexpr int kWaves = 8;
@@ -74,11 +72,6 @@ struct Elem<true> {
   typedef f16x2 x2;
   __device__ static __forceinline__ f32x16 mfma(x8 a, x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
 };
-template <bool kHalf>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  f32x2 f = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, typename Elem<kHalf>::x2));
-}
 template <bool kHalf>
 __device__ __forceinline__ f32x2 unpack2(uint32_t w) {
   if constexpr (kHalf) return __builtin_convertvector(__builtin_bit_cast(f16x2, w), f32x2);
@@ -234,17 +227,16 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
   const bool mine = n_wave < 3 * a.N;
   const int p = mine ? n_wave / a.N : 0, n_proj = mine ? n_wave - p * a.N : 0;
   const auto& pr = a.proj[p];
-  u32x2 bias[2][4], nw[2][4], nb[2][4];   // zero, one and zero where there are none
-  const uint32_t one = pack2<kHalf>(1.f, 1.f);
+  u32x2 bias[2][4];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d = 32 * j + 8 * g + 4 * hh;
-      bias[j][g] = pr.bias ? *reinterpret_cast<const u32x2*>(pr.bias + n_proj + d) : u32x2{0, 0};
-      nw[j][g] = pr.nw ? *reinterpret_cast<const u32x2*>(pr.nw + d) : u32x2{one, one};
-      nb[j][g] = pr.nb ? *reinterpret_cast<const u32x2*>(pr.nb + d) : u32x2{0, 0};
-    }
+    for (int g = 0; g < 4; ++g)
+      bias[j][g] = pr.bias ? *reinterpret_cast<const u32x2*>(pr.bias + n_proj + 32 * j + 8 * g + 4 * hh) : u32x2{0, 0};
+  const int d = 8 * (lane & 7);   // of a row that comes back from the stage
+  const uint32_t one = pack2<kHalf>(1.f, 1.f);
+  const u32x4 nw = pr.nw ? *reinterpret_cast<const u32x4*>(pr.nw + d) : u32x4{one, one, one, one};
+  const u32x4 nb = pr.nb ? *reinterpret_cast<const u32x4*>(pr.nb + d) : u32x4{0, 0, 0, 0};
   wait_loads<0>();
   step_barrier();
   if (!mine) return;
@@ -253,58 +245,65 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
   for (int i = 0; i < MB; ++i) {
     const int block = (wm * MB + i) * 32, m_first = m0 + block;
     if (m_first >= a.M) break;
-    float v[32];
-#pragma unroll
-    for (int e = 0; e < 32; e += 2) {   // rounded as the projection's output is
-      const f32x2 b = unpack2<kHalf>(bias[e >> 4][(e >> 2) & 3][(e >> 1) & 1]);
-      const f32x2 r = unpack2<kHalf>(pack2<kHalf>(acc[e >> 4][i][e & 15] + b.x, acc[e >> 4][i][(e & 15) + 1] + b.y));
-      v[e] = r.x;
-      v[e + 1] = r.y;
-    }
-    if (pr.norm != DT_NORM_NONE) {
-      float sum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 32; ++e) sum += v[e];
-      sum += __shfl_xor(sum, 32);
-      const float mean = sum * (1.0f / kHead);
-      float ss = 0.f;
-#pragma unroll
-      for (int e = 0; e < 32; ++e) ss += (v[e] - mean) * (v[e] - mean);
-      ss += __shfl_xor(ss, 32);
-      const float rs = 1.0f / sqrtf(ss * (1.0f / kHead) + pr.eps);
-#pragma unroll
-      for (int e = 0; e < 32; e += 2) {
-        const f32x2 w = unpack2<kHalf>(nw[e >> 4][(e >> 2) & 3][(e >> 1) & 1]), b = unpack2<kHalf>(nb[e >> 4][(e >> 2) & 3][(e >> 1) & 1]);
-        v[e] = (v[e] - mean) * rs * w.x + b.x;
-        v[e + 1] = (v[e + 1] - mean) * rs * w.y + b.y;
-      }
-    }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {   // rounded as the norm's output is
-        const float* x = v + 16 * j + 4 * g;
-        *reinterpret_cast<u32x2*>(stage + col * (kHead * 2) + (((4 * j + g) ^ ((col >> 1) & 7)) << 4) + 8 * hh) =
-            u32x2{pack2<kHalf>(x[0], x[1]), pack2<kHalf>(x[2], x[3])};
+      for (int g = 0; g < 4; ++g) {   // rounded as the projection's output is
+        u32x2 x;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const f32x2 b = unpack2<kHalf>(bias[j][g][e]);
+          x[e] = pack2<kHalf>(acc[j][i][4 * g + 2 * e] + b.x, acc[j][i][4 * g + 2 * e + 1] + b.y);
+        }
+        *reinterpret_cast<u32x2*>(stage + col * (kHead * 2) + (((4 * j + g) ^ ((col >> 1) & 7)) << 4) + 8 * hh) = x;
       }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    // eight lanes a row, as in qk_norm_rope_kernel
+    u32x4 raw[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = 8 * r + (lane >> 3), d = 8 * (lane & 7);
-      u32x4 x = *reinterpret_cast<const u32x4*>(stage + row * (kHead * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
-      const int m = m_first + row;
+      const int row = 8 * r + (lane >> 3);
+      raw[r] = *reinterpret_cast<const u32x4*>(stage + row * (kHead * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+    }
+    if (pr.norm != DT_NORM_NONE) {
+      float mean[4], ss[4], rs[4], w[8], b[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v[8];
+        unpack8<kHalf>(raw[r], v);
+        mean[r] = row_sum<8>(v) * (1.0f / kHead);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] -= mean[r];
+        ss[r] = row_squares<8>(v);
+      }
+      inverse_rms4<kHead>(ss[0], ss[1], ss[2], ss[3], pr.eps, rs);
+      unpack8<kHalf>(nw, w);
+      unpack8<kHalf>(nb, b);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v[8];
+        unpack8<kHalf>(raw[r], v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = layer_norm16<kHalf>(v[e], mean[r], rs[r], w[e], b[e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) raw[r][e] = pack2<kHalf>(v[2 * e], v[2 * e + 1]);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 8 * r + (lane >> 3), m = m_first + row;
       if (pr.rope) {
         const float* c = tables + (block + row) * kHead + d;
         const bool video = m % a.S >= a.T;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const f32x2 z = unpack2<kHalf>(x[e]);
+          const f32x2 z = unpack2<kHalf>(raw[r][e]);
           const f32x2 cs = *reinterpret_cast<const f32x2*>(c + 2 * e), sn = *reinterpret_cast<const f32x2*>(c + kTable / 4 + 2 * e);
-          const uint32_t y = pack2<kHalf>(z.x * cs.x + -z.y * sn.x, z.y * cs.y + z.x * sn.y);
-          x[e] = video ? y : x[e];
+          const uint32_t y = pack2<kHalf>(rotated(z.x, -z.y, cs.x, sn.x), rotated(z.y, z.x, cs.y, sn.y));
+          raw[r][e] = video ? y : raw[r][e];
         }
       }
-      if (m < a.M) *reinterpret_cast<u32x4*>(pr.y + (int64_t)m * a.N + n_proj + d) = x;
+      if (m < a.M) *reinterpret_cast<u32x4*>(pr.y + (int64_t)m * a.N + n_proj + d) = raw[r];
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }

@@ -86,6 +86,39 @@ def test_projections_match_fp64(hip, B, T, V, H, K, dtype, bias, rotated):
         _check(got, _exact(attn, text, video, rope), dtype)
 
 
+@pytest.mark.parametrize("B,T,V,H,K", [
+    (2, 26, 170, 3, 128),
+    (2, 30, 1500, 30, 1920),     # columns of 22.5 tiles of 256, or 11.25 of 512; rows of two samples in one tile
+    (1, 113, 2500, 24, 1536),
+    (1, 28, 2194, 48, 3072),
+    (1, 28, 3301, 48, 3072),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_norm_and_rotation_are_the_producers_bit_for_bit(hip, B, T, V, H, K, dtype):
+    """The projections alone, then ``prepare_qk`` as the adapter calls it, against all of it in one launch; and the modules' products,
+    which the library adds up in one chain at these sizes."""
+    from ditango_amd.executor.cogvideox.projection import project_qkv
+    from ditango_amd.producer import prepare_qk
+    attn = _layer(H, K, dtype)
+    text, video, rope = _tokens(B, T, V, K, dtype)
+    bare = SimpleNamespace(**{**vars(attn), "norm_q": None, "norm_k": None})
+    x = torch.cat([text, video], 1)
+    with torch.no_grad():
+        got = project_qkv(attn, text, video, rope)
+        plain = project_qkv(bare, text, video, None)
+        for m, y in zip((attn.to_q, attn.to_k, attn.to_v), plain):
+            assert torch.equal(m(x).view_as(y), y)
+        for y, n, z in zip(plain, (attn.norm_q, attn.norm_k), got):
+            want = prepare_qk(y, norm="layer_norm", weight=n.weight, bias=n.bias, eps=n.eps, match_eager_rounding=True, rope="interleaved",
+                              freqs_cis=rope, rope_begin=T)
+            assert torch.equal(want, z)
+        for y, n, z in zip(plain, (attn.norm_q, attn.norm_k), project_qkv(attn, text, video, None)):
+            assert torch.equal(prepare_qk(y, norm="layer_norm", weight=n.weight, bias=n.bias, eps=n.eps, match_eager_rounding=True), z)
+        for y, z in zip(plain[:2], project_qkv(bare, text, video, rope)):
+            assert torch.equal(prepare_qk(y, rope="interleaved", freqs_cis=rope, rope_begin=T, match_eager_rounding=True), z)
+        assert torch.equal(plain[2], got[2])
+
+
 @pytest.mark.parametrize("H,K,V", [(2, 128, 150), (24, 1536, 2500), (48, 3072, 2194)])
 def test_a_row_depends_on_its_own_tokens_only(hip, H, K, V):
     """Every tile form: rows one by one, in another tile and beside other rows, come out bit for bit the same (one order of the sums)."""
