@@ -213,7 +213,10 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
   // workgroup's tokens come into the LDS once for all of its heads (from memory for each, the launch took 25 us longer).
   constexpr int kTable = BM * kHead * 4;
   float* tables = reinterpret_cast<float*>(lds + kStageBytes);
-  if (n0 < 2 * a.N && (a.proj[0].rope || a.proj[1].rope)) {
+  bool rotates = false;   // a projection of the workgroup's columns
+#pragma unroll
+  for (int p = 0; p < 3; ++p) rotates |= a.proj[p].rope && n0 < (p + 1) * a.N && n0 + BN > p * a.N;
+  if (rotates) {
 #pragma unroll
     for (int i = 0; i < BM / 32; ++i) {
       const int row = (i * kWaves + wave) * 4 + (lane >> 4), s = min(m0 + row, a.M - 1) % a.S;

@@ -119,6 +119,28 @@ def test_norm_and_rotation_are_the_producers_bit_for_bit(hip, B, T, V, H, K, dty
         assert torch.equal(plain[2], got[2])
 
 
+@pytest.mark.parametrize("T,V,H,K", [
+    (5, 100, 3, 64),           # one projection's columns end inside a tile
+    (113, 2500, 24, 1536),
+    (28, 2194, 48, 3072),
+    (28, 3301, 48, 3072),
+])
+@pytest.mark.parametrize("which", range(3))
+def test_rotation_of_one_projection_alone(hip, T, V, H, K, which):
+    """Every tile form, and each of the three places: bit for bit the producer's rotation of the bare product, the others untouched."""
+    from ditango_amd.producer import prepare_qk
+    attn = _layer(H, K, torch.bfloat16)
+    text, video, rope = _tokens(1, T, V, K, torch.bfloat16)
+    with torch.no_grad():
+        table = lambda turned: [(m.weight, m.bias, hip.DT_NORM_NONE, None, None, 0.0, i in turned)
+                                for i, m in enumerate((attn.to_q, attn.to_k, attn.to_v))]
+        plain = hip.qkv_project(text, video, H, table(()))
+        got = hip.qkv_project(text, video, H, table((which,)), *rope)
+        for i, (a, b) in enumerate(zip(plain, got)):
+            want = prepare_qk(a, rope="interleaved", freqs_cis=rope, rope_begin=T) if i == which else a
+            assert torch.equal(want, b), i
+
+
 @pytest.mark.parametrize("H,K,V", [(2, 128, 150), (24, 1536, 2500), (48, 3072, 2194)])
 def test_a_row_depends_on_its_own_tokens_only(hip, H, K, V):
     """Every tile form: rows one by one, in another tile and beside other rows, come out bit for bit the same (one order of the sums)."""
