@@ -62,9 +62,6 @@ __device__ __forceinline__ f32x2 load2(Rsrc r, uint32_t off, uint32_t uniform_of
   return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, uniform_off, 0));
 }
 
-// What stands in for a row of V past the end of a chunk.
-__device__ const float kZeroRow[4] = {};
-
 struct F32Chunk {
   const float *k, *v;
   int64_t sb, ss, sh;   // element strides
@@ -124,7 +121,9 @@ struct F32Lds {
   static constexpr int kPitch = D + 4;             // floats per query row of a wavefront's partial output
   static constexpr int kFloatsPerWave = kTile * kPitch + 2 * kTile;   // + maximum and sum of every query
   static constexpr int kWalk = kWavesF32 / QW * kGroupBytes, kEnd = kWavesF32 * kFloatsPerWave * 4;
-  static constexpr int kBytes = kWalk > kEnd ? kWalk : kEnd;
+  // behind both: a flag of every wavefront, and which columns of V have anything but zeros in the keys that a lane looked through
+  static constexpr int kFlags = kWalk > kEnd ? kWalk : kEnd, kColumns = kFlags + 64;
+  static constexpr int kBytes = kColumns + kThreadsF32 * 16;
 };
 // Transposing LDS read, see attn_fwd.hip.
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -185,7 +184,7 @@ __device__ __forceinline__ void tile_barrier() {
 // the end of the exponent range, which 2^90 times as large a K would bring back.
 constexpr uint32_t kTiny = (uint32_t)(127 - 100) << 23, kHuge = (uint32_t)(127 + 90) << 23;
 // Whether an element of O^T is one that the split products may have got wrong: not finite (an infinity leaves NaN behind where
-// it is split), or so small that its terms ended below the exponent range (or zero, which is as rare).
+// it is split), or so small that its terms may have ended below the exponent range, zero among them.
 constexpr uint32_t kOddFrom = 0xff000000u - 2 * kTiny;
 __device__ __forceinline__ uint32_t oddity(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 2 * kTiny; }
 
@@ -362,18 +361,21 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   const int d_mine = 4 * (lane % kRowLanes);
   auto row_mine = [&](int i) { return (i * QW + member) * kRowsPer + lane / kRowLanes; };
   f32x4 kreg[kLoads], vreg[kLoads];
+  // 16 bytes of a row of a tile; zeros past the end of the chunk
+  auto load_row = [&](const Cursor<kFar>& at, const float* base, int row, int d) __attribute__((always_inline)) {
+    if constexpr (kFar) {
+      f32x4 x = 0.f;
+      const int key = at.k0 + row;
+      if (key < at.len) x = *reinterpret_cast<const f32x4*>(base + (int64_t)key * at.ss + d);
+      return x;
+    } else {
+      // (the tile's offset is the scalar one: inside the buffer, as the range check subtracts it from the length)
+      return load4(buffer_of(base, at.plane), ((uint32_t)row * (uint32_t)at.ss + d) * 4u, (uint32_t)at.k0 * (uint32_t)at.ss * 4u);
+    }
+  };
   auto load_tile = [&](const Cursor<kFar>& at, const float* base, f32x4 (&reg)[kLoads]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      if constexpr (kFar) {
-        reg[i] = 0.f;
-        const int key = at.k0 + row_mine(i);
-        if (key < at.len) reg[i] = *reinterpret_cast<const f32x4*>(base + (int64_t)key * at.ss + d_mine);
-      } else {
-        // (the tile's offset is the scalar one: inside the buffer, as the range check subtracts it from the length)
-        reg[i] = load4(buffer_of(base, at.plane), ((uint32_t)row_mine(i) * (uint32_t)at.ss + d_mine) * 4u, (uint32_t)at.k0 * (uint32_t)at.ss * 4u);
-      }
-    }
+    for (int i = 0; i < kLoads; ++i) reg[i] = load_row(at, base, row_mine(i), d_mine);
   };
   uint8_t* planes = lds_f32 + group * L::kGroupBytes;
   auto put = [&](uint8_t* to, const f32x4& x) __attribute__((always_inline)) {
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
       qs[s] = split8(x);
     }
     big = fmaxf(big, __shfl_xor(big, 32));
-    odd_q = __builtin_bit_cast(uint32_t, big) - kTiny > kHuge - kTiny;
+    odd_q = big != 0.f && __builtin_bit_cast(uint32_t, big) - kTiny > kHuge - kTiny;   // (zero is three times zero)
   }
 
   f32x16 o[kNB];   // O^T: register r of block i is d = 32 i + 8 (r / 4) + 4 hh + r % 4
@@ -590,33 +592,80 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
       }
       *reinterpret_cast<f32x4*>(mine + col * L::kPitch + 32 * i + 8 * g + 4 * hh) = x;
     }
-  const bool odd_row = odd_q || !(l > 0.f && l < INFINITY);   // (no sum: a maximum whose reference is past the exponent range, or scores of -inf only)
-  if (__builtin_expect(any && __any(odd_row || worst >= kOddFrom), 0)) {
-    // Once more with fp32 products, for the elements and rows that need it; the others stay what they are.
-    float m2, l2;
-    walk_fp32<D, kFar>(a, b, h, job, q0, begin + group, KW, n_tiles, o, m2, l2);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const bool whole_row = odd_row || __shfl_xor((int)odd_row, 32) != 0;
-    const float f = __builtin_amdgcn_exp2f((m2 - m) * c);
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-#pragma unroll
-      for (int i = 0; i < kNB; ++i) {
-        float* x = mine + col * L::kPitch + (8 * (r >> 2) + 4 * hh + (r & 3)) * kNB + i;
-        if (whole_row) *x = o[i][r];
-        else if (oddity(*x) >= kOddFrom) *x = o[i][r] * f;
-      }
-    if (whole_row) {
-      m = m2;
-      l = l2;
-    }
-  }
   if (hh == 0) {
     mine[kTile * L::kPitch + col] = m;
     mine[kTile * L::kPitch + kTile + col] = l;
   }
-  if constexpr (KW > 1) __syncthreads();
-  else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // a wavefront reads back only what it wrote itself
+  const bool odd_row = odd_q || !(l > 0.f && l < INFINITY);   // (no sum: a maximum whose reference is past the exponent range, or scores of -inf only)
+  const bool suspect = any && __any(odd_row || worst >= kOddFrom);
+  uint32_t* flags = reinterpret_cast<uint32_t*>(lds_f32 + L::kFlags);
+  if (lane == 0) flags[wave] = suspect;
+  tile_barrier();
+  const u32x4 flag = *reinterpret_cast<const u32x4*>(flags);
+  if (__builtin_expect(__builtin_amdgcn_readfirstlane(flag.x | flag.y | flag.z | flag.w) != 0, 0)) {
+    // A zero below a column of V that is zero (a narrower head's padding, keys that are padding) is exact: the group's V is looked
+    // through once more, each wavefront its rows.  us, no zeros / a zero column computed once more / looked through: 12 heads x 1053 queries x
+    // 4212 keys, d = 64 105 / 260 / 106; 10 x 847 x 1694, d = 128 72 / 222 / 76; 12 x 355 x 2840 69 / 199 / 76.  (The columns' maxima taken
+    // while V is split cost every launch at d = 64 3 %.)
+    constexpr int kAtOnce = D / 4 / kLoads;   // tiles on their way together
+    // (a lane number of its own: with the loop's, the loop's addresses stay in registers until here and its schedule is 2 % longer)
+    int here = threadIdx.x & 63;
+    asm volatile("" : "+v"(here));
+    const int quad = here % kRowLanes, first_row = member * kRowsPer + here / kRowLanes;
+    u32x4 used = {0, 0, 0, 0};
+    Cursor<kFar> at(a, job, n_tiles);
+    bool left = at.advance(a, b, h, begin + group);
+    while (left) {
+      f32x4 x[kAtOnce][kLoads];
+#pragma unroll
+      for (int t = 0; t < kAtOnce; ++t) {   // (behind the last tile: zeros)
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) x[t][i] = load_row(at, at.vb, first_row + i * QW * kRowsPer, 4 * quad);
+        left = at.advance(a, b, h, KW);
+      }
+#pragma unroll
+      for (int t = 0; t < kAtOnce; ++t)
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) used |= __builtin_bit_cast(u32x4, x[t][i]) << 1;
+    }
+    uint8_t* columns = lds_f32 + L::kColumns + 1024 * group * QW + 16 * here;
+    *reinterpret_cast<u32x4*>(columns + 1024 * member) = used;
+    tile_barrier();
+    columns += 16 * (quad - here);
+    used = u32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < QW * kRowsPer; ++w) used |= *reinterpret_cast<const u32x4*>(columns + 16 * kRowLanes * w);
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(mine + (here & 31) * L::kPitch + 8 * i + 4 * (here >> 5));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool zeros = __shfl((int)used[e], 2 * i + (here >> 5)) == 0;   // (by all lanes)
+        odd |= !zeros && oddity(x[e]) >= kOddFrom;
+      }
+    }
+    if (any && __any(odd_row || odd)) {
+      // Once more with fp32 products, for the elements and rows that need it; the others stay what they are.
+      float m2, l2;
+      walk_fp32<D, kFar>(a, b, h, job, q0, begin + group, KW, n_tiles, o, m2, l2);
+      const bool whole_row = odd_row || __shfl_xor((int)odd_row, 32) != 0;
+      const float f = __builtin_amdgcn_exp2f((m2 - m) * c);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int i = 0; i < kNB; ++i) {
+          float* x = mine + col * L::kPitch + (8 * (r >> 2) + 4 * hh + (r & 3)) * kNB + i;
+          if (whole_row) *x = o[i][r];
+          else if (oddity(*x) >= kOddFrom) *x = o[i][r] * f;
+        }
+      if (whole_row && hh == 0) {
+        mine[kTile * L::kPitch + col] = m2;
+        mine[kTile * L::kPitch + kTile + col] = l2;
+      }
+    }
+    tile_barrier();
+  }
   const float* halves = reinterpret_cast<float*>(lds_f32) + member * L::kFloatsPerWave;   // group g: QW wavefronts on
   constexpr int kRowsPerWave = kTile / KW;
   // `row` of the workgroup's 32 QW

@@ -68,6 +68,58 @@ def test_infinities_in_one_part_of_the_keys(hip):
     assert torch.equal(out, want) and torch.equal(lse, want_lse)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_zeros_split_as_well_as_other_numbers(hip, D):
+    """Scores of zero from a row of Q that is zero, and from one that meets a zero column of K: the same numbers on the same way, bit for
+    bit; a zero column of V is zero, and the other columns are what they are beside another column."""
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(1, n, 3, D, generator=g) for n in (130, 700, 700))
+    k[..., 3] = 0
+    q[:, ::7] = 0
+    e3 = q.clone()
+    e3[:, ::7, :, 3] = 1
+    run = lambda q, v: hip.attn_jobs_f32_fwd(q.cuda(), [k.cuda()], [v.cuda()], [[0]])[0]
+    out, lse = run(q, v)
+    want, want_lse = run(e3, v)
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+    v0 = v.clone()
+    v0[..., 40] = 0
+    out, lse = run(e3, v0)
+    want = want.clone()
+    want[..., 40] = 0
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+
+
+@pytest.mark.parametrize("H,Sq,Sk,D", [(12, 1053, 4212, 64), (10, 847, 1694, 128)])
+def test_zeros_do_not_send_wavefronts_through_their_keys_again(hip, H, Sq, Sk, D):
+    """A padded row of Q in every tile, a padded column of V, padded keys: as long as without (2.2 to 2.6 times where a wavefront computes
+    once more; half as long again is allowed, runs differ by some per cent)."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q, k, v = (torch.randn(1, n, H, D, generator=g, device="cuda") for n in (Sq, Sk, Sk))
+
+    def us(q, k, v):
+        best = float("inf")
+        for _ in range(5):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            for _ in range(10):
+                hip.attn_jobs_f32_fwd(q, [k], [v], [[0]])
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 100)
+        return best
+
+    q0, k0, v0, v1 = q.clone(), k.clone(), v.clone(), v.clone()
+    q0[:, ::32] = 0
+    v0[..., 5] = 0
+    k0[:, -Sk // 4:] = 0
+    v1[:, -Sk // 4:] = 0
+    us(q, k, v)
+    plain = us(q, k, v)
+    for case in ((q0, k, v), (q, k, v0), (q, k0, v1)):
+        assert us(*case) < 1.5 * plain
+
+
 def test_scores_whose_reference_leaves_the_range(hip):
     """The largest score is finite and the next multiple of the grid above it is not: one key has all the weight."""
     q, k = torch.zeros(1, 40, 1, 64), torch.zeros(1, 70, 1, 64)
