@@ -11,8 +11,10 @@
 // below 2^-25 of the product, less than the one rounding of an fp32 multiply-add.  Small terms are added first, and a tile's share of O^T is
 // summed for itself and then added once.  Against fp64, over 22 launches of 96 ... 1680 queries x 190 ... 9560 keys: relative error (2-norm)
 // 1.6 ... 2.4e-7, where v_mfma_f32_32x32x2_f32 (64 cycles for two values a lane) gave 2.9 ... 4.6e-7 of the same numbers.
-// Numbers that do not split -- infinities, NaN, what ends below the exponent range -- show in the result (NaN, or less than 2^-100);
-// a wavefront that sees them walks its keys once more with fp32 products and takes the elements or rows concerned from there.
+// Numbers that do not split -- infinities, NaN, what ends below the exponent range -- show in Q or in the result (NaN, or less than
+// 2^-100); a wavefront that sees them walks its keys once more with fp32 products and takes the elements or rows concerned from there.
+// What does not show: a weight below 2^-110 loses up to 2^-126, which counts where its V is more than 2^100 times the result, and an element
+// of K below 2^-110 as much, which with |Q| <= 2^90 is 2^-36 of a score.
 //
 // What bounds it: a wavefront issues in order, and an MFMA holds it up (24 MFMAs with 88 vector instructions between them take as long as
 // one behind the other), so a tile takes 48 MFMAs x 32 cycles + 330 vector instructions x 4 at d = 64 (twice the MFMAs at 128), less what
@@ -180,9 +182,19 @@ __device__ __forceinline__ void tile_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// Magnitudes of a row of Q for which three bf16 values hold what counts of an fp32 one: below 2^-110 the last of them loses bits to
+// Magnitudes of an element of Q for which three bf16 values hold what counts of an fp32 one: below 2^-110 the last of them loses bits to
 // the end of the exponent range, which 2^90 times as large a K would bring back.
 constexpr uint32_t kTiny = (uint32_t)(127 - 100) << 23, kHuge = (uint32_t)(127 + 90) << 23;
+struct QRange {
+  float most = 0.f;
+  uint32_t least = ~0u;   // twice the bits, less one: zero, which is three times zero, is the largest
+  __device__ __forceinline__ void add(float x, float y) {
+    // (in assembly: fmaxf would first quiet what was loaded)
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(most) : "v"(x), "v"(y));
+    least = min(least, min((__builtin_bit_cast(uint32_t, x) << 1) - 1, (__builtin_bit_cast(uint32_t, y) << 1) - 1));
+  }
+  __device__ __forceinline__ bool odd() const { return __builtin_bit_cast(uint32_t, most) > kHuge || least < 2 * kTiny - 1; }
+};
 // Whether an element of O^T is one that the split products may have got wrong: not finite (an infinity leaves NaN behind where
 // it is split), or so small that its terms may have ended below the exponent range, zero among them.
 constexpr uint32_t kOddFrom = 0xff000000u - 2 * kTiny;
@@ -244,13 +256,13 @@ struct Cursor {
   }
 };
 
-// O^T of 32 queries against the cursor's tiles with fp32 products (v_mfma_f32_32x32x2_f32), straight from global memory: for the few
-// wavefronts whose numbers do not split.  An MFMA contracts two values, one per half of the wavefront; which two is free as long
+// O^T of 32 queries against the cursor's tiles with fp32 products (v_mfma_f32_32x32x2_f32), straight from global memory, and which half rows of Q
+// do not split: for the few wavefronts that have such numbers.  An MFMA contracts two values, one per half of the wavefront; which two is free as long
 // as both operands agree: halves 0 and 1 take d = 8 j + t and 8 j + 4 + t, and of P V the two keys whose probabilities they hold in
 // the same accumulator register.  Register r of block i is d = (8 (r / 4) + 4 hh + r % 4) D/32 + i.
 template <int D, bool kFar>
 __device__ __forceinline__ void walk_fp32(KernArgsF32& a, int b, int h, int job, int q0, int first, int step, int n, f32x16 (&o)[D / 32],
-                                          float& m, float& l) {
+                                          float& m, float& l, bool& odd_q) {
   constexpr int kNB = D / 32;
   constexpr int kKL = D / 8;       // 16-byte K loads of a lane per tile
   typedef float vvec __attribute__((ext_vector_type(kNB), aligned(4)));
@@ -260,6 +272,12 @@ __device__ __forceinline__ void walk_fp32(KernArgsF32& a, int b, int h, int job,
   const float* qp = a.q + (int64_t)b * a.q_sb + (int64_t)min(q0 + col, a.Sq - 1) * a.q_ss + (int64_t)h * a.q_sh + 4 * hh;
 #pragma unroll
   for (int j = 0; j < kKL; ++j) qf[j] = *reinterpret_cast<const f32x4*>(qp + 8 * j);
+  QRange range;
+#pragma unroll
+  for (int j = 0; j < kKL; ++j)
+#pragma unroll
+    for (int t = 0; t < 4; t += 2) range.add(qf[j][t], qf[j][t + 1]);
+  odd_q = range.odd();
 #pragma unroll
   for (int i = 0; i < kNB; ++i)
 #pragma unroll
@@ -431,7 +449,7 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
 
   // Q: B operand, d = 16 s + 8 hh + e (rows past Sq repeat the last one; their results are not stored)
   Split8 qs[D / 16];
-  bool odd_q;   // a row of Q outside the magnitudes that can be split
+  bool odd_q;   // a row of the wavefront's is outside the magnitudes that can be split
   {
     // Whole rows through the LDS (the output rows' place): as loads of 16 bytes of 32 different rows 0.2 to 1 us longer (us per call, 12 heads
     // x 280 queries x 560 keys, d = 128 27.9 -> 26.9, 10 x 114 x 456 22.7 -> 22.3; 4 x 512 x 2048, d = 64 21.7 -> 21.4).
@@ -447,19 +465,17 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) qv[i] = *reinterpret_cast<const f32x4*>(rows + col * L::kPitch + 16 * (i >> 1) + 8 * hh + 4 * (i & 1));
-    float big = 0.f;
+    QRange range;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        x[t] = qv[2 * s + (t >> 2)][t & 3];
-        big = fmaxf(big, __builtin_fabsf(x[t]));
-      }
+      for (int t = 0; t < 8; ++t) x[t] = qv[2 * s + (t >> 2)][t & 3];
+#pragma unroll
+      for (int t = 0; t < 8; t += 2) range.add(x[t], x[t + 1]);
       qs[s] = split8(x);
     }
-    big = fmaxf(big, __shfl_xor(big, 32));
-    odd_q = big != 0.f && __builtin_bit_cast(uint32_t, big) - kTiny > kHuge - kTiny;   // (zero is three times zero)
+    odd_q = __builtin_amdgcn_readfirstlane(__any(range.odd())) != 0;
   }
 
   f32x16 o[kNB];   // O^T: register r of block i is d = 32 i + 8 (r / 4) + 4 hh + r % 4
@@ -596,8 +612,8 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
     mine[kTile * L::kPitch + col] = m;
     mine[kTile * L::kPitch + kTile + col] = l;
   }
-  const bool odd_row = odd_q || !(l > 0.f && l < INFINITY);   // (no sum: a maximum whose reference is past the exponent range, or scores of -inf only)
-  const bool suspect = any && __any(odd_row || worst >= kOddFrom);
+  const bool odd_sum = !(l > 0.f && l < INFINITY);   // (no sum: a maximum whose reference is past the exponent range, or scores of -inf only)
+  const bool suspect = any && (odd_q || __any(odd_sum || worst >= kOddFrom));
   uint32_t* flags = reinterpret_cast<uint32_t*>(lds_f32 + L::kFlags);
   if (lane == 0) flags[wave] = suspect;
   tile_barrier();
@@ -645,11 +661,13 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
         odd |= !zeros && oddity(x[e]) >= kOddFrom;
       }
     }
-    if (any && __any(odd_row || odd)) {
+    if (any && (odd_q || __any(odd_sum || odd))) {
       // Once more with fp32 products, for the elements and rows that need it; the others stay what they are.
       float m2, l2;
-      walk_fp32<D, kFar>(a, b, h, job, q0, begin + group, KW, n_tiles, o, m2, l2);
-      const bool whole_row = odd_row || __shfl_xor((int)odd_row, 32) != 0;
+      bool odd_half;   // (of the lane's half of its row of Q)
+      walk_fp32<D, kFar>(a, b, h, job, q0, begin + group, KW, n_tiles, o, m2, l2, odd_half);
+      const bool other_half = __shfl_xor((int)odd_half, 32) != 0;   // (exchanged by all lanes)
+      const bool whole_row = odd_sum || odd_half || other_half;
       const float f = __builtin_amdgcn_exp2f((m2 - m) * c);
 #pragma unroll
       for (int r = 0; r < 16; ++r)

@@ -54,6 +54,16 @@ def test_magnitudes_at_the_ends_of_the_range(hip, D, q_scale, k_scale, v_scale):
     _check(hip, q, ks, vs, [[0]], True)
 
 
+@pytest.mark.parametrize("D,column", [(64, 3), (64, 60), (128, 5), (128, 77)])
+def test_one_small_element_of_q_that_a_large_one_of_k_makes_count(hip, D, column):
+    """The rest of the row is of ordinary size, and so are the scores."""
+    g = torch.Generator().manual_seed(column)
+    q, k, v = (torch.randn(1, n, 2, D, generator=g) for n in (70, 300, 300))
+    q[..., column] *= 2.0 ** -122
+    k[..., column] *= 2.0 ** 124
+    _check(hip, q, [k], [v], [[0]], True)
+
+
 def test_infinities_in_one_part_of_the_keys(hip):
     """An infinity of V leaves the other columns, and a key of infinite score the other rows, bit for bit what they are."""
     g = torch.Generator().manual_seed(5)
