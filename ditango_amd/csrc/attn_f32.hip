@@ -123,7 +123,7 @@ struct F32Lds {
   static constexpr int kPitch = D + 4;             // floats per query row of a wavefront's partial output
   static constexpr int kFloatsPerWave = kTile * kPitch + 2 * kTile;   // + maximum and sum of every query
   static constexpr int kWalk = kWavesF32 / QW * kGroupBytes, kEnd = kWavesF32 * kFloatsPerWave * 4;
-  // behind both: a flag of every wavefront, and which columns of V have anything but zeros in the keys that a lane looked through
+  // behind both: a flag of every wavefront, and the largest of every column of V in the keys that a lane looked through
   static constexpr int kFlags = kWalk > kEnd ? kWalk : kEnd, kColumns = kFlags + 64;
   static constexpr int kBytes = kColumns + kThreadsF32 * 16;
 };
@@ -196,7 +196,8 @@ struct QRange {
   __device__ __forceinline__ bool odd() const { return __builtin_bit_cast(uint32_t, most) > kHuge || least < 2 * kTiny - 1; }
 };
 // Whether an element of O^T is one that the split products may have got wrong: not finite (an infinity leaves NaN behind where
-// it is split), or so small that its terms may have ended below the exponent range, zero among them.
+// it is split), or so small that its terms may have ended below the exponent range, zero among them.  A zero is also what terms of ordinary
+// size leave now and then (once in some million elements of random numbers), or a column of V that is zero.
 constexpr uint32_t kOddFrom = 0xff000000u - 2 * kTiny;
 __device__ __forceinline__ uint32_t oddity(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 2 * kTiny; }
 
@@ -619,16 +620,17 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   tile_barrier();
   const u32x4 flag = *reinterpret_cast<const u32x4*>(flags);
   if (__builtin_expect(__builtin_amdgcn_readfirstlane(flag.x | flag.y | flag.z | flag.w) != 0, 0)) {
-    // A zero below a column of V that is zero (a narrower head's padding, keys that are padding) is exact: the group's V is looked
-    // through once more, each wavefront its rows.  us, no zeros / a zero column computed once more / looked through: 12 heads x 1053 queries x
-    // 4212 keys, d = 64 105 / 260 / 106; 10 x 847 x 1694, d = 128 72 / 222 / 76; 12 x 355 x 2840 69 / 199 / 76.  (The columns' maxima taken
-    // while V is split cost every launch at d = 64 3 %.)
+    // A zero below a column of V that is zero (a narrower head's padding, keys that are padding) is exact.  Below one with an element of
+    // ordinary size it is what terms leave that cancel; what small elements beside that one lost is below 2^-126.  So the group's V is looked
+    // through once more for the largest of every column, each wavefront its rows.  us, no zeros / a zero column computed once more /
+    // looked through: 12 heads x 1053 queries x 4212 keys, d = 64 105 / 260 / 106; 10 x 847 x 1694, d = 128 72 / 222 / 76; 12 x 355 x 2840
+    // 69 / 199 / 76.  (The maxima taken while V is split cost every launch at d = 64 3 %.)
     constexpr int kAtOnce = D / 4 / kLoads;   // tiles on their way together
     // (a lane number of its own: with the loop's, the loop's addresses stay in registers until here and its schedule is 2 % longer)
     int here = threadIdx.x & 63;
     asm volatile("" : "+v"(here));
     const int quad = here % kRowLanes, first_row = member * kRowsPer + here / kRowLanes;
-    u32x4 used = {0, 0, 0, 0};
+    u32x4 most = {0, 0, 0, 0};   // (twice the bits: the order of magnitudes)
     Cursor<kFar> at(a, job, n_tiles);
     bool left = at.advance(a, b, h, begin + group);
     while (left) {
@@ -642,23 +644,23 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
 #pragma unroll
       for (int t = 0; t < kAtOnce; ++t)
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) used |= __builtin_bit_cast(u32x4, x[t][i]) << 1;
+        for (int i = 0; i < kLoads; ++i) most = __builtin_elementwise_max(most, __builtin_bit_cast(u32x4, x[t][i]) << 1);
     }
     uint8_t* columns = lds_f32 + L::kColumns + 1024 * group * QW + 16 * here;
-    *reinterpret_cast<u32x4*>(columns + 1024 * member) = used;
+    *reinterpret_cast<u32x4*>(columns + 1024 * member) = most;
     tile_barrier();
     columns += 16 * (quad - here);
-    used = u32x4{0, 0, 0, 0};
+    most = u32x4{0, 0, 0, 0};
 #pragma unroll
-    for (int w = 0; w < QW * kRowsPer; ++w) used |= *reinterpret_cast<const u32x4*>(columns + 16 * kRowLanes * w);
+    for (int w = 0; w < QW * kRowsPer; ++w) most = __builtin_elementwise_max(most, *reinterpret_cast<const u32x4*>(columns + 16 * kRowLanes * w));
     bool odd = false;
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(mine + (here & 31) * L::kPitch + 8 * i + 4 * (here >> 5));
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bool zeros = __shfl((int)used[e], 2 * i + (here >> 5)) == 0;   // (by all lanes)
-        odd |= !zeros && oddity(x[e]) >= kOddFrom;
+        const uint32_t column = (uint32_t)__shfl((int)most[e], 2 * i + (here >> 5));   // (by all lanes)
+        odd |= oddity(x[e]) >= kOddFrom && column != 0 && (x[e] != 0.f || column < 2 * kTiny);
       }
     }
     if (any && (odd_q || __any(odd_sum || odd))) {

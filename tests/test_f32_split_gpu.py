@@ -102,8 +102,8 @@ def test_zeros_split_as_well_as_other_numbers(hip, D):
 
 @pytest.mark.parametrize("H,Sq,Sk,D", [(12, 1053, 4212, 64), (10, 847, 1694, 128)])
 def test_zeros_do_not_send_wavefronts_through_their_keys_again(hip, H, Sq, Sk, D):
-    """A padded row of Q in every tile, a padded column of V, padded keys: as long as without (2.2 to 2.6 times where a wavefront computes
-    once more; half as long again is allowed, runs differ by some per cent)."""
+    """A padded row of Q in every tile, a padded column of V, padded keys, terms that cancel: as long as without (2.2 to 2.6 times where a
+    wavefront computes once more; half as long again is allowed, runs differ by some per cent)."""
     g = torch.Generator(device="cuda").manual_seed(9)
     q, k, v = (torch.randn(1, n, H, D, generator=g, device="cuda") for n in (Sq, Sk, Sk))
 
@@ -124,9 +124,16 @@ def test_zeros_do_not_send_wavefronts_through_their_keys_again(hip, H, Sq, Sk, D
     v0[..., 5] = 0
     k0[:, -Sk // 4:] = 0
     v1[:, -Sk // 4:] = 0
+    # in every tile of 32 keys two equal ones, whose V in one column are opposite and the others' zero: a sum of exactly zero
+    k2, v2 = k.clone(), v0.clone()
+    k2[:, 1::32] = k2[:, 0::32][:, :k2[:, 1::32].shape[1]]
+    v2[:, 0::32, :, 5] = 1
+    v2[:, 1::32, :, 5] = -1
+    v2[:, -(Sk % 32) or Sk:, :, 5] = 0
+    assert (hip.attn_jobs_f32_fwd(q, [k2], [v2], [[0]])[0][0][..., 5] == 0).all()
     us(q, k, v)
     plain = us(q, k, v)
-    for case in ((q0, k, v), (q, k, v0), (q, k0, v1)):
+    for case in ((q0, k, v), (q, k, v0), (q, k0, v1), (q, k2, v2)):
         assert us(*case) < 1.5 * plain
 
 
