@@ -260,7 +260,7 @@ def attn_jobs_f32_fwd(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunk
     counters."""
     _require(q.is_cuda and q.dim() == 4, "q must be fp32 [B,S,H,D] on the GPU with contiguous D")
     B, Sq, H, _ = q.shape
-    need = len(jobs) * B * H * (-(-Sq // 64))
+    need = len(jobs) * B * H * (-(-Sq // 32))
     counters = torch.zeros(need, dtype=torch.int32, device=q.device) if torch.cuda.is_current_stream_capturing() \
         else _stream_counters(q.device, need)
     return _host().attn_states_f32(q, k_chunks, v_chunks, jobs, softmax_scale, _stream(), lse_bsh, attn_workspace(q.device), counters)

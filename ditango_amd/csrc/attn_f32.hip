@@ -26,6 +26,7 @@
 //   * Scores are computed transposed, S^T = K Q^T: a lane owns ONE query (column lane % 32) and 16 of the tile's keys, the row maximum is an
 //     in-register reduction plus one exchange with lane ^ 32, and with the rows of K permuted the probabilities are where the
 //     second product needs them.
+//   * In a small launch nothing is shared (QW = 1): a wavefront splits all of its tiles from memory to registers, and nobody waits for anybody.
 //   * Where the queries alone leave the chip idle, `parts` workgroups share the keys of a work item (plan_f32).
 //   * Measured (us per call with the GPU kept busy, kernel of fp32 products and merge kernel behind it -> this, which needs no other):
 //     4 heads x 512 queries x 2048 keys, d = 64 30 -> 21; 12 x 1053 x 4212 163 -> 101; 8 x 1195 x 9560 258 -> 154 (157 TFLOP/s, as much as
@@ -122,7 +123,7 @@ struct F32Lds {
   // behind that: the output rows of every wavefront
   static constexpr int kPitch = D + 4;             // floats per query row of a wavefront's partial output
   static constexpr int kFloatsPerWave = kTile * kPitch + 2 * kTile;   // + maximum and sum of every query
-  static constexpr int kWalk = kWavesF32 / QW * kGroupBytes, kEnd = kWavesF32 * kFloatsPerWave * 4;
+  static constexpr int kWalk = QW == 1 ? 0 : kWavesF32 / QW * kGroupBytes, kEnd = kWavesF32 * kFloatsPerWave * 4;
   // behind both: a flag of every wavefront, and the largest of every column of V in the keys that a lane looked through
   static constexpr int kFlags = kWalk > kEnd ? kWalk : kEnd, kColumns = kFlags + 64;
   static constexpr int kBytes = kColumns + kThreadsF32 * 16;
@@ -337,7 +338,8 @@ __device__ __forceinline__ void walk_fp32(KernArgsF32& a, int b, int h, int job,
 }
 
 // QW query tiles of 32 and KW groups of key tiles: wavefront w works on query tile w % QW of the workgroup and on every KW-th key
-// tile of the workgroup's part.  The QW wavefronts of a group share what they split.
+// tile of the workgroup's part.  The QW wavefronts of a group share what they split; with QW = 1 there is nothing to share, and operands go from
+// memory to the registers that the MFMAs read.
 template <int D, int QW, bool kFar>
 __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(const AttnF32Args args_by_value) {
   constexpr int KW = kWavesF32 / QW;
@@ -380,21 +382,23 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   const int d_mine = 4 * (lane % kRowLanes);
   auto row_mine = [&](int i) { return (i * QW + member) * kRowsPer + lane / kRowLanes; };
   f32x4 kreg[kLoads], vreg[kLoads];
-  // 16 bytes of a row of a tile; zeros past the end of the chunk
-  auto load_row = [&](const Cursor<kFar>& at, const float* base, int row, int d) __attribute__((always_inline)) {
+  // 16 bytes (or 8) of a row of a tile; zeros past the end of the chunk
+  auto load_row = [&](const Cursor<kFar>& at, const float* base, int row, int d, auto x) __attribute__((always_inline)) {
+    x = 0.f;
     if constexpr (kFar) {
-      f32x4 x = 0.f;
       const int key = at.k0 + row;
-      if (key < at.len) x = *reinterpret_cast<const f32x4*>(base + (int64_t)key * at.ss + d);
+      if (key < at.len) x = *reinterpret_cast<const decltype(x)*>(base + (int64_t)key * at.ss + d);
       return x;
     } else {
       // (the tile's offset is the scalar one: inside the buffer, as the range check subtracts it from the length)
-      return load4(buffer_of(base, at.plane), ((uint32_t)row * (uint32_t)at.ss + d) * 4u, (uint32_t)at.k0 * (uint32_t)at.ss * 4u);
+      const uint32_t off = ((uint32_t)row * (uint32_t)at.ss + d) * 4u, tile_off = (uint32_t)at.k0 * (uint32_t)at.ss * 4u;
+      if constexpr (sizeof(x) == 16) return load4(buffer_of(base, at.plane), off, tile_off);
+      else return load2(buffer_of(base, at.plane), off, tile_off);
     }
   };
   auto load_tile = [&](const Cursor<kFar>& at, const float* base, f32x4 (&reg)[kLoads]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) reg[i] = load_row(at, base, row_mine(i), d_mine);
+    for (int i = 0; i < kLoads; ++i) reg[i] = load_row(at, base, row_mine(i), d_mine, f32x4());
   };
   uint8_t* planes = lds_f32 + group * L::kGroupBytes;
   auto put = [&](uint8_t* to, const f32x4& x) __attribute__((always_inline)) {
@@ -445,8 +449,19 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
 
   const bool any = at_k.advance(a, b, h, begin + group);
   bool more = at_v.advance(a, b, h, begin + group);
-  load_tile(at_k, at_k.kb, kreg);
-  load_tile(at_v, at_v.vb, vreg);
+  // QW = 1: the elements of a lane's operands, key krow of K and keys 16 (r / 8) + 8 hh + r % 8 of V, d = col D/32 + i
+  typedef float vvec __attribute__((ext_vector_type(kNB), aligned(4)));
+  f32x4 k1[QW == 1 ? D / 8 : 1];
+  auto load_k1 = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) k1[j] = load_row(at_k, at_k.kb, krow, 16 * (j >> 1) + 8 * hh + 4 * (j & 1), f32x4());
+  };
+  if constexpr (QW == 1) {
+    load_k1();
+  } else {
+    load_tile(at_k, at_k.kb, kreg);
+    load_tile(at_v, at_v.vb, vreg);
+  }
 
   // Q: B operand, d = 16 s + 8 hh + e (rows past Sq repeat the last one; their results are not stored)
   Split8 qs[D / 16];
@@ -488,6 +503,105 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
   // exp2(-inf) = 0 and no sum, without a test for it.
   float m = -FLT_MAX, l = 0.f;
 
+  // (the small terms for themselves: D / 16 sums at the magnitude of the score are rounded, not six times as many)
+  auto scores = [&](const bf16x8& kh, const bf16x8& km, const bf16x8& kl, const Split8& q, f32x16& s, f32x16& small) __attribute__((always_inline)) {
+    small = mfma16(kl, q.h, small);
+    small = mfma16(kh, q.l, small);
+    small = mfma16(km, q.m, small);
+    small = mfma16(km, q.h, small);
+    small = mfma16(kh, q.m, small);
+    s = mfma16(kh, q.h, s);
+  };
+  // weights of a tile's scores, as operands; the factor of what was summed before
+  auto weigh = [&](f32x16& s, int valid, float& alpha, Split8 (&ps)[2]) __attribute__((always_inline)) {
+    if (__builtin_expect(valid < kTile, 0)) {
+      asm volatile("" ::: "memory");   // keeps this a real branch
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (16 * (r >> 3) + 8 * hh + (r & 7) >= valid) s[r] = -INFINITY;
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    // The reference is the next multiple of a.grid (a power of two, 2 to 4 in the exponent): rows, groups and parts of one magnitude have
+    // the same one, and their sums meet with weights that are exactly 1.
+    const float m_new = fmaxf(m, ceilf(mx * a.inv_grid) * a.grid);
+    alpha = __builtin_amdgcn_exp2f((m - m_new) * c);   // (0 on the first tile, or 1 with nothing to rescale)
+    m = m_new;
+    // the difference first, then the scale: the exponent is exact to its own rounding however large the scores are
+    float sum[2] = {0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f((s[r] - m) * c);
+      sum[r & 1] += s[r];
+    }
+    l = fmaf(l, alpha, sum[0] + sum[1]);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float p[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) p[e] = s[8 * g + e];
+      ps[g] = split8(p);
+    }
+  };
+  if constexpr (QW == 1) {
+    while (more) {
+      const int valid = at_v.len - at_v.k0;
+      vvec v1[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) v1[r] = load_row(at_v, at_v.vb, 16 * (r >> 3) + 8 * hh + (r & 7), kNB * col, vvec());
+      __builtin_amdgcn_sched_barrier(0);   // V is on its way before the scores are computed
+      f32x16 s, small;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = small[r] = 0.f;
+#pragma unroll
+      for (int j = 0; j < D / 16; ++j) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = k1[2 * j + (e >> 2)][e & 3];
+        const Split8 ks = split8(x);
+        scores(ks.h, ks.m, ks.l, qs[j], s, small);
+      }
+      at_k.advance(a, b, h, KW);
+      load_k1();
+      __builtin_amdgcn_sched_barrier(0);
+      more = at_v.advance(a, b, h, KW);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] += small[r];
+      float alpha;
+      Split8 ps[2];
+      weigh(s, valid, alpha, ps);
+#pragma unroll
+      for (int i = 0; i < kNB; ++i) {
+        Split8 vs[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          float x[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[e] = v1[8 * g + e][i];
+          vs[g] = split8(x);
+        }
+        f32x16 t;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[r] = 0.f;
+        t = mfma16(vs[0].l, ps[0].h, t);
+        t = mfma16(vs[1].l, ps[1].h, t);
+        t = mfma16(vs[0].h, ps[0].l, t);
+        t = mfma16(vs[1].h, ps[1].l, t);
+        t = mfma16(vs[0].m, ps[0].m, t);
+        t = mfma16(vs[1].m, ps[1].m, t);
+        t = mfma16(vs[0].m, ps[0].h, t);
+        t = mfma16(vs[1].m, ps[1].h, t);
+        t = mfma16(vs[0].h, ps[0].m, t);
+        t = mfma16(vs[1].h, ps[1].m, t);
+        t = mfma16(vs[0].h, ps[0].h, t);
+        t = mfma16(vs[1].h, ps[1].h, t);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] = fmaf(o[i][r], alpha, t[r]);
+      }
+    }
+  } else {
   tile_barrier();   // (everybody has Q)
   if (turns > 0) {
     put_k();
@@ -504,55 +618,19 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
 #pragma unroll
       for (int p = 0; p < 3; ++p) kf[j][p] = k_frag(p, j);
     put_v();
-    f32x16 s, small;   // (the small terms for themselves: D / 16 sums at the magnitude of the score are rounded, not six times as many)
+    f32x16 s, small;
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = small[r] = 0.f;
 #pragma unroll
-    for (int j = 0; j < D / 16; ++j) {
-      const bf16x8 kh = kf[j][0], km = kf[j][1], kl = kf[j][2];
-      small = mfma16(kl, qs[j].h, small);
-      small = mfma16(kh, qs[j].l, small);
-      small = mfma16(km, qs[j].m, small);
-      small = mfma16(km, qs[j].h, small);
-      small = mfma16(kh, qs[j].m, small);
-      s = mfma16(kh, qs[j].h, s);
-    }
+    for (int j = 0; j < D / 16; ++j) scores(kf[j][0], kf[j][1], kf[j][2], qs[j], s, small);
     interleave(std::integral_constant<int, 3 * D / 16>(), std::integral_constant<int, 6 * D / 16>());
     more = at_v.advance(a, b, h, KW);
     load_tile(at_v, at_v.vb, vreg);
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] += small[r];
-    if (__builtin_expect(valid < kTile, 0)) {
-      asm volatile("" ::: "memory");   // keeps this a real branch
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (16 * (r >> 3) + 8 * hh + (r & 7) >= valid) s[r] = -INFINITY;
-    }
-    float mx = s[0];
-#pragma unroll
-    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    // The reference is the next multiple of a.grid (a power of two, 2 to 4 in the exponent): rows, groups and parts of one magnitude have
-    // the same one, and their sums meet with weights that are exactly 1.
-    const float m_new = fmaxf(m, ceilf(mx * a.inv_grid) * a.grid);
-    const float alpha = __builtin_amdgcn_exp2f((m - m_new) * c);   // (0 on the first tile, or 1 with nothing to rescale)
-    m = m_new;
-    // the difference first, then the scale: the exponent is exact to its own rounding however large the scores are
-    float sum[2] = {0.f, 0.f};
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f((s[r] - m) * c);
-      sum[r & 1] += s[r];
-    }
-    l = fmaf(l, alpha, sum[0] + sum[1]);
+    float alpha;
     Split8 ps[2];
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      float p[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) p[e] = s[8 * g + e];
-      ps[g] = split8(p);
-    }
+    weigh(s, valid, alpha, ps);
     tile_barrier();
     // V of this tile is in the LDS, and nobody reads its K any more
     // The tile's share of O^T is summed for itself, the small terms first: one rounding at the magnitude of O^T per tile.
@@ -592,23 +670,37 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
     load_tile(at_k, at_k.kb, kreg);
     tile_barrier();
   }
+  }
   l += __shfl_xor(l, 32);
 
   // ---- epilogue: O^T -> LDS as [query][d] (the tiles' place), then whole rows to memory; the groups are folded on the way
   float* mine = reinterpret_cast<float*>(lds_f32) + wave * L::kFloatsPerWave;
   uint32_t worst = 0;
+  if constexpr (QW == 1) {   // (register r of block i is d = (8 (r / 4) + 4 hh + r % 4) D/32 + i)
 #pragma unroll
-  for (int i = 0; i < kNB; ++i)
+    for (int r = 0; r < 16; ++r) {
+      vvec x;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f32x4 x;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[e] = o[i][4 * g + e];
-        worst = max(worst, oddity(x[e]));
+      for (int i = 0; i < kNB; ++i) {
+        x[i] = o[i][r];
+        worst = max(worst, oddity(x[i]));
       }
-      *reinterpret_cast<f32x4*>(mine + col * L::kPitch + 32 * i + 8 * g + 4 * hh) = x;
+      *reinterpret_cast<vvec*>(mine + col * L::kPitch + (8 * (r >> 2) + 4 * hh + (r & 3)) * kNB) = x;
     }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kNB; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[e] = o[i][4 * g + e];
+          worst = max(worst, oddity(x[e]));
+        }
+        *reinterpret_cast<f32x4*>(mine + col * L::kPitch + 32 * i + 8 * g + 4 * hh) = x;
+      }
+  }
   if (hh == 0) {
     mine[kTile * L::kPitch + col] = m;
     mine[kTile * L::kPitch + kTile + col] = l;
@@ -638,7 +730,7 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
 #pragma unroll
       for (int t = 0; t < kAtOnce; ++t) {   // (behind the last tile: zeros)
 #pragma unroll
-        for (int i = 0; i < kLoads; ++i) x[t][i] = load_row(at, at.vb, first_row + i * QW * kRowsPer, 4 * quad);
+        for (int i = 0; i < kLoads; ++i) x[t][i] = load_row(at, at.vb, first_row + i * QW * kRowsPer, 4 * quad, f32x4());
         left = at.advance(a, b, h, KW);
       }
 #pragma unroll
@@ -827,40 +919,49 @@ int launch_f32(AttnF32Args& a, int n_jobs, hipStream_t stream) {
 }
 
 // Query tiles of a workgroup and workgroups that share the keys of a work item.  What a launch takes, in us: its rounds of workgroups
-// times the turns of one times what a turn takes (one workgroup on a CU, and at d = 64 two), and what a workgroup costs on top: start, end,
-// and the fold of the parts.  Four query tiles a workgroup split K and V half as often as two, but fold twice the bytes and leave a
-// small launch fewer workgroups.  The constants are fitted to 22 launches of 1 ... 12 heads x 96 ... 1680 queries against 2 ... 8
-// chunks of as many keys, in every split up to 16 (300 timings): the plan takes at most 2.8 % more than the best of them, 0.3 % on average.
-// us unsplit, -> as planned: 4 heads x 512 queries x 2048 keys, d = 64 67 -> 21 (8 parts); 12 x 1680 x 3360, d = 64 168 -> 111 (3 parts
-// of 4 query tiles); 10 x 847 x 1694, d = 128 111 -> 73 (3 of 4); 2 x 553 x 4424, d = 128 152 -> 53 (8).
+// times the turns of one times what a turn takes (one workgroup on a CU, and at d = 64 two), and what a launch, a round, a second workgroup on a CU and
+// the fold of the parts cost on top.  Four query tiles a workgroup split K and V half as often as two, but fold twice the bytes and leave a
+// small launch fewer workgroups; one query tile splits everything itself, and starts and ends sooner, with four groups of keys and no barriers
+// in between.  The constants are fitted to 190 shapes of 1 ... 24 heads x 32 ... 4096 queries against 1 ... 8 chunks of 64 ... 2048 keys, as one
+// job and a job a chunk, in every form and split (7300 timings, errors 5 to 8 %); in launches of several rounds, where the forms are close, a
+// split or one query tile has to gain more than 3 %.  The plan takes 0.5 % more than the best form on average with scratch and 0.1 %
+// without, at most 14 % (6 heads x 1005 queries x 8 jobs of 24 tiles, d = 64).
+// us unsplit -> as planned, two query tiles or more -> one too: 4 heads x 512 queries x 2048 keys, d = 64 67 -> 22 -> 19 (4 parts);
+// 2 x 553 x 4424 134 -> 30 -> 22, d = 128 245 -> 48 -> 39; 1 x 32 x 64, d = 128 13.8 -> 11.1 (1 part); without scratch, which parts
+// need, 4 x 512 x 2048, d = 64 67 -> 37, d = 128 119 -> 66.
 struct F32Plan {
   int qw = 2, parts = 1;
 };
 struct F32Cost {
-  double one, two, base, fold;   // a turn alone, beside another workgroup's; a launch; a part
+  double one, two;      // a turn alone, beside another workgroup's
+  double launch, parts, part;
+  double round, pair;   // a further round; a second workgroup on a CU
 };
-F32Plan plan_f32(int D, int heads, int Sq, int n_jobs, int tiles, int64_t workspace_bytes, int64_t n_counters) {
-  constexpr F32Cost kCost[2][2] = {{{1.45, 3.15, 14.0, 0.15}, {1.4, 2.66, 14.5, 0.5}}, {{3.15, 0, 17.0, 0.3}, {2.6, 0, 23.0, 0.6}}};
+F32Plan plan_f32(int D, int heads, int Sq, int n_jobs, int tiles, bool far, int64_t workspace_bytes, int64_t n_counters) {
+  constexpr F32Cost kCost[2][3] = {{{1.84, 3.18, 5.8, 3.2, 0.15, 2.1, 1.5}, {1.87, 2.95, 7.3, 2.7, 0.42, 2.1, 1.0}, {1.58, 2.57, 7.9, 2.8, 0.57, 1.1, 2.9}},
+                                   {{3.7, 0, 8.5, 3.2, 0.36, 5.2, 0}, {3.49, 0, 10.9, 2.9, 0.6, 6.3, 0}, {2.92, 0, 12.4, 3.1, 0.86, 6.0, 0}}};
   constexpr int64_t kCus = 32;   // of an XCD
   F32Plan best;
   double least = 1e30;
-  for (int qw = 2; qw <= 4; qw += 2) {
-    const F32Cost& t = kCost[D == 128][qw == 4];
-    const int64_t items = (int64_t)heads * ((Sq + kTile * qw - 1) / (kTile * qw)) * n_jobs, per_xcd = (items + 7) / 8;
+  for (int qw = 1; qw <= (far ? 2 : 4); qw *= 2) {
+    const F32Cost& t = kCost[D == 128][qw >> 1];
+    const int64_t items = (int64_t)heads * ((Sq + kTile * qw - 1) / (kTile * qw)), per_xcd = (items + 7) / 8 * n_jobs;
     const int kw = kWavesF32 / qw;
     for (int parts = 1; parts <= kMaxParts; ++parts) {
-      if (parts > 1 && (parts * kw > tiles || items > n_counters || items * parts * (kTile * qw) * (D + 2) * 4 > workspace_bytes)) break;
+      if (parts > 1 && (parts * kw > tiles || items * n_jobs > n_counters || items * n_jobs * parts * (kTile * qw) * (D + 2) * 4 > workspace_bytes)) break;
       const double turns = (tiles + kw * parts - 1) / (kw * parts);
       const int64_t groups = per_xcd * parts;
-      double time = t.base + (parts > 1 ? 1.0 + t.fold * parts : 0.0);
+      double time = t.launch + (parts > 1 ? t.parts + t.part * parts : 0.0);
       if (D == 128) {
         const int64_t rounds = (groups + kCus - 1) / kCus;
-        time += rounds * turns * t.one + (rounds - 1) * 7.0;
+        time += rounds * turns * t.one + (rounds - 1) * t.round;
       } else {
         const int64_t full = groups / (2 * kCus), rest = groups % (2 * kCus);
         time += full * turns * t.two + (rest == 0 ? 0.0 : rest <= kCus ? turns * t.one : turns * t.two);
-        time += (full + (rest > 0) - 1) * 2.5;
+        time += (full + (rest > 0) - 1) * t.round + (groups > kCus ? t.pair : 0.0);
       }
+      if (parts > 1 && per_xcd > kCus) time *= 1.03;
+      if (qw == 1 && groups > 2 * kCus) time *= 1.03;
       if (time < least) {
         least = time;
         best.qw = qw;
@@ -957,9 +1058,9 @@ extern "C" int dt_attn_jobs_f32_ws_fwd(const float* q, int32_t B, int32_t Sq, in
     for (int e = job_begin[j]; e < job_begin[j + 1]; ++e) n += ((int64_t)kv_lens[job_chunks[e]] + kTile - 1) / kTile;
     tiles = std::max(tiles, (int)std::min<int64_t>(n, INT32_MAX / 2));
   }
-  const bool scratch = workspace && counters && !far;
-  const F32Plan plan = plan_f32(D, B * H, Sq, n_jobs, tiles, scratch ? workspace_bytes : 0, scratch ? n_counters : 0);
-  const int qw = far ? 2 : plan.qw;
+  const bool scratch = workspace && counters;
+  const F32Plan plan = plan_f32(D, B * H, Sq, n_jobs, tiles, far, scratch ? workspace_bytes : 0, scratch ? n_counters : 0);
+  const int qw = plan.qw;
   a.parts = plan.parts;
   a.n_qg = (Sq + kTile * qw - 1) / (kTile * qw);
   a.total = B * H * a.n_qg;
@@ -969,9 +1070,15 @@ extern "C" int dt_attn_jobs_f32_ws_fwd(const float* q, int32_t B, int32_t Sq, in
   hipStream_t s = (hipStream_t)stream;
   std::unique_lock<std::mutex> lock;   // (another thread's parts, on the same stream and workspace, may wait for a fold kernel)
   if (a.parts > 1) lock = std::unique_lock<std::mutex>(workspace_lock(workspace));
-  if (far) return D == 128 ? launch_f32<128, 2, true>(a, n_jobs, s) : launch_f32<64, 2, true>(a, n_jobs, s);
-  if (D == 128) return qw == 2 ? launch_f32<128, 2, false>(a, n_jobs, s) : launch_f32<128, 4, false>(a, n_jobs, s);
-  return qw == 2 ? launch_f32<64, 2, false>(a, n_jobs, s) : launch_f32<64, 4, false>(a, n_jobs, s);
+  auto launch = [&](auto d, auto w, auto f) { return launch_f32<decltype(d)::value, decltype(w)::value, decltype(f)::value>(a, n_jobs, s); };
+  auto launch_d = [&](auto d) {
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    if (far) return qw == 1 ? launch(d, one, std::true_type()) : launch(d, two, std::true_type());
+    if (qw == 4) return launch(d, std::integral_constant<int, 4>(), std::false_type());
+    return qw == 1 ? launch(d, one, std::false_type()) : launch(d, two, std::false_type());
+  };
+  return D == 128 ? launch_d(std::integral_constant<int, 128>()) : launch_d(std::integral_constant<int, 64>());
 }
 
 extern "C" int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D, int64_t q_sb, int64_t q_ss,

@@ -109,7 +109,8 @@ int dt_attn_chunk_f32_fwd(const float* q, const float* k, const float* v, float*
  * Several fp32 states in one launch (core/attention.py:185-196): job j attends q to the concatenation of the
  * chunks job_chunks[job_begin[j] .. job_begin[j+1]) and writes (out_ptrs[j], lse_ptrs[j]), fp32 throughout as
  * above.  At most DT_MAX_CHUNKS chunks, DT_MAX_JOBS jobs and DT_MAX_JOB_ENTRIES chunk references; the tables
- * are HOST arrays, with strides of their own for every chunk.
+ * are HOST arrays, with strides of their own for every chunk.  Small calls are faster with scratch (below): 4 heads x 512 queries x 2048
+ * keys, D = 64, 37 us here and 19 there.
  */
 int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
                          int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
@@ -124,8 +125,8 @@ int dt_attn_jobs_f32_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32
  * utils.py:49, so that a job over all chunks of a call is the call's result, core/attention.py:185-196) and with scratch: where
  * the queries alone leave the GPU idle, the key tiles of a job are shared by several workgroups, which put partial sums into the
  * workspace; the last one folds them.  workspace: device memory, 16-byte aligned, used up to workspace_bytes.  counters: n_counters words of
- * device memory that are zero; every launch leaves them at zero.  Launches that share either must not overlap on the GPU.
- * Without them, or where they are too few, as dt_attn_jobs_f32_fwd.
+ * device memory that are zero; every launch leaves them at zero (one per job and 32 queries of a batch and head is enough).  Launches that
+ * share either must not overlap on the GPU.  Without them, or where they are too few, as dt_attn_jobs_f32_fwd.
  */
 int dt_attn_jobs_f32_ws_fwd(const float* q, int32_t B, int32_t Sq, int32_t H, int32_t D,
                             int64_t q_stride_b, int64_t q_stride_s, int64_t q_stride_h,
