@@ -335,6 +335,8 @@ class ChunkTable:
     ``convert`` is called on chunks that are neither bf16 nor fp16."""
 
     def __init__(self, k_chunks: Sequence[torch.Tensor], v_chunks: Sequence[torch.Tensor], batch: int = 0, convert=None):
+        # (the binding takes sequences; a tensor of chunks or an iterator becomes one)
+        k_chunks, v_chunks = (c if type(c) is list or type(c) is tuple else list(c) for c in (k_chunks, v_chunks))
         self.native = _host().ChunkTable(k_chunks, v_chunks, batch, convert)
 
     n = property(lambda self: self.native.n)
