@@ -246,7 +246,8 @@ class proAttention:
 
     # ---- stride mode ------------------------------------------------------------------------------
     def _strides(self, timestep: int) -> Tuple[int, int]:
-        return get_redundancy_map().get_isp_strides(timestep, self.layer_id)
+        rm = get_redundancy_map()
+        return rm.get_curr_isp_stride(timestep, self.layer_id), rm.get_next_isp_stride(timestep, self.layer_id)
 
     @get_timer("oAttn")
     def attn(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> Optional[torch.Tensor]:

@@ -71,25 +71,25 @@ class RedundancyMap:
         assert self.base_weight % divider == 0, f"Invalid divider {divider} for base weight {self.base_weight}"
         return max(self.base_weight // divider, 1)
 
+    def _divider(self, row: int, col: int) -> int:
+        host = _hip._host_module   # (there from the first launch on; the map itself needs none)
+        if host is not None and type(self.divider_map) is torch.Tensor and type(row) is int and type(col) is int:
+            value = host.element(self.divider_map, row, col)
+            if value is not None:
+                return value
+        return int(self.divider_map[row, col].item())
+
     def get_curr_isp_stride(self, timestep: int, layer_id: int) -> int:
         """:49-67"""
         if self.auto_setting:
             return self.base_weight
-        return self._stride_of(int(self.divider_map[timestep, layer_id].item()))
+        return self._stride_of(self._divider(timestep, layer_id))
 
     def get_next_isp_stride(self, timestep: int, layer_id: int) -> int:
         """:69-87 -- the last step announces a full refresh."""
         if self.auto_setting or timestep == self.num_timesteps - 1:
             return self.base_weight
-        return self._stride_of(int(self.divider_map[timestep + 1, layer_id].item()))
-
-    def get_isp_strides(self, timestep: int, layer_id: int):
-        """(``get_curr_isp_stride``, ``get_next_isp_stride``), the map read once."""
-        if not self.auto_setting and timestep != self.num_timesteps - 1:
-            both = _hip._host().two_rows(self.divider_map, timestep, layer_id)
-            if both is not None:
-                return self._stride_of(both[0]), self._stride_of(both[1])
-        return self.get_curr_isp_stride(timestep, layer_id), self.get_next_isp_stride(timestep, layer_id)
+        return self._stride_of(self._divider(timestep + 1, layer_id))
 
     def set_pattern_for_row(self, row_idx: int, split_list: Sequence[int], pattern_list: Sequence[int]) -> None:
         """:90-119 -- piecewise-constant dividers over the layers of one step."""

@@ -821,12 +821,12 @@ std::vector<Tensor> qkv_project(const Tensor& text_rows, const Tensor& video, in
 
 // ---- host state of a call -------------------------------------------------------------------------------------
 
-// Elements [row, col] and [row + 1, col] of a 2-D int64 CPU tensor, or nothing where it is another one or a row or column is not there.
-std::optional<std::pair<int64_t, int64_t>> two_rows(const Tensor& t, int64_t row, int64_t col) {
-  if (t.is_cuda() || t.scalar_type() != at::kLong || t.dim() != 2 || row < 0 || row + 1 >= t.size(0) || col < 0 || col >= t.size(1))
+// Element [row, col] of a 2-D int64 tensor in host memory, or nothing where it is another one or the place is not there.
+std::optional<int64_t> element(const Tensor& t, int64_t row, int64_t col) {
+  if (!t.device().is_cpu() || t.layout() != at::kStrided || t.scalar_type() != at::kLong || t.is_neg() || t.dim() != 2 || row < 0 || row >= t.size(0) ||
+      col < 0 || col >= t.size(1))
     return std::nullopt;
-  const int64_t* at = t.const_data_ptr<int64_t>() + row * t.stride(0) + col * t.stride(1);
-  return std::make_pair(at[0], at[t.stride(0)]);
+  return t.const_data_ptr<int64_t>()[row * t.stride(0) + col * t.stride(1)];
 }
 // Bytes that PyTorch's allocator has handed out on a device.
 int64_t allocated_bytes(int64_t device) {
@@ -887,6 +887,6 @@ PYBIND11_MODULE(_ditango_host, m) {
   m.def("zero_rows_from", &zero_rows_from);
   m.def("qk_norm_rope", &qk_norm_rope);
   m.def("qkv_project", &qkv_project);
-  m.def("two_rows", &two_rows);
+  m.def("element", &element);
   m.def("allocated_bytes", &allocated_bytes);
 }
