@@ -540,7 +540,10 @@ def qk_norm_rope(x: torch.Tensor, *, norm: int = DT_NORM_NONE, weight: Optional[
     ``[rope_end-rope_begin, D]`` or ``[B, rope_end-rope_begin, D]``.  ``out_scale`` multiplies the result
     before its rounding to the output dtype; the ``DT_ROUND_*`` bits round to x's dtype.  weight / bias are fp32, or
     with ``DT_WEIGHTS_16`` in ``rounding`` of x's dtype."""
-    return _host().qk_norm_rope(x, norm, weight, bias, eps, rope, cos, sin, rope_begin, rope_end, sections, rounding, out, out_scale,
+    _require(x.is_cuda, "x must be bf16 or fp16 [B,S,H,D] on the GPU")   # (before a stream is asked for)
+    # (the binding takes no float for a whole number and no array for a list)
+    return _host().qk_norm_rope(x, int(norm), weight, bias, float(eps), int(rope), cos, sin, int(rope_begin),
+                                None if rope_end is None else int(rope_end), [int(v) for v in sections], int(rounding), out, float(out_scale),
                                 _stream())
 
 

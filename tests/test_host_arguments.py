@@ -70,3 +70,8 @@ def test_strides_are_asked_of_the_map(strides):
         get_next_isp_stride = staticmethod(lambda timestep, layer_id: 5)
 
     assert strides(0, 0, kind=Bare()) == (3, 5)
+
+
+def test_producer_refuses_host_tensors_itself():
+    with pytest.raises(_hip.DitangoHipError, match="x must be"):
+        _hip.qk_norm_rope(torch.zeros(1, 4, 2, 64, dtype=torch.bfloat16))

@@ -8,6 +8,7 @@ differ by one bf16 ulp where a reduction-order difference flips a rounding.
 """
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -239,6 +240,19 @@ def test_norm_parameters_in_the_dtype_of_x_are_read_in_place(hip, D, H, dtype, n
     assert torch.equal(prepare_qk(x, weight=w.float(), bias=b, **kw), want)
     with pytest.raises(hip.DitangoHipError):
         hip.qk_norm_rope(x, norm=P.NORM_RMS, weight=w)   # without the flag the binding takes fp32 only
+
+
+def test_numbers_of_any_kind(hip):
+    """Sections as an array or a tensor, codes and rows as NumPy's numbers or whole floats."""
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(1, 10, 2, 64, generator=g).to(DEV, torch.bfloat16)
+    cos, sin = (t.to(DEV) for t in _tables(P.ROPE_HALVES, 7, 64, (32, 16, 16)))
+    run = lambda norm, rope, begin, end, sections: hip.qk_norm_rope(x, norm=norm, rope=rope, cos=cos, sin=sin, rope_begin=begin, rope_end=end,
+                                                                   sections=sections)
+    want = run(hip.DT_NORM_RMS, hip.DT_ROPE_HALVES, 2, 9, (32, 16, 16))
+    for kind in (np.int64, float, torch.tensor):
+        for sections in (np.array([32, 16, 16]), torch.tensor([32, 16, 16]), (32.0, 16.0, 16.0)):
+            assert torch.equal(run(*(kind(v) for v in (hip.DT_NORM_RMS, hip.DT_ROPE_HALVES, 2, 9)), sections), want)
 
 
 @pytest.mark.parametrize("D", [64, 128])
