@@ -10,6 +10,7 @@ from __future__ import annotations
 from ...core.attention import proAttention
 from ...core.parallel_state import get_isp_group
 
+_VARLEN_ATTN = proAttention.varlen_attn
 MEMORY_LAYOUT = {
     "flash": (lambda x: x.view(x.shape[0] * x.shape[1], *x.shape[2:]), lambda x: x),
     "torch": (lambda x: x.transpose(1, 2), lambda x: x.transpose(1, 2)),
@@ -23,9 +24,13 @@ class Hunyuan_DiTangoProcessor:
         self.oAttn = proAttention(layer_id, get_isp_group())
         self.varlen_Attn = self.oAttn.varlen_attn
 
+    def _calls_varlen_attn(self) -> bool:
+        """Whether ``varlen_Attn`` is ``proAttention.varlen_attn`` of this object and nothing that a caller has put in its place."""
+        return getattr(self.varlen_Attn, "__func__", None) is _VARLEN_ATTN and self.varlen_Attn.__self__ is self.oAttn
+
     def ringfusion_attn(self, q, k, v, drop_rate=0, attn_mask=None, causal=False, cu_seqlens_q=None, cu_seqlens_kv=None,
                         max_seqlen_q=None, max_seqlen_kv=None, batch_size=1):
-        if cu_seqlens_q is not None and q.shape[0] == k.shape[0] == v.shape[0] == 1:
+        if cu_seqlens_q is not None and q.shape[0] == k.shape[0] == v.shape[0] == 1 and self._calls_varlen_attn():
             x = self.oAttn.varlen_sample(q, k, v, cu_seqlens_q, cu_seqlens_kv, max_seqlen_q)
             return x.view(batch_size, max_seqlen_q, x.shape[2] * x.shape[3])
         pre_attn_layout, post_attn_layout = MEMORY_LAYOUT["flash"]

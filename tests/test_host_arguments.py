@@ -6,6 +6,7 @@ import torch
 from ditango_amd import _hip
 from ditango_amd.core import config, parallel_state, redundancy_map
 from ditango_amd.core.attention import proAttention
+from ditango_amd.executor.hunyuanvideo import attention_hunyuan
 
 
 @pytest.mark.parametrize("kind", ["list", "tuple", "iterator", "generator", "stacked", "values"])
@@ -75,3 +76,41 @@ def test_strides_are_asked_of_the_map(strides):
 def test_producer_refuses_host_tensors_itself():
     with pytest.raises(_hip.DitangoHipError, match="x must be"):
         _hip.qk_norm_rope(torch.zeros(1, 4, 2, 64, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("place", ["processor", "attention", "class", "own class"])
+def test_hunyuan_processor_calls_a_replaced_varlen_attn(monkeypatch, place):
+    """One packed sample takes a way without views, unless somebody listens at ``varlen_attn``."""
+    parallel_state.init_local_groups(1, 0)
+    seen = []
+
+    def listen(*args, **kwargs):
+        seen.append(tuple(args[-7].shape))
+        return args[-7]
+
+    monkeypatch.setattr(proAttention, "varlen_sample", lambda self, q, *args: seen.append("sample") or q)
+    if place == "class":
+        monkeypatch.setattr(proAttention, "varlen_attn", listen)
+    processor = attention_hunyuan.Hunyuan_DiTangoProcessor(0)
+    if place == "processor":
+        processor.varlen_Attn = listen
+    elif place == "attention":
+        monkeypatch.setattr(processor.oAttn, "varlen_attn", listen)
+        processor.varlen_Attn = processor.oAttn.varlen_attn
+    elif place == "own class":
+        processor.oAttn.__class__ = type("Own", (proAttention,), {"varlen_attn": listen})
+        processor.varlen_Attn = processor.oAttn.varlen_attn
+    q = torch.zeros(1, 6, 2, 64)
+    cu = torch.tensor([0, 4, 6], dtype=torch.int32)
+    out = processor.ringfusion_attn(q, q, q, cu_seqlens_q=cu, cu_seqlens_kv=cu, max_seqlen_q=6, max_seqlen_kv=6)
+    assert out.shape == (1, 6, 128) and seen == [(6, 2, 64)]
+
+
+def test_hunyuan_processor_of_one_sample_makes_no_views(monkeypatch):
+    parallel_state.init_local_groups(1, 0)
+    seen = []
+    monkeypatch.setattr(proAttention, "varlen_sample", lambda self, q, *args: seen.append(tuple(q.shape)) or q)
+    q = torch.zeros(1, 6, 2, 64)
+    cu = torch.tensor([0, 4, 6], dtype=torch.int32)
+    attention_hunyuan.Hunyuan_DiTangoProcessor(0).ringfusion_attn(q, q, q, cu_seqlens_q=cu, cu_seqlens_kv=cu, max_seqlen_q=6, max_seqlen_kv=6)
+    assert seen == [(1, 6, 2, 64)]
