@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 from torch.nn import LayerNorm, Linear, Parameter
 from torch.nn.modules import module as _module
 
@@ -14,16 +15,19 @@ HEAD_DIM = 64
 MOST_FLOPS = 2.0e11
 
 
+_FORWARD = {Linear: Linear.forward, LayerNorm: LayerNorm.forward}   # (a tool may patch the class)
+
+
 def _only_arithmetic() -> bool:
-    """No mode, transform or autocast that would see the modules' operations."""
+    """No mode, transform, autocast or forward-mode derivative that would see the modules' operations."""
     return not (torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack() or torch.is_autocast_enabled("cuda")
                 or torch._C._functorch.peek_interpreter_stack() is not None or torch.compiler.is_compiling()
-                or torch.jit.is_tracing() or _module._has_any_global_hook())
+                or torch.jit.is_tracing() or _module._has_any_global_hook() or forward_ad._current_level >= 0)
 
 
 def _plain(m, kind) -> bool:
     """A module of exactly this class, whose call is its forward."""
-    return (type(m) is kind and "forward" not in m.__dict__
+    return (type(m) is kind and "forward" not in m.__dict__ and kind.forward is _FORWARD[kind]
             and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
 
 

@@ -6,6 +6,7 @@ import torch
 from ditango_amd import _hip
 from ditango_amd.core import config, parallel_state, redundancy_map
 from ditango_amd.core.attention import proAttention
+from ditango_amd.executor.cogvideox import projection
 from ditango_amd.executor.hunyuanvideo import attention_hunyuan
 
 
@@ -114,3 +115,13 @@ def test_hunyuan_processor_of_one_sample_makes_no_views(monkeypatch):
     cu = torch.tensor([0, 4, 6], dtype=torch.int32)
     attention_hunyuan.Hunyuan_DiTangoProcessor(0).ringfusion_attn(q, q, q, cu_seqlens_q=cu, cu_seqlens_kv=cu, max_seqlen_q=6, max_seqlen_kv=6)
     assert seen == [(1, 6, 2, 64)]
+
+
+def test_fused_projections_step_aside_for_whoever_sees_the_modules(monkeypatch):
+    """Forward-mode derivatives (v carries its tangent to the caller of project_qkv) and a patched nn.Linear."""
+    linear = torch.nn.Linear(64, 64)
+    assert projection._only_arithmetic() and projection._plain(linear, torch.nn.Linear)
+    with torch.autograd.forward_ad.dual_level():
+        assert not projection._only_arithmetic()
+    monkeypatch.setattr(torch.nn.Linear, "forward", lambda self, x: x)
+    assert not projection._plain(linear, torch.nn.Linear)
