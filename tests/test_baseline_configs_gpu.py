@@ -458,8 +458,9 @@ def test_every_row_at_full_size_against_the_fp32_kernel(hip, name, dtype):
     """The oracle runs on the host, so at full size it covers a sample of the query rows.  The rows in between are
     covered here: one chunk state of every configuration's real shape, ALL rows, heads and keys, computed by the
     bf16 MFMA kernel (plain launch and tail-balanced launch) against the fp32 kernel
-    ``dt_attn_chunk_f32_fwd`` on the same (bf16-valued) numbers -- an independent implementation (fp32 matrix
-    instructions, operands straight from memory, nothing rounded to 16 bits) that the small-shape tests pin against the oracle.  Bar as everywhere:
+    ``dt_attn_chunk_f32_fwd`` on the same (bf16-valued) numbers -- a kernel of its own with fp32 accuracy, of whose operands' three
+    bf16 parts only the first is not zero here, that the small-shape tests pin against the oracle; it runs the same matrix
+    instructions and transposing LDS reads, so what those get wrong does not show between the two.  Bar as everywhere:
     out <= 2e-2, lse <= 1e-3; observed two orders below.  The two head dimensions also run on fp16 tensors (the
     fp16 MFMA variant; out held to 4e-3)."""
     if name == "sweep_chunk":

@@ -41,7 +41,7 @@ def test_attention_kernel_keeps_its_arguments_out_of_scratch(resources):
 
 def test_streaming_kernels_use_no_scratch(resources):
     for fragment in ("merge_states_kernel", "merge_update_kernel", "state_convert_kernel", "flat_copy_kernel", "state_copy_kernel", "state_copy_units_kernel",
-                     "rel_l1_sums_kernel", "qk_norm_rope_kernel", "attn_tail_fold_kernel", "attn_f32_kernel", "build_schedule_kernel",
+                     "rel_l1_sums_kernel", "qk_norm_rope_kernel", "attn_tail_fold_kernel", "attn_f32_kernel", "qkv_kernel", "build_schedule_kernel",
                      "zero_rows_from_kernel"):
         for name, r in _kernels(resources, fragment).items():
             assert r["ScratchSize [bytes/lane]"] == 0 and r["VGPRs Spill"] == 0, (name, r)

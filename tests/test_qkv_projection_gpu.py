@@ -73,6 +73,13 @@ def _check(got, want, dtype):
     (1, 113, 2500, 24, 1536, torch.bfloat16),  # 192 x 256
     (1, 28, 2212, 48, 3072, torch.float16),    # 160 x 512, 14 full tiles of rows
     (1, 28, 3301, 48, 3072, torch.bfloat16),   # 256 x 256, one row more than 13 tiles
+    # columns of 22.5 tiles of 256 or 11.25 of 512, in each of the large tiles; rows of two samples in one tile
+    (1, 30, 1970, 30, 1920, torch.bfloat16),
+    (1, 30, 2970, 30, 1920, torch.float16),
+    (1, 30, 4970, 30, 1920, torch.bfloat16),
+    (2, 30, 1470, 30, 1920, torch.bfloat16),
+    (2, 30, 1970, 30, 1920, torch.float16),
+    (2, 30, 3970, 30, 1920, torch.bfloat16),
 ])
 @pytest.mark.parametrize("bias,rotated", [(True, True), (False, False)])
 def test_projections_match_fp64(hip, B, T, V, H, K, dtype, bias, rotated):
@@ -141,7 +148,7 @@ def test_rotation_of_one_projection_alone(hip, T, V, H, K, which):
             assert torch.equal(want, b), i
 
 
-@pytest.mark.parametrize("H,K,V", [(2, 128, 150), (24, 1536, 2500), (48, 3072, 2194)])
+@pytest.mark.parametrize("H,K,V", [(2, 128, 150), (24, 1536, 2500), (48, 3072, 2194), (48, 3072, 3272)])
 def test_a_row_depends_on_its_own_tokens_only(hip, H, K, V):
     """Every tile form: rows one by one, in another tile and beside other rows, come out bit for bit the same (one order of the sums)."""
     from ditango_amd.executor.cogvideox.projection import project_qkv
