@@ -16,10 +16,11 @@
 // What does not show: a weight below 2^-110 loses up to 2^-126, which counts where its V is more than 2^100 times the result, and an element
 // of K below 2^-110 as much, which with |Q| <= 2^90 is 2^-36 of a score.
 //
-// What bounds it: a wavefront issues in order, and an MFMA holds it up (24 MFMAs with 88 vector instructions between them take as long as
-// one behind the other), so a tile takes 48 MFMAs x 32 cycles + 330 vector instructions x 4 at d = 64 (twice the MFMAs at 128), less what
-// the other wavefront of the SIMD hides of it: counters of 8 heads x 1195 queries x 9560 keys, MFMA pipe busy 41 % of the SIMDs' cycles, vector
-// ALU 37 %.  So the split of K and V, half of the vector instructions where every wavefront does its own, is shared:
+// What bounds it: a wavefront issues in order, and an MFMA holds it up (24 MFMAs with 88 vector instructions between them take about as
+// long as one behind the other), so a tile takes 48 MFMAs x 32 cycles + 330 vector instructions x 4 at d = 64 (twice the MFMAs at 128), less what
+// the other wavefront of the SIMD hides of it: counters of 8 heads x 1195 queries x 9560 keys, MFMA pipe busy 46 % of the SIMDs' cycles, vector
+// ALU 49 %, both at once in a third of the former.  So the split of K and V, half of the vector instructions where every wavefront does its
+// own (7 of them per MFMA against 15), is shared:
 //   * QW (2 or 4) wavefronts of a workgroup own 32 queries each and walk the same key tiles of 32.  Each loads its share of a tile in whole
 //     lines, a turn ahead, splits it and puts the three parts into the LDS, from where all read operands (16-byte reads of K,
 //     transposing reads of V, as in attn_fwd.hip).  The KW = 4 / QW groups of a workgroup take every KW-th tile.
@@ -29,8 +30,8 @@
 //   * In a small launch nothing is shared (QW = 1): a wavefront splits all of its tiles from memory to registers, and nobody waits for anybody.
 //   * Where the queries alone leave the chip idle, `parts` workgroups share the keys of a work item (plan_f32).
 //   * Measured (us per call with the GPU kept busy, kernel of fp32 products and merge kernel behind it -> this, which needs no other):
-//     4 heads x 512 queries x 2048 keys, d = 64 30 -> 21; 12 x 1053 x 4212 163 -> 101; 8 x 1195 x 9560 258 -> 154 (157 TFLOP/s, as much as
-//     the fp32 pipe has); d = 128 12 x 355 x 2840 107 -> 71, 10 x 847 x 1694 120 -> 73.
+//     4 heads x 512 queries x 2048 keys, d = 64 30 -> 19; 12 x 1053 x 4212 163 -> 101; 8 x 1195 x 9560 258 -> 153 (157 TFLOP/s, as much as
+//     the fp32 pipe has); d = 128 12 x 355 x 2840 107 -> 72, 10 x 847 x 1694 120 -> 72.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -203,7 +204,8 @@ constexpr uint32_t kOddFrom = 0xff000000u - 2 * kTiny;
 __device__ __forceinline__ uint32_t oddity(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 2 * kTiny; }
 
 // m scale + log(den), rounded about once: the logarithm of den's exponent and of its significand, and the two large terms' sum
-// with its error.  (Plainly, the rounding of a logarithm of 2 to 5 comes on top: 2-norm error of the lse against fp64, 4 heads x 512
+// with its error.  ln 2 in two parts after Cody and Waite: 355 / 512, its nearest with ten bits, and what is left of it; the significand between
+// the square roots of 1/2 and 2, where its logarithm is smallest.  (Plainly, the rounding of a logarithm of 2 to 5 comes on top: 2-norm error of the lse against fp64, 4 heads x 512
 // queries x 2048 keys, 5.2e-8 -> 3.44e-8; the rounding of the exact value to fp32 alone is 3.38e-8.)
 __device__ __forceinline__ float lse_of(float m, float den, float scale) {
   if (!(den > 0.f)) return -INFINITY;
@@ -213,7 +215,7 @@ __device__ __forceinline__ float lse_of(float m, float den, float scale) {
     f *= 2.f;
     k -= 1.f;
   }
-  constexpr float kLn2Hi = 0.693359375f, kLn2Lo = -2.12194440e-4f;   // (10 bits: k kLn2Hi is exact)
+  constexpr float kLn2Hi = 355.f / 512.f, kLn2Lo = (float)(0.693147180559945309 - 355.0 / 512.0);   // (10 bits: k kLn2Hi is exact)
   const float a = m * scale, b = k * kLn2Hi, sum = a + b;
   if (!(__builtin_fabsf(sum) < INFINITY)) return sum;
   const float back = sum - a;
@@ -435,7 +437,8 @@ __global__ __launch_bounds__(kThreadsF32, D == 64 ? 2 : 1) void attn_f32_kernel(
     return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
-  // The instructions that split the next operand go between the MFMAs, which are then the longer of the two.
+  // The instructions that split the next operand go between the MFMAs, for the other wavefront's to fall into (left to the compiler 0.3 to
+  // 1.4 % longer: 12 heads x 1053 queries x 4212 keys 109.4 -> 111.4 us, 24 x 2048 x 4096 288 -> 291, d = 128 614 -> 616).
   auto interleave = [](auto reads, auto products) __attribute__((always_inline)) {
     constexpr int kValu = (44 * kLoads / 2 + decltype(products)::value - 1) / decltype(products)::value;
     __builtin_amdgcn_sched_group_barrier(0x100, decltype(reads)::value, 0);
@@ -1022,7 +1025,8 @@ extern "C" int dt_attn_jobs_f32_ws_fwd(const float* q, int32_t B, int32_t Sq, in
       return DT_ERR_INVALID;
     }
     a.chunk[i] = {k_ptrs[i], v_ptrs[i], kv_sb[i], kv_ss[i], kv_sh[i], kv_lens[i]};
-    // (a chunk's keys of one batch and head beyond 2 GiB, or in falling order: 64-bit offsets, slower)
+    // (a chunk's keys of one batch and head beyond 2 GiB, or in falling order: 64-bit offsets.  us, 32 -> 64 bits: 4 heads x 512 queries x 2048
+    // keys, d = 64 20 -> 23; 24 x 2048 x 4096 286 -> 338, d = 128 613 -> 755)
     far = far || kv_ss[i] < 0 || (kv_lens[i] > 0 && (uint64_t)kv_ss[i] > (1ull << 29) / ((uint64_t)kv_lens[i] + kTile));
   }
   if (job_begin[0] != 0) {

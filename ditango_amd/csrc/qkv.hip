@@ -3,10 +3,10 @@
 // Replaces the concatenation, the three library products and the two producer launches of
 // executor/cogvideox/attention_processor.py:39-71.
 //
-// What bounds it: the matrix pipe, with LDS reads behind it (70 to 85 % as many cycles as the MFMAs); of 141 us for 48 heads x 2222
-// tokens x 3072 channels (126 GFLOP) 28 are the loads of the tiles, 18 of those their issue (timed with loads left out, and with
-// loads of one place), 18 start and end.  In a loop of calls, modules and producer -> this: the same 153 -> 130 us (970 TFLOP/s), 16 heads x 602
-// x 1024 42 -> 18.  From 200 GFLOP on the library's products take less (48 x 8016 429 -> 458), and the adapter calls the modules.
+// What bounds it: the matrix pipe, busy 54 % of the time for 48 heads x 2222 tokens x 3072 channels (126 GFLOP), with LDS reads behind it (70 to
+// 85 % as many cycles as the MFMAs); of 141 us, with the tables of cos and sin not yet in the LDS, 28 were the loads of the tiles, 18 of those
+// their issue (timed with loads left out, and with loads of one place), 18 start and end.  In a loop of calls, modules and producer -> this:
+// the same 153 -> 127 us (990 TFLOP/s), 16 heads x 602 x 1024 42 -> 16.  From 200 GFLOP on the library's products take less (48 x 8016 429 -> 458), and the adapter calls the modules.
 // out^T = W X^T with v_mfma_f32_32x32x16, accumulated in fp32.  A wavefront owns one head (64 output columns) of 32 MB tokens; with
 // the product transposed a lane holds 32 of the 64 columns of ONE token, four neighbouring ones at a time.
 //   * A workgroup of 8 wavefronts takes BM = 32 MB WM tokens x BN = 64 (8 / WM) columns of the three outputs side by side.
@@ -344,7 +344,7 @@ int launch(QkvArgs& a, bool half, hipStream_t stream) {
 // (8 ... 48 steps) x 280 ... 12 000 tokens (errors 4 to 5 %; the choice takes 0.9 % more than the best on average).  us, modules and producer ->
 // 64 x 256 / 192 x 256 / 256 x 256 / 160 x 512: 16 heads x 602 tokens 42 -> 18 / 34 / 39 / 49; 24 x 4330 108 -> 94 / 87 / 105 / 78; 48 x 2222
 // 153 -> 167 / 141 / 171 / 130 (252 workgroups of 160 x 512, one round); 48 x 3328 198 -> 248 / 214 / 186 / 235 (468 of 256 x 256, two).
-enum Tiles { kFew, kSome, kMost, kMany };
+enum Tiles { kFew, kSome, kMore, kMany };
 Tiles plan(int M, int N, int K) {
   constexpr int kCus = 32;   // of an XCD
   const double steps = K / 64.0;
@@ -419,7 +419,7 @@ extern "C" int dt_qkv_project(const void* text, int64_t text_stride_b, int64_t t
   switch (plan(a.M, a.N, K)) {
     case kFew: return launch<1, 2, 4, 2>(a, half, s);
     case kSome: return launch<3, 2, 4, 2>(a, half, s);
-    case kMost: return launch<4, 2, 4, 2>(a, half, s);
+    case kMore: return launch<4, 2, 4, 2>(a, half, s);
     default: return launch<5, 1, 2, 3>(a, half, s);
   }
 }
