@@ -276,6 +276,13 @@ __device__ __forceinline__ void load_next_block_to_lds(u32x4 rsrc, uint32_t lane
                : "v"(lane_off), "s"(r), "s"(__builtin_amdgcn_readfirstlane(uniform_off))
                : "memory");
 }
+// The same from an address of each lane's own.
+__device__ __forceinline__ void load_rows_to_lds(const uint16_t* from, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :
+               : "v"(from), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
+               : "memory", "m0");
+}
 
 // Segment boundaries are read through the constant address space, i.e. with scalar loads: the lists were
 // written before the launch and the address is uniform.  (As a vector load the compiler follows it with
@@ -664,14 +671,29 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   const int q0 = q_begin + row0 + (kSplitKeys ? wave & 3 : wave) * 32;
   const int key0 = kSplitKeys ? 32 * group : 0;  // first key of a tile that this wavefront works on
 
-  // ---- Q fragments: B operand of S^T = K Q^T, kept in registers ----------------------
+  typedef __attribute__((address_space(3))) uint8_t* lds_ptr_t;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
+
+  // ---- Q: B operand of S^T = K Q^T, kept in registers --------------------------------
+  // The wavefront's 32 rows come as whole lines, through the LDS: half of them through its staging rows, a quarter each through
+  // its own shares of V buffers 3 and 2, which nothing but its own later tile loads writes.  Read from memory as fragments, a load
+  // instruction touched 32 lines for 32 bytes each, in front of all tile loads: from the start of a work item to its first scores 5.4 ->
+  // 4.2 us (stamps of 24 heads x 119 056 queries, D = 128), of 98.  us per call, together with the addresses in the epilogue (2.1 -> 1.4 us
+  // an item): 16 heads x 300 queries, 2 of 4 chunks, D = 128 19.7 -> 18.0, 24 x 1000, 4 of 8 67.5 -> 65.1, 2 x 24 x 1861, 3 of 8 283.3 ->
+  // 278.7; D = 64 4 x 512, 2 of 4 15.4 -> 14.7, 48 x 2222, 5 of 8 340 -> 336; launches at the power cap (24 x 14 882) stay as they are.
   ex8 qf[D / 16];
+  constexpr int kQuarter = T::kLoads;   // 1 KB blocks of 8 rows
+  const uint32_t q_quarter[4] = {(uint32_t)(T::kLdsTiles + wave * T::kStageBytes), (uint32_t)(T::kLdsTiles + wave * T::kStageBytes + kQuarter * 1024),
+                                 (uint32_t)(T::kOffV + 3 * T::kBytesV + wave * kQuarter * 1024),
+                                 (uint32_t)(T::kOffV + 2 * T::kBytesV + wave * kQuarter * 1024)};
   {
-    int qrow = q0 + col;
-    if (qrow > q_end - 1) qrow = q_end - 1;
-    const uint16_t* qp = a.q + (int64_t)b * a.q_sb + (int64_t)qrow * a.q_ss + (int64_t)h * a.q_sh + 8 * hh;
+    const uint16_t* qp = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh;
 #pragma unroll
-    for (int s = 0; s < D / 16; ++s) qf[s] = *reinterpret_cast<const ex8*>(qp + 16 * s);
+    for (int i = 0; i < 4 * kQuarter; ++i) {
+      const int row = i * T::kRowsPerBlock + lane / T::kChunks;
+      const uint32_t chunk = (uint32_t)(lane % T::kChunks) ^ T::swz_k(row);
+      load_rows_to_lds(qp + (int64_t)min(q0 + row, q_end - 1) * a.q_ss + 8 * chunk, lds_base + q_quarter[i / kQuarter] + i % kQuarter * 1024);
+    }
   }
   // ---- tile bookkeeping -----------------------------------------------------------------
   // Two cursors walk the job's chunks tile by tile, all in scalar registers: the load cursor
@@ -778,8 +800,6 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
     v_goff[i] = (uint32_t)lrow * row_bytes + 16u * (uint32_t)((((pos >> 2) ^ T::swz_v(lrow)) << 2) | (pos & 3)) - 1024u * i;
   }
   static_assert(T::kLoads <= 2 && T::kRowsPerBlock * T::kRowBytes == 1024, "one immediate offset of 1 KB, whole rows per block");
-  typedef __attribute__((address_space(3))) uint8_t* lds_ptr_t;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
   // Issues this wavefront's loads of V of the tile before the one under the load cursor and of
   // K of the tile under it (tile X, into K buffer X & 3; V is needed two phases later than K, so
   // its loads run one tile behind), and moves the cursor on.  Past the last tile the loads are still
@@ -788,8 +808,8 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   // V of the previous tile: its offset, and -- only in the call after the cursor changed chunks -- the
   // descriptor of the chunk it belongs to.
   uint32_t v_off = 0u;
-  u32x4 rv_old = make_rsrc(nullptr, 0u);   // the very first call has no previous tile: zeros into a buffer nobody reads
-  bool v_lags = true;
+  u32x4 rv_old;
+  bool v_lags = false, no_v = true;   // the very first call has no previous tile: its share of the V buffer holds rows of Q
   auto load_tile = [&](int kbuf) __attribute__((always_inline)) {
     const int vbuf = (kbuf + kNumBuf - 1) & (kNumBuf - 1);
     const uint32_t kdst = lds_base + kbuf * T::kBytesK + wave * (1024 * T::kLoads);
@@ -799,7 +819,9 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
       if constexpr (T::kLoads == 2) load_next_block_to_lds(rsrc, goff[1], off);
     };
     // V first: the barrier waits let the K half of a call stay in flight one vector phase longer
-    if (__builtin_expect(v_lags, 0)) {
+    if (no_v) {
+      no_v = false;
+    } else if (__builtin_expect(v_lags, 0)) {
       load_blocks(rv_old, v_goff, v_off, vdst);
       v_lags = false;
     } else {
@@ -964,30 +986,35 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   //   * At D = 64 the calls are made behind the MFMAs of the matrix phase instead (see
   //     kLoadAfterMatrix); the barrier of the next vector phase then lets only the K half of the
   //     newest call stay in flight.
-  // Here: the calls Y = 0..2 (group 1: ..3) -- the V half of the first has no tile, it stores
-  // zeros into a buffer nobody reads -- of which K of tile 0 (first scores) and V of tile 0 (first
-  // prefill) are awaited; the trailing group then waits one phase, which staggers the two groups.
+  // Here: the calls Y = 0..2 -- the V half of the first has no tile, the wavefront's share of that
+  // buffer holds rows of Q -- of which K of tile 0 (first scores) and V of tile 0 (first prefill) are
+  // awaited, and Q with them.  The trailing group makes the call Y = 3 once its rows of Q are out of
+  // the buffer that it fills, and waits one phase, which staggers the two groups.
   using U0 = std::integral_constant<int, 0>;
   using U1 = std::integral_constant<int, 1>;
   using U2 = std::integral_constant<int, 2>;
   using U3 = std::integral_constant<int, 3>;
 #pragma unroll
   for (int y = 0; y < DT_SCHED_PROLOGUE_CALLS_LEADING; ++y) load_tile(y);
-  if (group == 1) {
+  // in flight behind this wait: K of tile 1 and the two shares of the call behind it
+  static_assert(DT_SCHED_PROLOGUE_INFLIGHT_TRAILING - 2 * (DT_SCHED_PROLOGUE_CALLS_TRAILING - DT_SCHED_PROLOGUE_CALLS_LEADING) ==
+                    DT_SCHED_PROLOGUE_INFLIGHT_LEADING, "the trailing group's last call comes behind the wait: two shares fewer in flight");
+  wait_tile_loads<DT_SCHED_PROLOGUE_INFLIGHT_LEADING * T::kLoads>();
+  {
+    const uint32_t at = q_quarter[0] + col * T::kRowBytes;
+    const uint32_t row_at = col < 16 ? at : (col < 24 ? q_quarter[2] : q_quarter[3]) + (col & 7) * T::kRowBytes;
 #pragma unroll
-    for (int y = DT_SCHED_PROLOGUE_CALLS_LEADING; y < DT_SCHED_PROLOGUE_CALLS_TRAILING; ++y) load_tile(y);
+    for (int s = 0; s < D / 16; ++s) qf[s] = *reinterpret_cast<const ex8*>(lds + row_at + 16 * ((2 * s + hh) ^ T::swz_k(col)));
   }
-  // Route the fragments through an empty asm: they are then defined by it, not by loads.  The
-  // compiler otherwise keeps "Q may still be in flight" alive round the loop and waits for ALL
-  // outstanding vector-memory loads (including the K/V prefetch just issued) before the first
-  // MFMA that reads Q in every iteration.  (Here, behind the first tile loads: Q and the tiles arrive together.)
+  // Route the fragments through an empty asm: they are then defined by it, not by loads that the compiler could repeat.
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) asm volatile("" : "+v"(qf[s]));
-  // in flight behind this wait: K of tile 1 and the calls after it (kLoads + 2 kLoads (1 + g) loads)
-  if (group == 0) wait_tile_loads<DT_SCHED_PROLOGUE_INFLIGHT_LEADING * T::kLoads>();
-  else wait_tile_loads<DT_SCHED_PROLOGUE_INFLIGHT_TRAILING * T::kLoads>();
   phase_barrier();
-  if (group == 1) phase_barrier();
+  if (group == 1) {
+#pragma unroll
+    for (int y = DT_SCHED_PROLOGUE_CALLS_LEADING; y < DT_SCHED_PROLOGUE_CALLS_TRAILING; ++y) load_tile(y);   // (over rows of Q)
+    phase_barrier();
+  }
   // first matrix phase: scores of tile 0
   if (n_tiles > 0) {
     qk_only();
@@ -1095,11 +1122,13 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         alpha = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m_ref - m_new) * c) : 1.f;
       }
       m_ref = m_new;
-      l_run *= alpha;
+      if (t > 0) {   // (nothing to scale yet)
+        l_run *= alpha;
 #pragma unroll
-      for (int i = 0; i < D / 32; ++i)
+        for (int i = 0; i < D / 32; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o_acc[i][r] *= alpha;
+          for (int r = 0; r < 16; ++r) o_acc[i][r] *= alpha;
+      }
       // a row whose keys are all masked so far keeps m_ref = -inf: use 0 so that exp2(-inf - 0) = 0
       mc = kPre ? mx : (m_new > -INFINITY ? m_new * c : 0.f);
       if constexpr (kPre) any_off = any_off || __any(m_ref != 0.f);
@@ -1283,6 +1312,11 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   constexpr int kHalfChunks = D / 16;                 // 16-byte chunks in half a row
   constexpr int kRowsPerPass = 64 / kHalfChunks;
   const int rr = lane / kHalfChunks, cc = lane % kHalfChunks;
+  // (a lane's rows by steps from its first: with a product of 64 bits for each row the epilogue took 2.1 us, 1.4 without)
+  uint16_t* const out0 = view.out + (((int64_t)b * e.Sq + q0) * e.H + h) * D;
+  const uint32_t row_elems = (uint32_t)e.H * D;
+  uint16_t* const out_lane = out0 + (int64_t)rr * row_elems + cc * 8;
+  const int64_t out_step = (int64_t)kRowsPerPass * row_elems;
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -1304,16 +1338,12 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
 #pragma unroll
     for (int p = 0; p < 32 / kRowsPerPass; ++p) {
       const int row = p * kRowsPerPass + rr;
-      const int qg = q0 + row;
       const u32x4 val = *reinterpret_cast<const u32x4*>(stage + row * D + ((cc ^ T::swz_o(row)) << 4));
-      if (qg < q_end) {
-        if constexpr (kMerge) {
-          const Rsrc dst = buffer_of(view.out + (((int64_t)b * e.Sq + q0) * e.H + h) * D, 32u * D * 2u * (uint32_t)e.H);
-          __builtin_amdgcn_raw_buffer_store_b128(val, dst, (uint32_t)(row * e.H) * (D * 2u) + half * D + cc * 16, 0, kDeviceNt);
-        } else {
-          uint16_t* dst = view.out + (((int64_t)b * e.Sq + qg) * e.H + h) * D + half * (D / 2) + cc * 8;
-          __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst));
-        }
+      if (q0 + row < q_end) {
+        if constexpr (kMerge)
+          __builtin_amdgcn_raw_buffer_store_b128(val, buffer_of(out0, 64u * row_elems),
+                                                 (uint32_t)rr * row_elems * 2u + half * D + cc * 16 + (uint32_t)(2 * p * kRowsPerPass) * row_elems, 0, kDeviceNt);
+        else __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(out_lane + p * out_step + half * (D / 2)));
       }
     }
   }
