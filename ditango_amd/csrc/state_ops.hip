@@ -545,44 +545,6 @@ struct CopyArgs {
   int32_t src_dtype, src_bsh, dst_dtype, dst_bsh;   // DT_BF16 / DT_FP32 / DT_FP16
 };
 
-// An fp32 state rounded to a 16-bit one (a cache store) or a 16-bit one widened (a load): a lane moves 4 elements, as in
-// merge_update_kernel above, and the first lane of a row its lse.  A short launch is bound by its start and its last workgroups'
-// waits, of which this has two, one behind the other.  us per launch, the kernels below -> this, for stores at D = 64 2222 x 48
-// heads 10.3 -> 9.7, 6001 x 7 5.3 -> 4.9, 14 882 x 24 26.3 -> 25.5, 14 882 x 48 48.3 -> 47.6; for loads of less than 2^16 rows 2001
-// x 30 heads, D = 64 7.7 -> 6.1, D = 128 10.4 -> 10.1, 6001 x 7, D = 64 5.4 -> 4.7, 300 x 5, D = 128 2.7 -> 2.4.
-template <int D, int SRC, int DST>
-__global__ __launch_bounds__(kUpdateThreads) void state_convert_kernel(const CopyArgs a, const RowIndex at) {
-  static_assert((SRC == DT_FP32) != (DST == DT_FP32), "fp32 on one side");
-  const int64_t elem = lane_elem(), row64 = elem / D;
-  if (row64 >= at.rows) return;
-  const bool my_lse = a.dst_lse != nullptr && a.src_lse != nullptr && elem % D == 0;
-  uint32_t row = 0, bhs = 0;
-  float l = 0.f;
-  u32x4 w;
-  u32x2 n;
-  if (SRC == DT_FP32) w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(static_cast<const float*>(a.src_out) + elem));
-  else n = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(a.src_out) + elem));
-  if (my_lse) {
-    row = (uint32_t)row64;
-    bhs = !a.src_bsh || !a.dst_bsh ? bhs_of(at, row) : row;
-    l = a.src_lse[a.src_bsh ? row : bhs];
-  }
-  if (SRC == DT_FP32) {
-    n.x = pack16x2(__uint_as_float(w[0]), __uint_as_float(w[1]), DST == DT_FP16);
-    n.y = pack16x2(__uint_as_float(w[2]), __uint_as_float(w[3]), DST == DT_FP16);
-    __builtin_nontemporal_store(n, reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.dst_out) + elem));
-  } else {
-    float x[4];
-    widen16x2(n.x, SRC == DT_FP16, x[0], x[1]);
-    widen16x2(n.y, SRC == DT_FP16, x[2], x[3]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = __float_as_uint(x[i]);
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<float*>(a.dst_out) + elem));
-  }
-  if (my_lse) a.dst_lse[a.dst_bsh ? row : bhs] = l;
-}
-
-
 constexpr int kCopyRows = 1;  // rows per lane group (2 and 4 measured: -6 % and -12 %)
 
 // SRC / DST: the DT_* codes of the two sides, fixed at compile time (the launcher picks the instantiation).
@@ -688,53 +650,109 @@ __global__ __launch_bounds__(kThreads) void state_copy_units_kernel(const CopyAr
       a.dst_lse[lse_index(a.dst_bsh != 0, u[0].b[r], u[0].h[r], u[0].s[r], a.H, a.Sq)] = l;
 }
 
-// bf16 or fp16 state -> fp32 state (a cache load): `out` is an elementwise widening in the same element order,
-// so it runs as a flat pass -- a lane takes 4 consecutive elements (8 bytes in, 16 bytes out), one
-// load and one store, both non-temporal (+5 % over the row-mapped kernel above in this direction; in
-// the narrowing direction the row-mapped kernel is the faster one by 5-13 %, so it keeps that).  The
-// workgroups in front of those of `out` (dispatched first, so that they run beside the streaming ones
-// instead of as a tail) move the lse: one run of `lse_run` query positions x all heads per workgroup,
-// read in the source's order, written in the destination's, through the LDS in between, so that
-// both sides are coalesced whichever way the [H][S] / [S][H] layouts differ.
+// An fp32 state rounded to a 16-bit one (kNarrow: a cache store), or a 16-bit one widened (a load), kHalf: to or from fp16.
+// `out` is converted element by element in the same order, so it runs as a flat pass: a lane takes twice 4 elements, a
+// workgroup 8 KB of the fp32 side.  The workgroups in front of those of `out` (dispatched first, so that they run beside them
+// instead of as a tail) move the lse: tiles of a power of two of query positions x up to 256 heads, through the LDS as [s][h], so that
+// both sides are read and written in runs whichever way the [H][S] / [S][H] layouts differ, each lane's up to 4 loads side by side.
+//
+// What bounds it: memory, and in small launches the lse's two waits, one behind the other.  A store reads what has just been computed,
+// and what it writes is read next, so both go through the caches; what a load reads and writes does not.  us per store and load of
+// one state, 3 states taking turns [16 of them], rows mapped to lane groups, a row's lse moved by its first lane, nothing cached ->
+// this: 2222 x 48 heads, D = 64 19.0 -> 14.5 [19.1 -> 16.2], 9001 x 48 60.2 -> 51.8 [60.0 -> 52.0], 2000 x 12 6.5 -> 5.8 [7.0 -> 5.9]; D =
+// 128 900 x 24 9.4 -> 7.7 [9.9 -> 8.0], 3001 x 30 26.9 -> 22.4 [27.1 -> 24.2], 14 882 x 24 88.3 -> 81.6 [88.2 -> 81.5]; 300 x 8, D =
+// 64, two launches of little more than nothing, 4.5 -> 5.1.  Of the first the lse is 0.3 us (tiles with a division an element and one load
+// at a time 2.1); a store that caches neither side costs 1 us more with 3 states and 0.9 less with 16.
 constexpr int kConvThreads = 256;
+constexpr int kConvGroups = 2;      // groups of 4 elements of a lane
+constexpr int kLseHeads = 256;      // most heads of an lse tile
+struct ConvertPlan {
+  int64_t groups;                   // of 4 elements
+  uint32_t lse_wgs;
+  int32_t run_shift;                // log2 of an lse tile's query positions
+};
 
-__global__ __launch_bounds__(kConvThreads) void state_widen_kernel(const CopyArgs a, int64_t groups, uint32_t wgs_lse,
-                                                                   int lse_run) {
-  extern __shared__ float conv_lds[];   // [H][lse_run]
-  if (blockIdx.x >= wgs_lse) {
-    const int64_t g = (int64_t)(blockIdx.x - wgs_lse) * kConvThreads + threadIdx.x;   // 4 elements
-    if (g >= groups) return;
-    const u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(a.src_out) + g);
-    const bool f16 = a.src_dtype == DT_FP16;
-    float x[4];
-    widen16x2(v.x, f16, x[0], x[1]);
-    widen16x2(v.y, f16, x[2], x[3]);
-    u32x4 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = __float_as_uint(x[i]);
-    __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(a.dst_out) + g);
-    return;
-  }
-  const int runs = (a.Sq + lse_run - 1) / lse_run;
-  const int b = blockIdx.x / runs;
-  const int s0 = (blockIdx.x - b * runs) * lse_run;
-  const int ns = min(lse_run, a.Sq - s0);
-  const int n = ns * a.H;
-  // element i of the piece in a layout's own order -> (h, s)
-  auto decode = [&](bool bsh, int i, int& h, int& s) {
-    if (bsh) { s = i / a.H; h = i - s * a.H; }
-    else { h = i / ns; s = i - h * ns; }
+// One lse tile.
+__device__ __forceinline__ void move_lse_tile(const CopyArgs& a, int wg, int run_shift, float* tile) {
+  const int blocks = (a.H + kLseHeads - 1) / kLseHeads, runs = (a.Sq + (1 << run_shift) - 1) >> run_shift;
+  const int h0 = wg % blocks * kLseHeads, b = wg / blocks / runs, s0 = (wg / blocks - b * runs) << run_shift;
+  const int ns = min(1 << run_shift, a.Sq - s0), nh = min(kLseHeads, a.H - h0);
+  const int pitch = blocks == 1 ? a.H : kLseHeads;
+  constexpr int kBatch = 4;
+  // element i of this lane: its place in the tile and in a tensor of the given layout; place -1 where there is none
+  auto at = [&](bool bsh, int i, int& place, int64_t& index) __attribute__((always_inline)) {
+    const int t = threadIdx.x + kConvThreads * i;
+    int s, h;
+    bool there;
+    if (bsh) {           // (all heads: a contiguous piece of the tensor)
+      s = blocks == 1 ? 0 : t / kLseHeads;
+      h = blocks == 1 ? t : t % kLseHeads;
+      there = blocks == 1 ? t < ns * a.H : s < ns && h < nh;
+      index = ((int64_t)b * a.Sq + s0 + s) * a.H + h0 + h;
+    } else {
+      s = t & ((1 << run_shift) - 1);
+      h = t >> run_shift;
+      there = s < ns && h < nh;
+      index = ((int64_t)b * a.H + h0 + h) * a.Sq + s0 + s;
+    }
+    place = there ? s * pitch + h : -1;
   };
-  for (int i = threadIdx.x; i < n; i += kConvThreads) {
-    int h, s;
-    decode(a.src_bsh != 0, i, h, s);
-    conv_lds[h * ns + s] = a.src_lse[lse_index(a.src_bsh != 0, b, h, s0 + s, a.H, a.Sq)];
+  const int n = ((pitch << run_shift) + kConvThreads - 1) / kConvThreads;   // of a lane, in either order
+  for (int i0 = 0; i0 < n; i0 += kBatch) {
+    int place[kBatch];
+    float x[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      int64_t index;
+      at(a.src_bsh != 0, i0 + i, place[i], index);
+      if (place[i] >= 0) x[i] = a.src_lse[index];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (place[i] >= 0) tile[place[i]] = x[i];
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < n; i += kConvThreads) {
-    int h, s;
-    decode(a.dst_bsh != 0, i, h, s);
-    a.dst_lse[lse_index(a.dst_bsh != 0, b, h, s0 + s, a.H, a.Sq)] = conv_lds[h * ns + s];
+  for (int i = 0; i < n; ++i) {
+    int place;
+    int64_t index;
+    at(a.dst_bsh != 0, i, place, index);
+    if (place >= 0) a.dst_lse[index] = tile[place];
+  }
+}
+
+template <bool kNarrow, bool kHalf>
+__global__ __launch_bounds__(kConvThreads) void state_convert_kernel(const CopyArgs a, const ConvertPlan plan) {
+  extern __shared__ float conv_lds[];
+  if (blockIdx.x < plan.lse_wgs) {
+    move_lse_tile(a, blockIdx.x, plan.run_shift, conv_lds);
+    return;
+  }
+  const int64_t g0 = (int64_t)(blockIdx.x - plan.lse_wgs) * (kConvThreads * kConvGroups) + threadIdx.x;
+  u32x4 wide[kConvGroups];
+  u32x2 narrow[kConvGroups];
+#pragma unroll
+  for (int u = 0; u < kConvGroups; ++u) {
+    const int64_t g = g0 + u * kConvThreads;
+    if (g >= plan.groups) continue;
+    if constexpr (kNarrow) wide[u] = reinterpret_cast<const u32x4*>(a.src_out)[g];
+    else narrow[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(a.src_out) + g);
+  }
+#pragma unroll
+  for (int u = 0; u < kConvGroups; ++u) {
+    const int64_t g = g0 + u * kConvThreads;
+    if (g >= plan.groups) continue;
+    if constexpr (kNarrow) {
+      narrow[u].x = pack16x2(__uint_as_float(wide[u][0]), __uint_as_float(wide[u][1]), kHalf);
+      narrow[u].y = pack16x2(__uint_as_float(wide[u][2]), __uint_as_float(wide[u][3]), kHalf);
+      reinterpret_cast<u32x2*>(a.dst_out)[g] = narrow[u];
+    } else {
+      float x[4];
+      widen16x2(narrow[u].x, kHalf, x[0], x[1]);
+      widen16x2(narrow[u].y, kHalf, x[2], x[3]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wide[u][i] = __float_as_uint(x[i]);
+      __builtin_nontemporal_store(wide[u], reinterpret_cast<u32x4*>(a.dst_out) + g);
+    }
   }
 }
 
@@ -971,9 +989,8 @@ template <template <int, int> class Launch>
 static void dispatch_copy_dtypes(const CopyArgs& a, unsigned wgs, hipStream_t stream) {
 #define DT_COPY_CASE(S, T) \
   if (a.src_dtype == S && a.dst_dtype == T) return Launch<S, T>::run(a, wgs, stream);
-  DT_COPY_CASE(DT_BF16, DT_BF16) DT_COPY_CASE(DT_BF16, DT_FP32) DT_COPY_CASE(DT_BF16, DT_FP16)
-  DT_COPY_CASE(DT_FP32, DT_BF16) DT_COPY_CASE(DT_FP32, DT_FP32) DT_COPY_CASE(DT_FP32, DT_FP16)
-  DT_COPY_CASE(DT_FP16, DT_BF16) DT_COPY_CASE(DT_FP16, DT_FP32) DT_COPY_CASE(DT_FP16, DT_FP16)
+  DT_COPY_CASE(DT_BF16, DT_BF16) DT_COPY_CASE(DT_BF16, DT_FP16) DT_COPY_CASE(DT_FP32, DT_FP32)
+  DT_COPY_CASE(DT_FP16, DT_BF16) DT_COPY_CASE(DT_FP16, DT_FP16)
 #undef DT_COPY_CASE
 }
 template <int SRC, int DST>
@@ -995,23 +1012,35 @@ struct LaunchCopyRows64 {
   }
 };
 
-// The launches of state_convert_kernel.  Stores: D = 64 (D = 128, row-mapped kernel -> this: 1000 x 40 heads 7.7 -> 7.6 us, but 2001 x
-// 30 10.1 -> 10.4 and 14 882 x 24 43.5 -> 46.8).  Loads: below 2^16 rows (2222 x 48, D = 64, state_widen_kernel -> this: 9.5 -> 9.8,
-// 6851 x 48, D = 128 41.5 -> 42.1).
-static bool is_convert(const CopyArgs& a, int D) {
-  if ((a.src_dtype == DT_FP32) == (a.dst_dtype == DT_FP32) || !lanes_fit(a.B, a.Sq, a.H, D)) return false;
-  return a.src_dtype == DT_FP32 ? D == 64 : (int64_t)a.B * a.Sq * a.H < (1 << 16);
-}
-
-static int launch_convert(const CopyArgs& a, int D, hipStream_t stream) {
-  const RowIndex at = row_index(a.B, a.Sq, a.H);
-  const dim3 grid = lane_grid(at, D), block(kUpdateThreads);
-  if (a.dst_dtype == DT_BF16) hipLaunchKernelGGL((state_convert_kernel<64, DT_FP32, DT_BF16>), grid, block, 0, stream, a, at);
-  else if (a.dst_dtype == DT_FP16) hipLaunchKernelGGL((state_convert_kernel<64, DT_FP32, DT_FP16>), grid, block, 0, stream, a, at);
-  else if (D == 64 && a.src_dtype == DT_BF16) hipLaunchKernelGGL((state_convert_kernel<64, DT_BF16, DT_FP32>), grid, block, 0, stream, a, at);
-  else if (D == 64) hipLaunchKernelGGL((state_convert_kernel<64, DT_FP16, DT_FP32>), grid, block, 0, stream, a, at);
-  else if (a.src_dtype == DT_BF16) hipLaunchKernelGGL((state_convert_kernel<128, DT_BF16, DT_FP32>), grid, block, 0, stream, a, at);
-  else hipLaunchKernelGGL((state_convert_kernel<128, DT_FP16, DT_FP32>), grid, block, 0, stream, a, at);
+// An lse tile's query positions: one value a lane or two, in runs of at least 16, or where there are many rows 64 (whole lines of a [H][S]
+// tensor; with fewer rows the few workgroups that result finish long behind the others), and no more than 4096 values: every
+// workgroup of the launch holds that much LDS.
+static int launch_convert(const CopyArgs& a, int D, bool with_lse, hipStream_t stream) {
+  const int64_t rows = (int64_t)a.B * a.Sq * a.H;
+  const int heads = std::min(a.H, kLseHeads);
+  ConvertPlan plan{};
+  plan.groups = rows * D / 4;
+  plan.run_shift = 4;
+  while (plan.run_shift < 8 && heads << plan.run_shift <= 128) ++plan.run_shift;
+  if (rows >= 1 << 18)
+    while (plan.run_shift < 6 && heads << (plan.run_shift + 1) <= 4096) ++plan.run_shift;
+  const int64_t runs = ((int64_t)a.Sq + (1 << plan.run_shift) - 1) >> plan.run_shift;
+  const int64_t w_lse = with_lse ? a.B * runs * ((a.H + kLseHeads - 1) / kLseHeads) : 0;
+  const int64_t w_out = (plan.groups + kConvThreads * kConvGroups - 1) / (kConvThreads * kConvGroups);
+  if (w_out + w_lse >= 1ll << 24) {   // (fewer than 2^32 lanes)
+    set_error("copy grid too large");
+    return DT_ERR_INVALID;
+  }
+  plan.lse_wgs = (uint32_t)w_lse;
+  const dim3 grid((unsigned)(w_out + w_lse)), block(kConvThreads);
+  const size_t lds = with_lse ? (size_t)(heads << plan.run_shift) * 4 : 0;
+  if (a.src_dtype == DT_FP32) {
+    if (a.dst_dtype == DT_FP16) hipLaunchKernelGGL((state_convert_kernel<true, true>), grid, block, lds, stream, a, plan);
+    else hipLaunchKernelGGL((state_convert_kernel<true, false>), grid, block, lds, stream, a, plan);
+  } else {
+    if (a.src_dtype == DT_FP16) hipLaunchKernelGGL((state_convert_kernel<false, true>), grid, block, lds, stream, a, plan);
+    else hipLaunchKernelGGL((state_convert_kernel<false, false>), grid, block, lds, stream, a, plan);
+  }
   return hip_fail(hipGetLastError(), "state_convert launch");
 }
 
@@ -1039,31 +1068,9 @@ int launch_copy(const CopyArgs& a, int D, hipStream_t stream) {
     set_error("head dim %d not built (64 and 128 are)", D);
     return DT_ERR_UNSUPPORTED;
   }
-  if (is_convert(a, D)) return launch_convert(a, D, stream);
-  if (a.src_dtype != DT_FP32 && a.dst_dtype == DT_FP32) {
-    const int64_t rows = (int64_t)a.B * a.Sq * a.H;
-    const int64_t groups = rows * D / 4;
-    const int64_t w_out = (groups + kConvThreads - 1) / kConvThreads;
-    // Query positions per lse workgroup.  Runs of 64 floats per head read whole 256-byte lines of a [H][S] source,
-    // but on a small state the few workgroups that result each walk a dozen dependent rounds of loads and finish
-    // long after the streaming part (2222 x 48 heads: 35 workgroups of 3072 values, 16.6 us for a 42 MB launch
-    // against 10 us with runs of 16); so a workgroup takes about 1024 values, in runs of at least 16 floats.
-    int lse_run = a.H <= 256 ? 64 : std::max(1, 16384 / a.H);   // at most 64 KB of LDS
-    if ((int64_t)a.B * a.Sq * a.H < (1 << 18)) lse_run = std::min(lse_run, std::max(16, 1024 / a.H / 16 * 16));
-    const int64_t w_lse = with_lse ? (int64_t)a.B * ((a.Sq + lse_run - 1) / lse_run) : 0;
-    if (w_out + w_lse <= 0) return DT_OK;
-    if (w_out + w_lse > 0x7fffffffLL || (int64_t)lse_run * a.H * 4 > 65536) {
-      set_error("copy grid too large");
-      return DT_ERR_INVALID;
-    }
-    hipLaunchKernelGGL(state_widen_kernel, dim3((unsigned)(w_out + w_lse)), dim3(kConvThreads),
-                       with_lse ? (size_t)lse_run * a.H * 4 : 0, stream, a, groups, (uint32_t)w_lse, lse_run);
-    return hip_fail(hipGetLastError(), "state_widen launch");
-  }
+  if ((a.src_dtype == DT_FP32) != (a.dst_dtype == DT_FP32)) return launch_convert(a, D, with_lse, stream);
   if (D == 64 && unit_tiles_fit(a.H, D)) {
-    // one 16-bit type into another, or another lse layout: two neighbouring rows per lane group, query x head tiles (fp32 -> slot
-    // at 714 336 rows, which is state_convert_kernel's now: 5.70 against 5.44 TB/s for the row mapping; at D = 128 the row mapping
-    // with its contiguous lse runs is the faster one, 6.3 against 6.0)
+    // one 16-bit type into another, or another lse layout: two neighbouring rows per lane group, query x head tiles
     const int64_t wgs = unit_grid(a.B, a.Sq, a.H, D, true, 1);
     if (wgs <= 0) return DT_OK;
     if (wgs > 0x7fffffffLL) {
