@@ -11,6 +11,21 @@ namespace dt {
 void set_error(const char* fmt, ...);
 int hip_fail(hipError_t e, const char* what);
 
+// n / d for n < 2^31, with mul = ceil(2^(31 + L) / d) and shift = L - 1 for the smallest L with d <= 2^L: the error of mul, less
+// than d, times n stays below 2^(31 + L).  d = 1: shift -1.
+struct Quotient {
+  uint32_t mul;
+  int32_t shift;
+};
+static inline Quotient quotient_by(int32_t d) {
+  int L = 0;
+  while ((1ll << L) < d) ++L;
+  return {L == 0 ? 0u : (uint32_t)(((1ull << (31 + L)) + (uint64_t)d - 1) / (uint64_t)d), L - 1};
+}
+__device__ __forceinline__ uint32_t quotient(uint32_t n, const Quotient& by) {
+  return by.shift < 0 ? n : __umulhi(n, by.mul) >> by.shift;
+}
+
 // One KV chunk, one reference of a job to a chunk, one job of an attention launch: a record each, so that a workgroup finds
 // what it needs in one or two cache lines.
 struct AttnChunk {

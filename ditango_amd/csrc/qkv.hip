@@ -3,18 +3,20 @@
 // Replaces the concatenation, the three library products and the two producer launches of
 // executor/cogvideox/attention_processor.py:39-71.
 //
-// What bounds it: the matrix pipe, busy 54 % of the time for 48 heads x 2222 tokens x 3072 channels (126 GFLOP), with LDS reads behind it (70 to
-// 85 % as many cycles as the MFMAs); of 141 us, with the tables of cos and sin not yet in the LDS, 28 were the loads of the tiles, 18 of those
-// their issue (timed with loads left out, and with loads of one place), 18 start and end.  In a loop of calls, modules and producer -> this:
-// the same 153 -> 127 us (990 TFLOP/s), 16 heads x 602 x 1024 42 -> 16.  From 200 GFLOP on the library's products take less (48 x 8016 429 -> 458), and the adapter calls the modules.
+// What bounds it: loads and MFMAs, which overlap only in part.  48 heads x 2222 tokens x 3072 channels (126 GFLOP), us per call, timed with work
+// left out: all 122, without the loads of the loop 103, without its MFMAs 84, four steps of 96 27 (41 MB of results leave at once; tables
+// and norm); MFMAs alone hold 1.8 GHz and take 67.  The loads are some 37 KB a CU and step, which come at 58 GB/s a CU whatever their rows and
+// however far ahead they are issued.  In a loop of calls, modules and producer -> this: the same 153 -> 122 us (1030 TFLOP/s), 16 heads x 602 x
+// 1024 42 -> 17.  From 200 GFLOP on the library's products take less (48 x 8016 429 -> 458), and the adapter calls the modules.
 // out^T = W X^T with v_mfma_f32_32x32x16, accumulated in fp32.  A wavefront owns one head (64 output columns) of 32 MB tokens; with
 // the product transposed a lane holds 32 of the 64 columns of ONE token, four neighbouring ones at a time.
 //   * A workgroup of 8 wavefronts takes BM = 32 MB WM tokens x BN = 64 (8 / WM) columns of the three outputs side by side.
-//   * Steps of 64 input channels with two LDS buffers, of 32 with three where the tile is 160 x 512: tiles go from memory straight into the
+//   * Steps of 64 input channels with two LDS buffers, of 32 with three where the tile is 320 x 256: tiles go from memory straight into the
 //     LDS (global_load_lds, one or two steps ahead) as rows of 128 or 64 bytes, their 16-byte pieces permuted by the row so that operand
 //     reads meet in no bank.
 //   * The two wavefronts of a SIMD issue their loads at different halves of the step (an M0 write and a load each 20 cycles or so,
-//     in which a wavefront issues no MFMA): 48 heads x 2222 tokens 140 -> 128 us together with the epilogue's tables through the LDS.
+//     in which a wavefront issues no MFMA; together with the epilogue's tables through the LDS 140 -> 128 us), and an operand read follows
+//     each MFMA (128 -> 125).
 //   * One barrier a step, in its middle: in front of it a wavefront has read the last operands it needs of the step's buffer and
 //     waited for its own loads of the next one; behind it come the first operands of the next step, half a step before the MFMAs
 //     that take them.
@@ -41,6 +43,9 @@ constexpr int kHead = 64;
 constexpr int kXcds = 8;
 constexpr int kStageBytes = kWaves * 32 * kHead * 2;   // output rows on their way
 
+constexpr int kLds = 163840;                           // of a CU
+constexpr int table_pieces(int MB, int WM) { return std::min(MB, (kLds - kStageBytes) / (2 * 32 * WM * kHead * 4)); }   // that fit beside the rows
+
 struct QkvProj {
   const uint16_t* w;          // [N, K]
   const uint16_t* bias;       // [N] or null
@@ -55,6 +60,7 @@ struct QkvArgs {
   int32_t T, S, M;            // text tokens, all tokens of a sample, of the batch
   int32_t N, K;               // output columns of one projection, input channels
   int32_t m_tiles, tiles, per_xcd;
+  Quotient by_s;              // tokens by S
   const float *cos, *sin;     // [S - T, 64]
   QkvProj proj[3];
 };
@@ -123,6 +129,8 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
   const int wm = wave / WN, wn = wave - wm * WN;
   const int steps = a.K / kStep;
 
+  // (a division by a variable is some 30 instructions)
+  auto batch_of = [&](int m) __attribute__((always_inline)) { return (int)quotient((uint32_t)m, Quotient{a.by_s.mul, a.by_s.shift}); };
   // ---- this lane's place in the tiles it loads: rows past the end are the last one's again
   const uint16_t* from[kMost];
 #pragma unroll
@@ -130,10 +138,10 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
     const int row = (i * kWaves + wave) * kRowsPer + lane / kPieces;
     const int piece = (lane % kPieces) ^ ((row >> kSwzShift) & (kPieces - 1));
     if (row < BM) {
-      const int m = min(m0 + row, a.M - 1), b = m / a.S, s = m - b * a.S;
+      const int m = min(m0 + row, a.M - 1), b = batch_of(m), s = m - b * a.S;
       from[i] = s < a.T ? a.text + b * a.text_sb + s * a.text_ss : a.video + b * a.video_sb + (int64_t)(s - a.T) * a.video_ss;
     } else {
-      const int n = min(n0 + row - BM, 3 * a.N - 1), p = n / a.N;
+      const int n = min(n0 + row - BM, 3 * a.N - 1), p = (n >= a.N) + (n >= 2 * a.N);
       const uint16_t* w = p == 0 ? a.proj[0].w : p == 1 ? a.proj[1].w : a.proj[2].w;
       from[i] = w + (int64_t)(n - p * a.N) * a.K;
     }
@@ -172,13 +180,20 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
     for (int j = 0; j < 2; ++j) o.w[j] = *reinterpret_cast<const typename E::x8*>(at + (BM + wn * kHead + 32 * j) * kRowBytes);
 #pragma unroll
     for (int i = 0; i < MB; ++i) o.x[i] = *reinterpret_cast<const typename E::x8*>(at + (wm * 32 * MB + 32 * i) * kRowBytes);
-    __builtin_amdgcn_sched_barrier(0);
   };
   auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[j][i] = E::mfma(o.w[j], o.x[i], acc[j][i]);
+    // the reads in front of them, one behind each: in front of all, the first MFMA waits until the LDS has taken every one
+    constexpr int kReads = MB + 2, kMfmas = 2 * MB;
+#pragma unroll
+    for (int i = 0; i < kReads; ++i) {
+      if (i < kMfmas) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    if (kMfmas > kReads) __builtin_amdgcn_sched_group_barrier(0x008, kMfmas - kReads, 0);
     __builtin_amdgcn_sched_barrier(0);
   };
   load_step(0);
@@ -211,21 +226,26 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
 
   // ---- bias, LayerNorm, RoPE; a wavefront's rows go through LDS of its own, so that stores are whole rows.  The tables of the
   // workgroup's tokens come into the LDS once for all of its heads (from memory for each, the launch took 25 us longer).
-  constexpr int kTable = BM * kHead * 4;
-  float* tables = reinterpret_cast<float*>(lds + kStageBytes);
+  // They come in pieces, 32 rows for each of the WM wavefronts along the tokens, as many at a time as the LDS holds.
+  constexpr int kTable = 32 * WM * kHead * 4, kPieces32 = table_pieces(MB, WM);
   bool rotates = false;   // a projection of the workgroup's columns
 #pragma unroll
   for (int p = 0; p < 3; ++p) rotates |= a.proj[p].rope && n0 < (p + 1) * a.N && n0 + BN > p * a.N;
-  if (rotates) {
+  auto tables = [&](int piece) __attribute__((always_inline)) { return (uint32_t)(kStageBytes + piece % kPieces32 * 2 * kTable); };
+  auto load_tables = [&](int piece) __attribute__((always_inline)) {
+    if (!rotates) return;
 #pragma unroll
-    for (int i = 0; i < BM / 32; ++i) {
-      const int row = (i * kWaves + wave) * 4 + (lane >> 4), s = min(m0 + row, a.M - 1) % a.S;
+    for (int i = 0; i < WM; ++i) {
+      const int row = (i * kWaves + wave) * 4 + (lane >> 4);
+      const int m = min(m0 + (row / 32 * MB + piece) * 32 + row % 32, a.M - 1), s = m - batch_of(m) * a.S;
       const int64_t at = (int64_t)max(s - a.T, 0) * kHead + 4 * (lane & 15);
-      const uint32_t to = lds0 + kStageBytes + (i * kWaves + wave) * 1024;
+      const uint32_t to = lds0 + tables(piece) + (i * kWaves + wave) * 1024;
       load_block_to_lds(reinterpret_cast<const uint16_t*>(a.cos + at), to);
       load_block_to_lds(reinterpret_cast<const uint16_t*>(a.sin + at), to + kTable);
     }
-  }
+  };
+#pragma unroll
+  for (int piece = 0; piece < kPieces32; ++piece) load_tables(piece);
   const int n_wave = n0 + wn * kHead;
   const bool mine = n_wave < 3 * a.N;
   const int p = mine ? n_wave / a.N : 0, n_proj = mine ? n_wave - p * a.N : 0;
@@ -242,88 +262,98 @@ __global__ __launch_bounds__(kThreads, 2) void qkv_kernel(const QkvArgs args_by_
   const u32x4 nb = pr.nb ? *reinterpret_cast<const u32x4*>(pr.nb + d) : u32x4{0, 0, 0, 0};
   wait_loads<0>();
   step_barrier();
-  if (!mine) return;
   uint8_t* stage = lds + wave * (32 * kHead * 2);
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
-    const int block = (wm * MB + i) * 32, m_first = m0 + block;
-    if (m_first >= a.M) break;
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {   // rounded as the projection's output is
-        u32x2 x;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const f32x2 b = unpack2<kHalf>(bias[j][g][e]);
-          x[e] = pack2<kHalf>(acc[j][i][4 * g + 2 * e] + b.x, acc[j][i][4 * g + 2 * e + 1] + b.y);
-        }
-        *reinterpret_cast<u32x2*>(stage + col * (kHead * 2) + (((4 * j + g) ^ ((col >> 1) & 7)) << 4) + 8 * hh) = x;
-      }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    // eight lanes a row, as in qk_norm_rope_kernel
-    u32x4 raw[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 8 * r + (lane >> 3);
-      raw[r] = *reinterpret_cast<const u32x4*>(stage + row * (kHead * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+    if (i >= kPieces32) {   // its tables have come into the place of an earlier piece's
+      wait_loads<0>();
+      step_barrier();
     }
-    if (pr.norm != DT_NORM_NONE) {
-      float mean[4], ss[4], rs[4], w[8], b[8];
+    const int m_first = m0 + (wm * MB + i) * 32;
+    if (mine && m_first < a.M) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {   // rounded as the projection's output is
+          u32x2 x;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const f32x2 b = unpack2<kHalf>(bias[j][g][e]);
+            x[e] = pack2<kHalf>(acc[j][i][4 * g + 2 * e] + b.x, acc[j][i][4 * g + 2 * e + 1] + b.y);
+          }
+          *reinterpret_cast<u32x2*>(stage + col * (kHead * 2) + (((4 * j + g) ^ ((col >> 1) & 7)) << 4) + 8 * hh) = x;
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      // eight lanes a row, as in qk_norm_rope_kernel
+      u32x4 raw[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float v[8];
-        unpack8<kHalf>(raw[r], v);
-        mean[r] = row_sum<8>(v) * (1.0f / kHead);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] -= mean[r];
-        ss[r] = row_squares<8>(v);
+        const int row = 8 * r + (lane >> 3);
+        raw[r] = *reinterpret_cast<const u32x4*>(stage + row * (kHead * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
       }
-      inverse_rms4<kHead>(ss[0], ss[1], ss[2], ss[3], pr.eps, rs);
-      unpack8<kHalf>(nw, w);
-      unpack8<kHalf>(nb, b);
+      if (pr.norm != DT_NORM_NONE) {
+        float mean[4], ss[4], rs[4], w[8], b[8];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v[8];
-        unpack8<kHalf>(raw[r], v);
+        for (int r = 0; r < 4; ++r) {
+          float v[8];
+          unpack8<kHalf>(raw[r], v);
+          mean[r] = row_sum<8>(v) * (1.0f / kHead);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = layer_norm16<kHalf>(v[e], mean[r], rs[r], w[e], b[e]);
+          for (int e = 0; e < 8; ++e) v[e] -= mean[r];
+          ss[r] = row_squares<8>(v);
+        }
+        inverse_rms4<kHead>(ss[0], ss[1], ss[2], ss[3], pr.eps, rs);
+        unpack8<kHalf>(nw, w);
+        unpack8<kHalf>(nb, b);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) raw[r][e] = pack2<kHalf>(v[2 * e], v[2 * e + 1]);
-      }
-    }
+        for (int r = 0; r < 4; ++r) {
+          float v[8];
+          unpack8<kHalf>(raw[r], v);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 8 * r + (lane >> 3), m = m_first + row;
-      if (pr.rope) {
-        const float* c = tables + (block + row) * kHead + d;
-        const bool video = m % a.S >= a.T;
+          for (int e = 0; e < 8; ++e) v[e] = layer_norm16<kHalf>(v[e], mean[r], rs[r], w[e], b[e]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const f32x2 z = unpack2<kHalf>(raw[r][e]);
-          const f32x2 cs = *reinterpret_cast<const f32x2*>(c + 2 * e), sn = *reinterpret_cast<const f32x2*>(c + kTable / 4 + 2 * e);
-          const uint32_t y = pack2<kHalf>(rotated(z.x, -z.y, cs.x, sn.x), rotated(z.y, z.x, cs.y, sn.y));
-          raw[r][e] = video ? y : raw[r][e];
+          for (int e = 0; e < 4; ++e) raw[r][e] = pack2<kHalf>(v[2 * e], v[2 * e + 1]);
         }
       }
-      if (m < a.M) *reinterpret_cast<u32x4*>(pr.y + (int64_t)m * a.N + n_proj + d) = raw[r];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 8 * r + (lane >> 3), m = m_first + row;
+        if (pr.rope) {
+          const float* c = reinterpret_cast<const float*>(lds + tables(i)) + (32 * wm + row) * kHead + d;
+          const bool video = m - batch_of(m) * a.S >= a.T;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const f32x2 z = unpack2<kHalf>(raw[r][e]);
+            const f32x2 cs = *reinterpret_cast<const f32x2*>(c + 2 * e), sn = *reinterpret_cast<const f32x2*>(c + kTable / 4 + 2 * e);
+            const uint32_t y = pack2<kHalf>(rotated(z.x, -z.y, cs.x, sn.x), rotated(z.y, z.x, cs.y, sn.y));
+            raw[r][e] = video ? y : raw[r][e];
+          }
+        }
+        if (m < a.M) *reinterpret_cast<u32x4*>(pr.y + (int64_t)m * a.N + n_proj + d) = raw[r];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + kPieces32 < MB) {   // everybody is done with this piece's tables
+      step_barrier();
+      load_tables(i + kPieces32);
+    }
   }
 }
 
 template <int MB, int WM, int KH, int NBUF>
-constexpr int lds_bytes() { return std::max(NBUF * (32 * MB * WM + kHead * (kWaves / WM)) * KH * 32, kStageBytes + 2 * 32 * MB * WM * kHead * 4); }
+constexpr int lds_bytes() {
+  return std::max(NBUF * (32 * MB * WM + kHead * (kWaves / WM)) * KH * 32, kStageBytes + table_pieces(MB, WM) * 2 * 32 * WM * kHead * 4);
+}
 
 template <int MB, int WM, int KH, int NBUF, bool kHalf>
 int launch_t(QkvArgs& a, hipStream_t stream) {
-  constexpr int BM = 32 * MB * WM, BN = kHead * (kWaves / WM), kLds = lds_bytes<MB, WM, KH, NBUF>();
-  static_assert(kLds <= 163840, "the LDS of a CU");
+  constexpr int BM = 32 * MB * WM, BN = kHead * (kWaves / WM), kBytes = lds_bytes<MB, WM, KH, NBUF>();
+  static_assert(kBytes <= kLds, "the LDS of a CU");
   static thread_local int allowed_dev = -1;   // more than 64 KB of dynamic LDS has to be allowed once per kernel and device
   int dev = 0;
   if (int rc = hip_fail(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (allowed_dev != dev) {
-    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&qkv_kernel<MB, WM, KH, NBUF, kHalf>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds),
+    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&qkv_kernel<MB, WM, KH, NBUF, kHalf>), hipFuncAttributeMaxDynamicSharedMemorySize, kBytes),
                           "hipFuncSetAttribute"))
       return rc;
     allowed_dev = dev;
@@ -331,7 +361,8 @@ int launch_t(QkvArgs& a, hipStream_t stream) {
   a.m_tiles = (a.M + BM - 1) / BM;
   a.tiles = a.m_tiles * ((3 * a.N + BN - 1) / BN);
   a.per_xcd = (a.tiles + kXcds - 1) / kXcds;
-  hipLaunchKernelGGL((qkv_kernel<MB, WM, KH, NBUF, kHalf>), dim3((unsigned)a.per_xcd * kXcds), dim3(kThreads), kLds, stream, a);
+  a.by_s = quotient_by(a.S);
+  hipLaunchKernelGGL((qkv_kernel<MB, WM, KH, NBUF, kHalf>), dim3((unsigned)a.per_xcd * kXcds), dim3(kThreads), kBytes, stream, a);
   return hip_fail(hipGetLastError(), "qkv launch");
 }
 template <int MB, int WM, int KH, int NBUF>
@@ -339,10 +370,10 @@ int launch(QkvArgs& a, bool half, hipStream_t stream) {
   return half ? launch_t<MB, WM, KH, NBUF, true>(a, stream) : launch_t<MB, WM, KH, NBUF, false>(a, stream);
 }
 
-// Which tile a launch takes: 64 x 256, two workgroups a CU, 192 x 256, 256 x 256 or 160 x 512.  The time of each in us is its rounds of the
+// Which tile a launch takes: 64 x 256, two workgroups a CU, 192 x 256, 256 x 256 or 320 x 256.  The time of each in us is its rounds of the
 // 256 CUs times the 64-channel steps of one, and what a round and the launch cost on top; constants fitted to 70 launches of 8 ... 48 heads
 // (8 ... 48 steps) x 280 ... 12 000 tokens (errors 4 to 5 %; the choice takes 0.9 % more than the best on average).  us, modules and producer ->
-// 64 x 256 / 192 x 256 / 256 x 256 / 160 x 512: 16 heads x 602 tokens 42 -> 18 / 34 / 39 / 49; 24 x 4330 108 -> 94 / 87 / 105 / 78; 48 x 2222
+// 64 x 256 / 192 x 256 / 256 x 256 / 160 x 512 (now 320 x 256, which loads a seventh less and takes 1 % less): 16 heads x 602 tokens 42 -> 18 / 34 / 39 / 49; 24 x 4330 108 -> 94 / 87 / 105 / 78; 48 x 2222
 // 153 -> 167 / 141 / 171 / 130 (252 workgroups of 160 x 512, one round); 48 x 3328 198 -> 248 / 214 / 186 / 235 (468 of 256 x 256, two).
 enum Tiles { kFew, kSome, kMore, kMany };
 Tiles plan(int M, int N, int K) {
@@ -356,7 +387,7 @@ Tiles plan(int M, int N, int K) {
   const int64_t pairs = per_xcd(64, 256) / (2 * kCus), rest = per_xcd(64, 256) % (2 * kCus);
   const double shared = (double)(pairs + (rest > kCus ? 1 : 0)), alone = rest > 0 && rest <= kCus ? 1 : 0;
   const double of[4] = {4.2 + alone * (2.7 + 0.80 * steps) + shared * (9.1 + 1.08 * steps), time(192, 256, 15.4, 1.18, 16.0),
-                        time(256, 256, 17.0, 1.45, 16.0), time(160, 512, 19.8, 1.96, 24.9)};
+                        time(256, 256, 17.0, 1.45, 16.0), time(320, 256, 19.8, 1.96, 24.9)};
   return (Tiles)(std::min_element(of, of + 4) - of);
 }
 
@@ -420,6 +451,6 @@ extern "C" int dt_qkv_project(const void* text, int64_t text_stride_b, int64_t t
     case kFew: return launch<1, 2, 4, 2>(a, half, s);
     case kSome: return launch<3, 2, 4, 2>(a, half, s);
     case kMore: return launch<4, 2, 4, 2>(a, half, s);
-    default: return launch<5, 1, 2, 3>(a, half, s);
+    default: return launch<5, 2, 2, 3>(a, half, s);
   }
 }

@@ -453,8 +453,7 @@ __global__ __launch_bounds__(kThreads) void merge_states_kernel(const MergeArgs 
 struct RowIndex {         // row ((b * Sq) + s) * H + h of B * Sq * H < 2^31 -> its place in the [B,H,Sq] layout
   int32_t Sq, H;
   uint32_t rows;          // B * Sq * H
-  uint32_t mul_h, mul_s;  // n / H and n / Sq for n < 2^31 (see quotient)
-  int32_t shift_h, shift_s;
+  Quotient by_h, by_s;
 };
 struct UpdateArgs {
   const float* run;
@@ -469,20 +468,9 @@ struct UpdateArgs {
 constexpr int kUpdateThreads = 256;
 constexpr int kUpdateGroup = 64;   // workgroups that follow each other on one XCD (1: 3 % slower, 8: the same)
 
-// n / d for n < 2^31, with mul = ceil(2^(31 + L) / d) and shift = L - 1 for the smallest L with d <= 2^L: the error of mul, less
-// than d, times n stays below 2^(31 + L).  d = 1: shift -1.
-__device__ __forceinline__ uint32_t quotient(uint32_t n, uint32_t mul, int shift) {
-  return shift < 0 ? n : __umulhi(n, mul) >> shift;
-}
-static void set_quotient(int32_t d, uint32_t& mul, int32_t& shift) {
-  int L = 0;
-  while ((1ll << L) < d) ++L;
-  mul = L == 0 ? 0u : (uint32_t)(((1ull << (31 + L)) + (uint64_t)d - 1) / (uint64_t)d);
-  shift = L - 1;
-}
 __device__ __forceinline__ uint32_t bhs_of(const RowIndex& at, uint32_t row) {
-  const uint32_t bs = quotient(row, at.mul_h, at.shift_h), h = row - bs * (uint32_t)at.H;
-  const uint32_t b = quotient(bs, at.mul_s, at.shift_s), q = bs - b * (uint32_t)at.Sq;
+  const uint32_t bs = quotient(row, at.by_h), h = row - bs * (uint32_t)at.H;
+  const uint32_t b = quotient(bs, at.by_s), q = bs - b * (uint32_t)at.Sq;
   return (b * (uint32_t)at.H + h) * (uint32_t)at.Sq + q;
 }
 static RowIndex row_index(int B, int Sq, int H) {
@@ -490,8 +478,8 @@ static RowIndex row_index(int B, int Sq, int H) {
   at.Sq = Sq;
   at.H = H;
   at.rows = (uint32_t)((int64_t)B * Sq * H);
-  set_quotient(H, at.mul_h, at.shift_h);
-  set_quotient(Sq, at.mul_s, at.shift_s);
+  at.by_h = quotient_by(H);
+  at.by_s = quotient_by(Sq);
   return at;
 }
 // A grid holds fewer than 2^32 lanes, and these kernels take D / 4 of them a row.

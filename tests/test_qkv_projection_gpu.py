@@ -71,9 +71,10 @@ def _check(got, want, dtype):
     (1, 28, 37, 8, 192, torch.bfloat16),       # one row more than a tile of 64
     (3, 5, 300, 5, 320, torch.bfloat16),       # rows of three samples in one tile
     (1, 113, 2500, 24, 1536, torch.bfloat16),  # 192 x 256
-    (1, 28, 2212, 48, 3072, torch.float16),    # 160 x 512, 14 full tiles of rows
+    (1, 28, 2212, 48, 3072, torch.float16),    # 320 x 256, 7 full tiles of rows
+    (1, 28, 1893, 48, 3072, torch.bfloat16),   # ... one row more than 6
     (1, 28, 3301, 48, 3072, torch.bfloat16),   # 256 x 256, one row more than 13 tiles
-    # columns of 22.5 tiles of 256 or 11.25 of 512, in each of the large tiles; rows of two samples in one tile
+    # columns of 22.5 tiles of 256, in each of the large tiles; rows of two samples in one tile
     (1, 30, 1970, 30, 1920, torch.bfloat16),
     (1, 30, 2970, 30, 1920, torch.float16),
     (1, 30, 4970, 30, 1920, torch.bfloat16),
@@ -95,7 +96,7 @@ def test_projections_match_fp64(hip, B, T, V, H, K, dtype, bias, rotated):
 
 @pytest.mark.parametrize("B,T,V,H,K", [
     (2, 26, 170, 3, 128),
-    (2, 30, 1500, 30, 1920),     # columns of 22.5 tiles of 256, or 11.25 of 512; rows of two samples in one tile
+    (2, 30, 1500, 30, 1920),     # columns of 22.5 tiles of 256; rows of two samples in one tile
     (1, 113, 2500, 24, 1536),
     (1, 28, 2194, 48, 3072),
     (1, 28, 3301, 48, 3072),
