@@ -186,6 +186,9 @@ constexpr float kSumLimit = 4096.0f;
 // simply exp2(score), and a tile is redone when its sum exceeds 2^40.
 constexpr float kSumLimitPre = 1099511627776.0f;
 constexpr float kBandLo = -40.f, kBandHi = 24.f;
+// References of up to this many log2 units are taken off by the MFMAs themselves (see kRefInC).  A score near 0 under a reference
+// of 64 keeps an absolute error of 2^-18, some times that of a score of this size; beyond it the reference comes off in the vector ALU.
+constexpr float kRefInCMost = 64.f;
 
 template <int D>
 struct Tile {
@@ -653,6 +656,12 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   typedef typename E::x8 ex8;
   typedef typename E::x4 ex4;
   typedef typename E::x2 ex2;
+  // The scores of a tile start from minus the reference instead of from zero: C of a product's first MFMA, 16 registers of one value
+  // since a lane owns one query.  What is left to the softmax is a multiplication in place of the multiply-add: an instruction of
+  // half the bytes and operands, which is power the matrix pipe can use.  us per call: 24 heads x 14 882 queries, 4 of 8 chunks 8198 -> 8036, 24 x
+  // 119 056, 3 of 32 15 503 -> 15 256, 24 x 4001, 2 of 4 338.4 -> 332.8, 2 x 24 x 1861, 3 of 8 272 -> 269.  (At D = 64 the registers
+  // are not there: 56 spilled.)
+  constexpr bool kRefInC = D == 128 && !kPre;
   constexpr int kKeyBlocks = kSplitKeys ? 1 : 2;   // 32-key blocks of a tile that a wavefront works on
   // A reference of its own for every place that reads arguments, unrelated to the others as far as the compiler can see:
   // it otherwise reads whole lines at the top and holds what later places need in spilled scalar registers (119 at D = 128 and
@@ -847,7 +856,12 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   // reference (raw scores; kPre: log2 units) the accumulators are scaled to
   float m_ref = kPre ? 0.f : -INFINITY;
   float rs_bias = kPre ? INFINITY : 0.f;  // kPre: inf until the row has seen a key (forces the exact path)
-  bool any_off = false;                   // kPre: some row of this wavefront has a reference other than 0
+  bool any_off = false;                   // some row of this wavefront has a reference that the scores do not start from (kPre: other than 0)
+  float limit = kSumLimit;                // kRefInC: -1, below every sum, while some row of this wavefront has no reference
+  f32x16 neg_ref;                         // kRefInC: what the scores start from
+#pragma unroll
+  for (int r = 0; r < 16; ++r) neg_ref[r] = 0.f;
+  if constexpr (kRefInC) asm volatile("" : "+v"(neg_ref));   // registers, not a constant to be built for every product
   float l_run = 0.f;        // running sum over THIS lane's keys (halves combined at the end)
   const float c = kPre ? 1.f : a.scale_log2;
 
@@ -948,7 +962,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
           f32x16 zero;
 #pragma unroll
           for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-          s_acc[kb] = E::mfma(cur, qf[sidx], zero);
+          s_acc[kb] = E::mfma(cur, qf[sidx], kRefInC ? neg_ref : zero);
         } else {
           s_acc[kb] = E::mfma(cur, qf[sidx], s_acc[kb]);
         }
@@ -1045,11 +1059,12 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
     if constexpr (!kLoadAfterMatrix) load_tile((kU + DT_SCHED_CALL_AHEAD + group) & (kNumBuf - 1));
     // (kPre: the same rare branch takes the reference off the scores of a wavefront in which some
     // row has left the band; everywhere else the reference is 0 and there is nothing to subtract)
-    if (__builtin_expect(cp_valid < kBK || (kPre && any_off), 0)) {
+    if (__builtin_expect(cp_valid < kBK || ((kPre || kRefInC) && any_off), 0)) {
       // the empty asm has side effects as far as the compiler knows, which keeps this a real
       // branch: otherwise the selects below are hoisted out and run for every tile
       asm volatile("" ::: "memory");
       const int lim = cp_valid - key0;
+      const float ref_taken = m_ref > -INFINITY ? m_ref : 0.f;
 #pragma unroll
       for (int kb = 0; kb < kKeyBlocks; ++kb)
 #pragma unroll
@@ -1057,6 +1072,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
           const int key = 32 * kb + 16 * (r >> 3) + 8 * hh + (r & 7);
           if (key >= lim) s_acc[kb][r] = -INFINITY;
           if constexpr (kPre) s_acc[kb][r] -= m_ref;
+          if constexpr (kRefInC) s_acc[kb][r] -= ref_taken + neg_ref[0];
         }
     }
     // Probabilities relative to the reference maximum the accumulators are scaled to.  The
@@ -1082,6 +1098,9 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         if constexpr (kPre) {
           p.x = __builtin_amdgcn_exp2f(s_acc[kb][r]);
           p.y = __builtin_amdgcn_exp2f(s_acc[kb][r + 1]);
+        } else if constexpr (kRefInC) {
+          p.x = __builtin_amdgcn_exp2f(s_acc[kb][r] * c);
+          p.y = __builtin_amdgcn_exp2f(s_acc[kb][r + 1] * c);
         } else {
           p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r], c, -mc));
           p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r + 1], c, -mc));
@@ -1097,7 +1116,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         p_frag[kb][r >> 3][r & 7] = pb.x;
         p_frag[kb][r >> 3][(r & 7) + 1] = pb.y;
       }
-    if (__builtin_expect(__any(!(rs0 + rs1 <= (kPre ? kSumLimitPre : kSumLimit))), 0)) {
+    if (__builtin_expect(__any(!(rs0 + rs1 <= (kPre ? kSumLimitPre : kRefInC ? limit : kSumLimit))), 0)) {
       float mx = s_acc[0][0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s_acc[0][r]);
@@ -1118,7 +1137,9 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         rs_bias = first && !(mx > -INFINITY) ? INFINITY : 0.f;
         mx = m_new - m_ref;  // what the scores in s_acc still have to lose
       } else {
-        m_new = fmaxf(m_ref, mx);
+        const float taken = kRefInC && m_ref > -INFINITY ? m_ref : 0.f;   // off the scores already
+        m_new = fmaxf(m_ref, mx + taken);
+        mx = m_new - taken;
         alpha = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m_ref - m_new) * c) : 1.f;
       }
       m_ref = m_new;
@@ -1130,7 +1151,15 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
           for (int r = 0; r < 16; ++r) o_acc[i][r] *= alpha;
       }
       // a row whose keys are all masked so far keeps m_ref = -inf: use 0 so that exp2(-inf - 0) = 0
-      mc = kPre ? mx : (m_new > -INFINITY ? m_new * c : 0.f);
+      mc = kPre ? mx : (m_new > -INFINITY ? mx * c : 0.f);
+      if constexpr (kRefInC) {
+        const bool in_c = __builtin_fabsf(m_new * c) <= kRefInCMost;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) neg_ref[r] = in_c ? -m_new : 0.f;
+        asm volatile("" : "+v"(neg_ref));
+        any_off = __any(!in_c && m_new > -INFINITY);
+        limit = __any(!(m_new > -INFINITY)) ? -1.f : kSumLimit;
+      }
       if constexpr (kPre) any_off = any_off || __any(m_ref != 0.f);
       rs0 = 0.f;
       rs1 = 0.f;
