@@ -8,6 +8,8 @@
 //   * One workgroup = 8 wavefronts = 256 queries of one (batch, head); each
 //     wavefront owns 32 queries.  D = 128: one workgroup per CU, two wavefronts per
 //     SIMD (256 VGPRs each); D = 64: two workgroups per CU (128 VGPRs each).
+//     (Launches too small to fill the chip with those: 32 queries, whose keys
+//     the wavefronts share, see attn_rows32.)
 //   * The 8 wavefronts form two groups of 4 that run the same loop ONE PHASE
 //     APART ("ping-pong"): while group A issues the MFMAs of a tile
 //     (O^T += V^T P^T of the previous tile, then S^T = K Q^T of this one), group B
@@ -413,9 +415,9 @@ constexpr int kWavesPerSimdD64 = 4;
 // for the argument reads in front of the first tile load, 1.4 with them prefetched; the launch against one key tile 9.5 -> 7.9 us at
 // D = 64, 10.3 -> 9.4 at D = 128, together with the wait for Q behind the first tile loads).  The loads and their wait are one asm statement, so no register is pending behind it.
 constexpr int kArgLine = 64;
+constexpr int kJobAt = (int)offsetof(AttnArgs, job), kChunkAt = (int)offsetof(AttnArgs, chunk), kEntryAt = (int)offsetof(AttnArgs, entry);
 __device__ __forceinline__ void prefetch_args(uint64_t args) {
   uint32_t t0, t1, t2, t3, t4, t5, t6, t7, t8, t9, t10, t11, t12, t13;
-  constexpr int kJob = (int)offsetof(AttnArgs, job), kChunk = (int)offsetof(AttnArgs, chunk), kEntry = (int)offsetof(AttnArgs, entry);
   asm volatile(
       "s_load_dword %0, %14, 0x0\n\ts_load_dword %1, %14, 0x40\n\ts_load_dword %2, %14, 0x80\n\ts_load_dword %3, %14, 0xc0\n\t"
       "s_load_dword %4, %14, %15\n\ts_load_dword %5, %14, %16\n\ts_load_dword %6, %14, %17\n\ts_load_dword %7, %14, %18\n\t"
@@ -423,8 +425,8 @@ __device__ __forceinline__ void prefetch_args(uint64_t args) {
       "s_load_dword %12, %14, %23\n\ts_load_dword %13, %14, %24\n\ts_waitcnt lgkmcnt(0)"
       : "=&s"(t0), "=&s"(t1), "=&s"(t2), "=&s"(t3), "=&s"(t4), "=&s"(t5), "=&s"(t6), "=&s"(t7), "=&s"(t8), "=&s"(t9), "=&s"(t10),
         "=&s"(t11), "=&s"(t12), "=&s"(t13)
-      : "s"(args), "i"(kJob), "i"(kJob + kArgLine), "i"(kJob + 2 * kArgLine), "i"(kJob + 3 * kArgLine), "i"(kChunk),
-        "i"(kChunk + kArgLine), "i"(kChunk + 2 * kArgLine), "i"(kChunk + 3 * kArgLine), "i"(kEntry), "i"(kEntry + kArgLine)
+      : "s"(args), "i"(kJobAt), "i"(kJobAt + kArgLine), "i"(kJobAt + 2 * kArgLine), "i"(kJobAt + 3 * kArgLine), "i"(kChunkAt),
+        "i"(kChunkAt + kArgLine), "i"(kChunkAt + 2 * kArgLine), "i"(kChunkAt + 3 * kArgLine), "i"(kEntryAt), "i"(kEntryAt + kArgLine)
       : "memory");
 }
 
@@ -476,16 +478,17 @@ __device__ __forceinline__ bool arrive_last(uint32_t* counter, int expected) {
 // heads x 96 queries, two states, D = 64 12.8 -> 12.6, D = 128 15.3 -> 15.2, 4 states 15.9 -> 16.4; 12 x 700, D = 64 17.3 -> 17.2; 24 x 4000,
 // 3 of 8 chunks 540 -> 540).  More states keep 32 rows of sums in registers and two steps in flight (three make no difference to 29
 // states of 743 MB).
-template <int D, bool kHalf, int kStates, bool kOneBatch>
+template <int D, bool kHalf, int kStates, bool kOneBatch, int kRows = 32>
 __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row0) {
   typedef Elem<kHalf> E;
   constexpr int kLoads = D == 128 ? kStates : 4;        // states of a step
   constexpr int kParts = kStates / kLoads;              // steps of the same rows
-  constexpr int kDepth = (kOneBatch ? D / 4 : D / 8) / kLoads;   // steps in flight
   constexpr int kRowLanes = D / 8;                      // a lane holds 8 columns of a row
   constexpr int kRowsPer = 64 / kRowLanes;              // rows of a load instruction
-  constexpr int kRowSteps = 32 / kRowsPer;
+  constexpr int kRowSteps = kRows / kRowsPer;
   constexpr int kSteps = kRowSteps * kParts;            // steps of a batch of states
+  constexpr int kDepthMost = (kOneBatch ? D / 4 : D / 8) / kLoads;
+  constexpr int kDepth = kDepthMost < kSteps ? kDepthMost : kSteps;   // steps in flight
   static_assert(kMergeBatch % kStates == 0, "the lists are filled up to whole batches");
   static_assert(kSteps % kDepth == 0, "a step's registers are known at compile time");
   KernArgs& a = kernel_args();
@@ -493,7 +496,7 @@ __device__ __forceinline__ void merge_rows(uint8_t* stage, int b, int h, int row
   KernState* states = a.dev_ids ? a.arena : a.state;
   const int lane = threadIdx.x & 63, col = lane & 31;
   const int n = a.merge_n, H = a.H, Sq = a.Sq;
-  const int rows = min(32, Sq - row0);
+  const int rows = min(kRows, Sq - row0);
   const int64_t lse_at = ((int64_t)b * H + h) * Sq + row0;
   const int64_t out_at = (((int64_t)b * Sq + row0) * H + h) * D;
   const uint32_t row_bytes = (uint32_t)H * D * 2u;
@@ -1476,6 +1479,321 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   }
 }
 
+// ---- launches of few query rows -----------------------------------------------------------------
+// A launch that leaves CUs idle is a chain of waits: start, tiles one after the other at the pace of two groups that meet at
+// barriers (0.7 us a tile where nothing else runs: 4 heads x 512 queries, D = 64), result, merge.  Here a workgroup has 32
+// queries instead of 256, and its eight wavefronts share the KEYS: wavefront w takes the tiles w, w + 8 ..., by itself, from
+// registers and LDS of its own, with no barrier; their states meet once, in fp32 through the LDS.  A chunk of 512 keys is one
+// tile deep.  The keys and values are read by eight times as many workgroups: 110 GB/s a CU out of the L2 is what longer
+// ones are bound by, and why short_rows ends at 32 tiles.
+// us per call, workgroups of 256 (128) queries -> this: D = 64 4 heads x 512 queries, 2 of 4 chunks 15.1 -> 9.2, 8 x 1024, 1 of 4 18.9 ->
+// 10.9, 16 x 300, 2 of 4 17.8 -> 10.3, 16 x 64 10.4 -> 7.1; D = 128 4 x 512 17.7 -> 13.5, 4 x 128 14.7 -> 8.8, 24 x 128 15.3 -> 9.9,
+// 8 x 1024 24.1 -> 18.7.
+// K and V of a tile take the same 8 (16) KB of LDS in turn.  K read from memory as fragments, beside V, was 1.2 ... 4 us longer at
+// the sizes above: an instruction then touches 32 lines for 32 bytes each, and what the L1 holds of them is gone before the
+// next one asks for the rest of the line.
+struct AttnRows : AttnArgs {};   // (names the kernel; part_ways: slices of 32 rows of a head, tail_items: slices of an XCD)
+constexpr int kRowsStates = 4;    // states that such a launch merges itself, at most (short_launch_merges allows no more)
+// LDS: the tile of each wavefront (afterwards its share of the state), references and sums, 32 result rows.
+template <int D>
+struct Rows32 {
+  static constexpr int kOffRef = kWaves * Tile<D>::kBytesV;           // [8 wavefronts][reference, sum][32 queries]
+  static constexpr int kOffRows = kOffRef + kWaves * 2 * 32 * 4;
+  static constexpr int kOffFlag = kOffRows + 32 * Tile<D>::kRowBytes;
+  static constexpr int kLdsBytes = kOffFlag + 16;
+  static constexpr int kGroups = D / 8;                               // 4-element groups of a lane's accumulators
+  static_assert(kGroups * 1024 == Tile<D>::kBytesV, "a wavefront's accumulators take the place of its V tile");
+};
+
+// 32 queries of one job, batch and head: wavefront w works on the key tiles w, w + 8 ... on its own.
+template <int D, bool kHalf, bool kMerge>
+__device__ __forceinline__ void attn_rows32(const JobView& view, int b, int h, int row0) {
+  using T = Tile<D>;
+  using R = Rows32<D>;
+  using E = Elem<kHalf>;
+  typedef typename E::x8 ex8;
+  typedef typename E::x4 ex4;
+  typedef typename E::x2 ex2;
+  KernArgs& a = kernel_args();
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  typedef __attribute__((address_space(3))) uint8_t* lds_ptr_t;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, hh = lane >> 5;
+  const int q0 = view.q_begin + row0;
+  uint8_t* const v_tile = lds + wave * T::kBytesV;
+  const uint32_t v_addr = (uint32_t)(uintptr_t)(lds_ptr_t)lds + wave * T::kBytesV;
+
+  // ---- the cursor: tile `tile` of the chunk reference `seg`
+  const uint32_t row_bytes = (uint32_t)a.kv_ss * 2u;
+  int seg = view.seg_begin, tile = wave;
+  u32x4 rk, rv;
+  int keys = 0;
+  bool opened = false;
+  // Finds the tile; false behind the last one.
+  auto seek = [&]() __attribute__((always_inline)) -> bool {
+    while (seg < view.seg_end) {
+      if (!opened) {
+        const KeyRef r = key_ref(view, seg);
+        keys = r.len;
+        if (keys > 0) {
+          const int64_t head_off = (int64_t)b * a.chunk[r.cid].sb + (int64_t)h * a.kv_sh + (int64_t)r.begin * a.kv_ss;
+          const uint32_t valid = (uint32_t)(keys - 1) * row_bytes + (uint32_t)(D * 2);
+          rk = make_rsrc(a.chunk[r.cid].k + head_off, valid);
+          rv = make_rsrc(a.chunk[r.cid].v + head_off, valid);
+        }
+        opened = true;
+      }
+      const int tiles = (keys + kBK - 1) / kBK;
+      if (tile < tiles) return true;
+      tile -= tiles;
+      ++seg;
+      opened = false;
+    }
+    return false;
+  };
+  // K is read into registers, then V is loaded over it.  The swizzles are those of the other form.
+  uint32_t k_row, k_chunk, kld;
+  {
+    const int lrow = lane / T::kChunks, pos = lane % T::kChunks, krow = key_of_row(col);
+    k_row = (uint32_t)lrow * row_bytes;
+    k_chunk = 16u * (uint32_t)(pos ^ T::swz_k(lrow));
+    kld = krow * T::kRowBytes + 16 * (hh ^ T::swz_k(krow));
+  }
+  auto load_k = [&]() __attribute__((always_inline)) {
+    const uint32_t off = (uint32_t)(tile * kBK) * row_bytes;
+    uint32_t block = T::kRowsPerBlock * row_bytes;
+    asm volatile("" : "+s"(block));   // (added where it is used: the sums would be held in registers)
+#pragma unroll
+    for (int i = 0; i < T::kBlocks; ++i)
+      load_block_to_lds(rk, k_row + (k_chunk ^ (16 * T::swz_k(T::kRowsPerBlock * i))) + i * block, off, v_addr + i * 1024);
+  };
+  uint32_t v_lane;
+  {
+    const int lrow = lane / T::kChunks, pos = lane % T::kChunks;
+    v_lane = (uint32_t)lrow * row_bytes + 16u * (uint32_t)((((pos >> 2) ^ T::swz_v(lrow)) << 2) | (pos & 3));
+    static_assert(T::swz_v(T::kRowsPerBlock) == T::swz_v(0), "the swizzle of a block's rows is that of the first block's");
+  }
+  auto load_v = [&]() __attribute__((always_inline)) {
+    const uint32_t off = (uint32_t)(tile * kBK) * row_bytes;
+    uint32_t block = T::kRowsPerBlock * row_bytes;
+    asm volatile("" : "+s"(block));
+#pragma unroll
+    for (int i = 0; i < T::kBlocks; ++i) load_block_to_lds(rv, v_lane + i * block, off, v_addr + i * 1024);
+  };
+
+  bool more = seek();
+  ex8 qf[D / 16];
+  {
+    const uint16_t* qp = a.q + (int64_t)b * a.q_sb + (int64_t)h * a.q_sh + (int64_t)min(q0 + col, view.q_end - 1) * a.q_ss + 8 * hh;
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) qf[s] = *reinterpret_cast<const ex8*>(qp + 16 * s);
+  }
+  f32x16 o_acc[D / 32];
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.f;
+  float m_ref = -INFINITY, l_run = 0.f;
+  const float c = a.scale_log2;
+  uint32_t vld[T::kSegs];
+  {
+    const int vrow = 8 * hh + ((lane & 15) >> 2);
+#pragma unroll
+    for (int g = 0; g < T::kSegs; ++g)
+      vld[g] = vrow * T::kRowBytes + 64 * (g ^ T::swz_v(vrow)) + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  }
+  if (more) load_k();
+  while (more) {
+    ex8 kf[2][D / 16];
+    wait_tile_loads<0>();
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) kf[kb][s] = *reinterpret_cast<const ex8*>(v_tile + (kld ^ (32 * s)) + kb * 32 * T::kRowBytes);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // nothing is read from the tile any more
+    load_v();
+    const int lim = keys - tile * kBK;
+    f32x16 s_acc[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_acc[kb][r] = 0.f;
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) s_acc[kb] = E::mfma(kf[kb][s], qf[s], s_acc[kb]);
+    }
+    tile += kWaves;
+    more = seek();
+    if (lim < kBK) {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * kb + 16 * (r >> 3) + 8 * hh + (r & 7) >= lim) s_acc[kb][r] = -INFINITY;
+    }
+    float mx = s_acc[0][0];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s_acc[kb][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    // (the reference in log2 units, rounded once: what the probabilities lose and what the states are weighted by is then the same number)
+    const float m_new = fmaxf(m_ref, mx * c);
+    const float alpha = m_new > -INFINITY ? __builtin_amdgcn_exp2f(m_ref - m_new) : 1.f;
+    m_ref = m_new;
+    l_run *= alpha;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o_acc[i][r] *= alpha;
+    const float mc = m_new > -INFINITY ? m_new : 0.f;
+    float rs0 = 0.f, rs1 = 0.f;
+    ex8 p_frag[2][2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        f32x2 p;
+        p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r], c, -mc));
+        p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r + 1], c, -mc));
+        rs0 += p.x;
+        rs1 += p.y;
+        const ex2 pb = __builtin_convertvector(p, ex2);
+        p_frag[kb][r >> 3][r & 7] = pb.x;
+        p_frag[kb][r >> 3][(r & 7) + 1] = pb.y;
+      }
+    l_run += rs0 + rs1;
+    wait_tile_loads<0>();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        if (kb + half > 0) __builtin_amdgcn_sched_barrier(0x40f);   // no more than the operands of a step at a time
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) {
+          const uint8_t* p = v_tile + vld[db] + (32 * kb + 16 * half) * T::kRowBytes;
+          const s16x4 lo = lds_read_tr(p);
+          const s16x4 hi = lds_read_tr(p + 4 * T::kRowBytes);
+          const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+          o_acc[db] = E::mfma(__builtin_bit_cast(ex8, both), p_frag[kb][half], o_acc[db]);
+        }
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // nothing is read from the tile any more
+    if (more) load_k();
+  }
+
+  // ---- the eight states meet in the LDS: every wavefront adds up an eighth of the columns
+  float* const refs = reinterpret_cast<float*>(lds + R::kOffRef);
+  l_run += __shfl_xor(l_run, 32);
+  if (hh == 0) {
+    refs[wave * 64 + col] = m_ref;
+    refs[wave * 64 + 32 + col] = l_run;
+  }
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(v_tile + (4 * i + g) * 1024 + lane * 16) =
+          f32x4{o_acc[i][4 * g], o_acc[i][4 * g + 1], o_acc[i][4 * g + 2], o_acc[i][4 * g + 3]};
+  phase_barrier();
+  float w[kWaves], l_tot = 0.f, m = -INFINITY;
+#pragma unroll
+  for (int j = 0; j < kWaves; ++j) {
+    w[j] = refs[j * 64 + col];
+    m = fmaxf(m, w[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < kWaves; ++j) {
+    w[j] = m > -INFINITY ? __builtin_amdgcn_exp2f(w[j] - m) : 0.f;
+    l_tot = __builtin_fmaf(refs[j * 64 + 32 + col], w[j], l_tot);
+  }
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  uint8_t* const rows = lds + R::kOffRows;
+#pragma unroll
+  for (int k = 0; k < R::kGroups / kWaves; ++k) {
+    const int g = wave * (R::kGroups / kWaves) + k;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < kWaves; ++j) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(lds + j * T::kBytesV + g * 1024 + lane * 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] = __builtin_fmaf(x[e], w[j], sum[e]);
+    }
+    f32x2 lo, hi;
+    lo.x = sum[0] * inv; lo.y = sum[1] * inv;
+    hi.x = sum[2] * inv; hi.y = sum[3] * inv;
+    const ex2 l2 = __builtin_convertvector(lo, ex2);
+    const ex2 h2 = __builtin_convertvector(hi, ex2);
+    ex4 pk;
+    pk.x = l2.x; pk.y = l2.y; pk.z = h2.x; pk.w = h2.y;
+    *reinterpret_cast<ex4*>(rows + col * T::kRowBytes + ((g ^ T::swz_k(col)) << 4) + 8 * hh) = pk;
+  }
+  if (wave == 0 && hh == 0 && q0 + col < view.q_end) {
+    // log(2^m * sum), the sum by its exponent and mantissa: what the logarithm's last bits are worth does not grow with the number of keys
+    constexpr float kLn2 = 0.6931471805599453f;
+    const float fraction = __builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(l_tot)) * kLn2;
+    const float log_sum = __builtin_fmaf((float)__builtin_amdgcn_frexp_expf(l_tot), kLn2, __builtin_fmaf(m, kLn2, fraction));
+    const float lse = l_tot > 0.f ? log_sum : -INFINITY;
+    float* dst = view.lse + ((int64_t)b * a.H + h) * a.Sq + q0 + col;
+    if constexpr (kMerge) store_device(dst, lse);
+    else *dst = lse;
+  }
+  phase_barrier();
+  const int row = tid / T::kChunks, cc = tid % T::kChunks;
+  if (row < 32 && q0 + row < view.q_end) {
+    const u32x4 val = *reinterpret_cast<const u32x4*>(rows + row * T::kRowBytes + ((cc ^ T::swz_k(row)) << 4));
+    uint16_t* const out0 = view.out + (((int64_t)b * a.Sq + q0) * a.H + h) * D;
+    const uint32_t row_elems = (uint32_t)a.H * D;
+    if constexpr (kMerge)
+      __builtin_amdgcn_raw_buffer_store_b128(val, buffer_of(out0, 64u * row_elems), 2u * row * row_elems + 16u * cc, 0, kDeviceNt);
+    else __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(out0 + (int64_t)row * row_elems + 8 * cc));
+  }
+}
+
+// The attention kernel of a launch of few query rows (see short_rows): a workgroup for every 32 rows of a job.
+template <int D, bool kPre, bool kHalf, bool kMerge>
+__global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn_fwd_kernel(const AttnRows args_by_value) {
+  static_assert(!kPre, "built for queries that the kernel scales");
+  using R = Rows32<D>;
+  (void)args_by_value;
+  prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
+  KernArgs& a = kernel_args();
+  // the slices of 32 rows of all (batch, head): part_ways a head, tail_items an XCD
+  const int at = (int)(blockIdx.x & (kXcds - 1)) * a.tail_items + (int)(blockIdx.x >> 3);
+  const int bh = at / a.part_ways;
+  const int slice = at - bh * a.part_ways;
+  const int b = bh / a.H;
+  const int h = bh - b * a.H;
+  if (b >= a.B) return;
+  const int row0 = 32 * slice;
+  JobView view;
+  const bool there = view_job(a, blockIdx.y, view);
+  const int rows = there ? view.q_end - view.q_begin - row0 : 0;
+  if (rows > 0) attn_rows32<D, kHalf, kMerge>(view, b, h, row0);
+  if constexpr (kMerge) {
+    KernArgs& m = kernel_args();
+    if (row0 >= m.Sq) return;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int* const flag = reinterpret_cast<int*>(lds + R::kOffFlag);
+    wait_tile_loads<0>();   // this wavefront's stores
+    phase_barrier();        // everybody's
+    if (wave == 0) {
+      const bool last = arrive_last(m.arrive + kPartCounters + (int64_t)bh * m.nqt * kWaves + slice, m.merge_jobs);
+      if ((threadIdx.x & 63) == 0) *flag = last;
+    }
+    phase_barrier();
+    if (!__builtin_amdgcn_readfirstlane(*flag)) return;
+    constexpr int kMine = 64 / Tile<D>::kChunks;   // rows of a wavefront: those of one load
+    const int first = row0 + kMine * wave;
+    if (kMine * wave >= 32 || first >= m.Sq) return;
+    uint8_t* const stage = lds + wave * Tile<D>::kBytesV;
+    merge_rows<D, kHalf, kRowsStates, true, kMine>(stage, b, h, first);
+  }
+}
+
 // Folds the part_ways partial states of every split item into the item's rows of its destination.  A workgroup takes 64
 // columns of the 32 query rows of one wavefront of the item's workgroup: its four wavefronts share the 4-element groups
 // of a row, lane L of a group holds query L % 32 as in the attention kernel, and the rows go through the LDS so that
@@ -1589,30 +1907,34 @@ __global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const Attn
 static_assert(Tile<128>::kLdsBytes == kAttnLdsBytes128 && Tile<64>::kLdsBytes == kAttnLdsBytes64,
               "dt_common.h states the LDS footprint of the attention kernel");
 
-template <int D, bool kPre, bool kHalf, bool kMerge>
-static int launch_one(const AttnArgs& a, dim3 grid, hipStream_t stream) {
+// Args: AttnArgs or AttnRows, which names the kernel.
+template <int D, bool kPre, bool kHalf, bool kMerge, typename Args>
+static int launch_one(const Args& a, dim3 grid, hipStream_t stream) {
+  constexpr int kLdsBytes = std::is_same_v<Args, AttnRows> ? Rows32<D>::kLdsBytes : Tile<D>::kLdsBytes;
+  void (*const kernel)(const Args) = attn_fwd_kernel<D, kPre, kHalf, kMerge>;
   // more than 64 KB of dynamic LDS has to be allowed once per kernel and device
   static thread_local int allowed_dev = -1;
   int dev = 0;
   if (int rc = hip_fail(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (allowed_dev != dev) {
-    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_fwd_kernel<D, kPre, kHalf, kMerge>),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, Tile<D>::kLdsBytes),
+    if (int rc = hip_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes),
                           "hipFuncSetAttribute"))
       return rc;
     allowed_dev = dev;
   }
-  hipLaunchKernelGGL((attn_fwd_kernel<D, kPre, kHalf, kMerge>), grid, dim3(kThreads), Tile<D>::kLdsBytes, stream, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(kThreads), kLdsBytes, stream, a);
   return hip_fail(hipGetLastError(), "attn_fwd launch");
 }
 
-static int launch_dim(const AttnArgs& a, int D, dim3 grid, hipStream_t stream) {
+template <typename Args>
+static int launch_dim(const Args& a, int D, dim3 grid, hipStream_t stream) {
   if (a.arrive) {
     if (a.elem_f16) return D == 128 ? launch_one<128, false, true, true>(a, grid, stream) : launch_one<64, false, true, true>(a, grid, stream);
     return D == 128 ? launch_one<128, false, false, true>(a, grid, stream) : launch_one<64, false, false, true>(a, grid, stream);
   }
   if (a.elem_f16) return D == 128 ? launch_one<128, false, true, false>(a, grid, stream) : launch_one<64, false, true, false>(a, grid, stream);
-  if (a.q_prescaled) return D == 128 ? launch_one<128, true, false, false>(a, grid, stream) : launch_one<64, true, false, false>(a, grid, stream);
+  if constexpr (!std::is_same_v<Args, AttnRows>)
+    if (a.q_prescaled) return D == 128 ? launch_one<128, true, false, false>(a, grid, stream) : launch_one<64, true, false, false>(a, grid, stream);
   return D == 128 ? launch_one<128, false, false, false>(a, grid, stream) : launch_one<64, false, false, false>(a, grid, stream);
 }
 
@@ -1869,10 +2191,38 @@ std::mutex& workspace_lock(const void* workspace) {
   return locks[(reinterpret_cast<uintptr_t>(workspace) >> 4) * 0x9e3779b97f4a7c15ull >> (64 - kBits)];
 }
 
+// Whether a launch runs as workgroups of 32 query rows (see attn_rows32): the slices of a head, or 0.
+// Like the other ways to split, for launches with a workspace (without one the items stay whole), though it needs none.
+// The workgroups have to be resident together -- two workgroups a CU at D = 64, one at D = 128 -- and an item no longer than 32 key
+// tiles.  us per call, other form -> this, by workgroups of one job and key tiles:
+//   * D = 64, 512: 1 tile 14.0 -> 8.9, 8 15.6 -> 12.4, 32 27.3 -> 26.2, 48 31.3 -> 31.3; 640: 1 tile 14.2 -> 13.9, 8 16.2 -> 19.1;
+//     256: 32 tiles 24.0 -> 17.8, 48 24.6 -> 21.6, 96 (16 parts) 30.9 -> 33.2; 16: 8 14.1 -> 8.5, 32 21.0 -> 15.0, 48 20.4 -> 18.7, 96 21.7 -> 27.7;
+//   * D = 128, 256: 1 tile 13.5 -> 11.4, 8 18.9 -> 14.9, 32 28.9 -> 24.4, 48 32.9 -> 30.6; 320: 1 tile 13.8 -> 16.0, 8 19.5 -> 23.0;
+//     128: 8 18.1 -> 13.5, 32 25.0 -> 23.8, 48 27.6 -> 29.8; 16: 8 17.2 -> 12.4, 32 22.4 -> 20.5, 48 22.5 -> 25.6.
+static int short_rows(const AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus) {
+  const int rows_most = std::min(a.nqt * kBQ, a.Sq);
+  int rows = 0, tiles = 0;
+  for (int j = 0; j < n_jobs; ++j) {
+    rows = std::max(rows, a.cu_q ? rows_most : size[j].rows);
+    tiles = std::max(tiles, size[j].tiles);
+  }
+  const int slices = (rows + 31) / 32;
+  const int64_t per_xcd = ((int64_t)a.B * a.H * slices + kXcds - 1) / kXcds;
+  constexpr int kMostTiles = 32;
+  return a.q_prescaled || per_xcd * n_jobs > (D == 64 ? 2 : 1) * cus || tiles > kMostTiles ? 0 : slices;
+}
+
 // The launch as it is planned (and the fold kernel behind it).
-static int launch_planned(AttnArgs& a, int D, int n_jobs, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
+static int launch_planned(AttnArgs& a, int D, int n_jobs, int slices, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
   const int64_t slot_bytes = partial_state_bytes(D);
   const unsigned planes_x = (unsigned)a.per_xcd * kXcds;
+  if (slices > 0) {
+    AttnRows r;
+    static_cast<AttnArgs&>(r) = a;
+    r.part_ways = slices;
+    r.tail_items = (int)(((int64_t)a.B * a.H * slices + kXcds - 1) / kXcds);
+    return launch_dim(r, D, dim3((unsigned)r.tail_items * kXcds, (unsigned)n_jobs, 1), stream);
+  }
   if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);
   const int64_t slots = (int64_t)a.tail_items * kXcds * a.part_ways;
   if (a.arrive && !a.row_split && (int64_t)a.tail_items * kXcds * kWaves > kPartCounters) {
@@ -1940,6 +2290,7 @@ static bool long_launch_merges(int D, int n_jobs, int per_xcd, int tiles, int cu
 //     160 and 2 (8 x 147, 2 tiles 1.16, 20 x 156, one 1.11; 3 tiles are even: 12 x 142 1.01, 24 x 156 0.95); 48 x 119, 18 items 0.95, 24 x
 //     103, 7 tiles 0.94, 12 x 200, 4 tiles 18.4 -> 20.8 [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94.  With the host's
 //     list up to 24 items of 4 key tiles (48 x 254, 24 items 32.1 -> 29.8 [20.8 -> 25.0]; 48 x 400, 48 items 32.3 -> 36.4);
+//   * (measured with workgroups of 256 rows; those of 32 follow the same rule, a merge of 4 or 8 rows a wavefront being shorter);
 //   * up to 4 states: 8 are twice the loads of the chain (D = 64 24 x 269 17.0 -> 21.7, D = 128 20 x 200 19 -> 25);
 //   * items in up to two parts: three and more are folded one after the other (3 x 1706, D = 64, 4 parts 0.91).
 static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles, int cus) {
@@ -1998,12 +2349,14 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   a.row_split = 0;
   constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
   bool merge_after = false;
+  int slices = 0;   // of 32 rows, where workgroups take one each
   if (n_jobs <= kMaxLaunchJobs) {
     JobSize size[kMaxLaunchJobs];
     job_sizes(a, n_jobs, size);
     const int cus = xcd_cus();
-    const TailPlan plan = plan_launch(a, D, n_jobs, size, cus,
-                                      cus > 0 && workspace ? std::min(workspace_bytes, kWorkspaceBytes) / partial_state_bytes(D) : -1);
+    const bool split = cus > 0 && workspace;
+    if (split) slices = short_rows(a, D, n_jobs, size, cus);
+    const TailPlan plan = plan_launch(a, D, n_jobs, size, cus, split ? std::min(workspace_bytes, kWorkspaceBytes) / partial_state_bytes(D) : -1);
     a.tail_items = plan.items;
     a.part_ways = plan.ways;
     a.row_split = plan.rows ? 1 : 0;
@@ -2011,12 +2364,12 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
     if (a.arrive) {
       int longest = 0;
       for (int j = 0; j < n_jobs; ++j) longest = std::max(longest, size[j].tiles);
-      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan);
+      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan) || (slices > 0 && a.merge_n > kRowsStates);
     }
   }
-  if (!merge_after) return launch_planned(a, D, n_jobs, stream, workspace, workspace_bytes);
+  if (!merge_after) return launch_planned(a, D, n_jobs, slices, stream, workspace, workspace_bytes);
   a.arrive = nullptr;
-  if (int rc = launch_planned(a, D, n_jobs, stream, workspace, workspace_bytes)) return rc;
+  if (int rc = launch_planned(a, D, n_jobs, slices, stream, workspace, workspace_bytes)) return rc;
   return merge_behind(a, D, stream);
 }
 
