@@ -322,6 +322,23 @@ def _stream_counters(dev: torch.device, need: int) -> Optional[torch.Tensor]:
     return c
 
 
+def attn_scratch(dev: torch.device):
+    """``attn_workspace``, and the counters that the current stream keeps (``None``: it has none yet, or is being captured) for a caller
+    that may merge: one look at the stream for both."""
+    if torch.cuda.is_current_stream_capturing():
+        return attn_workspace(dev), None
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    key = (dev.type, index, _raw_stream(index))
+    ws = _workspaces.pop(key, None)
+    if ws is None:
+        return attn_workspace(dev), None
+    _workspaces[key] = ws
+    c = _counters.pop(key, None)
+    if c is not None:
+        _counters[key] = c
+    return ws, c
+
+
 def release_workspaces() -> None:
     """Drop every attention workspace (they are re-created on demand)."""
     _workspaces.clear()
@@ -355,6 +372,11 @@ class ChunkTable:
     v_ptrs = property(lambda self: self.whole()[1])
     lens = property(lambda self: self.whole()[2])
     sb = property(lambda self: self.whole()[3])
+
+
+def native_table(k_chunks: list, v_chunks: list, batch: int = 0, convert=None):
+    """What ``ChunkTable(...).native`` is, for a caller that has lists and needs no more of the table."""
+    return _host().ChunkTable(k_chunks, v_chunks, batch, convert)
 
 
 class DeviceSegments:
@@ -427,13 +449,16 @@ def attn_states_merge(q: torch.Tensor, k_chunks: Sequence[torch.Tensor], v_chunk
                                      lambda need: _stream_counters(q.device, need), _stream())
 
 
-def attn_sched_merge(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor, max_jobs: int,
+def attn_sched_merge(q: torch.Tensor, table, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor, max_jobs: int,
                      slot_out: torch.Tensor, slot_lse: torch.Tensor, diag: int, diag_out: torch.Tensor, diag_lse: torch.Tensor,
-                     dst_dtype: torch.dtype, workspace: Optional[torch.Tensor] = None, q_prescaled: bool = False, row: int = 0):
-    """``attn_sched_fwd`` on whole queries and ``merge_arena``, in the same launch where it can.  Returns (out, lse)."""
-    return _host().attn_sched_merge(q, table.native, dev_compute_ids, dev_count, row, max_jobs, slot_out, slot_lse, diag, diag_out,
+                     dst_dtype: torch.dtype, workspace: Optional[torch.Tensor] = None, q_prescaled: bool = False, row: int = 0,
+                     counters: Optional[torch.Tensor] = None):
+    """``attn_sched_fwd`` on whole queries and ``merge_arena``, in the same launch where it can.  ``table`` is a ``ChunkTable`` or a
+    ``native_table``; ``counters`` those that ``attn_scratch`` found for this stream.  Returns (out, lse)."""
+    return _host().attn_sched_merge(q, table.native if type(table) is ChunkTable else table, dev_compute_ids, dev_count, row, max_jobs, slot_out, slot_lse, diag, diag_out,
                                     diag_lse, dst_dtype, workspace,
-                                    lambda need: _stream_counters(q.device, need), _attn_flags(q, q_prescaled), _stream())
+                                    (lambda need: _stream_counters(q.device, need)) if counters is None else counters,
+                                    _attn_flags(q, q_prescaled), _stream())
 
 
 def attn_sched_fwd(q: torch.Tensor, table: ChunkTable, dev_compute_ids: torch.Tensor, dev_count: torch.Tensor,

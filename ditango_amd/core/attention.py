@@ -39,6 +39,7 @@ from ..timer import get_timer
 from ..utils import get_timestep
 from .cache import proCache
 from .config import get_config
+from .parallel_state import LocalRingGroup
 from .redundancy_map import get_redundancy_map
 
 logger = init_logger(__name__)
@@ -419,15 +420,21 @@ class proAttention:
         row = rm.mask_rows[t][l]
         C = len(row)
         local = self.local_chunk_id if (self.local_chunk_id == diag and key is not None) else -1
-        kv = [(key, value) if c == local else self.group.kv_chunk(c) for c in range(C)]
-        ks, vs = [k for k, _ in kv], [v for _, v in kv]
+        if type(self.group) is LocalRingGroup:
+            ks, vs = self.group.kv_lists(C, local, key, value)
+        else:
+            kv = [(key, value) if c == local else self.group.kv_chunk(c) for c in range(C)]
+            ks, vs = [k for k, _ in kv], [v for _, v in kv]
         if not cache.ensure_arena(C, B, Sq, H, D, query.device, query.dtype):
             out = self._attn_uncached(query, [_as4d(k, B) for k in ks], [_as4d(v, B) for v in vs])
             rm.record_out_redundancy(timestep=t, layer_id=l, curr_out=out)
             return out
         valid = cache.arena_valid
-        for c in range(C):
-            if row[c] != 0 and c != diag and not valid[c]:
+        stored = []
+        for c, reuse in enumerate(row):
+            if reuse == 0:
+                stored.append(c)
+            elif not valid[c] and c != diag:
                 raise RuntimeError(f"T{t}L{l}: mask asks to reuse chunk {c} but no state was ever stored for it")
         seg_q = seg_kv = dev_seg = None
         if self._segments is not None:
@@ -439,13 +446,13 @@ class proAttention:
                 seg_q = [(cu_q[i], cu_q[i + 1] - cu_q[i]) for i in range(len(cu_q) - 1)]
                 seg_kv = [[(cu_kv_of(c)[i], cu_kv_of(c)[i + 1] - cu_kv_of(c)[i]) for i in range(len(cu_q) - 1)]
                           for c in range(C)]
-        ws = _hip.attn_workspace(query.device)
+        ws, counters = _hip.attn_scratch(query.device)
         out = None
         if not rm.sched_windows and self._segments is None:
-            out, lse = _hip.attn_sched_merge(query, _hip.ChunkTable(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
+            out, lse = _hip.attn_sched_merge(query, _hip.native_table(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
                                              rm.compute_counts[t][l], cache.arena_out, cache.arena_lse, diag, cache.diag_out,
                                              cache.diag_lse, self.out_dtype, ws, self.q_prescaled,
-                                             (t % rm.num_timesteps) * rm.num_layers + l % rm.num_layers)
+                                             (t % rm.num_timesteps) * rm.num_layers + l % rm.num_layers, counters)
         elif not rm.sched_windows:
             _hip.attn_sched_fwd(query, _hip.ChunkTable(ks, vs, B, _kernel_input), rm.sched_compute_ids, rm.sched_counts,
                                 rm.compute_counts[t][l], cache.arena_out, cache.arena_lse, diag, cache.diag_out,
@@ -475,8 +482,8 @@ class proAttention:
                                     cache.diag_lse, seg_q=seg_q, seg_kv=None if seg_kv is None else seg_kv[w0:w1],
                                     workspace=ws, q_prescaled=self.q_prescaled,
                                     dev_segments=None if dev_seg is None else dev_seg.window(w0, w1))
-        for c in range(C):
-            if row[c] == 0 and c != diag:
+        for c in stored:
+            if c != diag:
                 valid[c] = True
         if out is None:
             out, lse = _hip.merge_arena(cache.arena_out, cache.arena_lse, diag, cache.diag_out, cache.diag_lse, self.out_dtype)

@@ -204,7 +204,7 @@ class proCache:
         (cache.py:103-128) -- and a layer without arena recomputes every chunk on every call, which is
         what the reference's guard falls back to (core/attention.py:97-98: stride forced to N)."""
         shape = (n_chunks, B, Sq, H, D)
-        if (self.arena_out is not None and tuple(self.arena_out.shape) == shape and self.arena_out.device == device
+        if (self.arena_out is not None and self.arena_out.shape == shape and self.arena_out.device == device
                 and self.arena_out.dtype == dtype):
             return True
         if self.arena_refused == shape:

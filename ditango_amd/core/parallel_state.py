@@ -58,6 +58,21 @@ class LocalRingGroup:
             raise RuntimeError(f"KV chunk {chunk_id} was not provided to the ring group (set_kv_chunks)")
         return k, v
 
+    def kv_lists(self, n: int, local: int, key, value) -> Tuple[list, list]:
+        """K and V of chunks 0 ... n - 1 as two lists, chunk ``local`` (-1: none) being ``(key, value)``: what ``kv_chunk`` gives one
+        by one.  With every chunk in place that is two copied lists; whatever ``kv_chunk`` would raise, it raises."""
+        if n == len(self._k) and "kv_chunk" not in self.__dict__:
+            ks, vs = self._k.copy(), self._v.copy()
+            if local >= 0:
+                ks[local], vs[local] = key, value
+            for k, v in zip(ks, vs):
+                if k is None or v is None:
+                    break
+            else:
+                return ks, vs
+        kv = [(key, value) if c == local else self.kv_chunk(c) for c in range(n)]
+        return [k for k, _ in kv], [v for _, v in kv]
+
     def _no_p2p(self, *a, **kw):
         raise NotImplementedError(
             "on one GPU the K/V exchange of the ring is a chunk lookup (LocalRingGroup.kv_chunk); "

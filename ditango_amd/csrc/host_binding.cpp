@@ -330,7 +330,7 @@ std::pair<Tensor, Tensor> merge(const std::vector<Tensor>& outs, const std::vect
 
 // The counters of a launch that merges n_states states into one of dst_dtype (see dt_merge_result); none where it cannot, or where its
 // sizes are better served by the merge kernel behind it.  Only a launch that merges asks for them, with counters(how many): host work, and
-// memory of the stream's.
+// memory of the stream's.  `counters` may be the stream's set itself.
 std::optional<Tensor> merge_counters(const Tensor& q, const Dims& d, at::ScalarType dst_dtype, int32_t flags, int64_t n_jobs,
                                      bool host_listed, int64_t key_tiles, int64_t n_states, const py::object& counters) {
   if (counters.is_none() || (flags & DT_ATTN_Q_PRESCALED) || (dst_dtype != at::kFloat && dst_dtype != q.scalar_type()) ||
@@ -338,7 +338,10 @@ std::optional<Tensor> merge_counters(const Tensor& q, const Dims& d, at::ScalarT
     return std::nullopt;
   const int need = dt_attn_merges_in_launch(d.B, d.S, d.H, d.D, n_jobs, host_listed, key_tiles, n_states);
   if (need == 0) return std::nullopt;
-  auto c = py::cast<std::optional<Tensor>>(counters(need));
+  // (a set that is kept already, or who is asked for one; a set too small for this launch: as if there were none)
+  const bool kept = !PyCallable_Check(counters.ptr());
+  auto c = py::cast<std::optional<Tensor>>(kept ? counters : counters(need));
+  if (kept && c->numel() < need) return std::nullopt;
   REQUIRE(!c || (c->is_cuda() && c->scalar_type() == at::kInt && c->is_contiguous()), "counters must be int32 on the GPU");
   return c;   // (their number is checked with the launch)
 }
