@@ -1484,32 +1484,35 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
 // barriers (0.7 us a tile where nothing else runs: 4 heads x 512 queries, D = 64), result, merge.  Here a workgroup has 32
 // queries instead of 256, and its eight wavefronts share the KEYS: wavefront w takes the tiles w, w + 8 ..., by itself, from
 // registers and LDS of its own, with no barrier; their states meet once, in fp32 through the LDS.  A chunk of 512 keys is one
-// tile deep.  The keys and values are read by eight times as many workgroups: 110 GB/s a CU out of the L2 is what longer
-// ones are bound by, and why short_rows ends at 32 tiles.
+// tile deep.  Four wavefronts do the same where there are more slices than CUs, or fewer tiles than wavefronts.  The keys and values
+// are read by eight times as many workgroups: 110 GB/s a CU out of the L2 is what long items are bound by, and why short_rows
+// ends at 32 tiles.
 // us per call, workgroups of 256 (128) queries -> this: D = 64 4 heads x 512 queries, 2 of 4 chunks 15.1 -> 9.2, 8 x 1024, 1 of 4 18.9 ->
 // 10.9, 16 x 300, 2 of 4 17.8 -> 10.3, 16 x 64 10.4 -> 7.1; D = 128 4 x 512 17.7 -> 13.5, 4 x 128 14.7 -> 8.8, 24 x 128 15.3 -> 9.9,
 // 8 x 1024 24.1 -> 18.7.
 // K and V of a tile take the same 8 (16) KB of LDS in turn.  K read from memory as fragments, beside V, was 1.2 ... 4 us longer at
 // the sizes above: an instruction then touches 32 lines for 32 bytes each, and what the L1 holds of them is gone before the
 // next one asks for the rest of the line.
-struct AttnRows : AttnArgs {};   // (names the kernel; part_ways: slices of 32 rows of a head, tail_items: slices of an XCD)
+// (They name the kernel, by its wavefronts; part_ways: slices of 32 rows of a head, tail_items: slices of an XCD.)
+struct AttnRows8 : AttnArgs {};
+struct AttnRows4 : AttnArgs {};
 constexpr int kRowsStates = 4;    // states that such a launch merges itself, at most (short_launch_merges allows no more)
 // LDS: the tile of each wavefront (afterwards its share of the state), references and sums, 32 result rows.
-template <int D>
+template <int D, int W>
 struct Rows32 {
-  static constexpr int kOffRef = kWaves * Tile<D>::kBytesV;           // [8 wavefronts][reference, sum][32 queries]
-  static constexpr int kOffRows = kOffRef + kWaves * 2 * 32 * 4;
+  static constexpr int kOffRef = W * Tile<D>::kBytesV;                // [wavefront][reference, sum][32 queries]
+  static constexpr int kOffRows = kOffRef + W * 2 * 32 * 4;
   static constexpr int kOffFlag = kOffRows + 32 * Tile<D>::kRowBytes;
   static constexpr int kLdsBytes = kOffFlag + 16;
   static constexpr int kGroups = D / 8;                               // 4-element groups of a lane's accumulators
   static_assert(kGroups * 1024 == Tile<D>::kBytesV, "a wavefront's accumulators take the place of its V tile");
 };
 
-// 32 queries of one job, batch and head: wavefront w works on the key tiles w, w + 8 ... on its own.
-template <int D, bool kHalf, bool kMerge>
+// 32 queries of one job, batch and head: of W wavefronts, w works on the key tiles w, w + W ... on its own.
+template <int D, bool kHalf, bool kMerge, int W>
 __device__ __forceinline__ void attn_rows32(const JobView& view, int b, int h, int row0) {
   using T = Tile<D>;
-  using R = Rows32<D>;
+  using R = Rows32<D, W>;
   using E = Elem<kHalf>;
   typedef typename E::x8 ex8;
   typedef typename E::x4 ex4;
@@ -1622,7 +1625,7 @@ __device__ __forceinline__ void attn_rows32(const JobView& view, int b, int h, i
 #pragma unroll
       for (int s = 0; s < D / 16; ++s) s_acc[kb] = E::mfma(kf[kb][s], qf[s], s_acc[kb]);
     }
-    tile += kWaves;
+    tile += W;
     more = seek();
     if (lim < kBK) {
 #pragma unroll
@@ -1684,7 +1687,7 @@ __device__ __forceinline__ void attn_rows32(const JobView& view, int b, int h, i
     if (more) load_k();
   }
 
-  // ---- the eight states meet in the LDS: every wavefront adds up an eighth of the columns
+  // ---- the states meet in the LDS: every wavefront adds up its share of the columns
   float* const refs = reinterpret_cast<float*>(lds + R::kOffRef);
   l_run += __shfl_xor(l_run, 32);
   if (hh == 0) {
@@ -1698,25 +1701,25 @@ __device__ __forceinline__ void attn_rows32(const JobView& view, int b, int h, i
       *reinterpret_cast<f32x4*>(v_tile + (4 * i + g) * 1024 + lane * 16) =
           f32x4{o_acc[i][4 * g], o_acc[i][4 * g + 1], o_acc[i][4 * g + 2], o_acc[i][4 * g + 3]};
   phase_barrier();
-  float w[kWaves], l_tot = 0.f, m = -INFINITY;
+  float w[W], l_tot = 0.f, m = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < kWaves; ++j) {
+  for (int j = 0; j < W; ++j) {
     w[j] = refs[j * 64 + col];
     m = fmaxf(m, w[j]);
   }
 #pragma unroll
-  for (int j = 0; j < kWaves; ++j) {
+  for (int j = 0; j < W; ++j) {
     w[j] = m > -INFINITY ? __builtin_amdgcn_exp2f(w[j] - m) : 0.f;
     l_tot = __builtin_fmaf(refs[j * 64 + 32 + col], w[j], l_tot);
   }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   uint8_t* const rows = lds + R::kOffRows;
 #pragma unroll
-  for (int k = 0; k < R::kGroups / kWaves; ++k) {
-    const int g = wave * (R::kGroups / kWaves) + k;
+  for (int k = 0; k < R::kGroups / W; ++k) {
+    const int g = wave * (R::kGroups / W) + k;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < kWaves; ++j) {
+    for (int j = 0; j < W; ++j) {
       const f32x4 x = *reinterpret_cast<const f32x4*>(lds + j * T::kBytesV + g * 1024 + lane * 16);
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum[e] = __builtin_fmaf(x[e], w[j], sum[e]);
@@ -1741,23 +1744,24 @@ __device__ __forceinline__ void attn_rows32(const JobView& view, int b, int h, i
     else *dst = lse;
   }
   phase_barrier();
-  const int row = tid / T::kChunks, cc = tid % T::kChunks;
-  if (row < 32 && q0 + row < view.q_end) {
+  constexpr int kRowsPerPass = 64 * W / T::kChunks;
+  uint16_t* const out0 = view.out + (((int64_t)b * a.Sq + q0) * a.H + h) * D;
+  const uint32_t row_elems = (uint32_t)a.H * D;
+#pragma unroll
+  for (int pass = 0; pass < 32; pass += kRowsPerPass) {
+    const int row = pass + tid / T::kChunks, cc = tid % T::kChunks;
+    if (row >= 32 || q0 + row >= view.q_end) break;
     const u32x4 val = *reinterpret_cast<const u32x4*>(rows + row * T::kRowBytes + ((cc ^ T::swz_k(row)) << 4));
-    uint16_t* const out0 = view.out + (((int64_t)b * a.Sq + q0) * a.H + h) * D;
-    const uint32_t row_elems = (uint32_t)a.H * D;
     if constexpr (kMerge)
       __builtin_amdgcn_raw_buffer_store_b128(val, buffer_of(out0, 64u * row_elems), 2u * row * row_elems + 16u * cc, 0, kDeviceNt);
     else __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(out0 + (int64_t)row * row_elems + 8 * cc));
   }
 }
 
-// The attention kernel of a launch of few query rows (see short_rows): a workgroup for every 32 rows of a job.
-template <int D, bool kPre, bool kHalf, bool kMerge>
-__global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn_fwd_kernel(const AttnRows args_by_value) {
-  static_assert(!kPre, "built for queries that the kernel scales");
-  using R = Rows32<D>;
-  (void)args_by_value;
+// A launch of few query rows (see short_rows): a workgroup of W wavefronts for every 32 rows of a job.
+template <int D, bool kHalf, bool kMerge, int W>
+__device__ __forceinline__ void attn_rows32_kernel() {
+  using R = Rows32<D, W>;
   prefetch_args((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
   KernArgs& a = kernel_args();
   // the slices of 32 rows of all (batch, head): part_ways a head, tail_items an XCD
@@ -1771,7 +1775,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
   JobView view;
   const bool there = view_job(a, blockIdx.y, view);
   const int rows = there ? view.q_end - view.q_begin - row0 : 0;
-  if (rows > 0) attn_rows32<D, kHalf, kMerge>(view, b, h, row0);
+  if (rows > 0) attn_rows32<D, kHalf, kMerge, W>(view, b, h, row0);
   if constexpr (kMerge) {
     KernArgs& m = kernel_args();
     if (row0 >= m.Sq) return;
@@ -1786,12 +1790,22 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
     }
     phase_barrier();
     if (!__builtin_amdgcn_readfirstlane(*flag)) return;
-    constexpr int kMine = 64 / Tile<D>::kChunks;   // rows of a wavefront: those of one load
+    constexpr int kOfLoad = 64 / Tile<D>::kChunks, kMine = kOfLoad * W < 32 ? 32 / W : kOfLoad;   // rows of a wavefront
     const int first = row0 + kMine * wave;
     if (kMine * wave >= 32 || first >= m.Sq) return;
     uint8_t* const stage = lds + wave * Tile<D>::kBytesV;
     merge_rows<D, kHalf, kRowsStates, true, kMine>(stage, b, h, first);
   }
+}
+template <int D, bool kPre, bool kHalf, bool kMerge>
+__global__ __launch_bounds__(512, D == 64 ? 4 : 2) void attn_fwd_kernel(const AttnRows8 args_by_value) {
+  (void)args_by_value;
+  attn_rows32_kernel<D, kHalf, kMerge, 8>();
+}
+template <int D, bool kPre, bool kHalf, bool kMerge>
+__global__ __launch_bounds__(256, D == 64 ? 4 : 2) void attn_fwd_kernel(const AttnRows4 args_by_value) {
+  (void)args_by_value;
+  attn_rows32_kernel<D, kHalf, kMerge, 4>();
 }
 
 // Folds the part_ways partial states of every split item into the item's rows of its destination.  A workgroup takes 64
@@ -1907,10 +1921,12 @@ __global__ __launch_bounds__(kFoldThreads) void attn_tail_fold_kernel(const Attn
 static_assert(Tile<128>::kLdsBytes == kAttnLdsBytes128 && Tile<64>::kLdsBytes == kAttnLdsBytes64,
               "dt_common.h states the LDS footprint of the attention kernel");
 
-// Args: AttnArgs or AttnRows, which names the kernel.
+// Args: AttnArgs, or what names another form of the kernel.
 template <int D, bool kPre, bool kHalf, bool kMerge, typename Args>
 static int launch_one(const Args& a, dim3 grid, hipStream_t stream) {
-  constexpr int kLdsBytes = std::is_same_v<Args, AttnRows> ? Rows32<D>::kLdsBytes : Tile<D>::kLdsBytes;
+  constexpr int kLdsBytes = std::is_same_v<Args, AttnRows8> ? Rows32<D, 8>::kLdsBytes
+                            : std::is_same_v<Args, AttnRows4> ? Rows32<D, 4>::kLdsBytes : Tile<D>::kLdsBytes;
+  constexpr int kThreadsOf = std::is_same_v<Args, AttnRows4> ? 256 : kThreads;
   void (*const kernel)(const Args) = attn_fwd_kernel<D, kPre, kHalf, kMerge>;
   // more than 64 KB of dynamic LDS has to be allowed once per kernel and device
   static thread_local int allowed_dev = -1;
@@ -1922,7 +1938,7 @@ static int launch_one(const Args& a, dim3 grid, hipStream_t stream) {
       return rc;
     allowed_dev = dev;
   }
-  hipLaunchKernelGGL(kernel, grid, dim3(kThreads), kLdsBytes, stream, a);
+  hipLaunchKernelGGL(kernel, grid, dim3(kThreadsOf), kLdsBytes, stream, a);
   return hip_fail(hipGetLastError(), "attn_fwd launch");
 }
 
@@ -1933,7 +1949,7 @@ static int launch_dim(const Args& a, int D, dim3 grid, hipStream_t stream) {
     return D == 128 ? launch_one<128, false, false, true>(a, grid, stream) : launch_one<64, false, false, true>(a, grid, stream);
   }
   if (a.elem_f16) return D == 128 ? launch_one<128, false, true, false>(a, grid, stream) : launch_one<64, false, true, false>(a, grid, stream);
-  if constexpr (!std::is_same_v<Args, AttnRows>)
+  if constexpr (std::is_same_v<Args, AttnArgs>)
     if (a.q_prescaled) return D == 128 ? launch_one<128, true, false, false>(a, grid, stream) : launch_one<64, true, false, false>(a, grid, stream);
   return D == 128 ? launch_one<128, false, false, false>(a, grid, stream) : launch_one<64, false, false, false>(a, grid, stream);
 }
@@ -2191,37 +2207,49 @@ std::mutex& workspace_lock(const void* workspace) {
   return locks[(reinterpret_cast<uintptr_t>(workspace) >> 4) * 0x9e3779b97f4a7c15ull >> (64 - kBits)];
 }
 
-// Whether a launch runs as workgroups of 32 query rows (see attn_rows32): the slices of a head, or 0.
+// How a launch runs as workgroups of 32 query rows (see attn_rows32): wavefronts of one (0: it does not), slices of 32 rows of a head,
+// slices of an XCD.
+struct ShortRows {
+  int waves = 0, slices = 0;
+  int64_t per_xcd = 0;
+};
 // Like the other ways to split, for launches with a workspace (without one the items stay whole), though it needs none.
-// The workgroups have to be resident together -- two workgroups a CU at D = 64, one at D = 128 -- and an item no longer than 32 key
-// tiles.  us per call, other form -> this, by workgroups of one job and key tiles:
-//   * D = 64, 512: 1 tile 14.0 -> 8.9, 8 15.6 -> 12.4, 32 27.3 -> 26.2, 48 31.3 -> 31.3; 640: 1 tile 14.2 -> 13.9, 8 16.2 -> 19.1;
-//     256: 32 tiles 24.0 -> 17.8, 48 24.6 -> 21.6, 96 (16 parts) 30.9 -> 33.2; 16: 8 14.1 -> 8.5, 32 21.0 -> 15.0, 48 20.4 -> 18.7, 96 21.7 -> 27.7;
-//   * D = 128, 256: 1 tile 13.5 -> 11.4, 8 18.9 -> 14.9, 32 28.9 -> 24.4, 48 32.9 -> 30.6; 320: 1 tile 13.8 -> 16.0, 8 19.5 -> 23.0;
-//     128: 8 18.1 -> 13.5, 32 25.0 -> 23.8, 48 27.6 -> 29.8; 16: 8 17.2 -> 12.4, 32 22.4 -> 20.5, 48 22.5 -> 25.6.
-static int short_rows(const AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus) {
+// The workgroups have to be resident together: of eight wavefronts one a CU at D = 128 and two at D = 64, of four twice as many.
+// us per call, workgroups of 256 rows -> of 32 with eight wavefronts, with four, by workgroups and key tiles:
+//   * D = 64 128 workgroups, 3 tiles 15.2 -> 8.0, 7.8; 6 17.6 -> 8.8, 9.2; 16 19.5 -> 10.9, 11.8; 32 22.7 -> 16.5, 19.0; (256, 48 tiles 24.6 -> 21.6;
+//     16, 48 tiles 20.4 -> 18.7, 96 in up to 16 parts 21.7 -> 27.7);
+//     512, 1 tile 13.9 -> 8.8, 7.8; 10 17.2 -> 13.6, 13.2; 32 28.5 -> 25.2, 25.2; 768, 1 tile 15.5 -> 14.6, 9.5; 10 18.6 -> 21.8, 17.1; 32 30.3 -> 31.7, 29.4;
+//     1024, 6 tiles 20.6 -> 23.6, 19.8; 10 21.8 -> 27.1, 23.7; 1536, 1 tile 16.3 -> 22.8, 17.9;
+//   * D = 128 128 workgroups, 3 tiles 14.4 -> 11.0, 10.8; 6 17.7 -> 12.5, 12.8; 32 24.6 -> 23.4, 27.2; (16, 32 tiles 22.4 -> 20.5; 128, 48 tiles
+//     27.6 -> 29.8); 384, 1 tile 13.8 -> 15.9, 11.7; 6 19.1 -> 20.8, 17.3; 10 21.0 -> 25.0, 21.4; 512, 6 tiles 21.3 -> 23.4, 19.6; 768, 1 tile
+//     15.5 -> 22.5, 18.2.
+static ShortRows short_rows(const AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus) {
   const int rows_most = std::min(a.nqt * kBQ, a.Sq);
   int rows = 0, tiles = 0;
   for (int j = 0; j < n_jobs; ++j) {
     rows = std::max(rows, a.cu_q ? rows_most : size[j].rows);
     tiles = std::max(tiles, size[j].tiles);
   }
-  const int slices = (rows + 31) / 32;
-  const int64_t per_xcd = ((int64_t)a.B * a.H * slices + kXcds - 1) / kXcds;
-  constexpr int kMostTiles = 32;
-  return a.q_prescaled || per_xcd * n_jobs > (D == 64 ? 2 : 1) * cus || tiles > kMostTiles ? 0 : slices;
+  ShortRows s;
+  s.slices = (rows + 31) / 32;
+  s.per_xcd = ((int64_t)a.B * a.H * s.slices + kXcds - 1) / kXcds;
+  if (a.q_prescaled) return {};
+  const int64_t units = s.per_xcd * n_jobs;
+  const bool one_a_cu = units <= cus;
+  if (tiles > (D == 64 || one_a_cu ? 32 : 8) || units > (D == 128 ? 2 : tiles <= 6 ? 4 : 3) * cus) return {};
+  s.waves = one_a_cu && tiles > 4 ? 8 : 4;
+  return s;
 }
 
 // The launch as it is planned (and the fold kernel behind it).
-static int launch_planned(AttnArgs& a, int D, int n_jobs, int slices, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
+static int launch_planned(AttnArgs& a, int D, int n_jobs, const ShortRows& rows, hipStream_t stream, void* workspace, int64_t workspace_bytes) {
   const int64_t slot_bytes = partial_state_bytes(D);
   const unsigned planes_x = (unsigned)a.per_xcd * kXcds;
-  if (slices > 0) {
-    AttnRows r;
-    static_cast<AttnArgs&>(r) = a;
-    r.part_ways = slices;
-    r.tail_items = (int)(((int64_t)a.B * a.H * slices + kXcds - 1) / kXcds);
-    return launch_dim(r, D, dim3((unsigned)r.tail_items * kXcds, (unsigned)n_jobs, 1), stream);
+  if (rows.waves > 0) {
+    a.part_ways = rows.slices;
+    a.tail_items = (int)rows.per_xcd;
+    const dim3 grid((unsigned)rows.per_xcd * kXcds, (unsigned)n_jobs, 1);
+    return rows.waves == 8 ? launch_dim(AttnRows8{a}, D, grid, stream) : launch_dim(AttnRows4{a}, D, grid, stream);
   }
   if (a.tail_items == 0) return launch_dim(a, D, dim3(planes_x, (unsigned)n_jobs, 1), stream);
   const int64_t slots = (int64_t)a.tail_items * kXcds * a.part_ways;
@@ -2349,13 +2377,13 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
   a.row_split = 0;
   constexpr int kMaxLaunchJobs = DT_MAX_JOBS * DT_MAX_SEGMENTS;   // (more: no planning)
   bool merge_after = false;
-  int slices = 0;   // of 32 rows, where workgroups take one each
+  ShortRows rows;
   if (n_jobs <= kMaxLaunchJobs) {
     JobSize size[kMaxLaunchJobs];
     job_sizes(a, n_jobs, size);
     const int cus = xcd_cus();
     const bool split = cus > 0 && workspace;
-    if (split) slices = short_rows(a, D, n_jobs, size, cus);
+    if (split) rows = short_rows(a, D, n_jobs, size, cus);
     const TailPlan plan = plan_launch(a, D, n_jobs, size, cus, split ? std::min(workspace_bytes, kWorkspaceBytes) / partial_state_bytes(D) : -1);
     a.tail_items = plan.items;
     a.part_ways = plan.ways;
@@ -2364,12 +2392,12 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
     if (a.arrive) {
       int longest = 0;
       for (int j = 0; j < n_jobs; ++j) longest = std::max(longest, size[j].tiles);
-      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan) || (slices > 0 && a.merge_n > kRowsStates);
+      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan) || (rows.waves > 0 && a.merge_n > kRowsStates);
     }
   }
-  if (!merge_after) return launch_planned(a, D, n_jobs, slices, stream, workspace, workspace_bytes);
+  if (!merge_after) return launch_planned(a, D, n_jobs, rows, stream, workspace, workspace_bytes);
   a.arrive = nullptr;
-  if (int rc = launch_planned(a, D, n_jobs, slices, stream, workspace, workspace_bytes)) return rc;
+  if (int rc = launch_planned(a, D, n_jobs, rows, stream, workspace, workspace_bytes)) return rc;
   return merge_behind(a, D, stream);
 }
 

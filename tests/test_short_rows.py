@@ -1,4 +1,4 @@
-"""Launches of few query rows: workgroups of 32 queries whose wavefronts take every eighth key tile each (``short_rows`` and
+"""Launches of few query rows: workgroups of 32 queries whose eight or four wavefronts take every eighth or fourth key tile each (``short_rows`` and
 ``attn_rows32`` in ditango_amd/csrc/attn_fwd.hip).  Without a GPU: which launches these are.  On it: every number of rows and keys at
 which a slice, a tile or a wavefront's turn begins or ends, against fp64 on the CPU.
 
@@ -12,32 +12,36 @@ from oracle import attention_math as om
 from tests.launch_log import record
 
 OUT_TOL, LSE_TOL = 2e-2, 1e-3
-TAKES_ROWS = "AttnRowsE"
 
 
 def _listed(D, H, Sq, jobs, keys, B=1, **k):
     return dict(B=B, Sq=Sq, H=H, D=D, lens=[keys] * jobs, jobs=[[j] for j in range(jobs)], merged=0, **k)
 
 
-RULE = [
-    # slices of an XCD: 64 and 65 at D = 64, 32 and 33 at D = 128; ragged slices count whole
-    (_listed(64, 16, 1024, 1, 64), True), (_listed(64, 17, 1024, 1, 64), False), (_listed(64, 16, 1025, 1, 64), False),
-    (_listed(128, 8, 1024, 1, 64), True), (_listed(128, 8, 1025, 1, 64), False), (_listed(128, 1, 256 * 32, 1, 64), True),
-    (_listed(128, 4, 500, 4, 64), True), (_listed(128, 4, 500, 5, 64), False), (_listed(64, 2, 33, 1, 64, B=128), True), (_listed(64, 2, 33, 1, 64, B=129), False),
-    # key tiles of the longest job; fp16; without a workspace items stay whole
-    (_listed(64, 4, 100, 2, 2048), True), (_listed(64, 4, 100, 2, 2049), False), (_listed(128, 4, 100, 2, 2048), True),
-    (_listed(128, 4, 100, 2, 2049), False), (_listed(128, 4, 100, 1, 7, fp16=True), True), (_listed(128, 4, 100, 1, 7, workspace=False), False),
-    (dict(B=1, Sq=40, H=3, D=64, lens=[1000, 1000, 48], jobs=[[0, 1, 2], [2]], merged=0), False),
-    (dict(B=1, Sq=40, H=3, D=64, lens=[1000, 1000, 0], jobs=[[0, 1, 2], [2]], merged=0), True),
-    (dict(B=1, Sq=300, H=3, D=64, lens=[300, 2049], jobs=None, max_jobs=1, merged=0), False),
-    (dict(B=1, Sq=300, H=3, D=64, lens=[300, 2048], jobs=None, max_jobs=2, merged=0), True),
+RULE = [   # the launch, wavefronts of a workgroup of 32 rows (0: other workgroups)
+    # slices of an XCD, 32 CUs: at D = 64 128 for up to 6 key tiles and 96 beyond, at D = 128 64; ragged slices count whole
+    (_listed(64, 32, 1024, 1, 384), 4), (_listed(64, 33, 1024, 1, 384), 0), (_listed(64, 32, 1025, 1, 64), 0),
+    (_listed(64, 24, 1024, 1, 385), 4), (_listed(64, 25, 1024, 1, 385), 0), (_listed(64, 2, 33, 1, 2048, B=192), 4), (_listed(64, 2, 33, 1, 2048, B=193), 0),
+    (_listed(128, 16, 1024, 1, 64), 4), (_listed(128, 17, 1024, 1, 64), 0), (_listed(128, 4, 500, 8, 64), 4), (_listed(128, 4, 500, 9, 64), 0),
+    # eight wavefronts: one workgroup a CU, more than 4 tiles
+    (_listed(64, 8, 1024, 1, 256), 4), (_listed(64, 8, 1024, 1, 257), 8), (_listed(64, 8, 1025, 1, 257), 4),
+    (_listed(128, 8, 1024, 1, 256), 4), (_listed(128, 8, 1024, 1, 257), 8), (_listed(128, 8, 1025, 1, 257), 4),
+    # key tiles of the longest job: 32, and 8 at D = 128 with more workgroups than CUs
+    (_listed(64, 4, 100, 2, 2048), 8), (_listed(64, 4, 100, 2, 2049), 0), (_listed(128, 4, 100, 2, 2048), 8),
+    (_listed(128, 4, 100, 2, 2049), 0), (_listed(128, 8, 1025, 1, 512), 4), (_listed(128, 8, 1025, 1, 513), 0),
+    (dict(B=1, Sq=40, H=3, D=64, lens=[1000, 1000, 48], jobs=[[0, 1, 2], [2]], merged=0), 0),
+    (dict(B=1, Sq=40, H=3, D=64, lens=[1000, 1000, 0], jobs=[[0, 1, 2], [2]], merged=0), 8),
+    (dict(B=1, Sq=300, H=3, D=64, lens=[300, 2049], jobs=None, max_jobs=1, merged=0), 0),
+    (dict(B=1, Sq=300, H=3, D=64, lens=[300, 2048], jobs=None, max_jobs=2, merged=0), 8),
+    # fp16; without a workspace items stay whole
+    (_listed(128, 4, 100, 1, 7, fp16=True), 4), (_listed(128, 4, 100, 1, 7, workspace=False), 0),
 ]
 
 
 def test_which_launches_take_32_rows_a_workgroup(tmp_path):
-    for (call, short), kernels in zip(RULE, record(tmp_path, [call for call, _ in RULE])):
-        assert (TAKES_ROWS in kernels[0][1]) == short, call
-        assert not short or len(kernels) == 1, call
+    for (call, waves), kernels in zip(RULE, record(tmp_path, [call for call, _ in RULE])):
+        assert [w for w in (4, 8) if f"AttnRows{w}E" in kernels[0][1]] == [waves] * (waves > 0), call
+        assert not waves or len(kernels) == 1, call
 
 
 def _view(x, order):
@@ -57,14 +61,14 @@ def _view(x, order):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128])
 def test_edges_of_slices_and_tiles(hip, D, dtype, order):
-    B, H = 2, 2
+    B = 2
     g = torch.Generator().manual_seed(D + (dtype == torch.float16))
-    for rows in (1, 31, 32, 33, 100, 257):
+    for rows, H in ((1, 2), (31, 2), (32, 2), (33, 2), (100, 2), (257, 2), (257, 16)):   # (the last: more workgroups than CUs)
         q = torch.randn(B, rows, H, D, generator=g).to(dtype)
         dq = _view(q, order)
         # one chunk; several with short and empty ones between, so that turns end inside and between chunks
-        for lens in ((1,), (31,), (33,), (64,), (65,), (448,), (513,), (2048,), (0, 1, 0, 64, 63), (130, 0, 300, 5, 700)):
-            print(f"case D={D} {dtype} {order} rows={rows} keys={lens}", flush=True)
+        for lens in ((1,), (31,), (33,), (64,), (65,), (256,), (257,), (448,), (512,), (513,), (2048,), (0, 1, 0, 64, 63), (130, 0, 300, 5, 700)):
+            print(f"case D={D} {dtype} {order} rows={rows} heads={H} keys={lens}", flush=True)
             ks, vs = ([torch.randn(B, n, H, D, generator=g).to(dtype) for n in lens] for _ in range(2))
             laid = "plain" if order == "heads" and len(lens) > 1 else order   # (the chunks of a table share their strides)
             table = hip.ChunkTable([_view(k, laid) for k in ks], [_view(v, laid) for v in vs])
