@@ -188,8 +188,10 @@ constexpr float kSumLimit = 4096.0f;
 // simply exp2(score), and a tile is redone when its sum exceeds 2^40.
 constexpr float kSumLimitPre = 1099511627776.0f;
 constexpr float kBandLo = -40.f, kBandHi = 24.f;
-// References of up to this many log2 units are taken off by the MFMAs themselves (see kRefInC).  A score near 0 under a reference
-// of 64 keeps an absolute error of 2^-18, some times that of a score of this size; beyond it the reference comes off in the vector ALU.
+// References of up to this many log2 units are taken off by the MFMAs themselves (see kRefInC).  A score near 0 then keeps the
+// roundings of D / 16 MFMAs at the size of the reference: 8 times 2^-18 at most, 2^-15 log2 units, for references of 64.  (Where the reference is
+// above it, its weight is 2^-64; one below it is a first tile's, which a later one leaves.)  Beyond that the scores stay whole and the
+// reference comes off in the exponent.
 constexpr float kRefInCMost = 64.f;
 
 template <int D>
@@ -1062,12 +1064,11 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
     if constexpr (!kLoadAfterMatrix) load_tile((kU + DT_SCHED_CALL_AHEAD + group) & (kNumBuf - 1));
     // (kPre: the same rare branch takes the reference off the scores of a wavefront in which some
     // row has left the band; everywhere else the reference is 0 and there is nothing to subtract)
-    if (__builtin_expect(cp_valid < kBK || ((kPre || kRefInC) && any_off), 0)) {
+    if (__builtin_expect(cp_valid < kBK || (kPre && any_off), 0)) {
       // the empty asm has side effects as far as the compiler knows, which keeps this a real
       // branch: otherwise the selects below are hoisted out and run for every tile
       asm volatile("" ::: "memory");
       const int lim = cp_valid - key0;
-      const float ref_taken = m_ref > -INFINITY ? m_ref : 0.f;
 #pragma unroll
       for (int kb = 0; kb < kKeyBlocks; ++kb)
 #pragma unroll
@@ -1075,7 +1076,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
           const int key = 32 * kb + 16 * (r >> 3) + 8 * hh + (r & 7);
           if (key >= lim) s_acc[kb][r] = -INFINITY;
           if constexpr (kPre) s_acc[kb][r] -= m_ref;
-          if constexpr (kRefInC) s_acc[kb][r] -= ref_taken + neg_ref[0];
+          if constexpr (kRefInC) asm volatile("" : "+v"(s_acc[kb][r]));   // one compare and select after the other: 115 spilled scalars otherwise
         }
     }
     // Probabilities relative to the reference maximum the accumulators are scaled to.  The
@@ -1086,12 +1087,37 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
     // with its exact maximum.
     float mc = m_ref * c;
     float rs0 = rs_bias, rs1 = 0.f;
+    auto weigh = [&](float off) __attribute__((always_inline)) {   // probabilities and their sums, `off` (log2 units) off the scores
+      rs0 = 0.f;
+      rs1 = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < kKeyBlocks; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          f32x2 p;
+          p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r], c, -off));
+          p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r + 1], c, -off));
+          rs0 += p.x;
+          rs1 += p.y;
+          const ex2 pb = __builtin_convertvector(p, ex2);
+          p_frag[kb][r >> 3][r & 7] = pb.x;
+          p_frag[kb][r >> 3][(r & 7) + 1] = pb.y;
+        }
+    };
     // The first tile of a work item always takes the exact path below (its reference is still -inf), so its pass
     // through the common path is thrown away: skip it.  Results are bit-identical; +0.4-0.5 % at D = 128.  (At
     // D = 64 the extra branch costs registers the kernel does not have: 36 spills, -18 %; it keeps the plain form.)
     if (D == 128 && __builtin_expect(t == 0, 0)) {
       asm volatile("" ::: "memory");   // keeps this a real branch
       rs0 = INFINITY;
+    } else if (kRefInC && __builtin_expect(any_off, 0)) {
+      // Rows whose reference is beyond what the MFMAs take: their scores are whole, and the reference comes off in the exponent
+      // (0 for the wavefront's other rows).  Taken off the scores themselves it would leave them no more than its own last bits, which a
+      // later tile with a larger maximum needs: behind 64 keys at scores of -1e5 a score of 1 was off by 6e-3.  us per call, off the
+      // scores -> this: 24 heads x 4001 queries, 2 chunks, logits of sigma 16 437 -> 390, of sigma 1 (no such row) 319 -> 320; 24 x 14 882, 4
+      // chunks 10 720 -> 9220, 8270 -> 8310.
+      asm volatile("" ::: "memory");   // a real branch
+      weigh(((m_ref > -INFINITY ? m_ref : 0.f) + neg_ref[0]) * c);
     } else
 #pragma unroll
     for (int kb = 0; kb < kKeyBlocks; ++kb)
@@ -1140,7 +1166,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         rs_bias = first && !(mx > -INFINITY) ? INFINITY : 0.f;
         mx = m_new - m_ref;  // what the scores in s_acc still have to lose
       } else {
-        const float taken = kRefInC && m_ref > -INFINITY ? m_ref : 0.f;   // off the scores already
+        const float taken = kRefInC ? -neg_ref[0] : 0.f;   // off the scores already
         m_new = fmaxf(m_ref, mx + taken);
         mx = m_new - taken;
         alpha = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m_ref - m_new) * c) : 1.f;
@@ -1164,21 +1190,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         limit = __any(!(m_new > -INFINITY)) ? -1.f : kSumLimit;
       }
       if constexpr (kPre) any_off = any_off || __any(m_ref != 0.f);
-      rs0 = 0.f;
-      rs1 = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < kKeyBlocks; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          f32x2 p;
-          p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r], c, -mc));
-          p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r + 1], c, -mc));
-          rs0 += p.x;
-          rs1 += p.y;
-          const ex2 pb = __builtin_convertvector(p, ex2);
-          p_frag[kb][r >> 3][r & 7] = pb.x;
-          p_frag[kb][r >> 3][(r & 7) + 1] = pb.y;
-        }
+      weigh(mc);
     }
     l_run += rs0 + rs1;
     ring_prefill(u_tag);

@@ -62,3 +62,34 @@ def test_rows_whose_first_tiles_hold_no_finite_score(hip, D):
     torch.cuda.synchronize()
     assert (out.float().cpu() - ref_out).abs().max().item() <= OUT_TOL
     assert (lse.cpu() - ref_lse).abs().max().item() <= LSE_TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+def test_scores_behind_a_reference_far_below_keep_their_bits(hip, D, dtype):
+    """A first tile of scores about -``below`` for every row, then keys of ordinary ones: the lse is that of the ordinary keys alone, and its
+    error that of their own sums, however far below the first reference lies.  Tolerance: |q| |k| / sqrt(D) is below 5, so 128 roundings of
+    2^-24 of it are below 4e-5; a reference that the MFMAs take (up to 64 log2 units, 44 natural ones) adds D / 16 roundings of 2^-18 log2
+    units, 2.2e-5 in all."""
+    H = 2
+    for below in (38.0, 60.0, 1e3, 3e4) + ((1e5, 1e7) if dtype == torch.bfloat16 else ()):
+        for rows in (40, 100, 300):
+            for keys in (1, 3, 150):
+                print(f"case D={D} {dtype} below={below} rows={rows} keys={keys}", flush=True)
+                g = torch.Generator().manual_seed(rows + keys)
+                base = torch.randn(1, 1, H, D, generator=g)
+                base /= base.norm(dim=-1, keepdim=True)
+                q = (torch.randn(1, rows, H, D, generator=g) * 0.3 + 6 * base).to(dtype)
+                first = (-base * (below * D ** 0.5 / 6)).expand(1, 64, H, D).to(dtype)
+                k = (torch.randn(1, keys, H, D, generator=g) * 0.4).to(dtype)
+                v = [torch.randn(1, n, H, D, generator=g).to(dtype) for n in (64, keys)]
+                assert (q.float().norm(dim=-1).max() * k.float().norm(dim=-1).max() / D ** 0.5).item() < 5
+                ref_out, ref_lse = om.chunk_attention(q, torch.cat([first, k], 1), torch.cat(v, 1), compute_dtype=torch.float64)
+                table = hip.ChunkTable([first.cuda(), k.cuda()], [x.cuda() for x in v])
+                for workspace in (None, hip.attn_workspace("cuda")):
+                    out = torch.empty(1, rows, H, D, dtype=dtype, device="cuda")
+                    lse = torch.empty(1, H, rows, device="cuda")
+                    hip.attn_jobs_fwd(q.cuda(), table, [[0, 1]], [out], [lse], workspace=workspace)
+                    torch.cuda.synchronize()
+                    assert (out.double().cpu() - ref_out).abs().max().item() <= OUT_TOL
+                    assert (lse.double().cpu() - ref_lse).abs().max().item() <= (6.2e-5 if below < 44 else 4e-5)
