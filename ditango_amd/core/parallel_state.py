@@ -60,8 +60,9 @@ class LocalRingGroup:
 
     def kv_lists(self, n: int, local: int, key, value) -> Tuple[list, list]:
         """K and V of chunks 0 ... n - 1 as two lists, chunk ``local`` (-1: none) being ``(key, value)``: what ``kv_chunk`` gives one
-        by one.  With every chunk in place that is two copied lists; whatever ``kv_chunk`` would raise, it raises."""
-        if n == len(self._k) and "kv_chunk" not in self.__dict__:
+        by one.  With every chunk in place and a ``kv_chunk`` that nobody has replaced, on the object or on the class, that is two
+        copied lists; whatever ``kv_chunk`` would raise, it raises."""
+        if n == len(self._k) and type(self).kv_chunk is _KV_CHUNK and "kv_chunk" not in self.__dict__:
             ks, vs = self._k.copy(), self._v.copy()
             if local >= 0:
                 ks[local], vs[local] = key, value
@@ -80,6 +81,8 @@ class LocalRingGroup:
 
     p2p_isend = p2p_irecv = p2p_commit = p2p_wait = _no_p2p
 
+
+_KV_CHUNK = LocalRingGroup.kv_chunk
 
 _USP: Optional[LocalRingGroup] = None
 _ISP: Dict[int, LocalRingGroup] = {}

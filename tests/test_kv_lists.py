@@ -31,3 +31,20 @@ def test_lists_are_the_chunks_one_by_one(n, local, missing, patched):
     got = group.kv_lists(n, local, key, value)
     assert all(a is b for g, w in zip(got, want) for a, b in zip(g, w)) and [len(g) for g in got] == [n, n]
     assert got[0] is not group._k and all(a is b for a, b in zip(group._k, ks))
+
+
+def test_a_lookup_replaced_on_the_class_is_called(monkeypatch):
+    group = LocalRingGroup(3)
+    ks, vs = ([torch.full((1,), float(10 * s + i)) for i in range(3)] for s in (1, 2))
+    group.set_kv_chunks(ks, vs)
+    asked = []
+
+    def lookup(self, c):
+        asked.append(c)
+        return ks[0], vs[c]
+
+    monkeypatch.setattr(LocalRingGroup, "kv_chunk", lookup)
+    key, value = torch.zeros(1), torch.ones(1)
+    got = group.kv_lists(3, 1, key, value)
+    assert asked == [0, 2]
+    assert all(a is b for g, w in zip(got, ([ks[0], key, ks[0]], [vs[0], value, vs[2]])) for a, b in zip(g, w))
