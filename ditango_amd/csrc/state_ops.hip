@@ -644,13 +644,16 @@ __global__ __launch_bounds__(kThreads) void state_copy_units_kernel(const CopyAr
 // instead of as a tail) move the lse: tiles of a power of two of query positions x up to 256 heads, through the LDS as [s][h], so that
 // both sides are read and written in runs whichever way the [H][S] / [S][H] layouts differ, each lane's up to 4 loads side by side.
 //
-// What bounds it: memory, and in small launches the lse's two waits, one behind the other.  A store reads what has just been computed,
-// and what it writes is read next, so both go through the caches; what a load reads and writes does not.  us per store and load of
-// one state, 3 states taking turns [16 of them], rows mapped to lane groups, a row's lse moved by its first lane, nothing cached ->
-// this: 2222 x 48 heads, D = 64 19.0 -> 14.5 [19.1 -> 16.2], 9001 x 48 60.2 -> 51.8 [60.0 -> 52.0], 2000 x 12 6.5 -> 5.8 [7.0 -> 5.9]; D =
-// 128 900 x 24 9.4 -> 7.7 [9.9 -> 8.0], 3001 x 30 26.9 -> 22.4 [27.1 -> 24.2], 14 882 x 24 88.3 -> 81.6 [88.2 -> 81.5]; 300 x 8, D =
-// 64, two launches of little more than nothing, 4.5 -> 5.1.  Of the first the lse is 0.3 us (tiles with a division an element and one load
-// at a time 2.1); a store that caches neither side costs 1 us more with 3 states and 0.9 less with 16.
+// What bounds it: memory, and in small launches the lse's two waits, one behind the other.  Nothing is cached, in either direction: what a
+// sampler stores it loads a denoising step later, behind every other layer.  us, rows mapped to lane groups with a row's lse moved
+// by its first lane -> this through the caches -> this:
+//   * the state computed and stored, 16 states taking turns (the time of both): 14 882 x 24 heads, D = 128 96.9 -> 110.0 -> 93.8, 6851 x 48 91.9 ->
+//     99.8 -> 86.0, 3001 x 30 30.9 -> 30.6 -> 28.3, 900 x 24 9.4 -> 11.5 -> 9.1; D = 64 9001 x 48 64.3 -> 66.8 -> 59.0, 2222 x 48 19.9 -> 20.7 -> 18.8;
+//   * stored, and the state of 15 stores before loaded: 14 882 x 24 89.3 -> 95.2 -> 91.3, 6851 x 48 82.7 -> 87.5 -> 84.1, 3001 x 30 27.7 ->
+//     29.4 -> 28.2; D = 64 9001 x 48 61.0 -> 60.8 -> 58.2, 2222 x 48 19.6 -> 19.2 -> 18.0;
+//   * stored and loaded at once, the only order that the caches serve, 3 states taking turns: 2222 x 48 19.6 -> 16.4 -> 18.3, 14 882 x 24 90.9 ->
+//     83.6 -> 91.9.
+// Of the 2222 x 48 the lse is 0.3 us (tiles with a division an element and one load at a time 2.1).
 constexpr int kConvThreads = 256;
 constexpr int kConvGroups = 2;      // groups of 4 elements of a lane
 constexpr int kLseHeads = 256;      // most heads of an lse tile
@@ -722,7 +725,7 @@ __global__ __launch_bounds__(kConvThreads) void state_convert_kernel(const CopyA
   for (int u = 0; u < kConvGroups; ++u) {
     const int64_t g = g0 + u * kConvThreads;
     if (g >= plan.groups) continue;
-    if constexpr (kNarrow) wide[u] = reinterpret_cast<const u32x4*>(a.src_out)[g];
+    if constexpr (kNarrow) wide[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.src_out) + g);
     else narrow[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(a.src_out) + g);
   }
 #pragma unroll
@@ -732,7 +735,7 @@ __global__ __launch_bounds__(kConvThreads) void state_convert_kernel(const CopyA
     if constexpr (kNarrow) {
       narrow[u].x = pack16x2(__uint_as_float(wide[u][0]), __uint_as_float(wide[u][1]), kHalf);
       narrow[u].y = pack16x2(__uint_as_float(wide[u][2]), __uint_as_float(wide[u][3]), kHalf);
-      reinterpret_cast<u32x2*>(a.dst_out)[g] = narrow[u];
+      __builtin_nontemporal_store(narrow[u], reinterpret_cast<u32x2*>(a.dst_out) + g);
     } else {
       float x[4];
       widen16x2(narrow[u].x, kHalf, x[0], x[1]);
