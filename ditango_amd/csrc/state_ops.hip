@@ -473,6 +473,11 @@ __device__ __forceinline__ uint32_t bhs_of(const RowIndex& at, uint32_t row) {
   const uint32_t b = quotient(bs, at.by_s), q = bs - b * (uint32_t)at.Sq;
   return (b * (uint32_t)at.H + h) * (uint32_t)at.Sq + q;
 }
+__device__ __forceinline__ uint32_t bsh_of(const RowIndex& at, uint32_t row) {   // the other way round
+  const uint32_t bh = quotient(row, at.by_s), q = row - bh * (uint32_t)at.Sq;
+  const uint32_t b = quotient(bh, at.by_h), h = bh - b * (uint32_t)at.H;
+  return (b * (uint32_t)at.Sq + q) * (uint32_t)at.H + h;
+}
 static RowIndex row_index(int B, int Sq, int H) {
   RowIndex at{};
   at.Sq = Sq;
@@ -657,10 +662,12 @@ __global__ __launch_bounds__(kThreads) void state_copy_units_kernel(const CopyAr
 constexpr int kConvThreads = 256;
 constexpr int kConvGroups = 2;      // groups of 4 elements of a lane
 constexpr int kLseHeads = 256;      // most heads of an lse tile
+constexpr int kDirectRows = 1 << 14;   // below: a lane moves one value of the lse
 struct ConvertPlan {
   int64_t groups;                   // of 4 elements
   uint32_t lse_wgs;
-  int32_t run_shift;                // log2 of an lse tile's query positions
+  int32_t run_shift;                // log2 of an lse tile's query positions; -1: a lane moves one value
+  RowIndex at;                      // of those lanes
 };
 
 // One lse tile.
@@ -711,11 +718,22 @@ __device__ __forceinline__ void move_lse_tile(const CopyArgs& a, int wg, int run
   }
 }
 
+// One value of the lse, in the destination's order.  A launch of few rows is over before a tile's two waits and its barrier: us per store
+// and load, 16 states taking turns, rows mapped to lane groups -> tiles -> this: D = 64 300 x 8 heads 4.4 -> 5.1 -> 4.3, 512 x 4 4.3 -> 4.9 -> 4.0, 1000 x
+// 12 5.5 -> 5.8 -> 5.2; D = 128 300 x 8 4.9 -> 5.4 -> 4.4; from 2^14 rows on tiles: 2000 x 12 6.4 -> 6.3 -> 6.3, D = 128 900 x 24 9.3 -> 8.5 -> 8.8.
+__device__ __forceinline__ void move_lse_value(const CopyArgs& a, const RowIndex& at) {
+  const uint32_t i = blockIdx.x * kConvThreads + threadIdx.x;
+  if (i >= at.rows) return;
+  const bool src_bsh = a.src_bsh != 0, dst_bsh = a.dst_bsh != 0;
+  a.dst_lse[i] = a.src_lse[src_bsh == dst_bsh ? i : dst_bsh ? bhs_of(at, i) : bsh_of(at, i)];
+}
+
 template <bool kNarrow, bool kHalf>
 __global__ __launch_bounds__(kConvThreads) void state_convert_kernel(const CopyArgs a, const ConvertPlan plan) {
   extern __shared__ float conv_lds[];
   if (blockIdx.x < plan.lse_wgs) {
-    move_lse_tile(a, blockIdx.x, plan.run_shift, conv_lds);
+    if (plan.run_shift < 0) move_lse_value(a, plan.at);
+    else move_lse_tile(a, blockIdx.x, plan.run_shift, conv_lds);
     return;
   }
   const int64_t g0 = (int64_t)(blockIdx.x - plan.lse_wgs) * (kConvThreads * kConvGroups) + threadIdx.x;
@@ -1005,18 +1023,25 @@ struct LaunchCopyRows64 {
 
 // An lse tile's query positions: one value a lane or two, in runs of at least 16, or where there are many rows 64 (whole lines of a [H][S]
 // tensor; with fewer rows the few workgroups that result finish long behind the others), and no more than 4096 values: every
-// workgroup of the launch holds that much LDS.
+// workgroup of the launch holds that much LDS.  Launches of few rows have no tiles.
 static int launch_convert(const CopyArgs& a, int D, bool with_lse, hipStream_t stream) {
   const int64_t rows = (int64_t)a.B * a.Sq * a.H;
   const int heads = std::min(a.H, kLseHeads);
   ConvertPlan plan{};
   plan.groups = rows * D / 4;
-  plan.run_shift = 4;
-  while (plan.run_shift < 8 && heads << plan.run_shift <= 128) ++plan.run_shift;
-  if (rows >= 1 << 18)
-    while (plan.run_shift < 6 && heads << (plan.run_shift + 1) <= 4096) ++plan.run_shift;
-  const int64_t runs = ((int64_t)a.Sq + (1 << plan.run_shift) - 1) >> plan.run_shift;
-  const int64_t w_lse = with_lse ? a.B * runs * ((a.H + kLseHeads - 1) / kLseHeads) : 0;
+  int64_t w_lse = 0;
+  if (with_lse && rows < kDirectRows) {
+    plan.run_shift = -1;
+    plan.at = row_index(a.B, a.Sq, a.H);
+    w_lse = (rows + kConvThreads - 1) / kConvThreads;
+  } else if (with_lse) {
+    plan.run_shift = 4;
+    while (plan.run_shift < 8 && heads << plan.run_shift <= 128) ++plan.run_shift;
+    if (rows >= 1 << 18)
+      while (plan.run_shift < 6 && heads << (plan.run_shift + 1) <= 4096) ++plan.run_shift;
+    const int64_t runs = ((int64_t)a.Sq + (1 << plan.run_shift) - 1) >> plan.run_shift;
+    w_lse = a.B * runs * ((a.H + kLseHeads - 1) / kLseHeads);
+  }
   const int64_t w_out = (plan.groups + kConvThreads * kConvGroups - 1) / (kConvThreads * kConvGroups);
   if (w_out + w_lse >= 1ll << 24) {   // (fewer than 2^32 lanes)
     set_error("copy grid too large");
@@ -1024,7 +1049,7 @@ static int launch_convert(const CopyArgs& a, int D, bool with_lse, hipStream_t s
   }
   plan.lse_wgs = (uint32_t)w_lse;
   const dim3 grid((unsigned)(w_out + w_lse)), block(kConvThreads);
-  const size_t lds = with_lse ? (size_t)(heads << plan.run_shift) * 4 : 0;
+  const size_t lds = with_lse && plan.run_shift >= 0 ? (size_t)(heads << plan.run_shift) * 4 : 0;
   if (a.src_dtype == DT_FP32) {
     if (a.dst_dtype == DT_FP16) hipLaunchKernelGGL((state_convert_kernel<true, true>), grid, block, lds, stream, a, plan);
     else hipLaunchKernelGGL((state_convert_kernel<true, false>), grid, block, lds, stream, a, plan);

@@ -33,3 +33,26 @@ def test_store_and_load_are_one_rounding_and_its_widening(hip, D, dtype, bsh):
         back_out, back_lse = hip.cache_load(slot_out, slot_lse, torch.float32, bsh)
         assert torch.equal(back_out, slot_out.float())
         assert torch.equal(back_lse.reshape(given.shape), given)
+
+
+# 2^14 rows: below, a lane moves one value of the lse, from there on it goes in tiles
+DIRECT_EDGE = [(1, 16383, 1), (1, 16384, 1), (2, 8192, 1), (1, 2340, 7), (1, 2341, 7), (3, 1820, 3), (3, 1821, 3), (3, 455, 12), (1, 63, 257), (1, 64, 257),
+               (2, 13, 600), (2, 14, 600), (1, 40000, 1)]
+
+
+@pytest.mark.parametrize("src_bsh", [False, True])
+@pytest.mark.parametrize("dst_bsh", [False, True])
+def test_few_rows_and_tiles_move_every_value_of_the_lse(hip, src_bsh, dst_bsh):
+    for B, S, H in DIRECT_EDGE:
+        print(f"case {src_bsh} -> {dst_bsh} {B} x {S} x {H}", flush=True)
+        g = torch.Generator(device="cuda").manual_seed(S * H)
+        out = torch.randn(B, S, H, 64, generator=g, device="cuda")
+        lse, given = _lse(B, S, H, src_bsh, g)
+        slot_out = torch.full((B, S, H, 64), 7.0, dtype=torch.bfloat16, device="cuda")
+        slot_lse = torch.full((B, H, S), 7.0, device="cuda")
+        hip.cache_store(out, given, slot_out, slot_lse)
+        assert torch.equal(slot_out, out.bfloat16()) and torch.equal(slot_lse, lse)
+        back_out, back_lse = hip.cache_load(slot_out, slot_lse, torch.float32, dst_bsh)
+        assert torch.equal(back_out, slot_out.float())
+        want = lse.transpose(1, 2).unsqueeze(-1) if dst_bsh else lse
+        assert torch.equal(back_lse.reshape(want.shape), want)
