@@ -1508,7 +1508,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
 // (They name the kernel, by its wavefronts; part_ways: slices of 32 rows of a head, tail_items: slices of an XCD.)
 struct AttnRows8 : AttnArgs {};
 struct AttnRows4 : AttnArgs {};
-constexpr int kRowsStates = 4;    // states that such a launch merges itself, at most (short_launch_merges allows no more)
+constexpr int kRowsStates = 4;    // states that a short launch merges itself, at most (short_launch_merges)
 // LDS: the tile of each wavefront (afterwards its share of the state), references and sums, 32 result rows.
 template <int D, int W>
 struct Rows32 {
@@ -1957,8 +1957,16 @@ static int launch_one(const Args& a, dim3 grid, hipStream_t stream) {
 template <typename Args>
 static int launch_dim(const Args& a, int D, dim3 grid, hipStream_t stream) {
   if (a.arrive) {
-    if (a.elem_f16) return D == 128 ? launch_one<128, false, true, true>(a, grid, stream) : launch_one<64, false, true, true>(a, grid, stream);
-    return D == 128 ? launch_one<128, false, false, true>(a, grid, stream) : launch_one<64, false, false, true>(a, grid, stream);
+    // (eight wavefronts are for more than 4 key tiles, and at D = 128 a launch of so few rows merges up to 4: this cannot fire; it guards later
+    // edits to either rule)
+    constexpr bool kBuilt128 = !std::is_same_v<Args, AttnRows8>;
+    if (D == 128 && !kBuilt128) {
+      set_error("internal: no merging launch of eight wavefronts a workgroup is built for head dim 128");
+      return DT_ERR_INVALID;
+    }
+    if constexpr (kBuilt128)
+      if (D == 128) return a.elem_f16 ? launch_one<128, false, true, true>(a, grid, stream) : launch_one<128, false, false, true>(a, grid, stream);
+    return a.elem_f16 ? launch_one<64, false, true, true>(a, grid, stream) : launch_one<64, false, false, true>(a, grid, stream);
   }
   if (a.elem_f16) return D == 128 ? launch_one<128, false, true, false>(a, grid, stream) : launch_one<64, false, true, false>(a, grid, stream);
   if constexpr (std::is_same_v<Args, AttnArgs>)
@@ -2330,13 +2338,16 @@ static bool long_launch_merges(int D, int n_jobs, int per_xcd, int tiles, int cu
 //     160 and 2 (8 x 147, 2 tiles 1.16, 20 x 156, one 1.11; 3 tiles are even: 12 x 142 1.01, 24 x 156 0.95); 48 x 119, 18 items 0.95, 24 x
 //     103, 7 tiles 0.94, 12 x 200, 4 tiles 18.4 -> 20.8 [17.9 -> 20.7], 24 x 200, one tile 0.98, 12 x 253, one tile 0.94.  With the host's
 //     list up to 24 items of 4 key tiles (48 x 254, 24 items 32.1 -> 29.8 [20.8 -> 25.0]; 48 x 400, 48 items 32.3 -> 36.4);
-//   * (measured with workgroups of 256 rows; those of 32 follow the same rule, a merge of 4 or 8 rows a wavefront being shorter);
+//   * measured with workgroups of 256 rows, and kept for those of 32, whose wavefronts merge 4 or 8 rows each;
 //   * up to 4 states: 8 are twice the loads of the chain (D = 64 24 x 269 17.0 -> 21.7, D = 128 20 x 200 19 -> 25);
-//   * items in up to two parts: three and more are folded one after the other (3 x 1706, D = 64, 4 parts 0.91).
+//   * items in up to two parts: three and more are folded one after the other (3 x 1706, D = 64, 4 parts 0.91).  The parts are those of
+//     workgroups of 256 rows also where the launch takes 32, which has none: such a launch of 17 to 32 key tiles at D = 64 leaves its merge to the
+//     kernel behind it and would be shorter with its own (3 x 1706, 1 of 4 chunks 16.5 -> 13.7 [15.0 -> 12.6], 24 x 96, 1 of 2 of 2048 keys 16.1 -> 14.0
+//     [15.5 -> 13.8], 12 x 900, 1 of 2 of 1600 20.5 -> 18.2 [20.2 -> 18.1]).
 static bool short_launch_merges(int D, int Sq, int n_states, int n_jobs, bool host_listed, int per_xcd, int tiles, int cus) {
   const int64_t items = (int64_t)n_jobs * per_xcd;
   const bool small = Sq <= kBQ / 2;
-  if (n_states > 4) return false;
+  if (n_states > kRowsStates) return false;
   if (D == 64) return small || items <= (host_listed ? 48 : 12) || (n_jobs == 1 && tiles >= 24) || (cus > 0 && per_xcd >= cus && tiles >= 10);
   return (items <= (host_listed ? 24 : 12) && (small || host_listed) && tiles <= 4) || (items <= 12 && Sq <= 160 && tiles <= 2);
 }
@@ -2404,7 +2415,7 @@ int launch_attn(const AttnArgs& a_in, int D, int n_jobs, hipStream_t stream, voi
     if (a.arrive) {
       int longest = 0;
       for (int j = 0; j < n_jobs; ++j) longest = std::max(longest, size[j].tiles);
-      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan) || (rows.waves > 0 && a.merge_n > kRowsStates);
+      merge_after = !merges_in_launch(a, D, n_jobs, longest, cus, plan);
     }
   }
   if (!merge_after) return launch_planned(a, D, n_jobs, rows, stream, workspace, workspace_bytes);

@@ -5,9 +5,12 @@ which a slice, a tile or a wavefront's turn begins or ends, against fp64 on the 
 Tolerances: a result is one rounding to its type away from a sum of values below 4.5 (2^-9 of them, 9e-3; fp16 2^-12), whose
 probabilities are rounded to the same type (2^-9 of a weighted mean of such values): 2e-2, as in the kernels' other tests.  The lse
 is fp32: 1e-3."""
+import json
+
 import pytest
 import torch
 
+from ditango_amd import build
 from oracle import attention_math as om
 from tests.launch_log import record
 
@@ -145,3 +148,14 @@ def test_scores_of_minus_infinity_and_nan(hip, D):
     assert (lse[:, :1, fine] - ref_lse[:, :, fine]).abs().max().item() <= LSE_TOL
     assert out[:, 40, 0].isnan().all()
     assert (out[:, :, 1] == 0).all() and (lse[:, 1] == float("-inf")).all()
+
+
+def test_no_form_is_built_that_no_launch_takes(tmp_path):
+    """At D = 128 eight wavefronts take more than 4 key tiles and a merging launch up to 4: no call, whoever lists its jobs, takes both, and the
+    kernel for it is not there.  Every other form is taken by some call."""
+    calls = [dict(B=1, Sq=Sq, H=H, D=D, lens=[64 * tiles] * 4, jobs=listed, max_jobs=0 if listed else jobs, merged=merged, fp16=fp16)
+             for D in (64, 128) for Sq, H in ((32, 1), (96, 24), (128, 16), (160, 20), (512, 4), (300, 16)) for tiles in (1, 2, 4, 5, 8)
+             for jobs in (1, 2) for listed in (None, [[j] for j in range(jobs)]) for merged in (0, 2) for fp16 in (False, True)]
+    taken = {k for kernels in record(tmp_path, calls) for _, k in kernels if "AttnRows" in k}
+    built = {k for kernels in json.loads(build.RESOURCES_PATH.read_text()).values() for k in kernels if "AttnRows" in k}
+    assert taken == built
