@@ -1044,7 +1044,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   // Behind this barrier the leading group computes the scores of tile 1, so K of tile 1 has to be in
   // the LDS from ALL wavefronts.  The leading group waits for its share at the end of its vector
   // phase; the trailing group is in its score-only phase here and has no vector phase in between,
-  // so it waits for its share now (of its 8 kLoads loads, the 4 kLoads oldest: V(-1), K0, V0, K1).
+  // so it waits for its share now (of the 7 shares of its four calls, the 3 oldest: K0, V0, K1).
   // From tile 2 on, the wait that ends a group's vector phase covers the tile the other group
   // reads next.
   if (group == 1) wait_tile_loads<DT_SCHED_TRAILING_K1_INFLIGHT * T::kLoads>();
