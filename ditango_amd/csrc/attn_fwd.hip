@@ -1498,7 +1498,7 @@ __global__ __launch_bounds__(kThreads, D == 64 ? kWavesPerSimdD64 : 2) void attn
 // registers and LDS of its own, with no barrier; their states meet once, in fp32 through the LDS.  A chunk of 512 keys is one
 // tile deep.  Four wavefronts do the same where there are more slices than CUs, or fewer tiles than wavefronts.  The keys and values
 // are read by eight times as many workgroups: 110 GB/s a CU out of the L2 is what long items are bound by, and why short_rows
-// ends at 32 tiles.
+// ends at 32 tiles, or earlier (most_tiles).
 // us per call, workgroups of 256 (128) queries -> this: D = 64 4 heads x 512 queries, 2 of 4 chunks 15.1 -> 9.2, 8 x 1024, 1 of 4 18.9 ->
 // 10.9, 16 x 300, 2 of 4 17.8 -> 10.3, 16 x 64 10.4 -> 7.1; D = 128 4 x 512 17.7 -> 13.5, 4 x 128 14.7 -> 8.8, 24 x 128 15.3 -> 9.9,
 // 8 x 1024 24.1 -> 18.7.
@@ -2243,6 +2243,20 @@ struct ShortRows {
 //   * D = 128 128 workgroups, 3 tiles 14.4 -> 11.0, 10.8; 6 17.7 -> 12.5, 12.8; 32 24.6 -> 23.4, 27.2; (16, 32 tiles 22.4 -> 20.5; 128, 48 tiles
 //     27.6 -> 29.8); 384, 1 tile 13.8 -> 15.9, 11.7; 6 19.1 -> 20.8, 17.3; 10 21.0 -> 25.0, 21.4; 512, 6 tiles 21.3 -> 23.4, 19.6; 768, 1 tile
 //     15.5 -> 22.5, 18.2.
+// At D = 64 with more workgroups than CUs, long jobs come back to workgroups of 256 rows.  A job's keys are then read by several workgroups
+// that share CUs with others (time of 32 rows against 256, some 600 launches of 1 ... 384 heads x 8 ... 4000 queries, batch and jobs in all splits):
+//   * a head's rows in one slice: 0.77 ... 1.00 up to 32 tiles, however many heads there are;
+//   * in two: up to 2 workgroups a CU 0.88 ... 1.00 for 16 tiles, 0.94 ... 1.21 for 22 and more (8 x 24 heads x 48, 30 tiles 29.6 -> 36.0); up to 3 1.01 ... 1.14
+//     from 14 tiles on (16 x 24 x 64, 17 tiles 30.3 -> 34.6), but 0.82 ... 0.97 where a head's keys lie within 256 bytes of each other (two heads
+//     of a contiguous tensor: 192 x 2 x 33, 32 tiles 51.7 -> 42.7);
+//   * in more: up to 2 workgroups a CU 0.77 ... 1.05, 0.88 on average; up to 3 0.93 ... 1.03 for 10 tiles, 0.96 ... 1.07 for 13, to 1.5 for more (4 x 48 x 109, 29 tiles
+//     29.5 -> 44.1; 24 x 969, 31 tiles 24.2 -> 26.1; 1 x 48 x 254, two jobs of 32 24.6 -> 27.4).
+static int most_tiles(const AttnArgs& a, int D, int slices, int64_t units, int cus) {
+  if (units <= cus) return 32;
+  if (D == 128) return 8;
+  if (slices == 1 || (slices == 2 && a.kv_ss <= 2 * D)) return 32;
+  return units > 2 * cus ? 10 : slices == 2 ? 16 : 32;
+}
 static ShortRows short_rows(const AttnArgs& a, int D, int n_jobs, const JobSize* size, int cus) {
   const int rows_most = std::min(a.nqt * kBQ, a.Sq);
   int rows = 0, tiles = 0;
@@ -2255,9 +2269,8 @@ static ShortRows short_rows(const AttnArgs& a, int D, int n_jobs, const JobSize*
   s.per_xcd = ((int64_t)a.B * a.H * s.slices + kXcds - 1) / kXcds;
   if (a.q_prescaled) return {};
   const int64_t units = s.per_xcd * n_jobs;
-  const bool one_a_cu = units <= cus;
-  if (tiles > (D == 64 || one_a_cu ? 32 : 8) || units > (D == 128 ? 2 : tiles <= 6 ? 4 : 3) * cus) return {};
-  s.waves = one_a_cu && tiles > 4 ? 8 : 4;
+  if (units > (D == 128 ? 2 : tiles <= 6 ? 4 : 3) * cus || tiles > most_tiles(a, D, s.slices, units, cus)) return {};
+  s.waves = units <= cus && tiles > 4 ? 8 : 4;
   return s;
 }
 

@@ -159,3 +159,19 @@ def test_no_form_is_built_that_no_launch_takes(tmp_path):
     taken = {k for kernels in record(tmp_path, calls) for _, k in kernels if "AttnRows" in k}
     built = {k for kernels in json.loads(build.RESOURCES_PATH.read_text()).values() for k in kernels if "AttnRows" in k}
     assert taken == built
+
+
+# at D = 64 with more workgroups than CUs: key tiles by the slices of a head (one, two, two of heads side by side, more)
+LONG_JOBS = [
+    (_listed(64, 24, 32, 2, 2048, B=7), 4), (_listed(64, 24, 32, 1, 2048, B=11), 4), (_listed(64, 24, 32, 2, 2049, B=7), 0),
+    (_listed(64, 24, 33, 1, 1024, B=8), 4), (_listed(64, 24, 33, 1, 1025, B=8), 0), (_listed(64, 24, 64, 1, 1025, B=8), 0),
+    (_listed(64, 24, 64, 1, 640, B=16), 4), (_listed(64, 24, 64, 1, 641, B=16), 0),
+    (_listed(64, 2, 64, 1, 2048, B=190), 4), (_listed(64, 3, 64, 1, 2048, B=127), 0), (_listed(64, 2, 65, 1, 641, B=120), 0),
+    (_listed(64, 24, 65, 1, 2048, B=4), 4), (_listed(64, 16, 1024, 1, 2048), 4), (_listed(64, 16, 1025, 1, 640), 4), (_listed(64, 16, 1025, 1, 641), 0),
+    (_listed(64, 48, 109, 1, 1830, B=4), 0), (_listed(64, 24, 969, 1, 1984), 0), (_listed(64, 8, 1024, 1, 2048), 8),
+]
+
+
+def test_long_jobs_of_more_workgroups_than_cus_keep_256_rows(tmp_path):
+    for (call, waves), kernels in zip(LONG_JOBS, record(tmp_path, [call for call, _ in LONG_JOBS])):
+        assert [w for w in (4, 8) if f"AttnRows{w}E" in kernels[0][1]] == [waves] * (waves > 0), call
