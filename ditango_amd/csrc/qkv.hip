@@ -371,10 +371,11 @@ int launch(QkvArgs& a, bool half, hipStream_t stream) {
 }
 
 // Which tile a launch takes: 64 x 256, two workgroups a CU, 192 x 256, 256 x 256 or 320 x 256.  The time of each in us is its rounds of the
-// 256 CUs times the 64-channel steps of one, and what a round and the launch cost on top; constants fitted to 70 launches of 8 ... 48 heads
-// (8 ... 48 steps) x 280 ... 12 000 tokens (errors 4 to 5 %; the choice takes 0.9 % more than the best on average).  us, modules and producer ->
-// 64 x 256 / 192 x 256 / 256 x 256 / 160 x 512 (now 320 x 256, which loads a seventh less and takes 1 % less): 16 heads x 602 tokens 42 -> 18 / 34 / 39 / 49; 24 x 4330 108 -> 94 / 87 / 105 / 78; 48 x 2222
-// 153 -> 167 / 141 / 171 / 130 (252 workgroups of 160 x 512, one round); 48 x 3328 198 -> 248 / 214 / 186 / 235 (468 of 256 x 256, two).
+// 256 CUs times the 64-channel steps of one, and what a round and the launch cost on top; constants fitted in loops of calls, those of the last one with
+// tiles of 160 x 512, whose place it has taken.  Over 77 launches of 8 ... 48 heads (8 ... 48 steps) x 280 ... 12 000 tokens with the GPU kept busy the
+// choice takes 0.04 % more than the best of the four on average and 2.7 % at most (24 x 11 853: 206 us, 320 x 256 200); the times are 11 to 17 % above
+// the measured ones, those of each tile alike.  us, 64 x 256 / 192 x 256 / 256 x 256 / 320 x 256: 16 heads x 602 tokens 15 / 27 / 33 / 42; 24 x 4330
+// 93 / 81 / 95 / 70; 48 x 2222 162 / 129 / 157 / 120 (252 workgroups of 320 x 256, one round); 48 x 3328 241 / 194 / 172 / 207 (468 of 256 x 256, two).
 enum Tiles { kFew, kSome, kMore, kMany };
 Tiles plan(int M, int N, int K) {
   constexpr int kCus = 32;   // of an XCD

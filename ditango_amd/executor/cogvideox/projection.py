@@ -11,7 +11,7 @@ from ...producer import _f32
 
 HEAD_DIM = 64
 # Operations beyond which the library's products may be faster, the launches around them included (us, modules -> one launch): 48 heads x
-# 2222 tokens x 3072 channels, 126 GFLOP, 153 -> 127; 3328 tokens, 188 GFLOP, 198 -> 181; 4454, 252 GFLOP, 239 -> 253; 8016 429 -> 458.
+# 2222 tokens x 3072 channels, 126 GFLOP, 153 -> 122; 3328 tokens, 188 GFLOP, 198 -> 173; 4454, 252 GFLOP, 239 -> 253; 8016 429 -> 458.
 MOST_FLOPS = 2.0e11
 
 
