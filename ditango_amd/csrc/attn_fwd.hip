@@ -190,8 +190,8 @@ constexpr float kSumLimitPre = 1099511627776.0f;
 constexpr float kBandLo = -40.f, kBandHi = 24.f;
 // References of up to this many log2 units are taken off by the MFMAs themselves (see kRefInC).  A score near 0 then keeps the
 // roundings of D / 16 MFMAs at the size of the reference: 8 times 2^-18 at most, 2^-15 log2 units, for references of 64.  (Where the reference is
-// above it, its weight is 2^-64; one below it is a first tile's, which a later one leaves.)  Beyond that the scores stay whole and the
-// reference comes off in the exponent.
+// above it, its weight is 2^-64; one below it is a first tile's, which a later one leaves.)  Beyond that the scores stay whole and their
+// maximum comes off in the exponent.
 constexpr float kRefInCMost = 64.f;
 
 template <int D>
@@ -861,7 +861,7 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
   // reference (raw scores; kPre: log2 units) the accumulators are scaled to
   float m_ref = kPre ? 0.f : -INFINITY;
   float rs_bias = kPre ? INFINITY : 0.f;  // kPre: inf until the row has seen a key (forces the exact path)
-  bool any_off = false;                   // some row of this wavefront has a reference that the scores do not start from (kPre: other than 0)
+  bool any_off = kRefInC;                 // some row of this wavefront has a reference that the scores do not start from (kPre: other than 0)
   float limit = kSumLimit;                // kRefInC: -1, below every sum, while some row of this wavefront has no reference
   f32x16 neg_ref;                         // kRefInC: what the scores start from
 #pragma unroll
@@ -1087,37 +1087,17 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
     // with its exact maximum.
     float mc = m_ref * c;
     float rs0 = rs_bias, rs1 = 0.f;
-    auto weigh = [&](float off) __attribute__((always_inline)) {   // probabilities and their sums, `off` (log2 units) off the scores
-      rs0 = 0.f;
-      rs1 = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < kKeyBlocks; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          f32x2 p;
-          p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r], c, -off));
-          p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r + 1], c, -off));
-          rs0 += p.x;
-          rs1 += p.y;
-          const ex2 pb = __builtin_convertvector(p, ex2);
-          p_frag[kb][r >> 3][r & 7] = pb.x;
-          p_frag[kb][r >> 3][(r & 7) + 1] = pb.y;
-        }
-    };
     // The first tile of a work item always takes the exact path below (its reference is still -inf), so its pass
     // through the common path is thrown away: skip it.  Results are bit-identical; +0.4-0.5 % at D = 128.  (At
     // D = 64 the extra branch costs registers the kernel does not have: 36 spills, -18 %; it keeps the plain form.)
-    if (D == 128 && __builtin_expect(t == 0, 0)) {
+    // So do all tiles of a wavefront with a reference beyond what the MFMAs take (any_off, which stands for the first tile as well): its scores
+    // are whole, and their maximum comes off in the exponent.  With the reference taken off the scores themselves, those behind a first
+    // tile far below them lost their last bits: behind 64 keys at scores of -1e5 a score of 1 was off by 6e-3.  us per call, off the scores ->
+    // this: 24 heads x 4001 queries, 2 chunks, logits of sigma 16 433 -> 386; 24 x 14 882, 4 chunks 10 500 -> 9780, of sigma 1 (no such row)
+    // 8034 -> 8063.  A branch of its own for these tiles, without the maximum, was faster with them (8910) and slower without (8090).
+    if (D == 128 && __builtin_expect(kRefInC ? any_off : t == 0, 0)) {
       asm volatile("" ::: "memory");   // keeps this a real branch
       rs0 = INFINITY;
-    } else if (kRefInC && __builtin_expect(any_off, 0)) {
-      // Rows whose reference is beyond what the MFMAs take: their scores are whole, and the reference comes off in the exponent
-      // (0 for the wavefront's other rows).  Taken off the scores themselves it would leave them no more than its own last bits, which a
-      // later tile with a larger maximum needs: behind 64 keys at scores of -1e5 a score of 1 was off by 6e-3.  us per call, off the
-      // scores -> this: 24 heads x 4001 queries, 2 chunks, logits of sigma 16 437 -> 390, of sigma 1 (no such row) 319 -> 320; 24 x 14 882, 4
-      // chunks 10 720 -> 9220, 8270 -> 8310.
-      asm volatile("" ::: "memory");   // a real branch
-      weigh(((m_ref > -INFINITY ? m_ref : 0.f) + neg_ref[0]) * c);
     } else
 #pragma unroll
     for (int kb = 0; kb < kKeyBlocks; ++kb)
@@ -1172,7 +1152,8 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         alpha = m_new > -INFINITY ? __builtin_amdgcn_exp2f((m_ref - m_new) * c) : 1.f;
       }
       m_ref = m_new;
-      if (t > 0) {   // (nothing to scale yet)
+      if (t > 0 && (!kRefInC || __any(alpha != 1.f))) {   // (nothing to scale yet, or nothing that changes)
+        if constexpr (kRefInC) asm volatile("" ::: "memory");
         l_run *= alpha;
 #pragma unroll
         for (int i = 0; i < D / 32; ++i)
@@ -1190,7 +1171,21 @@ __device__ __forceinline__ void attn_item(const JobView& view, int b, int h, int
         limit = __any(!(m_new > -INFINITY)) ? -1.f : kSumLimit;
       }
       if constexpr (kPre) any_off = any_off || __any(m_ref != 0.f);
-      weigh(mc);
+      rs0 = 0.f;
+      rs1 = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < kKeyBlocks; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          f32x2 p;
+          p.x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r], c, -mc));
+          p.y = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[kb][r + 1], c, -mc));
+          rs0 += p.x;
+          rs1 += p.y;
+          const ex2 pb = __builtin_convertvector(p, ex2);
+          p_frag[kb][r >> 3][r & 7] = pb.x;
+          p_frag[kb][r >> 3][(r & 7) + 1] = pb.y;
+        }
     }
     l_run += rs0 + rs1;
     ring_prefill(u_tag);
